@@ -5,12 +5,15 @@ built, importing this module raises, and nothing falls back to PyTorch or CPU
 code.  Build it with ``python cnn-mellin_amd/build.py`` (hipcc, gfx950).
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libmellin_hip.so")
+TORCH_PATH = os.path.join(_HERE, "lib", "_mellin_torch.so")
 
 AX_MCORR, AX_MCONV, AX_LCORR, AX_LCONV = 0, 1, 2, 3
 
@@ -19,13 +22,25 @@ _int = ctypes.c_int
 _ptr = ctypes.c_void_p
 _size_t = ctypes.c_size_t
 
-if not os.path.isfile(LIB_PATH):
-    raise ImportError(
-        "%s is missing: build the HIP library first (python %s)"
-        % (LIB_PATH, os.path.join(_HERE, "build.py"))
-    )
+for _path in (LIB_PATH, TORCH_PATH):
+    if not os.path.isfile(_path):
+        raise ImportError(
+            "%s is missing: build the HIP library first (python %s)"
+            % (_path, os.path.join(_HERE, "build.py"))
+        )
 
 lib = ctypes.CDLL(LIB_PATH)
+
+
+def _load_native():
+    """The layers' host path (csrc/torch_layer.cpp), linked against the same library."""
+    loader = importlib.machinery.ExtensionFileLoader("_mellin_torch", TORCH_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mellin_torch", loader))
+    loader.exec_module(module)
+    return module
+
+
+native = _load_native()
 
 _SUFFIX = {torch.float32: "f32", torch.float64: "f64", torch.float16: "f16"}
 
@@ -63,6 +78,10 @@ SYMBOLS["mellin_corr2d_forward_f16"] = (_int, [_int, _ptr, _ptr, _ptr] + _DIMS +
 SYMBOLS["mellin_corr2d_forward_act_f16"] = (_int, [_int, _int, _ptr, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _size_t, _ptr])
 SYMBOLS["mellin_corr2d_backward_input_f16"] = (_int, [_int, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _size_t, _ptr])
 SYMBOLS["mellin_corr2d_backward_weight_f16"] = (_int, [_int, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _size_t, _ptr])
+SYMBOLS["mellin_layer_forward_workspace"] = (_size_t, [_int, _int] + _DIMS)
+SYMBOLS["mellin_layer_forward"] = (_int, [_int, _int, _int, _ptr, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _size_t, _ptr])
+SYMBOLS["mellin_layer_backward_workspace"] = (_size_t, [_int, _int, _int] + _DIMS)
+SYMBOLS["mellin_layer_backward"] = (_int, [_int, _int, _int] + [_ptr] * 4 + _DIMS + [_ptr] * 4 + [_size_t, _ptr])
 _dbl = ctypes.c_double
 PW_LOG, PW_LIFT = 1, 2
 for _t in ("f32", "f64"):

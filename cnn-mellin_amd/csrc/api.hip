@@ -1541,4 +1541,87 @@ int mellin_corr2d_backward_weight_f64(int kind_x, const double *input,
                                         grad_weight, workspace, workspace_bytes, stream);
 }
 
+
+// ---- section 5: whole passes of a layer in one call ---------------------------------------
+size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
+  if (elem_bytes == 2) return mellin_corr2d_forward_f16_workspace(kind_x, CORR2D_ARGS);
+  return mellin_corr2d_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS);
+}
+int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void *input, const void *weight,
+                         const void *bias, MELLIN_CORR2D_DIMS, void *out, void *workspace, size_t workspace_bytes,
+                         void *stream) {
+  if (elem_bytes == 2)
+    return mellin_corr2d_forward_act_f16(kind_x, activation, input, weight, bias, CORR2D_ARGS, out, workspace,
+                                         workspace_bytes, stream);
+  if (elem_bytes == 4)
+    return mellin_corr2d_forward_ws_f32(kind_x, activation, (const float *)input, (const float *)weight,
+                                        (const float *)bias, CORR2D_ARGS, (float *)out, workspace, workspace_bytes,
+                                        stream);
+  return fail(MELLIN_ERR_ARGUMENT, "%s: elements of 2 (half) or 4 (float) bytes only (got %d)", __func__, elem_bytes);
+}
+
+// The regions of the backward call's workspace: the gradient at the convolution's output (with a fused ReLU), then
+// one region that the passes use after each other.
+static size_t layer_backward_layout(int kind_x, int elem, int want, MELLIN_CORR2D_DIMS, size_t *masked_bytes) {
+  size_t pass = 0;
+  if (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)) pass = mellin_bias_grad_workspace(batch, c_out, nhx * nhy);
+  // (a ReLU's backward writes the bias gradient, asked for or not: one more row of partial results)
+  if ((want & MELLIN_WANT_RELU) && !(want & MELLIN_WANT_BIAS)) pass += align256((size_t)c_out * elem);
+  if (want & MELLIN_WANT_INPUT)
+    pass = std::max(pass, elem == 2 ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS)
+                                    : mellin_corr2d_backward_input_workspace(kind_x, elem, CORR2D_ARGS));
+  if (want & MELLIN_WANT_WEIGHT)
+    pass = std::max(pass, elem == 2 ? mellin_corr2d_backward_weight_f16_workspace(kind_x, CORR2D_ARGS)
+                                    : mellin_corr2d_backward_weight_workspace(kind_x, elem, CORR2D_ARGS));
+  *masked_bytes = (want & MELLIN_WANT_RELU) ? align256((size_t)(batch * c_out * nhx * nhy) * elem) : 0;
+  return *masked_bytes + pass;
+}
+size_t mellin_layer_backward_workspace(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS) {
+  if (elem_bytes != 2 && elem_bytes != 4) return 0;
+  if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
+  size_t masked = 0;
+  return layer_backward_layout(kind_x, elem_bytes, want, CORR2D_ARGS, &masked);
+}
+int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *input, const void *weight,
+                          const void *grad_out, const void *out, MELLIN_CORR2D_DIMS, void *grad_input,
+                          void *grad_weight, void *grad_bias, void *workspace, size_t workspace_bytes, void *stream) {
+  int rc;
+  if (elem_bytes != 2 && elem_bytes != 4)
+    return fail(MELLIN_ERR_ARGUMENT, "%s: elements of 2 (half) or 4 (float) bytes only (got %d)", __func__, elem_bytes);
+  if ((rc = check_corr2d(__func__, kind_x, CORR2D_ARGS))) return rc;
+  if (((want & MELLIN_WANT_RELU) && !out) || ((want & MELLIN_WANT_INPUT) && !grad_input) ||
+      ((want & MELLIN_WANT_WEIGHT) && !grad_weight) || ((want & MELLIN_WANT_BIAS) && !grad_bias))
+    return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  size_t masked_bytes = 0;
+  const size_t need = layer_backward_layout(kind_x, elem_bytes, want, CORR2D_ARGS, &masked_bytes);
+  if (need && (!workspace || workspace_bytes < need))
+    return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, need, workspace_bytes);
+  char *pass = (char *)workspace + masked_bytes;
+  const size_t pass_bytes = need - masked_bytes;
+  const bool half = elem_bytes == 2;
+  if (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)) {
+    void *masked = (want & MELLIN_WANT_RELU) ? workspace : nullptr;
+    const size_t own = mellin_bias_grad_workspace(batch, c_out, nhx * nhy);
+    void *gb = (want & MELLIN_WANT_BIAS) ? grad_bias : pass + (pass_bytes - align256((size_t)c_out * elem_bytes));
+    rc = half ? mellin_bias_grad_f16(grad_out, masked ? out : nullptr, batch, c_out, nhx * nhy, masked, gb, pass, own, stream)
+              : mellin_bias_grad_f32((const float *)grad_out, masked ? (const float *)out : nullptr, batch, c_out,
+                                     nhx * nhy, (float *)masked, (float *)gb, pass, own, stream);
+    if (rc) return rc;
+    if (masked) grad_out = masked;
+  }
+  if (want & MELLIN_WANT_INPUT) {
+    rc = half ? mellin_corr2d_backward_input_f16(kind_x, weight, grad_out, CORR2D_ARGS, grad_input, pass, pass_bytes, stream)
+              : mellin_corr2d_backward_input_f32(kind_x, (const float *)weight, (const float *)grad_out, CORR2D_ARGS,
+                                                 (float *)grad_input, pass, pass_bytes, stream);
+    if (rc) return rc;
+  }
+  if (want & MELLIN_WANT_WEIGHT) {
+    rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, grad_weight, pass, pass_bytes, stream)
+              : mellin_corr2d_backward_weight_f32(kind_x, (const float *)input, (const float *)grad_out, CORR2D_ARGS,
+                                                  (float *)grad_weight, pass, pass_bytes, stream);
+    if (rc) return rc;
+  }
+  return MELLIN_OK;
+}
+
 }  // extern "C"

@@ -195,6 +195,12 @@ def _dense_or_transposed(t: torch.Tensor):
 # ---------------------------------------------------------------------------
 # differentiable correlation (MCorr1DOp / MCorrLCorrOp, ext/torch.cpp:176-309)
 # ---------------------------------------------------------------------------
+# Float and half layers run through csrc/torch_layer.cpp (checks, allocations, autograd node and
+# launches in native code); it returns None for whatever it does not handle -- float64, CPU
+# tensors, empty results, arguments that are errors -- and the function below takes those.
+_native_corr = _hip.native.corr
+
+
 class _Corr2dFunction(torch.autograd.Function):
     """out = bias + correlation(input, weight); x axis Mellin or linear, y axis linear."""
 
@@ -253,10 +259,17 @@ class _Corr2dFunction(torch.autograd.Function):
 
 
 def _corr2d(kind_x, name, input, weight, bias, s, d, p, u, r, activation=None):
+    out = _native_corr(kind_x, 2, input, weight, bias, s, d, p, u, r, activation)
+    if out is not None:
+        return out
+    s, d, p, u, r = (_pair(name, k, v) for k, v in zip("sdpur", (s, d, p, u, r)))
     return _Corr2dFunction.apply(input, weight, bias, kind_x, s, d, p, u, r, name, activation)
 
 
 def _corr1d(kind, name, input, weight, bias, s, d, p, u, r, activation=None):
+    out = _native_corr(kind, 1, input, weight, bias, s, d, p, u, r, activation)
+    if out is not None:
+        return out
     # a 1-D layer is the 2-D layer with a unit second axis
     _check_dim(name, weight, "weight", 2, 3)
     _check_dim(name, input, "input", 1, 3)
@@ -274,7 +287,6 @@ def _ext_mcorr1d(input, weight, bias=None, s=1, d=1, p=0, u=1, r=0, activation=N
 def _ext_mcorrlcorr(input, weight, bias=None, s=(1, 1), d=(1, 1), p=(0, 0), u=(1, 1), r=(0, 0),
                     activation=None):
     """``torch.ops.mellin.mcorrlcorr`` (ext/torch.cpp:470)."""
-    s, d, p, u, r = (_pair("mcorrlcorr", k, v) for k, v in zip("sdpur", (s, d, p, u, r)))
     return _corr2d(AX_MCORR, "mcorrlcorr", input, weight, bias, s, d, p, u, r, activation)
 
 
@@ -284,7 +296,6 @@ def _ext_lcorr1d(input, weight, bias=None, s=1, d=1, p=0, u=1, r=0, activation=N
 
 def _ext_lcorrlcorr(input, weight, bias=None, s=(1, 1), d=(1, 1), p=(0, 0), u=(1, 1), r=(0, 0),
                     activation=None):
-    s, d, p, u, r = (_pair("lcorrlcorr", k, v) for k, v in zip("sdpur", (s, d, p, u, r)))
     return _corr2d(AX_LCORR, "lcorrlcorr", input, weight, bias, s, d, p, u, r, activation)
 
 
@@ -442,7 +453,7 @@ def mcorr1d(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
 
     ``activation="relu"`` (not in the reference) returns ``relu(result)`` from the same kernel."""
     _pick_impl("mcorr1d", _impl)
-    return _ext_mcorr1d(input, weight, bias, s, d, p, 1, r, activation)
+    return _corr1d(AX_MCORR, "mcorr1d", input, weight, bias, s, d, p, 1, r, activation)
 
 
 def mcorrlcorr(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -451,24 +462,22 @@ def mcorrlcorr(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     """2-D correlation, Mellin along axis 2 and linear along axis 3; see :class:`MCorrLCorr`.
 
     ``activation="relu"`` (not in the reference) returns ``relu(result)`` from the same kernel."""
-    s_, d_, p_, r_ = (_pair("mcorrlcorr", k, v) for k, v in zip("sdpr", (s, d, p, r)))
     _pick_impl("mcorrlcorr", _impl)
-    return _ext_mcorrlcorr(input, weight, bias, s_, d_, p_, (1, 1), r_, activation)
+    return _corr2d(AX_MCORR, "mcorrlcorr", input, weight, bias, s, d, p, 1, r, activation)
 
 
 def lcorr1d(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
             s: int = 1, d: int = 1, p: int = 0, r: int = 0,
             activation: Optional[str] = None) -> torch.Tensor:
     """1-D linear correlation with left padding ``p`` and right padding ``r``."""
-    return _ext_lcorr1d(input, weight, bias, s, d, p, 1, r, activation)
+    return _corr1d(AX_LCORR, "lcorr1d", input, weight, bias, s, d, p, 1, r, activation)
 
 
 def lcorrlcorr(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                s: Any = 1, d: Any = 1, p: Any = 0, r: Any = 0,
                activation: Optional[str] = None) -> torch.Tensor:
     """2-D linear correlation ("lconv2d") with asymmetric padding ``p`` (left) / ``r`` (right)."""
-    s_, d_, p_, r_ = (_pair("lcorrlcorr", k, v) for k, v in zip("sdpr", (s, d, p, r)))
-    return _ext_lcorrlcorr(input, weight, bias, s_, d_, p_, (1, 1), r_, activation)
+    return _corr2d(AX_LCORR, "lcorrlcorr", input, weight, bias, s, d, p, 1, r, activation)
 
 
 def snd2col(input: torch.Tensor, kernel_width: int, s: int = 1, d: int = 1, p: int = 0,

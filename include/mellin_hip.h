@@ -398,6 +398,32 @@ int mellin_pool_pairs_forward_f16(const void *x, int64_t rows, int64_t f, void *
 int mellin_pool_pairs_backward_f16(const void *grad_y, const unsigned char *which,
                                    int64_t rows, int64_t f, void *grad_x, void *stream);
 
+/* ------------------------------------------------------------------------
+ * 5. Whole passes of a layer in one call: what a training framework's layer needs in its
+ * forward and in its backward pass, on float (elem_bytes 4) or half (elem_bytes 2) tensors,
+ * with the layouts of section 2.  The backward call works out whichever gradients `want`
+ * names; MELLIN_WANT_RELU says that the forward pass applied MELLIN_ACT_RELU, `out` being
+ * its result.  Knowing all that is asked for, it shares between the gradients what they
+ * have in common, so it may be faster than the calls of sections 2 and 4 one by one.
+ * At most 65535 images and output channels in the backward call.  Scratch: the byte count
+ * of the *_workspace call under the same settings, 256-byte aligned.
+ * ------------------------------------------------------------------------ */
+#define MELLIN_WANT_INPUT 1
+#define MELLIN_WANT_WEIGHT 2
+#define MELLIN_WANT_BIAS 4
+#define MELLIN_WANT_RELU 8
+size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS);
+int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void *input,
+                         const void *weight, const void *bias, MELLIN_CORR2D_DIMS,
+                         void *out, void *workspace, size_t workspace_bytes, void *stream);
+size_t mellin_layer_backward_workspace(int kind_x, int elem_bytes, int want,
+                                       MELLIN_CORR2D_DIMS);
+int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *input,
+                          const void *weight, const void *grad_out, const void *out,
+                          MELLIN_CORR2D_DIMS, void *grad_input, void *grad_weight,
+                          void *grad_bias, void *workspace, size_t workspace_bytes,
+                          void *stream);
+
 /* Name of the kernel variant the most recent operator-level call of the
  * process (on any thread: PyTorch runs backward passes on a thread of its own)
  * dispatched to (for tests and profiling): "generic", "mfma" (tiled

@@ -14,6 +14,7 @@
 #include "igrad_gemm.hpp"
 #include "tile_gemm.hpp"
 #include "gather_kernels.hpp"
+#include "block_gemm.hpp"
 #include "narrow_gemm.hpp"
 
 using namespace mellin;
@@ -38,6 +39,7 @@ std::atomic<int> g_no_yfold{0};         // tap products stored per filter column
 std::atomic<int> g_whole_classes{0};    // ... a class's rows never cut into ranges ("whole-classes": for comparisons)
 std::atomic<int> g_gather{0};          // 1: the LDS-gather kernels (vector ALUs) wherever they apply ("lds-gather"); -1: never ("no-gather")
 std::atomic<int> g_no_narrow{0};       // 1: few-channel linear forward passes through the tiled kernel ("no-narrow": for comparisons); -1: their own kernel whatever the size ("narrow": for tests)
+std::atomic<int> g_no_blocks{0};        // layer entry points: never through the channel-blocked kernels ("no-blocks": for comparisons)
 std::atomic<int> g_widen{0};            // half-precision entry points: always through fp32 copies (mellin_set_variant "widen")
 std::atomic<int> g_math{MATH_BF16X3};   // how fp32 products are formed on the matrix cores (mellin_set_math)
 std::atomic<int> g_last_math{MATH_FP32};   // what the kernels of the most recent operator-level call multiplied with
@@ -1393,8 +1395,8 @@ int mellin_last_math(void) { return g_last_math; }
 
 int mellin_set_variant(const char *name) {
   // the name is parsed first: an unknown one changes nothing
-  struct Setting { int forced, widen, no_classes, all_classes, split_classes, whole_classes, no_yfold, gather, no_narrow; };
-  Setting v = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  struct Setting { int forced, widen, no_classes, all_classes, split_classes, whole_classes, no_yfold, gather, no_narrow, no_blocks; };
+  Setting v = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   if (!name || !*name || !strcmp(name, "auto")) {}
   else if (!strcmp(name, "generic")) v.forced = 1;
   else if (!strcmp(name, "two-pass")) v.forced = 2;
@@ -1408,6 +1410,7 @@ int mellin_set_variant(const char *name) {
   else if (!strcmp(name, "no-gather")) v.gather = -1;
   else if (!strcmp(name, "no-narrow")) v.no_narrow = 1;
   else if (!strcmp(name, "narrow")) v.no_narrow = -1;
+  else if (!strcmp(name, "no-blocks")) v.no_blocks = 1;
   else return fail(MELLIN_ERR_ARGUMENT, "mellin_set_variant: unknown variant '%s'", name);
   g_widen = v.widen;
   g_no_classes = v.no_classes;
@@ -1417,6 +1420,7 @@ int mellin_set_variant(const char *name) {
   g_no_yfold = v.no_yfold;
   g_gather = v.gather;
   g_no_narrow = v.no_narrow;
+  g_no_blocks = v.no_blocks;
   g_forced = v.forced;
   return MELLIN_OK;
 }
@@ -1543,44 +1547,119 @@ int mellin_corr2d_backward_weight_f64(int kind_x, const double *input,
 
 
 // ---- section 5: whole passes of a layer in one call ---------------------------------------
+static size_t blocked_region(i64 batch, i64 channels, i64 plane, bool half) {
+  return align256(blocked_bytes(batch, channels, plane, half));
+}
+// Whether the settings in force leave the layer entry points their channel-blocked kernels.
+static bool blocks_allowed(bool half) {
+  return g_forced == 0 && !g_no_blocks && !g_widen && !g_no_classes && !g_all_classes && !g_split_classes && !g_whole_classes &&
+         !g_no_yfold && !g_gather && !g_no_narrow && (half || g_math != MATH_FP32);
+}
+static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp) {
+  if (!blocks_allowed(half) || c_in < 16 || batch * c_out * nhx * nhy == 0) return false;
+  SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
+  pr.out_half = half;
+  return make_block_plan(pr, half, bp);
+}
+static bool plan_block_input(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp) {
+  if (!blocks_allowed(half) || c_in < 16 || batch * c_out * nhx * nhy == 0) return false;
+  SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
+  pr.out_half = half;
+  return make_block_plan(pr, half, bp);
+}
+
 size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
+  if (elem_bytes != 2 && elem_bytes != 4) return 0;
+  if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
+  BlockPlan bp;
+  if (plan_block_forward(kind_x, elem_bytes == 2, CORR2D_ARGS, bp))
+    return blocked_region(batch, c_in, ngx * ngy, elem_bytes == 2) + bp.filter_bytes;
   if (elem_bytes == 2) return mellin_corr2d_forward_f16_workspace(kind_x, CORR2D_ARGS);
   return mellin_corr2d_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS);
 }
 int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void *input, const void *weight,
                          const void *bias, MELLIN_CORR2D_DIMS, void *out, void *workspace, size_t workspace_bytes,
                          void *stream) {
-  if (elem_bytes == 2)
+  int rc;
+  if (elem_bytes != 2 && elem_bytes != 4)
+    return fail(MELLIN_ERR_ARGUMENT, "%s: elements of 2 (half) or 4 (float) bytes only (got %d)", __func__, elem_bytes);
+  if ((rc = check_corr2d(__func__, kind_x, CORR2D_ARGS))) return rc;
+  const bool half = elem_bytes == 2;
+  BlockPlan bp;
+  if (plan_block_forward(kind_x, half, CORR2D_ARGS, bp)) {
+    const size_t signal = blocked_region(batch, c_in, ngx * ngy, half), need = signal + bp.filter_bytes;
+    if (!workspace || workspace_bytes < need)
+      return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, need, workspace_bytes);
+    if (!input || !weight || !out) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+    if (activation != MELLIN_ACT_NONE && activation != MELLIN_ACT_RELU)
+      return fail(MELLIN_ERR_ARGUMENT, "%s: activation must be MELLIN_ACT_NONE or MELLIN_ACT_RELU (got %d)", __func__, activation);
+    bp.relu = activation == MELLIN_ACT_RELU;
+    g_variant = half ? "mfma-f16" : "mfma-blocks";
+    g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
+    hipStream_t st = (hipStream_t)stream;
+    char *ws = (char *)workspace;
+    hipError_t e = launch_pack_filter(bp, (int)c_in, weight, ws + signal, st);
+    if (e == hipSuccess) e = launch_pack_signal(input, nullptr, half, batch, c_in, ngx * ngy, ws, nullptr, st);
+    if (e == hipSuccess) e = launch_block_gemm(bp, ws, ws + signal, bias, out, st);
+    return check_hip(e, __func__);
+  }
+  if (half)
     return mellin_corr2d_forward_act_f16(kind_x, activation, input, weight, bias, CORR2D_ARGS, out, workspace,
                                          workspace_bytes, stream);
-  if (elem_bytes == 4)
-    return mellin_corr2d_forward_ws_f32(kind_x, activation, (const float *)input, (const float *)weight,
-                                        (const float *)bias, CORR2D_ARGS, (float *)out, workspace, workspace_bytes,
-                                        stream);
-  return fail(MELLIN_ERR_ARGUMENT, "%s: elements of 2 (half) or 4 (float) bytes only (got %d)", __func__, elem_bytes);
+  return mellin_corr2d_forward_ws_f32(kind_x, activation, (const float *)input, (const float *)weight,
+                                      (const float *)bias, CORR2D_ARGS, (float *)out, workspace, workspace_bytes, stream);
 }
 
-// The regions of the backward call's workspace: the gradient at the convolution's output (with a fused ReLU), then
-// one region that the passes use after each other.
-static size_t layer_backward_layout(int kind_x, int elem, int want, MELLIN_CORR2D_DIMS, size_t *masked_bytes) {
+// The backward call.  Where the channel-blocked kernels serve a gradient, grad_out is blocked once for all of them, with
+// the backward of a fused ReLU and the bias sums in the same pass; a gradient they do not serve takes the kernels of
+// section 2, on grad_out as it lies (through a fused ReLU: on a masked copy).
+struct LayerBackward {
+  bool input_blocked, weight_blocked, plain;           // plain: some gradient takes the section-2 kernels
+  size_t masked_off, go_off, x_off, frag_off, pass_off, pass_bytes, total;
+  BlockPlan bp;
+  BlockWgradPlan wp;
+};
+static bool plan_block_weight(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockWgradPlan &wp) {
+  if (!blocks_allowed(half) || c_in < 16 || batch * c_out * nhx * nhy == 0) return false;
+  return make_block_wgrad_plan(forward_problem(kind_x, CORR2D_ARGS), half, wp) && wp.ws_bytes <= kMaxWorkspaceBytes;
+}
+static void plan_layer_backward(int kind_x, int elem, int want, MELLIN_CORR2D_DIMS, LayerBackward &lb) {
+  const bool half = elem == 2;
+  const bool wi = want & MELLIN_WANT_INPUT, ww = want & MELLIN_WANT_WEIGHT;
+  lb.input_blocked = wi && plan_block_input(kind_x, half, CORR2D_ARGS, lb.bp);
+  lb.weight_blocked = ww && plan_block_weight(kind_x, half, CORR2D_ARGS, lb.wp);
+  const bool any = lb.input_blocked || lb.weight_blocked;
+  lb.plain = (wi && !lb.input_blocked) || (ww && !lb.weight_blocked) || !any;
+  size_t at = 0;
+  auto take = [&](size_t bytes) { const size_t off = at; at += align256(bytes); return off; };
+  lb.masked_off = take(lb.plain && (want & MELLIN_WANT_RELU) ? (size_t)(batch * c_out * nhx * nhy) * elem : 0);
+  lb.go_off = take(any ? blocked_bytes(batch, c_out, nhx * nhy, half) : 0);
+  lb.x_off = take(lb.weight_blocked ? blocked_bytes(batch, c_in, ngx * ngy, half) : 0);
+  lb.frag_off = take(lb.input_blocked ? lb.bp.filter_bytes : 0);
   size_t pass = 0;
-  if (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)) pass = mellin_bias_grad_workspace(batch, c_out, nhx * nhy);
-  // (a ReLU's backward writes the bias gradient, asked for or not: one more row of partial results)
-  if ((want & MELLIN_WANT_RELU) && !(want & MELLIN_WANT_BIAS)) pass += align256((size_t)c_out * elem);
-  if (want & MELLIN_WANT_INPUT)
-    pass = std::max(pass, elem == 2 ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS)
-                                    : mellin_corr2d_backward_input_workspace(kind_x, elem, CORR2D_ARGS));
-  if (want & MELLIN_WANT_WEIGHT)
-    pass = std::max(pass, elem == 2 ? mellin_corr2d_backward_weight_f16_workspace(kind_x, CORR2D_ARGS)
-                                    : mellin_corr2d_backward_weight_workspace(kind_x, elem, CORR2D_ARGS));
-  *masked_bytes = (want & MELLIN_WANT_RELU) ? align256((size_t)(batch * c_out * nhx * nhy) * elem) : 0;
-  return *masked_bytes + pass;
+  if (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)) {
+    if (lb.plain)                                      // (a ReLU's backward writes the bias gradient, asked for or not)
+      pass = align256(mellin_bias_grad_workspace(batch, c_out, nhx * nhy)) + align256((size_t)c_out * elem);
+    else
+      pass = pack_partial_count(batch, c_out, nhx * nhy) * 4;
+  }
+  if (wi && !lb.input_blocked)
+    pass = std::max(pass, half ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS)
+                               : mellin_corr2d_backward_input_workspace(kind_x, elem, CORR2D_ARGS));
+  if (lb.weight_blocked) pass = std::max(pass, lb.wp.ws_bytes);
+  else if (ww)
+    pass = std::max(pass, half ? mellin_corr2d_backward_weight_f16_workspace(kind_x, CORR2D_ARGS)
+                               : mellin_corr2d_backward_weight_workspace(kind_x, elem, CORR2D_ARGS));
+  lb.pass_bytes = pass;
+  lb.pass_off = take(pass);
+  lb.total = at;
 }
 size_t mellin_layer_backward_workspace(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS) {
   if (elem_bytes != 2 && elem_bytes != 4) return 0;
   if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
-  size_t masked = 0;
-  return layer_backward_layout(kind_x, elem_bytes, want, CORR2D_ARGS, &masked);
+  LayerBackward lb;
+  plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb);
+  return lb.total;
 }
 int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *input, const void *weight,
                           const void *grad_out, const void *out, MELLIN_CORR2D_DIMS, void *grad_input,
@@ -1592,33 +1671,57 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   if (((want & MELLIN_WANT_RELU) && !out) || ((want & MELLIN_WANT_INPUT) && !grad_input) ||
       ((want & MELLIN_WANT_WEIGHT) && !grad_weight) || ((want & MELLIN_WANT_BIAS) && !grad_bias))
     return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
-  size_t masked_bytes = 0;
-  const size_t need = layer_backward_layout(kind_x, elem_bytes, want, CORR2D_ARGS, &masked_bytes);
-  if (need && (!workspace || workspace_bytes < need))
-    return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, need, workspace_bytes);
-  char *pass = (char *)workspace + masked_bytes;
-  const size_t pass_bytes = need - masked_bytes;
-  const bool half = elem_bytes == 2;
-  if (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)) {
-    void *masked = (want & MELLIN_WANT_RELU) ? workspace : nullptr;
+  LayerBackward lb;
+  plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb);
+  if (lb.total && (!workspace || workspace_bytes < lb.total))
+    return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, lb.total, workspace_bytes);
+  char *ws = (char *)workspace, *pass = ws + lb.pass_off;
+  const bool half = elem_bytes == 2, relu = want & MELLIN_WANT_RELU;
+  hipStream_t st = (hipStream_t)stream;
+  hipError_t e = hipSuccess;
+  if (lb.plain && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU))) {
+    void *masked = relu ? ws + lb.masked_off : nullptr;
     const size_t own = mellin_bias_grad_workspace(batch, c_out, nhx * nhy);
-    void *gb = (want & MELLIN_WANT_BIAS) ? grad_bias : pass + (pass_bytes - align256((size_t)c_out * elem_bytes));
+    void *gb = (want & MELLIN_WANT_BIAS) ? grad_bias : pass + align256(own);
     rc = half ? mellin_bias_grad_f16(grad_out, masked ? out : nullptr, batch, c_out, nhx * nhy, masked, gb, pass, own, stream)
               : mellin_bias_grad_f32((const float *)grad_out, masked ? (const float *)out : nullptr, batch, c_out,
                                      nhx * nhy, (float *)masked, (float *)gb, pass, own, stream);
     if (rc) return rc;
     if (masked) grad_out = masked;
   }
-  if (want & MELLIN_WANT_INPUT) {
-    rc = half ? mellin_corr2d_backward_input_f16(kind_x, weight, grad_out, CORR2D_ARGS, grad_input, pass, pass_bytes, stream)
+  if (lb.input_blocked || lb.weight_blocked) {
+    if (!grad_out || (lb.input_blocked && !weight) || (lb.weight_blocked && !input))
+      return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+    const bool sums = !lb.plain && (want & MELLIN_WANT_BIAS);
+    e = launch_pack_signal(grad_out, relu && !lb.plain ? out : nullptr, half, batch, c_out, nhx * nhy, ws + lb.go_off,
+                           sums ? (float *)pass : nullptr, st);
+    if (e == hipSuccess && sums)
+      e = launch_bias_reduce((const float *)pass, (i64)pack_partial_count(batch, 1, nhx * nhy), c_out, grad_bias, half, st);
+  }
+  if (lb.input_blocked && e == hipSuccess) {
+    lb.bp.relu = 0;
+    g_variant = half ? "mfma-f16" : "mfma-blocks";
+    g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
+    e = launch_pack_filter(lb.bp, (int)c_out, weight, ws + lb.frag_off, st);
+    if (e == hipSuccess) e = launch_block_gemm(lb.bp, ws + lb.go_off, ws + lb.frag_off, nullptr, grad_input, st);
+  }
+  if (e != hipSuccess) return check_hip(e, __func__);
+  if ((want & MELLIN_WANT_INPUT) && !lb.input_blocked) {
+    rc = half ? mellin_corr2d_backward_input_f16(kind_x, weight, grad_out, CORR2D_ARGS, grad_input, pass, lb.pass_bytes, stream)
               : mellin_corr2d_backward_input_f32(kind_x, (const float *)weight, (const float *)grad_out, CORR2D_ARGS,
-                                                 (float *)grad_input, pass, pass_bytes, stream);
+                                                 (float *)grad_input, pass, lb.pass_bytes, stream);
     if (rc) return rc;
   }
-  if (want & MELLIN_WANT_WEIGHT) {
-    rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, grad_weight, pass, pass_bytes, stream)
+  if (lb.weight_blocked) {
+    g_variant = half ? "mfma-f16" : "mfma-blocks";
+    g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
+    e = launch_pack_signal(input, nullptr, half, batch, c_in, ngx * ngy, ws + lb.x_off, nullptr, st);
+    if (e == hipSuccess) e = launch_block_wgrad(lb.wp, ws + lb.go_off, ws + lb.x_off, grad_weight, (float *)pass, st);
+    if (e != hipSuccess) return check_hip(e, __func__);
+  } else if (want & MELLIN_WANT_WEIGHT) {
+    rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, grad_weight, pass, lb.pass_bytes, stream)
               : mellin_corr2d_backward_weight_f32(kind_x, (const float *)input, (const float *)grad_out, CORR2D_ARGS,
-                                                  (float *)grad_weight, pass, pass_bytes, stream);
+                                                  (float *)grad_weight, pass, lb.pass_bytes, stream);
     if (rc) return rc;
   }
   return MELLIN_OK;

@@ -1,0 +1,624 @@
+// Forward pass and gather-form input gradient of layers with many channels, from the
+// channel-blocked signal (block_gemm.hpp) on the bf16 / f16 matrix cores.
+//
+//   H[n, m, ox, oy] = bias[m] + sum_{fx, fy, c} F[m, c, fx, fy] * G[n, c, tap_x(ox, fx), tap_y(oy, fy)]
+//
+// The contracted index of a matrix instruction runs over CHANNELS of one tap (two groups of
+// eight), so an operand of the signal is 16 consecutive bytes of one position: one LDS read per
+// register quadruple, nothing to gather, pack or cut in the loop.  What bounded the kernel that
+// reads the tensors as they lie (tile_gemm.hip: eight LDS reads and 44 vector instructions per
+// 16 taps and 32 positions; matrix pipe 8-19 % busy on half tensors, 39-47 % on fp32) is paid
+// once per element in block_pack.hip instead of once per tap and tile of output channels.
+//
+// Tile: P = WN * NT * 32 consecutive output positions of one image x MT * 32 output channels.
+// A stage is F filter rows x G channel groups.  Its signal rows are copied by direct
+// global->LDS loads (16 bytes per lane, any source) into virtual rows as in tile_gemm.hip:
+//   Mellin axis   virtual row (filter row of the stage, output row): the row of that tap;
+//   linear axis   virtual row = coordinate ax ox + bx fx + cx, all filter rows in one stage;
+// positions without a source read the blocked tensor's unit of zeros, so nothing is cleared and
+// a buffer needs no memory of what it held.  The sources of a tile's virtual positions are worked
+// out once per tile into an LDS table.  While a stage multiplies, the next one's loads are issued
+// a few at a time between the steps.  Filter fragments come from L1 / L2 straight to registers,
+// two steps ahead: the WN wavefronts of a workgroup use the same ones at the same time.
+//
+// Mellin axes: output rows are taken in the order of the residue classes of the axis, so the rows
+// of a tile have taps for the same filter rows and only those are staged and multiplied; filter
+// rows none of whose taps lies inside the signal for the tile's rows are left out as well.
+//
+// Few tiles (one utterance, deep layers): WK = 4 wavefronts share the positions of a tile and
+// take every fourth step of a stage; their sums are added in wavefront order through LDS.
+//
+// Measured, 256 -> 256 channels, 4 x 4 taps, 16 x 100 x 41 positions, linear: fp32 1312 -> 1190 us and 107 us
+// for the cut (six bf16 products each: 1.39 PF, matrix pipe 57 % busy at 1.9 GHz, near the rate the board's
+// power allows); half, on Mellin rows, 286 -> 183 us.  One utterance (few tiles, WK = 4): 980 -> 330 us for ten layers.
+#include <algorithm>
+#include <type_traits>
+
+#include "block_gemm.hpp"
+#include "tile_stage.hpp"
+
+namespace mellin {
+
+namespace {
+
+// The plan stays in the kernel arguments and is read by scalar loads where it is used: held in
+// registers for a whole stage its fields would not fit the scalar register file.
+typedef const __attribute__((address_space(4))) BlockPlan ConstBlockPlan;
+
+struct BlockTile {
+  int n, q0, count, row_lo, rows;
+  int vx_min, units;               // linear axes: first coordinate; virtual positions of the whole tile
+  unsigned mask;                   // filter rows with a tap for some row of the tile
+  int nv;                          // how many
+};
+
+__device__ __forceinline__ int nth_bit(unsigned mask, int j) {
+  for (int i = 0; i < j; ++i) mask &= mask - 1;
+  return __builtin_ctz(mask);
+}
+
+// output row of position `row` in the order of the classes
+__device__ __forceinline__ int class_row(ConstBlockPlan &pl, int row) {
+  int ox = row;
+  for (int k = 0; k < pl.n_classes; ++k)
+    if (row >= pl.cls[k].start) ox = pl.cls[k].first + (row - pl.cls[k].start) * pl.cls_stride;
+  return ox;
+}
+
+template <int P>
+__device__ __forceinline__ BlockTile block_tile(ConstBlockPlan &pl, int tile_id, bool mellin_x) {
+  BlockTile g;
+  g.n = tile_id / pl.tiles_per_image;
+  g.q0 = (tile_id - g.n * pl.tiles_per_image) * P;
+  g.count = min(P, pl.Q - g.q0);
+  g.row_lo = g.q0 / pl.noy;
+  const int row_hi = (g.q0 + g.count - 1) / pl.noy;
+  g.rows = row_hi - g.row_lo + 1;
+  g.vx_min = pl.ax * g.row_lo + pl.cx + pl.bx_min;
+  g.mask = 0;
+  if (mellin_x) {
+    for (int k = 0; k < pl.n_classes; ++k) {
+      const int lo = max(g.row_lo, pl.cls[k].start), hi = min(row_hi, (k + 1 < pl.n_classes ? pl.cls[k + 1].start : pl.nox) - 1);
+      if (lo > hi) continue;
+      const int h_lo = pl.cls[k].first + (lo - pl.cls[k].start) * pl.cls_stride + pl.sx;
+      const int h_hi = pl.cls[k].first + (hi - pl.cls[k].start) * pl.cls_stride + pl.sx;
+      for (int f = 0; f < pl.nfx; ++f) {
+        // the tap grows with the row: inside for some row iff the first is not past the end and the last not before 0
+        const int num = pl.kind_x == AX_MCORR ? f + pl.dx : pl.px + 1, den = pl.kind_x == AX_MCORR ? pl.px + 1 : f + pl.dx;
+        if ((pl.cls[k].mask >> f & 1) && h_lo * num <= (pl.ngx - 1 + pl.ux) * den && h_hi * num >= pl.ux * den) g.mask |= 1u << f;
+      }
+    }
+    if (g.mask == 0) g.mask = 1;                     // no tap at all: a stage of zeros
+    g.nv = __builtin_popcount(g.mask);
+    g.units = g.nv * g.rows * pl.RS;
+  } else {
+    g.nv = pl.nfx;
+    g.units = (pl.ax * (g.rows - 1) + pl.bx_span + 1) * pl.RS;
+  }
+  return g;
+}
+
+template <int MT, int NT, int WM, int WK, bool F16, bool HOUT>
+__global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_arg, const char *__restrict__ X,
+                                                                 const char *__restrict__ AF, const void *__restrict__ bias,
+                                                                 void *__restrict__ Hv) {
+  constexpr int PARTS = F16 ? 1 : 3, UB = 16 * PARTS;
+  constexpr int WN = kWaves / WK / WM, P = WN * NT * 32, M_T = WM * MT * 32;
+  constexpr int kALoads = 2 * MT * PARTS;              // fragment loads of two steps
+  extern __shared__ __align__(16) char blk_lds[];
+  ConstBlockPlan *plp = (ConstBlockPlan *)__builtin_amdgcn_kernarg_segment_ptr();
+#define pl (*plp)
+  char *bufs = blk_lds;                                                    // [2][buf_bytes]
+  float *Bs = (float *)(bufs + 2 * pl.buf_bytes);                          // [M_T]
+  int *tab = (int *)(Bs + M_T);                                            // [tab_units] source byte offset in a group's plane
+  int2 *ents = (int2 *)(tab + pl.tab_units);                               // [2][ents] (LDS offset, fragment offset) of a step's half
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, l32 = lane & 31;
+  const int wk = WK > 1 ? wave : 0, wm = WM > 1 ? wave & (WM - 1) : 0, wn = WK > 1 ? 0 : wave / WM;
+  const bool mellin_x = pl.kind_x == AX_MCORR || pl.kind_x == AX_MCONV;
+  const int taps = pl.nfx * pl.nfy;
+  const int m_tile = blockIdx.y;
+  const unsigned zero_frag = (unsigned)(pl.CG * taps * PARTS * 512);       // the tile's fragment of zeros, behind the others
+  const unsigned af_tile = zero_frag + PARTS * 512;                        // bytes of 32 channels' fragments
+  const char *AFm = AF + (i64)(m_tile * WM + wm) * MT * af_tile, *AFm1 = AFm + af_tile;
+  const i64 plane_bytes = (i64)(pl.plane + 1) * UB;
+  const unsigned lds0 = lds_address((const float *)blk_lds);
+  const int my_tiles = (pl.total_tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+
+  if (tid < M_T) {
+    const int m = m_tile * M_T + tid;
+    float b = 0.f;
+    if (bias && m < pl.M) b = F16 ? (float)((const _Float16 *)bias)[m] : ((const float *)bias)[m];
+    Bs[tid] = b;
+  }
+
+  // the sources of a tile's virtual positions, and the operand offsets of its steps
+  constexpr int kWrap = 4 * WK;                        // halves of two steps of every wavefront that shares a tile's steps
+  auto stage_halves = [](int n) { return max((n + 2 * WK - 1) / (2 * WK) * (2 * WK), kWrap); };
+  auto build_tile = [&](const BlockTile &g, int parity, int2 *before) {
+    const FastDiv by_RS(pl.RS), by_rows(g.rows);
+    const int padded = min(pl.tab_units, g.units + 64);
+    for (int v = tid; v < padded; v += kThreads) {
+      int src = pl.plane;
+      if (v < g.units) {
+        int vr, col;
+        by_RS.divmod(v, vr, col);
+        const int vy = pl.cy + pl.by_min + col;
+        int gy = -1, gx = -1;
+        if (vy >= 0) {
+          if (pl.uy == 1) gy = vy;
+          else { const int q = vy / pl.uy; if (q * pl.uy == vy) gy = q; }
+          if (gy >= pl.ngy) gy = -1;
+        }
+        if (mellin_x) {
+          int j, r;
+          by_rows.divmod(vr, j, r);
+          gx = mellin_tap32(pl.kind_x, class_row(pl, g.row_lo + r), nth_bit(g.mask, j), pl.ngx, pl.sx, pl.dx, pl.px + 1, pl.ux,
+                            pl.mg_p1);
+        } else {
+          const int vx = g.vx_min + vr;
+          if (vx >= 0) {
+            if (pl.ux == 1) gx = vx;
+            else { const int q = vx / pl.ux; if (q * pl.ux == vx) gx = q; }
+            if (gx >= pl.ngx) gx = -1;
+          }
+        }
+        if (gx >= 0 && gy >= 0) src = gx * pl.ngy + gy;
+      }
+      tab[v] = src * UB;
+    }
+    // Entries of the tile's stages one behind the other (a last odd half is paired with the fragment of zeros), then
+    // the first two steps again: a stage reads on into the one that follows it.  `before`: the first two steps of
+    // this tile also go behind the entries of the tile before it, whose last stage is running.
+    int2 *out = ents + parity * pl.ents;
+    const int per_row = pl.nfy * pl.G, full = stage_halves(pl.F * per_row), subsets = (g.nv + pl.F - 1) / pl.F;
+    const int tail = stage_halves((g.nv - (subsets - 1) * pl.F) * per_row), n_ents = (subsets - 1) * full + tail;
+    for (int e = tid; e < n_ents + kWrap; e += kThreads) {
+      const int at0 = e < n_ents ? e : e - n_ents;                       // (n_ents >= kWrap)
+      const int sub = min(at0 / full, subsets - 1), at = at0 - sub * full;
+      const int n_e = min(pl.F, g.nv - sub * pl.F) * per_row, k = min(at, n_e - 1);
+      const int jj = k / per_row, rest = k - jj * per_row, fy = rest / pl.G, gi = rest - fy * pl.G;
+      const int fx = mellin_x ? nth_bit(g.mask, sub * pl.F + jj) : jj;
+      const int row = mellin_x ? jj * g.rows : pl.bx * fx - pl.bx_min;
+      const int2 v = make_int2(gi * pl.group_bytes + (row * pl.RS + pl.by * fy - pl.by_min) * UB,
+                               at < n_e ? ((gi * pl.nfx + fx) * pl.nfy + fy) * (PARTS * 512) : 0x40000000);
+      out[e] = v;
+      if (e < kWrap && before) before[e] = v;
+    }
+    return n_ents;
+  };
+
+  // the loads of a stage: group g's slots (16 bytes each) b * 64 .. of block b, blocks dealt to the wavefronts
+  int is_b = 0, is_g = 0, is_left = 0, is_v0 = 0, is_raw = 0, is_part = 0;    // the issue in progress: block, group, loads to go ...
+  int groups = 0, group_bytes = 0;
+  unsigned is_dst = 0, is_to = 0;
+  const char *is_src = nullptr, *is_from = nullptr;
+  auto issue_block = [&]() {                           // (the source is read here and first used a load later)
+    const int slot = is_b * 64 + lane;
+    const int unit = F16 ? slot : slot / 3;
+    is_part = F16 ? 0 : (slot - unit * 3) * 16;
+    is_raw = tab[is_v0 + unit];
+    is_from = is_src;
+    is_to = is_dst + (unsigned)(is_b * 1024);
+  };
+  auto issue_begin = [&](const BlockTile &g, int c0, int j0, int buf) {
+    const int nF = min(pl.F, g.nv - j0);
+    const int units = mellin_x ? nF * g.rows * pl.RS : g.units;
+    is_v0 = mellin_x ? j0 * g.rows * pl.RS : 0;
+    is_b = wave;
+    is_g = 0;
+    is_src = X + ((i64)g.n * pl.CG + c0) * plane_bytes;
+    is_dst = lds0 + (unsigned)(buf * pl.buf_bytes);
+    groups = pl.G;
+    group_bytes = pl.group_bytes;
+    asm volatile("" : "+s"(groups), "+s"(group_bytes));      // (kept in registers: a scalar load in the loop would wait for LDS as well)
+    is_left = max(0, (((units * PARTS + 63) >> 6) - wave + kWaves - 1) / kWaves) * groups;
+    if (is_left > 0) issue_block();
+  };
+  auto issue_one = [&]() {
+    load16_to_lds_at((const float *)is_from, (unsigned)(is_raw + is_part), is_to);
+    is_from += plane_bytes;
+    is_to += (unsigned)group_bytes;
+    --is_left;
+    if (++is_g == groups) {
+      is_g = 0;
+      is_b += kWaves;
+      if (is_left > 0) issue_block();
+    }
+  };
+  auto issue_down_to = [&](int left) {
+    while (is_left > left) issue_one();
+  };
+
+  floatx16 acc[MT][NT];
+  int lane_vpos[NT], lane_q[NT];
+  struct Operands { uintx4 a[MT][PARTS]; };
+  struct SignalOps { uintx4 b[NT][PARTS]; };
+  Operands A0, A1;
+  SignalOps B0, B1;
+
+  const unsigned lane_frag = (unsigned)(l32 * 16), zero_at = zero_frag + lane_frag;
+  auto fetch_a = [&](const int2 &e, unsigned af_c, Operands &o) {
+    const unsigned off = min((unsigned)e.y + af_c + lane_frag, zero_at);
+#pragma unroll
+    for (int k = 0; k < MT; ++k)
+#pragma unroll
+      for (int pt = 0; pt < PARTS; ++pt) o.a[k][pt] = *(const uintx4 *)((k ? AFm1 : AFm) + off + pt * 512);
+  };
+
+  BlockTile tg = block_tile<P>(pl, (int)blockIdx.x, mellin_x), next_tg = tg;
+  if (my_tiles <= 0) return;
+  int n_ents = build_tile(tg, 0, nullptr), next_ents = n_ents;
+  __syncthreads();
+  issue_begin(tg, 0, 0, 0);
+  issue_down_to(0);
+  int c0 = 0, j0 = 0, buf = 0, ti = 0;
+  int se = 0;                                          // the stage's first entry (of this tile's)
+  unsigned af_c = 0;
+  const int2 *my_ents = ents + 2 * wk + half;          // this half-wave's entries (of parity 0)
+  int2 e0 = my_ents[0], e1 = my_ents[2 * WK];
+  fetch_a(e0, 0, A0);
+  fetch_a(e1, 0, A1);
+  wait_and_barrier<0>();
+
+  for (bool first = true;;) {
+    {
+      unsigned zero;                                   // a zero the compiler cannot see through: plan fields are loaded anew per stage
+      asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
+      plp = (ConstBlockPlan *)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + zero);
+    }
+    if (first) {
+      const FastDiv by_noy(pl.noy);
+      // position -> virtual position of its (first filter row, first column) tap; accumulators start from the bias
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        int local = (wn * NT + t) * 32 + l32;
+        if (local >= tg.count) local = 0;
+        int row, oy;
+        by_noy.divmod(tg.q0 + local, row, oy);
+        lane_vpos[t] = (((mellin_x ? 1 : pl.ax) * (row - tg.row_lo)) * pl.RS + pl.ay * oy) * UB;
+        lane_q[t] = (mellin_x ? class_row(pl, row) : row) * pl.noy + oy;
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          float4 bv = *(const float4 *)(Bs + (wm * MT + i) * 32 + g4 * 8 + half * 4);
+          if (WK > 1 && wk > 0) bv = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            acc[i][t][4 * g4 + 0] = bv.x; acc[i][t][4 * g4 + 1] = bv.y;
+            acc[i][t][4 * g4 + 2] = bv.z; acc[i][t][4 * g4 + 3] = bv.w;
+          }
+        }
+    }
+    const char *Xb = bufs + buf * pl.buf_bytes;
+    auto fetch_b = [&](const int2 &e, SignalOps &o) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int pt = 0; pt < PARTS; ++pt) o.b[t][pt] = *(const uintx4 *)(Xb + (lane_vpos[t] + e.x) + pt * 16);
+    };
+    fetch_b(e0, B0);
+    // ---- the stage after this one: its loads are issued under this stage's steps, its first fragments in the last two
+    const int halves = stage_halves((mellin_x ? min(pl.F, tg.nv - j0) : tg.nv) * pl.nfy * pl.G);
+    const int steps = halves / (2 * WK);
+    int nj0 = mellin_x ? j0 + pl.F : tg.nv, nc0 = c0, n_se = se + halves;
+    if (nj0 >= tg.nv) { nj0 = 0; nc0 = c0 + pl.G; n_se = 0; }
+    const bool last = nc0 >= pl.CG;
+    const bool more = !last || ti + 1 < my_tiles;
+    const int2 *ep = my_ents + (ti & 1) * pl.ents + se;
+    is_left = 0;
+    if (last) {
+      nc0 = 0;
+      nj0 = 0;
+      if (more) {
+        // another tile: its tables (every load of this tile has been issued, every wavefront is past the barrier)
+        next_tg = block_tile<P>(pl, (int)blockIdx.x + (ti + 1) * (int)gridDim.x, mellin_x);
+        next_ents = build_tile(next_tg, (ti + 1) & 1, ents + (ti & 1) * pl.ents + n_ents);
+        lds_barrier();
+        issue_begin(next_tg, 0, 0, buf ^ 1);
+      }
+    } else {
+      issue_begin(tg, nc0, nj0, buf ^ 1);
+    }
+    issue_down_to(0);
+    const unsigned n_af = (unsigned)(nc0 * taps * PARTS * 512);
+    // A step: the next step's signal operands are requested before its multiplies and the fragments of the step
+    // after next behind them (pinned: the scheduler moves reads next to their use).  Nothing here depends on which
+    // step it is, so that every wait counts exactly what is younger: the last pair's last signal reads are of no use,
+    // and its fragment fetches are the next stage's.
+    int2 e2 = ep[4 * WK];
+    for (int i = 0; i + 1 < steps; i += 2) {
+      fetch_b(e1, B1);
+      const int2 e3 = ep[6 * WK];
+      __builtin_amdgcn_sched_barrier(0);
+      block_multiply<MT, NT, PARTS>(acc, A0.a, B0.b);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_a(e2, i + 2 < steps ? af_c : n_af, A0);
+      fetch_b(e2, B0);
+      const int2 e4 = ep[8 * WK];
+      __builtin_amdgcn_sched_barrier(0);
+      block_multiply<MT, NT, PARTS>(acc, A1.a, B1.b);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_a(e3, i + 3 < steps ? af_c : n_af, A1);
+      e0 = e2;
+      e1 = e3;
+      e2 = e4;
+      ep += 4 * WK;
+    }
+    if (steps & 1) {
+      // one step left, whose operands are in A0 and B0; A1 holds the next stage's first fragments where its second's belong
+      block_multiply<MT, NT, PARTS>(acc, A0.a, B0.b);
+      e0 = e1;
+      e1 = e2;
+      fetch_a(e0, n_af, A0);
+      fetch_a(e1, n_af, A1);
+    }
+    // every wavefront's loads for the next stage have landed (the newest in flight are the two fragment fetches),
+    // and every wavefront is done with this stage's buffer
+    wait_and_barrier<kALoads>();
+    first = last;
+    if (last) {
+      // ---- the tile is finished
+      if constexpr (WK > 1) {
+        // sums of the wavefronts, in their order (one tile per workgroup: the buffers are free)
+        float *red = (float *)bufs;
+#pragma unroll
+        for (int k = 0; k < MT; ++k)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4)
+              *(float4 *)(red + (((wk * MT * NT + k * NT + t) * 4 + r4) * 64 + lane) * 4) =
+                  make_float4(acc[k][t][4 * r4], acc[k][t][4 * r4 + 1], acc[k][t][4 * r4 + 2], acc[k][t][4 * r4 + 3]);
+        __syncthreads();
+      }
+      // A store is one add and one buffer store: the descriptor ends with the block's last channel, so rows past it
+      // and lanes without a position (an offset past any end) are dropped by its range check.
+      constexpr int ES = HOUT ? 2 : 4;
+      const int h_m = (int)pl.h_m * ES, m0 = m_tile * M_T + wm * MT * 32;
+      const bool relu = pl.relu;
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          (char *)Hv + ((i64)tg.n * pl.h_n * ES + (i64)m0 * h_m), 0, max(0, min(MT * 32, pl.M - m0)) * h_m, 0x00020000);
+      int at[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        at[t] = (wn * NT + t) * 32 + l32 < tg.count ? half * 4 * h_m + lane_q[t] * ES : (int)0x80000000u;
+#pragma unroll
+      for (int k = 0; k < MT; ++k) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            float v = acc[k][t][r];
+            bool mine = true;
+            if constexpr (WK > 1) {
+              mine = ((k * NT + t) & (WK - 1)) == wk;
+              if (mine) {
+                const float *red = (const float *)bufs;
+                v = 0.f;
+#pragma unroll
+                for (int w = 0; w < WK; ++w) v += red[(((w * MT * NT + k * NT + t) * 4 + (r >> 2)) * 64 + lane) * 4 + (r & 3)];
+              }
+            }
+            if (relu) v = fmaxf(v, 0.f);
+            if (mine) {
+              if constexpr (HOUT)
+                __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(short, (_Float16)v), rsrc, at[t], 0, 0);
+              else
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rsrc, at[t], 0, 0);
+            }
+            at[t] += (r & 3) == 3 ? 5 * h_m : h_m;     // (registers 4 g .. 4 g + 3 are rows 8 g + 4 half ..)
+          }
+        }
+      }
+      if (!more) break;
+      ++ti;
+      tg = next_tg;
+      n_ents = next_ents;
+    }
+    c0 = nc0;
+    j0 = nj0;
+    buf ^= 1;
+    se = n_se;
+    af_c = n_af;
+  }
+#undef pl
+}
+
+template <int MT, int NT, int WM, int WK, bool F16, bool HOUT>
+hipError_t launch_instance(const BlockPlan &pl, const void *x, const void *frag, const void *bias, void *out, hipStream_t stream) {
+  auto kern = block_gemm_kernel<MT, NT, WM, WK, F16, HOUT>;
+  static std::atomic<int> lds_allowed{0};
+  hipError_t e = allow_large_lds((const void *)kern, pl.lds_bytes, lds_allowed);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)pl.grid_x, (unsigned)pl.m_tiles), dim3(kThreads), pl.lds_bytes, stream, pl,
+                     (const char *)x, (const char *)frag, bias, out);
+  return hipGetLastError();
+}
+
+// Residue classes of a Mellin axis (mellin_common.hpp: tap relations), those with the same filter
+// rows next to each other.
+void plan_classes(const Axis &x, BlockPlan &pl) {
+  auto gcd = [](i64 a, i64 b) { while (b) { const i64 t = a % b; a = b; b = t; } return a; };
+  i64 L = 1;
+  if (x.kind == AX_MCORR) L = x.p + 1;
+  else if (x.kind == AX_MCONV)
+    for (i64 f = 0; f < x.nf && L <= kBlockClasses; ++f) {
+      const i64 m = (f + x.d) / gcd(f + x.d, x.p + 1);
+      L = L / gcd(L, m) * m;
+    }
+  pl.n_classes = 1;
+  pl.cls_stride = 1;
+  pl.cls[0] = BlockClass{0, 0, (1u << x.nf) - 1};
+  if (L < 2 || L > kBlockClasses) return;
+  struct Item { unsigned mask; int first; } items[kBlockClasses];
+  int n = 0;
+  for (i64 r = 0; r < L; ++r) {
+    const i64 first = ((r - x.s) % L + L) % L;
+    if (first >= x.nh) continue;
+    unsigned mask = 0;
+    for (i64 f = 0; f < x.nf; ++f) {
+      const bool has = x.kind == AX_MCORR ? (r * (f + x.d)) % (x.p + 1) == 0 : r % ((f + x.d) / gcd(f + x.d, x.p + 1)) == 0;
+      if (has) mask |= 1u << f;
+    }
+    items[n++] = Item{mask, (int)first};
+  }
+  std::sort(items, items + n, [](const Item &a, const Item &b) {
+    const int ca = __builtin_popcount(a.mask), cb = __builtin_popcount(b.mask);
+    return ca != cb ? ca > cb : (a.mask != b.mask ? a.mask < b.mask : a.first < b.first);
+  });
+  int start = 0;
+  for (int i = 0; i < n; ++i) {
+    pl.cls[i] = BlockClass{items[i].first, start, items[i].mask};
+    start += (int)((x.nh - items[i].first + L - 1) / L);
+  }
+  pl.n_classes = n;
+  pl.cls_stride = (int)L;
+}
+
+}  // namespace
+
+bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
+  const Axis &X = pr.x, &Y = pr.y;
+  const i64 lim = (i64)1 << 30;
+  if (pr.accumulate || pr.batch < 1 || pr.c_out < 1 || pr.c_in < 1 || X.nf < 1 || Y.nf < 1 || X.nf > kBlockFilterRows) return false;
+  if (Y.kind != AX_LCORR && Y.kind != AX_LCONV) return false;
+  const i64 plane = X.ng * Y.ng, Q = X.nh * Y.nh;
+  if (plane < 1 || Q < 1 || plane >= (i64)1 << 22 || Q >= (i64)1 << 22) return false;
+  if (pr.batch > 65535 || pr.c_in > 8 * 65535 || pr.c_out * Q >= lim / 2 || Q >= (i64)1 << 20) return false;   // (32-bit byte offsets)
+  if (X.s > 4096 || X.d > 4096 || X.u > 4096 || X.p > 4096 || X.p < -lim || Y.s > 64 || Y.d > 4096 || Y.u > 64 || Y.p > lim || Y.p < -lim)
+    return false;
+  pl.f16 = f16;
+  pl.batch = (int)pr.batch; pl.M = (int)pr.c_out; pl.CG = (int)((pr.c_in + 7) / 8);
+  pl.nox = (int)X.nh; pl.noy = (int)Y.nh; pl.Q = (int)Q;
+  pl.ngx = (int)X.ng; pl.ngy = (int)Y.ng; pl.plane = (int)plane;
+  pl.h_n = pr.h_n; pl.h_m = pr.h_m; pl.f_m = pr.f_m; pl.f_c = pr.f_c;
+  pl.relu = pr.relu; pl.half_out = pr.out_half;
+  // filter columns with a tap inside the signal for some output column (the rest meet padding only)
+  i64 fy_lo = 0, fy_hi = Y.nf - 1;
+  if (Y.u == 1) {
+    const i64 span = Y.s * (Y.nh - 1);
+    const i64 lo = Y.kind == AX_LCORR ? -floor_div(-(Y.p - span), Y.d) : -floor_div(-(Y.p - (Y.ng - 1)), Y.d);
+    const i64 hi = Y.kind == AX_LCORR ? floor_div(Y.ng - 1 + Y.p, Y.d) : floor_div(Y.p + span, Y.d);
+    if (std::max<i64>(lo, 0) <= std::min<i64>(hi, Y.nf - 1)) { fy_lo = std::max<i64>(lo, 0); fy_hi = std::min<i64>(hi, Y.nf - 1); }
+  }
+  pl.nfx = (int)X.nf; pl.nfy = (int)(fy_hi - fy_lo + 1);
+  pl.f_pitch = (int)Y.nf; pl.f_off = (int)fy_lo;
+  if (pl.nfy > 64) return false;
+  const i64 py = Y.p - Y.d * fy_lo;
+  pl.ay = (int)Y.s; pl.by = Y.kind == AX_LCORR ? (int)Y.d : -(int)Y.d; pl.cy = Y.kind == AX_LCORR ? -(int)py : (int)py;
+  pl.uy = (int)Y.u;
+  const i64 by_ext = (i64)pl.by * (pl.nfy - 1);
+  pl.by_min = (int)std::min<i64>(by_ext, 0);
+  const i64 RS = (i64)pl.ay * (pl.noy - 1) + (by_ext < 0 ? -by_ext : by_ext) + 1;
+  if (RS > 4096) return false;
+  pl.RS = (int)RS;
+  const bool mellin = X.kind == AX_MCORR || X.kind == AX_MCONV;
+  pl.kind_x = X.kind; pl.sx = (int)X.s; pl.dx = (int)X.d; pl.px = (int)X.p; pl.ux = (int)X.u;
+  pl.mg_p1 = X.p <= 0 ? 0xFFFFFFFFu : (unsigned)(0x100000000ull / (unsigned)(X.p + 1));
+  pl.ax = pl.bx = pl.cx = pl.bx_min = pl.bx_span = 0;
+  if (mellin) {
+    const i64 hmax = X.nh + X.s, fmax = X.nf + X.d;
+    if (hmax * fmax >= lim || (X.p + 1) * hmax >= lim || (X.ng + X.u) * std::max(fmax, X.p + 1) >= lim) return false;
+    plan_classes(X, pl);
+  } else {
+    pl.ax = (int)X.s; pl.bx = X.kind == AX_LCORR ? (int)X.d : -(int)X.d; pl.cx = X.kind == AX_LCORR ? -(int)X.p : (int)X.p;
+    const i64 ext = (i64)pl.bx * (pl.nfx - 1);
+    pl.bx_min = (int)std::min<i64>(ext, 0);
+    pl.bx_span = (int)(ext < 0 ? -ext : ext);
+    pl.n_classes = 1; pl.cls_stride = 1; pl.cls[0] = BlockClass{0, 0, 0};
+  }
+  const int parts = f16 ? 1 : 3;
+  pl.mt = pr.c_out > 32 ? 2 : 1;
+  pl.wm = 1;
+
+  // A tile shape's stage: the channel groups and filter rows that fit twice into the LDS that a
+  // workgroup may take, two workgroups to a CU
+  auto shape = [&](int nt, int wm, int wk) {
+    const int P = (kWaves / wk / wm) * nt * 32, M_T = wm * pl.mt * 32;
+    const i64 RT = std::min<i64>(pl.nox, (P - 1 + pl.noy - 1) / pl.noy + 1);
+    const i64 vrows = mellin ? RT : (i64)pl.ax * (RT - 1) + pl.bx_span + 1;
+    const i64 tab = ((mellin ? vrows * pl.nfx : vrows) * pl.RS + 64 + 64 + 3) & ~(i64)3;
+    auto pad = [&](i64 halves) { return std::max<i64>((halves + 2 * wk - 1) / (2 * wk) * (2 * wk), 4 * wk); };
+    int best_f = 0, best_g = 0;
+    double best = 0;
+    for (int F = mellin ? pl.nfx : 1; F >= 1; --F) {
+      const int rows = mellin ? F : pl.nfx;
+      const i64 units = vrows * (mellin ? F : 1) * pl.RS;
+      const i64 gb = (units * parts + 63) / 64 * 1024;
+      for (int G = std::min(pl.CG, 8); G >= 1; --G) {
+        if (pl.CG % G) continue;
+        const i64 ents = (mellin ? (pl.nfx + F - 1) / F : 1) * pad((i64)rows * pl.nfy * G) + 8 * wk;
+        const i64 bytes = 2 * gb * G + 4 * tab + 16 * ents + M_T * 4;
+        if (bytes > 79 * 1024) continue;
+        // what a stage's steps fill of their whole pairs, against what a stage costs on top (its barrier and first reads)
+        const i64 halves = (i64)rows * pl.nfy * G;
+        const double rate = (double)halves / (double)(pad(halves) + 2 * wk);
+        if (rate > best) { best = rate; best_f = F; best_g = G; }
+      }
+    }
+    if (!best_f) return false;
+    const i64 units = vrows * (mellin ? best_f : 1) * pl.RS;
+    pl.F = mellin ? best_f : pl.nfx;
+    pl.G = best_g;
+    pl.tab_units = (int)tab;
+    pl.ents = (int)((mellin ? (pl.nfx + pl.F - 1) / pl.F : 1) * pad((i64)pl.F * pl.nfy * best_g) + 8 * wk);
+    pl.group_bytes = (int)((units * parts + 63) / 64 * 1024);
+    pl.buf_bytes = pl.group_bytes * best_g;
+    pl.nt = nt; pl.wm = wm; pl.wk = wk;
+    pl.tiles_per_image = (pl.Q + P - 1) / P;
+    if ((i64)pl.tiles_per_image * pl.batch >= lim) return false;
+    pl.total_tiles = pl.tiles_per_image * pl.batch;
+    size_t bytes = 2 * (size_t)pl.buf_bytes;
+    if (wk > 1) bytes = std::max(bytes, (size_t)wk * pl.mt * nt * 4096);
+    if (wk > 1) pl.buf_bytes = (int)(bytes / 2);
+    bytes += 4 * (size_t)tab + 16 * (size_t)pl.ents + M_T * 4;
+    pl.lds_bytes = bytes;
+    pl.m_tiles = (int)((pr.c_out + M_T - 1) / M_T);
+    return bytes <= 79 * 1024;
+  };
+  const i64 slots = 512;
+  auto tiles = [&](int P, int M_T) { return pl.batch * ((Q + P - 1) / P) * ((pr.c_out + M_T - 1) / M_T); };
+  const int m1 = 32 * pl.mt;
+  bool ok = false;
+  if (f16 && pr.c_out > 96 && tiles(256, 128) >= slots) ok = shape(4, 2, 1);
+  if (!ok && f16 && tiles(512, m1) >= slots) ok = shape(4, 1, 1);
+  if (!ok && tiles(256, m1) >= slots) ok = shape(2, 1, 1);
+  if (!ok && tiles(128, m1) >= slots / 2) ok = shape(1, 1, 1);
+  if (!ok) ok = shape(2, 1, 4) || shape(1, 1, 4);
+  if (!ok) ok = shape(2, 1, 1) || shape(1, 1, 1);
+  if (!ok) return false;
+  pl.filter_bytes = (size_t)pl.m_tiles * pl.wm * pl.mt * ((size_t)pl.CG * pl.nfx * pl.nfy + 1) * parts * 512;
+  if (pl.filter_bytes >= (size_t)lim) return false;
+  pl.grid_x = pl.wk > 1 ? pl.total_tiles : (int)std::min<i64>(pl.total_tiles, std::max<i64>(1, slots / pl.m_tiles));
+  return true;
+}
+
+hipError_t launch_block_gemm(const BlockPlan &pl, const void *signal, const void *frag, const void *bias, void *out,
+                             hipStream_t stream) {
+#define MELLIN_BLOCK_CASE(MT_, NT_, WM_, WK_)                                                                \
+  if (pl.mt == MT_ && pl.nt == NT_ && pl.wm == WM_ && pl.wk == WK_) {                                        \
+    if (pl.f16) return launch_instance<MT_, NT_, WM_, WK_, true, true>(pl, signal, frag, bias, out, stream); \
+    return launch_instance<MT_, NT_, WM_, WK_, false, false>(pl, signal, frag, bias, out, stream);           \
+  }
+  if (pl.f16 && pl.nt == 4) {
+    if (pl.wm == 2) return launch_instance<2, 4, 2, 1, true, true>(pl, signal, frag, bias, out, stream);
+    if (pl.mt == 2) return launch_instance<2, 4, 1, 1, true, true>(pl, signal, frag, bias, out, stream);
+    return launch_instance<1, 4, 1, 1, true, true>(pl, signal, frag, bias, out, stream);
+  }
+  MELLIN_BLOCK_CASE(2, 2, 1, 1)
+  MELLIN_BLOCK_CASE(2, 1, 1, 1)
+  MELLIN_BLOCK_CASE(1, 2, 1, 1)
+  MELLIN_BLOCK_CASE(1, 1, 1, 1)
+  MELLIN_BLOCK_CASE(2, 2, 1, 4)
+  MELLIN_BLOCK_CASE(2, 1, 1, 4)
+  MELLIN_BLOCK_CASE(1, 2, 1, 4)
+  MELLIN_BLOCK_CASE(1, 1, 1, 4)
+#undef MELLIN_BLOCK_CASE
+  return hipErrorInvalidValue;
+}
+
+}  // namespace mellin

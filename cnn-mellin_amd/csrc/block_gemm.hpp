@@ -1,0 +1,95 @@
+// Channel-blocked forms of a layer's passes, for layers with many channels: operands are first
+// laid out with eight channels of a position side by side (16 bytes: what a lane feeds one matrix
+// instruction), cut into their bf16 parts once per element, and the matrix kernels then read
+// ready-made operands (block_pack.hip, block_gemm.hip, block_wgrad.hip).
+#pragma once
+
+#include "mellin_common.hpp"
+
+namespace mellin {
+
+constexpr int kBlockClasses = 32;                  // residue classes of a Mellin axis a plan can hold
+constexpr int kBlockFilterRows = 16;
+
+// A blocked tensor of `channels` channels and `plane` positions per image:
+//   [image][group of eight channels][plane + 1][part][8 channels]
+// with three bf16 parts (fp32 tensors) or one f16 part (half tensors); channels past the last are
+// zeros, and so is the unit past the plane's last position (the source of padding).
+inline size_t blocked_bytes(i64 batch, i64 channels, i64 plane, bool f16) {
+  return (size_t)batch * (size_t)((channels + 7) / 8) * (size_t)(plane + 1) * (f16 ? 16 : 48);
+}
+
+// A class of output rows: every `stride`-th row from `first` on, with the filter rows of `mask`.
+struct BlockClass { int first, start; unsigned mask; };     // start: the class's first row in the order of the classes
+
+struct BlockPlan {
+  int f16;
+  int batch, M, CG;                // images, output channels, groups of eight contracted channels
+  int nfx, nfy;                    // filter rows; filter columns (those that have taps)
+  int nox, noy, Q;                 // output extent
+  int ngx, ngy, plane;             // signal extent
+  // x axis.  Mellin kinds: tap_index(); linear kinds: (ax ox + bx fx + cx) / ux
+  int kind_x, sx, dx, px, ux, ax, bx, cx, bx_min, bx_span;
+  unsigned mg_p1;                  // floor(2^32 / (px + 1)) (see udiv)
+  int ay, by, cy, uy, by_min;      // y axis: (ay oy + by fy + cy) / uy
+  int RS;                          // units per virtual row
+  int F, G;                        // filter rows and channel groups of a stage
+  int tab_units;                   // positions of a tile's source table
+  int ents;                        // operand offsets of a tile's steps
+  int group_bytes, buf_bytes;      // LDS of one group of a stage, of a stage
+  int tiles_per_image, total_tiles;
+  i64 h_n, h_m;
+  int relu, half_out;
+  int n_classes, cls_stride;
+  BlockClass cls[kBlockClasses];
+  // filter (block_pack.hip)
+  i64 f_m, f_c;
+  int f_pitch, f_off;
+  // launch
+  int mt, nt, wm, wk, m_tiles, grid_x;
+  size_t lds_bytes, filter_bytes;
+};
+
+// False: the kernel does not apply.
+bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl);
+// The filter of `pl` as fragments: f (fp32 or half storage) -> filter_bytes at `frag`.
+hipError_t launch_pack_filter(const BlockPlan &pl, int channels, const void *f, void *frag, hipStream_t stream);
+// out = [relu](bias + sum) from a blocked signal and packed filter; bias (fp32 / half, or null).
+hipError_t launch_block_gemm(const BlockPlan &pl, const void *signal, const void *frag, const void *bias, void *out,
+                             hipStream_t stream);
+
+// The rows of one filter row in the weight gradient: output rows ox0 + i step and input rows gx0 + i gstep for
+// i < count; its share of the launch: `slices` workgroups from slice0 on.
+struct BlockWgradRow { int ox0, step, gx0, gstep, count, slice0, slices; };
+
+struct BlockWgradPlan {
+  int f16;
+  int batch, M, C, MG, CG;         // images, channels of grad_out and input, their groups of eight
+  int q_out, plane, noy, ngy;
+  int nfx, nfy, f_pitch, f_off;    // filter columns f_off .. f_off + nfy - 1 have taps
+  int ay, by, cy, uy, by_span;     // y axis: (ay oy + by fy + cy) / uy
+  int nw, mt, nt, wm, ctb;         // wavefronts, tiles of each, how many lie along the output channels, 32-channel tiles of the input in a block
+  int m_blocks, c_blocks, mgt, cgt;
+  int VP, zero_unit;               // units of a channel group's input in a stage, the first that is always zero
+  int slices;
+  BlockWgradRow row[kBlockFilterRows];
+  size_t lds_bytes, ws_bytes;
+};
+
+// `fwd`: the forward pass's problem (x axis Mellin or linear correlation, y linear correlation).
+bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl);
+// grad_out, input: blocked; grad_weight: fp32 / half.
+hipError_t launch_block_wgrad(const BlockWgradPlan &pl, const void *grad_out, const void *input, void *grad_weight,
+                              float *workspace, hipStream_t stream);
+
+// x (batch, channels, plane), fp32 or half -> blocked.  With `relu_out` (the layer's output) values
+// whose output is not positive are zeros (the backward of the fused ReLU).  With `partial`:
+// per-channel sums of what was written, block by block, for launch_bias_reduce
+// (pack_partial_count(): floats).
+hipError_t launch_pack_signal(const void *x, const void *relu_out, bool f16, i64 batch, i64 channels, i64 plane,
+                              void *blocked, float *partial, hipStream_t stream);
+size_t pack_partial_count(i64 batch, i64 channels, i64 plane);
+hipError_t launch_bias_reduce(const float *partial, i64 per_channel, i64 channels, void *grad_bias, bool f16,
+                              hipStream_t stream);
+
+}  // namespace mellin

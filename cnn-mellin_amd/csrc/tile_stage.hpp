@@ -65,6 +65,15 @@ __device__ __forceinline__ void wait_all_memory() {
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 }
 
+// All but the newest N vector-memory instructions of this wavefront are complete and its LDS accesses are
+// done; then the workgroup's barrier.  One statement, so that no access moves between the two.
+template <int N>
+__device__ __forceinline__ void wait_and_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+// LDS accesses only.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // x / d for 0 <= x < 2^31 and d >= 1 with m = floor(2^32 / d) (0xFFFFFFFF for d = 1):
 // the product's high word is the quotient or one less.  On wave-uniform values this
 // is a handful of scalar instructions; a plain integer division goes through the
@@ -596,6 +605,29 @@ __device__ __forceinline__ void multiply_taps_f16(floatx16 (&acc)[MT][NT], const
     multiply(b);
   }
   if (s < steps) multiply(a);
+}
+
+// acc += A * B over sixteen values of k, operands ready-made (channel-blocked kernels); three-part operands: the six largest of the nine cross products, small ones
+// first, each over all the wavefront's tiles (consecutive instructions do not wait for each other's sums)
+template <int MT, int NT, int PARTS>
+__device__ __forceinline__ void block_multiply(floatx16 (&acc)[MT][NT], const uintx4 (&a)[MT][PARTS], const uintx4 (&b)[NT][PARTS]) {
+  if constexpr (PARTS == 1) {
+#pragma unroll
+    for (int k = 0; k < MT; ++k)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[k][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, a[k][0]), __builtin_bit_cast(halfx8, b[t][0]),
+                                                           acc[k][t], 0, 0, 0);
+  } else {
+    constexpr int ta[6] = {2, 0, 1, 1, 0, 0}, tb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+      for (int k = 0; k < MT; ++k)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          acc[k][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a[k][ta[i]]), as_bf16x8(b[t][tb[i]]), acc[k][t], 0, 0, 0);
+  }
 }
 
 }  // namespace mellin

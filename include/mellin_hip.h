@@ -440,7 +440,8 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
  * (row, filter row) pair without a tap), "mfma-f16", "mfma-f16-classes" (the
  * classes of a half-precision layer sharing one launch) and
  * "mfma-f16-class-launches" (a launch each),
- * "mfma-f16-fused", "mfma-f16+fold" and "mfma-f16-filter-rows+fold"
+ * "mfma-f16-fused", "mfma-f16+fold", "mfma-f16-filter-rows+fold" and, for fp32 layers
+ * of section 5 through channel-blocked operands, "mfma-blocks"
  * (half-precision tensors on the f16 matrix cores), "mfma-narrow" (forward pass
  * of a linear x linear layer with few input channels, bf16 matrix cores) and
  * "lds-gather" (vector-ALU forward kernel, only under mellin_set_variant). */
@@ -494,7 +495,8 @@ int mellin_last_math(void);
  * "lds-gather": automatic choice, but fp32 forward passes with at most eight input
  * channels and unit stride and dilation along y take the vector-ALU kernel that gathers
  * its taps from LDS (reported as "lds-gather", MELLIN_MATH_FP32: the non-matrix form the
- * matrix kernels are measured against), "no-gather": never; "no-narrow": automatic choice,
+ * matrix kernels are measured against), "no-gather": never; "no-blocks":
+ * the layers of section 5 never through channel-blocked operands; "no-narrow": automatic choice,
  * but linear x linear forward passes with few input channels go through the tiled kernel
  * instead of their own ("mfma-narrow": both axes correlations without padding or
  * up-sampling, unit stride and dilation along y, an even number of filter columns,

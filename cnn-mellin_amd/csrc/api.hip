@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <memory>
 #include <mutex>
 #include <numeric>
 
@@ -1555,17 +1556,61 @@ static bool blocks_allowed(bool half) {
   return g_forced == 0 && !g_no_blocks && !g_widen && !g_no_classes && !g_all_classes && !g_split_classes && !g_whole_classes &&
          !g_no_yfold && !g_gather && !g_no_narrow && (half || g_math != MATH_FP32);
 }
+// Plans of the layer entry points, kept per thread: a layer asks for the same ones with every step (its workspace, then
+// the launch), and choosing among tile shapes takes some microseconds.  A place for each of the last sizes; the sizes
+// decide the plan, so nothing has to be thrown away.
+struct LayerPlans {
+  int known[3];                                        // 0 not yet, 1 applies, -1 does not
+  BlockPlan forward, input;
+  BlockWgradPlan weight;
+};
+static LayerPlans &layer_plans(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
+  constexpr int kPlaces = 64;
+  struct Place { int64_t key[18]; LayerPlans plans; };
+  static thread_local std::unique_ptr<Place[]> places;
+  if (!places) places.reset(new Place[kPlaces]());
+  const int64_t key[18] = {kind_x * 2 + half + 1, CORR2D_ARGS};
+  uint64_t h = 0;
+  for (int64_t k : key) h = (h ^ (uint64_t)k) * 0x9E3779B97F4A7C15ull, h ^= h >> 29;
+  Place &p = places[h % kPlaces];
+  if (memcmp(p.key, key, sizeof key) != 0) {
+    memcpy(p.key, key, sizeof key);
+    p.plans.known[0] = p.plans.known[1] = p.plans.known[2] = 0;
+  }
+  return p.plans;
+}
+static bool blocks_apply(bool half, MELLIN_CORR2D_DIMS) {
+  return blocks_allowed(half) && c_in >= 16 && batch * c_out * nhx * nhy != 0;
+}
 static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp) {
-  if (!blocks_allowed(half) || c_in < 16 || batch * c_out * nhx * nhy == 0) return false;
-  SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
-  pr.out_half = half;
-  return make_block_plan(pr, half, bp);
+  if (!blocks_apply(half, CORR2D_ARGS)) return false;
+  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
+  if (!lp.known[0]) {
+    SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
+    pr.out_half = half;
+    lp.known[0] = make_block_plan(pr, half, lp.forward) ? 1 : -1;
+  }
+  if (lp.known[0] > 0) bp = lp.forward;
+  return lp.known[0] > 0;
 }
 static bool plan_block_input(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp) {
-  if (!blocks_allowed(half) || c_in < 16 || batch * c_out * nhx * nhy == 0) return false;
-  SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
-  pr.out_half = half;
-  return make_block_plan(pr, half, bp);
+  if (!blocks_apply(half, CORR2D_ARGS)) return false;
+  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
+  if (!lp.known[1]) {
+    SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
+    pr.out_half = half;
+    lp.known[1] = make_block_plan(pr, half, lp.input) ? 1 : -1;
+  }
+  if (lp.known[1] > 0) bp = lp.input;
+  return lp.known[1] > 0;
+}
+static bool plan_block_weight(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockWgradPlan &wp) {
+  if (!blocks_apply(half, CORR2D_ARGS)) return false;
+  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
+  if (!lp.known[2])
+    lp.known[2] = make_block_wgrad_plan(forward_problem(kind_x, CORR2D_ARGS), half, lp.weight) && lp.weight.ws_bytes <= kMaxWorkspaceBytes ? 1 : -1;
+  if (lp.known[2] > 0) wp = lp.weight;
+  return lp.known[2] > 0;
 }
 
 size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
@@ -1573,7 +1618,7 @@ size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_
   if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
   BlockPlan bp;
   if (plan_block_forward(kind_x, elem_bytes == 2, CORR2D_ARGS, bp))
-    return blocked_region(batch, c_in, ngx * ngy, elem_bytes == 2) + bp.filter_bytes;
+    return blocked_region(batch, c_in, ngx * ngy, elem_bytes == 2) + align256(bp.filter_bytes) + bp.slice_bytes;
   if (elem_bytes == 2) return mellin_corr2d_forward_f16_workspace(kind_x, CORR2D_ARGS);
   return mellin_corr2d_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS);
 }
@@ -1587,7 +1632,8 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
   const bool half = elem_bytes == 2;
   BlockPlan bp;
   if (plan_block_forward(kind_x, half, CORR2D_ARGS, bp)) {
-    const size_t signal = blocked_region(batch, c_in, ngx * ngy, half), need = signal + bp.filter_bytes;
+    const size_t signal = blocked_region(batch, c_in, ngx * ngy, half), filter = align256(bp.filter_bytes);
+    const size_t need = signal + filter + bp.slice_bytes;
     if (!workspace || workspace_bytes < need)
       return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, need, workspace_bytes);
     if (!input || !weight || !out) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
@@ -1598,9 +1644,15 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
     g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
     hipStream_t st = (hipStream_t)stream;
     char *ws = (char *)workspace;
-    hipError_t e = launch_pack_filter(bp, (int)c_in, weight, ws + signal, st);
-    if (e == hipSuccess) e = launch_pack_signal(input, nullptr, half, batch, c_in, ngx * ngy, ws, nullptr, st);
-    if (e == hipSuccess) e = launch_block_gemm(bp, ws, ws + signal, bias, out, st);
+    float *sums = (float *)(ws + signal + filter);
+    const PackSignal x = {input, nullptr, ws, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
+    hipError_t e = launch_block_pack(half, &x, nullptr, &bp, (int)c_in, weight, ws + signal, st);
+    if (e == hipSuccess) e = launch_block_gemm(bp, ws, ws + signal, bias, out, sums, st);
+    if (e == hipSuccess && bp.rest > 0) {
+      BlockFinish fin = {};
+      fin.slices = &bp; fin.frag = ws + signal; fin.slice_sums = sums; fin.out = out;
+      e = launch_block_finish(half, fin, st);
+    }
     return check_hip(e, __func__);
   }
   if (half)
@@ -1615,14 +1667,10 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
 // section 2, on grad_out as it lies (through a fused ReLU: on a masked copy).
 struct LayerBackward {
   bool input_blocked, weight_blocked, plain;           // plain: some gradient takes the section-2 kernels
-  size_t masked_off, go_off, x_off, frag_off, pass_off, pass_bytes, total;
+  size_t masked_off, go_off, x_off, frag_off, slice_off, bias_off, wgrad_off, pass_off, pass_bytes, total;
   BlockPlan bp;
   BlockWgradPlan wp;
 };
-static bool plan_block_weight(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockWgradPlan &wp) {
-  if (!blocks_allowed(half) || c_in < 16 || batch * c_out * nhx * nhy == 0) return false;
-  return make_block_wgrad_plan(forward_problem(kind_x, CORR2D_ARGS), half, wp) && wp.ws_bytes <= kMaxWorkspaceBytes;
-}
 static void plan_layer_backward(int kind_x, int elem, int want, MELLIN_CORR2D_DIMS, LayerBackward &lb) {
   const bool half = elem == 2;
   const bool wi = want & MELLIN_WANT_INPUT, ww = want & MELLIN_WANT_WEIGHT;
@@ -1636,18 +1684,16 @@ static void plan_layer_backward(int kind_x, int elem, int want, MELLIN_CORR2D_DI
   lb.go_off = take(any ? blocked_bytes(batch, c_out, nhx * nhy, half) : 0);
   lb.x_off = take(lb.weight_blocked ? blocked_bytes(batch, c_in, ngx * ngy, half) : 0);
   lb.frag_off = take(lb.input_blocked ? lb.bp.filter_bytes : 0);
+  lb.slice_off = take(lb.input_blocked ? lb.bp.slice_bytes : 0);
+  lb.bias_off = take(!lb.plain && (want & MELLIN_WANT_BIAS) ? pack_partial_count(batch, c_out, nhx * nhy) * 4 : 0);
+  lb.wgrad_off = take(lb.weight_blocked ? lb.wp.ws_bytes : 0);
   size_t pass = 0;
-  if (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)) {
-    if (lb.plain)                                      // (a ReLU's backward writes the bias gradient, asked for or not)
-      pass = align256(mellin_bias_grad_workspace(batch, c_out, nhx * nhy)) + align256((size_t)c_out * elem);
-    else
-      pass = pack_partial_count(batch, c_out, nhx * nhy) * 4;
-  }
+  if (lb.plain && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)))   // (a ReLU's backward writes the bias gradient, asked for or not)
+    pass = align256(mellin_bias_grad_workspace(batch, c_out, nhx * nhy)) + align256((size_t)c_out * elem);
   if (wi && !lb.input_blocked)
     pass = std::max(pass, half ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS)
                                : mellin_corr2d_backward_input_workspace(kind_x, elem, CORR2D_ARGS));
-  if (lb.weight_blocked) pass = std::max(pass, lb.wp.ws_bytes);
-  else if (ww)
+  if (ww && !lb.weight_blocked)
     pass = std::max(pass, half ? mellin_corr2d_backward_weight_f16_workspace(kind_x, CORR2D_ARGS)
                                : mellin_corr2d_backward_weight_workspace(kind_x, elem, CORR2D_ARGS));
   lb.pass_bytes = pass;
@@ -1689,42 +1735,46 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
     if (rc) return rc;
     if (masked) grad_out = masked;
   }
-  if (lb.input_blocked || lb.weight_blocked) {
-    if (!grad_out || (lb.input_blocked && !weight) || (lb.weight_blocked && !input))
-      return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
-    const bool sums = !lb.plain && (want & MELLIN_WANT_BIAS);
-    e = launch_pack_signal(grad_out, relu && !lb.plain ? out : nullptr, half, batch, c_out, nhx * nhy, ws + lb.go_off,
-                           sums ? (float *)pass : nullptr, st);
-    if (e == hipSuccess && sums)
-      e = launch_bias_reduce((const float *)pass, (i64)pack_partial_count(batch, 1, nhx * nhy), c_out, grad_bias, half, st);
-  }
-  if (lb.input_blocked && e == hipSuccess) {
-    lb.bp.relu = 0;
-    g_variant = half ? "mfma-f16" : "mfma-blocks";
-    g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
-    e = launch_pack_filter(lb.bp, (int)c_out, weight, ws + lb.frag_off, st);
-    if (e == hipSuccess) e = launch_block_gemm(lb.bp, ws + lb.go_off, ws + lb.frag_off, nullptr, grad_input, st);
-  }
-  if (e != hipSuccess) return check_hip(e, __func__);
   if ((want & MELLIN_WANT_INPUT) && !lb.input_blocked) {
     rc = half ? mellin_corr2d_backward_input_f16(kind_x, weight, grad_out, CORR2D_ARGS, grad_input, pass, lb.pass_bytes, stream)
               : mellin_corr2d_backward_input_f32(kind_x, (const float *)weight, (const float *)grad_out, CORR2D_ARGS,
                                                  (float *)grad_input, pass, lb.pass_bytes, stream);
     if (rc) return rc;
   }
-  if (lb.weight_blocked) {
-    g_variant = half ? "mfma-f16" : "mfma-blocks";
-    g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
-    e = launch_pack_signal(input, nullptr, half, batch, c_in, ngx * ngy, ws + lb.x_off, nullptr, st);
-    if (e == hipSuccess) e = launch_block_wgrad(lb.wp, ws + lb.go_off, ws + lb.x_off, grad_weight, (float *)pass, st);
-    if (e != hipSuccess) return check_hip(e, __func__);
-  } else if (want & MELLIN_WANT_WEIGHT) {
+  if ((want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked) {
     rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, grad_weight, pass, lb.pass_bytes, stream)
               : mellin_corr2d_backward_weight_f32(kind_x, (const float *)input, (const float *)grad_out, CORR2D_ARGS,
                                                   (float *)grad_weight, pass, lb.pass_bytes, stream);
     if (rc) return rc;
   }
-  return MELLIN_OK;
+  if (!lb.input_blocked && !lb.weight_blocked) return MELLIN_OK;
+  if (!grad_out || (lb.input_blocked && !weight) || (lb.weight_blocked && !input))
+    return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  g_variant = half ? "mfma-f16" : "mfma-blocks";
+  g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
+  const bool sums = !lb.plain && (want & MELLIN_WANT_BIAS);
+  const PackSignal go = {grad_out, relu && !lb.plain ? out : nullptr, ws + lb.go_off, sums ? (float *)(ws + lb.bias_off) : nullptr,
+                         (int)batch, (int)c_out, (int)(nhx * nhy)};
+  const PackSignal x = {input, nullptr, ws + lb.x_off, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
+  e = launch_block_pack(half, &go, lb.weight_blocked ? &x : nullptr, lb.input_blocked ? &lb.bp : nullptr, (int)c_out, weight,
+                        ws + lb.frag_off, st);
+  BlockFinish fin = {};
+  if (lb.input_blocked) {
+    lb.bp.relu = 0;
+    fin.slices = &lb.bp; fin.frag = ws + lb.frag_off; fin.slice_sums = (float *)(ws + lb.slice_off); fin.out = grad_input;
+    if (e == hipSuccess)
+      e = launch_block_gemm(lb.bp, ws + lb.go_off, ws + lb.frag_off, nullptr, grad_input, (float *)(ws + lb.slice_off), st);
+  }
+  if (lb.weight_blocked) {
+    fin.weight = &lb.wp; fin.weight_partial = (float *)(ws + lb.wgrad_off); fin.grad_weight = grad_weight;
+    if (e == hipSuccess) e = launch_block_wgrad(lb.wp, ws + lb.go_off, ws + lb.x_off, (float *)(ws + lb.wgrad_off), st);
+  }
+  if (sums) {
+    fin.bias_partial = (const float *)(ws + lb.bias_off); fin.grad_bias = grad_bias;
+    fin.bias_count = (i64)pack_partial_count(batch, 1, nhx * nhy); fin.channels = c_out;
+  }
+  if (e == hipSuccess) e = launch_block_finish(half, fin, st);
+  return check_hip(e, __func__);
 }
 
 }  // extern "C"

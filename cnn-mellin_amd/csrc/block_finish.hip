@@ -1,0 +1,201 @@
+// The sums that end a pass of the channel-blocked kernels (block_gemm.hpp), in one launch: weight
+// gradients from their partial blocks, bias gradients from the packing pass's partial sums, and the
+// output of a pass whose contracted channels were dealt to several workgroups.  Each is a short
+// streaming sum in a fixed order; on small layers a launch of its own (3-5 us each) cost more than
+// the sum, so they share one.
+#include <algorithm>
+
+#include "block_gemm.hpp"
+#include "tile_stage.hpp"
+
+namespace mellin {
+
+namespace {
+
+constexpr int kFinishThreads = 256;
+constexpr int kSliceValues = kFinishThreads * 4;       // values of a tile that a block adds up
+
+struct FinishArgs {
+  BlockWgradPlan w;
+  const float *w_partial;
+  void *gw;
+  unsigned w_blocks, w_zero_blocks;
+  int w_pairs;
+  const float *b_partial;
+  void *gb;
+  i64 b_count;
+  unsigned b_blocks;
+  BlockPlan s;
+  const float *s_sums;
+  const int2 *s_rows;
+  void *out;
+};
+
+// gw[m, c, fx, fy] = the sum of its partial sums in slice order.  A block owns 32 weights that lie side by side in
+// the partial blocks; its eight groups of 32 threads add an eighth of the slices each, and those sums are added in order.
+template <typename T>
+__device__ void finish_weight(const BlockWgradPlan &pl, const float *__restrict__ ws, T *__restrict__ gw, int b, float (*red)[32]) {
+  const int cl = threadIdx.x & 31, grp = threadIdx.x >> 5;
+  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.wm * pl.mt * 32;
+  // block -> (filter row, column tile, channel)
+  const int tiles = pl.ctb * pl.nfy;
+  const int m = b % pl.M;
+  b /= pl.M;
+  const int tile = b % tiles;
+  b /= tiles;
+  const int cb = b % pl.c_blocks, fx = b / pl.c_blocks;
+  const int ct = tile / pl.nfy, fy = tile - ct * pl.nfy, c = (cb * pl.ctb + ct) * 32 + cl;
+  const int mb = m / m_t, ml = m - mb * m_t;
+  const int slices = pl.row[fx].slices, blocks = pl.m_blocks * pl.c_blocks;
+  const i64 stride = (i64)blocks * m_t * cols;
+  const float *p = ws + ((i64)pl.row[fx].slice0 * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols + tile * 32 + cl;
+  const int lo = slices * grp / 8, hi = slices * (grp + 1) / 8;
+  float s = 0.f;
+  int k = lo;
+  for (; k + 4 <= hi; k += 4) {
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = p[(k + i) * stride];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s += v[i];
+  }
+  for (; k < hi; ++k) s += p[k * stride];
+  red[grp][cl] = s;
+  __syncthreads();
+  if (grp == 0 && c < pl.C) {
+    float a = red[0][cl];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) a += red[i][cl];
+    gw[(((i64)m * pl.C + c) * pl.nfx + fx) * pl.f_pitch + pl.f_off + fy] = (T)a;
+  }
+}
+
+// The same for weights that are many and have few slices (few: less than 16; a block per 32 weights would mostly wait):
+// a block owns eight output channels and 32 input channels, a thread all taps of one pair, which lie side by side in gw.
+template <typename T>
+__device__ void finish_weight_pairs(const BlockWgradPlan &pl, const float *__restrict__ ws, T *__restrict__ gw, int b) {
+  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.wm * pl.mt * 32, c_tiles = (pl.C + 31) / 32;
+  const int mt8 = b / c_tiles, ct_all = b - mt8 * c_tiles;
+  const int m = mt8 * 8 + (threadIdx.x >> 5), c = ct_all * 32 + (threadIdx.x & 31);
+  if (m >= pl.M || c >= pl.C) return;
+  const int mb = m / m_t, ml = m - mb * m_t, cb = ct_all / pl.ctb, ct = ct_all - cb * pl.ctb;
+  const int blocks = pl.m_blocks * pl.c_blocks;
+  const i64 stride = (i64)blocks * m_t * cols;
+  T *out = gw + ((i64)m * pl.C + c) * pl.nfx * pl.f_pitch + pl.f_off;
+  for (int fx = 0; fx < pl.nfx; ++fx) {
+    const float *p = ws + ((i64)pl.row[fx].slice0 * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols +
+                     ct * pl.nfy * 32 + (threadIdx.x & 31);
+    const int slices = pl.row[fx].slices;
+    int fy = 0;
+    for (; fy + 4 <= pl.nfy; fy += 4) {
+      float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+      for (int k = 0; k < slices; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += p[k * stride + (fy + i) * 32];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[fx * pl.f_pitch + fy + i] = (T)v[i];
+    }
+    for (; fy < pl.nfy; ++fy) {
+      float v = 0.f;
+      for (int k = 0; k < slices; ++k) v += p[k * stride + fy * 32];
+      out[fx * pl.f_pitch + fy] = (T)v;
+    }
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs a) {
+  __shared__ float red[8][32];
+  const int tid = threadIdx.x;
+  unsigned b = blockIdx.x;
+  if (b < a.w_blocks) {
+    if (a.w_pairs) finish_weight_pairs<T>(a.w, a.w_partial, (T *)a.gw, (int)b);
+    else finish_weight<T>(a.w, a.w_partial, (T *)a.gw, (int)b, red);
+    return;
+  }
+  b -= a.w_blocks;
+  if (b < a.w_zero_blocks) {                           // filter columns that have no tap at all: zeros
+    const i64 i = (i64)b * kFinishThreads + tid;
+    const int fy = (int)(i % a.w.f_pitch);
+    if (i < (i64)a.w.M * a.w.C * a.w.nfx * a.w.f_pitch && (fy < a.w.f_off || fy >= a.w.f_off + a.w.nfy)) ((T *)a.gw)[i] = (T)0;
+    return;
+  }
+  b -= a.w_zero_blocks;
+  if (b < a.b_blocks) {
+    // one channel: thread sums, a shuffle tree per wavefront, the wavefronts in order
+    const float *p = a.b_partial + (i64)b * a.b_count;
+    float s = 0.f;
+    for (i64 i = tid; i < a.b_count; i += kFinishThreads) s += p[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o);
+    if ((tid & 63) == 0) red[0][tid >> 6] = s;
+    __syncthreads();
+    if (tid == 0) ((T *)a.gb)[b] = (T)(red[0][0] + red[0][1] + red[0][2] + red[0][3]);
+    return;
+  }
+  b -= a.b_blocks;
+  // a block: kSliceValues values of a tile, four positions of a channel a thread, the slices in order
+  const BlockPlan &pl = a.s;
+  const int m_t = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32, chunks = m_t * P / kSliceValues;
+  const int tm = (int)b / chunks, at = ((int)b - tm * chunks) * kSliceValues + tid * 4;   // (tile, tile of channels), value in it
+  const int r = tm / pl.m_tiles, c = at / P, p = at - c * P, m = (tm - r * pl.m_tiles) * m_t + c;
+  const int id = pl.whole + r, qt = id / pl.batch, n = id - qt * pl.batch, q0 = qt * P, count = min(P, pl.Q - q0) - p;
+  if (m >= pl.M || count <= 0) return;
+  const i64 slice = (i64)pl.rest * pl.m_tiles * m_t * P;
+  const float *from = a.s_sums + (i64)tm * m_t * P + at;
+  float4 v = *(const float4 *)from;
+#pragma unroll 4
+  for (int k = 1; k < pl.slices; ++k) {
+    const float4 w = *(const float4 *)(from + k * slice);
+    v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w;
+  }
+  if (pl.relu) v = make_float4(fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f));
+  const float o[4] = {v.x, v.y, v.z, v.w};
+  int row = (q0 + p) / pl.noy, oy = q0 + p - row * pl.noy;
+  T *out = (T *)a.out + n * pl.h_n + m * pl.h_m;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i < count) out[(a.s_rows ? a.s_rows[row].x : row) * pl.noy + oy] = (T)o[i];
+    if (++oy == pl.noy) { oy = 0; ++row; }
+  }
+}
+
+}  // namespace
+
+hipError_t launch_block_finish(bool f16, const BlockFinish &job, hipStream_t stream) {
+  FinishArgs a = {};
+  if (job.weight) {
+    a.w = *job.weight;
+    a.w_partial = job.weight_partial;
+    a.gw = job.grad_weight;
+    int most = 0;
+    for (int f = 0; f < a.w.nfx; ++f) most = std::max(most, a.w.row[f].slices);
+    a.w_pairs = most < 16 && (i64)a.w.M * a.w.C >= 1 << 14;
+    a.w_blocks = a.w_pairs ? (unsigned)((a.w.M + 7) / 8 * ((a.w.C + 31) / 32))
+                           : (unsigned)(a.w.nfx * a.w.c_blocks * a.w.ctb * a.w.nfy * a.w.M);
+    if (a.w.nfy != a.w.f_pitch)
+      a.w_zero_blocks = (unsigned)(((i64)a.w.M * a.w.C * a.w.nfx * a.w.f_pitch + kFinishThreads - 1) / kFinishThreads);
+  }
+  if (job.grad_bias) {
+    a.b_partial = job.bias_partial;
+    a.gb = job.grad_bias;
+    a.b_count = job.bias_count;
+    a.b_blocks = (unsigned)job.channels;
+  }
+  i64 s_blocks = 0;
+  if (job.slices && job.slices->rest > 0) {
+    a.s = *job.slices;
+    a.s_sums = job.slice_sums;
+    a.out = job.out;
+    if (a.s.kind_x == AX_MCORR || a.s.kind_x == AX_MCONV) a.s_rows = (const int2 *)((const char *)job.frag + a.s.rows_off);
+    s_blocks = (i64)a.s.rest * a.s.m_tiles * (a.s.wm * a.s.mt * 32 * (kWaves / a.s.wk / a.s.wm * a.s.nt * 32) / kSliceValues);
+  }
+  const i64 blocks = (i64)a.w_blocks + a.w_zero_blocks + a.b_blocks + s_blocks;
+  if (blocks == 0) return hipSuccess;
+  if (f16) hipLaunchKernelGGL(block_finish_kernel<_Float16>, dim3((unsigned)blocks), dim3(kFinishThreads), 0, stream, a);
+  else hipLaunchKernelGGL(block_finish_kernel<float>, dim3((unsigned)blocks), dim3(kFinishThreads), 0, stream, a);
+  return hipGetLastError();
+}
+
+}  // namespace mellin

@@ -32,6 +32,7 @@
 // for the cut (six bf16 products each: 1.39 PF, matrix pipe 57 % busy at 1.9 GHz, near the rate the board's
 // power allows); half, on Mellin rows, 286 -> 183 us.  One utterance (few tiles, WK = 4): 980 -> 330 us for ten layers.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "block_gemm.hpp"
@@ -47,61 +48,90 @@ typedef const __attribute__((address_space(4))) BlockPlan ConstBlockPlan;
 
 struct BlockTile {
   int n, q0, count, row_lo, rows;
-  int vx_min, units;               // linear axes: first coordinate; virtual positions of the whole tile
-  unsigned mask;                   // filter rows with a tap for some row of the tile
+  int c_first, c_end, slot, slice; // its channel groups; in slices: place in the workspace, which slice (whole tiles: -1, 0)
+  int vx_min, vrows, units;        // linear axes: first coordinate; virtual rows and positions of the whole tile
+  unsigned long long filter_rows;  // Mellin axes: the filter rows with a tap for some row of the tile, four bits each
   int nv;                          // how many
 };
 
-__device__ __forceinline__ int nth_bit(unsigned mask, int j) {
-  for (int i = 0; i < j; ++i) mask &= mask - 1;
-  return __builtin_ctz(mask);
-}
+__device__ __forceinline__ int filter_row(const BlockTile &g, int j) { return (int)(g.filter_rows >> (4 * j)) & 15; }
 
-// output row of position `row` in the order of the classes
-__device__ __forceinline__ int class_row(ConstBlockPlan &pl, int row) {
-  int ox = row;
-  for (int k = 0; k < pl.n_classes; ++k)
-    if (row >= pl.cls[k].start) ox = pl.cls[k].first + (row - pl.cls[k].start) * pl.cls_stride;
-  return ox;
-}
-
+// Item `id` of the launch: the images of a position tile lie side by side, so that the position tiles
+// with the most filter rows come first for all images and every workgroup gets its share of them.
+// `rows`: the output rows in the order of their classes, with their filter rows (Mellin axes).
 template <int P>
-__device__ __forceinline__ BlockTile block_tile(ConstBlockPlan &pl, int tile_id, bool mellin_x) {
+__device__ __forceinline__ BlockTile block_tile(ConstBlockPlan &pl, const int2 *__restrict__ rows, int id, bool mellin_x) {
   BlockTile g;
-  g.n = tile_id / pl.tiles_per_image;
-  g.q0 = (tile_id - g.n * pl.tiles_per_image) * P;
+  g.c_first = 0;
+  g.c_end = pl.CG;
+  g.slot = -1;
+  g.slice = 0;
+  if (id >= pl.whole) {
+    const int i = id - pl.whole, r = i / pl.slices, stages = pl.CG / pl.G;
+    g.slice = i - r * pl.slices;
+    g.slot = g.slice * pl.rest + r;
+    g.c_first = g.slice * stages / pl.slices * pl.G;
+    g.c_end = (g.slice + 1) * stages / pl.slices * pl.G;
+    id = pl.whole + r;
+  }
+  const int qt = udiv(id, pl.batch, pl.mg_batch);
+  g.n = id - qt * pl.batch;
+  g.q0 = qt * P;
   g.count = min(P, pl.Q - g.q0);
-  g.row_lo = g.q0 / pl.noy;
-  const int row_hi = (g.q0 + g.count - 1) / pl.noy;
-  g.rows = row_hi - g.row_lo + 1;
+  g.row_lo = udiv(g.q0, pl.noy, pl.mg_noy);
+  g.rows = udiv(g.q0 + g.count - 1, pl.noy, pl.mg_noy) - g.row_lo + 1;
   g.vx_min = pl.ax * g.row_lo + pl.cx + pl.bx_min;
-  g.mask = 0;
+  g.filter_rows = 0;
   if (mellin_x) {
-    for (int k = 0; k < pl.n_classes; ++k) {
-      const int lo = max(g.row_lo, pl.cls[k].start), hi = min(row_hi, (k + 1 < pl.n_classes ? pl.cls[k + 1].start : pl.nox) - 1);
-      if (lo > hi) continue;
-      const int h_lo = pl.cls[k].first + (lo - pl.cls[k].start) * pl.cls_stride + pl.sx;
-      const int h_hi = pl.cls[k].first + (hi - pl.cls[k].start) * pl.cls_stride + pl.sx;
-      for (int f = 0; f < pl.nfx; ++f) {
-        // the tap grows with the row: inside for some row iff the first is not past the end and the last not before 0
-        const int num = pl.kind_x == AX_MCORR ? f + pl.dx : pl.px + 1, den = pl.kind_x == AX_MCORR ? pl.px + 1 : f + pl.dx;
-        if ((pl.cls[k].mask >> f & 1) && h_lo * num <= (pl.ngx - 1 + pl.ux) * den && h_hi * num >= pl.ux * den) g.mask |= 1u << f;
-      }
-    }
-    if (g.mask == 0) g.mask = 1;                     // no tap at all: a stage of zeros
-    g.nv = __builtin_popcount(g.mask);
-    g.units = g.nv * g.rows * pl.RS;
+    int mask = 0;
+    for (int r = (int)threadIdx.x & 63; r < g.rows; r += 64) mask |= rows[g.row_lo + r].y;
+    g.nv = 0;
+    for (int f = 0; f < pl.nfx; ++f)
+      if (__ballot(mask >> f & 1)) g.filter_rows |= (unsigned long long)f << (4 * g.nv++);
+    g.nv = max(g.nv, 1);                             // (no tap at all: a stage of zeros)
+    g.vrows = g.nv * g.rows;
   } else {
     g.nv = pl.nfx;
-    g.units = (pl.ax * (g.rows - 1) + pl.bx_span + 1) * pl.RS;
+    g.vrows = pl.ax * (g.rows - 1) + pl.bx_span + 1;
   }
+  g.units = g.vrows * pl.RS;
   return g;
+}
+
+typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+
+// Value `I` of the four lanes that this lane belongs to; the lanes' values exchanged in pairs.
+template <int I>
+__device__ __forceinline__ int quad_lane(int v) { return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xf, 0xf, true); }
+__device__ __forceinline__ unsigned swap1(unsigned v) { return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true); }
+__device__ __forceinline__ unsigned swap2(unsigned v) { return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true); }
+
+// 4 x 4 transpose over four neighbouring lanes: lane j gets the four lanes' values v[j].
+__device__ __forceinline__ uintx4 transpose_words(const float4 &v, int lane) {
+  const unsigned a = __float_as_uint(v.x), b = __float_as_uint(v.y), c = __float_as_uint(v.z), d = __float_as_uint(v.w);
+  const bool odd = lane & 1, upper = lane & 2;
+  const unsigned a1 = swap1(a), b1 = swap1(b), c1 = swap1(c), d1 = swap1(d);     // (by every lane, so not in the selections)
+  const unsigned n0 = odd ? b1 : a, n1 = odd ? b : a1, n2 = odd ? d1 : c, n3 = odd ? d : c1;
+  const unsigned m0 = swap2(n0), m1 = swap2(n1), m2 = swap2(n2), m3 = swap2(n3);
+  return uintx4{upper ? m2 : n0, upper ? m3 : n1, upper ? n2 : m0, upper ? n3 : m1};
+}
+// the same of values rounded to half
+__device__ __forceinline__ uintx2 transpose_half(const float4 &v, int lane) {
+  auto pair = [](float lo, float hi) {
+    return (unsigned)__builtin_bit_cast(unsigned short, (_Float16)lo) | ((unsigned)__builtin_bit_cast(unsigned short, (_Float16)hi) << 16);
+  };
+  const unsigned ab = pair(v.x, v.y), cd = pair(v.z, v.w);
+  const bool odd = lane & 1, upper = lane & 2;
+  const unsigned ab2 = swap2(ab), cd2 = swap2(cd);
+  const unsigned n0 = upper ? cd2 : ab, n1 = upper ? cd : ab2;                   // two channels at positions 0/1 and 2/3
+  const unsigned sel = odd ? 0x03020706u : 0x05040100u;                          // high halves (other, own) or low halves (own, other)
+  return uintx2{__builtin_amdgcn_perm(swap1(n0), n0, sel), __builtin_amdgcn_perm(swap1(n1), n1, sel)};
 }
 
 template <int MT, int NT, int WM, int WK, bool F16, bool HOUT>
 __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_arg, const char *__restrict__ X,
                                                                  const char *__restrict__ AF, const void *__restrict__ bias,
-                                                                 void *__restrict__ Hv) {
+                                                                 void *__restrict__ Hv, float *__restrict__ sums) {
   constexpr int PARTS = F16 ? 1 : 3, UB = 16 * PARTS;
   constexpr int WN = kWaves / WK / WM, P = WN * NT * 32, M_T = WM * MT * 32;
   constexpr int kALoads = 2 * MT * PARTS;              // fragment loads of two steps
@@ -112,6 +142,8 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   float *Bs = (float *)(bufs + 2 * pl.buf_bytes);                          // [M_T]
   int *tab = (int *)(Bs + M_T);                                            // [tab_units] source byte offset in a group's plane
   int2 *ents = (int2 *)(tab + pl.tab_units);                               // [2][ents] (LDS offset, fragment offset) of a step's half
+  int *row_src = (int *)(ents + 2 * pl.ents);                              // Mellin axes: [filter row of the tile][row] first source of the row
+  const int2 *rows = (const int2 *)(AF + pl.rows_off);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
@@ -124,7 +156,8 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   const char *AFm = AF + (i64)(m_tile * WM + wm) * MT * af_tile, *AFm1 = AFm + af_tile;
   const i64 plane_bytes = (i64)(pl.plane + 1) * UB;
   const unsigned lds0 = lds_address((const float *)blk_lds);
-  const int my_tiles = (pl.total_tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int items = pl.whole + pl.rest * pl.slices;
+  const int my_tiles = (items - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
 
   if (tid < M_T) {
     const int m = m_tile * M_T + tid;
@@ -137,98 +170,104 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   constexpr int kWrap = 4 * WK;                        // halves of two steps of every wavefront that shares a tile's steps
   auto stage_halves = [](int n) { return max((n + 2 * WK - 1) / (2 * WK) * (2 * WK), kWrap); };
   auto build_tile = [&](const BlockTile &g, int parity, int2 *before) {
-    const FastDiv by_RS(pl.RS), by_rows(g.rows);
-    const int padded = min(pl.tab_units, g.units + 64);
-    for (int v = tid; v < padded; v += kThreads) {
-      int src = pl.plane;
-      if (v < g.units) {
-        int vr, col;
-        by_RS.divmod(v, vr, col);
-        const int vy = pl.cy + pl.by_min + col;
-        int gy = -1, gx = -1;
-        if (vy >= 0) {
-          if (pl.uy == 1) gy = vy;
-          else { const int q = vy / pl.uy; if (q * pl.uy == vy) gy = q; }
-          if (gy >= pl.ngy) gy = -1;
-        }
-        if (mellin_x) {
-          int j, r;
-          by_rows.divmod(vr, j, r);
-          gx = mellin_tap32(pl.kind_x, class_row(pl, g.row_lo + r), nth_bit(g.mask, j), pl.ngx, pl.sx, pl.dx, pl.px + 1, pl.ux,
-                            pl.mg_p1);
-        } else {
-          const int vx = g.vx_min + vr;
-          if (vx >= 0) {
-            if (pl.ux == 1) gx = vx;
-            else { const int q = vx / pl.ux; if (q * pl.ux == vx) gx = q; }
-            if (gx >= pl.ngx) gx = -1;
-          }
-        }
-        if (gx >= 0 && gy >= 0) src = gx * pl.ngy + gy;
+    // (fields of the plan, read together: one wait for the scalar loads instead of one each)
+    int RS = pl.RS, cy = pl.cy + pl.by_min, uy = pl.uy, ux = pl.ux, ngx = pl.ngx, ngy = pl.ngy, tab_units = pl.tab_units, F = pl.F,
+        G = pl.G, nfx = pl.nfx, nfy = pl.nfy, none = pl.plane, group_bytes = pl.group_bytes, n_before = pl.ents;
+    asm volatile("" : "+s"(RS), "+s"(cy), "+s"(uy), "+s"(ux), "+s"(ngx), "+s"(ngy), "+s"(tab_units), "+s"(F), "+s"(G), "+s"(nfx),
+                 "+s"(nfy), "+s"(none), "+s"(group_bytes), "+s"(n_before));
+    int kx = pl.kind_x, sx = pl.sx, dx = pl.dx, px = pl.px, bx = pl.bx, bx_min = pl.bx_min, by = pl.by, by_min = pl.by_min;
+    unsigned mg_p1 = pl.mg_p1, mg_full = pl.mg_full, mg_per_row = pl.mg_per_row, mg_G = pl.mg_G;
+    asm volatile("" : "+s"(kx), "+s"(sx), "+s"(dx), "+s"(px), "+s"(bx), "+s"(bx_min), "+s"(by), "+s"(by_min), "+s"(mg_p1),
+                 "+s"(mg_full), "+s"(mg_per_row), "+s"(mg_G));
+    if (mellin_x) {
+      const FastDiv by_rows(g.rows);
+      for (int t = tid; t < g.nv * g.rows; t += kThreads) {
+        int j, r;
+        by_rows.divmod(t, j, r);
+        const int gx = mellin_tap32(kx, rows[g.row_lo + r].x, filter_row(g, j), ngx, sx, dx, px + 1, ux, mg_p1);
+        row_src[t] = gx >= 0 ? gx * ngy : -1;
       }
-      tab[v] = src * UB;
+      lds_barrier();
     }
+    // wavefronts take 64 / RS virtual rows (or a 64th piece of one) at a time: a lane keeps its column
+    const int per = RS <= 64 ? 64 / RS : 1, vrows = g.vrows;
+    const int lr = RS <= 64 ? lane / RS : 0;
+    for (int col = lane - lr * RS; col < RS; col += RS <= 64 ? RS : 64) {
+      const int vy = cy + col;
+      int gy = -1;
+      if (vy >= 0) {
+        if (uy == 1) gy = vy;
+        else { const int q = vy / uy; if (q * uy == vy) gy = q; }
+        if (gy >= ngy) gy = -1;
+      }
+      if (lr < per)
+        for (int vr = wave * per + lr; vr < vrows; vr += kWaves * per) {
+          int first = -1;
+          if (mellin_x) {
+            first = row_src[vr];
+          } else {
+            const int vx = g.vx_min + vr;
+            int gx = -1;
+            if (vx >= 0) {
+              if (ux == 1) gx = vx;
+              else { const int q = vx / ux; if (q * ux == vx) gx = q; }
+            }
+            if (gx >= 0 && gx < ngx) first = gx * ngy;
+          }
+          tab[vr * RS + col] = (first >= 0 && gy >= 0 ? first + gy : none) * UB;
+        }
+    }
+    if (tid < 64 && g.units + tid < tab_units) tab[g.units + tid] = none * UB;
     // Entries of the tile's stages one behind the other (a last odd half is paired with the fragment of zeros), then
     // the first two steps again: a stage reads on into the one that follows it.  `before`: the first two steps of
     // this tile also go behind the entries of the tile before it, whose last stage is running.
-    int2 *out = ents + parity * pl.ents;
-    const int per_row = pl.nfy * pl.G, full = stage_halves(pl.F * per_row), subsets = (g.nv + pl.F - 1) / pl.F;
-    const int tail = stage_halves((g.nv - (subsets - 1) * pl.F) * per_row), n_ents = (subsets - 1) * full + tail;
+    int2 *out = ents + parity * n_before;
+    const int per_row = nfy * G, full = stage_halves(F * per_row), subsets = (g.nv + F - 1) / F;
+    const int tail = stage_halves((g.nv - (subsets - 1) * F) * per_row), n_ents = (subsets - 1) * full + tail;
     for (int e = tid; e < n_ents + kWrap; e += kThreads) {
       const int at0 = e < n_ents ? e : e - n_ents;                       // (n_ents >= kWrap)
-      const int sub = min(at0 / full, subsets - 1), at = at0 - sub * full;
-      const int n_e = min(pl.F, g.nv - sub * pl.F) * per_row, k = min(at, n_e - 1);
-      const int jj = k / per_row, rest = k - jj * per_row, fy = rest / pl.G, gi = rest - fy * pl.G;
-      const int fx = mellin_x ? nth_bit(g.mask, sub * pl.F + jj) : jj;
-      const int row = mellin_x ? jj * g.rows : pl.bx * fx - pl.bx_min;
-      const int2 v = make_int2(gi * pl.group_bytes + (row * pl.RS + pl.by * fy - pl.by_min) * UB,
-                               at < n_e ? ((gi * pl.nfx + fx) * pl.nfy + fy) * (PARTS * 512) : 0x40000000);
+      const int sub = min(udiv(at0, full, mg_full), subsets - 1), at = at0 - sub * full;
+      const int n_e = min(F, g.nv - sub * F) * per_row, k = min(at, n_e - 1);
+      const int jj = udiv(k, per_row, mg_per_row), rest = k - jj * per_row, fy = udiv(rest, G, mg_G), gi = rest - fy * G;
+      const int fx = mellin_x ? filter_row(g, sub * F + jj) : jj;
+      const int row = mellin_x ? jj * g.rows : bx * fx - bx_min;
+      const int2 v = make_int2(gi * group_bytes + (row * RS + by * fy - by_min) * UB,
+                               at < n_e ? ((gi * nfx + fx) * nfy + fy) * (PARTS * 512) : 0x40000000);
       out[e] = v;
       if (e < kWrap && before) before[e] = v;
     }
     return n_ents;
   };
 
-  // the loads of a stage: group g's slots (16 bytes each) b * 64 .. of block b, blocks dealt to the wavefronts
-  int is_b = 0, is_g = 0, is_left = 0, is_v0 = 0, is_raw = 0, is_part = 0;    // the issue in progress: block, group, loads to go ...
-  int groups = 0, group_bytes = 0;
-  unsigned is_dst = 0, is_to = 0;
-  const char *is_src = nullptr, *is_from = nullptr;
-  auto issue_block = [&]() {                           // (the source is read here and first used a load later)
-    const int slot = is_b * 64 + lane;
-    const int unit = F16 ? slot : slot / 3;
-    is_part = F16 ? 0 : (slot - unit * 3) * 16;
-    is_raw = tab[is_v0 + unit];
-    is_from = is_src;
-    is_to = is_dst + (unsigned)(is_b * 1024);
-  };
-  auto issue_begin = [&](const BlockTile &g, int c0, int j0, int buf) {
+  // the loads of a stage: 16-byte slots in blocks of 64, dealt to the wavefronts; the sources of four blocks are read
+  // before the first is used
+  auto issue = [&](const BlockTile &g, int c0, int j0, int buf) {
     const int nF = min(pl.F, g.nv - j0);
-    const int units = mellin_x ? nF * g.rows * pl.RS : g.units;
-    is_v0 = mellin_x ? j0 * g.rows * pl.RS : 0;
-    is_b = wave;
-    is_g = 0;
-    is_src = X + ((i64)g.n * pl.CG + c0) * plane_bytes;
-    is_dst = lds0 + (unsigned)(buf * pl.buf_bytes);
-    groups = pl.G;
-    group_bytes = pl.group_bytes;
+    const int units = mellin_x ? nF * g.rows * pl.RS : g.units, blocks = (units * PARTS + 63) >> 6;
+    const int *from = tab + (mellin_x ? j0 * g.rows * pl.RS : 0);
+    const char *src0 = X + ((i64)g.n * pl.CG + c0) * plane_bytes;
+    const unsigned dst0 = lds0 + (unsigned)(buf * pl.buf_bytes);
+    int groups = pl.G, group_bytes = pl.group_bytes;
     asm volatile("" : "+s"(groups), "+s"(group_bytes));      // (kept in registers: a scalar load in the loop would wait for LDS as well)
-    is_left = max(0, (((units * PARTS + 63) >> 6) - wave + kWaves - 1) / kWaves) * groups;
-    if (is_left > 0) issue_block();
-  };
-  auto issue_one = [&]() {
-    load16_to_lds_at((const float *)is_from, (unsigned)(is_raw + is_part), is_to);
-    is_from += plane_bytes;
-    is_to += (unsigned)group_bytes;
-    --is_left;
-    if (++is_g == groups) {
-      is_g = 0;
-      is_b += kWaves;
-      if (is_left > 0) issue_block();
+    for (int b = wave; b < blocks; b += 4 * kWaves) {
+      unsigned at[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int slot = min(b + i * kWaves, blocks - 1) * 64 + lane, unit = F16 ? slot : slot / 3;
+        at[i] = (unsigned)from[unit] + (F16 ? 0 : (slot - unit * 3) * 16);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (b + i * kWaves < blocks) {
+          const char *src = src0;
+          unsigned dst = dst0 + (unsigned)((b + i * kWaves) * 1024);
+          for (int k = 0; k < groups; ++k) {
+            load16_to_lds_at((const float *)src, at[i], dst);
+            src += plane_bytes;
+            dst += (unsigned)group_bytes;
+          }
+        }
     }
-  };
-  auto issue_down_to = [&](int left) {
-    while (is_left > left) issue_one();
   };
 
   floatx16 acc[MT][NT];
@@ -247,19 +286,18 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       for (int pt = 0; pt < PARTS; ++pt) o.a[k][pt] = *(const uintx4 *)((k ? AFm1 : AFm) + off + pt * 512);
   };
 
-  BlockTile tg = block_tile<P>(pl, (int)blockIdx.x, mellin_x), next_tg = tg;
+  BlockTile tg = block_tile<P>(pl, rows, (int)blockIdx.x, mellin_x), next_tg = tg;
   if (my_tiles <= 0) return;
   int n_ents = build_tile(tg, 0, nullptr), next_ents = n_ents;
   __syncthreads();
-  issue_begin(tg, 0, 0, 0);
-  issue_down_to(0);
-  int c0 = 0, j0 = 0, buf = 0, ti = 0;
+  issue(tg, tg.c_first, 0, 0);
+  int c0 = tg.c_first, j0 = 0, buf = 0, ti = 0;
   int se = 0;                                          // the stage's first entry (of this tile's)
-  unsigned af_c = 0;
+  unsigned af_c = (unsigned)(c0 * taps * PARTS * 512);
   const int2 *my_ents = ents + 2 * wk + half;          // this half-wave's entries (of parity 0)
   int2 e0 = my_ents[0], e1 = my_ents[2 * WK];
-  fetch_a(e0, 0, A0);
-  fetch_a(e1, 0, A1);
+  fetch_a(e0, af_c, A0);
+  fetch_a(e1, af_c, A1);
   wait_and_barrier<0>();
 
   for (bool first = true;;) {
@@ -269,23 +307,21 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       plp = (ConstBlockPlan *)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + zero);
     }
     if (first) {
-      const FastDiv by_noy(pl.noy);
       // position -> virtual position of its (first filter row, first column) tap; accumulators start from the bias
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         int local = (wn * NT + t) * 32 + l32;
         if (local >= tg.count) local = 0;
-        int row, oy;
-        by_noy.divmod(tg.q0 + local, row, oy);
+        const int row = udiv(tg.q0 + local, pl.noy, pl.mg_noy), oy = tg.q0 + local - row * pl.noy;
         lane_vpos[t] = (((mellin_x ? 1 : pl.ax) * (row - tg.row_lo)) * pl.RS + pl.ay * oy) * UB;
-        lane_q[t] = (mellin_x ? class_row(pl, row) : row) * pl.noy + oy;
+        lane_q[t] = (mellin_x ? rows[row].x : row) * pl.noy + oy;
       }
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int g4 = 0; g4 < 4; ++g4) {
           float4 bv = *(const float4 *)(Bs + (wm * MT + i) * 32 + g4 * 8 + half * 4);
-          if (WK > 1 && wk > 0) bv = make_float4(0.f, 0.f, 0.f, 0.f);
+          if ((WK > 1 && wk > 0) || tg.slice > 0) bv = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
             acc[i][t][4 * g4 + 0] = bv.x; acc[i][t][4 * g4 + 1] = bv.y;
@@ -306,24 +342,23 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
     const int steps = halves / (2 * WK);
     int nj0 = mellin_x ? j0 + pl.F : tg.nv, nc0 = c0, n_se = se + halves;
     if (nj0 >= tg.nv) { nj0 = 0; nc0 = c0 + pl.G; n_se = 0; }
-    const bool last = nc0 >= pl.CG;
+    const bool last = nc0 >= tg.c_end;
     const bool more = !last || ti + 1 < my_tiles;
     const int2 *ep = my_ents + (ti & 1) * pl.ents + se;
-    is_left = 0;
     if (last) {
       nc0 = 0;
       nj0 = 0;
       if (more) {
         // another tile: its tables (every load of this tile has been issued, every wavefront is past the barrier)
-        next_tg = block_tile<P>(pl, (int)blockIdx.x + (ti + 1) * (int)gridDim.x, mellin_x);
+        next_tg = block_tile<P>(pl, rows, (int)blockIdx.x + (ti + 1) * (int)gridDim.x, mellin_x);
         next_ents = build_tile(next_tg, (ti + 1) & 1, ents + (ti & 1) * pl.ents + n_ents);
         lds_barrier();
-        issue_begin(next_tg, 0, 0, buf ^ 1);
+        nc0 = next_tg.c_first;
+        issue(next_tg, nc0, 0, buf ^ 1);
       }
     } else {
-      issue_begin(tg, nc0, nj0, buf ^ 1);
+      issue(tg, nc0, nj0, buf ^ 1);
     }
-    issue_down_to(0);
     const unsigned n_af = (unsigned)(nc0 * taps * PARTS * 512);
     // A step: the next step's signal operands are requested before its multiplies and the fragments of the step
     // after next behind them (pinned: the scheduler moves reads next to their use).  Nothing here depends on which
@@ -375,43 +410,89 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
                   make_float4(acc[k][t][4 * r4], acc[k][t][4 * r4 + 1], acc[k][t][4 * r4 + 2], acc[k][t][4 * r4 + 3]);
         __syncthreads();
       }
-      // A store is one add and one buffer store: the descriptor ends with the block's last channel, so rows past it
-      // and lanes without a position (an offset past any end) are dropped by its range check.
-      constexpr int ES = HOUT ? 2 : 4;
-      const int h_m = (int)pl.h_m * ES, m0 = m_tile * M_T + wm * MT * 32;
-      const bool relu = pl.relu;
-      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-          (char *)Hv + ((i64)tg.n * pl.h_n * ES + (i64)m0 * h_m), 0, max(0, min(MT * 32, pl.M - m0)) * h_m, 0x00020000);
+      // The descriptor ends with the block's last channel, so rows past it and lanes without a position (an offset past
+      // any end) are dropped by its range check.  A slice's sums are fp32, in the order of the tile.
+      const bool whole = tg.slot < 0, relu = pl.relu && whole, as_half = HOUT && whole;
+      const int m0 = m_tile * M_T + wm * MT * 32, ES = as_half ? 2 : 4, h_m = (whole ? (int)pl.h_m : P) * ES;
+      char *base = whole ? (char *)Hv + ((i64)tg.n * pl.h_n + (i64)m0 * (int)pl.h_m) * ES
+                         : (char *)(sums + (((i64)tg.slot * gridDim.y + m_tile) * M_T + wm * MT * 32) * P);
+      const __amdgpu_buffer_rsrc_t rsrc =
+          __builtin_amdgcn_make_buffer_rsrc(base, 0, max(0, min(MT * 32, pl.M - m0)) * h_m, 0x00020000);
       int at[NT];
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-        at[t] = (wn * NT + t) * 32 + l32 < tg.count ? half * 4 * h_m + lane_q[t] * ES : (int)0x80000000u;
+      for (int t = 0; t < NT; ++t) {
+        const int local = (wn * NT + t) * 32 + l32;
+        at[t] = local < tg.count ? (whole ? lane_q[t] : local) * ES : (int)0x80000000u;
+      }
+      auto store_one = [&](float v, int to) {
+        if (as_half) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(short, (_Float16)v), rsrc, to, 0, 0);
+        else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rsrc, to, 0, 0);
+      };
+      const int row0 = half * 4 * h_m;
+      auto relu4 = [&](float4 v) { return relu ? make_float4(fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f)) : v; };
+      auto store_four = [&](float4 v, int to) {        // four channels of the lane's position
+        v = relu4(v);
+        store_one(v.x, to);
+        store_one(v.y, to + h_m);
+        store_one(v.z, to + 2 * h_m);
+        store_one(v.w, to + 3 * h_m);
+      };
+      if constexpr (WK > 1) {
+        // the tile's 32 x 32 blocks are dealt to the wavefronts
+        const float *red = (const float *)bufs;
+        for (int kt = wk; kt < MT * NT; kt += WK) {
+          const int k = kt / NT, t = kt - k * NT;
+          int to = (NT > 1 && t ? at[NT - 1] : at[0]) + row0 + k * 32 * h_m;
 #pragma unroll
-      for (int k = 0; k < MT; ++k) {
+          for (int r4 = 0; r4 < 4; ++r4) {
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
+            for (int w = 0; w < WK; ++w) {
+              const float4 p = *(const float4 *)(red + (((w * MT * NT + kt) * 4 + r4) * 64 + lane) * 4);
+              v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
+            }
+            store_four(v, to);
+            to += 8 * h_m;                             // (registers 4 g .. 4 g + 3 are rows 8 g + 4 half ..)
+          }
+        }
+      } else {
+        // A 4 x 4 transpose over four lanes makes four channels of a position four positions of a channel, side by side
+        // in memory: a quarter of the stores (128 x 256 half values: 22000 -> 12000 cycles).  Not for the rows of a class
+        // (n_classes > 1), which do not follow each other; the last positions of an image, less than four, go one by one.
+        bool single = true;
+        if (pl.n_classes == 1 || !whole) {
+          int to[NT];
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
-            float v = acc[k][t][r];
-            bool mine = true;
-            if constexpr (WK > 1) {
-              mine = ((k * NT + t) & (WK - 1)) == wk;
-              if (mine) {
-                const float *red = (const float *)bufs;
-                v = 0.f;
-#pragma unroll
-                for (int w = 0; w < WK; ++w) v += red[(((w * MT * NT + k * NT + t) * 4 + (r >> 2)) * 64 + lane) * 4 + (r & 3)];
-              }
-            }
-            if (relu) v = fmaxf(v, 0.f);
-            if (mine) {
-              if constexpr (HOUT)
-                __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(short, (_Float16)v), rsrc, at[t], 0, 0);
-              else
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rsrc, at[t], 0, 0);
-            }
-            at[t] += (r & 3) == 3 ? 5 * h_m : h_m;     // (registers 4 g .. 4 g + 3 are rows 8 g + 4 half ..)
+            const int first = quad_lane<0>(at[t]), last = quad_lane<3>(at[t]);
+            to[t] = last >= 0 ? row0 + (lane & 3) * h_m + first : (int)0x80000000u;
+            if (last >= 0) at[t] = (int)0x80000000u;
           }
+#pragma unroll
+          for (int k = 0; k < MT; ++k)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4)
+#pragma unroll
+              for (int t = 0; t < NT; ++t) {
+                const float4 v = relu4(make_float4(acc[k][t][4 * g4], acc[k][t][4 * g4 + 1], acc[k][t][4 * g4 + 2], acc[k][t][4 * g4 + 3]));
+                if (as_half) __builtin_amdgcn_raw_buffer_store_b64(transpose_half(v, lane), rsrc, to[t], 0, 0);
+                else __builtin_amdgcn_raw_buffer_store_b128(transpose_words(v, lane), rsrc, to[t], 0, 0);
+                to[t] += 8 * h_m;
+              }
+          single = tg.count & 3;
+        }
+        if (single) {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) at[t] += row0;
+#pragma unroll
+          for (int k = 0; k < MT; ++k)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4)
+#pragma unroll
+              for (int t = 0; t < NT; ++t) {
+                store_four(make_float4(acc[k][t][4 * g4], acc[k][t][4 * g4 + 1], acc[k][t][4 * g4 + 2], acc[k][t][4 * g4 + 3]), at[t]);
+                at[t] += 8 * h_m;
+              }
         }
       }
       if (!more) break;
@@ -429,13 +510,14 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
 }
 
 template <int MT, int NT, int WM, int WK, bool F16, bool HOUT>
-hipError_t launch_instance(const BlockPlan &pl, const void *x, const void *frag, const void *bias, void *out, hipStream_t stream) {
+hipError_t launch_instance(const BlockPlan &pl, const void *x, const void *frag, const void *bias, void *out, float *sums,
+                           hipStream_t stream) {
   auto kern = block_gemm_kernel<MT, NT, WM, WK, F16, HOUT>;
   static std::atomic<int> lds_allowed{0};
   hipError_t e = allow_large_lds((const void *)kern, pl.lds_bytes, lds_allowed);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)pl.grid_x, (unsigned)pl.m_tiles), dim3(kThreads), pl.lds_bytes, stream, pl,
-                     (const char *)x, (const char *)frag, bias, out);
+  hipLaunchKernelGGL(kern, dim3((unsigned)pl.grid_x, (unsigned)pl.m_tiles), dim3(kThreads), pl.lds_bytes, stream,
+                     pl, (const char *)x, (const char *)frag, bias, out, sums);
   return hipGetLastError();
 }
 
@@ -542,6 +624,7 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
     const i64 RT = std::min<i64>(pl.nox, (P - 1 + pl.noy - 1) / pl.noy + 1);
     const i64 vrows = mellin ? RT : (i64)pl.ax * (RT - 1) + pl.bx_span + 1;
     const i64 tab = ((mellin ? vrows * pl.nfx : vrows) * pl.RS + 64 + 64 + 3) & ~(i64)3;
+    const i64 row_src = mellin ? 4 * RT * pl.nfx : 0;
     auto pad = [&](i64 halves) { return std::max<i64>((halves + 2 * wk - 1) / (2 * wk) * (2 * wk), 4 * wk); };
     int best_f = 0, best_g = 0;
     double best = 0;
@@ -552,7 +635,7 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
       for (int G = std::min(pl.CG, 8); G >= 1; --G) {
         if (pl.CG % G) continue;
         const i64 ents = (mellin ? (pl.nfx + F - 1) / F : 1) * pad((i64)rows * pl.nfy * G) + 8 * wk;
-        const i64 bytes = 2 * gb * G + 4 * tab + 16 * ents + M_T * 4;
+        const i64 bytes = 2 * gb * G + 4 * tab + 16 * ents + row_src + M_T * 4;
         if (bytes > 79 * 1024) continue;
         // what a stage's steps fill of their whole pairs, against what a stage costs on top (its barrier and first reads)
         const i64 halves = (i64)rows * pl.nfy * G;
@@ -569,45 +652,97 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
     pl.group_bytes = (int)((units * parts + 63) / 64 * 1024);
     pl.buf_bytes = pl.group_bytes * best_g;
     pl.nt = nt; pl.wm = wm; pl.wk = wk;
-    pl.tiles_per_image = (pl.Q + P - 1) / P;
-    if ((i64)pl.tiles_per_image * pl.batch >= lim) return false;
-    pl.total_tiles = pl.tiles_per_image * pl.batch;
+    if ((i64)((pl.Q + P - 1) / P) * pl.batch >= (i64)1 << 26) return false;
     size_t bytes = 2 * (size_t)pl.buf_bytes;
     if (wk > 1) bytes = std::max(bytes, (size_t)wk * pl.mt * nt * 4096);
     if (wk > 1) pl.buf_bytes = (int)(bytes / 2);
-    bytes += 4 * (size_t)tab + 16 * (size_t)pl.ents + M_T * 4;
+    bytes += 4 * (size_t)tab + 16 * (size_t)pl.ents + row_src + M_T * 4;
     pl.lds_bytes = bytes;
     pl.m_tiles = (int)((pr.c_out + M_T - 1) / M_T);
     return bytes <= 79 * 1024;
   };
+  auto magic = [](i64 d) { return d <= 1 ? 0xFFFFFFFFu : (unsigned)(0x100000000ull / (unsigned)d); };
+  pl.mg_batch = magic(pl.batch); pl.mg_noy = magic(pl.noy);
+  double rows_used = pl.nfx;                           // filter rows of an output row, on average
+  if (mellin) {
+    rows_used = 0;
+    for (int k = 0; k < pl.n_classes; ++k)
+      rows_used += __builtin_popcount(pl.cls[k].mask) * (double)((k + 1 < pl.n_classes ? pl.cls[k + 1].start : pl.nox) - pl.cls[k].start);
+    rows_used = std::max(1.0, rows_used / pl.nox);
+  }
+
+  // The launch of a tile shape, in cycles.  Workgroups take tiles in turn, two to a CU (512 at a time).  What does not fill
+  // a last turn -- for few tiles: all of them -- can be cut into slices of the contracted channels, which another kernel
+  // adds up.  Measured on this chip, and rounded:
+  //   a step's matrix instructions at 65-80 % of their rate (larger tiles: the higher), shared by a CU's workgroups;
+  //   a stage at least 4000 (the latency of its loads);
+  //   per tile 5000 for its tables and its output at 9 bytes a cycle; 9000 for a launch's start, as much for the kernel
+  //   that adds the slices, and 2400 bytes a cycle for their sums.
   const i64 slots = 512;
-  auto tiles = [&](int P, int M_T) { return pl.batch * ((Q + P - 1) / P) * ((pr.c_out + M_T - 1) / M_T); };
-  const int m1 = 32 * pl.mt;
-  bool ok = false;
-  if (f16 && pr.c_out > 96 && tiles(256, 128) >= slots) ok = shape(4, 2, 1);
-  if (!ok && f16 && tiles(512, m1) >= slots) ok = shape(4, 1, 1);
-  if (!ok && tiles(256, m1) >= slots) ok = shape(2, 1, 1);
-  if (!ok && tiles(128, m1) >= slots / 2) ok = shape(1, 1, 1);
-  if (!ok) ok = shape(2, 1, 4) || shape(1, 1, 4);
-  if (!ok) ok = shape(2, 1, 1) || shape(1, 1, 1);
-  if (!ok) return false;
-  pl.filter_bytes = (size_t)pl.m_tiles * pl.wm * pl.mt * ((size_t)pl.CG * pl.nfx * pl.nfy + 1) * parts * 512;
-  if (pl.filter_bytes >= (size_t)lim) return false;
-  pl.grid_x = pl.wk > 1 ? pl.total_tiles : (int)std::min<i64>(pl.total_tiles, std::max<i64>(1, slots / pl.m_tiles));
+  auto cost = [&]() {
+    const int M_T = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32;
+    const i64 total = (i64)((Q + P - 1) / P) * pl.batch, per_m = std::max<i64>(1, slots / pl.m_tiles), c_stages = pl.CG / pl.G;
+    const double subsets = mellin ? std::max(1.0, std::ceil(rows_used / pl.F)) : 1, rows = rows_used / subsets;
+    const double rate = pl.mt * pl.nt >= 8 ? 0.8 : pl.mt * pl.nt >= 4 ? 0.65 : 0.55;
+    const double steps = std::ceil(rows * pl.nfy * pl.G / (2 * pl.wk)) * pl.mt * pl.nt * (f16 ? 1 : 6) * 32 / rate;
+    const double output = (double)M_T * P * (f16 ? 2 : 4) / 9;
+    auto turns_cost = [&](i64 items, double stages) {
+      const i64 full = items / per_m, left = items - full * per_m;
+      auto turn = [&](i64 n) { return stages * std::max(4000.0, steps * (n * pl.m_tiles > slots / 2 ? 2 : 1)) + 5000 + output; };
+      return full * turn(per_m) + (left ? turn(left) : 0);
+    };
+    double best = 9000 + turns_cost(total, c_stages * subsets);
+    pl.slices = 1;
+    i64 rest = 0;
+    for (int all = 0; all < 2; ++all) {
+      const i64 r = all ? total : total % per_m;
+      if (r == 0 || (all && total >= 2 * per_m) || (pl.wk > 1 && !all)) continue;
+      for (i64 s = 2; s <= std::min<i64>(c_stages, 16); ++s) {
+        const double bytes = (double)r * s * pl.m_tiles * M_T * P * 8;
+        const double c = 9000 + turns_cost(total - r, c_stages * subsets) + turns_cost(r * s, std::ceil((double)c_stages / s) * subsets) +
+                         9000 + bytes / 2400;
+        if (c < 0.95 * best) { best = c; pl.slices = (int)s; rest = r; }
+      }
+    }
+    pl.rest = (int)rest;
+    pl.whole = (int)(total - rest);
+    const i64 items = (i64)pl.whole + (i64)pl.rest * pl.slices;
+    pl.grid_x = (int)(pl.wk > 1 ? items : std::min<i64>(per_m, items));      // (wavefronts that share a tile's steps take one tile)
+    pl.slice_bytes = (size_t)pl.rest * pl.slices * pl.m_tiles * (size_t)(M_T * P) * 4;
+    return best;
+  };
+  static const int shapes[][3] = {{4, 2, 1}, {4, 1, 1}, {2, 1, 1}, {1, 1, 1}, {2, 1, 4}, {1, 1, 4}};   // nt, wm, wk
+  BlockPlan best_plan;
+  double best_cost = 0;
+  for (const auto &sh : shapes) {
+    if (sh[0] == 4 && !f16) continue;
+    if (sh[1] == 2 && pr.c_out <= 96) continue;        // (two wavefronts along the channels: most of 128)
+    if (!shape(sh[0], sh[1], sh[2])) continue;
+    const double c = cost();
+    if (best_cost == 0 || c < best_cost) { best_cost = c; best_plan = pl; }
+  }
+  if (best_cost == 0) return false;
+  pl = best_plan;
+  const i64 per_row = (i64)pl.nfy * pl.G, pairs = 2 * pl.wk;
+  pl.mg_per_row = magic(per_row); pl.mg_G = magic(pl.G);
+  pl.mg_full = magic(std::max<i64>((pl.F * per_row + pairs - 1) / pairs * pairs, 2 * pairs));
+  pl.rows_off = (size_t)pl.m_tiles * pl.wm * pl.mt * ((size_t)pl.CG * pl.nfx * pl.nfy + 1) * parts * 512;
+  if (pl.rows_off >= (size_t)lim) return false;
+  pl.filter_bytes = pl.rows_off + (mellin ? 8 * (size_t)pl.nox : 0);
   return true;
 }
 
 hipError_t launch_block_gemm(const BlockPlan &pl, const void *signal, const void *frag, const void *bias, void *out,
-                             hipStream_t stream) {
+                             float *sums, hipStream_t stream) {
 #define MELLIN_BLOCK_CASE(MT_, NT_, WM_, WK_)                                                                \
   if (pl.mt == MT_ && pl.nt == NT_ && pl.wm == WM_ && pl.wk == WK_) {                                        \
-    if (pl.f16) return launch_instance<MT_, NT_, WM_, WK_, true, true>(pl, signal, frag, bias, out, stream); \
-    return launch_instance<MT_, NT_, WM_, WK_, false, false>(pl, signal, frag, bias, out, stream);           \
+    if (pl.f16) return launch_instance<MT_, NT_, WM_, WK_, true, true>(pl, signal, frag, bias, out, sums, stream); \
+    return launch_instance<MT_, NT_, WM_, WK_, false, false>(pl, signal, frag, bias, out, sums, stream);           \
   }
   if (pl.f16 && pl.nt == 4) {
-    if (pl.wm == 2) return launch_instance<2, 4, 2, 1, true, true>(pl, signal, frag, bias, out, stream);
-    if (pl.mt == 2) return launch_instance<2, 4, 1, 1, true, true>(pl, signal, frag, bias, out, stream);
-    return launch_instance<1, 4, 1, 1, true, true>(pl, signal, frag, bias, out, stream);
+    if (pl.wm == 2) return launch_instance<2, 4, 2, 1, true, true>(pl, signal, frag, bias, out, sums, stream);
+    if (pl.mt == 2) return launch_instance<2, 4, 1, 1, true, true>(pl, signal, frag, bias, out, sums, stream);
+    return launch_instance<1, 4, 1, 1, true, true>(pl, signal, frag, bias, out, sums, stream);
   }
   MELLIN_BLOCK_CASE(2, 2, 1, 1)
   MELLIN_BLOCK_CASE(2, 1, 1, 1)

@@ -37,7 +37,10 @@ struct BlockPlan {
   int tab_units;                   // positions of a tile's source table
   int ents;                        // operand offsets of a tile's steps
   int group_bytes, buf_bytes;      // LDS of one group of a stage, of a stage
-  int tiles_per_image, total_tiles;
+  // tiles: (position tile, image), the images of a position tile side by side.  The last `rest` of them, which would
+  // leave workgroups without one, are dealt out in `slices` of the contracted channels, whose sums go to the workspace
+  int whole, rest, slices;
+  unsigned mg_batch, mg_noy, mg_per_row, mg_full, mg_G;      // floor(2^32 / d) (see udiv)
   i64 h_n, h_m;
   int relu, half_out;
   int n_classes, cls_stride;
@@ -47,16 +50,17 @@ struct BlockPlan {
   int f_pitch, f_off;
   // launch
   int mt, nt, wm, wk, m_tiles, grid_x;
-  size_t lds_bytes, filter_bytes;
+  size_t lds_bytes;
+  size_t rows_off, filter_bytes;   // the packed filter: fragments, then (Mellin axes) the output rows in the order of their classes
+  size_t slice_bytes;              // workspace of the slices' sums
 };
 
 // False: the kernel does not apply.
 bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl);
-// The filter of `pl` as fragments: f (fp32 or half storage) -> filter_bytes at `frag`.
-hipError_t launch_pack_filter(const BlockPlan &pl, int channels, const void *f, void *frag, hipStream_t stream);
-// out = [relu](bias + sum) from a blocked signal and packed filter; bias (fp32 / half, or null).
+// out = [relu](bias + sum) from a blocked signal and packed filter; bias (fp32 / half, or null).  Of tiles in slices
+// (pl.rest > 0) the sums go to `sums` and launch_block_finish makes the output.
 hipError_t launch_block_gemm(const BlockPlan &pl, const void *signal, const void *frag, const void *bias, void *out,
-                             hipStream_t stream);
+                             float *sums, hipStream_t stream);
 
 // The rows of one filter row in the weight gradient: output rows ox0 + i step and input rows gx0 + i gstep for
 // i < count; its share of the launch: `slices` workgroups from slice0 on.
@@ -78,18 +82,38 @@ struct BlockWgradPlan {
 
 // `fwd`: the forward pass's problem (x axis Mellin or linear correlation, y linear correlation).
 bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl);
-// grad_out, input: blocked; grad_weight: fp32 / half.
-hipError_t launch_block_wgrad(const BlockWgradPlan &pl, const void *grad_out, const void *input, void *grad_weight,
-                              float *workspace, hipStream_t stream);
-
-// x (batch, channels, plane), fp32 or half -> blocked.  With `relu_out` (the layer's output) values
-// whose output is not positive are zeros (the backward of the fused ReLU).  With `partial`:
-// per-channel sums of what was written, block by block, for launch_bias_reduce
-// (pack_partial_count(): floats).
-hipError_t launch_pack_signal(const void *x, const void *relu_out, bool f16, i64 batch, i64 channels, i64 plane,
-                              void *blocked, float *partial, hipStream_t stream);
-size_t pack_partial_count(i64 batch, i64 channels, i64 plane);
-hipError_t launch_bias_reduce(const float *partial, i64 per_channel, i64 channels, void *grad_bias, bool f16,
+// Partial blocks of the weight gradient (ws_bytes at `partial`) from blocked tensors.
+hipError_t launch_block_wgrad(const BlockWgradPlan &pl, const void *grad_out, const void *input, float *partial,
                               hipStream_t stream);
+
+// A tensor to lay out: x (batch, channels, plane), fp32 or half -> blocked.  With `relu_out` (the layer's output) values
+// whose output is not positive are zeros (the backward of the fused ReLU).  With `partial`: per-channel sums of what was
+// written, block by block, for launch_block_finish (pack_partial_count(): floats).
+struct PackSignal {
+  const void *x, *relu_out;
+  char *blocked;
+  float *partial;
+  int batch, channels, plane;
+};
+size_t pack_partial_count(i64 batch, i64 channels, i64 plane);
+// Everything a pass reads in one launch: up to two tensors and the filter of `pl` (f: fp32 or half, `channels`
+// contracted channels -> filter_bytes at `frag`); null for what there is not.
+hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b, const BlockPlan *pl, int channels,
+                             const void *f, void *frag, hipStream_t stream);
+
+// The sums that end a pass, in one launch; null pointers for those there are not.
+struct BlockFinish {
+  const BlockWgradPlan *weight;    // weight gradient from its partial blocks
+  const float *weight_partial;
+  void *grad_weight;
+  const float *bias_partial;       // bias gradient: `bias_count` partial sums of each of `channels`
+  void *grad_bias;
+  i64 bias_count, channels;
+  const BlockPlan *slices;         // the output of a block_gemm's tiles in slices
+  const void *frag;                // (its packed filter)
+  const float *slice_sums;
+  void *out;
+};
+hipError_t launch_block_finish(bool f16, const BlockFinish &job, hipStream_t stream);
 
 }  // namespace mellin

@@ -8,6 +8,9 @@
 // channels -- which kept those kernels' vector pipe as busy as their matrix pipe.  Where the
 // layer's backward pass also wants the bias gradient and the backward of a fused ReLU, they
 // ride along: the gradient is read once, and its masked form is written in this layout only.
+//
+// All that a pass reads is packed by one launch: small layers are bound by launches, and the
+// filter's few blocks hide behind the signal's.
 #include <algorithm>
 
 #include "block_gemm.hpp"
@@ -20,21 +23,27 @@ namespace {
 constexpr int kPackThreads = 256;
 constexpr int kPackPositions = 4;                  // per thread
 
+struct PackPart {                                  // a signal, dealt to blocks as (image, group, chunk of its plane)
+  PackSignal s;
+  int groups, chunks;
+  unsigned blocks;
+};
+
 template <bool F16, bool MASK, bool SUM>
-__global__ __launch_bounds__(kPackThreads) void pack_signal_kernel(const void *__restrict__ xv, const void *__restrict__ maskv,
-                                                                   int channels, int plane, char *__restrict__ blocked,
-                                                                   float *__restrict__ partial) {
+__device__ __forceinline__ void pack_signal(const PackPart &pt, unsigned block, float (*red)[8]) {
   typedef typename std::conditional<F16, _Float16, float>::type T;
   constexpr int UB = F16 ? 16 : 48;
-  const int groups = gridDim.y, cg = blockIdx.y, n = blockIdx.z, batch = gridDim.z;
+  const int groups = pt.groups, chunks = pt.chunks, plane = pt.s.plane, channels = pt.s.channels;
+  const int row = (int)(block / (unsigned)chunks), chunk = (int)(block - (unsigned)row * (unsigned)chunks);
+  const int n = row / groups, cg = row - n * groups;
   const int c0 = cg * 8, live = min(8, channels - c0);
-  const T *x = (const T *)xv + ((i64)n * channels + c0) * plane;
-  const T *mk = MASK ? (const T *)maskv + ((i64)n * channels + c0) * plane : nullptr;
-  char *out = blocked + ((i64)n * groups + cg) * (i64)(plane + 1) * UB;
+  const T *x = (const T *)pt.s.x + ((i64)n * channels + c0) * plane;
+  const T *mk = MASK ? (const T *)pt.s.relu_out + ((i64)n * channels + c0) * plane : nullptr;
+  char *out = pt.s.blocked + ((i64)n * groups + cg) * (i64)(plane + 1) * UB;
   float sum[8];
 #pragma unroll
   for (int c = 0; c < 8; ++c) sum[c] = 0.f;
-  const int q0 = blockIdx.x * (kPackThreads * kPackPositions) + threadIdx.x;
+  const int q0 = chunk * (kPackThreads * kPackPositions) + threadIdx.x;
 #pragma unroll
   for (int i = 0; i < kPackPositions; ++i) {
     const int q = q0 + i * kPackThreads;
@@ -74,7 +83,6 @@ __global__ __launch_bounds__(kPackThreads) void pack_signal_kernel(const void *_
   }
   if (SUM) {
     // sums in a fixed order: a shuffle tree per wavefront, the wavefronts in order
-    __shared__ float red[kPackThreads / 64][8];
 #pragma unroll
     for (int c = 0; c < 8; ++c)
 #pragma unroll
@@ -86,7 +94,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_signal_kernel(const void *_
     if ((int)threadIdx.x < live) {
       float a = 0.f;
       for (int w = 0; w < kPackThreads / 64; ++w) a += red[w][threadIdx.x];
-      partial[((i64)(c0 + threadIdx.x) * batch + n) * gridDim.x + blockIdx.x] = a;
+      pt.s.partial[((i64)(c0 + threadIdx.x) * pt.s.batch + n) * chunks + chunk] = a;
     }
   }
 }
@@ -96,10 +104,9 @@ __global__ __launch_bounds__(kPackThreads) void pack_signal_kernel(const void *_
 //   frag[((mt * (CG * nfx * nfy + 1) + (cg * nfx + fx) * nfy + fy) * parts + p) * 32 + r]   (16-byte words)
 // and a unit of zeros behind each tile of 32 channels.
 template <bool F16>
-__global__ __launch_bounds__(kPackThreads) void pack_filter_kernel(BlockPlan pl, int channels, const void *__restrict__ fv,
-                                                                   uintx4 *__restrict__ frag) {
+__device__ __forceinline__ void pack_filter(const BlockPlan &pl, int channels, const void *__restrict__ fv, uintx4 *__restrict__ frag,
+                                            i64 idx) {
   typedef typename std::conditional<F16, _Float16, float>::type T;
-  const i64 idx = (i64)blockIdx.x * kPackThreads + threadIdx.x;
   const int taps = pl.nfx * pl.nfy, per_tile = pl.CG * taps + 1;
   const i64 total = (i64)pl.m_tiles * pl.wm * pl.mt * per_tile * 32;
   if (idx >= total) return;
@@ -129,7 +136,65 @@ __global__ __launch_bounds__(kPackThreads) void pack_filter_kernel(BlockPlan pl,
   }
 }
 
+// Output row `row` of a Mellin axis in the order of its classes, with the filter rows that have a tap for it.
+__device__ __forceinline__ int2 class_row(const BlockPlan &pl, int row) {
+  int ox = row;
+  for (int k = 0; k < pl.n_classes; ++k)
+    if (row >= pl.cls[k].start) ox = pl.cls[k].first + (row - pl.cls[k].start) * pl.cls_stride;
+  int mask = 0;
+  for (int f = 0; f < pl.nfx; ++f)
+    if (mellin_tap32(pl.kind_x, ox, f, pl.ngx, pl.sx, pl.dx, pl.px + 1, pl.ux, pl.mg_p1) >= 0) mask |= 1 << f;
+  return make_int2(ox, mask);
+}
+
+struct PackArgs {
+  PackPart a, b;
+  BlockPlan pl;
+  int channels;
+  unsigned filter_blocks, row_blocks;
+  const void *f;
+  char *frag;
+};
+
+template <bool F16>
+__global__ __launch_bounds__(kPackThreads) void block_pack_kernel(PackArgs args) {
+  __shared__ float red[kPackThreads / 64][8];
+  unsigned b = blockIdx.x;
+  if (b < args.row_blocks) {
+    const int row = (int)(b * kPackThreads + threadIdx.x);
+    if (row < args.pl.nox) ((int2 *)(args.frag + args.pl.rows_off))[row] = class_row(args.pl, row);
+    return;
+  }
+  b -= args.row_blocks;
+  if (b < args.filter_blocks) {
+    pack_filter<F16>(args.pl, args.channels, args.f, (uintx4 *)args.frag, (i64)b * kPackThreads + threadIdx.x);
+    return;
+  }
+  b -= args.filter_blocks;
+  const bool second = b >= args.a.blocks;
+  const PackPart &pt = second ? args.b : args.a;
+  if (second) b -= args.a.blocks;
+  if (pt.s.relu_out) {
+    if (pt.s.partial) pack_signal<F16, true, true>(pt, b, red);
+    else pack_signal<F16, true, false>(pt, b, red);
+  } else {
+    if (pt.s.partial) pack_signal<F16, false, true>(pt, b, red);
+    else pack_signal<F16, false, false>(pt, b, red);
+  }
+}
+
 i64 pack_chunks(i64 plane) { return plane / (kPackThreads * kPackPositions) + 1; }     // (plane + 1 units)
+
+bool pack_part(const PackSignal *s, PackPart &pt) {
+  pt = PackPart{};
+  if (!s) return true;
+  pt.s = *s;
+  pt.groups = (s->channels + 7) / 8;
+  pt.chunks = (int)pack_chunks(s->plane);
+  const i64 blocks = (i64)s->batch * pt.groups * pt.chunks;
+  pt.blocks = (unsigned)blocks;
+  return blocks < (i64)1 << 30;
+}
 
 }  // namespace
 
@@ -137,32 +202,22 @@ size_t pack_partial_count(i64 batch, i64 channels, i64 plane) {
   return (size_t)(batch * channels * pack_chunks(plane));
 }
 
-hipError_t launch_pack_signal(const void *x, const void *relu_out, bool f16, i64 batch, i64 channels, i64 plane,
-                              void *blocked, float *partial, hipStream_t stream) {
-  const dim3 grid((unsigned)pack_chunks(plane), (unsigned)((channels + 7) / 8), (unsigned)batch);
-#define MELLIN_PACK_CASE(F_, M_, S_)                                                                                     \
-  if (f16 == F_ && (relu_out != nullptr) == M_ && (partial != nullptr) == S_)                                            \
-    hipLaunchKernelGGL((pack_signal_kernel<F_, M_, S_>), grid, dim3(kPackThreads), 0, stream, x, relu_out, (int)channels, \
-                       (int)plane, (char *)blocked, partial);
-  MELLIN_PACK_CASE(false, false, false)
-  MELLIN_PACK_CASE(false, false, true)
-  MELLIN_PACK_CASE(false, true, false)
-  MELLIN_PACK_CASE(false, true, true)
-  MELLIN_PACK_CASE(true, false, false)
-  MELLIN_PACK_CASE(true, false, true)
-  MELLIN_PACK_CASE(true, true, false)
-  MELLIN_PACK_CASE(true, true, true)
-#undef MELLIN_PACK_CASE
-  return hipGetLastError();
-}
-
-hipError_t launch_pack_filter(const BlockPlan &pl, int channels, const void *f, void *frag, hipStream_t stream) {
-  const i64 total = (i64)pl.m_tiles * pl.wm * pl.mt * ((i64)pl.CG * pl.nfx * pl.nfy + 1) * 32;
-  const dim3 grid((unsigned)((total + kPackThreads - 1) / kPackThreads));
-  if (pl.f16)
-    hipLaunchKernelGGL(pack_filter_kernel<true>, grid, dim3(kPackThreads), 0, stream, pl, channels, f, (uintx4 *)frag);
-  else
-    hipLaunchKernelGGL(pack_filter_kernel<false>, grid, dim3(kPackThreads), 0, stream, pl, channels, f, (uintx4 *)frag);
+hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b, const BlockPlan *pl, int channels,
+                             const void *f, void *frag, hipStream_t stream) {
+  PackArgs args = {};
+  if (!pack_part(a, args.a) || !pack_part(b, args.b)) return hipErrorInvalidValue;
+  if (pl) {
+    args.pl = *pl;
+    args.channels = channels;
+    args.f = f;
+    args.frag = (char *)frag;
+    const i64 total = (i64)pl->m_tiles * pl->wm * pl->mt * ((i64)pl->CG * pl->nfx * pl->nfy + 1) * 32;
+    args.filter_blocks = (unsigned)((total + kPackThreads - 1) / kPackThreads);
+    if (pl->kind_x == AX_MCORR || pl->kind_x == AX_MCONV) args.row_blocks = (unsigned)((pl->nox + kPackThreads - 1) / kPackThreads);
+  }
+  const unsigned blocks = args.row_blocks + args.filter_blocks + args.a.blocks + args.b.blocks;
+  if (f16) hipLaunchKernelGGL(block_pack_kernel<true>, dim3(blocks), dim3(kPackThreads), 0, stream, args);
+  else hipLaunchKernelGGL(block_pack_kernel<false>, dim3(blocks), dim3(kPackThreads), 0, stream, args);
   return hipGetLastError();
 }
 

@@ -20,7 +20,7 @@
 // are worked out two stages ahead, one entry per thread.  There are no register loads in the loop,
 // so the only wait for memory is the one at a stage's start, for loads issued a whole stage before.
 //
-// Every workgroup writes its sums as one partial block; block_wgrad_reduce_kernel adds a weight's partial
+// Every workgroup writes its sums as one partial block; block_finish.hip adds a weight's partial
 // sums in slice order (bit-reproducible).
 //
 // Measured, 256 -> 256 channels, 4 x 4 taps, 16 x 100 x 41 positions: fp32, linear rows 1172 -> 994 us; half, Mellin
@@ -239,58 +239,6 @@ __global__ __launch_bounds__(NW * 64, 2) void block_wgrad_kernel(BlockWgradPlan 
 #undef pl
 }
 
-// gw[m, c, fx, fy] = the sum of its partial sums in slice order.  A block owns 32 weights that lie side by side in
-// the partial blocks; its eight groups of 32 threads add an eighth of the slices each, and those sums are added in order.
-template <typename T>
-__global__ __launch_bounds__(256) void block_wgrad_reduce_kernel(BlockWgradPlan pl, const float *__restrict__ ws,
-                                                                 T *__restrict__ gw) {
-  __shared__ float red[8][32];
-  const int cl = threadIdx.x & 31, grp = threadIdx.x >> 5;
-  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.wm * pl.mt * 32;
-  // block -> (filter row, column tile, channel)
-  const int tiles = pl.ctb * pl.nfy;
-  int b = blockIdx.x;
-  const int m = b % pl.M;
-  b /= pl.M;
-  const int tile = b % tiles;
-  b /= tiles;
-  const int cb = b % pl.c_blocks, fx = b / pl.c_blocks;
-  const int ct = tile / pl.nfy, fy = tile - ct * pl.nfy, c = (cb * pl.ctb + ct) * 32 + cl;
-  const int mb = m / m_t, ml = m - mb * m_t;
-  const int slices = pl.row[fx].slices, blocks = pl.m_blocks * pl.c_blocks;
-  const i64 stride = (i64)blocks * m_t * cols;
-  const float *p = ws + ((i64)pl.row[fx].slice0 * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols + tile * 32 + cl;
-  const int lo = slices * grp / 8, hi = slices * (grp + 1) / 8;
-  float s = 0.f;
-  int k = lo;
-  for (; k + 4 <= hi; k += 4) {
-    float v[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = p[(k + i) * stride];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s += v[i];
-  }
-  for (; k < hi; ++k) s += p[k * stride];
-  red[grp][cl] = s;
-  __syncthreads();
-  if (grp == 0 && c < pl.C) {
-    float a = red[0][cl];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) a += red[i][cl];
-    gw[(((i64)m * pl.C + c) * pl.nfx + fx) * pl.f_pitch + pl.f_off + fy] = (T)a;
-  }
-}
-
-// Filter columns that have no tap at all: zeros.
-template <typename T>
-__global__ __launch_bounds__(256) void block_wgrad_zero_kernel(BlockWgradPlan pl, T *__restrict__ gw) {
-  const i64 n = (i64)pl.M * pl.C * pl.nfx * pl.f_pitch;
-  for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < n; i += (i64)gridDim.x * 256) {
-    const int fy = (int)(i % pl.f_pitch);
-    if (fy < pl.f_off || fy >= pl.f_off + pl.nfy) gw[i] = (T)0;
-  }
-}
-
 template <int MT, int NT, int NW, bool F16>
 hipError_t launch_wgrad_instance(const BlockWgradPlan &pl, const void *a, const void *g, float *ws, hipStream_t stream) {
   auto kern = block_wgrad_kernel<MT, NT, NW, F16>;
@@ -403,8 +351,8 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
   return pl.ws_bytes <= ((size_t)1 << 30);
 }
 
-hipError_t launch_block_wgrad(const BlockWgradPlan &pl, const void *grad_out, const void *input, void *grad_weight,
-                              float *workspace, hipStream_t stream) {
+hipError_t launch_block_wgrad(const BlockWgradPlan &pl, const void *grad_out, const void *input, float *workspace,
+                              hipStream_t stream) {
   hipError_t e = hipErrorInvalidValue;
 #define MELLIN_BW_CASE(MT_, NT_)                                                                    \
   if (pl.mt == MT_ && pl.nt == NT_) {                                                               \
@@ -425,19 +373,7 @@ hipError_t launch_block_wgrad(const BlockWgradPlan &pl, const void *grad_out, co
   MELLIN_BW_CASE(2, 3)
   MELLIN_BW_CASE(2, 4)
 #undef MELLIN_BW_CASE
-  if (e != hipSuccess) return e;
-  const unsigned blocks = (unsigned)(pl.nfx * pl.c_blocks * pl.ctb * pl.nfy * pl.M);
-  if (pl.f16)
-    hipLaunchKernelGGL(block_wgrad_reduce_kernel<_Float16>, dim3(blocks), dim3(256), 0, stream, pl, workspace, (_Float16 *)grad_weight);
-  else
-    hipLaunchKernelGGL(block_wgrad_reduce_kernel<float>, dim3(blocks), dim3(256), 0, stream, pl, workspace, (float *)grad_weight);
-  e = hipGetLastError();
-  if (e != hipSuccess || pl.nfy == pl.f_pitch) return e;
-  const i64 n = (i64)pl.M * pl.C * pl.nfx * pl.f_pitch;
-  const dim3 grid((unsigned)std::min<i64>((n + 255) / 256, 4096));
-  if (pl.f16) hipLaunchKernelGGL(block_wgrad_zero_kernel<_Float16>, grid, dim3(256), 0, stream, pl, (_Float16 *)grad_weight);
-  else hipLaunchKernelGGL(block_wgrad_zero_kernel<float>, grid, dim3(256), 0, stream, pl, (float *)grad_weight);
-  return hipGetLastError();
+  return e;
 }
 
 }  // namespace mellin

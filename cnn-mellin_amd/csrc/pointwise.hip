@@ -15,7 +15,6 @@
 // A thread owns one (t, inner) column of the (T, inner) plane and walks down the
 // outer axis: the power (t + 1)^tau, the only expensive function, is evaluated
 // once per thread, and consecutive threads touch consecutive words.
-#include "block_gemm.hpp"
 #include "mellin_common.hpp"
 
 namespace mellin {
@@ -253,16 +252,6 @@ hipError_t launch_bias_grad(const T *grad_out, const T *out, i64 batch, i64 chan
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(bias_reduce_kernel<T>, dim3((unsigned)channels), dim3(64), 0, stream, workspace, batch * chunks,
                      grad_bias);
-  return hipGetLastError();
-}
-hipError_t launch_bias_reduce(const float *partial, i64 per_channel, i64 channels, void *grad_bias, bool f16,
-                              hipStream_t stream) {
-  if (f16)
-    hipLaunchKernelGGL(bias_reduce_kernel<_Float16>, dim3((unsigned)channels), dim3(64), 0, stream, partial, per_channel,
-                       (_Float16 *)grad_bias);
-  else
-    hipLaunchKernelGGL(bias_reduce_kernel<float>, dim3((unsigned)channels), dim3(64), 0, stream, partial, per_channel,
-                       (float *)grad_bias);
   return hipGetLastError();
 }
 

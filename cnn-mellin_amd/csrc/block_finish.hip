@@ -13,6 +13,7 @@ namespace mellin {
 namespace {
 
 constexpr int kFinishThreads = 256;
+constexpr int kFinishTaps = 64;
 constexpr int kSliceValues = kFinishThreads * 4;       // values of a tile that a block adds up
 
 struct FinishArgs {
@@ -20,7 +21,7 @@ struct FinishArgs {
   const float *w_partial;
   void *gw;
   unsigned w_blocks, w_zero_blocks;
-  int w_pairs;
+  int w_taps;
   const float *b_partial;
   void *gb;
   i64 b_count;
@@ -70,47 +71,47 @@ __device__ void finish_weight(const BlockWgradPlan &pl, const float *__restrict_
   }
 }
 
-// The same for weights that are many and have few slices (few: less than 16; a block per 32 weights would mostly wait):
-// a block owns eight output channels and 32 input channels, a thread all taps of one pair, which lie side by side in gw.
+// The same for weights that are many and have few slices (less than 16 on average: a block per 32 weights would mostly wait, and write 4 bytes of
+// every line): a block owns an output channel and 32 input channels with all their taps, which it writes side by side.
 template <typename T>
-__device__ void finish_weight_pairs(const BlockWgradPlan &pl, const float *__restrict__ ws, T *__restrict__ gw, int b) {
-  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.wm * pl.mt * 32, c_tiles = (pl.C + 31) / 32;
-  const int mt8 = b / c_tiles, ct_all = b - mt8 * c_tiles;
-  const int m = mt8 * 8 + (threadIdx.x >> 5), c = ct_all * 32 + (threadIdx.x & 31);
-  if (m >= pl.M || c >= pl.C) return;
+__device__ void finish_weight_taps(const BlockWgradPlan &pl, const float *__restrict__ ws, T *__restrict__ gw, int b, float (*sum)[33]) {
+  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.wm * pl.mt * 32, c_tiles = (pl.C + 31) / 32, taps = pl.nfx * pl.nfy;
+  const int m = b / c_tiles, ct_all = b - m * c_tiles, cl = threadIdx.x & 31;
   const int mb = m / m_t, ml = m - mb * m_t, cb = ct_all / pl.ctb, ct = ct_all - cb * pl.ctb;
   const int blocks = pl.m_blocks * pl.c_blocks;
   const i64 stride = (i64)blocks * m_t * cols;
-  T *out = gw + ((i64)m * pl.C + c) * pl.nfx * pl.f_pitch + pl.f_off;
-  for (int fx = 0; fx < pl.nfx; ++fx) {
+  for (int tap = threadIdx.x >> 5; tap < taps; tap += kFinishThreads / 32) {
+    const int fx = tap / pl.nfy, fy = tap - fx * pl.nfy, slices = pl.row[fx].slices;
     const float *p = ws + ((i64)pl.row[fx].slice0 * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols +
-                     ct * pl.nfy * 32 + (threadIdx.x & 31);
-    const int slices = pl.row[fx].slices;
-    int fy = 0;
-    for (; fy + 4 <= pl.nfy; fy += 4) {
-      float v[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-      for (int k = 0; k < slices; ++k)
+                     (ct * pl.nfy + fy) * 32 + cl;
+    float s = 0.f;
+    int k = 0;
+    for (; k + 4 <= slices; k += 4) {
+      float v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] += p[k * stride + (fy + i) * 32];
+      for (int i = 0; i < 4; ++i) v[i] = p[(k + i) * stride];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) out[fx * pl.f_pitch + fy + i] = (T)v[i];
+      for (int i = 0; i < 4; ++i) s += v[i];
     }
-    for (; fy < pl.nfy; ++fy) {
-      float v = 0.f;
-      for (int k = 0; k < slices; ++k) v += p[k * stride + fy * 32];
-      out[fx * pl.f_pitch + fy] = (T)v;
-    }
+    for (; k < slices; ++k) s += p[k * stride];
+    sum[tap][cl] = s;
+  }
+  __syncthreads();
+  const int live = min(32, pl.C - ct_all * 32);
+  T *out = gw + ((i64)m * pl.C + ct_all * 32) * pl.nfx * pl.f_pitch + pl.f_off;
+  for (int i = threadIdx.x; i < live * taps; i += kFinishThreads) {
+    const int c = i / taps, tap = i - c * taps, fx = tap / pl.nfy, fy = tap - fx * pl.nfy;
+    out[(c * pl.nfx + fx) * pl.f_pitch + fy] = (T)sum[tap][c];
   }
 }
 
 template <typename T>
 __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs a) {
-  __shared__ float red[8][32];
+  __shared__ float red[8][32], taps[kFinishTaps][33];
   const int tid = threadIdx.x;
   unsigned b = blockIdx.x;
   if (b < a.w_blocks) {
-    if (a.w_pairs) finish_weight_pairs<T>(a.w, a.w_partial, (T *)a.gw, (int)b);
+    if (a.w_taps) finish_weight_taps<T>(a.w, a.w_partial, (T *)a.gw, (int)b, taps);
     else finish_weight<T>(a.w, a.w_partial, (T *)a.gw, (int)b, red);
     return;
   }
@@ -169,11 +170,9 @@ hipError_t launch_block_finish(bool f16, const BlockFinish &job, hipStream_t str
     a.w = *job.weight;
     a.w_partial = job.weight_partial;
     a.gw = job.grad_weight;
-    int most = 0;
-    for (int f = 0; f < a.w.nfx; ++f) most = std::max(most, a.w.row[f].slices);
-    a.w_pairs = most < 16 && (i64)a.w.M * a.w.C >= 1 << 14;
-    a.w_blocks = a.w_pairs ? (unsigned)((a.w.M + 7) / 8 * ((a.w.C + 31) / 32))
-                           : (unsigned)(a.w.nfx * a.w.c_blocks * a.w.ctb * a.w.nfy * a.w.M);
+    a.w_taps = a.w.slices < 16 * a.w.nfx && a.w.nfx * a.w.nfy <= kFinishTaps && (i64)a.w.M * a.w.C >= 1 << 14;
+    a.w_blocks = a.w_taps ? (unsigned)(a.w.M * ((a.w.C + 31) / 32))
+                          : (unsigned)(a.w.nfx * a.w.c_blocks * a.w.ctb * a.w.nfy * a.w.M);
     if (a.w.nfy != a.w.f_pitch)
       a.w_zero_blocks = (unsigned)(((i64)a.w.M * a.w.C * a.w.nfx * a.w.f_pitch + kFinishThreads - 1) / kFinishThreads);
   }

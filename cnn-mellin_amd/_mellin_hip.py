@@ -79,7 +79,7 @@ SYMBOLS["mellin_corr2d_forward_act_f16"] = (_int, [_int, _int, _ptr, _ptr, _ptr]
 SYMBOLS["mellin_corr2d_backward_input_f16"] = (_int, [_int, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _size_t, _ptr])
 SYMBOLS["mellin_corr2d_backward_weight_f16"] = (_int, [_int, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _size_t, _ptr])
 SYMBOLS["mellin_layer_forward_workspace"] = (_size_t, [_int, _int] + _DIMS)
-SYMBOLS["mellin_layer_forward"] = (_int, [_int, _int, _int, _ptr, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _size_t, _ptr])
+SYMBOLS["mellin_layer_forward"] = (_int, [_int, _int, _int, _ptr, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _ptr, _size_t, _ptr])
 SYMBOLS["mellin_layer_backward_workspace"] = (_size_t, [_int, _int, _int] + _DIMS)
 SYMBOLS["mellin_layer_backward"] = (_int, [_int, _int, _int] + [_ptr] * 4 + _DIMS + [_ptr] * 4 + [_size_t, _ptr])
 _dbl = ctypes.c_double

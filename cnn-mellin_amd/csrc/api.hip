@@ -1613,23 +1613,32 @@ static bool plan_block_weight(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockWg
   return lp.known[2] > 0;
 }
 
+// the elements of a layer call: 4 float, 2 half, 6 half with float parameters
+static bool layer_elements(int elem) { return elem == 2 || elem == 4 || elem == MELLIN_ELEM_HALF_FLOAT; }
+static int bad_elements(const char *who, int elem) {
+  return fail(MELLIN_ERR_ARGUMENT, "%s: elements of 2 (half) or 4 (float) bytes, or MELLIN_ELEM_HALF_FLOAT, only (got %d)", who, elem);
+}
+
 size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
-  if (elem_bytes != 2 && elem_bytes != 4) return 0;
+  if (!layer_elements(elem_bytes)) return 0;
   if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
+  const bool half = elem_bytes != 4;
   BlockPlan bp;
-  if (plan_block_forward(kind_x, elem_bytes == 2, CORR2D_ARGS, bp))
-    return blocked_region(batch, c_in, ngx * ngy, elem_bytes == 2) + align256(bp.filter_bytes) + bp.slice_bytes;
-  if (elem_bytes == 2) return mellin_corr2d_forward_f16_workspace(kind_x, CORR2D_ARGS);
-  return mellin_corr2d_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS);
+  if (plan_block_forward(kind_x, half, CORR2D_ARGS, bp))
+    return blocked_region(batch, c_in, ngx * ngy, half) + align256(bp.filter_bytes) + bp.slice_bytes;
+  if (!half) return mellin_corr2d_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS);
+  const size_t own = mellin_corr2d_forward_f16_workspace(kind_x, CORR2D_ARGS);
+  return elem_bytes == 2 ? own : align256(own) + align256(c_out * c_in * nfx * nfy * 2) + c_out * 2;
 }
 int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void *input, const void *weight,
-                         const void *bias, MELLIN_CORR2D_DIMS, void *out, void *workspace, size_t workspace_bytes,
-                         void *stream) {
+                         const void *bias, MELLIN_CORR2D_DIMS, void *out, void *weight_half, void *workspace,
+                         size_t workspace_bytes, void *stream) {
   int rc;
-  if (elem_bytes != 2 && elem_bytes != 4)
-    return fail(MELLIN_ERR_ARGUMENT, "%s: elements of 2 (half) or 4 (float) bytes only (got %d)", __func__, elem_bytes);
+  if (!layer_elements(elem_bytes)) return bad_elements(__func__, elem_bytes);
   if ((rc = check_corr2d(__func__, kind_x, CORR2D_ARGS))) return rc;
-  const bool half = elem_bytes == 2;
+  const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT;
+  const i64 n_w = c_out * c_in * nfx * nfy;
+  hipStream_t st = (hipStream_t)stream;
   BlockPlan bp;
   if (plan_block_forward(kind_x, half, CORR2D_ARGS, bp)) {
     const size_t signal = blocked_region(batch, c_in, ngx * ngy, half), filter = align256(bp.filter_bytes);
@@ -1640,20 +1649,31 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
     if (activation != MELLIN_ACT_NONE && activation != MELLIN_ACT_RELU)
       return fail(MELLIN_ERR_ARGUMENT, "%s: activation must be MELLIN_ACT_NONE or MELLIN_ACT_RELU (got %d)", __func__, activation);
     bp.relu = activation == MELLIN_ACT_RELU;
+    bp.wide = wide;
     g_variant = half ? "mfma-f16" : "mfma-blocks";
     g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
-    hipStream_t st = (hipStream_t)stream;
     char *ws = (char *)workspace;
     float *sums = (float *)(ws + signal + filter);
     const PackSignal x = {input, nullptr, ws, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
-    hipError_t e = launch_block_pack(half, &x, nullptr, &bp, (int)c_in, weight, ws + signal, st);
+    hipError_t e = launch_block_pack(half, &x, nullptr, &bp, (int)c_in, weight, ws + signal, wide ? weight_half : nullptr, n_w, st);
     if (e == hipSuccess) e = launch_block_gemm(bp, ws, ws + signal, bias, out, sums, st);
     if (e == hipSuccess && bp.rest > 0) {
       BlockFinish fin = {};
       fin.slices = &bp; fin.frag = ws + signal; fin.slice_sums = sums; fin.out = out;
-      e = launch_block_finish(half, fin, st);
+      e = launch_block_finish(half, wide, fin, st);
     }
     return check_hip(e, __func__);
+  }
+  if (wide) {
+    const size_t own = mellin_corr2d_forward_f16_workspace(kind_x, CORR2D_ARGS), copy = align256(n_w * 2), need = align256(own) + copy + c_out * 2;
+    if (!workspace || workspace_bytes < need)
+      return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, need, workspace_bytes);
+    if (!weight) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+    char *rounded = (char *)workspace + align256(own);
+    void *w_half = weight_half ? weight_half : rounded, *b_half = rounded + copy;
+    const hipError_t e = launch_cast_pair(true, weight, w_half, n_w, bias, b_half, c_out, st);
+    if (e != hipSuccess) return check_hip(e, __func__);
+    return mellin_corr2d_forward_act_f16(kind_x, activation, input, w_half, bias ? b_half : nullptr, CORR2D_ARGS, out, workspace, own, stream);
   }
   if (half)
     return mellin_corr2d_forward_act_f16(kind_x, activation, input, weight, bias, CORR2D_ARGS, out, workspace,
@@ -1667,12 +1687,13 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
 // section 2, on grad_out as it lies (through a fused ReLU: on a masked copy).
 struct LayerBackward {
   bool input_blocked, weight_blocked, plain;           // plain: some gradient takes the section-2 kernels
-  size_t masked_off, go_off, x_off, frag_off, slice_off, bias_off, wgrad_off, pass_off, pass_bytes, total;
+  size_t masked_off, go_off, x_off, frag_off, slice_off, bias_off, wgrad_off, gw_off, gb_off, pass_off, pass_bytes, total;
   BlockPlan bp;
   BlockWgradPlan wp;
 };
-static void plan_layer_backward(int kind_x, int elem, int want, MELLIN_CORR2D_DIMS, LayerBackward &lb) {
-  const bool half = elem == 2;
+static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS, LayerBackward &lb) {
+  const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT;
+  const int elem = half ? 2 : 4;
   const bool wi = want & MELLIN_WANT_INPUT, ww = want & MELLIN_WANT_WEIGHT;
   lb.input_blocked = wi && plan_block_input(kind_x, half, CORR2D_ARGS, lb.bp);
   lb.weight_blocked = ww && plan_block_weight(kind_x, half, CORR2D_ARGS, lb.wp);
@@ -1687,6 +1708,9 @@ static void plan_layer_backward(int kind_x, int elem, int want, MELLIN_CORR2D_DI
   lb.slice_off = take(lb.input_blocked ? lb.bp.slice_bytes : 0);
   lb.bias_off = take(!lb.plain && (want & MELLIN_WANT_BIAS) ? pack_partial_count(batch, c_out, nhx * nhy) * 4 : 0);
   lb.wgrad_off = take(lb.weight_blocked ? lb.wp.ws_bytes : 0);
+  // (half gradients of the parameters on their way to float)
+  lb.gw_off = take(wide && ww && !lb.weight_blocked ? (size_t)(c_out * c_in * nfx * nfy) * 2 : 0);
+  lb.gb_off = take(wide && lb.plain && (want & MELLIN_WANT_BIAS) ? (size_t)c_out * 2 : 0);
   size_t pass = 0;
   if (lb.plain && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)))   // (a ReLU's backward writes the bias gradient, asked for or not)
     pass = align256(mellin_bias_grad_workspace(batch, c_out, nhx * nhy)) + align256((size_t)c_out * elem);
@@ -1701,7 +1725,7 @@ static void plan_layer_backward(int kind_x, int elem, int want, MELLIN_CORR2D_DI
   lb.total = at;
 }
 size_t mellin_layer_backward_workspace(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS) {
-  if (elem_bytes != 2 && elem_bytes != 4) return 0;
+  if (!layer_elements(elem_bytes)) return 0;
   if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
   LayerBackward lb;
   plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb);
@@ -1711,8 +1735,7 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
                           const void *grad_out, const void *out, MELLIN_CORR2D_DIMS, void *grad_input,
                           void *grad_weight, void *grad_bias, void *workspace, size_t workspace_bytes, void *stream) {
   int rc;
-  if (elem_bytes != 2 && elem_bytes != 4)
-    return fail(MELLIN_ERR_ARGUMENT, "%s: elements of 2 (half) or 4 (float) bytes only (got %d)", __func__, elem_bytes);
+  if (!layer_elements(elem_bytes)) return bad_elements(__func__, elem_bytes);
   if ((rc = check_corr2d(__func__, kind_x, CORR2D_ARGS))) return rc;
   if (((want & MELLIN_WANT_RELU) && !out) || ((want & MELLIN_WANT_INPUT) && !grad_input) ||
       ((want & MELLIN_WANT_WEIGHT) && !grad_weight) || ((want & MELLIN_WANT_BIAS) && !grad_bias))
@@ -1722,13 +1745,13 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   if (lb.total && (!workspace || workspace_bytes < lb.total))
     return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, lb.total, workspace_bytes);
   char *ws = (char *)workspace, *pass = ws + lb.pass_off;
-  const bool half = elem_bytes == 2, relu = want & MELLIN_WANT_RELU;
+  const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT, relu = want & MELLIN_WANT_RELU;
   hipStream_t st = (hipStream_t)stream;
   hipError_t e = hipSuccess;
   if (lb.plain && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU))) {
     void *masked = relu ? ws + lb.masked_off : nullptr;
     const size_t own = mellin_bias_grad_workspace(batch, c_out, nhx * nhy);
-    void *gb = (want & MELLIN_WANT_BIAS) ? grad_bias : pass + align256(own);
+    void *gb = !(want & MELLIN_WANT_BIAS) ? pass + align256(own) : wide ? ws + lb.gb_off : grad_bias;
     rc = half ? mellin_bias_grad_f16(grad_out, masked ? out : nullptr, batch, c_out, nhx * nhy, masked, gb, pass, own, stream)
               : mellin_bias_grad_f32((const float *)grad_out, masked ? (const float *)out : nullptr, batch, c_out,
                                      nhx * nhy, (float *)masked, (float *)gb, pass, own, stream);
@@ -1742,10 +1765,17 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
     if (rc) return rc;
   }
   if ((want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked) {
-    rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, grad_weight, pass, lb.pass_bytes, stream)
+    rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, wide ? ws + lb.gw_off : grad_weight, pass,
+                                                  lb.pass_bytes, stream)
               : mellin_corr2d_backward_weight_f32(kind_x, (const float *)input, (const float *)grad_out, CORR2D_ARGS,
                                                   (float *)grad_weight, pass, lb.pass_bytes, stream);
     if (rc) return rc;
+  }
+  if (wide) {
+    const bool gw = (want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked, gb = lb.plain && (want & MELLIN_WANT_BIAS);
+    e = launch_cast_pair(false, gw ? ws + lb.gw_off : nullptr, grad_weight, c_out * c_in * nfx * nfy, gb ? ws + lb.gb_off : nullptr,
+                         grad_bias, c_out, st);
+    if (e != hipSuccess) return check_hip(e, __func__);
   }
   if (!lb.input_blocked && !lb.weight_blocked) return MELLIN_OK;
   if (!grad_out || (lb.input_blocked && !weight) || (lb.weight_blocked && !input))
@@ -1757,7 +1787,7 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
                          (int)batch, (int)c_out, (int)(nhx * nhy)};
   const PackSignal x = {input, nullptr, ws + lb.x_off, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
   e = launch_block_pack(half, &go, lb.weight_blocked ? &x : nullptr, lb.input_blocked ? &lb.bp : nullptr, (int)c_out, weight,
-                        ws + lb.frag_off, st);
+                        ws + lb.frag_off, nullptr, 0, st);
   BlockFinish fin = {};
   if (lb.input_blocked) {
     lb.bp.relu = 0;
@@ -1773,7 +1803,7 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
     fin.bias_partial = (const float *)(ws + lb.bias_off); fin.grad_bias = grad_bias;
     fin.bias_count = (i64)pack_partial_count(batch, 1, nhx * nhy); fin.channels = c_out;
   }
-  if (e == hipSuccess) e = launch_block_finish(half, fin, st);
+  if (e == hipSuccess) e = launch_block_finish(half, wide, fin, st);
   return check_hip(e, __func__);
 }
 

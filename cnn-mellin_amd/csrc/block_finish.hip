@@ -105,21 +105,21 @@ __device__ void finish_weight_taps(const BlockWgradPlan &pl, const float *__rest
   }
 }
 
-template <typename T>
+template <typename T, typename TG>                     // tensors, gradients of the parameters
 __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs a) {
   __shared__ float red[8][32], taps[kFinishTaps][33];
   const int tid = threadIdx.x;
   unsigned b = blockIdx.x;
   if (b < a.w_blocks) {
-    if (a.w_taps) finish_weight_taps<T>(a.w, a.w_partial, (T *)a.gw, (int)b, taps);
-    else finish_weight<T>(a.w, a.w_partial, (T *)a.gw, (int)b, red);
+    if (a.w_taps) finish_weight_taps<TG>(a.w, a.w_partial, (TG *)a.gw, (int)b, taps);
+    else finish_weight<TG>(a.w, a.w_partial, (TG *)a.gw, (int)b, red);
     return;
   }
   b -= a.w_blocks;
   if (b < a.w_zero_blocks) {                           // filter columns that have no tap at all: zeros
     const i64 i = (i64)b * kFinishThreads + tid;
     const int fy = (int)(i % a.w.f_pitch);
-    if (i < (i64)a.w.M * a.w.C * a.w.nfx * a.w.f_pitch && (fy < a.w.f_off || fy >= a.w.f_off + a.w.nfy)) ((T *)a.gw)[i] = (T)0;
+    if (i < (i64)a.w.M * a.w.C * a.w.nfx * a.w.f_pitch && (fy < a.w.f_off || fy >= a.w.f_off + a.w.nfy)) ((TG *)a.gw)[i] = (TG)0;
     return;
   }
   b -= a.w_zero_blocks;
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
     for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o);
     if ((tid & 63) == 0) red[0][tid >> 6] = s;
     __syncthreads();
-    if (tid == 0) ((T *)a.gb)[b] = (T)(red[0][0] + red[0][1] + red[0][2] + red[0][3]);
+    if (tid == 0) ((TG *)a.gb)[b] = (TG)(red[0][0] + red[0][1] + red[0][2] + red[0][3]);
     return;
   }
   b -= a.b_blocks;
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
 
 }  // namespace
 
-hipError_t launch_block_finish(bool f16, const BlockFinish &job, hipStream_t stream) {
+hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipStream_t stream) {
   FinishArgs a = {};
   if (job.weight) {
     a.w = *job.weight;
@@ -192,8 +192,10 @@ hipError_t launch_block_finish(bool f16, const BlockFinish &job, hipStream_t str
   }
   const i64 blocks = (i64)a.w_blocks + a.w_zero_blocks + a.b_blocks + s_blocks;
   if (blocks == 0) return hipSuccess;
-  if (f16) hipLaunchKernelGGL(block_finish_kernel<_Float16>, dim3((unsigned)blocks), dim3(kFinishThreads), 0, stream, a);
-  else hipLaunchKernelGGL(block_finish_kernel<float>, dim3((unsigned)blocks), dim3(kFinishThreads), 0, stream, a);
+  const dim3 grid((unsigned)blocks), threads(kFinishThreads);
+  if (f16 && wide) hipLaunchKernelGGL((block_finish_kernel<_Float16, float>), grid, threads, 0, stream, a);
+  else if (f16) hipLaunchKernelGGL((block_finish_kernel<_Float16, _Float16>), grid, threads, 0, stream, a);
+  else hipLaunchKernelGGL((block_finish_kernel<float, float>), grid, threads, 0, stream, a);
   return hipGetLastError();
 }
 

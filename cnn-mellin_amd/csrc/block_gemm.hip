@@ -162,7 +162,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   if (tid < M_T) {
     const int m = m_tile * M_T + tid;
     float b = 0.f;
-    if (bias && m < pl.M) b = F16 ? (float)((const _Float16 *)bias)[m] : ((const float *)bias)[m];
+    if (bias && m < pl.M) b = !F16 ? ((const float *)bias)[m] : (float)(pl.wide ? (_Float16)((const float *)bias)[m] : ((const _Float16 *)bias)[m]);
     Bs[tid] = b;
   }
 
@@ -574,6 +574,7 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   if (X.s > 4096 || X.d > 4096 || X.u > 4096 || X.p > 4096 || X.p < -lim || Y.s > 64 || Y.d > 4096 || Y.u > 64 || Y.p > lim || Y.p < -lim)
     return false;
   pl.f16 = f16;
+  pl.wide = 0;
   pl.batch = (int)pr.batch; pl.M = (int)pr.c_out; pl.CG = (int)((pr.c_in + 7) / 8);
   pl.nox = (int)X.nh; pl.noy = (int)Y.nh; pl.Q = (int)Q;
   pl.ngx = (int)X.ng; pl.ngy = (int)Y.ng; pl.plane = (int)plane;

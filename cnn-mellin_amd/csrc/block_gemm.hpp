@@ -24,6 +24,7 @@ struct BlockClass { int first, start; unsigned mask; };     // start: the class'
 
 struct BlockPlan {
   int f16;
+  int wide;                        // f16: filter and bias are float (rounded to half where they are read)
   int batch, M, CG;                // images, output channels, groups of eight contracted channels
   int nfx, nfy;                    // filter rows; filter columns (those that have taps)
   int nox, noy, Q;                 // output extent
@@ -97,9 +98,10 @@ struct PackSignal {
 };
 size_t pack_partial_count(i64 batch, i64 channels, i64 plane);
 // Everything a pass reads in one launch: up to two tensors and the filter of `pl` (f: fp32 or half, `channels`
-// contracted channels -> filter_bytes at `frag`); null for what there is not.
+// contracted channels -> filter_bytes at `frag`); null for what there is not.  `copy`: the filter's `copy_count`
+// floats, rounded to half.
 hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b, const BlockPlan *pl, int channels,
-                             const void *f, void *frag, hipStream_t stream);
+                             const void *f, void *frag, void *copy, i64 copy_count, hipStream_t stream);
 
 // The sums that end a pass, in one launch; null pointers for those there are not.
 struct BlockFinish {
@@ -114,6 +116,7 @@ struct BlockFinish {
   const float *slice_sums;
   void *out;
 };
-hipError_t launch_block_finish(bool f16, const BlockFinish &job, hipStream_t stream);
+// (wide: the gradients are float where the tensors are half)
+hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipStream_t stream);
 
 }  // namespace mellin

@@ -103,7 +103,7 @@ __device__ __forceinline__ void pack_signal(const PackPart &pt, unsigned block, 
 // column fy): the eight values of row r as part p at
 //   frag[((mt * (CG * nfx * nfy + 1) + (cg * nfx + fx) * nfy + fy) * parts + p) * 32 + r]   (16-byte words)
 // and a unit of zeros behind each tile of 32 channels.
-template <bool F16>
+template <bool F16, typename From>
 __device__ __forceinline__ void pack_filter(const BlockPlan &pl, int channels, const void *__restrict__ fv, uintx4 *__restrict__ frag,
                                             i64 idx) {
   typedef typename std::conditional<F16, _Float16, float>::type T;
@@ -116,10 +116,10 @@ __device__ __forceinline__ void pack_filter(const BlockPlan &pl, int channels, c
   const int cg = ct / taps, tap = ct - cg * taps;                      // (cg == CG: the zeros)
   const int fx = tap / pl.nfy, fy = tap - fx * pl.nfy;
   const int m = mt * 32 + r;
-  const T *f = (const T *)fv + (i64)m * pl.f_m + fx * pl.f_pitch + pl.f_off + fy;
+  const From *f = (const From *)fv + (i64)m * pl.f_m + fx * pl.f_pitch + pl.f_off + fy;
   T v[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = (m < pl.M && cg < pl.CG && cg * 8 + i < channels) ? f[(i64)(cg * 8 + i) * pl.f_c] : (T)0;
+  for (int i = 0; i < 8; ++i) v[i] = (m < pl.M && cg < pl.CG && cg * 8 + i < channels) ? (T)f[(i64)(cg * 8 + i) * pl.f_c] : (T)0;
   uintx4 *o = frag + (i64)unit * (F16 ? 32 : 96) + r;
   if constexpr (F16) {
     uintx4 w;
@@ -151,9 +151,11 @@ struct PackArgs {
   PackPart a, b;
   BlockPlan pl;
   int channels;
-  unsigned filter_blocks, row_blocks;
+  unsigned filter_blocks, row_blocks, copy_blocks;
   const void *f;
   char *frag;
+  _Float16 *copy;
+  i64 copy_count;
 };
 
 template <bool F16>
@@ -167,10 +169,18 @@ __global__ __launch_bounds__(kPackThreads) void block_pack_kernel(PackArgs args)
   }
   b -= args.row_blocks;
   if (b < args.filter_blocks) {
-    pack_filter<F16>(args.pl, args.channels, args.f, (uintx4 *)args.frag, (i64)b * kPackThreads + threadIdx.x);
+    const i64 idx = (i64)b * kPackThreads + threadIdx.x;
+    if (!F16 || args.pl.wide) pack_filter<F16, float>(args.pl, args.channels, args.f, (uintx4 *)args.frag, idx);
+    else pack_filter<F16, _Float16>(args.pl, args.channels, args.f, (uintx4 *)args.frag, idx);
     return;
   }
   b -= args.filter_blocks;
+  if (b < args.copy_blocks) {
+    const i64 at = ((i64)b * kPackThreads + threadIdx.x) * 4;
+    for (i64 i = at; i < min(at + 4, args.copy_count); ++i) args.copy[i] = (_Float16)((const float *)args.f)[i];
+    return;
+  }
+  b -= args.copy_blocks;
   const bool second = b >= args.a.blocks;
   const PackPart &pt = second ? args.b : args.a;
   if (second) b -= args.a.blocks;
@@ -203,7 +213,7 @@ size_t pack_partial_count(i64 batch, i64 channels, i64 plane) {
 }
 
 hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b, const BlockPlan *pl, int channels,
-                             const void *f, void *frag, hipStream_t stream) {
+                             const void *f, void *frag, void *copy, i64 copy_count, hipStream_t stream) {
   PackArgs args = {};
   if (!pack_part(a, args.a) || !pack_part(b, args.b)) return hipErrorInvalidValue;
   if (pl) {
@@ -215,7 +225,12 @@ hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b,
     args.filter_blocks = (unsigned)((total + kPackThreads - 1) / kPackThreads);
     if (pl->kind_x == AX_MCORR || pl->kind_x == AX_MCONV) args.row_blocks = (unsigned)((pl->nox + kPackThreads - 1) / kPackThreads);
   }
-  const unsigned blocks = args.row_blocks + args.filter_blocks + args.a.blocks + args.b.blocks;
+  if (copy) {
+    args.copy = (_Float16 *)copy;
+    args.copy_count = copy_count;
+    args.copy_blocks = (unsigned)((copy_count + 4 * kPackThreads - 1) / (4 * kPackThreads));
+  }
+  const unsigned blocks = args.row_blocks + args.filter_blocks + args.copy_blocks + args.a.blocks + args.b.blocks;
   if (f16) hipLaunchKernelGGL(block_pack_kernel<true>, dim3(blocks), dim3(kPackThreads), 0, stream, args);
   else hipLaunchKernelGGL(block_pack_kernel<false>, dim3(blocks), dim3(kPackThreads), 0, stream, args);
   return hipGetLastError();

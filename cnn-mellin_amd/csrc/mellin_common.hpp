@@ -189,5 +189,7 @@ hipError_t launch_pool_pairs_backward(const T *gy, const unsigned char *which, i
 // half <-> float copies of n elements (16 bytes at a time when both buffers are 16-byte aligned)
 hipError_t launch_half_to_float(const void *src, float *dst, i64 n, hipStream_t stream);
 hipError_t launch_float_to_half(const float *src, void *dst, i64 n, hipStream_t stream);
+// two arrays (either may be null) float -> half or back
+hipError_t launch_cast_pair(bool to_half, const void *a, void *to_a, i64 na, const void *b, void *to_b, i64 nb, hipStream_t stream);
 
 }  // namespace mellin

@@ -15,6 +15,8 @@
 // A thread owns one (t, inner) column of the (T, inner) plane and walks down the
 // outer axis: the power (t + 1)^tau, the only expensive function, is evaluated
 // once per thread, and consecutive threads touch consecutive words.
+#include <algorithm>
+
 #include "mellin_common.hpp"
 
 namespace mellin {
@@ -406,6 +408,31 @@ hipError_t launch_float_to_half(const float *src, void *dst, i64 n, hipStream_t 
   const bool vec = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
   hipLaunchKernelGGL(float_to_half_kernel, dim3((unsigned)blocks), dim3(kPwThreads), 0, stream, src,
                      (_Float16 *)dst, n, vec);
+  return hipGetLastError();
+}
+
+// a layer's weight and bias (or their gradients) in one launch
+namespace {
+template <typename From, typename To>
+__global__ __launch_bounds__(kPwThreads) void cast_pair_kernel(const From *__restrict__ a, To *__restrict__ to_a, i64 na,
+                                                               const From *__restrict__ b, To *__restrict__ to_b, i64 nb) {
+  for (i64 i = (i64)blockIdx.x * kPwThreads + threadIdx.x; i < na + nb; i += (i64)gridDim.x * kPwThreads) {
+    if (i < na) to_a[i] = (To)a[i];
+    else to_b[i - na] = (To)b[i - na];
+  }
+}
+}  // namespace
+hipError_t launch_cast_pair(bool to_half, const void *a, void *to_a, i64 na, const void *b, void *to_b, i64 nb, hipStream_t stream) {
+  if (!a) na = 0;
+  if (!b) nb = 0;
+  if (na + nb == 0) return hipSuccess;
+  const dim3 grid((unsigned)std::min<i64>((na + nb + kPwThreads - 1) / kPwThreads, 2048));
+  if (to_half)
+    hipLaunchKernelGGL((cast_pair_kernel<float, _Float16>), grid, dim3(kPwThreads), 0, stream, (const float *)a, (_Float16 *)to_a, na,
+                       (const float *)b, (_Float16 *)to_b, nb);
+  else
+    hipLaunchKernelGGL((cast_pair_kernel<_Float16, float>), grid, dim3(kPwThreads), 0, stream, (const _Float16 *)a, (float *)to_a, na,
+                       (const _Float16 *)b, (float *)to_b, nb);
   return hipGetLastError();
 }
 

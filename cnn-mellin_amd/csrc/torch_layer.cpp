@@ -51,6 +51,8 @@ Tensor scratch(const Tensor &like, size_t bytes) {
 struct Corr2dBackward : public torch::autograd::Node {
   Geometry g;
   bool relu = false, has_bias = false;
+  int elem = 4;                          // as the library's entry points take it
+  at::ScalarType param_kind = at::kFloat;
   torch::autograd::SavedVariable input_, weight_, out_;
   std::vector<int64_t> out_sizes;
   at::TensorOptions options;
@@ -79,10 +81,9 @@ struct Corr2dBackward : public torch::autograd::Node {
     Tensor grad_input, grad_weight, grad_bias;
     int want = relu ? MELLIN_WANT_RELU : 0;
     if (task_should_compute_output(0)) { want |= MELLIN_WANT_INPUT; grad_input = at::empty_like(input, at::MemoryFormat::Contiguous); }
-    if (task_should_compute_output(1)) { want |= MELLIN_WANT_WEIGHT; grad_weight = at::empty_like(weight, at::MemoryFormat::Contiguous); }
-    if (has_bias && task_should_compute_output(2)) { want |= MELLIN_WANT_BIAS; grad_bias = at::empty({g.c_out}, weight.options()); }
+    if (task_should_compute_output(1)) { want |= MELLIN_WANT_WEIGHT; grad_weight = at::empty(weight.sizes(), weight.options().dtype(param_kind)); }
+    if (has_bias && task_should_compute_output(2)) { want |= MELLIN_WANT_BIAS; grad_bias = at::empty({g.c_out}, weight.options().dtype(param_kind)); }
     if (want & ~MELLIN_WANT_RELU) {
-      const int elem = (int)input.element_size();
       const size_t need = mellin_layer_backward_workspace(g.kind, elem, want, GEOMETRY_ARGS(g));
       Tensor ws = scratch(input, need);
       check(mellin_layer_backward(g.kind, elem, want, pointer(input), pointer(weight), pointer(grad_out), pointer(out),
@@ -187,20 +188,28 @@ PyObject *corr(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     const c10::OptionalDeviceGuard guard(device);
     const bool differentiable =
         at::GradMode::is_enabled() && (input0.requires_grad() || weight0.requires_grad() || (bias0.defined() && bias0.requires_grad()));
-    Tensor input, weight, bias;
+    // half tensors of a layer with float parameters: the library rounds them, and keeps the rounded weight for the backward
+    const bool wide = kind_of == at::kHalf && weight0.scalar_type() == at::kFloat && (!bias0.defined() || bias0.scalar_type() == at::kFloat);
+    const int elem = wide ? MELLIN_ELEM_HALF_FLOAT : kind_of == at::kHalf ? 2 : 4;
+    Tensor input, weight, bias, weight_half;
     {
       at::AutoGradMode no_grad(false);
       input = input0.scalar_type() == kind_of ? input0.contiguous() : input0.to(kind_of).contiguous();
-      weight = weight0.scalar_type() == kind_of ? weight0.contiguous() : weight0.to(kind_of).contiguous();
-      if (bias0.defined()) bias = bias0.scalar_type() == kind_of ? bias0.contiguous() : bias0.to(kind_of).contiguous();
+      if (wide) {
+        weight = weight0.contiguous();
+        if (bias0.defined()) bias = bias0.contiguous();
+        if (differentiable) weight_half = at::empty(weight.sizes(), input.options());
+      } else {
+        weight = weight0.scalar_type() == kind_of ? weight0.contiguous() : weight0.to(kind_of).contiguous();
+        if (bias0.defined()) bias = bias0.scalar_type() == kind_of ? bias0.contiguous() : bias0.to(kind_of).contiguous();
+      }
       out = dims == 2 ? at::empty({g.batch, g.c_out, g.nh[0], g.nh[1]}, input.options())
                       : at::empty({g.batch, g.c_out, g.nh[0]}, input.options());
-      const int elem = (int)input.element_size();
       const size_t need = mellin_layer_forward_workspace(g.kind, elem, GEOMETRY_ARGS(g));
       Tensor ws = scratch(input, need);
       check(mellin_layer_forward(g.kind, elem, relu ? MELLIN_ACT_RELU : MELLIN_ACT_NONE, pointer(input), pointer(weight),
-                                 pointer(bias), GEOMETRY_ARGS(g), out.data_ptr(), ws.defined() ? ws.data_ptr() : nullptr,
-                                 need, launch_stream(input)));
+                                 pointer(bias), GEOMETRY_ARGS(g), out.data_ptr(),
+                                 weight_half.defined() ? weight_half.data_ptr() : nullptr, ws.defined() ? ws.data_ptr() : nullptr, need, launch_stream(input)));
     }
     if (differentiable) {
       auto node = std::shared_ptr<Corr2dBackward>(new Corr2dBackward(), torch::autograd::deleteNode);
@@ -209,7 +218,9 @@ PyObject *corr(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
       node->relu = relu;
       node->has_bias = bias0.defined();
       node->input_ = torch::autograd::SavedVariable(input, false);
-      node->weight_ = torch::autograd::SavedVariable(weight, false);
+      node->weight_ = torch::autograd::SavedVariable(wide ? weight_half : weight, false);
+      node->elem = elem;
+      node->param_kind = wide ? at::kFloat : kind_of;
       node->out_sizes = out.sizes().vec();
       node->options = out.options();
       torch::autograd::set_history(out, node);

@@ -401,7 +401,11 @@ int mellin_pool_pairs_backward_f16(const void *grad_y, const unsigned char *whic
 /* ------------------------------------------------------------------------
  * 5. Whole passes of a layer in one call: what a training framework's layer needs in its
  * forward and in its backward pass, on float (elem_bytes 4) or half (elem_bytes 2) tensors,
- * with the layouts of section 2.  The backward call works out whichever gradients `want`
+ * with the layouts of section 2.  MELLIN_ELEM_HALF_FLOAT: half tensors of a layer whose parameters
+ * are float (mixed-precision training): the forward call takes a float weight and bias, rounds
+ * them to half and leaves the weight so rounded in `weight_half` (which may be null, as it is
+ * with the other element sizes); the backward call takes that copy and writes float
+ * gradients of weight and bias, from the float sums.  The backward call works out whichever gradients `want`
  * names; MELLIN_WANT_RELU says that the forward pass applied MELLIN_ACT_RELU, `out` being
  * its result.  Knowing all that is asked for, it shares between the gradients what they
  * have in common, so it may be faster than the calls of sections 2 and 4 one by one.
@@ -412,10 +416,12 @@ int mellin_pool_pairs_backward_f16(const void *grad_y, const unsigned char *whic
 #define MELLIN_WANT_WEIGHT 2
 #define MELLIN_WANT_BIAS 4
 #define MELLIN_WANT_RELU 8
+#define MELLIN_ELEM_HALF_FLOAT 6
 size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS);
 int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void *input,
                          const void *weight, const void *bias, MELLIN_CORR2D_DIMS,
-                         void *out, void *workspace, size_t workspace_bytes, void *stream);
+                         void *out, void *weight_half, void *workspace, size_t workspace_bytes,
+                         void *stream);
 size_t mellin_layer_backward_workspace(int kind_x, int elem_bytes, int want,
                                        MELLIN_CORR2D_DIMS);
 int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *input,

@@ -29,13 +29,14 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("kinds", [(np.float32, np.float32), (np.float16, np.float16), (np.float16, np.float32)], ids=["f32", "f16", "amp"])
 @pytest.mark.parametrize("relu", [False, True], ids=["plain", "relu"])
 @pytest.mark.parametrize("case", CASES, ids=[str(i) for i in range(len(CASES))])
-def test_blocked_layers_match_checker(case, half, relu):
+def test_blocked_layers_match_checker(case, kinds, relu):
     op, n, c_in, c_out, nf, ng, s, d, p, r = case
     rng = np.random.default_rng(5100 + CASES.index(case))
-    kind = np.float16 if half else np.float32
+    kind, param_kind = kinds                           # tensors; parameters (float ones under autocast: rounded to half)
+    half = kind is np.float16
     x = rng.standard_normal((n, c_in) + ng).astype(kind)
     w = (rng.standard_normal((c_out, c_in) + nf) * (c_in * nf[0] * nf[1]) ** -0.5).astype(kind)
     b = rng.standard_normal(c_out).astype(kind)
@@ -45,9 +46,10 @@ def test_blocked_layers_match_checker(case, half, relu):
     exp = fwd(x64, w64, b.astype(np.float64), s, d, p, (1, 1), r)
     nh = exp.shape[2:]
     go = rng.standard_normal(exp.shape).astype(kind)
-    xg, wg, bg = (to_gpu(a).requires_grad_() for a in (x, w, b))
+    xg, wg, bg = (to_gpu(a).requires_grad_() for a in (x, w.astype(param_kind), b.astype(param_kind)))
     call = mconv._ext_mcorrlcorr if op == "mcorr" else mconv._ext_lcorrlcorr
-    out = call(xg, wg, bg, s, d, p, (1, 1), r, activation="relu" if relu else None)
+    with torch.autocast("cuda", torch.float16, enabled=kind is not param_kind):
+        out = call(xg, wg, bg, s, d, p, (1, 1), r, activation="relu" if relu else None)
     assert hip.last_variant() == ("mfma-f16" if half else "mfma-blocks")
     out.backward(to_gpu(go))
     assert hip.last_variant() == ("mfma-f16" if half else "mfma-blocks")
@@ -81,7 +83,7 @@ def test_blocked_passes_repeat_bit_for_bit_and_replay_in_a_graph():
 
     def both():
         st = hip._stream(x.device)
-        hip._check(hip.lib.mellin_layer_forward(hip.AX_MCORR, 4, 0, hip._dp(x), hip._dp(w), None, *dims, hip._dp(out), hip._dp(ws), nf, st))
+        hip._check(hip.lib.mellin_layer_forward(hip.AX_MCORR, 4, 0, hip._dp(x), hip._dp(w), None, *dims, hip._dp(out), None, hip._dp(ws), nf, st))
         hip._check(hip.lib.mellin_layer_backward(hip.AX_MCORR, 4, want, hip._dp(x), hip._dp(w), hip._dp(go), None, *dims, hip._dp(gi),
                                                  hip._dp(gw), hip._dp(gb), hip._dp(ws), nb, st))
     both()
@@ -109,10 +111,10 @@ def test_layer_entry_points_refuse_what_they_cannot_do():
     assert need > 0
     ws = torch.empty(need, dtype=torch.uint8, device="cuda")
     call = hip.lib.mellin_layer_forward
-    assert call(hip.AX_LCORR, 8, 0, hip._dp(x), hip._dp(w), None, *dims, hip._dp(out), hip._dp(ws), need, None) == 1
-    assert call(hip.AX_LCORR, 4, 0, hip._dp(x), hip._dp(w), None, *dims, hip._dp(out), hip._dp(ws), need - 1, None) == 3
-    assert call(hip.AX_LCORR, 4, 7, hip._dp(x), hip._dp(w), None, *dims, hip._dp(out), hip._dp(ws), need, None) == 1
-    assert call(hip.AX_LCORR, 4, 0, None, hip._dp(w), None, *dims, hip._dp(out), hip._dp(ws), need, None) == 1
+    assert call(hip.AX_LCORR, 8, 0, hip._dp(x), hip._dp(w), None, *dims, hip._dp(out), None, hip._dp(ws), need, None) == 1
+    assert call(hip.AX_LCORR, 4, 0, hip._dp(x), hip._dp(w), None, *dims, hip._dp(out), None, hip._dp(ws), need - 1, None) == 3
+    assert call(hip.AX_LCORR, 4, 7, hip._dp(x), hip._dp(w), None, *dims, hip._dp(out), None, hip._dp(ws), need, None) == 1
+    assert call(hip.AX_LCORR, 4, 0, None, hip._dp(w), None, *dims, hip._dp(out), None, hip._dp(ws), need, None) == 1
     back = hip.lib.mellin_layer_backward
     assert back(hip.AX_LCORR, 4, hip_want_input := 1, hip._dp(x), hip._dp(w), hip._dp(out), None, *dims, None, None, None, None, 0, None) == 1
     nb = hip.lib.mellin_layer_backward_workspace(hip.AX_LCORR, 4, hip_want_input, *dims)

@@ -1579,11 +1579,27 @@ static LayerPlans &layer_plans(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
   }
   return p.plans;
 }
-static bool blocks_apply(bool half, MELLIN_CORR2D_DIMS) {
-  return blocks_allowed(half) && c_in >= 16 && batch * c_out * nhx * nhy != 0;
+// Layers with few channels leave most of a channel block empty, and have kernels of their own in section 2.  Measured over
+// 80 layers with 1 to 15 input channels: for the gradients of short layers, bound by launches (up to these
+// multiply-adds of whole blocks), the blocked kernels' four launches beat section 2's six to eight 1.2 to 3 times; on
+// longer half-precision layers on linear axes from eight channels on, so does the input gradient alone (1.8 to 3.9 times).
+// A forward pass is one launch there and two here, and pays only for long Mellin layers of half tensors (1.2 to 2 times).
+constexpr double kShortLayerHalf = 4e9, kShortLayerFloat = 0.08e9;
+enum { PASS_FORWARD, PASS_INPUT, PASS_WEIGHT };
+static bool blocks_apply(int pass, int kind_x, bool half, MELLIN_CORR2D_DIMS) {
+  if (!blocks_allowed(half) || batch * c_out * nhx * nhy * c_in == 0) return false;
+  if (c_in >= 16) return true;
+  auto up = [](i64 v, i64 to) { return (double)((v + to - 1) / to * to); };
+  const double taps = (double)nfx * nfy, in = (double)batch * ngx * ngy, out = (double)batch * nhx * nhy;
+  if (pass == PASS_FORWARD)
+    return half && kind_x == AX_MCORR && c_in >= 8 && out * up(c_out, 32) * up(c_in, 8) * taps >= 0.5e9;
+  const double most = std::max(in * 32 * up(c_out, 8), out * 32 * up(c_out, 32)) * taps;
+  const double few = kind_x == AX_LCORR && c_in <= 3 && c_out <= 64 ? 0.25 : 1;     // (the streaming kernels' own class)
+  if (most <= few * (half ? kShortLayerHalf : kShortLayerFloat)) return true;
+  return pass == PASS_INPUT && half && kind_x == AX_LCORR && c_in >= 8 && nfx * nfy <= 16;
 }
 static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp) {
-  if (!blocks_apply(half, CORR2D_ARGS)) return false;
+  if (!blocks_apply(PASS_FORWARD, kind_x, half, CORR2D_ARGS)) return false;
   LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
   if (!lp.known[0]) {
     SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
@@ -1594,7 +1610,7 @@ static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockP
   return lp.known[0] > 0;
 }
 static bool plan_block_input(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp) {
-  if (!blocks_apply(half, CORR2D_ARGS)) return false;
+  if (!blocks_apply(PASS_INPUT, kind_x, half, CORR2D_ARGS)) return false;
   LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
   if (!lp.known[1]) {
     SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
@@ -1605,7 +1621,7 @@ static bool plan_block_input(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPla
   return lp.known[1] > 0;
 }
 static bool plan_block_weight(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockWgradPlan &wp) {
-  if (!blocks_apply(half, CORR2D_ARGS)) return false;
+  if (!blocks_apply(PASS_WEIGHT, kind_x, half, CORR2D_ARGS)) return false;
   LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
   if (!lp.known[2])
     lp.known[2] = make_block_wgrad_plan(forward_problem(kind_x, CORR2D_ARGS), half, lp.weight) && lp.weight.ws_bytes <= kMaxWorkspaceBytes ? 1 : -1;

@@ -20,6 +20,12 @@ import torch
 import mconv
 import _mellin_hip as _hip
 
+_native_stack = _hip.native.stack
+# hooks that PyTorch runs for every module
+_GLOBAL_HOOKS = [getattr(torch.nn.modules.module, name) for name in (
+    "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks", "_global_backward_pre_hooks")
+    if hasattr(torch.nn.modules.module, name)]
+
 __all__ = ["ConvStackParams", "ConvStack", "FrameClassifier", "layer_plan", "pack_windows"]
 
 
@@ -146,6 +152,8 @@ class ConvStack(torch.nn.Module):
                                   d=lay["d"], p=lay["p"], r=lay["r"]))
         if params.seed is not None:
             self.reset_parameters()
+        # (a pool behind the last layer stays outside the call of the whole stack)
+        self._pools = [bool(lay["pool"]) for lay in self.plan[:-1]] + [False]
 
     @property
     def out_channels(self) -> int:
@@ -161,10 +169,29 @@ class ConvStack(torch.nn.Module):
         for conv in self.convs:
             conv.reset_parameters()
 
+    def _plain(self) -> bool:
+        """Whether calling the layers one by one would run nothing but them: no hooks, no replaced modules."""
+        if any(_GLOBAL_HOOKS):
+            return False
+        cls = mconv.MCorrLCorr if self.params.mellin else mconv.LCorrLCorr
+        for conv in self.convs:
+            d = conv.__dict__
+            if (type(conv) is not cls or "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or
+                    d["_backward_hooks"] or d["_backward_pre_hooks"]):
+                return False
+        return len(self.convs) == len(self._pools)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # ReLU, the reference's default (models.py:96-101), is applied by the convolution
         # kernel itself on the way out; any other callable runs as a pass of its own
         fused = self.params.nonlinearity in (torch.relu, torch.nn.functional.relu)
+        if fused and x.is_cuda and self._plain():
+            # the whole stack in one call, its tensors in the kernels' layout from layer to layer
+            kind = _hip.AX_MCORR if self.params.mellin else _hip.AX_LCORR
+            y = _native_stack(kind, x, [(conv.weight, conv.bias, conv.s, conv.d, conv.p, conv.r, pool)
+                                         for conv, pool in zip(self.convs, self._pools)])
+            if y is not None:
+                return freq_max_pool(y) if self.plan[-1]["pool"] else y
         for lay, conv in zip(self.plan, self.convs):
             x = conv(x, activation="relu") if fused else self.params.nonlinearity(conv(x))
             if lay["pool"]:

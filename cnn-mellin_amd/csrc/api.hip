@@ -1671,11 +1671,13 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
     char *ws = (char *)workspace;
     float *sums = (float *)(ws + signal + filter);
     const PackSignal x = {input, nullptr, ws, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
-    hipError_t e = launch_block_pack(half, &x, nullptr, &bp, (int)c_in, weight, ws + signal, wide ? weight_half : nullptr, n_w, st);
-    if (e == hipSuccess) e = launch_block_gemm(bp, ws, ws + signal, bias, out, sums, st);
+    const PackFilter f = pack_filter(bp, (int)c_in, weight, ws + signal, wide ? weight_half : nullptr, n_w);
+    hipError_t e = launch_block_pack(half, &x, nullptr, &f, 1, st);
+    const BlockGemmArgs args = {ws, ws + signal, bias, out, sums, false, false, nullptr, nullptr};
+    if (e == hipSuccess) e = launch_block_gemm(bp, args, st);
     if (e == hipSuccess && bp.rest > 0) {
       BlockFinish fin = {};
-      fin.slices = &bp; fin.frag = ws + signal; fin.slice_sums = sums; fin.out = out;
+      fin.slices = &bp; fin.args = args;
       e = launch_block_finish(half, wide, fin, st);
     }
     return check_hip(e, __func__);
@@ -1802,14 +1804,14 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   const PackSignal go = {grad_out, relu && !lb.plain ? out : nullptr, ws + lb.go_off, sums ? (float *)(ws + lb.bias_off) : nullptr,
                          (int)batch, (int)c_out, (int)(nhx * nhy)};
   const PackSignal x = {input, nullptr, ws + lb.x_off, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
-  e = launch_block_pack(half, &go, lb.weight_blocked ? &x : nullptr, lb.input_blocked ? &lb.bp : nullptr, (int)c_out, weight,
-                        ws + lb.frag_off, nullptr, 0, st);
+  const PackFilter f = lb.input_blocked ? pack_filter(lb.bp, (int)c_out, weight, ws + lb.frag_off, nullptr, 0) : PackFilter{};
+  e = launch_block_pack(half, &go, lb.weight_blocked ? &x : nullptr, &f, lb.input_blocked, st);
   BlockFinish fin = {};
   if (lb.input_blocked) {
     lb.bp.relu = 0;
-    fin.slices = &lb.bp; fin.frag = ws + lb.frag_off; fin.slice_sums = (float *)(ws + lb.slice_off); fin.out = grad_input;
-    if (e == hipSuccess)
-      e = launch_block_gemm(lb.bp, ws + lb.go_off, ws + lb.frag_off, nullptr, grad_input, (float *)(ws + lb.slice_off), st);
+    fin.slices = &lb.bp;
+    fin.args = {ws + lb.go_off, ws + lb.frag_off, nullptr, grad_input, (float *)(ws + lb.slice_off), false, false, nullptr, nullptr};
+    if (e == hipSuccess) e = launch_block_gemm(lb.bp, fin.args, st);
   }
   if (lb.weight_blocked) {
     fin.weight = &lb.wp; fin.weight_partial = (float *)(ws + lb.wgrad_off); fin.grad_weight = grad_weight;
@@ -1821,6 +1823,281 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   }
   if (e == hipSuccess) e = launch_block_finish(half, wide, fin, st);
   return check_hip(e, __func__);
+}
+
+
+// ---- stacks --------------------------------------------------------------------------------
+#define STACK_DIMS(l)                                                                                                   \
+  (l).dims[0], (l).dims[1], (l).dims[2], (l).dims[3], (l).dims[4], (l).dims[5], (l).dims[6], (l).dims[7], (l).dims[8],  \
+      (l).dims[9], (l).dims[10], (l).dims[11], (l).dims[12], (l).dims[13], (l).dims[14], (l).dims[15], (l).dims[16]
+
+constexpr int kStackLayers = 64;
+
+struct StackLayer {
+  i64 batch, c_in, c_out, plane, q, rows, cols;        // of the input; of the output before pooling
+  size_t x_off, which_off;                             // saved: input, blocked; which value of a pair pooled into it
+  size_t frag_off;                                     // backward workspace: filter of the input gradient
+};
+// Where everything lies.  saved: the layers' blocked inputs, from the second layer on (without training two regions in
+// turn) and the poolings' choices.
+struct StackPlan {
+  StackLayer l[kStackLayers];
+  size_t saved, forward, backward;
+  size_t f_first, f_own, f_filters, f_unpooled, f_sums, own_bytes;                          // forward workspace
+  size_t b_grad[2], b_unpooled, b_bias[2], b_weight, b_sums, b_first, b_own, b_own_bytes;   // backward workspace
+};
+static bool plan_stack(int kind_x, int elem, bool train, int n, const mellin_stack_layer *layers, StackPlan &sp) {
+  const bool half = elem != 4;
+  if (n < 2 || n > kStackLayers) return false;
+  size_t saved = 0, in_turn[2] = {0, 0}, frags = 0, unpooled = 0, sums = 0;
+  size_t grad[2] = {0, 0}, b_unpooled = 0, bias[2] = {0, 0}, weight = 0, b_frags = 0, b_sums = 0;
+  auto region = [&](i64 channels, i64 plane, i64 batch) { return align256(blocked_bytes(batch, channels, plane, half)); };
+  for (int i = 0; i < n; ++i) {
+    const mellin_stack_layer &ly = layers[i];
+    StackLayer &l = sp.l[i];
+    if (check_corr2d(__func__, kind_x, STACK_DIMS(ly))) return false;
+    l.batch = ly.dims[0]; l.c_in = ly.dims[1]; l.c_out = ly.dims[2];
+    l.plane = ly.dims[5] * ly.dims[6]; l.rows = ly.dims[7]; l.cols = ly.dims[8]; l.q = l.rows * l.cols;
+    if (l.batch < 1 || l.batch > 65535 || l.c_out < 1 || l.c_out > 65535 || l.plane < 1 || l.q < 1 || l.batch != layers[0].dims[0]) return false;
+    if (ly.pool && (i == 0 || i == n - 1)) return false;
+    if (i == 0) continue;
+    const mellin_stack_layer &before = layers[i - 1];
+    if (l.c_in != before.dims[2] || ly.dims[5] != before.dims[7] || ly.dims[6] != (before.pool ? before.dims[8] / 2 : before.dims[8])) return false;
+    BlockPlan bp;
+    if (!plan_block_forward(kind_x, half, STACK_DIMS(ly), bp)) return false;
+    const size_t x = region(l.c_in, l.plane, l.batch);
+    if (train) {
+      l.x_off = saved;
+      saved += x;
+    } else {
+      in_turn[i & 1] = std::max(in_turn[i & 1], x);
+    }
+    l.which_off = saved;
+    if (train && before.pool) saved += align256((size_t)(l.batch * ((l.c_in + 7) / 8) * l.plane) * 8);
+    l.frag_off = frags;                                // (forward; the backward call lays out its own)
+    frags += align256(bp.filter_bytes);
+    sums = std::max(sums, bp.slice_bytes);
+    if (ly.pool) unpooled = std::max(unpooled, region(l.c_out, l.q, l.batch));
+    if (!train) continue;
+    BlockPlan ip;
+    BlockWgradPlan wp;
+    if (!plan_block_input(kind_x, half, STACK_DIMS(ly), ip) || !plan_block_weight(kind_x, half, STACK_DIMS(ly), wp)) return false;
+    b_frags += align256(ip.filter_bytes);
+    b_sums = std::max(b_sums, ip.slice_bytes);
+    weight = std::max(weight, wp.ws_bytes);
+    grad[i & 1] = std::max(grad[i & 1], region(l.c_out, l.q, l.batch));
+    if (before.pool) {
+      b_unpooled = std::max(b_unpooled, region(l.c_in, l.plane, l.batch));
+      bias[(i - 1) & 1] = std::max(bias[(i - 1) & 1], pool_partial_count(l.batch, l.c_in, before.dims[7], before.dims[8]) * 4);
+    } else {
+      bias[(i - 1) & 1] = std::max(bias[(i - 1) & 1], (size_t)l.c_in * ip.chan_slots * 4);
+    }
+    if (i == n - 1) bias[i & 1] = std::max(bias[i & 1], pack_partial_count(l.batch, l.c_out, l.q) * 4);
+  }
+  if (!train) {
+    for (int i = 1; i < n; ++i) sp.l[i].x_off = i & 1 ? in_turn[0] : 0;
+    saved = in_turn[0] + in_turn[1];
+  }
+  sp.saved = saved;
+  size_t at = 0;
+  auto take = [&](size_t bytes) { const size_t off = at; at += align256(bytes); return off; };
+  const StackLayer &l0 = sp.l[0];
+  const size_t first = (size_t)(l0.batch * l0.c_out * l0.q) * (half ? 2 : 4);
+  sp.f_first = take(first);
+  sp.own_bytes = mellin_layer_forward_workspace(kind_x, elem, STACK_DIMS(layers[0]));
+  sp.f_own = take(sp.own_bytes);
+  sp.f_filters = take(frags);
+  sp.f_unpooled = take(unpooled);
+  sp.f_sums = take(sums);
+  sp.forward = at;
+  at = 0;
+  sp.backward = 0;
+  if (!train) return true;
+  sp.b_grad[0] = take(grad[0]);
+  sp.b_grad[1] = take(grad[1]);
+  sp.b_unpooled = take(b_unpooled);
+  sp.b_bias[0] = take(bias[0]);
+  sp.b_bias[1] = take(bias[1]);
+  sp.b_weight = take(weight);
+  sp.b_sums = take(b_sums);
+  sp.b_first = take(first);
+  sp.b_own_bytes = mellin_layer_backward_workspace(kind_x, elem, MELLIN_WANT_INPUT | MELLIN_WANT_WEIGHT, STACK_DIMS(layers[0]));
+  sp.b_own = take(sp.b_own_bytes);
+  sp.backward = at + b_frags;
+  for (int i = 1; i < n; ++i) {
+    BlockPlan ip;
+    plan_block_input(kind_x, half, STACK_DIMS(layers[i]), ip);
+    sp.l[i].frag_off = at;                             // (with train: the backward's; mellin_stack_forward counts its own)
+    at += align256(ip.filter_bytes);
+  }
+  return true;
+}
+
+int mellin_stack_bytes(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers, size_t *saved,
+                       size_t *forward_workspace, size_t *backward_workspace) {
+  StackPlan sp;
+  if (!layer_elements(elem_bytes) || !layers || !plan_stack(kind_x, elem_bytes, train != 0, n_layers, layers, sp)) return 0;
+  *saved = sp.saved;
+  *forward_workspace = sp.forward;
+  *backward_workspace = sp.backward;
+  return 1;
+}
+
+static int stack_checks(const char *who, bool planned, const StackPlan &sp, const void *saved, size_t saved_bytes, const void *workspace,
+                        size_t workspace_bytes, size_t need) {
+  if (!planned) return fail(MELLIN_ERR_ARGUMENT, "%s: not a stack that can be run in one call (mellin_stack_bytes)", who);
+  if (!saved || saved_bytes < sp.saved) return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu saved bytes, got %zu", who, sp.saved, saved_bytes);
+  if (!workspace || workspace_bytes < need)
+    return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", who, need, workspace_bytes);
+  return MELLIN_OK;
+}
+
+int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers, const void *input,
+                         void *out, void *saved, size_t saved_bytes, void *workspace, size_t workspace_bytes, void *stream) {
+  StackPlan sp;
+  if (!layer_elements(elem_bytes)) return bad_elements(__func__, elem_bytes);
+  const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT;
+  const bool planned = layers && plan_stack(kind_x, elem_bytes, train != 0, n_layers, layers, sp);
+  int rc = stack_checks(__func__, planned, sp, saved, saved_bytes, workspace, workspace_bytes, sp.forward);
+  if (rc) return rc;
+  if (!input || !out) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  for (int i = 0; i < n_layers; ++i)
+    if (!layers[i].weight) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  char *ws = (char *)workspace, *keep = (char *)saved;
+  hipStream_t st = (hipStream_t)stream;
+  rc = mellin_layer_forward(kind_x, elem_bytes, MELLIN_ACT_RELU, input, layers[0].weight, layers[0].bias, STACK_DIMS(layers[0]),
+                            ws + sp.f_first, layers[0].weight_half, ws + sp.f_own, sp.own_bytes, stream);
+  if (rc) return rc;
+  // all filters, and the first layer's output
+  PackFilter filters[kStackLayers];
+  size_t frag_off[kStackLayers], at = sp.f_filters;
+  BlockPlan bp;
+  for (int i = 1; i < n_layers; ++i) {
+    const mellin_stack_layer &ly = layers[i];
+    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp);
+    bp.wide = wide;
+    filters[i - 1] = pack_filter(bp, (int)ly.dims[1], ly.weight, ws + at, wide ? ly.weight_half : nullptr,
+                                 ly.dims[1] * ly.dims[2] * ly.dims[3] * ly.dims[4]);
+    frag_off[i] = at;
+    at += align256(bp.filter_bytes);
+  }
+  const StackLayer &l1 = sp.l[1];
+  const PackSignal first = {ws + sp.f_first, nullptr, keep + l1.x_off, nullptr, (int)l1.batch, (int)l1.c_in, (int)l1.plane};
+  hipError_t e = launch_block_pack(half, &first, nullptr, filters, n_layers - 1, st);
+  for (int i = 1; i < n_layers && e == hipSuccess; ++i) {
+    const mellin_stack_layer &ly = layers[i];
+    const StackLayer &l = sp.l[i];
+    const bool last = i == n_layers - 1;
+    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp);
+    bp.relu = 1;
+    bp.wide = wide;
+    char *to = last ? (char *)out : ly.pool ? ws + sp.f_unpooled : keep + sp.l[i + 1].x_off;
+    const BlockGemmArgs args = {keep + l.x_off, ws + frag_off[i], ly.bias, to, (float *)(ws + sp.f_sums), !last, false, nullptr, nullptr};
+    e = launch_block_gemm(bp, args, st);
+    if (e == hipSuccess && bp.rest > 0) {
+      BlockFinish fin = {};
+      fin.slices = &bp; fin.args = args;
+      e = launch_block_finish(half, wide, fin, st);
+    }
+    if (e == hipSuccess && ly.pool)
+      e = launch_block_pool(half, to, l.batch, l.c_out, l.rows, l.cols, keep + sp.l[i + 1].x_off,
+                            train ? keep + sp.l[i + 1].which_off : nullptr, st);
+  }
+  g_variant = half ? "mfma-f16" : "mfma-blocks";
+  g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
+  return check_hip(e, __func__);
+}
+
+int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin_stack_layer *layers, const void *input, const void *out,
+                          const void *grad_out, const void *saved, size_t saved_bytes, void *grad_input, void *workspace,
+                          size_t workspace_bytes, void *stream) {
+  StackPlan sp;
+  if (!layer_elements(elem_bytes)) return bad_elements(__func__, elem_bytes);
+  const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT;
+  const bool planned = layers && plan_stack(kind_x, elem_bytes, true, n_layers, layers, sp);
+  int rc = stack_checks(__func__, planned, sp, saved, saved_bytes, workspace, workspace_bytes, sp.backward);
+  if (rc) return rc;
+  if (!input || !out || !grad_out) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  // the first layer that anything is wanted of
+  int lowest = 0;
+  if (!grad_input)
+    while (lowest < n_layers && !layers[lowest].grad_weight && !layers[lowest].grad_bias) ++lowest;
+  if (lowest == n_layers) return MELLIN_OK;
+  char *ws = (char *)workspace;
+  const char *keep = (const char *)saved;
+  hipStream_t st = (hipStream_t)stream;
+  PackFilter filters[kStackLayers];
+  int n_filters = 0;
+  BlockPlan ip;
+  for (int i = std::max(lowest + 1, 1); i < n_layers; ++i) {
+    const mellin_stack_layer &ly = layers[i];
+    const void *w = wide ? ly.weight_half : ly.weight;
+    if (!w) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+    plan_block_input(kind_x, half, STACK_DIMS(ly), ip);
+    filters[n_filters++] = pack_filter(ip, (int)ly.dims[2], w, ws + sp.l[i].frag_off, nullptr, 0);
+  }
+  const int top = n_layers - 1;
+  i64 bias_count[2] = {0, 0};                          // partial sums of a channel in either region
+  const StackLayer &lt = sp.l[top];
+  const PackSignal go = {grad_out, out, ws + sp.b_grad[top & 1], (float *)(ws + sp.b_bias[top & 1]), (int)lt.batch, (int)lt.c_out, (int)lt.q};
+  bias_count[top & 1] = (i64)pack_partial_count(lt.batch, 1, lt.q);
+  hipError_t e = launch_block_pack(half, &go, nullptr, filters, n_filters, st);
+  for (int i = top; i >= std::max(lowest, 1) && e == hipSuccess; --i) {
+    const mellin_stack_layer &ly = layers[i];
+    const StackLayer &l = sp.l[i];
+    const int here = i & 1, below = here ^ 1;
+    const bool first_dense = i == 1, pooled = layers[i - 1].pool;
+    BlockFinish fin = {};
+    BlockWgradPlan wp;
+    if (ly.grad_weight) {
+      plan_block_weight(kind_x, half, STACK_DIMS(ly), wp);
+      e = launch_block_wgrad(wp, ws + sp.b_grad[here], keep + l.x_off, (float *)(ws + sp.b_weight), st);
+      fin.weight = &wp; fin.weight_partial = (const float *)(ws + sp.b_weight); fin.grad_weight = ly.grad_weight;
+    }
+    if (ly.grad_bias) {
+      fin.bias_partial = (const float *)(ws + sp.b_bias[here]); fin.grad_bias = ly.grad_bias;
+      fin.bias_count = bias_count[here]; fin.channels = l.c_out;
+    }
+    const bool go_on = i > lowest;
+    if (go_on && e == hipSuccess) {
+      plan_block_input(kind_x, half, STACK_DIMS(ly), ip);
+      ip.relu = 0;
+      char *to = first_dense ? ws + sp.b_first : pooled ? ws + sp.b_unpooled : ws + sp.b_grad[below];
+      fin.slices = &ip;
+      fin.args = {ws + sp.b_grad[here], ws + l.frag_off, nullptr, to, (float *)(ws + sp.b_sums), !first_dense, !pooled,
+                  keep + l.x_off, (float *)(ws + sp.b_bias[below])};
+      if (!pooled) bias_count[below] = ip.chan_slots;
+      e = launch_block_gemm(ip, fin.args, st);
+    }
+    if (e == hipSuccess) e = launch_block_finish(half, wide, fin, st);
+    if (go_on && pooled && e == hipSuccess) {
+      const mellin_stack_layer &before = layers[i - 1];
+      e = launch_block_pool_grad(half, ws + sp.b_unpooled, keep + l.x_off, keep + l.which_off, l.batch, l.c_in, before.dims[7],
+                                 before.dims[8], ws + sp.b_grad[below], (float *)(ws + sp.b_bias[below]), st);
+      bias_count[below] = (i64)pool_partial_count(l.batch, 1, before.dims[7], before.dims[8]);
+    }
+  }
+  if (e != hipSuccess) return check_hip(e, __func__);
+  if (lowest == 0) {
+    const mellin_stack_layer &ly = layers[0];
+    if (ly.grad_bias) {
+      BlockFinish fin = {};
+      fin.bias_partial = (const float *)(ws + sp.b_bias[0]); fin.grad_bias = ly.grad_bias;
+      fin.bias_count = bias_count[0]; fin.channels = sp.l[0].c_out;
+      if ((e = launch_block_finish(half, wide, fin, st)) != hipSuccess) return check_hip(e, __func__);
+    }
+    const int want = (grad_input ? MELLIN_WANT_INPUT : 0) | (ly.grad_weight ? MELLIN_WANT_WEIGHT : 0);
+    if (want) {
+      const size_t own = mellin_layer_backward_workspace(kind_x, elem_bytes, want, STACK_DIMS(ly));
+      if (own > sp.b_own_bytes) return fail(MELLIN_ERR_WORKSPACE, "%s: workspace of the first layer", __func__);
+      rc = mellin_layer_backward(kind_x, elem_bytes, want, input, wide ? ly.weight_half : ly.weight, ws + sp.b_first, nullptr,
+                                 STACK_DIMS(ly), grad_input, ly.grad_weight, nullptr, ws + sp.b_own, sp.b_own_bytes, stream);
+      if (rc) return rc;
+    }
+  }
+  g_variant = half ? "mfma-f16" : "mfma-blocks";
+  g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
+  return MELLIN_OK;
 }
 
 }  // extern "C"

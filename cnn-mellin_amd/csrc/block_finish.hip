@@ -27,9 +27,8 @@ struct FinishArgs {
   i64 b_count;
   unsigned b_blocks;
   BlockPlan s;
-  const float *s_sums;
+  BlockGemmArgs sa;
   const int2 *s_rows;
-  void *out;
 };
 
 // gw[m, c, fx, fy] = the sum of its partial sums in slice order.  A block owns 32 weights that lie side by side in
@@ -105,6 +104,88 @@ __device__ void finish_weight_taps(const BlockWgradPlan &pl, const float *__rest
   }
 }
 
+// Tiles in slices whose output is blocked or passes a ReLU: a thread makes a unit (eight channels of a position); a block
+// has 256 of a tile's, the positions side by side.
+template <typename T>
+__device__ void finish_units(const FinishArgs &a, int b, float (*red)[32]) {
+  constexpr bool F16 = sizeof(T) == 2;
+  constexpr int UB = F16 ? 16 : 48;
+  const BlockPlan &pl = a.s;
+  const int m_t = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32, units = m_t / 8 * P;
+  const int chunks = (units + kFinishThreads - 1) / kFinishThreads;
+  const int tm = b / chunks, at = (b - tm * chunks) * kFinishThreads + (int)threadIdx.x;      // (tile, tile of channels), unit in it
+  const int r = tm / pl.m_tiles, g_t = at / P, p = at - g_t * P, group = (tm - r * pl.m_tiles) * (m_t / 8) + g_t;
+  const int id = pl.whole + r, qt = id / pl.batch, n = id - qt * pl.batch, q0 = qt * P, count = min(P, pl.Q - q0);
+  const bool live = at < units && group < pl.out_groups && p < count;
+  float v[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) v[c] = 0.f;
+  int q = 0;
+  if (live) {
+    const i64 slice = (i64)pl.rest * pl.m_tiles * m_t * P;
+    const float *from = a.sa.sums + (i64)tm * m_t * P + (i64)g_t * 8 * P + p;
+    for (int k = 0; k < pl.slices; ++k)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) v[c] += from[k * slice + c * P];
+    const int row = (q0 + p) / pl.noy, oy = q0 + p - row * pl.noy;
+    q = (a.s_rows ? a.s_rows[row].x : row) * pl.noy + oy;
+    const i64 unit = ((i64)n * pl.out_groups + group) * (pl.Q + 1) + q;
+    if (a.sa.grad) {
+      const uintx4 x = *(const uintx4 *)((const char *)a.sa.mask + unit * UB);
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        if (!((short)(x[c >> 1] >> (16 * (c & 1))) > 0)) v[c] = 0.f;
+    } else if (pl.relu) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) v[c] = fmaxf(v[c], 0.f);
+    }
+    if (a.sa.blocked) {
+      uintx4 *o = (uintx4 *)((char *)a.sa.out + unit * UB);
+      if constexpr (F16) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          o[0][j] = (unsigned)__builtin_bit_cast(unsigned short, (_Float16)v[2 * j]) |
+                    ((unsigned)__builtin_bit_cast(unsigned short, (_Float16)v[2 * j + 1]) << 16);
+      } else {
+        uintx4 hi, mid, lo;
+        split8(v, hi, mid, lo);
+        o[0] = hi;
+        o[1] = mid;
+        o[2] = lo;
+      }
+      if (q0 + p == pl.Q - 1) {                        // the unit of zeros behind the image
+        uintx4 *z = (uintx4 *)((char *)a.sa.out + (((i64)n * pl.out_groups + group) * (pl.Q + 1) + pl.Q) * UB);
+        const uintx4 zero = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < UB / 16; ++j) z[j] = zero;
+      }
+    } else {
+      T *o = (T *)a.sa.out + n * pl.h_n + (i64)group * 8 * pl.h_m + q;
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        if (group * 8 + c < pl.M) o[c * pl.h_m] = (T)v[c];
+    }
+  }
+  if (a.sa.grad) {
+    // channel sums of 32 positions, then of the nt * 32 (or 32) that share a place
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+#pragma unroll
+      for (int o = 16; o > 0; o >>= 1) v[c] += __shfl_xor(v[c], o);
+    const int hw = (int)threadIdx.x >> 5, each = pl.wk > 1 ? 1 : pl.nt;
+    if ((threadIdx.x & 31) == 0)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) red[c][hw] = v[c];
+    __syncthreads();
+    if ((threadIdx.x & 31) < 8 && hw % each == 0 && at < units && group < pl.out_groups) {
+      const int c = threadIdx.x & 31, slots = P / 32 / each;
+      float s = red[c][hw];
+      for (int i = 1; i < each; ++i) s += red[c][hw + i];
+      if (group * 8 + c < pl.M) a.sa.chan_sums[(i64)(group * 8 + c) * pl.chan_slots + (i64)id * slots + (p & ~31) / (32 * each)] = s;
+    }
+  }
+}
+
 template <typename T, typename TG>                     // tensors, gradients of the parameters
 __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs a) {
   __shared__ float red[8][32], taps[kFinishTaps][33];
@@ -136,6 +217,10 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
     return;
   }
   b -= a.b_blocks;
+  if (a.sa.blocked || a.sa.grad) {
+    finish_units<T>(a, (int)b, red);
+    return;
+  }
   // a block: kSliceValues values of a tile, four positions of a channel a thread, the slices in order
   const BlockPlan &pl = a.s;
   const int m_t = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32, chunks = m_t * P / kSliceValues;
@@ -144,7 +229,7 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
   const int id = pl.whole + r, qt = id / pl.batch, n = id - qt * pl.batch, q0 = qt * P, count = min(P, pl.Q - q0) - p;
   if (m >= pl.M || count <= 0) return;
   const i64 slice = (i64)pl.rest * pl.m_tiles * m_t * P;
-  const float *from = a.s_sums + (i64)tm * m_t * P + at;
+  const float *from = a.sa.sums + (i64)tm * m_t * P + at;
   float4 v = *(const float4 *)from;
 #pragma unroll 4
   for (int k = 1; k < pl.slices; ++k) {
@@ -154,7 +239,7 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
   if (pl.relu) v = make_float4(fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f));
   const float o[4] = {v.x, v.y, v.z, v.w};
   int row = (q0 + p) / pl.noy, oy = q0 + p - row * pl.noy;
-  T *out = (T *)a.out + n * pl.h_n + m * pl.h_m;
+  T *out = (T *)a.sa.out + n * pl.h_n + m * pl.h_m;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if (i < count) out[(a.s_rows ? a.s_rows[row].x : row) * pl.noy + oy] = (T)o[i];
@@ -185,10 +270,11 @@ hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipS
   i64 s_blocks = 0;
   if (job.slices && job.slices->rest > 0) {
     a.s = *job.slices;
-    a.s_sums = job.slice_sums;
-    a.out = job.out;
-    if (a.s.kind_x == AX_MCORR || a.s.kind_x == AX_MCONV) a.s_rows = (const int2 *)((const char *)job.frag + a.s.rows_off);
-    s_blocks = (i64)a.s.rest * a.s.m_tiles * (a.s.wm * a.s.mt * 32 * (kWaves / a.s.wk / a.s.wm * a.s.nt * 32) / kSliceValues);
+    a.sa = job.args;
+    if (a.s.kind_x == AX_MCORR || a.s.kind_x == AX_MCONV) a.s_rows = (const int2 *)((const char *)job.args.frag + a.s.rows_off);
+    const i64 values = (i64)a.s.wm * a.s.mt * 32 * (kWaves / a.s.wk / a.s.wm * a.s.nt * 32);
+    const i64 each = a.sa.blocked || a.sa.grad ? kFinishThreads * 8 : kSliceValues;
+    s_blocks = (i64)a.s.rest * a.s.m_tiles * ((values + each - 1) / each);
   }
   const i64 blocks = (i64)a.w_blocks + a.w_zero_blocks + a.b_blocks + s_blocks;
   if (blocks == 0) return hipSuccess;

@@ -1,525 +1,14 @@
-// Forward pass and gather-form input gradient of layers with many channels, from the
-// channel-blocked signal (block_gemm.hpp) on the bf16 / f16 matrix cores.
-//
-//   H[n, m, ox, oy] = bias[m] + sum_{fx, fy, c} F[m, c, fx, fy] * G[n, c, tap_x(ox, fx), tap_y(oy, fy)]
-//
-// The contracted index of a matrix instruction runs over CHANNELS of one tap (two groups of
-// eight), so an operand of the signal is 16 consecutive bytes of one position: one LDS read per
-// register quadruple, nothing to gather, pack or cut in the loop.  What bounded the kernel that
-// reads the tensors as they lie (tile_gemm.hip: eight LDS reads and 44 vector instructions per
-// 16 taps and 32 positions; matrix pipe 8-19 % busy on half tensors, 39-47 % on fp32) is paid
-// once per element in block_pack.hip instead of once per tap and tile of output channels.
-//
-// Tile: P = WN * NT * 32 consecutive output positions of one image x MT * 32 output channels.
-// A stage is F filter rows x G channel groups.  Its signal rows are copied by direct
-// global->LDS loads (16 bytes per lane, any source) into virtual rows as in tile_gemm.hip:
-//   Mellin axis   virtual row (filter row of the stage, output row): the row of that tap;
-//   linear axis   virtual row = coordinate ax ox + bx fx + cx, all filter rows in one stage;
-// positions without a source read the blocked tensor's unit of zeros, so nothing is cleared and
-// a buffer needs no memory of what it held.  The sources of a tile's virtual positions are worked
-// out once per tile into an LDS table.  While a stage multiplies, the next one's loads are issued
-// a few at a time between the steps.  Filter fragments come from L1 / L2 straight to registers,
-// two steps ahead: the WN wavefronts of a workgroup use the same ones at the same time.
-//
-// Mellin axes: output rows are taken in the order of the residue classes of the axis, so the rows
-// of a tile have taps for the same filter rows and only those are staged and multiplied; filter
-// rows none of whose taps lies inside the signal for the tile's rows are left out as well.
-//
-// Few tiles (one utterance, deep layers): WK = 4 wavefronts share the positions of a tile and
-// take every fourth step of a stage; their sums are added in wavefront order through LDS.
-//
-// Measured, 256 -> 256 channels, 4 x 4 taps, 16 x 100 x 41 positions, linear: fp32 1312 -> 1190 us and 107 us
-// for the cut (six bf16 products each: 1.39 PF, matrix pipe 57 % busy at 1.9 GHz, near the rate the board's
-// power allows); half, on Mellin rows, 286 -> 183 us.  One utterance (few tiles, WK = 4): 980 -> 330 us for ten layers.
+// Plans of the channel-blocked matrix kernel (block_gemm_kernel.hpp): tile shape, stages and turns of a launch, and the
+// launches that write a layer's output as it lies.  The kernel's other endings are in block_gemm_out.hip and
+// block_gemm_grad_*.hip (a translation unit each, for the time they take to compile).
 #include <algorithm>
 #include <cmath>
-#include <type_traits>
 
-#include "block_gemm.hpp"
-#include "tile_stage.hpp"
+#include "block_gemm_kernel.hpp"
 
 namespace mellin {
 
 namespace {
-
-// The plan stays in the kernel arguments and is read by scalar loads where it is used: held in
-// registers for a whole stage its fields would not fit the scalar register file.
-typedef const __attribute__((address_space(4))) BlockPlan ConstBlockPlan;
-
-struct BlockTile {
-  int n, q0, count, row_lo, rows;
-  int c_first, c_end, slot, slice; // its channel groups; in slices: place in the workspace, which slice (whole tiles: -1, 0)
-  int vx_min, vrows, units;        // linear axes: first coordinate; virtual rows and positions of the whole tile
-  unsigned long long filter_rows;  // Mellin axes: the filter rows with a tap for some row of the tile, four bits each
-  int nv;                          // how many
-};
-
-__device__ __forceinline__ int filter_row(const BlockTile &g, int j) { return (int)(g.filter_rows >> (4 * j)) & 15; }
-
-// Item `id` of the launch: the images of a position tile lie side by side, so that the position tiles
-// with the most filter rows come first for all images and every workgroup gets its share of them.
-// `rows`: the output rows in the order of their classes, with their filter rows (Mellin axes).
-template <int P>
-__device__ __forceinline__ BlockTile block_tile(ConstBlockPlan &pl, const int2 *__restrict__ rows, int id, bool mellin_x) {
-  BlockTile g;
-  g.c_first = 0;
-  g.c_end = pl.CG;
-  g.slot = -1;
-  g.slice = 0;
-  if (id >= pl.whole) {
-    const int i = id - pl.whole, r = i / pl.slices, stages = pl.CG / pl.G;
-    g.slice = i - r * pl.slices;
-    g.slot = g.slice * pl.rest + r;
-    g.c_first = g.slice * stages / pl.slices * pl.G;
-    g.c_end = (g.slice + 1) * stages / pl.slices * pl.G;
-    id = pl.whole + r;
-  }
-  const int qt = udiv(id, pl.batch, pl.mg_batch);
-  g.n = id - qt * pl.batch;
-  g.q0 = qt * P;
-  g.count = min(P, pl.Q - g.q0);
-  g.row_lo = udiv(g.q0, pl.noy, pl.mg_noy);
-  g.rows = udiv(g.q0 + g.count - 1, pl.noy, pl.mg_noy) - g.row_lo + 1;
-  g.vx_min = pl.ax * g.row_lo + pl.cx + pl.bx_min;
-  g.filter_rows = 0;
-  if (mellin_x) {
-    int mask = 0;
-    for (int r = (int)threadIdx.x & 63; r < g.rows; r += 64) mask |= rows[g.row_lo + r].y;
-    g.nv = 0;
-    for (int f = 0; f < pl.nfx; ++f)
-      if (__ballot(mask >> f & 1)) g.filter_rows |= (unsigned long long)f << (4 * g.nv++);
-    g.nv = max(g.nv, 1);                             // (no tap at all: a stage of zeros)
-    g.vrows = g.nv * g.rows;
-  } else {
-    g.nv = pl.nfx;
-    g.vrows = pl.ax * (g.rows - 1) + pl.bx_span + 1;
-  }
-  g.units = g.vrows * pl.RS;
-  return g;
-}
-
-typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
-
-// Value `I` of the four lanes that this lane belongs to; the lanes' values exchanged in pairs.
-template <int I>
-__device__ __forceinline__ int quad_lane(int v) { return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xf, 0xf, true); }
-__device__ __forceinline__ unsigned swap1(unsigned v) { return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true); }
-__device__ __forceinline__ unsigned swap2(unsigned v) { return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true); }
-
-// 4 x 4 transpose over four neighbouring lanes: lane j gets the four lanes' values v[j].
-__device__ __forceinline__ uintx4 transpose_words(const float4 &v, int lane) {
-  const unsigned a = __float_as_uint(v.x), b = __float_as_uint(v.y), c = __float_as_uint(v.z), d = __float_as_uint(v.w);
-  const bool odd = lane & 1, upper = lane & 2;
-  const unsigned a1 = swap1(a), b1 = swap1(b), c1 = swap1(c), d1 = swap1(d);     // (by every lane, so not in the selections)
-  const unsigned n0 = odd ? b1 : a, n1 = odd ? b : a1, n2 = odd ? d1 : c, n3 = odd ? d : c1;
-  const unsigned m0 = swap2(n0), m1 = swap2(n1), m2 = swap2(n2), m3 = swap2(n3);
-  return uintx4{upper ? m2 : n0, upper ? m3 : n1, upper ? n2 : m0, upper ? n3 : m1};
-}
-// the same of values rounded to half
-__device__ __forceinline__ uintx2 transpose_half(const float4 &v, int lane) {
-  auto pair = [](float lo, float hi) {
-    return (unsigned)__builtin_bit_cast(unsigned short, (_Float16)lo) | ((unsigned)__builtin_bit_cast(unsigned short, (_Float16)hi) << 16);
-  };
-  const unsigned ab = pair(v.x, v.y), cd = pair(v.z, v.w);
-  const bool odd = lane & 1, upper = lane & 2;
-  const unsigned ab2 = swap2(ab), cd2 = swap2(cd);
-  const unsigned n0 = upper ? cd2 : ab, n1 = upper ? cd : ab2;                   // two channels at positions 0/1 and 2/3
-  const unsigned sel = odd ? 0x03020706u : 0x05040100u;                          // high halves (other, own) or low halves (own, other)
-  return uintx2{__builtin_amdgcn_perm(swap1(n0), n0, sel), __builtin_amdgcn_perm(swap1(n1), n1, sel)};
-}
-
-template <int MT, int NT, int WM, int WK, bool F16, bool HOUT>
-__global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_arg, const char *__restrict__ X,
-                                                                 const char *__restrict__ AF, const void *__restrict__ bias,
-                                                                 void *__restrict__ Hv, float *__restrict__ sums) {
-  constexpr int PARTS = F16 ? 1 : 3, UB = 16 * PARTS;
-  constexpr int WN = kWaves / WK / WM, P = WN * NT * 32, M_T = WM * MT * 32;
-  constexpr int kALoads = 2 * MT * PARTS;              // fragment loads of two steps
-  extern __shared__ __align__(16) char blk_lds[];
-  ConstBlockPlan *plp = (ConstBlockPlan *)__builtin_amdgcn_kernarg_segment_ptr();
-#define pl (*plp)
-  char *bufs = blk_lds;                                                    // [2][buf_bytes]
-  float *Bs = (float *)(bufs + 2 * pl.buf_bytes);                          // [M_T]
-  int *tab = (int *)(Bs + M_T);                                            // [tab_units] source byte offset in a group's plane
-  int2 *ents = (int2 *)(tab + pl.tab_units);                               // [2][ents] (LDS offset, fragment offset) of a step's half
-  int *row_src = (int *)(ents + 2 * pl.ents);                              // Mellin axes: [filter row of the tile][row] first source of the row
-  const int2 *rows = (const int2 *)(AF + pl.rows_off);
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int half = lane >> 5, l32 = lane & 31;
-  const int wk = WK > 1 ? wave : 0, wm = WM > 1 ? wave & (WM - 1) : 0, wn = WK > 1 ? 0 : wave / WM;
-  const bool mellin_x = pl.kind_x == AX_MCORR || pl.kind_x == AX_MCONV;
-  const int taps = pl.nfx * pl.nfy;
-  const int m_tile = blockIdx.y;
-  const unsigned zero_frag = (unsigned)(pl.CG * taps * PARTS * 512);       // the tile's fragment of zeros, behind the others
-  const unsigned af_tile = zero_frag + PARTS * 512;                        // bytes of 32 channels' fragments
-  const char *AFm = AF + (i64)(m_tile * WM + wm) * MT * af_tile, *AFm1 = AFm + af_tile;
-  const i64 plane_bytes = (i64)(pl.plane + 1) * UB;
-  const unsigned lds0 = lds_address((const float *)blk_lds);
-  const int items = pl.whole + pl.rest * pl.slices;
-  const int my_tiles = (items - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
-
-  if (tid < M_T) {
-    const int m = m_tile * M_T + tid;
-    float b = 0.f;
-    if (bias && m < pl.M) b = !F16 ? ((const float *)bias)[m] : (float)(pl.wide ? (_Float16)((const float *)bias)[m] : ((const _Float16 *)bias)[m]);
-    Bs[tid] = b;
-  }
-
-  // the sources of a tile's virtual positions, and the operand offsets of its steps
-  constexpr int kWrap = 4 * WK;                        // halves of two steps of every wavefront that shares a tile's steps
-  auto stage_halves = [](int n) { return max((n + 2 * WK - 1) / (2 * WK) * (2 * WK), kWrap); };
-  auto build_tile = [&](const BlockTile &g, int parity, int2 *before) {
-    // (fields of the plan, read together: one wait for the scalar loads instead of one each)
-    int RS = pl.RS, cy = pl.cy + pl.by_min, uy = pl.uy, ux = pl.ux, ngx = pl.ngx, ngy = pl.ngy, tab_units = pl.tab_units, F = pl.F,
-        G = pl.G, nfx = pl.nfx, nfy = pl.nfy, none = pl.plane, group_bytes = pl.group_bytes, n_before = pl.ents;
-    asm volatile("" : "+s"(RS), "+s"(cy), "+s"(uy), "+s"(ux), "+s"(ngx), "+s"(ngy), "+s"(tab_units), "+s"(F), "+s"(G), "+s"(nfx),
-                 "+s"(nfy), "+s"(none), "+s"(group_bytes), "+s"(n_before));
-    int kx = pl.kind_x, sx = pl.sx, dx = pl.dx, px = pl.px, bx = pl.bx, bx_min = pl.bx_min, by = pl.by, by_min = pl.by_min;
-    unsigned mg_p1 = pl.mg_p1, mg_full = pl.mg_full, mg_per_row = pl.mg_per_row, mg_G = pl.mg_G;
-    asm volatile("" : "+s"(kx), "+s"(sx), "+s"(dx), "+s"(px), "+s"(bx), "+s"(bx_min), "+s"(by), "+s"(by_min), "+s"(mg_p1),
-                 "+s"(mg_full), "+s"(mg_per_row), "+s"(mg_G));
-    if (mellin_x) {
-      const FastDiv by_rows(g.rows);
-      for (int t = tid; t < g.nv * g.rows; t += kThreads) {
-        int j, r;
-        by_rows.divmod(t, j, r);
-        const int gx = mellin_tap32(kx, rows[g.row_lo + r].x, filter_row(g, j), ngx, sx, dx, px + 1, ux, mg_p1);
-        row_src[t] = gx >= 0 ? gx * ngy : -1;
-      }
-      lds_barrier();
-    }
-    // wavefronts take 64 / RS virtual rows (or a 64th piece of one) at a time: a lane keeps its column
-    const int per = RS <= 64 ? 64 / RS : 1, vrows = g.vrows;
-    const int lr = RS <= 64 ? lane / RS : 0;
-    for (int col = lane - lr * RS; col < RS; col += RS <= 64 ? RS : 64) {
-      const int vy = cy + col;
-      int gy = -1;
-      if (vy >= 0) {
-        if (uy == 1) gy = vy;
-        else { const int q = vy / uy; if (q * uy == vy) gy = q; }
-        if (gy >= ngy) gy = -1;
-      }
-      if (lr < per)
-        for (int vr = wave * per + lr; vr < vrows; vr += kWaves * per) {
-          int first = -1;
-          if (mellin_x) {
-            first = row_src[vr];
-          } else {
-            const int vx = g.vx_min + vr;
-            int gx = -1;
-            if (vx >= 0) {
-              if (ux == 1) gx = vx;
-              else { const int q = vx / ux; if (q * ux == vx) gx = q; }
-            }
-            if (gx >= 0 && gx < ngx) first = gx * ngy;
-          }
-          tab[vr * RS + col] = (first >= 0 && gy >= 0 ? first + gy : none) * UB;
-        }
-    }
-    if (tid < 64 && g.units + tid < tab_units) tab[g.units + tid] = none * UB;
-    // Entries of the tile's stages one behind the other (a last odd half is paired with the fragment of zeros), then
-    // the first two steps again: a stage reads on into the one that follows it.  `before`: the first two steps of
-    // this tile also go behind the entries of the tile before it, whose last stage is running.
-    int2 *out = ents + parity * n_before;
-    const int per_row = nfy * G, full = stage_halves(F * per_row), subsets = (g.nv + F - 1) / F;
-    const int tail = stage_halves((g.nv - (subsets - 1) * F) * per_row), n_ents = (subsets - 1) * full + tail;
-    for (int e = tid; e < n_ents + kWrap; e += kThreads) {
-      const int at0 = e < n_ents ? e : e - n_ents;                       // (n_ents >= kWrap)
-      const int sub = min(udiv(at0, full, mg_full), subsets - 1), at = at0 - sub * full;
-      const int n_e = min(F, g.nv - sub * F) * per_row, k = min(at, n_e - 1);
-      const int jj = udiv(k, per_row, mg_per_row), rest = k - jj * per_row, fy = udiv(rest, G, mg_G), gi = rest - fy * G;
-      const int fx = mellin_x ? filter_row(g, sub * F + jj) : jj;
-      const int row = mellin_x ? jj * g.rows : bx * fx - bx_min;
-      const int2 v = make_int2(gi * group_bytes + (row * RS + by * fy - by_min) * UB,
-                               at < n_e ? ((gi * nfx + fx) * nfy + fy) * (PARTS * 512) : 0x40000000);
-      out[e] = v;
-      if (e < kWrap && before) before[e] = v;
-    }
-    return n_ents;
-  };
-
-  // the loads of a stage: 16-byte slots in blocks of 64, dealt to the wavefronts; the sources of four blocks are read
-  // before the first is used
-  auto issue = [&](const BlockTile &g, int c0, int j0, int buf) {
-    const int nF = min(pl.F, g.nv - j0);
-    const int units = mellin_x ? nF * g.rows * pl.RS : g.units, blocks = (units * PARTS + 63) >> 6;
-    const int *from = tab + (mellin_x ? j0 * g.rows * pl.RS : 0);
-    const char *src0 = X + ((i64)g.n * pl.CG + c0) * plane_bytes;
-    const unsigned dst0 = lds0 + (unsigned)(buf * pl.buf_bytes);
-    int groups = pl.G, group_bytes = pl.group_bytes;
-    asm volatile("" : "+s"(groups), "+s"(group_bytes));      // (kept in registers: a scalar load in the loop would wait for LDS as well)
-    for (int b = wave; b < blocks; b += 4 * kWaves) {
-      unsigned at[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int slot = min(b + i * kWaves, blocks - 1) * 64 + lane, unit = F16 ? slot : slot / 3;
-        at[i] = (unsigned)from[unit] + (F16 ? 0 : (slot - unit * 3) * 16);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (b + i * kWaves < blocks) {
-          const char *src = src0;
-          unsigned dst = dst0 + (unsigned)((b + i * kWaves) * 1024);
-          for (int k = 0; k < groups; ++k) {
-            load16_to_lds_at((const float *)src, at[i], dst);
-            src += plane_bytes;
-            dst += (unsigned)group_bytes;
-          }
-        }
-    }
-  };
-
-  floatx16 acc[MT][NT];
-  int lane_vpos[NT], lane_q[NT];
-  struct Operands { uintx4 a[MT][PARTS]; };
-  struct SignalOps { uintx4 b[NT][PARTS]; };
-  Operands A0, A1;
-  SignalOps B0, B1;
-
-  const unsigned lane_frag = (unsigned)(l32 * 16), zero_at = zero_frag + lane_frag;
-  auto fetch_a = [&](const int2 &e, unsigned af_c, Operands &o) {
-    const unsigned off = min((unsigned)e.y + af_c + lane_frag, zero_at);
-#pragma unroll
-    for (int k = 0; k < MT; ++k)
-#pragma unroll
-      for (int pt = 0; pt < PARTS; ++pt) o.a[k][pt] = *(const uintx4 *)((k ? AFm1 : AFm) + off + pt * 512);
-  };
-
-  BlockTile tg = block_tile<P>(pl, rows, (int)blockIdx.x, mellin_x), next_tg = tg;
-  if (my_tiles <= 0) return;
-  int n_ents = build_tile(tg, 0, nullptr), next_ents = n_ents;
-  __syncthreads();
-  issue(tg, tg.c_first, 0, 0);
-  int c0 = tg.c_first, j0 = 0, buf = 0, ti = 0;
-  int se = 0;                                          // the stage's first entry (of this tile's)
-  unsigned af_c = (unsigned)(c0 * taps * PARTS * 512);
-  const int2 *my_ents = ents + 2 * wk + half;          // this half-wave's entries (of parity 0)
-  int2 e0 = my_ents[0], e1 = my_ents[2 * WK];
-  fetch_a(e0, af_c, A0);
-  fetch_a(e1, af_c, A1);
-  wait_and_barrier<0>();
-
-  for (bool first = true;;) {
-    {
-      unsigned zero;                                   // a zero the compiler cannot see through: plan fields are loaded anew per stage
-      asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
-      plp = (ConstBlockPlan *)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + zero);
-    }
-    if (first) {
-      // position -> virtual position of its (first filter row, first column) tap; accumulators start from the bias
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        int local = (wn * NT + t) * 32 + l32;
-        if (local >= tg.count) local = 0;
-        const int row = udiv(tg.q0 + local, pl.noy, pl.mg_noy), oy = tg.q0 + local - row * pl.noy;
-        lane_vpos[t] = (((mellin_x ? 1 : pl.ax) * (row - tg.row_lo)) * pl.RS + pl.ay * oy) * UB;
-        lane_q[t] = (mellin_x ? rows[row].x : row) * pl.noy + oy;
-      }
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          float4 bv = *(const float4 *)(Bs + (wm * MT + i) * 32 + g4 * 8 + half * 4);
-          if ((WK > 1 && wk > 0) || tg.slice > 0) bv = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            acc[i][t][4 * g4 + 0] = bv.x; acc[i][t][4 * g4 + 1] = bv.y;
-            acc[i][t][4 * g4 + 2] = bv.z; acc[i][t][4 * g4 + 3] = bv.w;
-          }
-        }
-    }
-    const char *Xb = bufs + buf * pl.buf_bytes;
-    auto fetch_b = [&](const int2 &e, SignalOps &o) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int pt = 0; pt < PARTS; ++pt) o.b[t][pt] = *(const uintx4 *)(Xb + (lane_vpos[t] + e.x) + pt * 16);
-    };
-    fetch_b(e0, B0);
-    // ---- the stage after this one: its loads are issued under this stage's steps, its first fragments in the last two
-    const int halves = stage_halves((mellin_x ? min(pl.F, tg.nv - j0) : tg.nv) * pl.nfy * pl.G);
-    const int steps = halves / (2 * WK);
-    int nj0 = mellin_x ? j0 + pl.F : tg.nv, nc0 = c0, n_se = se + halves;
-    if (nj0 >= tg.nv) { nj0 = 0; nc0 = c0 + pl.G; n_se = 0; }
-    const bool last = nc0 >= tg.c_end;
-    const bool more = !last || ti + 1 < my_tiles;
-    const int2 *ep = my_ents + (ti & 1) * pl.ents + se;
-    if (last) {
-      nc0 = 0;
-      nj0 = 0;
-      if (more) {
-        // another tile: its tables (every load of this tile has been issued, every wavefront is past the barrier)
-        next_tg = block_tile<P>(pl, rows, (int)blockIdx.x + (ti + 1) * (int)gridDim.x, mellin_x);
-        next_ents = build_tile(next_tg, (ti + 1) & 1, ents + (ti & 1) * pl.ents + n_ents);
-        lds_barrier();
-        nc0 = next_tg.c_first;
-        issue(next_tg, nc0, 0, buf ^ 1);
-      }
-    } else {
-      issue(tg, nc0, nj0, buf ^ 1);
-    }
-    const unsigned n_af = (unsigned)(nc0 * taps * PARTS * 512);
-    // A step: the next step's signal operands are requested before its multiplies and the fragments of the step
-    // after next behind them (pinned: the scheduler moves reads next to their use).  Nothing here depends on which
-    // step it is, so that every wait counts exactly what is younger: the last pair's last signal reads are of no use,
-    // and its fragment fetches are the next stage's.
-    int2 e2 = ep[4 * WK];
-    for (int i = 0; i + 1 < steps; i += 2) {
-      fetch_b(e1, B1);
-      const int2 e3 = ep[6 * WK];
-      __builtin_amdgcn_sched_barrier(0);
-      block_multiply<MT, NT, PARTS>(acc, A0.a, B0.b);
-      __builtin_amdgcn_sched_barrier(0);
-      fetch_a(e2, i + 2 < steps ? af_c : n_af, A0);
-      fetch_b(e2, B0);
-      const int2 e4 = ep[8 * WK];
-      __builtin_amdgcn_sched_barrier(0);
-      block_multiply<MT, NT, PARTS>(acc, A1.a, B1.b);
-      __builtin_amdgcn_sched_barrier(0);
-      fetch_a(e3, i + 3 < steps ? af_c : n_af, A1);
-      e0 = e2;
-      e1 = e3;
-      e2 = e4;
-      ep += 4 * WK;
-    }
-    if (steps & 1) {
-      // one step left, whose operands are in A0 and B0; A1 holds the next stage's first fragments where its second's belong
-      block_multiply<MT, NT, PARTS>(acc, A0.a, B0.b);
-      e0 = e1;
-      e1 = e2;
-      fetch_a(e0, n_af, A0);
-      fetch_a(e1, n_af, A1);
-    }
-    // every wavefront's loads for the next stage have landed (the newest in flight are the two fragment fetches),
-    // and every wavefront is done with this stage's buffer
-    wait_and_barrier<kALoads>();
-    first = last;
-    if (last) {
-      // ---- the tile is finished
-      if constexpr (WK > 1) {
-        // sums of the wavefronts, in their order (one tile per workgroup: the buffers are free)
-        float *red = (float *)bufs;
-#pragma unroll
-        for (int k = 0; k < MT; ++k)
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4)
-              *(float4 *)(red + (((wk * MT * NT + k * NT + t) * 4 + r4) * 64 + lane) * 4) =
-                  make_float4(acc[k][t][4 * r4], acc[k][t][4 * r4 + 1], acc[k][t][4 * r4 + 2], acc[k][t][4 * r4 + 3]);
-        __syncthreads();
-      }
-      // The descriptor ends with the block's last channel, so rows past it and lanes without a position (an offset past
-      // any end) are dropped by its range check.  A slice's sums are fp32, in the order of the tile.
-      const bool whole = tg.slot < 0, relu = pl.relu && whole, as_half = HOUT && whole;
-      const int m0 = m_tile * M_T + wm * MT * 32, ES = as_half ? 2 : 4, h_m = (whole ? (int)pl.h_m : P) * ES;
-      char *base = whole ? (char *)Hv + ((i64)tg.n * pl.h_n + (i64)m0 * (int)pl.h_m) * ES
-                         : (char *)(sums + (((i64)tg.slot * gridDim.y + m_tile) * M_T + wm * MT * 32) * P);
-      const __amdgpu_buffer_rsrc_t rsrc =
-          __builtin_amdgcn_make_buffer_rsrc(base, 0, max(0, min(MT * 32, pl.M - m0)) * h_m, 0x00020000);
-      int at[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int local = (wn * NT + t) * 32 + l32;
-        at[t] = local < tg.count ? (whole ? lane_q[t] : local) * ES : (int)0x80000000u;
-      }
-      auto store_one = [&](float v, int to) {
-        if (as_half) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(short, (_Float16)v), rsrc, to, 0, 0);
-        else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rsrc, to, 0, 0);
-      };
-      const int row0 = half * 4 * h_m;
-      auto relu4 = [&](float4 v) { return relu ? make_float4(fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f)) : v; };
-      auto store_four = [&](float4 v, int to) {        // four channels of the lane's position
-        v = relu4(v);
-        store_one(v.x, to);
-        store_one(v.y, to + h_m);
-        store_one(v.z, to + 2 * h_m);
-        store_one(v.w, to + 3 * h_m);
-      };
-      if constexpr (WK > 1) {
-        // the tile's 32 x 32 blocks are dealt to the wavefronts
-        const float *red = (const float *)bufs;
-        for (int kt = wk; kt < MT * NT; kt += WK) {
-          const int k = kt / NT, t = kt - k * NT;
-          int to = (NT > 1 && t ? at[NT - 1] : at[0]) + row0 + k * 32 * h_m;
-#pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) {
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int w = 0; w < WK; ++w) {
-              const float4 p = *(const float4 *)(red + (((w * MT * NT + kt) * 4 + r4) * 64 + lane) * 4);
-              v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
-            }
-            store_four(v, to);
-            to += 8 * h_m;                             // (registers 4 g .. 4 g + 3 are rows 8 g + 4 half ..)
-          }
-        }
-      } else {
-        // A 4 x 4 transpose over four lanes makes four channels of a position four positions of a channel, side by side
-        // in memory: a quarter of the stores (128 x 256 half values: 22000 -> 12000 cycles).  Not for the rows of a class
-        // (n_classes > 1), which do not follow each other; the last positions of an image, less than four, go one by one.
-        bool single = true;
-        if (pl.n_classes == 1 || !whole) {
-          int to[NT];
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            const int first = quad_lane<0>(at[t]), last = quad_lane<3>(at[t]);
-            to[t] = last >= 0 ? row0 + (lane & 3) * h_m + first : (int)0x80000000u;
-            if (last >= 0) at[t] = (int)0x80000000u;
-          }
-#pragma unroll
-          for (int k = 0; k < MT; ++k)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4)
-#pragma unroll
-              for (int t = 0; t < NT; ++t) {
-                const float4 v = relu4(make_float4(acc[k][t][4 * g4], acc[k][t][4 * g4 + 1], acc[k][t][4 * g4 + 2], acc[k][t][4 * g4 + 3]));
-                if (as_half) __builtin_amdgcn_raw_buffer_store_b64(transpose_half(v, lane), rsrc, to[t], 0, 0);
-                else __builtin_amdgcn_raw_buffer_store_b128(transpose_words(v, lane), rsrc, to[t], 0, 0);
-                to[t] += 8 * h_m;
-              }
-          single = tg.count & 3;
-        }
-        if (single) {
-#pragma unroll
-          for (int t = 0; t < NT; ++t) at[t] += row0;
-#pragma unroll
-          for (int k = 0; k < MT; ++k)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4)
-#pragma unroll
-              for (int t = 0; t < NT; ++t) {
-                store_four(make_float4(acc[k][t][4 * g4], acc[k][t][4 * g4 + 1], acc[k][t][4 * g4 + 2], acc[k][t][4 * g4 + 3]), at[t]);
-                at[t] += 8 * h_m;
-              }
-        }
-      }
-      if (!more) break;
-      ++ti;
-      tg = next_tg;
-      n_ents = next_ents;
-    }
-    c0 = nc0;
-    j0 = nj0;
-    buf ^= 1;
-    se = n_se;
-    af_c = n_af;
-  }
-#undef pl
-}
-
-template <int MT, int NT, int WM, int WK, bool F16, bool HOUT>
-hipError_t launch_instance(const BlockPlan &pl, const void *x, const void *frag, const void *bias, void *out, float *sums,
-                           hipStream_t stream) {
-  auto kern = block_gemm_kernel<MT, NT, WM, WK, F16, HOUT>;
-  static std::atomic<int> lds_allowed{0};
-  hipError_t e = allow_large_lds((const void *)kern, pl.lds_bytes, lds_allowed);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)pl.grid_x, (unsigned)pl.m_tiles), dim3(kThreads), pl.lds_bytes, stream,
-                     pl, (const char *)x, (const char *)frag, bias, out, sums);
-  return hipGetLastError();
-}
 
 // Residue classes of a Mellin axis (mellin_common.hpp: tap relations), those with the same filter
 // rows next to each other.
@@ -570,11 +59,14 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   if (Y.kind != AX_LCORR && Y.kind != AX_LCONV) return false;
   const i64 plane = X.ng * Y.ng, Q = X.nh * Y.nh;
   if (plane < 1 || Q < 1 || plane >= (i64)1 << 22 || Q >= (i64)1 << 22) return false;
-  if (pr.batch > 65535 || pr.c_in > 8 * 65535 || pr.c_out * Q >= lim / 2 || Q >= (i64)1 << 20) return false;   // (32-bit byte offsets)
+  if (pr.batch > 65535 || pr.c_in > 8 * 65535 || pr.c_out * Q >= lim / 2 || Q >= (i64)1 << 20 ||
+      (pr.c_out + 7) / 8 * (Q + 1) * 48 >= (i64)1 << 31)
+    return false;                                      // (32-bit byte offsets)
   if (X.s > 4096 || X.d > 4096 || X.u > 4096 || X.p > 4096 || X.p < -lim || Y.s > 64 || Y.d > 4096 || Y.u > 64 || Y.p > lim || Y.p < -lim)
     return false;
   pl.f16 = f16;
   pl.wide = 0;
+  pl.out_groups = (int)((pr.c_out + 7) / 8);
   pl.batch = (int)pr.batch; pl.M = (int)pr.c_out; pl.CG = (int)((pr.c_in + 7) / 8);
   pl.nox = (int)X.nh; pl.noy = (int)Y.nh; pl.Q = (int)Q;
   pl.ngx = (int)X.ng; pl.ngy = (int)Y.ng; pl.plane = (int)plane;
@@ -707,6 +199,7 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
     }
     pl.rest = (int)rest;
     pl.whole = (int)(total - rest);
+    pl.chan_slots = (int)total * (pl.wk > 1 ? pl.nt : kWaves / pl.wm);
     const i64 items = (i64)pl.whole + (i64)pl.rest * pl.slices;
     pl.grid_x = (int)(pl.wk > 1 ? items : std::min<i64>(per_m, items));      // (wavefronts that share a tile's steps take one tile)
     pl.slice_bytes = (size_t)pl.rest * pl.slices * pl.m_tiles * (size_t)(M_T * P) * 4;
@@ -733,28 +226,9 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   return true;
 }
 
-hipError_t launch_block_gemm(const BlockPlan &pl, const void *signal, const void *frag, const void *bias, void *out,
-                             float *sums, hipStream_t stream) {
-#define MELLIN_BLOCK_CASE(MT_, NT_, WM_, WK_)                                                                \
-  if (pl.mt == MT_ && pl.nt == NT_ && pl.wm == WM_ && pl.wk == WK_) {                                        \
-    if (pl.f16) return launch_instance<MT_, NT_, WM_, WK_, true, true>(pl, signal, frag, bias, out, sums, stream); \
-    return launch_instance<MT_, NT_, WM_, WK_, false, false>(pl, signal, frag, bias, out, sums, stream);           \
-  }
-  if (pl.f16 && pl.nt == 4) {
-    if (pl.wm == 2) return launch_instance<2, 4, 2, 1, true, true>(pl, signal, frag, bias, out, sums, stream);
-    if (pl.mt == 2) return launch_instance<2, 4, 1, 1, true, true>(pl, signal, frag, bias, out, sums, stream);
-    return launch_instance<1, 4, 1, 1, true, true>(pl, signal, frag, bias, out, sums, stream);
-  }
-  MELLIN_BLOCK_CASE(2, 2, 1, 1)
-  MELLIN_BLOCK_CASE(2, 1, 1, 1)
-  MELLIN_BLOCK_CASE(1, 2, 1, 1)
-  MELLIN_BLOCK_CASE(1, 1, 1, 1)
-  MELLIN_BLOCK_CASE(2, 2, 1, 4)
-  MELLIN_BLOCK_CASE(2, 1, 1, 4)
-  MELLIN_BLOCK_CASE(1, 2, 1, 4)
-  MELLIN_BLOCK_CASE(1, 1, 1, 4)
-#undef MELLIN_BLOCK_CASE
-  return hipErrorInvalidValue;
+hipError_t launch_block_gemm(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream) {
+  if (a.grad) return a.blocked ? launch_grad_blocked(pl, a, stream) : launch_grad_plain(pl, a, stream);
+  return a.blocked ? launch_out_blocked(pl, a, stream) : launch_shape<OUT_PLAIN>(pl, a, stream);
 }
 
 }  // namespace mellin

@@ -41,6 +41,7 @@ struct BlockPlan {
   // tiles: (position tile, image), the images of a position tile side by side.  The last `rest` of them, which would
   // leave workgroups without one, are dealt out in `slices` of the contracted channels, whose sums go to the workspace
   int whole, rest, slices;
+  int out_groups, chan_slots;      // groups of eight output channels; partial sums of a channel over the positions
   unsigned mg_batch, mg_noy, mg_per_row, mg_full, mg_G;      // floor(2^32 / d) (see udiv)
   i64 h_n, h_m;
   int relu, half_out;
@@ -58,10 +59,22 @@ struct BlockPlan {
 
 // False: the kernel does not apply.
 bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl);
-// out = [relu](bias + sum) from a blocked signal and packed filter; bias (fp32 / half, or null).  Of tiles in slices
-// (pl.rest > 0) the sums go to `sums` and launch_block_finish makes the output.
-hipError_t launch_block_gemm(const BlockPlan &pl, const void *signal, const void *frag, const void *bias, void *out,
-                             float *sums, hipStream_t stream);
+// out = [relu](bias + sum) from a blocked signal and packed filter; bias (fp32 / half, or null), relu as the plan says.
+// With `grad`, the input gradient of a layer behind a ReLU: zero where `mask`, the blocked output of that ReLU, is not
+// positive; its sums over the positions go to chan_sums ([channel][pl.chan_slots]: partial sums for launch_block_finish).
+// Of tiles in slices (pl.rest > 0) the sums go to `sums`, and launch_block_finish does all that.
+struct BlockGemmArgs {
+  const void *signal, *frag, *bias;
+  void *out;
+  float *sums;
+  bool blocked, grad;              // out: blocked
+  const void *mask;
+  float *chan_sums;
+};
+hipError_t launch_block_gemm(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
+hipError_t launch_out_blocked(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
+hipError_t launch_grad_plain(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
+hipError_t launch_grad_blocked(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
 
 // The rows of one filter row in the weight gradient: output rows ox0 + i step and input rows gx0 + i gstep for
 // i < count; its share of the launch: `slices` workgroups from slice0 on.
@@ -97,11 +110,35 @@ struct PackSignal {
   int batch, channels, plane;
 };
 size_t pack_partial_count(i64 batch, i64 channels, i64 plane);
-// Everything a pass reads in one launch: up to two tensors and the filter of `pl` (f: fp32 or half, `channels`
-// contracted channels -> filter_bytes at `frag`); null for what there is not.  `copy`: the filter's `copy_count`
-// floats, rounded to half.
-hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b, const BlockPlan *pl, int channels,
-                             const void *f, void *frag, void *copy, i64 copy_count, hipStream_t stream);
+// A filter to pack for `pl`, and on Mellin axes the output rows in the order of their classes: f (fp32 or half; wide: fp32
+// where the tensors are half) of `channels` contracted channels -> filter_bytes at `frag`.  `copy`: the filter's
+// `copy_count` floats, rounded to half.
+struct PackFilter {
+  const void *f;
+  char *frag;
+  void *copy;
+  i64 copy_count, f_m, f_c;
+  size_t rows_off;
+  int channels, wide, M, CG, nfx, nfy, f_pitch, f_off, tiles;          // (tiles of 32 channels)
+  int kind_x, nox, ngx, sx, dx, px, ux;
+  unsigned mg_p1;
+  int n_classes, cls_stride;
+  BlockClass cls[kBlockClasses];
+};
+PackFilter pack_filter(const BlockPlan &pl, int channels, const void *f, void *frag, void *copy, i64 copy_count);
+// Everything a pass reads, in one launch (one for every kPackFilters filters): up to two tensors (null: not there) and filters.
+constexpr int kPackFilters = 6;
+hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b, const PackFilter *filters, int n_filters,
+                             hipStream_t stream);
+
+// Maximum over pairs of neighbouring columns of a blocked tensor (batch, channels, rows, cols), as pool_pairs: y is blocked
+// with cols / 2 columns; `which` (eight bytes a unit of y): 1 where the second was taken.
+hipError_t launch_block_pool(bool f16, const void *x, i64 batch, i64 channels, i64 rows, i64 cols, void *y, void *which, hipStream_t stream);
+// Its backward pass behind a ReLU: grad_x from grad_y (blocked), zero where y is not positive; the sums of a channel's
+// gradients go to `partial` (pool_partial_count(): floats, for launch_block_finish).
+hipError_t launch_block_pool_grad(bool f16, const void *grad_y, const void *y, const void *which, i64 batch, i64 channels, i64 rows,
+                                  i64 cols, void *grad_x, float *partial, hipStream_t stream);
+size_t pool_partial_count(i64 batch, i64 channels, i64 rows, i64 cols);
 
 // The sums that end a pass, in one launch; null pointers for those there are not.
 struct BlockFinish {
@@ -111,10 +148,8 @@ struct BlockFinish {
   const float *bias_partial;       // bias gradient: `bias_count` partial sums of each of `channels`
   void *grad_bias;
   i64 bias_count, channels;
-  const BlockPlan *slices;         // the output of a block_gemm's tiles in slices
-  const void *frag;                // (its packed filter)
-  const float *slice_sums;
-  void *out;
+  const BlockPlan *slices;         // what a block_gemm called with `args` made of tiles in slices
+  BlockGemmArgs args;
 };
 // (wide: the gradients are float where the tensors are half)
 hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipStream_t stream);

@@ -1,0 +1,10 @@
+// The channel-blocked matrix kernel as the input gradient of a layer behind a ReLU, blocked.
+#include "block_gemm_kernel.hpp"
+
+namespace mellin {
+
+hipError_t launch_grad_blocked(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream) {
+  return launch_shape<GRAD_BLOCKED>(pl, a, stream);
+}
+
+}  // namespace mellin

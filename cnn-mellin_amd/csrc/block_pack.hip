@@ -104,11 +104,10 @@ __device__ __forceinline__ void pack_signal(const PackPart &pt, unsigned block, 
 //   frag[((mt * (CG * nfx * nfy + 1) + (cg * nfx + fx) * nfy + fy) * parts + p) * 32 + r]   (16-byte words)
 // and a unit of zeros behind each tile of 32 channels.
 template <bool F16, typename From>
-__device__ __forceinline__ void pack_filter(const BlockPlan &pl, int channels, const void *__restrict__ fv, uintx4 *__restrict__ frag,
-                                            i64 idx) {
+__device__ __forceinline__ void pack_fragments(const PackFilter &pl, i64 idx) {
   typedef typename std::conditional<F16, _Float16, float>::type T;
   const int taps = pl.nfx * pl.nfy, per_tile = pl.CG * taps + 1;
-  const i64 total = (i64)pl.m_tiles * pl.wm * pl.mt * per_tile * 32;
+  const i64 total = (i64)pl.tiles * per_tile * 32;
   if (idx >= total) return;
   const int r = (int)(idx & 31);
   const int unit = (int)(idx >> 5);
@@ -116,11 +115,11 @@ __device__ __forceinline__ void pack_filter(const BlockPlan &pl, int channels, c
   const int cg = ct / taps, tap = ct - cg * taps;                      // (cg == CG: the zeros)
   const int fx = tap / pl.nfy, fy = tap - fx * pl.nfy;
   const int m = mt * 32 + r;
-  const From *f = (const From *)fv + (i64)m * pl.f_m + fx * pl.f_pitch + pl.f_off + fy;
+  const From *f = (const From *)pl.f + (i64)m * pl.f_m + fx * pl.f_pitch + pl.f_off + fy;
   T v[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = (m < pl.M && cg < pl.CG && cg * 8 + i < channels) ? (T)f[(i64)(cg * 8 + i) * pl.f_c] : (T)0;
-  uintx4 *o = frag + (i64)unit * (F16 ? 32 : 96) + r;
+  for (int i = 0; i < 8; ++i) v[i] = (m < pl.M && cg < pl.CG && cg * 8 + i < pl.channels) ? (T)f[(i64)(cg * 8 + i) * pl.f_c] : (T)0;
+  uintx4 *o = (uintx4 *)pl.frag + (i64)unit * (F16 ? 32 : 96) + r;
   if constexpr (F16) {
     uintx4 w;
 #pragma unroll
@@ -137,7 +136,7 @@ __device__ __forceinline__ void pack_filter(const BlockPlan &pl, int channels, c
 }
 
 // Output row `row` of a Mellin axis in the order of its classes, with the filter rows that have a tap for it.
-__device__ __forceinline__ int2 class_row(const BlockPlan &pl, int row) {
+__device__ __forceinline__ int2 class_row(const PackFilter &pl, int row) {
   int ox = row;
   for (int k = 0; k < pl.n_classes; ++k)
     if (row >= pl.cls[k].start) ox = pl.cls[k].first + (row - pl.cls[k].start) * pl.cls_stride;
@@ -149,38 +148,37 @@ __device__ __forceinline__ int2 class_row(const BlockPlan &pl, int row) {
 
 struct PackArgs {
   PackPart a, b;
-  BlockPlan pl;
-  int channels;
-  unsigned filter_blocks, row_blocks, copy_blocks;
-  const void *f;
-  char *frag;
-  _Float16 *copy;
-  i64 copy_count;
+  PackFilter filter[kPackFilters];
+  unsigned rows[kPackFilters], fragments[kPackFilters], copies[kPackFilters];      // blocks
+  int n_filters;
 };
 
 template <bool F16>
 __global__ __launch_bounds__(kPackThreads) void block_pack_kernel(PackArgs args) {
   __shared__ float red[kPackThreads / 64][8];
   unsigned b = blockIdx.x;
-  if (b < args.row_blocks) {
-    const int row = (int)(b * kPackThreads + threadIdx.x);
-    if (row < args.pl.nox) ((int2 *)(args.frag + args.pl.rows_off))[row] = class_row(args.pl, row);
-    return;
+  for (int i = 0; i < args.n_filters; ++i) {
+    const PackFilter &fl = args.filter[i];
+    if (b < args.rows[i]) {
+      const int row = (int)(b * kPackThreads + threadIdx.x);
+      if (row < fl.nox) ((int2 *)(fl.frag + fl.rows_off))[row] = class_row(fl, row);
+      return;
+    }
+    b -= args.rows[i];
+    if (b < args.fragments[i]) {
+      const i64 idx = (i64)b * kPackThreads + threadIdx.x;
+      if (!F16 || fl.wide) pack_fragments<F16, float>(fl, idx);
+      else pack_fragments<F16, _Float16>(fl, idx);
+      return;
+    }
+    b -= args.fragments[i];
+    if (b < args.copies[i]) {
+      const i64 at = ((i64)b * kPackThreads + threadIdx.x) * 4;
+      for (i64 k = at; k < min(at + 4, fl.copy_count); ++k) ((_Float16 *)fl.copy)[k] = (_Float16)((const float *)fl.f)[k];
+      return;
+    }
+    b -= args.copies[i];
   }
-  b -= args.row_blocks;
-  if (b < args.filter_blocks) {
-    const i64 idx = (i64)b * kPackThreads + threadIdx.x;
-    if (!F16 || args.pl.wide) pack_filter<F16, float>(args.pl, args.channels, args.f, (uintx4 *)args.frag, idx);
-    else pack_filter<F16, _Float16>(args.pl, args.channels, args.f, (uintx4 *)args.frag, idx);
-    return;
-  }
-  b -= args.filter_blocks;
-  if (b < args.copy_blocks) {
-    const i64 at = ((i64)b * kPackThreads + threadIdx.x) * 4;
-    for (i64 i = at; i < min(at + 4, args.copy_count); ++i) args.copy[i] = (_Float16)((const float *)args.f)[i];
-    return;
-  }
-  b -= args.copy_blocks;
   const bool second = b >= args.a.blocks;
   const PackPart &pt = second ? args.b : args.a;
   if (second) b -= args.a.blocks;
@@ -212,28 +210,40 @@ size_t pack_partial_count(i64 batch, i64 channels, i64 plane) {
   return (size_t)(batch * channels * pack_chunks(plane));
 }
 
-hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b, const BlockPlan *pl, int channels,
-                             const void *f, void *frag, void *copy, i64 copy_count, hipStream_t stream) {
+PackFilter pack_filter(const BlockPlan &pl, int channels, const void *f, void *frag, void *copy, i64 copy_count) {
+  PackFilter pf = {f, (char *)frag, copy, copy_count, pl.f_m, pl.f_c, pl.rows_off, channels, pl.wide, pl.M, pl.CG, pl.nfx, pl.nfy,
+                   pl.f_pitch, pl.f_off, pl.m_tiles * pl.wm * pl.mt, pl.kind_x, pl.nox, pl.ngx, pl.sx, pl.dx, pl.px, pl.ux, pl.mg_p1,
+                   pl.n_classes, pl.cls_stride, {}};
+  std::copy(pl.cls, pl.cls + kBlockClasses, pf.cls);
+  return pf;
+}
+
+hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b, const PackFilter *filters, int n_filters,
+                             hipStream_t stream) {
   PackArgs args = {};
   if (!pack_part(a, args.a) || !pack_part(b, args.b)) return hipErrorInvalidValue;
-  if (pl) {
-    args.pl = *pl;
-    args.channels = channels;
-    args.f = f;
-    args.frag = (char *)frag;
-    const i64 total = (i64)pl->m_tiles * pl->wm * pl->mt * ((i64)pl->CG * pl->nfx * pl->nfy + 1) * 32;
-    args.filter_blocks = (unsigned)((total + kPackThreads - 1) / kPackThreads);
-    if (pl->kind_x == AX_MCORR || pl->kind_x == AX_MCONV) args.row_blocks = (unsigned)((pl->nox + kPackThreads - 1) / kPackThreads);
-  }
-  if (copy) {
-    args.copy = (_Float16 *)copy;
-    args.copy_count = copy_count;
-    args.copy_blocks = (unsigned)((copy_count + 4 * kPackThreads - 1) / (4 * kPackThreads));
-  }
-  const unsigned blocks = args.row_blocks + args.filter_blocks + args.copy_blocks + args.a.blocks + args.b.blocks;
-  if (f16) hipLaunchKernelGGL(block_pack_kernel<true>, dim3(blocks), dim3(kPackThreads), 0, stream, args);
-  else hipLaunchKernelGGL(block_pack_kernel<false>, dim3(blocks), dim3(kPackThreads), 0, stream, args);
-  return hipGetLastError();
+  do {
+    args.n_filters = std::min(n_filters, kPackFilters);
+    unsigned blocks = args.a.blocks + args.b.blocks;
+    for (int i = 0; i < args.n_filters; ++i) {
+      const PackFilter &fl = args.filter[i] = filters[i];
+      const i64 units = (i64)fl.tiles * ((i64)fl.CG * fl.nfx * fl.nfy + 1) * 32;
+      args.fragments[i] = (unsigned)((units + kPackThreads - 1) / kPackThreads);
+      args.rows[i] = fl.kind_x == AX_MCORR || fl.kind_x == AX_MCONV ? (unsigned)((fl.nox + kPackThreads - 1) / kPackThreads) : 0;
+      args.copies[i] = fl.copy ? (unsigned)((fl.copy_count + 4 * kPackThreads - 1) / (4 * kPackThreads)) : 0;
+      blocks += args.rows[i] + args.fragments[i] + args.copies[i];
+    }
+    if (blocks) {
+      if (f16) hipLaunchKernelGGL(block_pack_kernel<true>, dim3(blocks), dim3(kPackThreads), 0, stream, args);
+      else hipLaunchKernelGGL(block_pack_kernel<false>, dim3(blocks), dim3(kPackThreads), 0, stream, args);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
+    args.a.blocks = args.b.blocks = 0;                 // (the signals went with the first launch)
+    filters += args.n_filters;
+    n_filters -= args.n_filters;
+  } while (n_filters > 0);
+  return hipSuccess;
 }
 
 }  // namespace mellin

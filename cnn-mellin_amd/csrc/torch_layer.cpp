@@ -7,6 +7,8 @@
 // corr(kind, dims, input, weight, bias, s, d, p, u, r, activation) returns the output tensor, or
 // None for whatever it does not handle (other element types, CPU tensors, arguments that are
 // errors): mconv.py then takes its own path, which has the checks and their messages.
+// stack(...) is the same for a stack of layers with ReLUs (conv_stack.py), whose tensors then stay
+// in the kernels' own layout from layer to layer.
 #include <ATen/ATen.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
@@ -18,7 +20,9 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
 
+#include <algorithm>
 #include <mutex>
+#include <vector>
 
 #include "../../include/mellin_hip.h"
 
@@ -231,7 +235,199 @@ PyObject *corr(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
+// The gradients of a stack of layers with ReLUs.  Edges: the input, then weight and bias of every layer.
+struct StackBackward : public torch::autograd::Node {
+  int kind = 0, elem = 4;
+  std::vector<mellin_stack_layer> layers;              // geometry; the pointers are filled in for each call
+  torch::autograd::SavedVariable input_, out_;
+  std::vector<torch::autograd::SavedVariable> weights_;
+  std::vector<bool> has_bias;
+  Tensor saved_;
+  size_t workspace = 0;
+  at::ScalarType param_kind = at::kFloat;
+
+  std::string name() const override { return "StackBackward"; }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    input_.reset_data();
+    out_.reset_data();
+    for (auto &w : weights_) w.reset_data();
+    saved_.reset();
+  }
+
+  torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+    at::AutoGradMode no_grad(false);
+    const size_t n = layers.size();
+    Tensor input, out, saved;
+    std::vector<Tensor> weights(n);
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      input = input_.unpack();                         // (raises if the variables have been released)
+      out = out_.unpack(shared_from_this());
+      for (size_t i = 0; i < n; ++i) weights[i] = weights_[i].unpack();
+      saved = saved_;
+    }
+    torch::autograd::variable_list result(1 + 2 * n);
+    Tensor grad_out = grads[0].defined() ? grads[0] : at::zeros_like(out);
+    if (grad_out.scalar_type() != out.scalar_type()) grad_out = grad_out.to(out.scalar_type());
+    grad_out = grad_out.contiguous();
+    const c10::OptionalDeviceGuard guard(input.device());
+    std::vector<mellin_stack_layer> call = layers;
+    if (task_should_compute_output(0)) result[0] = at::empty_like(input, at::MemoryFormat::Contiguous);
+    for (size_t i = 0; i < n; ++i) {
+      const Tensor &w = weights[i];
+      if (elem == MELLIN_ELEM_HALF_FLOAT) call[i].weight_half = w.data_ptr();
+      else call[i].weight = w.const_data_ptr();
+      if (task_should_compute_output(1 + 2 * i)) {
+        result[1 + 2 * i] = at::empty(w.sizes(), w.options().dtype(param_kind));
+        call[i].grad_weight = result[1 + 2 * i].data_ptr();
+      }
+      if (has_bias[i] && task_should_compute_output(2 + 2 * i)) {
+        result[2 + 2 * i] = at::empty({w.size(0)}, w.options().dtype(param_kind));
+        call[i].grad_bias = result[2 + 2 * i].data_ptr();
+      }
+    }
+    Tensor ws = scratch(input, workspace);
+    check(mellin_stack_backward(kind, elem, (int)n, call.data(), pointer(input), pointer(out), pointer(grad_out), saved.const_data_ptr(),
+                                (size_t)saved.numel(), result[0].defined() ? result[0].data_ptr() : nullptr, ws.data_ptr(), workspace,
+                                launch_stream(input)));
+    return result;
+  }
+};
+
+PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  if (n_args != 3 || !THPVariable_CheckExact(args[1]) || !PyList_CheckExact(args[2])) Py_RETURN_NONE;
+  const int kind = (int)PyLong_AsLong(args[0]);
+  const Tensor &input0 = THPVariable_Unpack(args[1]);
+  const Py_ssize_t n = PyList_GET_SIZE(args[2]);
+  if (n < 2 || !plain(input0) || input0.dim() != 4) Py_RETURN_NONE;
+  std::vector<mellin_stack_layer> layers(n);
+  std::vector<Tensor> weights(n), biases(n);
+  auto kind_of = input0.scalar_type();
+  const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
+  if (cast) {
+    if (!input0.is_floating_point() || kind_of == at::kDouble) Py_RETURN_NONE;
+    kind_of = at::kHalf;
+  }
+  if (kind_of != at::kFloat && kind_of != at::kHalf) Py_RETURN_NONE;
+  at::ScalarType param_kind = at::kFloat;
+  bool differentiable = input0.requires_grad();
+  int64_t c = input0.size(1), x = input0.size(2), y = input0.size(3);
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject *t = PyList_GET_ITEM(args[2], i);
+    if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != 7) Py_RETURN_NONE;
+    PyObject *w = PyTuple_GET_ITEM(t, 0), *b = PyTuple_GET_ITEM(t, 1);
+    if (!THPVariable_Check(w) || !(b == Py_None || THPVariable_Check(b))) Py_RETURN_NONE;
+    weights[i] = THPVariable_Unpack(w);
+    if (b != Py_None) biases[i] = THPVariable_Unpack(b);
+    const Tensor &wt = weights[i], &bt = biases[i];
+    if (!plain(wt) || wt.dim() != 4 || wt.device() != input0.device() || wt.size(1) != c) Py_RETURN_NONE;
+    if (bt.defined() && (!plain(bt) || bt.dim() != 1 || bt.size(0) != wt.size(0) || bt.device() != input0.device())) Py_RETURN_NONE;
+    if (i == 0) param_kind = wt.scalar_type();
+    if (wt.scalar_type() != param_kind || (bt.defined() && bt.scalar_type() != param_kind)) Py_RETURN_NONE;
+    Geometry g;
+    int64_t r[2];
+    if (!parse(PyTuple_GET_ITEM(t, 2), 2, 1, g.s) || !parse(PyTuple_GET_ITEM(t, 3), 2, 1, g.d) || !parse(PyTuple_GET_ITEM(t, 4), 2, 0, g.p) ||
+        !parse(PyTuple_GET_ITEM(t, 5), 2, 0, r))
+      Py_RETURN_NONE;
+    g.kind = kind;
+    g.batch = input0.size(0);
+    g.c_in = c;
+    g.c_out = wt.size(0);
+    g.ng[0] = x;
+    g.ng[1] = y;
+    for (int k = 0; k < 2; ++k) {
+      g.u[k] = 1;
+      g.nf[k] = wt.size(2 + k);
+      const int axis = k == 0 ? kind : MELLIN_AXIS_LCORR;
+      if (g.s[k] < 1 || g.d[k] < 1 || g.nf[k] < 1 || g.ng[k] < 1 || g.nf[k] > (1 << 30) || g.ng[k] > (1 << 30)) Py_RETURN_NONE;
+      if (axis == MELLIN_AXIS_MCORR && g.p[k] < 0) Py_RETURN_NONE;
+      g.nh[k] = valid_size(axis, g.nf[k], g.ng[k], g.s[k], g.d[k], g.p[k], 1) + r[k];
+      if (g.nh[k] < 1 || g.nh[k] > (1 << 30)) Py_RETURN_NONE;
+    }
+    if (g.batch < 1 || g.c_in < 1 || g.c_out < 1 || g.batch > 65535 || g.c_out > 65535 || g.c_in > (1 << 20)) Py_RETURN_NONE;
+    const int64_t dims[17] = {GEOMETRY_ARGS(g)};
+    layers[i] = mellin_stack_layer{};
+    std::copy(dims, dims + 17, layers[i].dims);
+    layers[i].pool = PyTuple_GET_ITEM(t, 6) == Py_True;
+    differentiable = differentiable || wt.requires_grad() || (bt.defined() && bt.requires_grad());
+    c = g.c_out;
+    x = g.nh[0];
+    y = layers[i].pool ? g.nh[1] / 2 : g.nh[1];
+  }
+  // float parameters of half tensors (autocast) are rounded by the library; any other mixture is not for this path
+  const bool wide = kind_of == at::kHalf && param_kind == at::kFloat;
+  if (!wide && param_kind != kind_of) Py_RETURN_NONE;
+  if (wide && !cast) Py_RETURN_NONE;
+  const int elem = wide ? MELLIN_ELEM_HALF_FLOAT : kind_of == at::kHalf ? 2 : 4;
+  differentiable = differentiable && at::GradMode::is_enabled();
+  size_t saved_bytes = 0, forward_bytes = 0, backward_bytes = 0;
+  if (!mellin_stack_bytes(kind, elem, differentiable, (int)n, layers.data(), &saved_bytes, &forward_bytes, &backward_bytes)) Py_RETURN_NONE;
+
+  Tensor out;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const c10::OptionalDeviceGuard guard(input0.device());
+    Tensor input, saved;
+    std::vector<Tensor> kept(n);
+    {
+      at::AutoGradMode no_grad(false);
+      input = input0.scalar_type() == kind_of ? input0.contiguous() : input0.to(kind_of).contiguous();
+      std::vector<mellin_stack_layer> call = layers;
+      std::vector<Tensor> dense(2 * n);
+      for (Py_ssize_t i = 0; i < n; ++i) {
+        dense[2 * i] = weights[i].contiguous();
+        call[i].weight = dense[2 * i].const_data_ptr();
+        if (biases[i].defined()) {
+          dense[2 * i + 1] = biases[i].contiguous();
+          call[i].bias = dense[2 * i + 1].const_data_ptr();
+        }
+        kept[i] = dense[2 * i];
+        if (wide && differentiable) {
+          kept[i] = at::empty(weights[i].sizes(), input.options());
+          call[i].weight_half = kept[i].data_ptr();
+        }
+      }
+      const int64_t *d = layers[n - 1].dims;
+      out = at::empty({d[0], d[2], d[7], d[8]}, input.options());
+      saved = scratch(input, saved_bytes);
+      Tensor ws = scratch(input, forward_bytes);
+      check(mellin_stack_forward(kind, elem, differentiable, (int)n, call.data(), pointer(input), out.data_ptr(), saved.data_ptr(),
+                                 saved_bytes, ws.data_ptr(), forward_bytes, launch_stream(input)));
+    }
+    if (differentiable) {
+      auto node = std::shared_ptr<StackBackward>(new StackBackward(), torch::autograd::deleteNode);
+      torch::autograd::edge_list edges;
+      auto edge = [&](const Tensor &t) {
+        edges.push_back(t.defined() && t.requires_grad() ? torch::autograd::impl::gradient_edge(t) : torch::autograd::Edge());
+      };
+      edge(input0);
+      for (Py_ssize_t i = 0; i < n; ++i) {
+        edge(weights[i]);
+        edge(biases[i]);
+        node->weights_.emplace_back(kept[i], false);
+        node->has_bias.push_back(biases[i].defined());
+      }
+      node->set_next_edges(std::move(edges));
+      node->kind = kind;
+      node->elem = elem;
+      node->layers = std::move(layers);
+      node->input_ = torch::autograd::SavedVariable(input, false);
+      node->saved_ = std::move(saved);
+      node->workspace = backward_bytes;
+      node->param_kind = wide ? at::kFloat : kind_of;
+      torch::autograd::set_history(out, node);
+      node->out_ = torch::autograd::SavedVariable(out, true);
+    }
+  }
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"stack", (PyCFunction)(void *)stack, METH_FASTCALL,
+     "stack(kind, input, [(weight, bias, s, d, p, r, pool), ...]): the last layer's output behind its ReLU, or None if not handled"},
     {"corr", (PyCFunction)(void *)corr, METH_FASTCALL,
      "corr(kind, dims, input, weight, bias, s, d, p, u, r, activation): the layer's output, or None if not handled"},
     {nullptr, nullptr, 0, nullptr}};

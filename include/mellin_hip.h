@@ -430,6 +430,32 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
                           void *grad_bias, void *workspace, size_t workspace_bytes,
                           void *stream);
 
+/* A stack of layers, each followed by a ReLU, in one call per direction.  Between layers the tensors stay in the layout of
+ * the matrix kernels (channel-blocked), so nothing is laid out anew, and the backward of the ReLUs, the bias gradients and
+ * the pooling ride along with the kernels.  Layer i reads what layer i - 1 leaves: dims are those of MELLIN_CORR2D_DIMS, in
+ * order; with `pool` its output is first reduced to the maxima of pairs of neighbouring columns (y axis, an odd last one is
+ * dropped; not after the first layer or the last).  elem_bytes as for a layer; weight_half: where the forward call leaves a
+ * float weight rounded to half, which the backward call takes (MELLIN_ELEM_HALF_FLOAT in training; null otherwise);
+ * grad_weight, grad_bias: null for gradients that are not wanted.
+ * mellin_stack_bytes: 1 if the stack can be run so under the settings in force, 0 if not (layers with too few channels for
+ * the blocked kernels behind the first: call them one by one), and the bytes of `saved` (what the forward call keeps: for
+ * the backward call, with train), of the forward call's workspace and of the backward call's; all 256-byte aligned.
+ * out: the last layer's output, as it lies. */
+typedef struct {
+  int64_t dims[17];
+  int pool;
+  const void *weight, *bias;
+  void *weight_half, *grad_weight, *grad_bias;
+} mellin_stack_layer;
+int mellin_stack_bytes(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers, size_t *saved,
+                       size_t *forward_workspace, size_t *backward_workspace);
+int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers,
+                         const void *input, void *out, void *saved, size_t saved_bytes, void *workspace,
+                         size_t workspace_bytes, void *stream);
+int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin_stack_layer *layers, const void *input,
+                          const void *out, const void *grad_out, const void *saved, size_t saved_bytes, void *grad_input,
+                          void *workspace, size_t workspace_bytes, void *stream);
+
 /* Name of the kernel variant the most recent operator-level call of the
  * process (on any thread: PyTorch runs backward passes on a thread of its own)
  * dispatched to (for tests and profiling): "generic", "mfma" (tiled

@@ -152,8 +152,6 @@ class ConvStack(torch.nn.Module):
                                   d=lay["d"], p=lay["p"], r=lay["r"]))
         if params.seed is not None:
             self.reset_parameters()
-        # (a pool behind the last layer stays outside the call of the whole stack)
-        self._pools = [bool(lay["pool"]) for lay in self.plan[:-1]] + [False]
 
     @property
     def out_channels(self) -> int:
@@ -179,7 +177,7 @@ class ConvStack(torch.nn.Module):
             if (type(conv) is not cls or "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or
                     d["_backward_hooks"] or d["_backward_pre_hooks"]):
                 return False
-        return len(self.convs) == len(self._pools)
+        return len(self.convs) == len(self.plan)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # ReLU, the reference's default (models.py:96-101), is applied by the convolution
@@ -188,8 +186,10 @@ class ConvStack(torch.nn.Module):
         if fused and x.is_cuda and self._plain():
             # the whole stack in one call, its tensors in the kernels' layout from layer to layer
             kind = _hip.AX_MCORR if self.params.mellin else _hip.AX_LCORR
+            # (a pool behind the last layer stays outside)
+            pools = [bool(lay["pool"]) for lay in self.plan[:-1]] + [False]
             y = _native_stack(kind, x, [(conv.weight, conv.bias, conv.s, conv.d, conv.p, conv.r, pool)
-                                         for conv, pool in zip(self.convs, self._pools)])
+                                        for conv, pool in zip(self.convs, pools)])
             if y is not None:
                 return freq_max_pool(y) if self.plan[-1]["pool"] else y
         for lay, conv in zip(self.plan, self.convs):

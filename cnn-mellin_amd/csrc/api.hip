@@ -1551,10 +1551,17 @@ int mellin_corr2d_backward_weight_f64(int kind_x, const double *input,
 static size_t blocked_region(i64 batch, i64 channels, i64 plane, bool half) {
   return align256(blocked_bytes(batch, channels, plane, half));
 }
+// A stack's backward call goes on from tensors that its forward call has blocked, whatever has been set since.
+static thread_local bool g_settled = false;
+struct Settled {
+  const bool before = g_settled;
+  explicit Settled(bool on) { g_settled = before || on; }
+  ~Settled() { g_settled = before; }
+};
 // Whether the settings in force leave the layer entry points their channel-blocked kernels.
 static bool blocks_allowed(bool half) {
-  return g_forced == 0 && !g_no_blocks && !g_widen && !g_no_classes && !g_all_classes && !g_split_classes && !g_whole_classes &&
-         !g_no_yfold && !g_gather && !g_no_narrow && (half || g_math != MATH_FP32);
+  return g_settled || (g_forced == 0 && !g_no_blocks && !g_widen && !g_no_classes && !g_all_classes && !g_split_classes && !g_whole_classes &&
+         !g_no_yfold && !g_gather && !g_no_narrow && (half || g_math != MATH_FP32));
 }
 // Plans of the layer entry points, kept per thread: a layer asks for the same ones with every step (its workspace, then
 // the launch), and choosing among tile shapes takes some microseconds.  A place for each of the last sizes; the sizes
@@ -1936,6 +1943,7 @@ static bool plan_stack(int kind_x, int elem, bool train, int n, const mellin_sta
 int mellin_stack_bytes(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers, size_t *saved,
                        size_t *forward_workspace, size_t *backward_workspace) {
   StackPlan sp;
+  const Settled settled(train == 2);
   if (!layer_elements(elem_bytes) || !layers || !plan_stack(kind_x, elem_bytes, train != 0, n_layers, layers, sp)) return 0;
   *saved = sp.saved;
   *forward_workspace = sp.forward;
@@ -2013,6 +2021,7 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
                           size_t workspace_bytes, void *stream) {
   StackPlan sp;
   if (!layer_elements(elem_bytes)) return bad_elements(__func__, elem_bytes);
+  const Settled settled(true);
   const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT;
   const bool planned = layers && plan_stack(kind_x, elem_bytes, true, n_layers, layers, sp);
   int rc = stack_checks(__func__, planned, sp, saved, saved_bytes, workspace, workspace_bytes, sp.backward);

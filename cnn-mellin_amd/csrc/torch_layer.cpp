@@ -10,8 +10,11 @@
 // stack(...) is the same for a stack of layers with ReLUs (conv_stack.py), whose tensors then stay
 // in the kernels' own layout from layer to layer.
 #include <ATen/ATen.h>
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
@@ -19,6 +22,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <algorithm>
 #include <mutex>
@@ -132,12 +136,24 @@ int64_t valid_size(int kind, int64_t nf, int64_t ng, int64_t s, int64_t d, int64
   return v > 0 ? v : 0;
 }
 
-// Whether the library's float and half kernels take `t` (and nothing watches it that this path does not serve).
-bool plain(const Tensor &t) { return t.is_cuda() && t.layout() == at::kStrided && !t._fw_grad(0).defined(); }
+// Whether the library's float and half kernels take `t`: memory of its own as it lies (no wrapper of a function
+// transform, no view that negates) and no tangent.
+bool plain(const Tensor &t) {
+  using K = c10::DispatchKey;
+  constexpr c10::DispatchKeySet wrapped({K::Python, K::FuncTorchBatched, K::BatchedNestedTensor, K::Batched, K::FuncTorchGradWrapper,
+                                         K::Functionalize, K::ZeroTensor, K::Negative, K::Conjugate});
+  return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(wrapped) && !t._fw_grad(0).defined();
+}
+// Whether someone follows the calls one by one (a tracer, a dispatch mode, a function transform); they are shown
+// torch.autograd.Function, which they know.
+bool followed() {
+  return torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
 
 PyObject *corr(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  if (n_args != 11) Py_RETURN_NONE;
+  if (n_args != 11 || followed()) Py_RETURN_NONE;
   Geometry g;
   g.kind = (int)PyLong_AsLong(args[0]);
   const int dims = (int)PyLong_AsLong(args[1]);
@@ -287,17 +303,27 @@ struct StackBackward : public torch::autograd::Node {
         call[i].grad_bias = result[2 + 2 * i].data_ptr();
       }
     }
-    Tensor ws = scratch(input, workspace);
-    check(mellin_stack_backward(kind, elem, (int)n, call.data(), pointer(input), pointer(out), pointer(grad_out), saved.const_data_ptr(),
-                                (size_t)saved.numel(), result[0].defined() ? result[0].data_ptr() : nullptr, ws.data_ptr(), workspace,
-                                launch_stream(input)));
+    auto launch = [&](size_t bytes) {
+      Tensor ws = scratch(input, bytes);
+      return mellin_stack_backward(kind, elem, (int)n, call.data(), pointer(input), pointer(out), pointer(grad_out), saved.const_data_ptr(),
+                                   (size_t)saved.numel(), result[0].defined() ? result[0].data_ptr() : nullptr, ws.data_ptr(), bytes,
+                                   launch_stream(input));
+    };
+    int rc = launch(workspace);
+    if (rc == MELLIN_ERR_WORKSPACE) {                  // (refused before any launch: a setting for the first layer has changed since)
+      size_t ignored[2], bytes = 0;
+      if (mellin_stack_bytes(kind, elem, 2, (int)n, call.data(), &ignored[0], &ignored[1], &bytes)) rc = launch(bytes);
+    }
+    check(rc);
     return result;
   }
 };
 
 PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  if (n_args != 3 || !THPVariable_CheckExact(args[1]) || !PyList_CheckExact(args[2])) Py_RETURN_NONE;
+  if (n_args != 3 || !THPVariable_CheckExact(args[1]) || !PyList_CheckExact(args[2]) || followed()) Py_RETURN_NONE;
+  // (hooks on saved tensors expect the layers' inputs, as the layers themselves save them)
+  if (at::GradMode::is_enabled() && at::SavedTensorDefaultHooks::get_hooks()) Py_RETURN_NONE;
   const int kind = (int)PyLong_AsLong(args[0]);
   const Tensor &input0 = THPVariable_Unpack(args[1]);
   const Py_ssize_t n = PyList_GET_SIZE(args[2]);
@@ -318,7 +344,7 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     PyObject *t = PyList_GET_ITEM(args[2], i);
     if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != 7) Py_RETURN_NONE;
     PyObject *w = PyTuple_GET_ITEM(t, 0), *b = PyTuple_GET_ITEM(t, 1);
-    if (!THPVariable_Check(w) || !(b == Py_None || THPVariable_Check(b))) Py_RETURN_NONE;
+    if (!THPVariable_CheckExact(w) || !(b == Py_None || THPVariable_CheckExact(b))) Py_RETURN_NONE;
     weights[i] = THPVariable_Unpack(w);
     if (b != Py_None) biases[i] = THPVariable_Unpack(b);
     const Tensor &wt = weights[i], &bt = biases[i];

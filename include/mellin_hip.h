@@ -440,6 +440,8 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
  * mellin_stack_bytes: 1 if the stack can be run so under the settings in force, 0 if not (layers with too few channels for
  * the blocked kernels behind the first: call them one by one), and the bytes of `saved` (what the forward call keeps: for
  * the backward call, with train), of the forward call's workspace and of the backward call's; all 256-byte aligned.
+ * train = 2: for the backward call of a forward call already made, which goes on whatever has been set since (the first
+ * layer's kernels follow the settings, so its workspace may have another size).
  * out: the last layer's output, as it lies. */
 typedef struct {
   int64_t dims[17];

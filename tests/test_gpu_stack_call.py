@@ -1,8 +1,13 @@
 """`ConvStack` through one call per direction (tensors blocked from layer to layer, ReLU masks, bias gradients and pooling
 inside the kernels) against the same layers called one by one, which the checker covers."""
+import io
+
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
+import _mellin_hip as hip
+import mconv
 from conv_stack import ConvStack, ConvStackParams
 
 pytestmark = pytest.mark.gpu
@@ -73,3 +78,70 @@ def test_stack_gives_the_gradients_that_are_asked_for():
     out = stack(x.detach())
     out.backward(grad)
     assert stack.convs[0].weight.grad is None and torch.equal(stack.convs[1].weight.grad, full[2])
+
+
+def _small_stack():
+    torch.manual_seed(5)
+    stack = ConvStack(60, 20, ConvStackParams(layers=4, mellin=True, kernel_time=3, kernel_freq=3, initial_channels=24,
+                                              factor_schedule=2, time_factor=1, in_channels=3)).cuda()
+    return stack, torch.randn(2, 3, 60, 20, device="cuda", requires_grad=True)
+
+
+def test_hooks_on_saved_tensors_see_the_layers_own():
+    stack, x = _small_stack()
+    want = torch.autograd.grad(stack(x).square().sum(), list(stack.parameters()) + [x])
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(t.dtype), t.cpu())[1], lambda t: t.cuda()):
+        out = stack(x)
+    assert "StackBackward" not in out.grad_fn.name() and set(seen) == {torch.float32}
+    got = torch.autograd.grad(out.square().sum(), list(stack.parameters()) + [x])
+    for a, b in zip(got, want):
+        assert float((a - b).norm()) <= 4e-6 * float(b.norm())     # (two orders of float32 sums, through four layers)
+    layer = stack.convs[1]
+    seen.clear()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(tuple(t.shape)), t)[1], lambda t: t):
+        layer(torch.randn(2, 24, 60, 20, device="cuda", requires_grad=True), activation="relu")
+    assert len(seen) == 3                                          # input, weight, output
+
+
+def test_settings_changed_between_the_directions():
+    stack, x = _small_stack()
+    grad = torch.randn_like(stack(x))
+    leaves = list(stack.parameters()) + [x]
+    want = torch.autograd.grad(stack(x), leaves, grad)
+    out = stack(x)
+    assert "StackBackward" in out.grad_fn.name()
+    try:
+        hip.set_math(hip.MATH_FP32)
+        got = torch.autograd.grad(out, leaves, grad)
+    finally:
+        hip.set_math(hip.MATH_BF16X3)
+    for a, b in zip(got, want):
+        assert float((a - b).norm()) <= 2e-6 * float(b.norm())
+
+
+def test_whoever_follows_the_calls_is_shown_the_autograd_function():
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    stack, x = _small_stack()
+    plain = stack(x)
+    with Mode():
+        out = stack(x)
+        one = mconv.mcorrlcorr(x, stack.convs[0].weight)
+    assert "StackBackward" in plain.grad_fn.name() and "Corr2dFunction" in out.grad_fn.name() and "Corr2dFunction" in one.grad_fn.name()
+    assert float((out - plain).detach().norm()) <= 1e-6 * float(plain.detach().norm())
+    for transform in (torch.func.vmap(lambda v: mconv.mcorrlcorr(v[None], stack.convs[0].weight)),
+                      torch.func.grad(lambda v: mconv.mcorrlcorr(v, stack.convs[0].weight).sum())):
+        with pytest.raises(RuntimeError):
+            transform(x.detach())
+
+
+def test_a_stack_read_from_a_file_runs():
+    stack, x = _small_stack()
+    file = io.BytesIO()
+    torch.save(stack, file)                                        # (written and read here)
+    file.seek(0)
+    again = torch.load(file, weights_only=False)
+    assert torch.equal(again(x), stack(x))

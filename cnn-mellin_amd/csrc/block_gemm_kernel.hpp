@@ -329,6 +329,11 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   };
 
   floatx16 acc[MT][NT];
+  // fp32: sums of their own for the small products (of the largest tiles they take the last registers).  Error against 64
+  // bits of 64 -> 128 channels, 5 x 3 taps, in the 2-norm: output 4.1e-7 -> 1.4e-7, input gradient 4.3e-7 -> 1.6e-7; time of
+  // a ten-layer stack's step 13.57 -> 13.58 ms.
+  constexpr bool LOW = !F16;
+  floatx16 low[LOW ? MT : 1][LOW ? NT : 1];
   int lane_vpos[NT], lane_q[NT];
   struct Operands { uintx4 a[MT][PARTS]; };
   struct SignalOps { uintx4 b[NT][PARTS]; };
@@ -365,6 +370,13 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       plp = (ConstBlockPlan *)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + zero);
     }
     if (first) {
+      if constexpr (LOW)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) low[i][t][r] = 0.f;
       // position -> virtual position of its (first filter row, first column) tap; accumulators start from the bias
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
@@ -422,18 +434,22 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
     // after next behind them (pinned: the scheduler moves reads next to their use).  Nothing here depends on which
     // step it is, so that every wait counts exactly what is younger: the last pair's last signal reads are of no use,
     // and its fragment fetches are the next stage's.
+    auto multiply = [&](const Operands &a, const SignalOps &b) {
+      if constexpr (LOW) block_multiply_low<MT, NT>(acc, low, a.a, b.b);
+      else block_multiply<MT, NT, PARTS>(acc, a.a, b.b);
+    };
     int2 e2 = ep[4 * WK];
     for (int i = 0; i + 1 < steps; i += 2) {
       fetch_b(e1, B1);
       const int2 e3 = ep[6 * WK];
       __builtin_amdgcn_sched_barrier(0);
-      block_multiply<MT, NT, PARTS>(acc, A0.a, B0.b);
+      multiply(A0, B0);
       __builtin_amdgcn_sched_barrier(0);
       fetch_a(e2, i + 2 < steps ? af_c : n_af, A0);
       fetch_b(e2, B0);
       const int2 e4 = ep[8 * WK];
       __builtin_amdgcn_sched_barrier(0);
-      block_multiply<MT, NT, PARTS>(acc, A1.a, B1.b);
+      multiply(A1, B1);
       __builtin_amdgcn_sched_barrier(0);
       fetch_a(e3, i + 3 < steps ? af_c : n_af, A1);
       e0 = e2;
@@ -443,7 +459,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
     }
     if (steps & 1) {
       // one step left, whose operands are in A0 and B0; A1 holds the next stage's first fragments where its second's belong
-      block_multiply<MT, NT, PARTS>(acc, A0.a, B0.b);
+      multiply(A0, B0);
       e0 = e1;
       e1 = e2;
       fetch_a(e0, n_af, A0);
@@ -455,6 +471,14 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
     first = last;
     if (last) {
       // ---- the tile is finished
+      if constexpr (LOW)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            acc[i][t] += low[i][t];
+            asm volatile("" : "+v"(acc[i][t]));        // (here, not next to their uses: `low` ends here)
+          }
       if constexpr (WK > 1) {
         // sums of the wavefronts, in their order (one tile per workgroup: the buffers are free)
         float *red = (float *)bufs;
@@ -696,9 +720,7 @@ hipError_t launch_shape(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t
   MELLIN_BLOCK_CASE(2, 1, 1, 1)
   MELLIN_BLOCK_CASE(1, 2, 1, 1)
   MELLIN_BLOCK_CASE(1, 1, 1, 1)
-  MELLIN_BLOCK_CASE(2, 2, 1, 4)
   MELLIN_BLOCK_CASE(2, 1, 1, 4)
-  MELLIN_BLOCK_CASE(1, 2, 1, 4)
   MELLIN_BLOCK_CASE(1, 1, 1, 4)
 #undef MELLIN_BLOCK_CASE
   return hipErrorInvalidValue;

@@ -47,6 +47,10 @@ __device__ __forceinline__ void read_transposed(unsigned at, unsigned &lo, unsig
   hi = w.y;
 }
 
+// Tiles of a wavefront that leave registers for separate sums of the small products (block_multiply_low).  Error of the
+// weight gradient against 64 bits, 64 -> 64 channels, 4 x 4 taps, 8 x 390 x 20 positions: 2.7e-7 -> 1.3e-7, at the same time.
+constexpr int kLowTiles = 4;
+
 // NW: wavefronts of a workgroup -- four, two workgroups to a CU, or eight where a stage's operands leave room for
 // one workgroup only
 template <int MT, int NT, int NW, bool F16>
@@ -154,6 +158,14 @@ __global__ __launch_bounds__(NW * 64, 2) void block_wgrad_kernel(BlockWgradPlan 
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][t][r] = 0.f;
+  // fp32: sums of their own for the small products, where registers allow
+  constexpr bool LOW = !F16 && MT * NT <= kLowTiles;
+  floatx16 low[LOW ? MT : 1][LOW ? NT : 1];
+  if constexpr (LOW)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) low[i][t] = acc[i][t];
 
   // transposing reads: lane -> position (4 in a read), channel pair of groups and half unit
   const int j16 = lane >> 4, l16 = lane & 15;
@@ -205,22 +217,31 @@ __global__ __launch_bounds__(NW * 64, 2) void block_wgrad_kernel(BlockWgradPlan 
           o.b[t][p] = uintx4{w0, w1, w2, w3};
         }
     };
+    auto multiply = [&](const Ops &o) {
+      if constexpr (LOW) block_multiply_low<MT, NT>(acc, low, o.a, o.b);
+      else block_multiply<MT, NT, PARTS>(acc, o.a, o.b);
+    };
     Ops o0, o1;
     fetch(0, o0);
 #pragma unroll
     for (int s = 0; s < KS / 16; s += 2) {
       fetch(s + 1, o1);
       __builtin_amdgcn_sched_barrier(0);
-      block_multiply<MT, NT, PARTS>(acc, o0.a, o0.b);
+      multiply(o0);
       __builtin_amdgcn_sched_barrier(0);
       if (s + 2 < KS / 16) fetch(s + 2, o0);
       __builtin_amdgcn_sched_barrier(0);
-      block_multiply<MT, NT, PARTS>(acc, o1.a, o1.b);
+      multiply(o1);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (u + 2 < u_hi) build_tables(u + 2);
   }
 
+  if constexpr (LOW)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[i][t] += low[i][t];
   // ---- the partial block: [channel of the block][column tile (input channels, filter column)][32]
   const int l32 = lane & 31, half = lane >> 5;
   const int cols = pl.ctb * pl.nfy * 32;
@@ -336,9 +357,11 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
   if (best == 0) return false;
   pl.mgt = pl.wm * pl.mt * 4;
   pl.cgt = pl.ctb * 4;
-  // slices: two workgroups per CU in all, dealt to the filter rows by their positions
-  const int blocks = pl.m_blocks * pl.c_blocks;
-  const i64 want = std::max<i64>(pl.nfx, (pl.nw == 4 ? 512 : 256) / blocks);
+  // slices: two workgroups per CU in all, dealt to the filter rows by their positions; twice as many, half as long, where a
+  // single accumulator takes all six products of fp32 parts (128 -> 256 channels, 3 x 3 taps, 32 x 256 x 41 positions:
+  // error 2.9e-6 -> 2.1e-6, its sums' launch 22 -> 28 us, 0.2 % of the step)
+  const int blocks = pl.m_blocks * pl.c_blocks, turns = !f16 && pl.mt * pl.nt > kLowTiles ? 2 : 1;
+  const i64 want = std::max<i64>(pl.nfx, (pl.nw == 4 ? 512 : 256) * turns / blocks);
   int total = 0;
   for (int f = 0; f < pl.nfx; ++f) {
     const i64 k = (i64)pl.row[f].count * pl.noy * pl.batch, units = (k + KS - 1) / KS;

@@ -69,6 +69,29 @@ def test_blocked_layers_match_checker(case, kinds, relu):
             assert_close(got, ref, fan, what)
 
 
+@pytest.mark.parametrize("case", [(2, 64, 32, (4, 4), (70, 21)), (2, 64, 64, (4, 4), (70, 21)), (24, 32, 96, (3, 3), (40, 20))],
+                         ids=["32 channels", "64 channels", "many tiles"])
+def test_long_float_sums_are_rounded_once_in_sixteen_products(case):
+    """The small products of the bf16 parts have sums of their own, so a sum of n products is rounded n / 16 times, each time
+    by 2^-24 / sqrt(3) at most in the mean square, of a partial sum that grows with the root of the products: 2^-24 sqrt(n / 96)
+    in the 2-norm, doubled for the partial sums that are added behind it, and 2^-23 for the products themselves."""
+    n, c_in, c_out, nf, ng = case
+    rng = np.random.default_rng(91)
+    x = rng.standard_normal((n, c_in) + ng).astype(np.float32)
+    w = rng.standard_normal((c_out, c_in) + nf).astype(np.float32)
+    exp = oracle.lcorrlcorr(x.astype(np.float64), w.astype(np.float64), None, (1, 1), (1, 1), (1, 1), (1, 1), (1, 1))
+    go = rng.standard_normal(exp.shape).astype(np.float32)
+    egi, egw, _ = oracle.lcorrlcorr_backward(x.astype(np.float64), w.astype(np.float64), go.astype(np.float64), (1, 1), (1, 1), (1, 1), (1, 1))
+    xg, wg = to_gpu(x).requires_grad_(), to_gpu(w).requires_grad_()
+    out = mconv._ext_lcorrlcorr(xg, wg, None, (1, 1), (1, 1), (1, 1), (1, 1), (1, 1))
+    assert hip.last_variant() == "mfma-blocks"
+    out.backward(to_gpu(go))
+    taps = nf[0] * nf[1]
+    for got, ref, terms in ((out, exp, c_in * taps), (xg.grad, egi, c_out * taps), (wg.grad, egw, n * exp.shape[2] * exp.shape[3])):
+        err = np.linalg.norm(got.detach().double().cpu().numpy() - ref) / np.linalg.norm(ref)
+        assert err <= 2.0 ** -24 * (2 * (terms / 96) ** 0.5 + 2), (err, terms)
+
+
 def test_blocked_passes_repeat_bit_for_bit_and_replay_in_a_graph():
     gen = torch.Generator(device="cuda").manual_seed(3)
     x = torch.randn(3, 24, 50, 21, device="cuda", generator=gen)

@@ -205,13 +205,15 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
     pl.slice_bytes = (size_t)pl.rest * pl.slices * pl.m_tiles * (size_t)(M_T * P) * 4;
     return best;
   };
-  // (wavefronts that share a tile have 32 positions of it: 64 leave no registers for a gradient's ending beside the separate
-  // sums, and were slower as they were -- windows of ten frames 2111 -> 1998 us a step, one utterance decoded 246 -> 233 us)
-  static const int shapes[][3] = {{4, 2, 1}, {4, 1, 1}, {2, 1, 1}, {1, 1, 1}, {1, 1, 4}};   // nt, wm, wk
+  // Wavefronts that share a tile have 32 positions of it in fp32: 64 leave no registers for a gradient's ending beside the
+  // separate sums, and were slower as they were (windows of ten frames 2111 -> 1998 us a step, one utterance decoded 246 ->
+  // 233 us).  Half has the registers, and its shorter steps are better shared (1-D layer, 41 -> 128 channels: 15.1 us
+  // without the 64 positions, 10.7 with them).
+  static const int shapes[][3] = {{4, 2, 1}, {4, 1, 1}, {2, 1, 1}, {1, 1, 1}, {2, 1, 4}, {1, 1, 4}};   // nt, wm, wk
   BlockPlan best_plan;
   double best_cost = 0;
   for (const auto &sh : shapes) {
-    if (sh[0] == 4 && !f16) continue;
+    if (!f16 && (sh[0] == 4 || (sh[0] == 2 && sh[2] == 4))) continue;
     if (sh[1] == 2 && pr.c_out <= 96) continue;        // (two wavefronts along the channels: most of 128)
     if (!shape(sh[0], sh[1], sh[2])) continue;
     const double c = cost();

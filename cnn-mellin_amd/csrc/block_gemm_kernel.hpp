@@ -716,6 +716,8 @@ hipError_t launch_shape(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t
     if (pl.mt == 2) return launch_instance<2, 4, 1, 1, true, OUT>(pl, a, stream);
     return launch_instance<1, 4, 1, 1, true, OUT>(pl, a, stream);
   }
+  if (pl.f16 && pl.nt == 2 && pl.wk == 4)
+    return pl.mt == 2 ? launch_instance<2, 2, 1, 4, true, OUT>(pl, a, stream) : launch_instance<1, 2, 1, 4, true, OUT>(pl, a, stream);
   MELLIN_BLOCK_CASE(2, 2, 1, 1)
   MELLIN_BLOCK_CASE(2, 1, 1, 1)
   MELLIN_BLOCK_CASE(1, 2, 1, 1)

@@ -30,7 +30,7 @@
 //
 // Measured, 256 -> 256 channels, 4 x 4 taps, 16 x 100 x 41 positions, linear: fp32 1312 -> 1190 us and 107 us
 // for the cut (six bf16 products each: 1.39 PF, matrix pipe 57 % busy at 1.9 GHz, near the rate the board's
-// power allows); half, on Mellin rows, 286 -> 183 us.  One utterance (few tiles, WK = 4): 980 -> 330 us for ten layers.
+// power allows); half, on Mellin rows, 286 -> 183 us.  One utterance (few tiles, WK = 4): 1039 -> 229 us for ten layers.
 #pragma once
 
 #include <type_traits>

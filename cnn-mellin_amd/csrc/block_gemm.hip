@@ -156,32 +156,68 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   };
   auto magic = [](i64 d) { return d <= 1 ? 0xFFFFFFFFu : (unsigned)(0x100000000ull / (unsigned)d); };
   pl.mg_batch = magic(pl.batch); pl.mg_noy = magic(pl.noy);
-  double rows_used = pl.nfx;                           // filter rows of an output row, on average
-  if (mellin) {
-    rows_used = 0;
-    for (int k = 0; k < pl.n_classes; ++k)
-      rows_used += __builtin_popcount(pl.cls[k].mask) * (double)((k + 1 < pl.n_classes ? pl.cls[k + 1].start : pl.nox) - pl.cls[k].start);
-    rows_used = std::max(1.0, rows_used / pl.nox);
-  }
+  // Mellin axes: which filter rows have a tap inside the signal, per output row in the order of the classes (axes of
+  // more rows, of which a tile's share a class: those of the class)
+  constexpr int kMaskRows = 4096;
+  unsigned row_mask[kMaskRows];
+  const bool masks = mellin && pl.nox <= kMaskRows;
+  double class_rows = 0;
+  if (mellin)
+    for (int k = 0; k < pl.n_classes; ++k) {
+      const int end = k + 1 < pl.n_classes ? pl.cls[k + 1].start : pl.nox;
+      class_rows += __builtin_popcount(pl.cls[k].mask) * (double)(end - pl.cls[k].start) / pl.nox;
+      for (int at = pl.cls[k].start; masks && at < end; ++at) {
+        const unsigned h = (unsigned)(pl.cls[k].first + (at - pl.cls[k].start) * pl.cls_stride + pl.sx), p1 = (unsigned)pl.px + 1;
+        unsigned mask = 0;
+        for (int f = 0; f < pl.nfx; ++f) {
+          const unsigned fd = (unsigned)(f + pl.dx), num = X.kind == AX_MCORR ? h * fd : h * p1, den = X.kind == AX_MCORR ? p1 : fd;
+          const unsigned q = num / den;
+          if (q * den == num && q >= (unsigned)pl.ux && q - (unsigned)pl.ux < (unsigned)pl.ngx) mask |= 1u << f;
+        }
+        row_mask[at] = mask;
+      }
+    }
+  // What a tile of P positions stages: filter rows, and stages of them, on average.  (Counted over the tile's rows together:
+  // with the average of single rows small images of many classes got tiles that stage nearly every filter row; windows of
+  // ten frames 1989 -> 1968 us a step, a ten-layer Mellin stack of 24 to 192 channels on two utterances 1175 -> 1117 us.)
+  auto tile_rows = [&](int P, double &filter_rows, double &subsets) {
+    filter_rows = mellin ? std::max(1.0, class_rows) : pl.nfx;
+    subsets = mellin ? std::ceil(filter_rows / pl.F) : 1;
+    if (!masks) return;
+    i64 rows = 0, stages = 0, tiles = 0;
+    for (i64 q0 = 0; q0 < Q; q0 += P, ++tiles) {
+      const i64 last = (std::min<i64>(q0 + P, Q) - 1) / pl.noy;
+      unsigned mask = 0;
+      for (i64 r = q0 / pl.noy; r <= last; ++r) mask |= row_mask[r];
+      const int n = std::max(1, __builtin_popcount(mask));
+      rows += n;
+      stages += (n + pl.F - 1) / pl.F;
+    }
+    filter_rows = (double)rows / tiles;
+    subsets = (double)stages / tiles;
+  };
 
   // The launch of a tile shape, in cycles.  Workgroups take tiles in turn, two to a CU (512 at a time).  What does not fill
   // a last turn -- for few tiles: all of them -- can be cut into slices of the contracted channels, which another kernel
   // adds up.  Measured on this chip, and rounded:
   //   a step's matrix instructions at 65-80 % of their rate (larger tiles: the higher), shared by a CU's workgroups;
   //   a stage at least 4000 (the latency of its loads);
-  //   per tile 5000 for its tables and its output at 9 bytes a cycle; 9000 for a launch's start, as much for the kernel
-  //   that adds the slices, and 2400 bytes a cycle for their sums.
+  //   per tile 5000 for its tables (9000 where wavefronts share it: nothing runs under them) and its output at 9 bytes a
+  //   cycle; 9000 for a launch's start, as much for the kernel that adds the slices, and 2400 bytes a cycle for their sums.
   const i64 slots = 512;
   auto cost = [&]() {
     const int M_T = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32;
     const i64 total = (i64)((Q + P - 1) / P) * pl.batch, per_m = std::max<i64>(1, slots / pl.m_tiles), c_stages = pl.CG / pl.G;
-    const double subsets = mellin ? std::max(1.0, std::ceil(rows_used / pl.F)) : 1, rows = rows_used / subsets;
+    double filter_rows, subsets;
+    tile_rows(P, filter_rows, subsets);
+    const double rows = filter_rows / subsets;
     const double rate = pl.mt * pl.nt >= 8 ? 0.8 : pl.mt * pl.nt >= 4 ? 0.65 : 0.55;
     const double steps = std::ceil(rows * pl.nfy * pl.G / (2 * pl.wk)) * pl.mt * pl.nt * (f16 ? 1 : 6) * 32 / rate;
     const double output = (double)M_T * P * (f16 ? 2 : 4) / 9;
+    const double tile = pl.wk > 1 ? 9000 : 5000;
     auto turns_cost = [&](i64 items, double stages) {
       const i64 full = items / per_m, left = items - full * per_m;
-      auto turn = [&](i64 n) { return stages * std::max(4000.0, steps * (n * pl.m_tiles > slots / 2 ? 2 : 1)) + 5000 + output; };
+      auto turn = [&](i64 n) { return stages * std::max(4000.0, steps * (n * pl.m_tiles > slots / 2 ? 2 : 1)) + tile + output; };
       return full * turn(per_m) + (left ? turn(left) : 0);
     };
     double best = 9000 + turns_cost(total, c_stages * subsets);

@@ -127,6 +127,10 @@ __device__ void finish_units(const FinishArgs &a, int b, float (*red)[32]) {
     for (int k = 0; k < pl.slices; ++k)
 #pragma unroll
       for (int c = 0; c < 8; ++c) v[c] += from[k * slice + c * P];
+    // (channels past the last have no sums: the matrix kernel's stores end with the last channel, and what the workspace
+    // held there must not become a blocked tensor's padding)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = group * 8 + c < pl.M ? v[c] : 0.f;
     const int row = (q0 + p) / pl.noy, oy = q0 + p - row * pl.noy;
     q = (a.s_rows ? a.s_rows[row].x : row) * pl.noy + oy;
     const i64 unit = ((i64)n * pl.out_groups + group) * (pl.Q + 1) + q;

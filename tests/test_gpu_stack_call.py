@@ -1,5 +1,6 @@
 """`ConvStack` through one call per direction (tensors blocked from layer to layer, ReLU masks, bias gradients and pooling
 inside the kernels) against the same layers called one by one, which the checker covers."""
+import ctypes
 import io
 
 import pytest
@@ -145,3 +146,60 @@ def test_a_stack_read_from_a_file_runs():
     file.seek(0)
     again = torch.load(file, weights_only=False)
     assert torch.equal(again(x), stack(x))
+
+
+class _Layer(ctypes.Structure):
+    """mellin_stack_layer of include/mellin_hip.h."""
+    _fields_ = [("dims", ctypes.c_int64 * 17), ("pool", ctypes.c_int)] + [
+        (name, ctypes.c_void_p) for name in ("weight", "bias", "weight_half", "grad_weight", "grad_bias")]
+
+
+@pytest.mark.parametrize("mellin,channels,frames,half", [(True, 100, 337, False), (False, 36, 100, False), (True, 100, 337, True),
+                                                         (False, 100, 337, True)])
+def test_channels_past_the_last_are_zeros_whatever_the_scratch_memory_held(mellin, channels, frames, half):
+    """One utterance, channel counts that are no multiple of eight: the layers' sums come in slices through the workspace, and
+    the rest of a layer's last group of eight channels has no sums there.  What the scratch memory held -- large values, which
+    are infinities in half precision, infinities and NaN -- must not pass into a result."""
+    kind, elem, dtype = (hip.AX_MCORR if mellin else hip.AX_LCORR), (2 if half else 4), (torch.float16 if half else torch.float32)
+    torch.manual_seed(70)
+    stack = ConvStack(frames, 41, ConvStackParams(layers=5, mellin=mellin, initial_channels=channels, time_factor=1, in_channels=3,
+                                                  freq_pool_after=(3,)))
+    n, c, x, y = len(stack.plan), 3, frames, 41
+    layers, tensors, sliced = (_Layer * n)(), [], []
+    for i, (lay, conv) in enumerate(zip(stack.plan, stack.convs)):
+        co, (nf, nhy) = lay["out_channels"], (lay["kernel"], lay["out_size"][1])
+        nh = (lay["out_size"][0], y if lay["pool"] else nhy)
+        dims = hip._dims(1, c, co, nf, (x, y), nh, lay["s"], lay["d"], lay["p"], (1, 1))
+        w = torch.empty(co, c, *nf, device="cuda").uniform_(-1, 1).mul_((6 / (c * nf[0] * nf[1])) ** 0.5).to(dtype)
+        b = torch.empty(co, device="cuda").uniform_(0, 0.1).to(dtype)
+        gw, gb = torch.empty_like(w), torch.empty_like(b)
+        layers[i].dims[:], layers[i].pool = list(dims), int(lay["pool"])
+        layers[i].weight, layers[i].bias, layers[i].grad_weight, layers[i].grad_bias = (t.data_ptr() for t in (w, b, gw, gb))
+        tensors.append((w, b, gw, gb))
+        if i:
+            # what a layer's workspace has beside the blocked signal and filter: the sums of slices
+            unit, groups, up = (16 if half else 48), (c + 7) // 8, lambda v: (v + 255) // 256 * 256
+            filters = 2 * ((co + 63) // 64) * (groups * nf[0] * nf[1] + 1) * 32 * unit + (8 * nh[0] if mellin else 0)
+            sliced.append(hip.lib.mellin_layer_forward_workspace(kind, elem, *dims) - up(groups * (x * y + 1) * unit) - up(filters) > 0)
+        c, x, y = co, lay["out_size"][0], nhy
+    assert any(sliced[:-1])                            # (the last layer's output is not blocked)
+    inp = torch.randn(1, 3, frames, 41, device="cuda").to(dtype)
+    out = torch.empty(1, c, x, y, device="cuda", dtype=dtype)
+    grad, gi = torch.randn_like(out), torch.empty_like(inp)
+    sizes = [ctypes.c_size_t() for _ in range(3)]
+    assert hip.lib.mellin_stack_bytes(kind, elem, 1, n, layers, *(ctypes.addressof(s) for s in sizes)) == 1
+    saved, fw, bw = (torch.empty(max(s.value, 4) // 4, device="cuda") for s in sizes)
+    results = []
+    for held in (0.0, 1e30, float("inf"), float("nan")):
+        for t in (saved, fw, bw):
+            t.fill_(held)
+        for t in [out, gi] + [g for ts in tensors for g in ts[2:]]:
+            t.fill_(float("nan"))
+        hip._check(hip.lib.mellin_stack_forward(kind, elem, 1, n, layers, hip._dp(inp), hip._dp(out), hip._dp(saved), sizes[0].value,
+                                                hip._dp(fw), sizes[1].value, hip._stream(inp.device)))
+        hip._check(hip.lib.mellin_stack_backward(kind, elem, n, layers, hip._dp(inp), hip._dp(out), hip._dp(grad), hip._dp(saved),
+                                                 sizes[0].value, hip._dp(gi), hip._dp(bw), sizes[2].value, hip._stream(inp.device)))
+        results.append([t.clone() for t in [out, gi] + [g for ts in tensors for g in ts[2:]]])
+    assert all(bool(t.isfinite().all()) for t in results[0]) and bool((results[0][0] > 0).any())
+    for other in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(results[0], other))

@@ -1673,7 +1673,7 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
       return fail(MELLIN_ERR_ARGUMENT, "%s: activation must be MELLIN_ACT_NONE or MELLIN_ACT_RELU (got %d)", __func__, activation);
     bp.relu = activation == MELLIN_ACT_RELU;
     bp.wide = wide;
-    g_variant = half ? "mfma-f16" : "mfma-blocks";
+    g_variant = half ? "mfma-f16-blocks" : "mfma-blocks";
     g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
     char *ws = (char *)workspace;
     float *sums = (float *)(ws + signal + filter);
@@ -1805,7 +1805,7 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   if (!lb.input_blocked && !lb.weight_blocked) return MELLIN_OK;
   if (!grad_out || (lb.input_blocked && !weight) || (lb.weight_blocked && !input))
     return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
-  g_variant = half ? "mfma-f16" : "mfma-blocks";
+  g_variant = half ? "mfma-f16-blocks" : "mfma-blocks";
   g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
   const bool sums = !lb.plain && (want & MELLIN_WANT_BIAS);
   const PackSignal go = {grad_out, relu && !lb.plain ? out : nullptr, ws + lb.go_off, sums ? (float *)(ws + lb.bias_off) : nullptr,
@@ -2011,7 +2011,7 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
       e = launch_block_pool(half, to, l.batch, l.c_out, l.rows, l.cols, keep + sp.l[i + 1].x_off,
                             train ? keep + sp.l[i + 1].which_off : nullptr, st);
   }
-  g_variant = half ? "mfma-f16" : "mfma-blocks";
+  g_variant = half ? "mfma-f16-blocks" : "mfma-blocks";
   g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
   return check_hip(e, __func__);
 }
@@ -2104,7 +2104,7 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
       if (rc) return rc;
     }
   }
-  g_variant = half ? "mfma-f16" : "mfma-blocks";
+  g_variant = half ? "mfma-f16-blocks" : "mfma-blocks";
   g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
   return MELLIN_OK;
 }

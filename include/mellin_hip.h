@@ -474,9 +474,10 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
  * (row, filter row) pair without a tap), "mfma-f16", "mfma-f16-classes" (the
  * classes of a half-precision layer sharing one launch) and
  * "mfma-f16-class-launches" (a launch each),
- * "mfma-f16-fused", "mfma-f16+fold", "mfma-f16-filter-rows+fold" and, for fp32 layers
- * of section 5 through channel-blocked operands, "mfma-blocks"
- * (half-precision tensors on the f16 matrix cores), "mfma-narrow" (forward pass
+ * "mfma-f16-fused", "mfma-f16+fold", "mfma-f16-filter-rows+fold"
+ * (half-precision tensors on the f16 matrix cores), "mfma-blocks" and
+ * "mfma-f16-blocks" (layers and stacks of section 5 through channel-blocked
+ * operands, fp32 and half-precision tensors), "mfma-narrow" (forward pass
  * of a linear x linear layer with few input channels, bf16 matrix cores) and
  * "lds-gather" (vector-ALU forward kernel, only under mellin_set_variant). */
 const char *mellin_last_variant(void);

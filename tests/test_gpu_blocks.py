@@ -50,9 +50,9 @@ def test_blocked_layers_match_checker(case, kinds, relu):
     call = mconv._ext_mcorrlcorr if op == "mcorr" else mconv._ext_lcorrlcorr
     with torch.autocast("cuda", torch.float16, enabled=kind is not param_kind):
         out = call(xg, wg, bg, s, d, p, (1, 1), r, activation="relu" if relu else None)
-    assert hip.last_variant() == ("mfma-f16" if half else "mfma-blocks")
+    assert hip.last_variant() == ("mfma-f16-blocks" if half else "mfma-blocks")
     out.backward(to_gpu(go))
-    assert hip.last_variant() == ("mfma-f16" if half else "mfma-blocks")
+    assert hip.last_variant() == ("mfma-f16-blocks" if half else "mfma-blocks")
     masked = go.astype(np.float64)
     if relu:
         exp = np.maximum(exp, 0)

@@ -6,7 +6,6 @@
 
 #include <algorithm>
 #include <atomic>
-#include <memory>
 #include <mutex>
 #include <numeric>
 
@@ -17,6 +16,7 @@
 #include "gather_kernels.hpp"
 #include "block_gemm.hpp"
 #include "narrow_gemm.hpp"
+#include "plan_table.hpp"
 
 using namespace mellin;
 
@@ -1564,27 +1564,16 @@ static bool blocks_allowed(bool half) {
          !g_no_yfold && !g_gather && !g_no_narrow && (half || g_math != MATH_FP32));
 }
 // Plans of the layer entry points, kept per thread: a layer asks for the same ones with every step (its workspace, then
-// the launch), and choosing among tile shapes takes some microseconds.  A place for each of the last sizes; the sizes
-// decide the plan, so nothing has to be thrown away.
+// the launch), and choosing among tile shapes takes some microseconds.  The sizes decide the plan, so nothing has to be
+// thrown away.
 struct LayerPlans {
   int known[3];                                        // 0 not yet, 1 applies, -1 does not
   BlockPlan forward, input;
   BlockWgradPlan weight;
 };
 static LayerPlans &layer_plans(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
-  constexpr int kPlaces = 64;
-  struct Place { int64_t key[18]; LayerPlans plans; };
-  static thread_local std::unique_ptr<Place[]> places;
-  if (!places) places.reset(new Place[kPlaces]());
-  const int64_t key[18] = {kind_x * 2 + half + 1, CORR2D_ARGS};
-  uint64_t h = 0;
-  for (int64_t k : key) h = (h ^ (uint64_t)k) * 0x9E3779B97F4A7C15ull, h ^= h >> 29;
-  Place &p = places[h % kPlaces];
-  if (memcmp(p.key, key, sizeof key) != 0) {
-    memcpy(p.key, key, sizeof key);
-    p.plans.known[0] = p.plans.known[1] = p.plans.known[2] = 0;
-  }
-  return p.plans;
+  static thread_local PlanTable<LayerPlans, 64, 18> table;
+  return table.at({kind_x * 2 + half + 1, CORR2D_ARGS});
 }
 // Layers with few channels leave most of a channel block empty, and have kernels of their own in section 2.  Measured over
 // 80 layers with 1 to 15 input channels: for the gradients of short layers, bound by launches (up to these

@@ -1625,6 +1625,17 @@ static bool plan_block_weight(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockWg
   return lp.known[2] > 0;
 }
 
+// A pass's blocked tensor is scratch memory beside the caller's own tensors, in fp32 half as large again as the tensor it was
+// made of.  A layer's forward pass and input gradient therefore take so many images at a time that it stays under 4 GiB (where
+// the weight gradient's 32-bit offsets end as well: beyond, that is a kernel of section 2): a launch of that size takes
+// milliseconds, so nothing is lost by the next one.
+constexpr size_t kMaxBlockedBytes = (size_t)4 << 30;
+static i64 blocked_images(i64 batch, i64 channels, i64 plane, bool half) {
+  if (blocked_bytes(batch, channels, plane, half) <= kMaxBlockedBytes) return batch;
+  const i64 most = std::max<i64>(1, (i64)(kMaxBlockedBytes / blocked_bytes(1, channels, plane, half))), parts = (batch + most - 1) / most;
+  return (batch + parts - 1) / parts;
+}
+
 // the elements of a layer call: 4 float, 2 half, 6 half with float parameters
 static bool layer_elements(int elem) { return elem == 2 || elem == 4 || elem == MELLIN_ELEM_HALF_FLOAT; }
 static int bad_elements(const char *who, int elem) {
@@ -1636,8 +1647,12 @@ size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_
   if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
   const bool half = elem_bytes != 4;
   BlockPlan bp;
-  if (plan_block_forward(kind_x, half, CORR2D_ARGS, bp))
+  if (plan_block_forward(kind_x, half, CORR2D_ARGS, bp)) {
+    const i64 per = blocked_images(batch, c_in, ngx * ngy, half), last = (batch - 1) % per + 1;
+    auto part = [&](i64 batch) { return mellin_layer_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS); };
+    if (per < batch) return std::max(part(per), part(last));
     return blocked_region(batch, c_in, ngx * ngy, half) + align256(bp.filter_bytes) + bp.slice_bytes;
+  }
   if (!half) return mellin_corr2d_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS);
   const size_t own = mellin_corr2d_forward_f16_workspace(kind_x, CORR2D_ARGS);
   return elem_bytes == 2 ? own : align256(own) + align256(c_out * c_in * nfx * nfy * 2) + c_out * 2;
@@ -1654,12 +1669,22 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
   BlockPlan bp;
   if (plan_block_forward(kind_x, half, CORR2D_ARGS, bp)) {
     const size_t signal = blocked_region(batch, c_in, ngx * ngy, half), filter = align256(bp.filter_bytes);
-    const size_t need = signal + filter + bp.slice_bytes;
+    const i64 per = blocked_images(batch, c_in, ngx * ngy, half);
+    const size_t need = per < batch ? mellin_layer_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS) : signal + filter + bp.slice_bytes;
     if (!workspace || workspace_bytes < need)
       return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, need, workspace_bytes);
     if (!input || !weight || !out) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
     if (activation != MELLIN_ACT_NONE && activation != MELLIN_ACT_RELU)
       return fail(MELLIN_ERR_ARGUMENT, "%s: activation must be MELLIN_ACT_NONE or MELLIN_ACT_RELU (got %d)", __func__, activation);
+    if (per < batch) {
+      const i64 size = half ? 2 : 4, x_image = c_in * ngx * ngy * size, h_image = c_out * nhx * nhy * size;
+      auto part = [&](i64 first, i64 batch) {
+        return mellin_layer_forward(kind_x, elem_bytes, activation, (const char *)input + first * x_image, weight, bias, CORR2D_ARGS,
+                                    (char *)out + first * h_image, weight_half, workspace, workspace_bytes, stream);
+      };
+      for (i64 n = 0; n < batch && !rc; n += per) rc = part(n, std::min(per, batch - n));
+      return rc;
+    }
     bp.relu = activation == MELLIN_ACT_RELU;
     bp.wide = wide;
     g_variant = half ? "mfma-f16-blocks" : "mfma-blocks";
@@ -1738,12 +1763,22 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
   lb.pass_off = take(pass);
   lb.total = at;
 }
+// The images that the input gradient takes at a time; less than `batch`: in calls of their own (INPUT_ONLY), beside one for
+// the other gradients (whose kernels are not the blocked ones at such sizes).
+#define INPUT_ONLY(want) ((want) & (MELLIN_WANT_INPUT | MELLIN_WANT_RELU))
+static i64 backward_images(const LayerBackward &lb, bool half, MELLIN_CORR2D_DIMS) {
+  return lb.input_blocked ? blocked_images(batch, c_out, nhx * nhy, half) : batch;
+}
 size_t mellin_layer_backward_workspace(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS) {
   if (!layer_elements(elem_bytes)) return 0;
   if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
   LayerBackward lb;
   plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb);
-  return lb.total;
+  const i64 per = backward_images(lb, elem_bytes != 4, CORR2D_ARGS);
+  if (per == batch) return lb.total;
+  auto part = [&](int want, i64 batch) { return mellin_layer_backward_workspace(kind_x, elem_bytes, want, CORR2D_ARGS); };
+  const size_t need = std::max(part(INPUT_ONLY(want), per), part(INPUT_ONLY(want), (batch - 1) % per + 1));
+  return want & (MELLIN_WANT_WEIGHT | MELLIN_WANT_BIAS) ? std::max(need, part(want & ~MELLIN_WANT_INPUT, batch)) : need;
 }
 int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *input, const void *weight,
                           const void *grad_out, const void *out, MELLIN_CORR2D_DIMS, void *grad_input,
@@ -1756,8 +1791,24 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
     return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
   LayerBackward lb;
   plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb);
-  if (lb.total && (!workspace || workspace_bytes < lb.total))
-    return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, lb.total, workspace_bytes);
+  const i64 per = backward_images(lb, elem_bytes != 4, CORR2D_ARGS);
+  const size_t need = per < batch ? mellin_layer_backward_workspace(kind_x, elem_bytes, want, CORR2D_ARGS) : lb.total;
+  if (need && (!workspace || workspace_bytes < need))
+    return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, need, workspace_bytes);
+  if (per < batch) {
+    if (!grad_out || !weight) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+    if (want & (MELLIN_WANT_WEIGHT | MELLIN_WANT_BIAS))
+      rc = mellin_layer_backward(kind_x, elem_bytes, want & ~MELLIN_WANT_INPUT, input, weight, grad_out, out, CORR2D_ARGS, nullptr,
+                                 grad_weight, grad_bias, workspace, workspace_bytes, stream);
+    const i64 size = elem_bytes == 4 ? 4 : 2, x_image = c_in * ngx * ngy * size, h_image = c_out * nhx * nhy * size;
+    auto part = [&](i64 first, i64 batch) {
+      return mellin_layer_backward(kind_x, elem_bytes, INPUT_ONLY(want), nullptr, weight, (const char *)grad_out + first * h_image,
+                                   out ? (const char *)out + first * h_image : nullptr, CORR2D_ARGS, (char *)grad_input + first * x_image,
+                                   nullptr, nullptr, workspace, workspace_bytes, stream);
+    };
+    for (i64 n = 0; n < batch && !rc; n += per) rc = part(n, std::min(per, batch - n));
+    return rc;
+  }
   char *ws = (char *)workspace, *pass = ws + lb.pass_off;
   const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT, relu = want & MELLIN_WANT_RELU;
   hipStream_t st = (hipStream_t)stream;

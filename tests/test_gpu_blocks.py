@@ -127,6 +127,46 @@ def test_blocked_passes_repeat_bit_for_bit_and_replay_in_a_graph():
         both()
 
 
+@pytest.mark.parametrize("op,half,relu", [("lcorr", False, True), ("mcorr", True, False)], ids=["f32", "amp"])
+def test_layers_whose_blocked_tensors_would_be_huge_go_through_them_in_parts(op, half, relu):
+    """Results of images of every part, and both sides of a part's end, as those of the images alone; the gradients of the
+    parameters as those of a call that wants nothing else."""
+    size = 2 if half else 4
+    image = 2 * (1024 * 41 + 1) * (16 if half else 48)           # blocked bytes of an image of 16 channels
+    n = 2 * ((4 << 30) // image) + 1                             # three parts
+    per = -(-n // 3)
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    dtype = torch.float16 if half else torch.float32
+    x = torch.empty(n, 16, 1024, 41, device="cuda", dtype=dtype).normal_(generator=gen).requires_grad_()
+    w = (torch.randn(16, 16, 3, 3, device="cuda", generator=gen) / 12).requires_grad_()
+    b = torch.randn(16, device="cuda", generator=gen).requires_grad_()
+    call = mconv._ext_mcorrlcorr if op == "mcorr" else mconv._ext_lcorrlcorr
+    r = (512, 1) if op == "mcorr" else (1, 1)
+
+    def passes(x):
+        with torch.autocast("cuda", torch.float16, enabled=half):
+            return call(x, w, b, (1, 1), (1, 1), (1, 1), (1, 1), r, activation="relu" if relu else None)
+
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    out = passes(x)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - before <= out.numel() * size + (5 << 30)
+    assert hip.last_variant() == ("mfma-f16-blocks" if half else "mfma-blocks")
+    go = torch.empty_like(out).normal_(std=0.1, generator=gen)   # (parameters' gradients in half stay finite)
+    gi, gw, gb = torch.autograd.grad(out, (x, w, b), go, retain_graph=True)
+    assert all(torch.equal(g, alone) for g, alone in zip((gw, gb), torch.autograd.grad(out, (w, b), go)))
+    tol = 1e-3 if half else 1e-6
+    for i in (0, per - 1, per, 2 * per - 1, 2 * per, n - 1):
+        xi = x[i:i + 1].detach().clone().requires_grad_()
+        oi = passes(xi)
+        gii, = torch.autograd.grad(oi, xi, go[i:i + 1])
+        assert float((oi - out[i:i + 1]).detach().double().norm() / oi.detach().double().norm()) <= tol
+        # (another order of summation may pass a value within its rounding error of the ReLU's kink: 1.7e-3 of the gradient)
+        assert float((gii - gi[i:i + 1]).double().norm() / gii.double().norm()) <= (5e-3 if relu else tol)
+
+
 def test_layer_entry_points_refuse_what_they_cannot_do():
     dims = hip._dims(2, 16, 8, (3, 3), (9, 9), (7, 7), (1, 1), (1, 1), (0, 0), (1, 1))
     x, w, out = torch.zeros(2, 16, 9, 9, device="cuda"), torch.zeros(8, 16, 3, 3, device="cuda"), torch.zeros(2, 8, 7, 7, device="cuda")

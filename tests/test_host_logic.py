@@ -202,3 +202,18 @@ def test_traffic_data_file_agrees_with_the_profile_summary():
         assert abs(float(cells[7]) - e["bytes"] / 1e6) <= 0.21
         assert bench.measured_traffic(name, e["variant"], e["math"]) == e["bytes"]
         assert bench.measured_traffic(name, "generic", e["math"]) is None
+
+
+@pytest.mark.parametrize("kind", [hip.AX_LCORR, hip.AX_MCORR], ids=["linear", "mellin"])
+@pytest.mark.parametrize("elem,unit", [(4, 48), (2, 16), (6, 16)], ids=["f32", "f16", "amp"])
+def test_scratch_memory_of_huge_layers_is_bounded(kind, elem, unit):
+    """A blocked tensor of a pass takes 4 GiB of scratch memory at most: larger layers go image by image range through it.
+    Beside it there are a filter and at most 1 GiB of partial sums."""
+    c, image = 128, (256 * 41 + 1) * 128 // 8 * unit
+    most = (4 << 30) // image                                    # images of the largest blocked tensor
+    for n in (most, most + 1, 3 * most + 1, 16 * most):
+        dims = hip._dims(n, c, c, (3, 3), (256, 41), (256, 41), (1, 1), (1, 1), (1, 1), (1, 1))
+        parts = -(-n // most)
+        for need in (hip.lib.mellin_layer_forward_workspace(kind, elem, *dims), hip.lib.mellin_layer_backward_workspace(kind, elem, 1, *dims)):
+            assert n // parts * image < need <= 5 << 30, (n, need)
+        assert hip.lib.mellin_layer_backward_workspace(kind, elem, 7, *dims) <= (9 if parts == 1 else 5) << 30

@@ -202,8 +202,13 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   // adds up.  Measured on this chip, and rounded:
   //   a step's matrix instructions at 65-80 % of their rate (larger tiles: the higher), shared by a CU's workgroups;
   //   a stage at least 4000 (the latency of its loads);
-  //   per tile 5000 for its tables (9000 where wavefronts share it: nothing runs under them) and its output at 9 bytes a
-  //   cycle; 9000 for a launch's start, as much for the kernel that adds the slices, and 2400 bytes a cycle for their sums.
+  //   per tile 5000 for its tables (9000 where wavefronts share it in fp32: nothing runs under them) and its output at 9
+  //   bytes a cycle; 9000 for a launch's start, as much for the kernel that adds the slices, and 2400 bytes a cycle for
+  //   their sums.
+  // Half tiles that wavefronts share cost 5000 as well: what the others pay on top is the wait for every short step's
+  // fragments, which the steps' rate leaves out.  Of 3000 passes of half layers and stacks drawn over 1 to 32 images of 100 to
+  // 780 rows, 1183 take other plans with 9000; 276 of those take 0.86 of the time with 5000 in the geometric mean (0.53 to
+  // 1.20, twelve of them more than 1.03).  In fp32 it decides 361 of 3000, for either side: 205 of them 0.66 to 1.29.
   const i64 slots = 512;
   auto cost = [&]() {
     const int M_T = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32;
@@ -214,7 +219,7 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
     const double rate = pl.mt * pl.nt >= 8 ? 0.8 : pl.mt * pl.nt >= 4 ? 0.65 : 0.55;
     const double steps = std::ceil(rows * pl.nfy * pl.G / (2 * pl.wk)) * pl.mt * pl.nt * (f16 ? 1 : 6) * 32 / rate;
     const double output = (double)M_T * P * (f16 ? 2 : 4) / 9;
-    const double tile = pl.wk > 1 ? 9000 : 5000;
+    const double tile = pl.wk > 1 && !f16 ? 9000 : 5000;
     auto turns_cost = [&](i64 items, double stages) {
       const i64 full = items / per_m, left = items - full * per_m;
       auto turn = [&](i64 n) { return stages * std::max(4000.0, steps * (n * pl.m_tiles > slots / 2 ? 2 : 1)) + tile + output; };

@@ -28,9 +28,11 @@
 // Few tiles (one utterance, deep layers): WK = 4 wavefronts share the positions of a tile and
 // take every fourth step of a stage; their sums are added in wavefront order through LDS.
 //
-// Measured, 256 -> 256 channels, 4 x 4 taps, 16 x 100 x 41 positions, linear: fp32 1312 -> 1190 us and 107 us
-// for the cut (six bf16 products each: 1.39 PF, matrix pipe 57 % busy at 1.9 GHz, near the rate the board's
-// power allows); half, on Mellin rows, 286 -> 183 us.  One utterance (few tiles, WK = 4): 1039 -> 229 us for ten layers.
+// Measured against the kernels that read the tensors as they lie, 128 -> 256 channels, 3 x 3 taps, 32 x 256 x 41 positions
+// (0.194 TFLOP): fp32, linear, forward and input gradient 1308 -> 1102 us each and 206 us a tensor for the cut (six bf16
+// products: 1.06 PF, matrix pipe 60 and 64 % busy at the 1.7 to 2.0 GHz the board's power leaves, where a plain bf16 product
+// of 8192^3 reaches 1.34 PF); half, Mellin rows, forward 259 -> 181 us, input gradient 420 -> 181, and 71 us a tensor.
+// One utterance (few tiles, WK = 4): 1039 -> 228 us for ten layers.
 #pragma once
 
 #include <type_traits>

@@ -23,8 +23,9 @@
 // Every workgroup writes its sums as one partial block; block_finish.hip adds a weight's partial
 // sums in slice order (bit-reproducible).
 //
-// Measured, 256 -> 256 channels, 4 x 4 taps, 16 x 100 x 41 positions: fp32, linear rows 1172 -> 994 us; half, Mellin
-// rows 356 -> 140 us (64 -> 64 channels of the ten-layer stack, fp32: 300 -> 215 us).
+// Measured against wgrad_pos.hip, 128 -> 256 channels, 3 x 3 taps, 32 x 256 x 41 positions: fp32, linear rows 1171 -> 1056 us;
+// half, Mellin rows 356 -> 146 us.  64 -> 64 channels, 4 x 4 taps, 32 x 780 x 20, fp32: Mellin rows 477 -> 275 us, linear
+// rows 424 -> 440.
 #include <algorithm>
 #include <type_traits>
 
@@ -359,7 +360,7 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
   pl.cgt = pl.ctb * 4;
   // slices: two workgroups per CU in all, dealt to the filter rows by their positions; twice as many, half as long, where a
   // single accumulator takes all six products of fp32 parts (128 -> 256 channels, 3 x 3 taps, 32 x 256 x 41 positions:
-  // error 2.9e-6 -> 2.1e-6, its sums' launch 22 -> 28 us, 0.2 % of the step)
+  // error 2.9e-6 -> 2.1e-6, wgrad_pos.hip 2.6e-6; its sums' launch 22 -> 28 us, 0.2 % of the step)
   const int blocks = pl.m_blocks * pl.c_blocks, turns = !f16 && pl.mt * pl.nt > kLowTiles ? 2 : 1;
   const i64 want = std::max<i64>(pl.nfx, (pl.nw == 4 ? 512 : 256) * turns / blocks);
   int total = 0;

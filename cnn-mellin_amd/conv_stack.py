@@ -180,11 +180,14 @@ class ConvStack(torch.nn.Module):
         return len(self.convs) == len(self.plan)
 
     def _frozen(self, x: torch.Tensor) -> int:
-        """How many layers there are below the first that anything learns from (nothing is kept of them)."""
+        """How many layers there are below the first that anything learns from (nothing is kept of them).  Fewer where
+        that one is pooled: one call takes no pool behind its first layer."""
         if not torch.is_grad_enabled() or x.requires_grad:
             return 0
         for i, conv in enumerate(self.convs):
             if conv.weight.requires_grad or (conv.bias is not None and conv.bias.requires_grad):
+                while i > 0 and self.plan[i]["pool"]:
+                    i -= 1
                 return i
         return 0                                            # (no layer learns, and one call keeps nothing either)
 

@@ -179,48 +179,24 @@ class ConvStack(torch.nn.Module):
                 return False
         return len(self.convs) == len(self.plan)
 
-    def _frozen(self, x: torch.Tensor) -> int:
-        """How many layers there are below the first that anything learns from (nothing is kept of them).  Fewer where
-        that one is pooled: one call takes no pool behind its first layer."""
-        if not torch.is_grad_enabled() or x.requires_grad:
-            return 0
-        for i, conv in enumerate(self.convs):
-            if conv.weight.requires_grad or (conv.bias is not None and conv.bias.requires_grad):
-                while i > 0 and self.plan[i]["pool"]:
-                    i -= 1
-                return i
-        return 0                                            # (no layer learns, and one call keeps nothing either)
-
-    def _layers(self, x: torch.Tensor, first: int, last: int, fused: bool, one_call: bool) -> torch.Tensor:
-        """Layers ``first`` to ``last - 1``."""
-        plan, convs = self.plan[first:last], list(self.convs)[first:last]
-        if one_call:
-            # all of them in one call, their tensors in the kernels' layout from layer to layer
-            kind = _hip.AX_MCORR if self.params.mellin else _hip.AX_LCORR
-            # (a pool behind the last layer stays outside)
-            pools = [bool(lay["pool"]) for lay in plan[:-1]] + [False]
-            y = _native_stack(kind, x, [(conv.weight, conv.bias, conv.s, conv.d, conv.p, conv.r, pool)
-                                        for conv, pool in zip(convs, pools)])
-            if y is not None:
-                return freq_max_pool(y) if plan[-1]["pool"] else y
-        for lay, conv in zip(plan, convs):
-            x = conv(x, activation="relu") if fused else self.params.nonlinearity(conv(x))
-            if lay["pool"]:
-                x = freq_max_pool(x)
-        return x
-
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # ReLU, the reference's default (models.py:96-101), is applied by the convolution
         # kernel itself on the way out; any other callable runs as a pass of its own
         fused = self.params.nonlinearity in (torch.relu, torch.nn.functional.relu)
-        one_call = fused and x.is_cuda and self._plain()
-        # a call keeps the inputs of all its layers for the backward pass, so frozen layers below have one of their own
-        # (a single one has no input that the call would keep beside the stack's own)
-        frozen = self._frozen(x) if one_call else 0
-        if frozen > 1:
-            x = self._layers(x, 0, frozen, fused, one_call)
-            return self._layers(x, frozen, len(self.convs), fused, one_call)
-        return self._layers(x, 0, len(self.convs), fused, one_call)
+        if fused and x.is_cuda and self._plain():
+            # the whole stack in one call, its tensors in the kernels' layout from layer to layer
+            kind = _hip.AX_MCORR if self.params.mellin else _hip.AX_LCORR
+            # (a pool behind the last layer stays outside)
+            pools = [bool(lay["pool"]) for lay in self.plan[:-1]] + [False]
+            y = _native_stack(kind, x, [(conv.weight, conv.bias, conv.s, conv.d, conv.p, conv.r, pool)
+                                        for conv, pool in zip(self.convs, pools)])
+            if y is not None:
+                return freq_max_pool(y) if self.plan[-1]["pool"] else y
+        for lay, conv in zip(self.plan, self.convs):
+            x = conv(x, activation="relu") if fused else self.params.nonlinearity(conv(x))
+            if lay["pool"]:
+                x = freq_max_pool(x)
+        return x
 
 
 class FrameClassifier(torch.nn.Module):

@@ -1882,21 +1882,24 @@ constexpr int kStackLayers = 64;
 
 struct StackLayer {
   i64 batch, c_in, c_out, plane, q, rows, cols;        // of the input; of the output before pooling
-  size_t x_off, which_off;                             // saved: input, blocked; which value of a pair pooled into it
+  bool kept;                                           // the input lies in `saved` (else: in the forward workspace)
+  size_t x_off, which_off;                             // input, blocked; saved: which value of a pair pooled into it
   size_t frag_off;                                     // backward workspace: filter of the input gradient
 };
 // Where everything lies.  saved: the layers' blocked inputs, from the second layer on (without training two regions in
-// turn) and the poolings' choices.
+// turn) and the poolings' choices.  In training the last layer's comes first and layers below `first`, which nothing is
+// wanted of, have none (their inputs lie in the forward workspace, two regions in turn): so a backward call finds what it
+// needs whichever of the layers above is the lowest that it is asked for.
 struct StackPlan {
   StackLayer l[kStackLayers];
   size_t saved, forward, backward;
-  size_t f_first, f_own, f_filters, f_unpooled, f_sums, own_bytes;                          // forward workspace
+  size_t f_first, f_own, f_filters, f_unpooled, f_sums, f_turn[2], own_bytes;                          // forward workspace
   size_t b_grad[2], b_unpooled, b_bias[2], b_weight, b_sums, b_first, b_own, b_own_bytes;   // backward workspace
 };
-static bool plan_stack(int kind_x, int elem, bool train, int n, const mellin_stack_layer *layers, StackPlan &sp) {
+static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const mellin_stack_layer *layers, StackPlan &sp) {
   const bool half = elem != 4;
-  if (n < 2 || n > kStackLayers) return false;
-  size_t saved = 0, in_turn[2] = {0, 0}, frags = 0, unpooled = 0, sums = 0;
+  if (n < 2 || n > kStackLayers || first < 0 || first >= n) return false;
+  size_t saved = 0, in_turn[2] = {0, 0}, frags = 0, unpooled = 0, sums = 0, x_bytes[kStackLayers], which_bytes[kStackLayers];
   size_t grad[2] = {0, 0}, b_unpooled = 0, bias[2] = {0, 0}, weight = 0, b_frags = 0, b_sums = 0;
   auto region = [&](i64 channels, i64 plane, i64 batch) { return align256(blocked_bytes(batch, channels, plane, half)); };
   for (int i = 0; i < n; ++i) {
@@ -1912,15 +1915,8 @@ static bool plan_stack(int kind_x, int elem, bool train, int n, const mellin_sta
     if (l.c_in != before.dims[2] || ly.dims[5] != before.dims[7] || ly.dims[6] != (before.pool ? before.dims[8] / 2 : before.dims[8])) return false;
     BlockPlan bp;
     if (!plan_block_forward(kind_x, half, STACK_DIMS(ly), bp)) return false;
-    const size_t x = region(l.c_in, l.plane, l.batch);
-    if (train) {
-      l.x_off = saved;
-      saved += x;
-    } else {
-      in_turn[i & 1] = std::max(in_turn[i & 1], x);
-    }
-    l.which_off = saved;
-    if (train && before.pool) saved += align256((size_t)(l.batch * ((l.c_in + 7) / 8) * l.plane) * 8);
+    x_bytes[i] = region(l.c_in, l.plane, l.batch);
+    which_bytes[i] = before.pool ? align256((size_t)(l.batch * ((l.c_in + 7) / 8) * l.plane) * 8) : 0;
     l.frag_off = frags;                                // (forward; the backward call lays out its own)
     frags += align256(bp.filter_bytes);
     sums = std::max(sums, bp.slice_bytes);
@@ -1941,21 +1937,35 @@ static bool plan_stack(int kind_x, int elem, bool train, int n, const mellin_sta
     }
     if (i == n - 1) bias[i & 1] = std::max(bias[i & 1], pack_partial_count(l.batch, l.c_out, l.q) * 4);
   }
+  for (int i = n - 1; i > 0; --i) {
+    StackLayer &l = sp.l[i];
+    l.kept = !train || i >= first;
+    if (!train || i < first) {
+      in_turn[i & 1] = std::max(in_turn[i & 1], x_bytes[i]);
+      continue;
+    }
+    l.x_off = saved;
+    saved += x_bytes[i];
+    l.which_off = saved;
+    if (i > first) saved += which_bytes[i];
+  }
   if (!train) {
     for (int i = 1; i < n; ++i) sp.l[i].x_off = i & 1 ? in_turn[0] : 0;
     saved = in_turn[0] + in_turn[1];
+    in_turn[0] = in_turn[1] = 0;
   }
   sp.saved = saved;
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t off = at; at += align256(bytes); return off; };
   const StackLayer &l0 = sp.l[0];
-  const size_t first = (size_t)(l0.batch * l0.c_out * l0.q) * (half ? 2 : 4);
-  sp.f_first = take(first);
+  const size_t dense = (size_t)(l0.batch * l0.c_out * l0.q) * (half ? 2 : 4);
+  sp.f_first = take(dense);
   sp.own_bytes = mellin_layer_forward_workspace(kind_x, elem, STACK_DIMS(layers[0]));
   sp.f_own = take(sp.own_bytes);
   sp.f_filters = take(frags);
   sp.f_unpooled = take(unpooled);
   sp.f_sums = take(sums);
+  for (int k = 0; k < 2; ++k) sp.f_turn[k] = take(in_turn[k]);
   sp.forward = at;
   at = 0;
   sp.backward = 0;
@@ -1967,7 +1977,7 @@ static bool plan_stack(int kind_x, int elem, bool train, int n, const mellin_sta
   sp.b_bias[1] = take(bias[1]);
   sp.b_weight = take(weight);
   sp.b_sums = take(b_sums);
-  sp.b_first = take(first);
+  sp.b_first = take(dense);
   sp.b_own_bytes = mellin_layer_backward_workspace(kind_x, elem, MELLIN_WANT_INPUT | MELLIN_WANT_WEIGHT, STACK_DIMS(layers[0]));
   sp.b_own = take(sp.b_own_bytes);
   sp.backward = at + b_frags;
@@ -1983,8 +1993,10 @@ static bool plan_stack(int kind_x, int elem, bool train, int n, const mellin_sta
 int mellin_stack_bytes(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers, size_t *saved,
                        size_t *forward_workspace, size_t *backward_workspace) {
   StackPlan sp;
+  const int first = train >> 8;                        // (MELLIN_STACK_TRAIN_FROM)
+  train &= 255;
   const Settled settled(train == 2);
-  if (!layer_elements(elem_bytes) || !layers || !plan_stack(kind_x, elem_bytes, train != 0, n_layers, layers, sp)) return 0;
+  if (!layer_elements(elem_bytes) || !layers || !plan_stack(kind_x, elem_bytes, train != 0, first, n_layers, layers, sp)) return 0;
   *saved = sp.saved;
   *forward_workspace = sp.forward;
   *backward_workspace = sp.backward;
@@ -2005,7 +2017,9 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
   StackPlan sp;
   if (!layer_elements(elem_bytes)) return bad_elements(__func__, elem_bytes);
   const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT;
-  const bool planned = layers && plan_stack(kind_x, elem_bytes, train != 0, n_layers, layers, sp);
+  const int first = train >> 8;
+  train &= 255;
+  const bool planned = layers && plan_stack(kind_x, elem_bytes, train != 0, first, n_layers, layers, sp);
   int rc = stack_checks(__func__, planned, sp, saved, saved_bytes, workspace, workspace_bytes, sp.forward);
   if (rc) return rc;
   if (!input || !out) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
@@ -2029,9 +2043,10 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
     frag_off[i] = at;
     at += align256(bp.filter_bytes);
   }
+  auto input_of = [&](int i) { return sp.l[i].kept ? keep + sp.l[i].x_off : ws + sp.f_turn[i & 1]; };
   const StackLayer &l1 = sp.l[1];
-  const PackSignal first = {ws + sp.f_first, nullptr, keep + l1.x_off, nullptr, (int)l1.batch, (int)l1.c_in, (int)l1.plane};
-  hipError_t e = launch_block_pack(half, &first, nullptr, filters, n_layers - 1, st);
+  const PackSignal dense = {ws + sp.f_first, nullptr, input_of(1), nullptr, (int)l1.batch, (int)l1.c_in, (int)l1.plane};
+  hipError_t e = launch_block_pack(half, &dense, nullptr, filters, n_layers - 1, st);
   for (int i = 1; i < n_layers && e == hipSuccess; ++i) {
     const mellin_stack_layer &ly = layers[i];
     const StackLayer &l = sp.l[i];
@@ -2039,8 +2054,8 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
     plan_block_forward(kind_x, half, STACK_DIMS(ly), bp);
     bp.relu = 1;
     bp.wide = wide;
-    char *to = last ? (char *)out : ly.pool ? ws + sp.f_unpooled : keep + sp.l[i + 1].x_off;
-    const BlockGemmArgs args = {keep + l.x_off, ws + frag_off[i], ly.bias, to, (float *)(ws + sp.f_sums), !last, false, nullptr, nullptr};
+    char *to = last ? (char *)out : ly.pool ? ws + sp.f_unpooled : input_of(i + 1);
+    const BlockGemmArgs args = {input_of(i), ws + frag_off[i], ly.bias, to, (float *)(ws + sp.f_sums), !last, false, nullptr, nullptr};
     e = launch_block_gemm(bp, args, st);
     if (e == hipSuccess && bp.rest > 0) {
       BlockFinish fin = {};
@@ -2048,8 +2063,8 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
       e = launch_block_finish(half, wide, fin, st);
     }
     if (e == hipSuccess && ly.pool)
-      e = launch_block_pool(half, to, l.batch, l.c_out, l.rows, l.cols, keep + sp.l[i + 1].x_off,
-                            train ? keep + sp.l[i + 1].which_off : nullptr, st);
+      e = launch_block_pool(half, to, l.batch, l.c_out, l.rows, l.cols, input_of(i + 1),
+                            train && i + 1 > first ? keep + sp.l[i + 1].which_off : nullptr, st);
   }
   g_variant = half ? "mfma-f16-blocks" : "mfma-blocks";
   g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
@@ -2063,14 +2078,14 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
   if (!layer_elements(elem_bytes)) return bad_elements(__func__, elem_bytes);
   const Settled settled(true);
   const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT;
-  const bool planned = layers && plan_stack(kind_x, elem_bytes, true, n_layers, layers, sp);
+  // the first layer that anything is wanted of
+  int lowest = 0;
+  if (!grad_input && layers && n_layers <= kStackLayers)
+    while (lowest < n_layers && !layers[lowest].grad_weight && !layers[lowest].grad_bias) ++lowest;
+  const bool planned = layers && plan_stack(kind_x, elem_bytes, true, std::max(0, std::min(lowest, n_layers - 1)), n_layers, layers, sp);
   int rc = stack_checks(__func__, planned, sp, saved, saved_bytes, workspace, workspace_bytes, sp.backward);
   if (rc) return rc;
   if (!input || !out || !grad_out) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
-  // the first layer that anything is wanted of
-  int lowest = 0;
-  if (!grad_input)
-    while (lowest < n_layers && !layers[lowest].grad_weight && !layers[lowest].grad_bias) ++lowest;
   if (lowest == n_layers) return MELLIN_OK;
   char *ws = (char *)workspace;
   const char *keep = (const char *)saved;

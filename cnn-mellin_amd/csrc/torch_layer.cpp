@@ -260,6 +260,7 @@ struct StackBackward : public torch::autograd::Node {
   std::vector<torch::autograd::SavedVariable> weights_;
   std::vector<bool> has_bias;
   Tensor saved_;
+  int first = 0;                                       // the lowest layer that gradients can be asked of
   size_t workspace = 0;
   at::ScalarType param_kind = at::kFloat;
 
@@ -293,8 +294,8 @@ struct StackBackward : public torch::autograd::Node {
     if (task_should_compute_output(0)) result[0] = at::empty_like(input, at::MemoryFormat::Contiguous);
     for (size_t i = 0; i < n; ++i) {
       const Tensor &w = weights[i];
-      if (elem == MELLIN_ELEM_HALF_FLOAT) call[i].weight_half = w.data_ptr();
-      else call[i].weight = w.const_data_ptr();
+      if (elem != MELLIN_ELEM_HALF_FLOAT) call[i].weight = w.const_data_ptr();
+      else if ((int)i >= first) call[i].weight_half = w.data_ptr();
       if (task_should_compute_output(1 + 2 * i)) {
         result[1 + 2 * i] = at::empty(w.sizes(), w.options().dtype(param_kind));
         call[i].grad_weight = result[1 + 2 * i].data_ptr();
@@ -339,7 +340,7 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   }
   if (kind_of != at::kFloat && kind_of != at::kHalf) Py_RETURN_NONE;
   at::ScalarType param_kind = at::kFloat;
-  bool differentiable = input0.requires_grad();
+  int first = input0.requires_grad() ? 0 : (int)n;     // the lowest layer that learns (input gradients: all)
   int64_t c = input0.size(1), x = input0.size(2), y = input0.size(3);
   for (Py_ssize_t i = 0; i < n; ++i) {
     PyObject *t = PyList_GET_ITEM(args[2], i);
@@ -378,7 +379,7 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     layers[i] = mellin_stack_layer{};
     std::copy(dims, dims + 17, layers[i].dims);
     layers[i].pool = PyTuple_GET_ITEM(t, 6) == Py_True;
-    differentiable = differentiable || wt.requires_grad() || (bt.defined() && bt.requires_grad());
+    if (wt.requires_grad() || (bt.defined() && bt.requires_grad())) first = std::min(first, (int)i);
     c = g.c_out;
     x = g.nh[0];
     y = layers[i].pool ? g.nh[1] / 2 : g.nh[1];
@@ -388,9 +389,10 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   if (!wide && param_kind != kind_of) Py_RETURN_NONE;
   if (wide && !cast) Py_RETURN_NONE;
   const int elem = wide ? MELLIN_ELEM_HALF_FLOAT : kind_of == at::kHalf ? 2 : 4;
-  differentiable = differentiable && at::GradMode::is_enabled();
+  const bool differentiable = first < (int)n && at::GradMode::is_enabled();
+  const int train = differentiable ? MELLIN_STACK_TRAIN_FROM(first) : 0;
   size_t saved_bytes = 0, forward_bytes = 0, backward_bytes = 0;
-  if (!mellin_stack_bytes(kind, elem, differentiable, (int)n, layers.data(), &saved_bytes, &forward_bytes, &backward_bytes)) Py_RETURN_NONE;
+  if (!mellin_stack_bytes(kind, elem, train, (int)n, layers.data(), &saved_bytes, &forward_bytes, &backward_bytes)) Py_RETURN_NONE;
 
   Tensor out;
   {
@@ -411,7 +413,7 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
           call[i].bias = dense[2 * i + 1].const_data_ptr();
         }
         kept[i] = dense[2 * i];
-        if (wide && differentiable) {
+        if (wide && differentiable && i >= first) {
           kept[i] = at::empty(weights[i].sizes(), input.options());
           call[i].weight_half = kept[i].data_ptr();
         }
@@ -420,7 +422,7 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
       out = at::empty({d[0], d[2], d[7], d[8]}, input.options());
       saved = scratch(input, saved_bytes);
       Tensor ws = scratch(input, forward_bytes);
-      check(mellin_stack_forward(kind, elem, differentiable, (int)n, call.data(), pointer(input), out.data_ptr(), saved.data_ptr(),
+      check(mellin_stack_forward(kind, elem, train, (int)n, call.data(), pointer(input), out.data_ptr(), saved.data_ptr(),
                                  saved_bytes, ws.data_ptr(), forward_bytes, launch_stream(input)));
     }
     if (differentiable) {
@@ -439,6 +441,7 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
       node->set_next_edges(std::move(edges));
       node->kind = kind;
       node->elem = elem;
+      node->first = first;
       node->layers = std::move(layers);
       node->input_ = torch::autograd::SavedVariable(input, false);
       node->saved_ = std::move(saved);

@@ -440,6 +440,8 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
  * mellin_stack_bytes: 1 if the stack can be run so under the settings in force, 0 if not (layers with too few channels for
  * the blocked kernels behind the first: call them one by one), and the bytes of `saved` (what the forward call keeps: for
  * the backward call, with train), of the forward call's workspace and of the backward call's; all 256-byte aligned.
+ * train = MELLIN_STACK_TRAIN_FROM(i), in both calls: as 1, for backward calls that want gradients of layers i and above only
+ * (a frozen stack below): nothing is kept of the layers below i.
  * train = 2: for the backward call of a forward call already made, which goes on whatever has been set since (the first
  * layer's kernels follow the settings, so its workspace may have another size).
  * out: the last layer's output, as it lies. */
@@ -449,6 +451,7 @@ typedef struct {
   const void *weight, *bias;
   void *weight_half, *grad_weight, *grad_bias;
 } mellin_stack_layer;
+#define MELLIN_STACK_TRAIN_FROM(i) (1 | (i) << 8)
 int mellin_stack_bytes(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers, size_t *saved,
                        size_t *forward_workspace, size_t *backward_workspace);
 int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers,

@@ -167,16 +167,13 @@ def test_frozen_layers_below_keep_nothing(frozen, pool_after, half):
         grad = torch.randn_like(out) if grad is None else grad
         leaves = [p for conv in stack.convs[frozen:] for p in conv.parameters()]
         grads.append([out.detach()] + list(torch.autograd.grad(out, leaves, grad)))
-        assert "StackBackward" in out.grad_fn.name() or n == 5     # (a layer alone)
+        assert "StackBackward" in out.grad_fn.name()
         del out
-    # what is kept then: the input of the first layer that learns as it lies, those of the layers above it in blocks (six bytes
-    # a value in float32), the filters of half tensors, the output; a first layer behind which there is a pool has the one
-    # below with it
-    first = frozen - (frozen + 1 in pool_after)
+    # what is kept then: the inputs of the layers that learn in blocks (six bytes a value in float32), a byte for each value
+    # that was pooled above the first of them, the filters of half tensors, the output
     size, value = (2 if half else 4), (2 if half else 6)
-    channels = 32 * 2 * 400
-    bins = [40 // 2 if pool_after and i + 1 >= pool_after[0] else 40 for i in range(6)]
-    most = channels * (bins[first - 1] * size + sum((b + 1) * (value + 1) for b in bins[first:5]) + bins[5] * size)
+    bins = [40 // 2 if pool_after and i + 1 >= pool_after[0] else 40 for i in range(6)]      # of a layer's output
+    most = 32 * 2 * 400 * (sum(b * (value + 1) for b in bins[frozen - 1:5]) + bins[5] * size)
     assert held[1] <= most + (1 << 18), (held, most)
     assert held[1] < held[0]
     for a, b in zip(*grads):
@@ -238,3 +235,9 @@ def test_channels_past_the_last_are_zeros_whatever_the_scratch_memory_held(melli
     assert all(bool(t.isfinite().all()) for t in results[0]) and bool((results[0][0] > 0).any())
     for other in results[1:]:
         assert all(torch.equal(a, b) for a, b in zip(results[0], other))
+    # a forward call for gradients of the layers from the fourth on keeps less, and a backward call that wants more is refused
+    fewer = [ctypes.c_size_t() for _ in range(3)]
+    assert hip.lib.mellin_stack_bytes(kind, elem, 1 | 3 << 8, n, layers, *(ctypes.addressof(s) for s in fewer)) == 1
+    assert fewer[0].value < sizes[0].value
+    assert hip.lib.mellin_stack_backward(kind, elem, n, layers, hip._dp(inp), hip._dp(out), hip._dp(grad), hip._dp(saved),
+                                         fewer[0].value, hip._dp(gi), hip._dp(bw), sizes[2].value, hip._stream(inp.device)) == 3

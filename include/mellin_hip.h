@@ -410,7 +410,9 @@ int mellin_pool_pairs_backward_f16(const void *grad_y, const unsigned char *whic
  * its result.  Knowing all that is asked for, it shares between the gradients what they
  * have in common, so it may be faster than the calls of sections 2 and 4 one by one.
  * At most 65535 images and output channels in the backward call.  Scratch: the byte count
- * of the *_workspace call under the same settings, 256-byte aligned.
+ * of the *_workspace call under the same settings, 256-byte aligned; copies of tensors in the
+ * kernels' own layout (6 bytes a float, 2 a half) take at most 4 GiB of it each: larger layers
+ * go through it in parts.
  * ------------------------------------------------------------------------ */
 #define MELLIN_WANT_INPUT 1
 #define MELLIN_WANT_WEIGHT 2

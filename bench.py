@@ -241,7 +241,7 @@ def other_math_leg(args, dev, torch, hip, steps=30, reps=30):
 
 
 def other_configs(torch, reps=20):
-    """Per-pass times of BASELINE configuration 4 (wide layer, linear and Mellin x axis) and
+    """Per-pass times of the widest layer (128 -> 256 channels, 3 x 3, linear and Mellin x axis) and
     forward + backward of the two 10-layer stacks of configuration 5, by time_layers.py's own
     routines, `reps` timed calls each (outside the main timed region; not bench lines)."""
     import time_layers

@@ -383,7 +383,7 @@ int mellin_bias_grad_f16(const void *grad_out, const void *out, int64_t batch,
                          void *grad_bias, void *workspace, size_t workspace_bytes,
                          void *stream);
 
-/* Frequency pooling of the convolution stack: the maximum over pairs of
+/* Frequency pooling of the convolution stack (the ten-layer stacks): the maximum over pairs of
  * neighbours along the last axis, y[r, j] = max(x[r, 2 j], x[r, 2 j + 1]) for x (rows, f) and
  * j < f / 2 -- what max_pool2d(x, (1, 2)) computes (the first of two equal values wins, NaN
  * propagates) -- with one byte per output in `which` (1: the second of the pair was taken)

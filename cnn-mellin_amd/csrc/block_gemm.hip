@@ -216,7 +216,7 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
     double filter_rows, subsets;
     tile_rows(P, filter_rows, subsets);
     const double rows = filter_rows / subsets;
-    const double rate = pl.mt * pl.nt >= 8 ? 0.8 : pl.mt * pl.nt >= 4 ? 0.65 : 0.55;
+    const double rate = pl.mt * pl.nt >= 8 ? 0.8 : pl.mt * pl.nt * pl.wm >= 8 ? 0.72 : pl.mt * pl.nt >= 4 ? 0.65 : 0.55;
     const double steps = std::ceil(rows * pl.nfy * pl.G / (2 * pl.wk)) * pl.mt * pl.nt * (f16 ? 1 : 6) * 32 / rate;
     const double output = (double)M_T * P * (f16 ? 2 : 4) / 9;
     const double tile = pl.wk > 1 && !f16 ? 9000 : 5000;
@@ -250,14 +250,19 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   // separate sums, and were slower as they were (windows of ten frames 2111 -> 1998 us a step, one utterance decoded 246 ->
   // 233 us).  Half has the registers, and its shorter steps are better shared (1-D layer, 41 -> 128 channels: 15.1 us
   // without the 64 positions, 10.7 with them).
-  static const int shapes[][3] = {{4, 2, 1}, {4, 1, 1}, {2, 1, 1}, {1, 1, 1}, {2, 1, 4}, {1, 1, 4}};   // nt, wm, wk
+  // fp32, two wavefronts along the channels: 128 channels x 128 positions instead of 64 x 256 stage half the signal for as
+  // many products, and a stage has twice the steps (128 -> 256 channels, 3 x 3, 32 x 256 x 41: 1075 -> 905 us).  77 passes of
+  // stacks and layers drawn over 1 to 32 images take it: with more workgroups than CUs 1.15 times as fast in the geometric mean
+  // (0.99 to 1.46), with less, which leave nothing on a CU to run beside a workgroup's waits, 0.95 (0.73 to 1.18): not those.
+  static const int shapes[][3] = {{4, 2, 1}, {4, 1, 1}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}, {2, 1, 4}, {1, 1, 4}};   // nt, wm, wk
   BlockPlan best_plan;
   double best_cost = 0;
   for (const auto &sh : shapes) {
-    if (!f16 && (sh[0] == 4 || (sh[0] == 2 && sh[2] == 4))) continue;
+    if (f16 ? sh[0] == 2 && sh[1] == 2 : sh[0] == 4 || (sh[0] == 2 && sh[2] == 4)) continue;
     if (sh[1] == 2 && pr.c_out <= 96) continue;        // (two wavefronts along the channels: most of 128)
     if (!shape(sh[0], sh[1], sh[2])) continue;
     const double c = cost();
+    if (!f16 && sh[1] == 2 && ((i64)pl.whole + (i64)pl.rest * pl.slices) * pl.m_tiles <= slots / 2) continue;
     if (best_cost == 0 || c < best_cost) { best_cost = c; best_plan = pl; }
   }
   if (best_cost == 0) return false;

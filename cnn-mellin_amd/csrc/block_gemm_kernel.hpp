@@ -29,9 +29,9 @@
 // take every fourth step of a stage; their sums are added in wavefront order through LDS.
 //
 // Measured against the kernels that read the tensors as they lie, 128 -> 256 channels, 3 x 3 taps, 32 x 256 x 41 positions
-// (0.194 TFLOP): fp32, linear, forward and input gradient 1308 -> 1102 us each and 206 us a tensor for the cut (six bf16
-// products: 1.06 PF, matrix pipe 60 and 64 % busy at the 1.7 to 2.0 GHz the board's power leaves, where a plain bf16 product
-// of 8192^3 reaches 1.34 PF); half, Mellin rows, forward 259 -> 181 us, input gradient 420 -> 181, and 71 us a tensor.
+// (0.194 TFLOP): fp32, linear, forward and input gradient 1308 -> 905 us each (1075 with tiles of 64 channels x 256 positions
+// instead of 128 x 128: make_block_plan) and 206 us a tensor for the cut (six bf16 products: 1.28 PF, at the 1.7 to 2.0 GHz
+// the board's power leaves, where a plain bf16 product of 8192^3 reaches 1.34 PF); half, Mellin rows, forward 259 -> 181 us, input gradient 420 -> 181, and 71 us a tensor.
 // One utterance (few tiles, WK = 4): 1039 -> 228 us for ten layers.
 #pragma once
 
@@ -720,6 +720,7 @@ hipError_t launch_shape(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t
   }
   if (pl.f16 && pl.nt == 2 && pl.wk == 4)
     return pl.mt == 2 ? launch_instance<2, 2, 1, 4, true, OUT>(pl, a, stream) : launch_instance<1, 2, 1, 4, true, OUT>(pl, a, stream);
+  if (!pl.f16 && pl.wm == 2) return launch_instance<2, 2, 2, 1, false, OUT>(pl, a, stream);
   MELLIN_BLOCK_CASE(2, 2, 1, 1)
   MELLIN_BLOCK_CASE(2, 1, 1, 1)
   MELLIN_BLOCK_CASE(1, 2, 1, 1)

@@ -786,7 +786,7 @@ int corr2d_backward_weight(const char *fn, int kind_x, const T *input,
                            i64 nfx, i64 nfy, i64 ngx, i64 ngy, i64 nhx, i64 nhy,
                            i64 sx, i64 sy, i64 dx, i64 dy, i64 px, i64 py, i64 ux,
                            i64 uy, T *grad_weight, void *workspace,
-                           size_t workspace_bytes, void *stream) {
+                           size_t workspace_bytes, void *stream, float *bias_ws = nullptr, float *grad_bias = nullptr) {
   int rc = check_corr2d(fn, kind_x, batch, c_in, c_out, nfx, nfy, ngx, ngy, nhx,
                         nhy, sx, sy, dx, dy, px, py, ux, uy);
   if (rc) return rc;
@@ -817,7 +817,7 @@ int corr2d_backward_weight(const char *fn, int kind_x, const T *input,
       g_last_math = wp.rows_mode == 2 ? MATH_BF16X3 : MATH_FP32;
       return check_hip(launch_wgrad(wp, (const float *)grad_out, (const float *)input,
                                     (float *)grad_weight, (float *)workspace,
-                                    (hipStream_t)stream), fn);
+                                    (hipStream_t)stream, bias_ws, grad_bias), fn);
     }
   }
   SepReduce pr;
@@ -1567,7 +1567,8 @@ static bool blocks_allowed(bool half) {
 // the launch), and choosing among tile shapes takes some microseconds.  The sizes decide the plan, so nothing has to be
 // thrown away.
 struct LayerPlans {
-  int known[3];                                        // 0 not yet, 1 applies, -1 does not
+  int known[4];                                        // 0 not yet, 1 applies, -1 does not
+  size_t bias_bytes;                                   // section 2's weight gradient: for the bias gradient beside it (known[3])
   BlockPlan forward, input;
   BlockWgradPlan weight;
 };
@@ -1623,6 +1624,20 @@ static bool plan_block_weight(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockWg
     lp.known[2] = make_block_wgrad_plan(forward_problem(kind_x, CORR2D_ARGS), half, lp.weight) && lp.weight.ws_bytes <= kMaxWorkspaceBytes ? 1 : -1;
   if (lp.known[2] > 0) wp = lp.weight;
   return lp.known[2] > 0;
+}
+
+// Scratch bytes with which section 2's weight gradient of a float layer also makes the bias gradient (0: it does not).
+static size_t bias_beside_weight(int kind_x, MELLIN_CORR2D_DIMS) {
+  if (!blocks_allowed(false) || batch * c_out * nhx * nhy * c_in == 0) return 0;
+  LayerPlans &lp = layer_plans(kind_x, false, CORR2D_ARGS);
+  if (!lp.known[3]) {
+    const SepConv fwd = forward_problem(kind_x, CORR2D_ARGS);
+    WgradPosPlan pp;
+    WgradPlan wp;
+    lp.bias_bytes = !plan_weight_positions(fwd, pp) && make_wgrad_plan(fwd, wp, g_forced != 2) ? wgrad_bias_bytes(wp) : 0;
+    lp.known[3] = 1;
+  }
+  return lp.bias_bytes;
 }
 
 // A pass's blocked tensor is scratch memory beside the caller's own tensors, in fp32 half as large again as the tensor it was
@@ -1726,7 +1741,8 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
 // section 2, on grad_out as it lies (through a fused ReLU: on a masked copy).
 struct LayerBackward {
   bool input_blocked, weight_blocked, plain;           // plain: some gradient takes the section-2 kernels
-  size_t masked_off, go_off, x_off, frag_off, slice_off, bias_off, wgrad_off, gw_off, gb_off, pass_off, pass_bytes, total;
+  bool bias_beside;                                    // section 2's weight gradient makes the bias gradient as well
+  size_t masked_off, go_off, x_off, frag_off, slice_off, bias_off, wgrad_off, gw_off, gb_off, beside_off, pass_off, pass_bytes, total;
   BlockPlan bp;
   BlockWgradPlan wp;
 };
@@ -1750,8 +1766,12 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
   // (half gradients of the parameters on their way to float)
   lb.gw_off = take(wide && ww && !lb.weight_blocked ? (size_t)(c_out * c_in * nfx * nfy) * 2 : 0);
   lb.gb_off = take(wide && lb.plain && (want & MELLIN_WANT_BIAS) ? (size_t)c_out * 2 : 0);
+  const size_t beside = !half && lb.plain && ww && !lb.weight_blocked && (want & MELLIN_WANT_BIAS) && !(want & MELLIN_WANT_RELU)
+                            ? bias_beside_weight(kind_x, CORR2D_ARGS) : 0;
+  lb.bias_beside = beside > 0;
+  lb.beside_off = take(beside);
   size_t pass = 0;
-  if (lb.plain && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)))   // (a ReLU's backward writes the bias gradient, asked for or not)
+  if (lb.plain && !lb.bias_beside && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)))   // (a ReLU's backward writes the bias gradient, asked for or not)
     pass = align256(mellin_bias_grad_workspace(batch, c_out, nhx * nhy)) + align256((size_t)c_out * elem);
   if (wi && !lb.input_blocked)
     pass = std::max(pass, half ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS)
@@ -1813,7 +1833,7 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT, relu = want & MELLIN_WANT_RELU;
   hipStream_t st = (hipStream_t)stream;
   hipError_t e = hipSuccess;
-  if (lb.plain && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU))) {
+  if (lb.plain && !lb.bias_beside && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU))) {
     void *masked = relu ? ws + lb.masked_off : nullptr;
     const size_t own = mellin_bias_grad_workspace(batch, c_out, nhx * nhy);
     void *gb = !(want & MELLIN_WANT_BIAS) ? pass + align256(own) : wide ? ws + lb.gb_off : grad_bias;
@@ -1832,8 +1852,9 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   if ((want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked) {
     rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, wide ? ws + lb.gw_off : grad_weight, pass,
                                                   lb.pass_bytes, stream)
-              : mellin_corr2d_backward_weight_f32(kind_x, (const float *)input, (const float *)grad_out, CORR2D_ARGS,
-                                                  (float *)grad_weight, pass, lb.pass_bytes, stream);
+              : corr2d_backward_weight<float>(__func__, kind_x, (const float *)input, (const float *)grad_out, CORR2D_ARGS,
+                                              (float *)grad_weight, pass, lb.pass_bytes, stream,
+                                              lb.bias_beside ? (float *)(ws + lb.beside_off) : nullptr, (float *)grad_bias);
     if (rc) return rc;
   }
   if (wide) {

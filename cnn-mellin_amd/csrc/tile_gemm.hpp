@@ -119,8 +119,10 @@ struct WgradPlan {
 bool make_wgrad_plan(const SepConv &fwd, WgradPlan &wp, bool allow_rows = true, int rows_mt = 0,
                      int rows_nbuf = 0, int rows_rpw = 0);
 
-hipError_t launch_wgrad(const WgradPlan &wp, const float *grad_out, const float *input,
-                        float *grad_weight, float *workspace, hipStream_t stream);
+// With bias_ws (wgrad_bias_bytes(): its size, 0 where the kernel does not do it) the sums of grad_out go to grad_bias.
+size_t wgrad_bias_bytes(const WgradPlan &wp);
+hipError_t launch_wgrad(const WgradPlan &wp, const float *grad_out, const float *input, float *grad_weight, float *workspace,
+                        hipStream_t stream, float *bias_ws = nullptr, float *grad_bias = nullptr);
 
 // wgrad_gemm.hip: W[m, j] = the sum of `partials` blocks of (M_pad x J_pad) floats, in index order;
 // W is float storage, or half-precision storage (rounded once) when half_out

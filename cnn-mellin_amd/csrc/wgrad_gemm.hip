@@ -259,11 +259,31 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_gemm_kernel(
 // vector instruction saved in the loop is matrix throughput gained.)
 // grad_out rows arrive by 16-byte direct loads (the four rows of a unit are
 // contiguous per channel); the input rows are staged as in the forward kernel.
+// The bias gradient beside the weight gradient: each of the kernels below holds every value of grad_out once per column
+// block, so the workgroups of the first column block also add them up, lane by lane.  Launches of their own read grad_out
+// once more (27 us and 5 to reduce, of a step's 230, for three channels to 64, 32 x 505 x 38 outputs: 198 us without them;
+// on Mellin rows, 32 x 64 x 38, 81.5 -> 74.8).  A lane adds in pairs, then steps of a unit or row, then units; the halves of
+// a wavefront, the wavefronts and (wgrad_reduce_kernel) the workgroups follow, in pairs as well: error against 64 bits over
+// these two layers and twenty drawn ones 1.09e-7 with launches of their own, 1.06e-7 so (added in turn: 1.7e-7).
+template <int MT>
+__device__ __forceinline__ void bias_to_lds(const float (&bias)[MT], float *dst, int wave, int half, int l32) {
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const float s = bias[i] + __shfl_xor(bias[i], 32);
+    if (half == 0) dst[wave * (MT * 32) + i * 32 + l32] = s;
+  }
+}
+template <int M_T>
+__device__ __forceinline__ float bias_of_waves(const float *src, int m) {
+  static_assert(kWaves == 4, "");
+  return (src[m] + src[M_T + m]) + (src[2 * M_T + m] + src[3 * M_T + m]);
+}
+
 constexpr int kRowsMemo = 8;                       // 64-word blocks per wave whose staging sources are kept
 template <int MT, int JT>
 __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
     WgradPlan wp, const float *__restrict__ A, const float *__restrict__ G,
-    float *__restrict__ ws) {
+    float *__restrict__ ws, float *__restrict__ bias_ws) {
   extern __shared__ __align__(16) float lds[];
   const TilePlan &pl = wp.t;
   constexpr int M_T = MT * 32, J_T = JT * 32;
@@ -372,8 +392,16 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][t][r] = 0.f;
 
+  // sums of this lane's grad_out values, for the bias gradient
+  float bias[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) bias[i] = 0.f;
+
   const int pairs = pl.noy >> 1;
   auto multiply_unit = [&](int ui) {
+    float unit_sum[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) unit_sum[i] = 0.f;
     const int ox_lo = ((first_unit + ui) / pl.batch) * RB;
     for (int row = wave; row < RB && ox_lo + row < pl.nox_eff; row += kWaves) {   // this wavefront's rows
       const int b = wp.nbuf == 2 ? (ui & 1) : 0;
@@ -384,8 +412,12 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
 #pragma unroll
       for (int t = 0; t < JT; ++t)
         bo[t] = col_off[t] + (pl.Ax * row + pl.Cx0) * pl.RS - pl.by_min + half;
+      float row_sum[MT];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) row_sum[i] = 0.f;
       int s = 0;
       for (; s + 8 <= pairs; s += 8) {
+        float last[MT], sum[MT];                         // (pairs of steps, then their sums, so that a rounding error meets few others)
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
           float a[MT], b[JT];
@@ -394,11 +426,20 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
 #pragma unroll
           for (int t = 0; t < JT; ++t) b[t] = Xs[bo[t] + 2 * k];
 #pragma unroll
+          for (int i = 0; i < MT; ++i) {
+            if (k & 1) last[i] += a[i];
+            else last[i] = a[i];
+            if (k == 1) sum[i] = last[i];
+            else if (k & 1) sum[i] += last[i];
+          }
+#pragma unroll
           for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int t = 0; t < JT; ++t)
               acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[t], acc[i][t], 0, 0, 0);
         }
+#pragma unroll
+        for (int i = 0; i < MT; ++i) row_sum[i] += sum[i];
         ao += 16;
 #pragma unroll
         for (int t = 0; t < JT; ++t) bo[t] += 16;
@@ -422,13 +463,19 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
             for (int t = 0; t < JT; ++t) b[t] = half ? 0.f : b[t];
           }
 #pragma unroll
+          for (int i = 0; i < MT; ++i) row_sum[i] += a[i];
+#pragma unroll
           for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int t = 0; t < JT; ++t)
               acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[t], acc[i][t], 0, 0, 0);
         }
       }
+#pragma unroll
+      for (int i = 0; i < MT; ++i) unit_sum[i] += row_sum[i];
     }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) bias[i] += unit_sum[i];
   };
   __syncthreads();
   if (wp.nbuf == 2) {
@@ -463,7 +510,8 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
   // the block is slab 0 + slab 1, i.e. (w0 + w1) + (w2 + w3) whatever the timing; the write-out
   // has several words in flight per thread.
   __syncthreads();
-  float *red = lds;                                   // [2][M_T][J_T]
+  float *red = lds;                                   // [2][M_T][J_T], then the bias sums
+  if (bias_ws && jg == 0) bias_to_lds<MT>(bias, red + 2 * M_T * J_T, wave, half, l32);
   for (int phase = 0; phase < 2; ++phase) {
     if ((wave & 1) == phase) {
       float *slab = red + (wave >> 1) * (M_T * J_T);
@@ -481,6 +529,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
     }
     __syncthreads();
   }
+  if (bias_ws && jg == 0 && tid < M_T) bias_ws[(i64)blockIdx.x * wp.M_pad + m0 + tid] = bias_of_waves<M_T>(red + 2 * M_T * J_T, tid);
   float *out = ws + (i64)blockIdx.x * wp.M_pad * wp.J_pad + (i64)m0 * wp.J_pad + j0;
   constexpr int kTrip = 4;                             // words a thread has in flight (M_T * J_T is a multiple of 1024)
   for (int e0 = tid; e0 < M_T * J_T; e0 += kTrip * kThreads) {
@@ -520,16 +569,18 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
 // flight and a wait for one never drags in the younger ones.  Needs unit y stride, no y
 // up-sampling and unit y dilation (consecutive filter columns read consecutive words).
 constexpr int kStreamTasks = 2;                    // (channel, row, group) tasks a thread can hold in registers
-template <int MT, int JT>
+template <int MT, int JT, bool BIAS>
 __global__ __launch_bounds__(kThreads, (MT == 1 ? 3 : 2)) void wgrad_stream_kernel(
     WgradPlan wp, const float *__restrict__ A, const float *__restrict__ G,
-    float *__restrict__ ws) {
+    float *__restrict__ ws, float *__restrict__ bias_ws) {
   extern __shared__ __align__(16) float lds[];
   const TilePlan &pl = wp.t;
   constexpr int M_T = MT * 32, J_T = JT * 32;
   const int RB = kWaves * wp.rpw;                    // output rows per unit
   const int NG = (pl.noy + 7) >> 3;                  // groups per row
   const int tail0 = pl.noy - 8;                      // first position of a row's last group
+  constexpr int kTailBit = 20;                       // (BIAS: a row's last group is marked in its fragment offset, below 2^20)
+  const int dead_tail = 8 * (NG - 1) - tail0;        // positions of it that the group before has
   const int tasks_max = wp.CCj * pl.R * NG;          // (channel, virtual row, group) triples
   const int bf_part = tasks_max * pl.nfy + 1;        // fragments per part; the last word of a part is zeros
   uintx4 *Bf = (uintx4 *)lds;                        // [3][CCj][R][NG][nfy] (+ the zero word)
@@ -575,7 +626,8 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 3 : 2)) void wgrad_stream_kern
   for (int i = tid; i < RB * NG + 1; i += kThreads) {
     int r, g;
     by_ng.divmod(i, r, g);                              // group i of the unit: row r, group g of the row
-    step_tab[i] = make_int2(r * pl.noy + (g == NG - 1 ? tail0 : 8 * g), (pl.Ax * r * NG + g) * pl.nfy);
+    step_tab[i] = make_int2(r * pl.noy + (g == NG - 1 ? tail0 : 8 * g),
+                            (pl.Ax * r * NG + g) * pl.nfy + (BIAS && g == NG - 1 ? 1 << kTailBit : 0));
   }
   if (tid < 3) Bf[tid * bf_part + bf_part - 1] = uintx4{0u, 0u, 0u, 0u};
 
@@ -697,6 +749,9 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 3 : 2)) void wgrad_stream_kern
   struct AOp { float4 lo[MT], hi[MT]; int bword; };
   const float *abase = A;                               // grad_out of the unit's image and first row (wave-uniform)
   int live_groups = 0;                                  // groups of the current unit
+  float bias[MT], unit_sum[MT];                         // (of a unit, then of units: a rounding error meets few others)
+#pragma unroll
+  for (int i = 0; i < MT; ++i) bias[i] = unit_sum[i] = 0.f;
   auto load_a = [&](int s, AOp &o) {
     int gi = 2 * s + half;
     const bool live = gi < live_groups;
@@ -715,13 +770,21 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 3 : 2)) void wgrad_stream_kern
     uintx4 bh[JT], bm[JT], bl[JT];
 #pragma unroll
     for (int t = 0; t < JT; ++t) {
-      const uintx4 *b = Bf + (o.bword >= 0 ? col_word[t] + o.bword : bf_part - 1);
+      const uintx4 *b = Bf + (o.bword >= 0 ? col_word[t] + (BIAS ? o.bword & ((1 << kTailBit) - 1) : o.bword) : bf_part - 1);
       bh[t] = b[0]; bm[t] = b[bf_part]; bl[t] = b[2 * bf_part];
     }
     uintx4 ah[MT], am[MT], al[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const float x[8] = {o.lo[i].x, o.lo[i].y, o.lo[i].z, o.lo[i].w, o.hi[i].x, o.hi[i].y, o.hi[i].z, o.hi[i].w};
+      if constexpr (BIAS) {
+        // (positions that the group before has, and groups past the last, do not count)
+        const int dead = o.bword < 0 ? 8 : (o.bword >> kTailBit) * dead_tail;
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = e >= dead ? x[e] : 0.f;
+        unit_sum[i] += ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
+      }
       split8(x, ah[i], am[i], al[i]);
     }
 #pragma unroll
@@ -760,11 +823,19 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 3 : 2)) void wgrad_stream_kern
       if (s + 4 * kWaves < steps) load_a(s + 4 * kWaves, b1);
       multiply_step(b2);
     }
+    if constexpr (BIAS)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        bias[i] += unit_sum[i];
+        unit_sum[i] = 0.f;
+      }
   }
 
   // ---- sum the four wavefronts in wave order, then write the partial block ------
   __syncthreads();
-  float *red = lds;                                   // [M_T][J_T]
+  float *red = lds;                                   // [M_T][J_T], then the bias sums
+  if constexpr (BIAS)
+    if (jg == 0) bias_to_lds<MT>(bias, red + M_T * J_T, wave, half, l32);
   for (int w = 0; w < kWaves; ++w) {
     if (wave == w) {
 #pragma unroll
@@ -781,6 +852,8 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 3 : 2)) void wgrad_stream_kern
     }
     __syncthreads();
   }
+  if constexpr (BIAS)
+    if (jg == 0 && tid < M_T) bias_ws[(i64)blockIdx.x * wp.M_pad + m0 + tid] = bias_of_waves<M_T>(red + M_T * J_T, tid);
   float *out = ws + (i64)blockIdx.x * wp.M_pad * wp.J_pad + (i64)m0 * wp.J_pad + j0;
   for (int e = tid; e < M_T * J_T; e += kThreads) {
     const int m = e / J_T, jj = e - m * J_T;
@@ -788,36 +861,44 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 3 : 2)) void wgrad_stream_kern
   }
 }
 
-// W[m, j] = sum over the S partial blocks, in index order.  A block of 256
+// W[m, j] = sum over the S partial blocks, in a fixed order.  A block of 256
 // threads handles 16 outputs: 16 threads per output add every 16th partial,
-// then thread 0 of each output adds the 16 sums in order.
+// then thread 0 of each output adds the 16 sums in pairs.  Behind the M J weights
+// come, with bias_ws, the M sums of grad_out: gb[m] of the partial sums bias_ws[s, m].
 template <typename O>                                  // O: float, or _Float16 (rounded once)
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restrict__ ws,
                                                            O *__restrict__ W, int S, int M,
-                                                           int J, int M_pad, int J_pad) {
+                                                           int J, int M_pad, int J_pad, const float *__restrict__ bias_ws,
+                                                           O *__restrict__ gb) {
   __shared__ float part[16][17];
   const int el = threadIdx.x & 15, ph = threadIdx.x >> 4;
-  const int e = blockIdx.x * 16 + el;
+  const int e = blockIdx.x * 16 + el, outputs = M * J + (bias_ws ? M : 0);
   float sum = 0.f;
-  if (e < M * J) {
+  if (e < outputs) {
     const int m = e / J, j = e - m * J;
-    const float *src = ws + (i64)m * J_pad + j;
-    const i64 stride = (i64)M_pad * J_pad;
+    const bool weight = e < M * J;
+    const float *src = weight ? ws + (i64)m * J_pad + j : bias_ws + (e - M * J);
+    const i64 stride = weight ? (i64)M_pad * J_pad : M_pad;
     int s = ph;
     for (; s + 48 < S; s += 64) {
       const float v0 = src[(i64)s * stride], v1 = src[(i64)(s + 16) * stride];
       const float v2 = src[(i64)(s + 32) * stride], v3 = src[(i64)(s + 48) * stride];
-      sum += v0; sum += v1; sum += v2; sum += v3;
+      sum += (v0 + v1) + (v2 + v3);
     }
     for (; s < S; s += 16) sum += src[(i64)s * stride];
   }
   part[ph][el] = sum;
   __syncthreads();
-  if (ph == 0 && e < M * J) {
-    float tot = part[0][el];
+  if (ph == 0 && e < outputs) {
+    float v[16];
 #pragma unroll
-    for (int k = 1; k < 16; ++k) tot += part[k][el];
-    W[e] = (O)tot;
+    for (int k = 0; k < 16; ++k) v[k] = part[k][el];
+#pragma unroll
+    for (int n = 8; n > 0; n >>= 1)
+#pragma unroll
+      for (int k = 0; k < n; ++k) v[k] += v[k + n];
+    const float tot = v[0];
+    (e < M * J ? W[e] : gb[e - M * J]) = (O)tot;
   }
 }
 
@@ -835,28 +916,30 @@ hipError_t launch_variant(const WgradPlan &wp, size_t lds_bytes, dim3 grid, cons
 }
 
 template <int MT, int JT>
-hipError_t launch_rows(const WgradPlan &wp, dim3 grid, const float *a, const float *g, float *ws,
+hipError_t launch_rows(const WgradPlan &wp, dim3 grid, const float *a, const float *g, float *ws, float *bias_ws,
                        hipStream_t stream) {
   auto kern = wgrad_rows_kernel<MT, JT>;
+  const size_t lds = bias_ws ? std::max(wp.lds_bytes, 4 * (size_t)(2 * MT * 32 * JT * 32 + kWaves * MT * 32)) : wp.lds_bytes;
   {
     static std::atomic<int> lds_allowed{0};                // (one per kernel instance)
-    hipError_t e = allow_large_lds((const void *)kern, wp.lds_bytes, lds_allowed);
+    hipError_t e = allow_large_lds((const void *)kern, lds, lds_allowed);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kern, grid, dim3(kThreads), wp.lds_bytes, stream, wp, a, g, ws);
+  hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds, stream, wp, a, g, ws, bias_ws);
   return hipGetLastError();
 }
 
-template <int MT, int JT>
-hipError_t launch_stream(const WgradPlan &wp, dim3 grid, const float *a, const float *g, float *ws,
+template <int MT, int JT, bool BIAS>
+hipError_t launch_stream(const WgradPlan &wp, dim3 grid, const float *a, const float *g, float *ws, float *bias_ws,
                          hipStream_t stream) {
-  auto kern = wgrad_stream_kernel<MT, JT>;
+  auto kern = wgrad_stream_kernel<MT, JT, BIAS>;
+  const size_t lds = BIAS ? std::max(wp.lds_bytes, 4 * (size_t)(MT * 32 * JT * 32 + kWaves * MT * 32)) : wp.lds_bytes;
   {
     static std::atomic<int> lds_allowed{0};                // (one per kernel instance)
-    hipError_t e = allow_large_lds((const void *)kern, wp.lds_bytes, lds_allowed);
+    hipError_t e = allow_large_lds((const void *)kern, lds, lds_allowed);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kern, grid, dim3(kThreads), wp.lds_bytes, stream, wp, a, g, ws);
+  hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds, stream, wp, a, g, ws, bias_ws);
   return hipGetLastError();
 }
 
@@ -1036,19 +1119,26 @@ static bool make_wgrad_plan_jt(const SepConv &fwd, WgradPlan &wp, bool g_allow_r
   return true;
 }
 
+size_t wgrad_bias_bytes(const WgradPlan &wp) {
+  // (the rows past the last that has a tap are not read)
+  return wp.rows_mode && wp.t.nox_eff == wp.t.nox ? (size_t)wp.S * wp.M_pad * sizeof(float) : 0;
+}
+
 hipError_t launch_wgrad(const WgradPlan &wp, const float *grad_out, const float *input,
-                        float *grad_weight, float *workspace, hipStream_t stream) {
+                        float *grad_weight, float *workspace, hipStream_t stream, float *bias_ws, float *grad_bias) {
   dim3 grid((unsigned)wp.S, (unsigned)(wp.m_groups * wp.j_groups));
   hipError_t e = hipErrorInvalidValue;
   if (wp.rows_mode == 2) {
 #define MELLIN_STREAM_CASE(MT_, JT_)                                                       \
-  if (wp.mt == MT_ && wp.jt == JT_) e = launch_stream<MT_, JT_>(wp, grid, grad_out, input, workspace, stream);
+  if (wp.mt == MT_ && wp.jt == JT_)                                                         \
+    e = bias_ws ? launch_stream<MT_, JT_, true>(wp, grid, grad_out, input, workspace, bias_ws, stream)       \
+                : launch_stream<MT_, JT_, false>(wp, grid, grad_out, input, workspace, nullptr, stream);
     MELLIN_STREAM_CASE(1, 1) MELLIN_STREAM_CASE(1, 2) MELLIN_STREAM_CASE(1, 3)
     MELLIN_STREAM_CASE(2, 1) MELLIN_STREAM_CASE(2, 2) MELLIN_STREAM_CASE(2, 3)
 #undef MELLIN_STREAM_CASE
   } else if (wp.rows_mode) {
 #define MELLIN_ROWS_CASE(MT_, JT_)                                                         \
-  if (wp.mt == MT_ && wp.jt == JT_) e = launch_rows<MT_, JT_>(wp, grid, grad_out, input, workspace, stream);
+  if (wp.mt == MT_ && wp.jt == JT_) e = launch_rows<MT_, JT_>(wp, grid, grad_out, input, workspace, bias_ws, stream);
     MELLIN_ROWS_CASE(1, 1) MELLIN_ROWS_CASE(1, 2) MELLIN_ROWS_CASE(1, 3)
     MELLIN_ROWS_CASE(2, 1) MELLIN_ROWS_CASE(2, 2) MELLIN_ROWS_CASE(2, 3)
 #undef MELLIN_ROWS_CASE
@@ -1062,9 +1152,9 @@ hipError_t launch_wgrad(const WgradPlan &wp, const float *grad_out, const float 
 #undef MELLIN_WGRAD_CASE
   }
   if (e != hipSuccess) return e;
-  const int outputs = wp.t.M * wp.J;
+  const int outputs = wp.t.M * wp.J + (bias_ws ? wp.t.M : 0);
   hipLaunchKernelGGL(wgrad_reduce_kernel<float>, dim3((unsigned)((outputs + 15) / 16)), dim3(256), 0, stream,
-                     (const float *)workspace, grad_weight, wp.S, wp.t.M, wp.J, wp.M_pad, wp.J_pad);
+                     (const float *)workspace, grad_weight, wp.S, wp.t.M, wp.J, wp.M_pad, wp.J_pad, (const float *)bias_ws, grad_bias);
   return hipGetLastError();
 }
 
@@ -1073,10 +1163,10 @@ hipError_t launch_wgrad_reduce(const float *partials_ws, void *W, bool half_out,
   const dim3 grid((unsigned)((M * J + 15) / 16));
   if (half_out)
     hipLaunchKernelGGL(wgrad_reduce_kernel<_Float16>, grid, dim3(256), 0, stream, partials_ws, (_Float16 *)W,
-                       partials, M, J, M_pad, J_pad);
+                       partials, M, J, M_pad, J_pad, (const float *)nullptr, (_Float16 *)nullptr);
   else
     hipLaunchKernelGGL(wgrad_reduce_kernel<float>, grid, dim3(256), 0, stream, partials_ws, (float *)W, partials,
-                       M, J, M_pad, J_pad);
+                       M, J, M_pad, J_pad, (const float *)nullptr, (float *)nullptr);
   return hipGetLastError();
 }
 

@@ -1766,12 +1766,13 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
   // (half gradients of the parameters on their way to float)
   lb.gw_off = take(wide && ww && !lb.weight_blocked ? (size_t)(c_out * c_in * nfx * nfy) * 2 : 0);
   lb.gb_off = take(wide && lb.plain && (want & MELLIN_WANT_BIAS) ? (size_t)c_out * 2 : 0);
-  const size_t beside = !half && lb.plain && ww && !lb.weight_blocked && (want & MELLIN_WANT_BIAS) && !(want & MELLIN_WANT_RELU)
+  const size_t beside = !half && lb.plain && ww && !lb.weight_blocked && (want & MELLIN_WANT_BIAS)
                             ? bias_beside_weight(kind_x, CORR2D_ARGS) : 0;
   lb.bias_beside = beside > 0;
   lb.beside_off = take(beside);
   size_t pass = 0;
-  if (lb.plain && !lb.bias_beside && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU)))   // (a ReLU's backward writes the bias gradient, asked for or not)
+  const int want_pass = want & (MELLIN_WANT_RELU | (lb.bias_beside ? 0 : MELLIN_WANT_BIAS));
+  if (lb.plain && want_pass)                           // (a ReLU's backward writes the bias gradient, asked for or not)
     pass = align256(mellin_bias_grad_workspace(batch, c_out, nhx * nhy)) + align256((size_t)c_out * elem);
   if (wi && !lb.input_blocked)
     pass = std::max(pass, half ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS)
@@ -1833,10 +1834,10 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT, relu = want & MELLIN_WANT_RELU;
   hipStream_t st = (hipStream_t)stream;
   hipError_t e = hipSuccess;
-  if (lb.plain && !lb.bias_beside && (want & (MELLIN_WANT_BIAS | MELLIN_WANT_RELU))) {
+  if (lb.plain && (want & (MELLIN_WANT_RELU | (lb.bias_beside ? 0 : MELLIN_WANT_BIAS)))) {
     void *masked = relu ? ws + lb.masked_off : nullptr;
     const size_t own = mellin_bias_grad_workspace(batch, c_out, nhx * nhy);
-    void *gb = !(want & MELLIN_WANT_BIAS) ? pass + align256(own) : wide ? ws + lb.gb_off : grad_bias;
+    void *gb = !(want & MELLIN_WANT_BIAS) || lb.bias_beside ? pass + align256(own) : wide ? ws + lb.gb_off : grad_bias;
     rc = half ? mellin_bias_grad_f16(grad_out, masked ? out : nullptr, batch, c_out, nhx * nhy, masked, gb, pass, own, stream)
               : mellin_bias_grad_f32((const float *)grad_out, masked ? (const float *)out : nullptr, batch, c_out,
                                      nhx * nhy, (float *)masked, (float *)gb, pass, own, stream);

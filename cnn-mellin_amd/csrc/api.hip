@@ -1567,7 +1567,7 @@ static bool blocks_allowed(bool half) {
 // the launch), and choosing among tile shapes takes some microseconds.  The sizes decide the plan, so nothing has to be
 // thrown away.
 struct LayerPlans {
-  int known[4];                                        // 0 not yet, 1 applies, -1 does not
+  int known[5];                                        // 0 not yet, 1 applies, -1 does not
   size_t bias_bytes;                                   // section 2's weight gradient: for the bias gradient beside it (known[3])
   BlockPlan forward, input;
   BlockWgradPlan weight;
@@ -1583,6 +1583,34 @@ static LayerPlans &layer_plans(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
 // A forward pass is one launch there and two here, and pays only for long Mellin layers of half tensors (1.2 to 2 times).
 constexpr double kShortLayerHalf = 4e9, kShortLayerFloat = 0.08e9;
 enum { PASS_FORWARD, PASS_INPUT, PASS_WEIGHT };
+// Input gradients of longer layers with few channels that section 2 has no good kernel for.  Both sides measured over 210 float
+// and 150 half layers drawn over 1 to 15 input channels (section 2 -> blocked, us):
+//   the gather form, whose matrix tiles hold c_in of 32 rows (more than 128 output channels, or taps that fill less than a
+//   quarter of their tiles): 1333 -> 413, 404 -> 230, 146 -> 19, none slower;
+//   float, the fused kernel on fp32 instructions (taps in no whole eights), whose work grows with c_in where a blocked tile's
+//   does not: 154 -> 64, 61 -> 40, 34 -> 19 within 0.5 G multiply-adds of whole blocks per channel, 71 -> 94 and 55 -> 111 beyond;
+//   one column (1-D layers), any kernel: 53 -> 19, 62 -> 19, 33 -> 17; but 19 -> 22 and 28 -> 40 beyond 0.3 G per channel;
+//   half, on linear axes, what would go through float copies: 1071 -> 98, 264 -> 64, 59 -> 41, none slower.
+static bool few_channels_input(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
+  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
+  if (!lp.known[4]) {
+    const bool one_column = nfy == 1 && ngy == 1 && nhy == 1;
+    const double work = (double)batch * ngx * ngy * 32 * ((c_out + 7) / 8 * 8) * nfx * nfy / (double)c_in;
+    bool blocked;
+    if (half) {
+      IgradPlan ip;
+      TwoPassInput tp;
+      blocked = one_column || (kind_x == AX_LCORR && !plan_half_fused(kind_x, CORR2D_ARGS, ip) && !plan_half_two_pass(kind_x, CORR2D_ARGS, tp));
+    } else {
+      InputPlans ips;
+      const int which = choose_input_plan(kind_x, CORR2D_ARGS, ips);
+      blocked = which == IN_GATHER || (one_column && (which != IN_FUSED || work <= 0.3e9)) ||
+                (!one_column && which == IN_FUSED && !ips.fused.stream && work <= 0.5e9);
+    }
+    lp.known[4] = blocked ? 1 : -1;
+  }
+  return lp.known[4] > 0;
+}
 static bool blocks_apply(int pass, int kind_x, bool half, MELLIN_CORR2D_DIMS) {
   if (!blocks_allowed(half) || batch * c_out * nhx * nhy * c_in == 0) return false;
   if (c_in >= 16) return true;
@@ -1593,7 +1621,8 @@ static bool blocks_apply(int pass, int kind_x, bool half, MELLIN_CORR2D_DIMS) {
   const double most = std::max(in * 32 * up(c_out, 8), out * 32 * up(c_out, 32)) * taps;
   const double few = kind_x == AX_LCORR && c_in <= 3 && c_out <= 64 ? 0.25 : 1;     // (the streaming kernels' own class)
   if (most <= few * (half ? kShortLayerHalf : kShortLayerFloat)) return true;
-  return pass == PASS_INPUT && half && kind_x == AX_LCORR && c_in >= 8 && nfx * nfy <= 16;
+  if (pass != PASS_INPUT) return false;
+  return (half && kind_x == AX_LCORR && c_in >= 8 && nfx * nfy <= 16) || few_channels_input(kind_x, half, CORR2D_ARGS);
 }
 static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp) {
   if (!blocks_apply(PASS_FORWARD, kind_x, half, CORR2D_ARGS)) return false;

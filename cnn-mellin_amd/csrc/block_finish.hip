@@ -115,7 +115,8 @@ __device__ void finish_units(const FinishArgs &a, int b, float (*red)[32]) {
   const int chunks = (units + kFinishThreads - 1) / kFinishThreads;
   const int tm = b / chunks, at = (b - tm * chunks) * kFinishThreads + (int)threadIdx.x;      // (tile, tile of channels), unit in it
   const int r = tm / pl.m_tiles, g_t = at / P, p = at - g_t * P, group = (tm - r * pl.m_tiles) * (m_t / 8) + g_t;
-  const int id = pl.whole + r, qt = id / pl.batch, n = id - qt * pl.batch, q0 = qt * P, count = min(P, pl.Q - q0);
+  const int id = pl.whole + r, qt = id / pl.tile_batch, q0 = qt * P, count = min(P, pl.tile_q - q0);
+  int n = id - qt * pl.tile_batch;
   const bool live = at < units && group < pl.out_groups && p < count;
   float v[8];
 #pragma unroll
@@ -131,7 +132,9 @@ __device__ void finish_units(const FinishArgs &a, int b, float (*red)[32]) {
     // held there must not become a blocked tensor's padding)
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] = group * 8 + c < pl.M ? v[c] : 0.f;
-    const int row = (q0 + p) / pl.noy, oy = q0 + p - row * pl.noy;
+    int row = (q0 + p) / pl.noy;
+    const int oy = q0 + p - row * pl.noy;
+    if (pl.joint) { n = row % pl.batch; row /= pl.batch; }
     q = (a.s_rows ? a.s_rows[row].x : row) * pl.noy + oy;
     const i64 unit = ((i64)n * pl.out_groups + group) * (pl.Q + 1) + q;
     if (a.sa.grad) {
@@ -157,7 +160,7 @@ __device__ void finish_units(const FinishArgs &a, int b, float (*red)[32]) {
         o[1] = mid;
         o[2] = lo;
       }
-      if (q0 + p == pl.Q - 1) {                        // the unit of zeros behind the image
+      if (pl.joint ? q == pl.Q - 1 : q0 + p == pl.Q - 1) {     // the unit of zeros behind the image
         uintx4 *z = (uintx4 *)((char *)a.sa.out + (((i64)n * pl.out_groups + group) * (pl.Q + 1) + pl.Q) * UB);
         const uintx4 zero = {0, 0, 0, 0};
 #pragma unroll
@@ -230,7 +233,7 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
   const int m_t = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32, chunks = m_t * P / kSliceValues;
   const int tm = (int)b / chunks, at = ((int)b - tm * chunks) * kSliceValues + tid * 4;   // (tile, tile of channels), value in it
   const int r = tm / pl.m_tiles, c = at / P, p = at - c * P, m = (tm - r * pl.m_tiles) * m_t + c;
-  const int id = pl.whole + r, qt = id / pl.batch, n = id - qt * pl.batch, q0 = qt * P, count = min(P, pl.Q - q0) - p;
+  const int id = pl.whole + r, qt = id / pl.tile_batch, n = id - qt * pl.tile_batch, q0 = qt * P, count = min(P, pl.tile_q - q0) - p;
   if (m >= pl.M || count <= 0) return;
   const i64 slice = (i64)pl.rest * pl.m_tiles * m_t * P;
   const float *from = a.sa.sums + (i64)tm * m_t * P + at;
@@ -246,7 +249,8 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
   T *out = (T *)a.sa.out + n * pl.h_n + m * pl.h_m;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    if (i < count) out[(a.s_rows ? a.s_rows[row].x : row) * pl.noy + oy] = (T)o[i];
+    const int at = pl.joint ? row / pl.batch : row;
+    if (i < count) out[(pl.joint ? (row - at * pl.batch) * pl.h_n : 0) + (a.s_rows ? a.s_rows[at].x : at) * pl.noy + oy] = (T)o[i];
     if (++oy == pl.noy) { oy = 0; ++row; }
   }
 }

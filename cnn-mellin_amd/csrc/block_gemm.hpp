@@ -55,6 +55,10 @@ struct BlockPlan {
   size_t lds_bytes;
   size_t rows_off, filter_bytes;   // the packed filter: fragments, then (Mellin axes) the output rows in the order of their classes
   size_t slice_bytes;              // workspace of the slices' sums
+  // `joint`: a tile's positions run over the images of an output row (row, image, column), not over the rows of an image;
+  // tile_batch and tile_q: images that are numbered apart (1) and positions that tiles are cut from (all there are), else
+  // batch and Q
+  int joint, tile_batch, tile_q;
 };
 
 // False: the kernel does not apply.

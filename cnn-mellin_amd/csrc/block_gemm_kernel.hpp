@@ -25,6 +25,9 @@
 // of a tile have taps for the same filter rows and only those are staged and multiplied; filter
 // rows none of whose taps lies inside the signal for the tile's rows are left out as well.
 //
+// Small images on Mellin axes (JOINT): a tile's positions run over the images of an output row, whose rows have taps for the
+// same filter rows; its virtual rows are those of (output row, image) pairs.
+//
 // Few tiles (one utterance, deep layers): WK = 4 wavefronts share the positions of a tile and
 // take every fourth step of a stage; their sums are added in wavefront order through LDS.
 //
@@ -54,7 +57,7 @@ enum { OUT_PLAIN, OUT_BLOCKED, GRAD_PLAIN, GRAD_BLOCKED };
 typedef const __attribute__((address_space(4))) BlockPlan ConstBlockPlan;
 
 struct BlockTile {
-  int n, q0, count, row_lo, rows;
+  int n, q0, count, row_lo, rows;  // (rows of a joint tile: the (output row, image) pairs that it has positions of)
   int id;                          // the tile
   int c_first, c_end, slot, slice; // its channel groups; in slices: place in the workspace, which slice (whole tiles: -1, 0)
   int vx_min, vrows, units;        // linear axes: first coordinate; virtual rows and positions of the whole tile
@@ -67,7 +70,7 @@ __device__ __forceinline__ int filter_row(const BlockTile &g, int j) { return (i
 // Item `id` of the launch: the images of a position tile lie side by side, so that the position tiles
 // with the most filter rows come first for all images and every workgroup gets its share of them.
 // `rows`: the output rows in the order of their classes, with their filter rows (Mellin axes).
-template <int P>
+template <int P, bool JOINT>
 __device__ __forceinline__ BlockTile block_tile(ConstBlockPlan &pl, const int2 *__restrict__ rows, int id, bool mellin_x) {
   BlockTile g;
   g.c_first = 0;
@@ -83,17 +86,20 @@ __device__ __forceinline__ BlockTile block_tile(ConstBlockPlan &pl, const int2 *
     id = pl.whole + r;
   }
   g.id = id;
-  const int qt = udiv(id, pl.batch, pl.mg_batch);
-  g.n = id - qt * pl.batch;
+  const int qt = JOINT ? id : udiv(id, pl.batch, pl.mg_batch);
+  g.n = JOINT ? 0 : id - qt * pl.batch;
   g.q0 = qt * P;
-  g.count = min(P, pl.Q - g.q0);
+  g.count = min(P, (JOINT ? pl.tile_q : pl.Q) - g.q0);
   g.row_lo = udiv(g.q0, pl.noy, pl.mg_noy);
   g.rows = udiv(g.q0 + g.count - 1, pl.noy, pl.mg_noy) - g.row_lo + 1;
   g.vx_min = pl.ax * g.row_lo + pl.cx + pl.bx_min;
   g.filter_rows = 0;
   if (mellin_x) {
     int mask = 0;
-    for (int r = (int)threadIdx.x & 63; r < g.rows; r += 64) mask |= rows[g.row_lo + r].y;
+    for (int r = (int)threadIdx.x & 63; r < g.rows; r += 64) {
+      const int at = g.row_lo + r;
+      mask |= rows[JOINT ? udiv(at, pl.batch, pl.mg_batch) : at].y;
+    }
     g.nv = 0;
     for (int f = 0; f < pl.nfx; ++f)
       if (__ballot(mask >> f & 1)) g.filter_rows |= (unsigned long long)f << (4 * g.nv++);
@@ -186,7 +192,7 @@ __device__ __forceinline__ void cut_four(const float4 &v, unsigned (&w)[F16 ? 1 
   }
 }
 
-template <int MT, int NT, int WM, int WK, bool F16, int OUT>
+template <int MT, int NT, int WM, int WK, bool F16, int OUT, bool JOINT>
 __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_arg, const char *__restrict__ X,
                                                                  const char *__restrict__ AF, const void *__restrict__ bias,
                                                                  void *__restrict__ Hv, float *__restrict__ sums,
@@ -208,7 +214,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
   const int wk = WK > 1 ? wave : 0, wm = WM > 1 ? wave & (WM - 1) : 0, wn = WK > 1 ? 0 : wave / WM;
-  const bool mellin_x = pl.kind_x == AX_MCORR || pl.kind_x == AX_MCONV;
+  const bool mellin_x = JOINT || pl.kind_x == AX_MCORR || pl.kind_x == AX_MCONV;
   const int taps = pl.nfx * pl.nfy;
   const int m_tile = blockIdx.y;
   const unsigned zero_frag = (unsigned)(pl.CG * taps * PARTS * 512);       // the tile's fragment of zeros, behind the others
@@ -242,10 +248,16 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
     if (mellin_x) {
       const FastDiv by_rows(g.rows);
       for (int t = tid; t < g.nv * g.rows; t += kThreads) {
-        int j, r;
+        int j, r, from = 0;
         by_rows.divmod(t, j, r);
-        const int gx = mellin_tap32(kx, rows[g.row_lo + r].x, filter_row(g, j), ngx, sx, dx, px + 1, ux, mg_p1);
-        row_src[t] = gx >= 0 ? gx * ngy : -1;
+        r += g.row_lo;
+        if (JOINT) {
+          const int pair = r;
+          r = udiv(pair, pl.batch, pl.mg_batch);
+          from = (pair - r * pl.batch) * pl.CG * (none + 1);               // the image's units
+        }
+        const int gx = mellin_tap32(kx, rows[r].x, filter_row(g, j), ngx, sx, dx, px + 1, ux, mg_p1);
+        row_src[t] = gx >= 0 ? from + gx * ngy : -1;
       }
       lds_barrier();
     }
@@ -351,7 +363,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       for (int pt = 0; pt < PARTS; ++pt) o.a[k][pt] = *(const uintx4 *)((k ? AFm1 : AFm) + off + pt * 512);
   };
 
-  BlockTile tg = block_tile<P>(pl, rows, (int)blockIdx.x, mellin_x), next_tg = tg;
+  BlockTile tg = block_tile<P, JOINT>(pl, rows, (int)blockIdx.x, mellin_x), next_tg = tg;
   if (my_tiles <= 0) return;
   int n_ents = build_tile(tg, 0, nullptr), next_ents = n_ents;
   __syncthreads();
@@ -386,7 +398,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
         if (local >= tg.count) local = 0;
         const int row = udiv(tg.q0 + local, pl.noy, pl.mg_noy), oy = tg.q0 + local - row * pl.noy;
         lane_vpos[t] = (((mellin_x ? 1 : pl.ax) * (row - tg.row_lo)) * pl.RS + pl.ay * oy) * UB;
-        lane_q[t] = (mellin_x ? rows[row].x : row) * pl.noy + oy;
+        lane_q[t] = (mellin_x ? rows[JOINT ? udiv(row, pl.batch, pl.mg_batch) : row].x : row) * pl.noy + oy;
       }
 #pragma unroll
       for (int i = 0; i < MT; ++i)
@@ -422,7 +434,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       nj0 = 0;
       if (more) {
         // another tile: its tables (every load of this tile has been issued, every wavefront is past the barrier)
-        next_tg = block_tile<P>(pl, rows, (int)blockIdx.x + (ti + 1) * (int)gridDim.x, mellin_x);
+        next_tg = block_tile<P, JOINT>(pl, rows, (int)blockIdx.x + (ti + 1) * (int)gridDim.x, mellin_x);
         next_ents = build_tile(next_tg, (ti + 1) & 1, ents + (ti & 1) * pl.ents + n_ents);
         lds_barrier();
         nc0 = next_tg.c_first;
@@ -499,13 +511,24 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       // A gradient's mask, and the sums of its channels over the tile's positions
       const unsigned unit_row = (unsigned)(pl.Q + 1) * UB;                  // bytes of a channel group of a blocked output
       const i64 image_bytes = (i64)pl.out_groups * unit_row;
+      // joint: the images of the lane's positions
+      int lane_n[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        lane_n[t] = 0;
+        if constexpr (JOINT) {
+          const int local = (wn * NT + t) * 32 + l32, pair = udiv(tg.q0 + (local < tg.count ? local : 0), pl.noy, pl.mg_noy);
+          lane_n[t] = pair - udiv(pair, pl.batch, pl.mg_batch) * pl.batch;
+        }
+      }
+      const int all_images = (int)image_bytes * (JOINT ? pl.batch : 1);
       __amdgpu_buffer_rsrc_t mask_rsrc;
       if constexpr (GRAD)
-        mask_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(mask) + tg.n * image_bytes, 0, (int)image_bytes, 0x00020000);
+        mask_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(mask) + tg.n * image_bytes, 0, all_images, 0x00020000);
       int unit_at[NT];                                 // the lane's quarter unit in its group (none: past any end)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        unit_at[t] = (wn * NT + t) * 32 + l32 < tg.count ? lane_q[t] * UB + half * 8 : (int)0x80000000u;
+        unit_at[t] = (wn * NT + t) * 32 + l32 < tg.count ? lane_n[t] * (int)image_bytes + lane_q[t] * UB + half * 8 : (int)0x80000000u;
       auto masked = [&](float4 v, int group, int at) {
         const uintx2 x = __builtin_amdgcn_raw_buffer_load_b64(mask_rsrc, at < 0 ? at : at + (int)(group * unit_row), 0, 0);   // (none: zeros)
         auto keep = [](float f, unsigned sixteen) { return (short)sixteen > 0 ? f : 0.f; };
@@ -526,13 +549,13 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       char *base = whole ? (char *)Hv + ((i64)tg.n * pl.h_n + (i64)m0 * (int)pl.h_m) * ES
                          : (char *)(sums + (((i64)tg.slot * gridDim.y + m_tile) * M_T + wm * MT * 32) * P);
       const __amdgpu_buffer_rsrc_t rsrc =
-          BLOCKED && whole ? __builtin_amdgcn_make_buffer_rsrc((char *)Hv + tg.n * image_bytes, 0, (int)image_bytes, 0x00020000)
-                           : __builtin_amdgcn_make_buffer_rsrc(base, 0, max(0, min(MT * 32, pl.M - m0)) * h_m, 0x00020000);
+          BLOCKED && whole ? __builtin_amdgcn_make_buffer_rsrc((char *)Hv + tg.n * image_bytes, 0, all_images, 0x00020000)
+                           : __builtin_amdgcn_make_buffer_rsrc(base, 0, max(0, min(MT * 32, pl.M - m0)) * h_m + (whole && JOINT ? (pl.batch - 1) * (int)pl.h_n * ES : 0), 0x00020000);
       int at[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const int local = (wn * NT + t) * 32 + l32;
-        at[t] = local < tg.count ? (whole ? lane_q[t] : local) * ES : (int)0x80000000u;
+        at[t] = local < tg.count ? (whole ? lane_n[t] * (int)pl.h_n + lane_q[t] : local) * ES : (int)0x80000000u;
       }
       auto store_one = [&](float v, int to) {
         if (as_half) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(short, (_Float16)v), rsrc, to, 0, 0);
@@ -637,7 +660,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
         // in memory: a quarter of the stores (128 x 256 half values: 22000 -> 12000 cycles).  Not for the rows of a class
         // (n_classes > 1), which do not follow each other; the last positions of an image, less than four, go one by one.
         bool single = true;
-        if (BLOCKED || pl.n_classes == 1 || !whole) {
+        if (BLOCKED || (pl.n_classes == 1 && !JOINT) || !whole) {
           int to[NT];
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
@@ -674,7 +697,17 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
         }
       }
       if constexpr (BLOCKED)
-        if (whole && tg.q0 + tg.count == pl.Q && tid < M_T / 8 && m_tile * (M_T / 8) + tid < pl.out_groups) {
+        if constexpr (JOINT) {
+          // the units of zeros behind the images, which are dealt to the tiles
+          const int tiles = max(pl.whole, 1), lo = (int)((i64)tg.id * pl.batch / tiles), hi = whole ? (int)((i64)(tg.id + 1) * pl.batch / tiles) : lo;
+          for (int i = tid; i < (hi - lo) * (M_T / 8); i += kThreads) {
+            const int n = lo + i / (M_T / 8), group = m_tile * (M_T / 8) + i % (M_T / 8);
+            uintx4 *z = (uintx4 *)((char *)Hv + n * image_bytes + (i64)group * unit_row + (i64)pl.Q * UB);
+            const uintx4 zero = {0, 0, 0, 0};
+#pragma unroll
+            for (int pt = 0; pt < PARTS; ++pt) z[pt] = zero;
+          }
+        } else if (whole && tg.q0 + tg.count == pl.Q && tid < M_T / 8 && m_tile * (M_T / 8) + tid < pl.out_groups) {
           // the units of zeros behind an image's last positions
           uintx4 *z = (uintx4 *)((char *)Hv + tg.n * image_bytes + (i64)(m_tile * (M_T / 8) + tid) * unit_row + (i64)pl.Q * UB);
           const uintx4 zero = {0, 0, 0, 0};
@@ -695,15 +728,20 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
 #undef pl
 }
 
-template <int MT, int NT, int WM, int WK, bool F16, int OUT>
-hipError_t launch_instance(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream) {
-  auto kern = block_gemm_kernel<MT, NT, WM, WK, F16, OUT>;
+template <int MT, int NT, int WM, int WK, bool F16, int OUT, bool JOINT>
+hipError_t launch_joint(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream) {
+  auto kern = block_gemm_kernel<MT, NT, WM, WK, F16, OUT, JOINT>;
   static std::atomic<int> lds_allowed{0};
   hipError_t e = allow_large_lds((const void *)kern, pl.lds_bytes, lds_allowed);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3((unsigned)pl.grid_x, (unsigned)pl.m_tiles), dim3(kThreads), pl.lds_bytes, stream, pl,
                      (const char *)a.signal, (const char *)a.frag, a.bias, a.out, a.sums, (const char *)a.mask, a.chan_sums);
   return hipGetLastError();
+}
+
+template <int MT, int NT, int WM, int WK, bool F16, int OUT>
+hipError_t launch_instance(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream) {
+  return pl.joint ? launch_joint<MT, NT, WM, WK, F16, OUT, true>(pl, a, stream) : launch_joint<MT, NT, WM, WK, F16, OUT, false>(pl, a, stream);
 }
 
 template <int OUT>

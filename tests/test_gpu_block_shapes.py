@@ -19,6 +19,15 @@ CASES = [
     ("mcorr", 9, 24, 100, (4, 3), (90, 41), (1, 1), (1, 1), (1, 1), (45, 1)),
     ("lcorr", 34, 130, 24, (3, 3), (20, 41), (1, 1), (1, 1), (1, 1), (1, 1)),
     ("mcorr", 9, 100, 24, (4, 3), (90, 41), (1, 1), (1, 1), (1, 1), (45, 1)),
+    # small images on Mellin axes, whose tiles take an output row of several images: more tiles than workgroups, wavefronts
+    # sharing a tile, slices of the contracted channels (the last), images ending inside tiles, rows of one column
+    ("mcorr", 200, 64, 64, (5, 3), (10, 41), (1, 1), (1, 1), (2, 1), (4, 1)),
+    ("mcorr", 1177, 64, 64, (5, 3), (5, 41), (1, 1), (6, 1), (2, 1), (0, 1)),
+    ("mcorr", 300, 32, 96, (3, 3), (5, 40), (1, 1), (1, 1), (1, 1), (2, 1)),
+    ("mcorr", 300, 32, 128, (3, 3), (5, 40), (1, 1), (1, 1), (1, 1), (2, 1)),
+    ("mcorr", 400, 40, 32, (5, 3), (7, 13), (1, 1), (1, 1), (2, 1), (3, 1)),
+    ("mcorr", 900, 32, 32, (5, 1), (11, 1), (1, 1), (2, 1), (2, 0), (2, 0)),
+    ("mcorr", 9, 128, 128, (4, 4), (12, 10), (1, 1), (1, 1), (1, 1), (6, 2)),
 ]
 
 

@@ -129,6 +129,12 @@ def pack_windows(x: torch.Tensor, lens: torch.Tensor, window_size: int, window_s
     utterance and window index (time-major, as ``pack_padded_sequence`` orders them).  Returns
     the windows ``(N', 1, window_size, F)``, the convolution stack's input, and the
     ``PackedSequence`` whose ``batch_sizes`` / ``unsorted_indices`` undo the packing."""
+    if x.is_cuda:
+        # one copy of the windows' index and one launch (None: tensors and lengths that are not for it)
+        packed = _hip.native.pack_windows(x, lens, window_size, window_stride)
+        if packed is not None:
+            packed = torch.nn.utils.rnn.PackedSequence(*packed)
+            return packed.data.unsqueeze(1), packed
     if window_size > 1:
         x = torch.nn.functional.pad(x, (0, 0, 0, window_size - 1))
     windows = x.unfold(1, window_size, window_stride).transpose(2, 3)      # (N, T', w, F)

@@ -936,13 +936,13 @@ int check_log_lift(const char *fn, double eps, int flags, i64 outer, i64 t, i64 
 
 template <typename T>
 int log_lift_forward(const char *fn, const T *x, double eps, double tau, int flags, i64 outer, i64 t, i64 inner,
-                     T *y, void *stream, const T *params = nullptr) {
+                     T *y, void *stream, const T *eps_at = nullptr, const T *tau_at = nullptr, bool logs = false) {
   int rc;
   if ((rc = check_log_lift(fn, eps, flags, outer, t, inner))) return rc;
   if (outer * t * inner == 0) return MELLIN_OK;
   if (!x || !y) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", fn);
   hipError_t e = launch_log_lift_forward<T>(x, (T)eps, (T)tau, flags & MELLIN_PW_LOG, flags & MELLIN_PW_LIFT,
-                                            outer, t, inner, y, (hipStream_t)stream, params);
+                                            outer, t, inner, y, (hipStream_t)stream, eps_at, tau_at, logs);
   if (e != hipSuccess) return fail(MELLIN_ERR_RUNTIME, "%s: %s", fn, hipGetErrorString(e));
   return MELLIN_OK;
 }
@@ -950,17 +950,17 @@ int log_lift_forward(const char *fn, const T *x, double eps, double tau, int fla
 template <typename T>
 int log_lift_backward(const char *fn, const T *x, const T *gy, double eps, double tau, int flags, i64 outer,
                       i64 t, i64 inner, T *gx, T *grad_params, void *workspace, size_t workspace_bytes,
-                      void *stream, const T *params = nullptr) {
+                      void *stream, const T *eps_at = nullptr, const T *tau_at = nullptr, bool logs = false) {
   int rc;
   if ((rc = check_log_lift(fn, eps, flags, outer, t, inner))) return rc;
   if (!grad_params) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", fn);
   const size_t need = log_lift_workspace_bytes(outer, t, inner, sizeof(T));
-  if (need && (!x || !gy || !gx)) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", fn);
+  if (need && (!x || !gy || (!gx && !logs))) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", fn);
   if (need && (!workspace || workspace_bytes < need))
     return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", fn, need, workspace_bytes);
   hipError_t e = launch_log_lift_backward<T>(x, gy, (T)eps, (T)tau, flags & MELLIN_PW_LOG, flags & MELLIN_PW_LIFT,
                                              outer, t, inner, gx, grad_params, (T *)workspace,
-                                             (hipStream_t)stream, params);
+                                             (hipStream_t)stream, eps_at, tau_at, logs);
   if (e != hipSuccess) return fail(MELLIN_ERR_RUNTIME, "%s: %s", fn, hipGetErrorString(e));
   return MELLIN_OK;
 }
@@ -1314,26 +1314,47 @@ int mellin_log_lift_forward_f64(const double *x, double eps, double tau, int fla
 int mellin_log_lift_forward_dev_f32(const float *x, const float *params, int flags, int64_t outer, int64_t t,
                                     int64_t inner, float *y, void *stream) {
   if (!params) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
-  return log_lift_forward<float>(__func__, x, 1.0, 0.0, flags, outer, t, inner, y, stream, params);
+  return log_lift_forward<float>(__func__, x, 1.0, 0.0, flags, outer, t, inner, y, stream, params, params + 1);
 }
 int mellin_log_lift_forward_dev_f64(const double *x, const double *params, int flags, int64_t outer, int64_t t,
                                     int64_t inner, double *y, void *stream) {
   if (!params) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
-  return log_lift_forward<double>(__func__, x, 1.0, 0.0, flags, outer, t, inner, y, stream, params);
+  return log_lift_forward<double>(__func__, x, 1.0, 0.0, flags, outer, t, inner, y, stream, params, params + 1);
 }
 int mellin_log_lift_backward_dev_f32(const float *x, const float *grad_y, const float *params, int flags,
                                      int64_t outer, int64_t t, int64_t inner, float *grad_x, float *grad_params,
                                      void *workspace, size_t workspace_bytes, void *stream) {
   if (!params) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
   return log_lift_backward<float>(__func__, x, grad_y, 1.0, 0.0, flags, outer, t, inner, grad_x, grad_params,
-                                  workspace, workspace_bytes, stream, params);
+                                  workspace, workspace_bytes, stream, params, params + 1);
 }
 int mellin_log_lift_backward_dev_f64(const double *x, const double *grad_y, const double *params, int flags,
                                      int64_t outer, int64_t t, int64_t inner, double *grad_x, double *grad_params,
                                      void *workspace, size_t workspace_bytes, void *stream) {
   if (!params) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
   return log_lift_backward<double>(__func__, x, grad_y, 1.0, 0.0, flags, outer, t, inner, grad_x, grad_params,
-                                   workspace, workspace_bytes, stream, params);
+                                   workspace, workspace_bytes, stream, params, params + 1);
+}
+// the same from the logarithms of eps and tau, and the gradients of those
+int mellin_log_lift_forward_logs_f32(const float *x, const float *log_eps, const float *log_tau, int flags, int64_t outer, int64_t t,
+                                     int64_t inner, float *y, void *stream) {
+  if (((flags & MELLIN_PW_LOG) && !log_eps) || ((flags & MELLIN_PW_LIFT) && !log_tau)) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  return log_lift_forward<float>(__func__, x, 1.0, 0.0, flags, outer, t, inner, y, stream, log_eps, log_tau, true);
+}
+int mellin_log_lift_backward_logs_f32(const float *x, const float *grad_y, const float *log_eps, const float *log_tau, int flags,
+                                      int64_t outer, int64_t t, int64_t inner, float *grad_x, float *grad_params, void *workspace,
+                                      size_t workspace_bytes, void *stream) {
+  if (((flags & MELLIN_PW_LOG) && !log_eps) || ((flags & MELLIN_PW_LIFT) && !log_tau)) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  return log_lift_backward<float>(__func__, x, grad_y, 1.0, 0.0, flags, outer, t, inner, grad_x, grad_params, workspace,
+                                  workspace_bytes, stream, log_eps, log_tau, true);
+}
+int mellin_pack_windows_f32(const float *x, const int64_t *at, int64_t windows, int64_t frames, int64_t row, float *out, void *stream) {
+  if (windows < 0 || frames < 0 || row < 0 || windows >= (int64_t)1 << 31 || (frames > 0 && row >= ((int64_t)1 << 31) / frames))
+    return fail(MELLIN_ERR_ARGUMENT, "%s: sizes out of range (windows=%lld frames=%lld row=%lld)", __func__, (long long)windows,
+                (long long)frames, (long long)row);
+  if (windows * frames * row == 0) return MELLIN_OK;
+  if (!x || !at || !out) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  return check_hip(launch_pack_windows(x, at, windows, (int)(frames * row), (int)row, out, (hipStream_t)stream), __func__);
 }
 size_t mellin_log_lift_backward_workspace(int elem_bytes, int64_t outer, int64_t t, int64_t inner) {
   return log_lift_workspace_bytes(outer, t, inner, (size_t)elem_bytes);

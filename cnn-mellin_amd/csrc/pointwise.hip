@@ -27,13 +27,24 @@ constexpr int kPwThreads = 256;
 
 template <typename T> __device__ __forceinline__ T sign_of(T v) { return v > T(0) ? T(1) : (v < T(0) ? T(-1) : T(0)); }
 
+// eps and tau where they live on the device (null: the kernel's arguments); logs: their logarithms, as the modules' parameters
+// are (two launches of exp, and as many in the backward pass, on one value each)
+template <typename T> struct LiftParams {
+  const T *eps, *tau;
+  int logs;
+  __device__ __forceinline__ void read(T &e, T &t) const {
+    if (eps) e = logs ? exp(*eps) : *eps;
+    if (tau) t = logs ? exp(*tau) : *tau;
+  }
+};
+
 template <typename T, bool LOG, bool LIFT>
 __global__ __launch_bounds__(kPwThreads) void log_lift_forward_kernel(
-    const T *__restrict__ x, T eps, T tau, const T *__restrict__ params, i64 outer, i64 plane, i64 inner,
+    const T *__restrict__ x, T eps, T tau, LiftParams<T> params, i64 outer, i64 plane, i64 inner,
     i64 rows_per_block, T *__restrict__ y) {
   const i64 col = (i64)blockIdx.x * kPwThreads + threadIdx.x;      // t * inner + i
   if (col >= plane) return;
-  if (params) { eps = params[0]; tau = params[1]; }               // the values live on the device
+  params.read(eps, tau);
   T p = T(1);
   if (LIFT) p = pow((T)(col / inner + 1), tau);
   const i64 n0 = (i64)blockIdx.y * rows_per_block, n1 = min(outer, n0 + rows_per_block);
@@ -47,10 +58,10 @@ __global__ __launch_bounds__(kPwThreads) void log_lift_forward_kernel(
 // grad_x, and partial sums of d/d eps and d/d tau per block (two values per block)
 template <typename T, bool LOG, bool LIFT>
 __global__ __launch_bounds__(kPwThreads) void log_lift_backward_kernel(
-    const T *__restrict__ x, const T *__restrict__ gy, T eps, T tau, const T *__restrict__ params, i64 outer,
+    const T *__restrict__ x, const T *__restrict__ gy, T eps, T tau, LiftParams<T> params, i64 outer,
     i64 plane, i64 inner, i64 rows_per_block, T *__restrict__ gx, T *__restrict__ partial) {
   __shared__ T red[2][kPwThreads / 64];
-  if (params) { eps = params[0]; tau = params[1]; }
+  params.read(eps, tau);
   const i64 col = (i64)blockIdx.x * kPwThreads + threadIdx.x;
   T s_eps = T(0), s_tau = T(0);
   if (col < plane) {
@@ -67,11 +78,11 @@ __global__ __launch_bounds__(kPwThreads) void log_lift_backward_kernel(
       if (LOG) {
         const T a = eps + fabs(v);
         const T inv = gp / a;
-        gx[n * plane + col] = inv * sign_of(v);
+        if (gx) gx[n * plane + col] = inv * sign_of(v);
         s_eps += inv;
         if (LIFT) s_tau += gp * lnt * log(a);
       } else {
-        gx[n * plane + col] = gp;
+        if (gx) gx[n * plane + col] = gp;
         s_tau += gp * lnt * v;
       }
     }
@@ -98,7 +109,7 @@ __global__ __launch_bounds__(kPwThreads) void log_lift_backward_kernel(
 // lane l adds partials l, l + 64, ..., then a fixed shuffle tree)
 template <typename T>
 __global__ __launch_bounds__(64) void log_lift_reduce_kernel(const T *__restrict__ partial, i64 blocks,
-                                                             T *__restrict__ grad_params) {
+                                                             T *__restrict__ grad_params, LiftParams<T> params) {
   T a = T(0), b = T(0);
   for (i64 i = threadIdx.x; i < blocks; i += 64) { a += partial[2 * i]; b += partial[2 * i + 1]; }
 #pragma unroll
@@ -106,7 +117,16 @@ __global__ __launch_bounds__(64) void log_lift_reduce_kernel(const T *__restrict
     a += __shfl_down(a, o);
     b += __shfl_down(b, o);
   }
-  if (threadIdx.x == 0) { grad_params[0] = a; grad_params[1] = b; }
+  if (threadIdx.x == 0) {
+    if (params.logs) {                                     // d/d log v = v d/d v
+      T eps = T(0), tau = T(0);
+      params.read(eps, tau);
+      a *= eps;
+      b *= tau;
+    }
+    grad_params[0] = a;
+    grad_params[1] = b;
+  }
 }
 
 // Blocks along the outer axis: enough workgroups to fill the chip several times
@@ -132,11 +152,12 @@ size_t log_lift_workspace_bytes(i64 outer, i64 t, i64 inner, size_t elem) {
 
 template <typename T>
 hipError_t launch_log_lift_forward(const T *x, T eps, T tau, bool with_log, bool with_lift, i64 outer, i64 t,
-                                   i64 inner, T *y, hipStream_t stream, const T *params) {
+                                   i64 inner, T *y, hipStream_t stream, const T *eps_at, const T *tau_at, bool logs) {
   if (outer <= 0 || t <= 0 || inner <= 0) return hipSuccess;
   dim3 grid;
   i64 rpb;
   shape_grid(outer, t * inner, grid, rpb);
+  const LiftParams<T> params = {eps_at, tau_at, logs};
 #define MELLIN_PW_FWD(L_, F_)                                                                    \
   hipLaunchKernelGGL((log_lift_forward_kernel<T, L_, F_>), grid, dim3(kPwThreads), 0, stream, x, \
                      eps, tau, params, outer, t * inner, inner, rpb, y)
@@ -150,9 +171,10 @@ hipError_t launch_log_lift_forward(const T *x, T eps, T tau, bool with_log, bool
 template <typename T>
 hipError_t launch_log_lift_backward(const T *x, const T *gy, T eps, T tau, bool with_log, bool with_lift,
                                     i64 outer, i64 t, i64 inner, T *gx, T *grad_params, T *workspace,
-                                    hipStream_t stream, const T *params) {
+                                    hipStream_t stream, const T *eps_at, const T *tau_at, bool logs) {
+  const LiftParams<T> params = {eps_at, tau_at, logs};
   if (outer <= 0 || t <= 0 || inner <= 0) {
-    hipLaunchKernelGGL((log_lift_reduce_kernel<T>), dim3(1), dim3(64), 0, stream, workspace, (i64)0, grad_params);
+    hipLaunchKernelGGL((log_lift_reduce_kernel<T>), dim3(1), dim3(64), 0, stream, workspace, (i64)0, grad_params, params);
     return hipGetLastError();
   }
   dim3 grid;
@@ -168,7 +190,28 @@ hipError_t launch_log_lift_backward(const T *x, const T *gy, T eps, T tau, bool 
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((log_lift_reduce_kernel<T>), dim3(1), dim3(64), 0, stream, workspace,
-                     (i64)grid.x * grid.y, grad_params);
+                     (i64)grid.x * grid.y, grad_params, params);
+  return hipGetLastError();
+}
+
+// ---- windows of utterances --------------------------------------------------------------
+// out[k, :] (run values): frames `first` .. `first + frames - 1` of x, which lie side by side, and zeros behind the
+// utterance batch's last frame; at[k] = first | frames << 32.  One pass over what the windows hold (bound by its launch at
+// windows of ten frames of 41 bins: 4 us for 1177), where padding, unfolding and packing took nine copies.
+namespace {
+__global__ __launch_bounds__(kPwThreads) void pack_windows_kernel(const unsigned *__restrict__ x, const i64 *__restrict__ at, int run,
+                                                                  int row, unsigned *__restrict__ out) {
+  const i64 k = blockIdx.x, a = at[k];
+  const int live = (int)(a >> 32) * row;
+  const unsigned *src = x + (i64)(unsigned)a * row;
+  for (int e = threadIdx.x; e < run; e += kPwThreads) out[k * run + e] = e < live ? src[e] : 0u;
+}
+}  // namespace
+
+hipError_t launch_pack_windows(const void *x, const i64 *at, i64 windows, int run, int row, void *out, hipStream_t stream) {
+  if (windows <= 0 || run <= 0) return hipSuccess;
+  hipLaunchKernelGGL(pack_windows_kernel, dim3((unsigned)windows), dim3(kPwThreads), 0, stream, (const unsigned *)x, at, run, row,
+                     (unsigned *)out);
   return hipGetLastError();
 }
 
@@ -436,14 +479,13 @@ hipError_t launch_cast_pair(bool to_half, const void *a, void *to_a, i64 na, con
   return hipGetLastError();
 }
 
-template hipError_t launch_log_lift_forward<float>(const float *, float, float, bool, bool, i64, i64, i64,
-                                                   float *, hipStream_t, const float *);
-template hipError_t launch_log_lift_forward<double>(const double *, double, double, bool, bool, i64, i64, i64,
-                                                    double *, hipStream_t, const double *);
-template hipError_t launch_log_lift_backward<float>(const float *, const float *, float, float, bool, bool, i64,
-                                                    i64, i64, float *, float *, float *, hipStream_t, const float *);
-template hipError_t launch_log_lift_backward<double>(const double *, const double *, double, double, bool, bool,
-                                                     i64, i64, i64, double *, double *, double *, hipStream_t,
-                                                     const double *);
+template hipError_t launch_log_lift_forward<float>(const float *, float, float, bool, bool, i64, i64, i64, float *, hipStream_t,
+                                                   const float *, const float *, bool);
+template hipError_t launch_log_lift_forward<double>(const double *, double, double, bool, bool, i64, i64, i64, double *, hipStream_t,
+                                                    const double *, const double *, bool);
+template hipError_t launch_log_lift_backward<float>(const float *, const float *, float, float, bool, bool, i64, i64, i64, float *,
+                                                    float *, float *, hipStream_t, const float *, const float *, bool);
+template hipError_t launch_log_lift_backward<double>(const double *, const double *, double, double, bool, bool, i64, i64, i64, double *,
+                                                     double *, double *, hipStream_t, const double *, const double *, bool);
 
 }  // namespace mellin

@@ -455,7 +455,157 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
+// The gradients of LogCompressionLift.
+struct LogLiftBackward : public torch::autograd::Node {
+  torch::autograd::SavedVariable input_, log_eps_, log_tau_;
+  int64_t outer = 0, t = 0, inner = 0;
+
+  std::string name() const override { return "LogLiftBackward"; }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    input_.reset_data();
+    log_eps_.reset_data();
+    log_tau_.reset_data();
+  }
+
+  torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+    at::AutoGradMode no_grad(false);
+    Tensor input, log_eps, log_tau;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      input = input_.unpack();
+      log_eps = log_eps_.unpack();
+      log_tau = log_tau_.unpack();
+    }
+    if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    const Tensor grad = grads[0].contiguous();
+    const c10::OptionalDeviceGuard guard(input.device());
+    Tensor grad_input, params = at::empty({2}, input.options());
+    if (task_should_compute_output(0)) grad_input = at::empty_like(input, at::MemoryFormat::Contiguous);
+    const size_t need = mellin_log_lift_backward_workspace(4, outer, t, inner);
+    Tensor ws = scratch(input, need);
+    check(mellin_log_lift_backward_logs_f32((const float *)pointer(input), (const float *)pointer(grad), (const float *)pointer(log_eps),
+                                            (const float *)pointer(log_tau), MELLIN_PW_LOG | MELLIN_PW_LIFT, outer, t, inner,
+                                            grad_input.defined() ? (float *)grad_input.data_ptr() : nullptr, (float *)params.data_ptr(),
+                                            ws.defined() ? ws.data_ptr() : nullptr, need, launch_stream(input)));
+    return {grad_input, task_should_compute_output(1) ? params.select(0, 0).view(log_eps.sizes()) : Tensor(),
+            task_should_compute_output(2) ? params.select(0, 1).view(log_tau.sizes()) : Tensor()};
+  }
+};
+
+PyObject *log_lift(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  if (n_args != 4 || followed()) Py_RETURN_NONE;
+  for (int i = 0; i < 3; ++i)
+    if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
+  const Tensor &input0 = THPVariable_Unpack(args[0]), &log_eps = THPVariable_Unpack(args[1]), &log_tau = THPVariable_Unpack(args[2]);
+  const int64_t dim = PyLong_AsLongLong(args[3]);
+  if (!plain(input0) || input0.scalar_type() != at::kFloat || dim < 0 || dim >= input0.dim() || input0.numel() == 0) Py_RETURN_NONE;
+  for (const Tensor *p : {&log_eps, &log_tau})
+    if (!plain(*p) || p->scalar_type() != at::kFloat || p->numel() != 1 || p->device() != input0.device()) Py_RETURN_NONE;
+  Tensor out;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const c10::OptionalDeviceGuard guard(input0.device());
+    const bool differentiable = at::GradMode::is_enabled() && (input0.requires_grad() || log_eps.requires_grad() || log_tau.requires_grad());
+    int64_t outer = 1, inner = 1;
+    for (int64_t i = 0; i < input0.dim(); ++i) (i < dim ? outer : inner) *= i == dim ? 1 : input0.size(i);
+    const int64_t t = input0.size(dim);
+    Tensor input;
+    {
+      at::AutoGradMode no_grad(false);
+      input = input0.contiguous();
+      out = at::empty_like(input, at::MemoryFormat::Contiguous);
+      check(mellin_log_lift_forward_logs_f32((const float *)pointer(input), (const float *)pointer(log_eps), (const float *)pointer(log_tau),
+                                             MELLIN_PW_LOG | MELLIN_PW_LIFT, outer, t, inner, (float *)out.data_ptr(), launch_stream(input)));
+    }
+    if (differentiable) {
+      auto node = std::shared_ptr<LogLiftBackward>(new LogLiftBackward(), torch::autograd::deleteNode);
+      node->set_next_edges(torch::autograd::collect_next_edges(input0, log_eps, log_tau));
+      node->input_ = torch::autograd::SavedVariable(input, false);
+      node->log_eps_ = torch::autograd::SavedVariable(log_eps, false);
+      node->log_tau_ = torch::autograd::SavedVariable(log_tau, false);
+      node->outer = outer;
+      node->t = t;
+      node->inner = inner;
+      torch::autograd::set_history(out, node);
+    }
+  }
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// Windows of utterances in the order of torch.nn.utils.rnn.pack_padded_sequence (longest first, then time step by time step):
+// (data, batch_sizes, sorted_indices, unsorted_indices).  The order is worked out here, as the reference does on the CPU, and
+// goes to the GPU from pinned memory, so that nothing waits for what the GPU has been given before (padding, unfolding and
+// packing by PyTorch took 58 to 92 us of host time and a synchronous copy).
+PyObject *pack_windows(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  if (n_args != 4 || followed() || !THPVariable_Check(args[0]) || !THPVariable_Check(args[1]) || !PyLong_CheckExact(args[2]) ||
+      !PyLong_CheckExact(args[3]))
+    Py_RETURN_NONE;
+  const Tensor &x0 = THPVariable_Unpack(args[0]), &lens0 = THPVariable_Unpack(args[1]);
+  const int64_t size = PyLong_AsLongLong(args[2]), stride = PyLong_AsLongLong(args[3]);
+  if (PyErr_Occurred()) { PyErr_Clear(); Py_RETURN_NONE; }
+  if (!plain(x0) || x0.scalar_type() != at::kFloat || x0.dim() != 3 || (x0.requires_grad() && at::GradMode::is_enabled())) Py_RETURN_NONE;
+  const int64_t n = x0.size(0), frames = x0.size(1), row = x0.size(2), lim = (int64_t)1 << 31;
+  if (n < 1 || frames < 1 || row < 1 || size < 1 || stride < 1 || size >= lim || n * frames >= lim || size * row >= lim) Py_RETURN_NONE;
+  if (!lens0.device().is_cpu() || lens0.layout() != at::kStrided || lens0.scalar_type() != at::kLong || lens0.dim() != 1 ||
+      lens0.size(0) != n || lens0.requires_grad())
+    Py_RETURN_NONE;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)launch_stream(x0), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) Py_RETURN_NONE;
+  Tensor counts, order;
+  int64_t windows = 0;
+  {
+    at::AutoGradMode no_grad(false);
+    counts = at::empty({n}, lens0.options());
+    const Tensor lens = lens0.contiguous();
+    const int64_t *l = lens.const_data_ptr<int64_t>();
+    int64_t *c = counts.mutable_data_ptr<int64_t>();
+    for (int64_t i = 0; i < n; ++i) {
+      if (l[i] < 1 || l[i] > frames) Py_RETURN_NONE;         // (errors, with PyTorch's messages)
+      c[i] = (l[i] - 1) / stride + 1;
+      windows += c[i];
+    }
+    std::tie(counts, order) = at::sort(counts, -1, true);
+  }
+  if (windows >= lim) Py_RETURN_NONE;
+  const int64_t *c = counts.const_data_ptr<int64_t>(), *o = order.const_data_ptr<int64_t>();
+  at::AutoGradMode no_grad(false);
+  const c10::OptionalDeviceGuard guard(x0.device());
+  Tensor batch_sizes = at::empty({c[0]}, lens0.options()), table = at::empty({2 * n + windows}, lens0.options().pinned_memory(true));
+  int64_t *b = batch_sizes.mutable_data_ptr<int64_t>(), *p = table.mutable_data_ptr<int64_t>(), *entry = p + 2 * n;
+  for (int64_t i = 0; i < n; ++i) {
+    p[i] = o[i];
+    p[n + o[i]] = i;
+  }
+  int64_t live = n;
+  for (int64_t step = 0; step < c[0]; ++step) {
+    while (c[live - 1] <= step) --live;
+    b[step] = live;
+    const int64_t first = step * stride, whole = std::min(size, frames - first);
+    for (int64_t i = 0; i < live; ++i) *entry++ = (o[i] * frames + first) | whole << 32;
+  }
+  const Tensor x = x0.contiguous(), there = table.to(x0.device(), /*non_blocking=*/true);
+  Tensor data = at::empty({windows, size, row}, x.options());
+  check(mellin_pack_windows_f32((const float *)pointer(x), there.const_data_ptr<int64_t>() + 2 * n, windows, size, row, (float *)data.data_ptr(),
+                                launch_stream(x)));
+  PyObject *result = PyTuple_New(4);
+  if (!result) return nullptr;
+  PyTuple_SET_ITEM(result, 0, THPVariable_Wrap(std::move(data)));
+  PyTuple_SET_ITEM(result, 1, THPVariable_Wrap(std::move(batch_sizes)));
+  PyTuple_SET_ITEM(result, 2, THPVariable_Wrap(there.narrow(0, 0, n)));
+  PyTuple_SET_ITEM(result, 3, THPVariable_Wrap(there.narrow(0, n, n)));
+  return result;
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"log_lift", (PyCFunction)(void *)log_lift, METH_FASTCALL,
+     "log_lift(input, log_eps, log_tau, dim): log compression and lift, or None if not handled"},
+    {"pack_windows", (PyCFunction)(void *)pack_windows, METH_FASTCALL,
+     "pack_windows(x, lens, size, stride): (data, batch_sizes, sorted_indices, unsorted_indices), or None if not handled"},
     {"stack", (PyCFunction)(void *)stack, METH_FASTCALL,
      "stack(kind, input, [(weight, bias, s, d, p, r, pool), ...]): the last layer's output behind its ReLU, or None if not handled"},
     {"corr", (PyCFunction)(void *)corr, METH_FASTCALL,

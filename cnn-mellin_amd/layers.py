@@ -155,7 +155,9 @@ class LogCompressionLift(torch.nn.Module):
         torch.nn.init.normal_(self.log_tau)
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
-        return log_compression_lift(input, self.log_eps.exp(), self.log_tau.exp(), self.dim)
+        # one launch, which takes the exponentials itself (None: tensors that are not for it)
+        y = _hip.native.log_lift(input, self.log_eps, self.log_tau, _check_dim(input, self.dim))
+        return y if y is not None else log_compression_lift(input, self.log_eps.exp(), self.log_tau.exp(), self.dim)
 
 
 def scaled_gaussian_noise(x: torch.Tensor, eps: float, dim: int, training: bool = True,

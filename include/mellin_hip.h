@@ -363,6 +363,24 @@ int mellin_log_lift_backward_dev_f64(const double *x, const double *grad_y,
                                      double *grad_params, void *workspace,
                                      size_t workspace_bytes, void *stream);
 
+/* The same with the LOGARITHMS of eps and tau in device memory, as the reference's modules hold them (a null pointer for the one
+ * that flags do not use): eps = exp(*log_eps), tau = exp(*log_tau), and backward writes the gradients of the logarithms.  There
+ * grad_x may be null: only the gradients of the parameters are made. */
+int mellin_log_lift_forward_logs_f32(const float *x, const float *log_eps, const float *log_tau,
+                                     int flags, int64_t outer, int64_t t, int64_t inner,
+                                     float *y, void *stream);
+int mellin_log_lift_backward_logs_f32(const float *x, const float *grad_y,
+                                      const float *log_eps, const float *log_tau, int flags,
+                                      int64_t outer, int64_t t, int64_t inner, float *grad_x,
+                                      float *grad_params, void *workspace,
+                                      size_t workspace_bytes, void *stream);
+
+/* Windows of a feature batch x, rows of `row` values: out (windows, frames, row), window k being the at[k] >> 32 rows from row
+ * (uint32_t)at[k] of x on, and zeros behind those (models.py:395-411: windows that reach past the batch's last frame are
+ * padded).  `at`, in device memory, comes from the caller and is not checked. */
+int mellin_pack_windows_f32(const float *x, const int64_t *at, int64_t windows, int64_t frames,
+                            int64_t row, float *out, void *stream);
+
 /* Bias gradient of a layer, grad_bias[c] = sum over images and positions of
  * g[n, c, :] for grad_out (batch, channels, plane) -- the reference leaves this to
  * grad_out.sum(...) (ext/torch.cpp:231,300) -- in one pass together with the backward of

@@ -529,8 +529,10 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         unit_at[t] = (wn * NT + t) * 32 + l32 < tg.count ? lane_n[t] * (int)image_bytes + lane_q[t] * UB + half * 8 : (int)0x80000000u;
-      auto masked = [&](float4 v, int group, int at) {
-        const uintx2 x = __builtin_amdgcn_raw_buffer_load_b64(mask_rsrc, at < 0 ? at : at + (int)(group * unit_row), 0, 0);   // (none: zeros)
+      auto load_mask = [&](int group, int at) -> uintx2 {
+        return __builtin_amdgcn_raw_buffer_load_b64(mask_rsrc, at < 0 ? at : at + (int)(group * unit_row), 0, 0);   // (none: zeros)
+      };
+      auto masked = [&](float4 v, uintx2 x) {
         auto keep = [](float f, unsigned sixteen) { return (short)sixteen > 0 ? f : 0.f; };
         return make_float4(keep(v.x, x[0]), keep(v.y, x[0] >> 16), keep(v.z, x[1]), keep(v.w, x[1] >> 16));
       };
@@ -590,7 +592,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
             const int group = m0 / 8 + k * 4 + r4;
             if constexpr (GRAD) {
               if (whole) {
-                v = masked(v, group, unit);
+                v = masked(v, load_mask(group, unit));
                 s[4 * r4] = v.x; s[4 * r4 + 1] = v.y; s[4 * r4 + 2] = v.z; s[4 * r4 + 3] = v.w;
               }
             }
@@ -611,6 +613,18 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       } else {
         if constexpr (GRAD) {
           if (whole) {
+            // The masks of kAhead groups of channels are requested before the first is used, in registers that are free
+            // here (fp32: of `low`; half: of the signal's operands); read where they were used, each of the tile's 16 or
+            // 32 waits took a trip to memory: 28000 of 90000 cycles of a tile of 64 x 512 half values.
+            constexpr int kGroups = MT * 4, kAhead = F16 ? (16 / NT < kGroups ? 16 / NT : kGroups) : kGroups;
+            uintx2 mask_of[kAhead][NT];
+            auto request = [&](int i) {
+#pragma unroll
+              for (int t = 0; t < NT; ++t) mask_of[i % kAhead][t] = load_mask(m0 / 8 + i, unit_at[t]);
+            };
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) request(i);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int k = 0; k < MT; ++k) {
               float s[16];
@@ -620,11 +634,12 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                   const float4 v = masked(make_float4(acc[k][t][4 * g4], acc[k][t][4 * g4 + 1], acc[k][t][4 * g4 + 2], acc[k][t][4 * g4 + 3]),
-                                          m0 / 8 + k * 4 + g4, unit_at[t]);
+                                          mask_of[(k * 4 + g4) % kAhead][t]);
                   acc[k][t][4 * g4] = v.x; acc[k][t][4 * g4 + 1] = v.y; acc[k][t][4 * g4 + 2] = v.z; acc[k][t][4 * g4 + 3] = v.w;
                   sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
                 }
                 s[4 * g4] = sum.x; s[4 * g4 + 1] = sum.y; s[4 * g4 + 2] = sum.z; s[4 * g4 + 3] = sum.w;
+                if (k * 4 + g4 + kAhead < kGroups) request(k * 4 + g4 + kAhead);
               }
               put_sums(s, k, first_slot + wn);
             }

@@ -208,7 +208,8 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   // The launch of a tile shape, in cycles.  Workgroups take tiles in turn, two to a CU (512 at a time).  What does not fill
   // a last turn -- for few tiles: all of them -- can be cut into slices of the contracted channels, which another kernel
   // adds up.  Measured on this chip, and rounded:
-  //   a step's matrix instructions at 65-80 % of their rate (larger tiles: the higher), shared by a CU's workgroups;
+  //   a step's matrix instructions at 55-80 % of their rate (larger tiles: the higher; 128 channels x 128 positions of two by
+  //   two wavefronts measure that of 64 x 512), shared by a CU's workgroups;
   //   a stage at least 4000 (the latency of its loads);
   //   per tile 5000 for its tables (9000 where wavefronts share it in fp32: nothing runs under them) and its output at 9
   //   bytes a cycle; 9000 for a launch's start, as much for the kernel that adds the slices, and 2400 bytes a cycle for
@@ -224,7 +225,7 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
     double filter_rows, subsets;
     tile_rows(P, filter_rows, subsets);
     const double rows = filter_rows / subsets;
-    const double rate = pl.mt * pl.nt >= 8 ? 0.8 : pl.mt * pl.nt * pl.wm >= 8 ? 0.72 : pl.mt * pl.nt >= 4 ? 0.65 : 0.55;
+    const double rate = pl.mt * pl.nt * pl.wm >= 8 ? 0.8 : pl.mt * pl.nt >= 4 ? 0.65 : 0.55;
     const double steps = std::ceil(rows * pl.nfy * pl.G / (2 * pl.wk)) * pl.mt * pl.nt * (f16 ? 1 : 6) * 32 / rate;
     const double output = (double)M_T * P * (f16 ? 2 : 4) / 9;
     const double tile = pl.wk > 1 && !f16 ? 9000 : 5000;

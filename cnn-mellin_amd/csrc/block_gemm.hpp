@@ -82,7 +82,7 @@ hipError_t launch_grad_blocked(const BlockPlan &pl, const BlockGemmArgs &a, hipS
 
 // The rows of one filter row in the weight gradient: output rows ox0 + i step and input rows gx0 + i gstep for
 // i < count; its share of the launch: `slices` workgroups from slice0 on.
-struct BlockWgradRow { int ox0, step, gx0, gstep, count, slice0, slices; };
+struct BlockWgradRow { int ox0, step, gx0, gstep, count, slice0, slices; unsigned mg_count; };
 
 struct BlockWgradPlan {
   int f16;
@@ -94,6 +94,7 @@ struct BlockWgradPlan {
   int m_blocks, c_blocks, mgt, cgt;
   int VP, zero_unit;               // units of a channel group's input in a stage, the first that is always zero
   int slices;
+  unsigned mg_noy;                 // reciprocals, as udiv() takes them
   BlockWgradRow row[kBlockFilterRows];
   size_t lds_bytes, ws_bytes;
 };

@@ -23,9 +23,11 @@
 // Every workgroup writes its sums as one partial block; block_finish.hip adds a weight's partial
 // sums in slice order (bit-reproducible).
 //
-// Measured against wgrad_pos.hip, 128 -> 256 channels, 3 x 3 taps, 32 x 256 x 41 positions: fp32, linear rows 1171 -> 1056 us;
-// half, Mellin rows 356 -> 146 us.  64 -> 64 channels, 4 x 4 taps, 32 x 780 x 20, fp32: Mellin rows 477 -> 275 us, linear
-// rows 424 -> 440.
+// Measured against wgrad_pos.hip, 128 -> 256 channels, 3 x 3 taps, 32 x 256 x 41 positions: fp32, linear rows 1171 -> 1000 us;
+// half, Mellin rows 356 -> 112 us.  64 -> 64 channels, 4 x 4 taps, 32 x 780 x 20, fp32: Mellin rows 477 -> 200 us.
+// Bound by what a stage costs beside its products (tables, loads' issue, the first operands after the barrier): a wavefront
+// has 2 x 24 matrix instructions a stage in fp32 (1536 cycles), 4 x 8 in half (1024).  256 -> 256 channels, 4 x 4 taps,
+// 32 x 780 x 5, fp32: 970 us with tables from divisions, 860 now (46 % of the cycles multiply), 660 without tables and loads.
 #include <algorithm>
 #include <type_traits>
 
@@ -65,16 +67,32 @@ __global__ __launch_bounds__(NW * 64, 2) void block_wgrad_kernel(BlockWgradPlan 
   const int WM = pl.wm;
   const int wm = wave % WM, wn = wave / WM;
   // this workgroup's filter row and slice, output-channel and input-channel block
-  int fx = 0;
-  while (fx + 1 < pl.nfx && (int)blockIdx.x >= pl.row[fx + 1].slice0) ++fx;
-  const int slice = (int)blockIdx.x - pl.row[fx].slice0, slices = pl.row[fx].slices;
-  const int mb = blockIdx.y / pl.c_blocks, cb = blockIdx.y - mb * pl.c_blocks;
+  const int blocks = pl.m_blocks * pl.c_blocks;
+  int fx, slice, block;
+  {
+    // XCD k (workgroups k, k + 8, ...) takes an eighth of the items without a gap: the blocks of a slice read the same rows
+    // through one L2 (256 -> 256 channels, 4 x 4 taps, 32 x 780 x 5, fp32: misses 4.0 GB -> 1.3 GB)
+    const int items = pl.slices * blocks, xcd = blockIdx.x & 7, item = xcd * (items >> 3) + min(xcd, items & 7) + (blockIdx.x >> 3);
+    int at = item / blocks, left = pl.slices;
+    block = item - at * blocks;
+    // the filter rows' slices in turn, each row's spread evenly over those of the rows behind it
+    for (fx = 0; fx + 1 < pl.nfx; ++fx) {
+      const int n = pl.row[fx].slices, before = at * n / left;
+      if ((at + 1) * n >= (before + 1) * left) { at = before; break; }
+      at -= before;
+      left -= n;
+    }
+    slice = at;
+  }
+  const int slices = pl.row[fx].slices;
+  const int mb = block / pl.c_blocks, cb = block - mb * pl.c_blocks;
   const int mg0 = mb * pl.mgt, cg0 = cb * pl.cgt;
   const int mgs = min(pl.mgt, pl.MG - mg0), cgs = min(pl.cgt, pl.CG - cg0);
   const int ox_first = pl.row[fx].ox0, ox_step = pl.row[fx].step, gx0 = pl.row[fx].gx0, gx_step = pl.row[fx].gstep;
   const int count = pl.row[fx].count, noy = pl.noy;
-  const i64 total = (i64)pl.batch * count * noy;       // positions (fits 31 bits)
-  const int units = (int)((total + KS - 1) / KS);
+  const int total = pl.batch * count * noy;            // positions (blocked tensors of < 2^32 bytes: fewer than 2^28)
+  const int units = (total + KS - 1) / KS;
+  const unsigned mg_noy = pl.mg_noy, mg_count = pl.row[fx].mg_count;
   const int u_lo = (int)((i64)units * slice / slices), u_hi = (int)((i64)units * (slice + 1) / slices);
   const int VP = pl.VP, a_bytes = pl.mgt * KSP * UB, buf_bytes = a_bytes + pl.cgt * VP * UB;
   const unsigned lds0 = lds_address((const float *)bw_lds);
@@ -83,72 +101,108 @@ __global__ __launch_bounds__(NW * 64, 2) void block_wgrad_kernel(BlockWgradPlan 
   const i64 a_plane = (i64)(pl.q_out + 1) * UB, g_plane = (i64)(pl.plane + 1) * UB;
   const char *A0 = A + (i64)mg0 * a_plane, *G0 = G + (i64)cg0 * g_plane;
 
-  // sources of stage u: one entry per thread (KS + VP <= threads)
-  auto build_tables = [&](int u) {
-    int *t = tabs + (u % 3) * tab_words;
-    const i64 first = (i64)u * KS;
-    const int row_lin = (int)(first / noy), oy0 = (int)(first - (i64)row_lin * noy);
-    const int valid = (int)min((i64)KS, total - first);
-    const int n0 = row_lin / count, i0 = row_lin - n0 * count;
-    const FastDiv by_noy(noy), by_count(count);
-    // virtual units: the first row's piece from column oy0 on, then whole rows
-    const int full = pl.ay * (noy - 1) + pl.by_span + 1, head = full - pl.ay * oy0;
+  // The sources of a stage, one entry per thread (KS + VP <= threads): a position's units of grad_out and of the staged
+  // input, or one of the staged units' source.  Threads keep their place (image, row, column) from stage to stage and add
+  // KS positions to it with two carries: worked out from the stage's number, with divisions and products, the tables took
+  // a fifth of the fp32 kernels' time and up to two fifths of half kernels'.
+  const int full = pl.ay * (noy - 1) + pl.by_span + 1;                 // virtual units of a row
+  const int wrap = full - pl.ay * noy;                                 // what a row's end adds to those of its positions
+  const int rows_on = udiv(KS, noy, mg_noy), k_col = KS - rows_on * noy;
+  const int k_image = udiv(rows_on, count, mg_count), k_row = rows_on - k_image * count;
+  const unsigned a_image = (unsigned)pl.MG * (unsigned)(pl.q_out + 1) * UB, a_row = (unsigned)(ox_step * noy * UB);
+  const unsigned g_image = (unsigned)pl.CG * (unsigned)(pl.plane + 1) * UB, g_row = (unsigned)(gx_step * pl.ngy * UB);
+  int first_col;                                       // of the stage whose table is next
+  int at_col, at_row, at_n;                            // (position: at_n its LDS address)
+  unsigned at_source;                                  // input: of the row's first unit
+  {
+    const int first = u_lo * KS, row0 = udiv(first, noy, mg_noy);
+    first_col = first - row0 * noy;
+    int row = row0;
     if (tid < KS) {
-      const bool live = tid < valid;
-      int r, oy, dn, i;
-      by_noy.divmod(oy0 + tid, r, oy);
-      by_count.divmod(i0 + r, dn, i);
-      const int q = (ox_first + i * ox_step) * noy + oy;
-      t[tid] = (int)(((unsigned)(n0 + dn) * (unsigned)pl.MG * (unsigned)(pl.q_out + 1) + (unsigned)(live ? q : pl.q_out)) * UB);
-      if (!live) t[tid] = (int)((unsigned)n0 * (unsigned)pl.MG * (unsigned)(pl.q_out + 1) + (unsigned)pl.q_out) * UB;
-      const int v = r == 0 ? pl.ay * (oy - oy0) : head + (r - 1) * full + pl.ay * oy;
-      t[KS + tid] = (live ? v : pl.zero_unit) * UB;
+      row = udiv(first + tid, noy, mg_noy);
+      at_col = first + tid - row * noy;
+    } else {
+      at_col = tid - KS + pl.ay * first_col;
+      const int r = at_col / full;
+      at_col -= r * full;
+      row += r;
+    }
+    const int n = udiv(row, count, mg_count);
+    at_row = row - n * count;
+    if (tid < KS) {
+      at_source = (unsigned)n * a_image + (unsigned)(ox_first * noy * UB) + (unsigned)at_row * a_row + (unsigned)(at_col * UB);
+      at_n = (pl.ay * (at_col - first_col) + (row - row0) * full) * UB;
+    } else {
+      at_source = (unsigned)n * g_image + (unsigned)(gx0 * pl.ngy * UB) + (unsigned)at_row * g_row;
+      at_n = tid - KS < pl.zero_unit ? n : 1 << 30;    // (an image that is not there: zeros)
+    }
+  }
+  auto build_tables = [&](int u) {                     // (called for u_lo, u_lo + 1, ...)
+    int *t = tabs + (u % 3) * tab_words;
+    const int next_col = first_col + k_col;
+    const bool first_wraps = next_col >= noy;
+    first_col = first_wraps ? next_col - noy : next_col;
+    if (tid < KS) {
+      const bool live = u * KS + tid < total;
+      t[tid] = (int)(live ? at_source : (unsigned)(pl.q_out * UB));
+      t[KS + tid] = live ? at_n : pl.zero_unit * UB;
+      at_col += k_col;
+      at_row += k_row;
+      at_source += k_image * a_image + k_row * a_row + k_col * UB;
+      at_n -= first_wraps ? wrap * UB : 0;
+      if (at_col >= noy) { at_col -= noy; ++at_row; at_source += a_row - noy * UB; at_n += wrap * UB; }
+      if (at_row >= count) { at_row -= count; at_source += a_image - count * a_row; }
     } else if (tid < KS + VP) {
-      const int v = tid - KS;
-      int r = 0, col = v + pl.ay * oy0;                // row piece and column (of the whole virtual row)
-      if (v >= head) {
-        const FastDiv by_full(full);
-        by_full.divmod(v - head, r, col);
-        ++r;
+      const int vy = pl.cy + at_col;
+      int gy = vy;
+      if (pl.uy != 1) {
+        gy = vy / pl.uy;
+        if (gy * pl.uy != vy) gy = -1;
       }
-      int dn, i;
-      by_count.divmod(i0 + r, dn, i);
-      const int vy = pl.cy + col;
-      int gy = -1;
-      if (vy >= 0) {
-        if (pl.uy == 1) gy = vy;
-        else { const int q = vy / pl.uy; if (q * pl.uy == vy) gy = q; }
-        if (gy >= pl.ngy) gy = -1;
-      }
-      const int n = n0 + dn;
-      const bool live = gy >= 0 && n < pl.batch && v < pl.zero_unit;
-      t[2 * KS + v] = (int)(((unsigned)(live ? n : 0) * (unsigned)pl.CG * (unsigned)(pl.plane + 1) +
-                             (unsigned)(live ? (gx0 + i * gx_step) * pl.ngy + gy : pl.plane)) * UB);
+      const bool live = vy >= 0 && (unsigned)gy < (unsigned)pl.ngy && at_n < pl.batch;
+      t[KS + tid] = (int)(live ? at_source + gy * UB : (unsigned)(pl.plane * UB));
+      at_col += pl.ay * k_col + (first_wraps ? wrap : 0);              // (0 <= what is added < full)
+      at_row += k_row;
+      at_n += k_image;
+      at_source += k_image * g_image + k_row * g_row;
+      if (at_col >= full) { at_col -= full; ++at_row; at_source += g_row; }
+      if (at_row >= count) { at_row -= count; ++at_n; at_source += g_image - count * g_row; }
     }
   };
   // the loads of stage u into buffer b: groups of channels dealt to the wavefronts
   auto issue = [&](int u, int b) {
     const int *t = tabs + (u % 3) * tab_words;
     const unsigned to = lds0 + (unsigned)(b * buf_bytes);
-#pragma unroll
-    for (int k = 0; k < (KS * PARTS + 63) / 64; ++k) {
-      const int slot = k * 64 + lane, unit = F16 ? slot : slot / 3, part = F16 ? 0 : slot - unit * 3;
-      if (slot < KS * PARTS) {
-        const unsigned src = (unsigned)t[unit] + part * 16;
-        const char *from = A0 + wave * a_plane;
-        for (int g = wave; g < mgs; g += NW, from += NW * a_plane)
-          load16_to_lds_at((const float *)from, src, to + (unsigned)(g * KSP * UB + k * 1024));
-      }
-    }
+    constexpr int kSlots = KS * PARTS, kA = (kSlots + 63) / 64, kG = 4;
     const int slots = VP * PARTS;
-    for (int k = 0; k * 64 < slots; ++k) {
-      const int slot = k * 64 + lane, unit = F16 ? slot : slot / 3, part = F16 ? 0 : slot - unit * 3;
-      if (slot < slots) {
-        const unsigned src = (unsigned)t[2 * KS + unit] + part * 16;
-        const char *from = G0 + wave * g_plane;
-        for (int g = wave; g < cgs; g += NW, from += NW * g_plane)
-          load16_to_lds_at((const float *)from, src, to + (unsigned)(a_bytes + g * VP * UB + k * 1024));
-      }
+    auto unit_of = [&](int slot) { return F16 ? slot : slot / 3; };
+    auto part_of = [&](int slot) { return F16 ? 0 : (slot - slot / 3 * 3) * 16; };
+    // every source that is needed (lanes without a slot: a slot that is there), then the loads: one wait for the tables
+    unsigned a_src[kA], g_src[kG];
+#pragma unroll
+    for (int k = 0; k < kA; ++k) { const int slot = min(k * 64 + lane, kSlots - 1); a_src[k] = (unsigned)t[unit_of(slot)] + part_of(slot); }
+#pragma unroll
+    for (int k = 0; k < kG; ++k)
+      if (k * 64 < slots) { const int slot = min(k * 64 + lane, slots - 1); g_src[k] = (unsigned)t[2 * KS + unit_of(slot)] + part_of(slot); }
+    auto load_a = [&](int k) {
+      const char *from = A0 + wave * a_plane;
+      for (int g = wave; g < mgs; g += NW, from += NW * a_plane)
+        load16_to_lds_at((const float *)from, a_src[k], to + (unsigned)(g * KSP * UB + k * 1024));
+    };
+    auto load_g = [&](int k, unsigned src) {
+      const char *from = G0 + wave * g_plane;
+      for (int g = wave; g < cgs; g += NW, from += NW * g_plane)
+        load16_to_lds_at((const float *)from, src, to + (unsigned)(a_bytes + g * VP * UB + k * 1024));
+    };
+#pragma unroll
+    for (int k = 0; k < kA; ++k)
+      if (k * 64 + lane < kSlots) load_a(k);
+#pragma unroll
+    for (int k = 0; k < kG; ++k)
+      if (k * 64 + lane < slots) load_g(k, g_src[k]);
+    for (int k = kG; k * 64 < slots; ++k) {
+      const int slot = k * 64 + lane;
+      if (slot < slots) load_g(k, (unsigned)t[2 * KS + unit_of(slot)] + part_of(slot));
     }
   };
 
@@ -192,7 +246,6 @@ __global__ __launch_bounds__(NW * 64, 2) void block_wgrad_kernel(BlockWgradPlan 
     const int b = (u - u_lo) & 1;
     // every wavefront's loads for this stage have landed, and every wavefront is done with the other buffer
     wait_and_barrier<0>();
-    if (u + 1 < u_hi) issue(u + 1, b ^ 1);
     const int *vt = tabs + (u % 3) * tab_words + KS + k_pos;
     const unsigned base = lds0 + (unsigned)(b * buf_bytes);
     struct Ops { uintx4 a[MT][PARTS], b[NT][PARTS]; };
@@ -223,7 +276,9 @@ __global__ __launch_bounds__(NW * 64, 2) void block_wgrad_kernel(BlockWgradPlan 
       else block_multiply<MT, NT, PARTS>(acc, o.a, o.b);
     };
     Ops o0, o1;
-    fetch(0, o0);
+    fetch(0, o0);                                      // (on its way while the next stage's loads are issued)
+    __builtin_amdgcn_sched_barrier(0);
+    if (u + 1 < u_hi) issue(u + 1, b ^ 1);
 #pragma unroll
     for (int s = 0; s < KS / 16; s += 2) {
       fetch(s + 1, o1);
@@ -246,7 +301,7 @@ __global__ __launch_bounds__(NW * 64, 2) void block_wgrad_kernel(BlockWgradPlan 
   // ---- the partial block: [channel of the block][column tile (input channels, filter column)][32]
   const int l32 = lane & 31, half = lane >> 5;
   const int cols = pl.ctb * pl.nfy * 32;
-  float *out = ws + ((i64)blockIdx.x * gridDim.y + blockIdx.y) * (i64)(WM * MT * 32) * cols;
+  float *out = ws + ((i64)(pl.row[fx].slice0 + slice) * blocks + block) * (i64)(WM * MT * 32) * cols;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int tile = wn * NT + t;
@@ -267,7 +322,7 @@ hipError_t launch_wgrad_instance(const BlockWgradPlan &pl, const void *a, const 
   static std::atomic<int> lds_allowed{0};
   hipError_t e = allow_large_lds((const void *)kern, pl.lds_bytes, lds_allowed);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)pl.slices, (unsigned)(pl.m_blocks * pl.c_blocks)), dim3(NW * 64), pl.lds_bytes, stream,
+  hipLaunchKernelGGL(kern, dim3((unsigned)(pl.slices * pl.m_blocks * pl.c_blocks)), dim3(NW * 64), pl.lds_bytes, stream,
                      pl, (const char *)a, (const char *)g, ws);
   return hipGetLastError();
 }
@@ -286,6 +341,7 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
   if (blocked_bytes(fwd.batch, fwd.c_in, plane, f16) >= ((size_t)1 << 32) || blocked_bytes(fwd.batch, fwd.c_out, Q, f16) >= ((size_t)1 << 32))
     return false;
   if (fwd.batch * Q >= (i64)1 << 31 || fwd.batch * X.nh >= (i64)1 << 21) return false;
+  auto magic = [](i64 d) { return d <= 1 ? 0xFFFFFFFFu : (unsigned)(0x100000000ull / (unsigned)d); };
   const int parts = f16 ? 1 : 3, UB = 16 * parts, KS = f16 ? 64 : 32;
   pl.f16 = f16;
   pl.batch = (int)fwd.batch; pl.M = (int)fwd.c_out; pl.C = (int)fwd.c_in;
@@ -297,6 +353,7 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
     if (std::max<i64>(lo, 0) <= std::min<i64>(hi, Y.nf - 1)) { fy_lo = std::max<i64>(lo, 0); fy_hi = std::min<i64>(hi, Y.nf - 1); }
   }
   pl.nfx = (int)X.nf; pl.nfy = (int)(fy_hi - fy_lo + 1); pl.f_pitch = (int)Y.nf; pl.f_off = (int)fy_lo;
+  pl.mg_noy = magic(pl.noy);
   pl.ay = (int)Y.s; pl.by = (int)Y.d; pl.cy = (int)-(Y.p - Y.d * fy_lo); pl.uy = (int)Y.u;
   const i64 span = (i64)pl.by * (pl.nfy - 1);
   if (span > 64) return false;
@@ -314,7 +371,7 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
     i64 first = -1;
     for (i64 o = 0; o < step && o <= hi; ++o)
       if (((num0 + numk * o) % den + den) % den == 0) { first = o; break; }
-    r = BlockWgradRow{0, 1, 0, 0, 0, 0, 0};
+    r = BlockWgradRow{0, 1, 0, 0, 0, 0, 0, 0};
     if (first < 0) continue;
     const i64 need_lo = off * den - num0, need_hi = (X.ng - 1 + off) * den - num0;   // numk ox in [need_lo, need_hi]
     lo = std::max<i64>(lo, -floor_div(-need_lo, numk));
@@ -324,6 +381,7 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
     r.ox0 = (int)first; r.step = (int)step; r.count = (int)((hi - first) / step + 1);
     r.gx0 = (int)((num0 + numk * first) / den - off);
     r.gstep = (int)(numk * step / den);
+    r.mg_count = magic(r.count);
     work += (i64)r.count * pl.noy * pl.batch;
   }
   if (work == 0) return false;

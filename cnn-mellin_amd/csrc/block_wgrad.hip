@@ -56,8 +56,11 @@ constexpr int kLowTiles = 4;
 
 // NW: wavefronts of a workgroup -- four, two workgroups to a CU, or eight where a stage's operands leave room for
 // one workgroup only
+// Wavefronts of a SIMD that registers allow: more than two where tiles are small, whose stages are all latency.
+constexpr int waves_per_simd(int mt, int nt, bool f16) { return f16 ? (mt * nt <= 4 ? 4 : mt * nt == 6 ? 3 : 2) : mt * nt == 1 ? 4 : mt * nt == 2 ? 3 : 2; }
+
 template <int MT, int NT, int NW, bool F16>
-__global__ __launch_bounds__(NW * 64, 2) void block_wgrad_kernel(BlockWgradPlan plan_arg, const char *__restrict__ A,
+__global__ __launch_bounds__(NW * 64, waves_per_simd(MT, NT, F16)) void block_wgrad_kernel(BlockWgradPlan plan_arg, const char *__restrict__ A,
                                                                   const char *__restrict__ G, float *__restrict__ ws) {
   constexpr int PARTS = F16 ? 1 : 3, UB = 16 * PARTS, KS = F16 ? 64 : 32, KSP = KS + 4;
   extern __shared__ __align__(16) char bw_lds[];
@@ -416,11 +419,17 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
   if (best == 0) return false;
   pl.mgt = pl.wm * pl.mt * 4;
   pl.cgt = pl.ctb * 4;
-  // slices: two workgroups per CU in all, dealt to the filter rows by their positions; twice as many, half as long, where a
-  // single accumulator takes all six products of fp32 parts (128 -> 256 channels, 3 x 3 taps, 32 x 256 x 41 positions:
-  // error 2.9e-6 -> 2.1e-6, wgrad_pos.hip 2.6e-6; its sums' launch 22 -> 28 us, 0.2 % of the step)
+  // slices: what a CU's registers and LDS hold of workgroups, dealt to the filter rows by their positions.  Small tiles have
+  // a few hundred cycles of products a stage, and more than two workgroups to hide the rest behind: 32 -> 32 channels, 4 x 4
+  // taps, 32 x 780 x 41, two workgroups and four: fp32 202 -> 147 us, half 111 -> 79 (their sums' launch 27 and 13 us either
+  // way) -- as long as a slice has eight stages.  Twice as many, half as long, where a single accumulator takes all six
+  // products of fp32 parts (128 -> 256 channels, 3 x 3 taps, 32 x 256 x 41 positions: error 2.9e-6 -> 2.1e-6, wgrad_pos.hip
+  // 2.6e-6; its sums' launch 22 -> 28 us, 0.2 % of the step)
   const int blocks = pl.m_blocks * pl.c_blocks, turns = !f16 && pl.mt * pl.nt > kLowTiles ? 2 : 1;
-  const i64 want = std::max<i64>(pl.nfx, (pl.nw == 4 ? 512 : 256) * turns / blocks);
+  const int resident = std::min<int>(waves_per_simd(pl.mt, pl.nt, f16) * 4 / pl.nw, (int)(160 * 1024 / pl.lds_bytes));
+  i64 want = 256 * resident * turns / blocks;
+  if (resident > 2) want = std::max<i64>(512 / blocks, std::min<i64>(want, work / KS / 8));
+  want = std::max<i64>(pl.nfx, want);
   int total = 0;
   for (int f = 0; f < pl.nfx; ++f) {
     const i64 k = (i64)pl.row[f].count * pl.noy * pl.batch, units = (k + KS - 1) / KS;

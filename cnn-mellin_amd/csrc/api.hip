@@ -1792,6 +1792,7 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
 struct LayerBackward {
   bool input_blocked, weight_blocked, plain;           // plain: some gradient takes the section-2 kernels
   bool bias_beside;                                    // section 2's weight gradient makes the bias gradient as well
+  bool bias_packed;                                    // the pass that blocks grad_out adds it up
   size_t masked_off, go_off, x_off, frag_off, slice_off, bias_off, wgrad_off, gw_off, gb_off, beside_off, pass_off, pass_bytes, total;
   BlockPlan bp;
   BlockWgradPlan wp;
@@ -1804,6 +1805,12 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
   lb.weight_blocked = ww && plan_block_weight(kind_x, half, CORR2D_ARGS, lb.wp);
   const bool any = lb.input_blocked || lb.weight_blocked;
   lb.plain = (wi && !lb.input_blocked) || (ww && !lb.weight_blocked) || !any;
+  const size_t beside = !half && lb.plain && ww && !lb.weight_blocked && (want & MELLIN_WANT_BIAS)
+                            ? bias_beside_weight(kind_x, CORR2D_ARGS) : 0;
+  lb.bias_beside = beside > 0;
+  // (a pass of its own over grad_out is two launches, and one less where the sums' launch has nothing else to do: 1 -> 125
+  // channels, 8 taps, 4 x 774 positions, eight launches a step with it and six without: FIXME us)
+  lb.bias_packed = any && (want & MELLIN_WANT_BIAS) && !lb.bias_beside;
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t off = at; at += align256(bytes); return off; };
   lb.masked_off = take(lb.plain && (want & MELLIN_WANT_RELU) ? (size_t)(batch * c_out * nhx * nhy) * elem : 0);
@@ -1811,17 +1818,14 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
   lb.x_off = take(lb.weight_blocked ? blocked_bytes(batch, c_in, ngx * ngy, half) : 0);
   lb.frag_off = take(lb.input_blocked ? lb.bp.filter_bytes : 0);
   lb.slice_off = take(lb.input_blocked ? lb.bp.slice_bytes : 0);
-  lb.bias_off = take(!lb.plain && (want & MELLIN_WANT_BIAS) ? pack_partial_count(batch, c_out, nhx * nhy) * 4 : 0);
+  lb.bias_off = take(lb.bias_packed ? pack_partial_count(batch, c_out, nhx * nhy) * 4 : 0);
   lb.wgrad_off = take(lb.weight_blocked ? lb.wp.ws_bytes : 0);
   // (half gradients of the parameters on their way to float)
   lb.gw_off = take(wide && ww && !lb.weight_blocked ? (size_t)(c_out * c_in * nfx * nfy) * 2 : 0);
-  lb.gb_off = take(wide && lb.plain && (want & MELLIN_WANT_BIAS) ? (size_t)c_out * 2 : 0);
-  const size_t beside = !half && lb.plain && ww && !lb.weight_blocked && (want & MELLIN_WANT_BIAS)
-                            ? bias_beside_weight(kind_x, CORR2D_ARGS) : 0;
-  lb.bias_beside = beside > 0;
+  lb.gb_off = take(wide && !lb.bias_packed && (want & MELLIN_WANT_BIAS) ? (size_t)c_out * 2 : 0);
   lb.beside_off = take(beside);
   size_t pass = 0;
-  const int want_pass = want & (MELLIN_WANT_RELU | (lb.bias_beside ? 0 : MELLIN_WANT_BIAS));
+  const int want_pass = want & (MELLIN_WANT_RELU | (lb.bias_beside || lb.bias_packed ? 0 : MELLIN_WANT_BIAS));
   if (lb.plain && want_pass)                           // (a ReLU's backward writes the bias gradient, asked for or not)
     pass = align256(mellin_bias_grad_workspace(batch, c_out, nhx * nhy)) + align256((size_t)c_out * elem);
   if (wi && !lb.input_blocked)
@@ -1884,10 +1888,11 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT, relu = want & MELLIN_WANT_RELU;
   hipStream_t st = (hipStream_t)stream;
   hipError_t e = hipSuccess;
-  if (lb.plain && (want & (MELLIN_WANT_RELU | (lb.bias_beside ? 0 : MELLIN_WANT_BIAS)))) {
+  const bool bias_here = (want & MELLIN_WANT_BIAS) && !lb.bias_beside && !lb.bias_packed;
+  if (lb.plain && (relu || bias_here)) {
     void *masked = relu ? ws + lb.masked_off : nullptr;
     const size_t own = mellin_bias_grad_workspace(batch, c_out, nhx * nhy);
-    void *gb = !(want & MELLIN_WANT_BIAS) || lb.bias_beside ? pass + align256(own) : wide ? ws + lb.gb_off : grad_bias;
+    void *gb = !bias_here ? pass + align256(own) : wide ? ws + lb.gb_off : grad_bias;
     rc = half ? mellin_bias_grad_f16(grad_out, masked ? out : nullptr, batch, c_out, nhx * nhy, masked, gb, pass, own, stream)
               : mellin_bias_grad_f32((const float *)grad_out, masked ? (const float *)out : nullptr, batch, c_out,
                                      nhx * nhy, (float *)masked, (float *)gb, pass, own, stream);
@@ -1909,7 +1914,7 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
     if (rc) return rc;
   }
   if (wide) {
-    const bool gw = (want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked, gb = lb.plain && (want & MELLIN_WANT_BIAS);
+    const bool gw = (want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked, gb = bias_here;
     e = launch_cast_pair(false, gw ? ws + lb.gw_off : nullptr, grad_weight, c_out * c_in * nfx * nfy, gb ? ws + lb.gb_off : nullptr,
                          grad_bias, c_out, st);
     if (e != hipSuccess) return check_hip(e, __func__);
@@ -1919,7 +1924,7 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
     return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
   g_variant = half ? "mfma-f16-blocks" : "mfma-blocks";
   g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
-  const bool sums = !lb.plain && (want & MELLIN_WANT_BIAS);
+  const bool sums = lb.bias_packed;
   const PackSignal go = {grad_out, relu && !lb.plain ? out : nullptr, ws + lb.go_off, sums ? (float *)(ws + lb.bias_off) : nullptr,
                          (int)batch, (int)c_out, (int)(nhx * nhy)};
   const PackSignal x = {input, nullptr, ws + lb.x_off, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
@@ -2084,6 +2089,31 @@ static int stack_checks(const char *who, bool planned, const StackPlan &sp, cons
   return MELLIN_OK;
 }
 
+// How a stack's first layer runs.  Where its kernel can store blocked tensors its output goes straight into the second
+// layer's input: as a plain tensor it is written, read back and laid out by a pass of its own, three trips to memory more
+// (FIXME).
+enum FirstLayer { FIRST_OWN, FIRST_BLOCKS, FIRST_TILES };   // a call of its own; the blocked kernels; the tiled kernel
+struct FirstPlan { BlockPlan blocks; TilePlan tiles; size_t lds; int mt, nt; };
+static FirstLayer first_layer(int kind_x, bool half, MELLIN_CORR2D_DIMS, FirstPlan &fp) {
+  if (plan_block_forward(kind_x, half, CORR2D_ARGS, fp.blocks))
+    return blocked_images(batch, c_in, ngx * ngy, half) < batch ? FIRST_OWN : FIRST_BLOCKS;
+  if (c_in * nfx * nfy * ngx * ngy == 0 || g_forced || g_gather > 0) return FIRST_OWN;
+  SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
+  pr.relu = 1;
+  if (half) {
+    HalfNative hn;
+    if (!plan_half_native(pr, hn) || hn.classes || hn.frag_bytes) return FIRST_OWN;
+    fp.tiles = hn.pl; fp.lds = hn.lds; fp.mt = hn.mt; fp.nt = hn.nt;
+  } else {
+    ClassPlans cp;
+    NarrowPlan np;
+    if (plan_mellin_classes(pr, cp) || (g_no_narrow <= 0 && make_narrow_plan(pr, np, g_no_narrow < 0)) ||
+        !make_tile_plan(pr, fp.tiles, &fp.lds, &fp.mt, &fp.nt))
+      return FIRST_OWN;
+  }
+  return tile_writes_blocked(fp.tiles, fp.mt) ? FIRST_TILES : FIRST_OWN;
+}
+
 int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers, const void *input,
                          void *out, void *saved, size_t saved_bytes, void *workspace, size_t workspace_bytes, void *stream) {
   StackPlan sp;
@@ -2099,10 +2129,18 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
     if (!layers[i].weight) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
   char *ws = (char *)workspace, *keep = (char *)saved;
   hipStream_t st = (hipStream_t)stream;
-  rc = mellin_layer_forward(kind_x, elem_bytes, MELLIN_ACT_RELU, input, layers[0].weight, layers[0].bias, STACK_DIMS(layers[0]),
-                            ws + sp.f_first, layers[0].weight_half, ws + sp.f_own, sp.own_bytes, stream);
-  if (rc) return rc;
-  // all filters, and the first layer's output
+  const mellin_stack_layer &ly0 = layers[0];
+  const i64 n_w0 = ly0.dims[1] * ly0.dims[2] * ly0.dims[3] * ly0.dims[4];
+  char *own = ws + sp.f_own;
+  FirstPlan fp;
+  const FirstLayer route = first_layer(kind_x, half, STACK_DIMS(ly0), fp);
+  hipError_t e = hipSuccess;
+  if (route == FIRST_OWN) {
+    rc = mellin_layer_forward(kind_x, elem_bytes, MELLIN_ACT_RELU, input, ly0.weight, ly0.bias, STACK_DIMS(ly0), ws + sp.f_first,
+                              ly0.weight_half, own, sp.own_bytes, stream);
+    if (rc) return rc;
+  }
+  // all filters, and the first signal that has to be laid out
   PackFilter filters[kStackLayers];
   size_t frag_off[kStackLayers], at = sp.f_filters;
   BlockPlan bp;
@@ -2117,8 +2155,39 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
   }
   auto input_of = [&](int i) { return sp.l[i].kept ? keep + sp.l[i].x_off : ws + sp.f_turn[i & 1]; };
   const StackLayer &l1 = sp.l[1];
-  const PackSignal dense = {ws + sp.f_first, nullptr, input_of(1), nullptr, (int)l1.batch, (int)l1.c_in, (int)l1.plane};
-  hipError_t e = launch_block_pack(half, &dense, nullptr, filters, n_layers - 1, st);
+  if (route == FIRST_OWN) {
+    const PackSignal dense = {ws + sp.f_first, nullptr, input_of(1), nullptr, (int)l1.batch, (int)l1.c_in, (int)l1.plane};
+    e = launch_block_pack(half, &dense, nullptr, filters, n_layers - 1, st);
+  } else if (route == FIRST_BLOCKS) {
+    const StackLayer &l0 = sp.l[0];
+    BlockPlan &p0 = fp.blocks;
+    p0.relu = 1;
+    p0.wide = wide;
+    const size_t filter_at = blocked_region(l0.batch, l0.c_in, l0.plane, half), sums_at = filter_at + align256(p0.filter_bytes);
+    filters[n_layers - 1] = pack_filter(p0, (int)l0.c_in, ly0.weight, own + filter_at, wide ? ly0.weight_half : nullptr, n_w0);
+    const PackSignal x = {input, nullptr, own, nullptr, (int)l0.batch, (int)l0.c_in, (int)l0.plane};
+    e = launch_block_pack(half, &x, nullptr, filters, n_layers, st);
+    const BlockGemmArgs args = {own, own + filter_at, ly0.bias, input_of(1), (float *)(own + sums_at), true, false, nullptr, nullptr};
+    if (e == hipSuccess) e = launch_block_gemm(p0, args, st);
+    if (e == hipSuccess && p0.rest > 0) {
+      BlockFinish fin = {};
+      fin.slices = &p0; fin.args = args;
+      e = launch_block_finish(half, wide, fin, st);
+    }
+  } else {
+    const void *w = ly0.weight, *b = ly0.bias;
+    if (wide) {                                        // (where mellin_layer_forward() rounds them)
+      char *rounded = own + align256(mellin_corr2d_forward_f16_workspace(kind_x, STACK_DIMS(ly0)));
+      void *w_half = ly0.weight_half ? ly0.weight_half : rounded, *b_half = rounded + align256(n_w0 * 2);
+      e = launch_cast_pair(true, w, w_half, n_w0, b, b_half, ly0.dims[2], st);
+      w = w_half;
+      b = b ? b_half : nullptr;
+    }
+    if (e == hipSuccess)
+      e = launch_tile_gemm(fp.tiles, fp.lds, fp.mt, fp.nt, (const float *)w, (const float *)input, (const float *)b, (float *)input_of(1),
+                           st, nullptr, true);
+    if (e == hipSuccess) e = launch_block_pack(half, nullptr, nullptr, filters, n_layers - 1, st);
+  }
   for (int i = 1; i < n_layers && e == hipSuccess; ++i) {
     const mellin_stack_layer &ly = layers[i];
     const StackLayer &l = sp.l[i];

@@ -177,21 +177,6 @@ __device__ __forceinline__ float lane_sums(const float (&v)[16], int lane) {
   return d + other(d, 1);
 }
 
-// Four values as a quarter unit of a blocked tensor: bf16 parts (fp32) or halves, two to a word.
-template <bool F16>
-__device__ __forceinline__ void cut_four(const float4 &v, unsigned (&w)[F16 ? 1 : 3][2]) {
-  if constexpr (F16) {
-    auto pair = [](float lo, float hi) {
-      return (unsigned)__builtin_bit_cast(unsigned short, (_Float16)lo) | ((unsigned)__builtin_bit_cast(unsigned short, (_Float16)hi) << 16);
-    };
-    w[0][0] = pair(v.x, v.y);
-    w[0][1] = pair(v.z, v.w);
-  } else {
-    split_pair(v.x, v.y, w[0][0], w[1][0], w[2][0]);
-    split_pair(v.z, v.w, w[0][1], w[1][1], w[2][1]);
-  }
-}
-
 template <int MT, int NT, int WM, int WK, bool F16, int OUT, bool JOINT>
 __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_arg, const char *__restrict__ X,
                                                                  const char *__restrict__ AF, const void *__restrict__ bias,

@@ -38,6 +38,7 @@
 #include <vector>
 #include <type_traits>
 
+#include "block_gemm.hpp"
 #include "mellin_common.hpp"
 #include "tile_gemm.hpp"
 #include "tile_stage.hpp"
@@ -65,7 +66,10 @@ namespace {
 // bx of gx: this workgroup among those that share the plan at plan_base (the whole launch,
 // or one residue class's share of it).
 typedef const __attribute__((address_space(4))) TilePlan ConstPlan;
-template <int MT, int NT, bool ACC, int MB, bool HOUT, int SPLIT>
+// BLOCKED: H is a channel-blocked tensor (block_gemm.hpp), for layers whose output the blocked kernels read next: no plain
+// output that a pass of its own reads back and lays out (1 -> 64 channels, 5 x 3 taps over 1177 windows of 10 x 41: 37 us
+// and 75 for the packing, 71 as one).  Bound by the stores, 6 bytes a value in fp32.
+template <int MT, int NT, bool ACC, int MB, bool HOUT, int SPLIT, bool BLOCKED>
 __device__ __forceinline__ void tile_gemm_body(
     ConstPlan *const plan_base, const int bx, const int gx, const float *__restrict__ F, const float *__restrict__ G,
     const float *__restrict__ bias, float *__restrict__ H, const float *__restrict__ AF) {
@@ -340,6 +344,44 @@ __device__ __forceinline__ void tile_gemm_body(
   // its multiplies, so that they drain behind the next matrix loop.
   auto write_tile = [&](auto full_tag) {
     constexpr bool FULL = decltype(full_tag)::value;
+    if constexpr (BLOCKED) {
+      // a unit is eight channels of a position: the halves of a wavefront exchange quarters, so that a lane stores whole
+      // ones, the lower half groups 0 and 2 of a tile's four, the upper one groups 1 and 3
+      constexpr int UB = 16 * PARTS;
+      const int groups = (pl.M + 7) / 8, unit_row = (pl.Q + 1) * UB, image = groups * unit_row;
+      char *const Hblk = (char *)H + (i64)tg.n * image;
+      const __amdgpu_buffer_rsrc_t h_rsrc = __builtin_amdgcn_make_buffer_rsrc(Hblk, 0, image, 0x00020000);
+      int to[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        to[t] = (wave * NT + t) * 32 + l32 < tg.count ? (m0 / 8 + half) * unit_row + lane_q[t] * UB : (int)0x80000000u;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; g4 += 2) {
+          // (groups past the last one are past the descriptor: dropped)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            unsigned lo[PARTS][2], hi[PARTS][2];
+            cut_four<F16>(make_float4(acc[i][t][4 * g4], acc[i][t][4 * g4 + 1], acc[i][t][4 * g4 + 2], acc[i][t][4 * g4 + 3]), lo);
+            cut_four<F16>(make_float4(acc[i][t][4 * g4 + 4], acc[i][t][4 * g4 + 5], acc[i][t][4 * g4 + 6], acc[i][t][4 * g4 + 7]), hi);
+#pragma unroll
+            for (int pt = 0; pt < PARTS; ++pt) {
+              const auto s0 = __builtin_amdgcn_permlane32_swap(lo[pt][0], hi[pt][0], false, false);
+              const auto s1 = __builtin_amdgcn_permlane32_swap(lo[pt][1], hi[pt][1], false, false);
+              __builtin_amdgcn_raw_buffer_store_b128(uintx4{s0[0], s1[0], s0[1], s1[1]}, h_rsrc, to[t] < 0 ? to[t] : to[t] + pt * 16, 0, 0);
+            }
+            if (to[t] >= 0) to[t] += 2 * unit_row;
+            __builtin_amdgcn_sched_barrier(0);           // (one block's registers at a time)
+          }
+        }
+      if (tg.q0 + tg.count == pl.Q && tid < M_T / 8 && m0 / 8 + tid < groups) {
+        uintx4 *z = (uintx4 *)(Hblk + (m0 / 8 + tid) * unit_row + pl.Q * UB);      // the unit of zeros behind the image
+#pragma unroll
+        for (int pt = 0; pt < PARTS; ++pt) z[pt] = uintx4{0, 0, 0, 0};
+      }
+      return;
+    }
     char *Himg = (char *)H + ((i64)tg.n * pl.h_n + (i64)m0 * pl.h_m) * ES;
     bool live[NT];
 #pragma unroll
@@ -438,7 +480,7 @@ __device__ __forceinline__ void tile_gemm_body(
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[i][t][r] = fmaxf(acc[i][t][r], 0.f);
     }
-    if (full_m) write_tile(std::true_type());
+    if (full_m || BLOCKED) write_tile(std::true_type());
     else write_tile(std::false_type());
   };
   FilterWords next_filter;
@@ -514,12 +556,12 @@ __device__ __forceinline__ void tile_gemm_body(
 #undef pl
 }
 
-template <int MT, int NT, bool ACC, int MB, bool HOUT, int SPLIT>
+template <int MT, int NT, bool ACC, int MB, bool HOUT, int SPLIT, bool BLOCKED>
 __global__ __launch_bounds__(kThreads, (NT == 1 ? (SPLIT ? 3 : 4) : 2)) void tile_gemm_kernel(
     TilePlan plan_arg, const float *__restrict__ F, const float *__restrict__ G,
     const float *__restrict__ bias, float *__restrict__ H, const float *__restrict__ AF) {
   // (the plan is the first argument: the kernel-argument segment starts with it)
-  tile_gemm_body<MT, NT, ACC, MB, HOUT, SPLIT>((ConstPlan *)__builtin_amdgcn_kernarg_segment_ptr(), (int)blockIdx.x,
+  tile_gemm_body<MT, NT, ACC, MB, HOUT, SPLIT, BLOCKED>((ConstPlan *)__builtin_amdgcn_kernarg_segment_ptr(), (int)blockIdx.x,
                                               (int)gridDim.x, F, G, bias, H, AF);
 }
 
@@ -542,7 +584,7 @@ __global__ __launch_bounds__(kThreads, (NT == 1 ? 3 : 2)) void tile_gemm_classes
   ConstArgs *const a = (ConstArgs *)__builtin_amdgcn_kernarg_segment_ptr();
   int c = 0, first = 0;
   for (; c + 1 < a->n && (int)blockIdx.x >= a->wg_end[c]; ++c) first = a->wg_end[c];
-  tile_gemm_body<MT, NT, false, 0, HOUT, SPLIT>((ConstPlan *)&a->pl[c], (int)blockIdx.x - first, a->wg_end[c] - first,
+  tile_gemm_body<MT, NT, false, 0, HOUT, SPLIT, false>((ConstPlan *)&a->pl[c], (int)blockIdx.x - first, a->wg_end[c] - first,
                                                (const float *)((const char *)F + a->f_bytes[c]), G, bias,
                                                (float *)((char *)H + a->h_bytes[c]), AF ? AF + a->af_words[c] : AF);
 }
@@ -602,11 +644,11 @@ __global__ __launch_bounds__(256) void filter_fragments_classes_kernel(ClassLaun
                              (uintx4 *)(AF + a->af_words[c]));
 }
 
-template <int MT, int NT, bool ACC, int MB, bool HOUT = false, int SPLIT = 0>
+template <int MT, int NT, bool ACC, int MB, bool HOUT = false, int SPLIT = 0, bool BLOCKED = false>
 hipError_t launch_variant(const TilePlan &pl, size_t lds_bytes, dim3 grid, const float *f,
                           const float *g, const float *bias, float *h, hipStream_t stream,
                           const float *af = nullptr) {
-  auto kern = tile_gemm_kernel<MT, NT, ACC, MB, HOUT, SPLIT>;
+  auto kern = tile_gemm_kernel<MT, NT, ACC, MB, HOUT, SPLIT, BLOCKED>;
   {
     static std::atomic<int> lds_allowed{0};                // (one per kernel instance)
     hipError_t e = allow_large_lds((const void *)kern, lds_bytes, lds_allowed);
@@ -975,9 +1017,14 @@ size_t tile_fragment_bytes(const TilePlan &pl, int mt) {
   return m_tiles * chunks * (pl.f16 ? 1 : 3) * (size_t)(pl.KC16 >> 3) * (mt * 32) * 16;
 }
 
+bool tile_writes_blocked(const TilePlan &pl, int mt) {
+  return pl.split && pl.CC >= pl.C && !pl.accumulate && !!pl.f16 == !!pl.out_half && mt <= 2 && pl.cls_stride == 1 && pl.cls_first == 0 &&
+         blocked_bytes(1, pl.M, pl.Q, pl.f16) < ((size_t)1 << 30);
+}
+
 hipError_t launch_tile_gemm(const TilePlan &pl, size_t lds_bytes, int mt, int nt,
                             const float *f, const float *g, const float *bias,
-                            float *h, hipStream_t stream, float *frag_ws) {
+                            float *h, hipStream_t stream, float *frag_ws, bool blocked) {
   const int M_T = mt * 32;
   const float *af = nullptr;
   if (pl.f16 && pl.accumulate) return hipErrorInvalidValue;
@@ -1001,6 +1048,19 @@ hipError_t launch_tile_gemm(const TilePlan &pl, size_t lds_bytes, int mt, int nt
   dim3 grid((unsigned)gx, (unsigned)m_tiles);
   // layers staged in three or more chunks of channels keep a tile's staging sources
   const bool memo = (pl.C + pl.CC - 1) / pl.CC > 2;
+  if (blocked) {
+    if (!tile_writes_blocked(pl, mt)) return hipErrorInvalidValue;
+#define MELLIN_BLOCKED_CASE(MT_, NT_)                                                                                          \
+  if (mt == MT_ && nt == NT_)                                                                                                  \
+    return pl.f16 ? launch_variant<MT_, NT_, false, 0, true, 3, true>(pl, lds_bytes, grid, f, g, bias, h, stream)              \
+                  : launch_variant<MT_, NT_, false, 0, false, 1, true>(pl, lds_bytes, grid, f, g, bias, h, stream);
+    MELLIN_BLOCKED_CASE(1, 1)
+    MELLIN_BLOCKED_CASE(1, 2)
+    MELLIN_BLOCKED_CASE(2, 1)
+    MELLIN_BLOCKED_CASE(2, 2)
+#undef MELLIN_BLOCKED_CASE
+    return hipErrorInvalidValue;
+  }
 #define MELLIN_TILE_CASE(MT_, NT_)                                                           \
   if (mt == MT_ && nt == NT_) {                                                              \
     if (pl.f16) return hipErrorInvalidValue;                                                 \

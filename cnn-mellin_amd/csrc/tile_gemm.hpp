@@ -78,10 +78,12 @@ size_t tile_fragment_bytes(const TilePlan &pl, int mt);
 // frag_ws: tile_fragment_bytes() of device memory, 16-byte aligned, or null (required by
 // a half-precision plan whose tile_fragment_bytes() is not zero).  For a plan made from a
 // problem with in_half, f, g and bias point to half-precision storage; h is half-precision
-// storage when the plan has out_half, else float.
+// storage when the plan has out_half, else float.  blocked: h is a channel-blocked tensor of the output (block_gemm.hpp)
+// instead, whose padding is written too (tile_writes_blocked(): the plan has such a kernel).
+bool tile_writes_blocked(const TilePlan &pl, int mt);
 hipError_t launch_tile_gemm(const TilePlan &pl, size_t lds_bytes, int mt, int nt,
                             const float *f, const float *g, const float *bias,
-                            float *h, hipStream_t stream, float *frag_ws = nullptr);
+                            float *h, hipStream_t stream, float *frag_ws = nullptr, bool blocked = false);
 
 // The plans of a Mellin layer's residue classes in ONE launch: every workgroup belongs to one
 // class for its whole life, the classes share the chip in proportion to their work.

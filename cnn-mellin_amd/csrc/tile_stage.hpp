@@ -471,6 +471,21 @@ __device__ __forceinline__ void split8(const float (&x)[8], uintx4 &hi, uintx4 &
   }
 }
 
+// Four values as a quarter unit of a blocked tensor: bf16 parts (fp32) or halves, two to a word.
+template <bool F16>
+__device__ __forceinline__ void cut_four(const float4 &v, unsigned (&w)[F16 ? 1 : 3][2]) {
+  if constexpr (F16) {
+    auto pair = [](float lo, float hi) {
+      return (unsigned)__builtin_bit_cast(unsigned short, (_Float16)lo) | ((unsigned)__builtin_bit_cast(unsigned short, (_Float16)hi) << 16);
+    };
+    w[0][0] = pair(v.x, v.y);
+    w[0][1] = pair(v.z, v.w);
+  } else {
+    split_pair(v.x, v.y, w[0][0], w[1][0], w[2][0]);
+    split_pair(v.z, v.w, w[0][1], w[1][1], w[2][1]);
+  }
+}
+
 // acc += A * B over 16 values of k, both operands as hi / mid / lo parts; small terms first
 __device__ __forceinline__ void mfma_split6(floatx16 &acc, const uintx4 &ah, const uintx4 &am, const uintx4 &al,
                                             const uintx4 &bh, const uintx4 &bm, const uintx4 &bl) {

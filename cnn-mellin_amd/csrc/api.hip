@@ -1938,13 +1938,10 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
     if (e == hipSuccess) e = launch_block_gemm(lb.bp, fin.args, st);
   }
   if (lb.weight_blocked) {
-    fin.weight = &lb.wp; fin.weight_partial = (float *)(ws + lb.wgrad_off); fin.grad_weight = grad_weight;
+    fin.add_weight(lb.wp, ws + lb.wgrad_off, grad_weight);
     if (e == hipSuccess) e = launch_block_wgrad(lb.wp, ws + lb.go_off, ws + lb.x_off, (float *)(ws + lb.wgrad_off), st);
   }
-  if (sums) {
-    fin.bias_partial = (const float *)(ws + lb.bias_off); fin.grad_bias = grad_bias;
-    fin.bias_count = (i64)pack_partial_count(batch, 1, nhx * nhy); fin.channels = c_out;
-  }
+  if (sums) fin.add_bias(ws + lb.bias_off, (i64)pack_partial_count(batch, 1, nhx * nhy), c_out, grad_bias);
   if (e == hipSuccess) e = launch_block_finish(half, wide, fin, st);
   return check_hip(e, __func__);
 }
@@ -1956,12 +1953,17 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
       (l).dims[9], (l).dims[10], (l).dims[11], (l).dims[12], (l).dims[13], (l).dims[14], (l).dims[15], (l).dims[16]
 
 constexpr int kStackLayers = 64;
+// Partial sums of weight and bias gradients that a stack's backward keeps at a time: those of layers that follow each other
+// are added up by one launch (nine layers, 64 channels and up, 4 x 252 frames, training: 718 -> 673 us with those of nine;
+// with four times as much ten layers on 32 x 780 frames, of which one fills it, are no faster).
+constexpr size_t kStackPartialBytes = (size_t)32 << 20;
 
 struct StackLayer {
   i64 batch, c_in, c_out, plane, q, rows, cols;        // of the input; of the output before pooling
   bool kept;                                           // the input lies in `saved` (else: in the forward workspace)
   size_t x_off, which_off;                             // input, blocked; saved: which value of a pair pooled into it
   size_t frag_off;                                     // backward workspace: filter of the input gradient
+  size_t bias_bytes;                                   // partial sums of the bias gradient
 };
 // Where everything lies.  saved: the layers' blocked inputs, from the second layer on (without training two regions in
 // turn) and the poolings' choices.  In training the last layer's comes first and layers below `first`, which nothing is
@@ -1971,13 +1973,13 @@ struct StackPlan {
   StackLayer l[kStackLayers];
   size_t saved, forward, backward;
   size_t f_first, f_own, f_filters, f_unpooled, f_sums, f_turn[2], own_bytes;                          // forward workspace
-  size_t b_grad[2], b_unpooled, b_bias[2], b_weight, b_sums, b_first, b_own, b_own_bytes;   // backward workspace
+  size_t b_grad[2], b_unpooled, b_partial, partial_bytes, b_sums, b_first, b_own, b_own_bytes;         // backward workspace
 };
 static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const mellin_stack_layer *layers, StackPlan &sp) {
   const bool half = elem != 4;
   if (n < 2 || n > kStackLayers || first < 0 || first >= n) return false;
   size_t saved = 0, in_turn[2] = {0, 0}, frags = 0, unpooled = 0, sums = 0, x_bytes[kStackLayers], which_bytes[kStackLayers];
-  size_t grad[2] = {0, 0}, b_unpooled = 0, bias[2] = {0, 0}, weight = 0, b_frags = 0, b_sums = 0;
+  size_t grad[2] = {0, 0}, b_unpooled = 0, b_frags = 0, b_sums = 0, partials = 0, most_partials = 0;
   auto region = [&](i64 channels, i64 plane, i64 batch) { return align256(blocked_bytes(batch, channels, plane, half)); };
   for (int i = 0; i < n; ++i) {
     const mellin_stack_layer &ly = layers[i];
@@ -2004,15 +2006,21 @@ static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const
     if (!plan_block_input(kind_x, half, STACK_DIMS(ly), ip) || !plan_block_weight(kind_x, half, STACK_DIMS(ly), wp)) return false;
     b_frags += align256(ip.filter_bytes);
     b_sums = std::max(b_sums, ip.slice_bytes);
-    weight = std::max(weight, wp.ws_bytes);
     grad[i & 1] = std::max(grad[i & 1], region(l.c_out, l.q, l.batch));
     if (before.pool) {
       b_unpooled = std::max(b_unpooled, region(l.c_in, l.plane, l.batch));
-      bias[(i - 1) & 1] = std::max(bias[(i - 1) & 1], pool_partial_count(l.batch, l.c_in, before.dims[7], before.dims[8]) * 4);
+      sp.l[i - 1].bias_bytes = align256(pool_partial_count(l.batch, l.c_in, before.dims[7], before.dims[8]) * 4);
     } else {
-      bias[(i - 1) & 1] = std::max(bias[(i - 1) & 1], (size_t)l.c_in * ip.chan_slots * 4);
+      sp.l[i - 1].bias_bytes = align256((size_t)l.c_in * ip.chan_slots * 4);
     }
-    if (i == n - 1) bias[i & 1] = std::max(bias[i & 1], pack_partial_count(l.batch, l.c_out, l.q) * 4);
+    const size_t both = align256(wp.ws_bytes) + sp.l[i - 1].bias_bytes;
+    partials += both;
+    most_partials = std::max(most_partials, both);
+    if (i == n - 1) {
+      l.bias_bytes = align256(pack_partial_count(l.batch, l.c_out, l.q) * 4);
+      partials += l.bias_bytes;
+      most_partials = std::max(most_partials, l.bias_bytes);
+    }
   }
   for (int i = n - 1; i > 0; --i) {
     StackLayer &l = sp.l[i];
@@ -2050,9 +2058,8 @@ static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const
   sp.b_grad[0] = take(grad[0]);
   sp.b_grad[1] = take(grad[1]);
   sp.b_unpooled = take(b_unpooled);
-  sp.b_bias[0] = take(bias[0]);
-  sp.b_bias[1] = take(bias[1]);
-  sp.b_weight = take(weight);
+  sp.partial_bytes = std::min(partials, std::max(kStackPartialBytes, most_partials));
+  sp.b_partial = take(sp.partial_bytes);
   sp.b_sums = take(b_sums);
   sp.b_first = take(dense);
   sp.b_own_bytes = mellin_layer_backward_workspace(kind_x, elem, MELLIN_WANT_INPUT | MELLIN_WANT_WEIGHT, STACK_DIMS(layers[0]));
@@ -2091,8 +2098,7 @@ static int stack_checks(const char *who, bool planned, const StackPlan &sp, cons
 
 // How a stack's first layer runs.  Where its kernel can store blocked tensors its output goes straight into the second
 // layer's input: as a plain tensor it is written, read back and laid out by a pass of its own, three trips to memory more
-// (32 x 780 x 41, 1 -> 32 channels: fp32 141 -> 78 us with the filters' packing, half 70 -> 40; one utterance's stack is a
-// launch's signal shorter).
+// (32 x 780 x 41, 1 -> 32 channels: fp32 141 -> 78 us with the filters' packing, half 70 -> 40).
 enum FirstLayer { FIRST_OWN, FIRST_BLOCKS, FIRST_TILES };   // a call of its own; the blocked kernels; the tiled kernel
 struct FirstPlan { BlockPlan blocks; TilePlan tiles; size_t lds; int mt, nt; };
 static FirstLayer first_layer(int kind_x, bool half, MELLIN_CORR2D_DIMS, FirstPlan &fp) {
@@ -2243,55 +2249,65 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
     filters[n_filters++] = pack_filter(ip, (int)ly.dims[2], w, ws + sp.l[i].frag_off, nullptr, 0);
   }
   const int top = n_layers - 1;
-  i64 bias_count[2] = {0, 0};                          // partial sums of a channel in either region
+  // sums that are left to do, and the bytes of their partial sums
+  BlockFinish fin = {};
+  size_t kept = 0;
+  auto take = [&](size_t bytes) { char *at = ws + sp.b_partial + kept; kept += bytes; return at; };
+  auto finish = [&]() {
+    const hipError_t r = launch_block_finish(half, wide, fin, st);
+    fin = BlockFinish{};
+    return r;
+  };
   const StackLayer &lt = sp.l[top];
-  const PackSignal go = {grad_out, out, ws + sp.b_grad[top & 1], (float *)(ws + sp.b_bias[top & 1]), (int)lt.batch, (int)lt.c_out, (int)lt.q};
-  bias_count[top & 1] = (i64)pack_partial_count(lt.batch, 1, lt.q);
+  const PackSignal go = {grad_out, out, ws + sp.b_grad[top & 1], (float *)take(lt.bias_bytes), (int)lt.batch, (int)lt.c_out, (int)lt.q};
   hipError_t e = launch_block_pack(half, &go, nullptr, filters, n_filters, st);
+  if (layers[top].grad_bias) fin.add_bias(go.partial, (i64)pack_partial_count(lt.batch, 1, lt.q), lt.c_out, layers[top].grad_bias);
   for (int i = top; i >= std::max(lowest, 1) && e == hipSuccess; --i) {
     const mellin_stack_layer &ly = layers[i];
     const StackLayer &l = sp.l[i];
     const int here = i & 1, below = here ^ 1;
     const bool first_dense = i == 1, pooled = layers[i - 1].pool;
-    BlockFinish fin = {};
-    BlockWgradPlan wp;
-    if (ly.grad_weight) {
-      plan_block_weight(kind_x, half, STACK_DIMS(ly), wp);
-      e = launch_block_wgrad(wp, ws + sp.b_grad[here], keep + l.x_off, (float *)(ws + sp.b_weight), st);
-      fin.weight = &wp; fin.weight_partial = (const float *)(ws + sp.b_weight); fin.grad_weight = ly.grad_weight;
-    }
-    if (ly.grad_bias) {
-      fin.bias_partial = (const float *)(ws + sp.b_bias[here]); fin.grad_bias = ly.grad_bias;
-      fin.bias_count = bias_count[here]; fin.channels = l.c_out;
-    }
     const bool go_on = i > lowest;
-    if (go_on && e == hipSuccess) {
+    BlockWgradPlan wp;
+    if (ly.grad_weight) plan_block_weight(kind_x, half, STACK_DIMS(ly), wp);
+    const size_t weight_bytes = ly.grad_weight ? align256(wp.ws_bytes) : 0, bias_bytes = go_on ? sp.l[i - 1].bias_bytes : 0;
+    if (kept + weight_bytes + bias_bytes > sp.partial_bytes || fin.n_weights == kFinishJobs || fin.n_biases == kFinishJobs) {
+      if ((e = finish()) != hipSuccess) break;
+      kept = 0;                                        // (every partial sum so far has its sum launched)
+    }
+    if (ly.grad_weight) {
+      float *partial = (float *)take(weight_bytes);
+      if ((e = launch_block_wgrad(wp, ws + sp.b_grad[here], keep + l.x_off, partial, st)) != hipSuccess) break;
+      fin.add_weight(wp, partial, ly.grad_weight);
+    }
+    float *const bias_below = go_on ? (float *)take(bias_bytes) : nullptr;
+    i64 bias_count = 0;
+    if (go_on) {
       plan_block_input(kind_x, half, STACK_DIMS(ly), ip);
       ip.relu = 0;
       char *to = first_dense ? ws + sp.b_first : pooled ? ws + sp.b_unpooled : ws + sp.b_grad[below];
-      fin.slices = &ip;
-      fin.args = {ws + sp.b_grad[here], ws + l.frag_off, nullptr, to, (float *)(ws + sp.b_sums), !first_dense, !pooled,
-                  keep + l.x_off, (float *)(ws + sp.b_bias[below])};
-      if (!pooled) bias_count[below] = ip.chan_slots;
-      e = launch_block_gemm(ip, fin.args, st);
+      const BlockGemmArgs args = {ws + sp.b_grad[here], ws + l.frag_off, nullptr, to, (float *)(ws + sp.b_sums), !first_dense, !pooled,
+                                  keep + l.x_off, bias_below};
+      bias_count = ip.chan_slots;
+      e = launch_block_gemm(ip, args, st);
+      if (e == hipSuccess && ip.rest > 0) {            // (what goes on from here needs the whole tiles: the sums go along)
+        fin.slices = &ip;
+        fin.args = args;
+        e = finish();
+      }
     }
-    if (e == hipSuccess) e = launch_block_finish(half, wide, fin, st);
     if (go_on && pooled && e == hipSuccess) {
       const mellin_stack_layer &before = layers[i - 1];
       e = launch_block_pool_grad(half, ws + sp.b_unpooled, keep + l.x_off, keep + l.which_off, l.batch, l.c_in, before.dims[7],
-                                 before.dims[8], ws + sp.b_grad[below], (float *)(ws + sp.b_bias[below]), st);
-      bias_count[below] = (i64)pool_partial_count(l.batch, 1, before.dims[7], before.dims[8]);
+                                 before.dims[8], ws + sp.b_grad[below], bias_below, st);
+      bias_count = (i64)pool_partial_count(l.batch, 1, before.dims[7], before.dims[8]);
     }
+    if (go_on && layers[i - 1].grad_bias) fin.add_bias(bias_below, bias_count, l.c_in, layers[i - 1].grad_bias);
   }
+  if (e == hipSuccess) e = finish();
   if (e != hipSuccess) return check_hip(e, __func__);
   if (lowest == 0) {
     const mellin_stack_layer &ly = layers[0];
-    if (ly.grad_bias) {
-      BlockFinish fin = {};
-      fin.bias_partial = (const float *)(ws + sp.b_bias[0]); fin.grad_bias = ly.grad_bias;
-      fin.bias_count = bias_count[0]; fin.channels = sp.l[0].c_out;
-      if ((e = launch_block_finish(half, wide, fin, st)) != hipSuccess) return check_hip(e, __func__);
-    }
     const int want = (grad_input ? MELLIN_WANT_INPUT : 0) | (ly.grad_weight ? MELLIN_WANT_WEIGHT : 0);
     if (want) {
       const size_t own = mellin_layer_backward_workspace(kind_x, elem_bytes, want, STACK_DIMS(ly));

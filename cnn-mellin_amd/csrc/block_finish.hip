@@ -2,7 +2,7 @@
 // gradients from their partial blocks, bias gradients from the packing pass's partial sums, and the
 // output of a pass whose contracted channels were dealt to several workgroups.  Each is a short
 // streaming sum in a fixed order; on small layers a launch of its own (3-5 us each) cost more than
-// the sum, so they share one.
+// the sum, so they share one -- those of all layers of a stack, as far as their partial sums are kept.
 #include <algorithm>
 
 #include "block_gemm.hpp"
@@ -17,19 +17,14 @@ constexpr int kFinishTaps = 64;
 constexpr int kSliceValues = kFinishThreads * 4;       // values of a tile that a block adds up
 
 struct FinishArgs {
-  BlockWgradPlan w;
-  const float *w_partial;
-  void *gw;
-  unsigned w_blocks, w_zero_blocks;
-  int w_taps;
-  const float *b_partial;
-  void *gb;
-  i64 b_count;
-  unsigned b_blocks;
+  int n_weights, n_biases;
+  WeightSums w[kFinishJobs];
+  BiasSums b[kFinishJobs];
   BlockPlan s;
   BlockGemmArgs sa;
   const int2 *s_rows;
 };
+static_assert(sizeof(FinishArgs) <= 4096, "kernel arguments are limited to 4 KB");
 
 // p[0] + p[step] + .. + p[(count - 1) step], added to `s` in that order.  Eight loads are on their way at a time: a sum is a
 // chain of trips to memory, and with one or four the sums of a few channels over an image's many tiles took 20-27 us a
@@ -56,9 +51,11 @@ __device__ __forceinline__ float add_chain(const float *__restrict__ p, i64 step
 // gw[m, c, fx, fy] = the sum of its partial sums in slice order.  A block owns 32 weights that lie side by side in
 // the partial blocks; its eight groups of 32 threads add an eighth of the slices each, and those sums are added in order.
 template <typename T>
-__device__ void finish_weight(const BlockWgradPlan &pl, const float *__restrict__ ws, T *__restrict__ gw, int b, float (*red)[32]) {
+__device__ void finish_weight(const WeightSums &pl, int b, float (*red)[32]) {
+  const float *__restrict__ ws = pl.partial;
+  T *__restrict__ gw = (T *)pl.grad;
   const int cl = threadIdx.x & 31, grp = threadIdx.x >> 5;
-  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.wm * pl.mt * 32;
+  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.m_t;
   // block -> (filter row, column tile, channel)
   const int tiles = pl.ctb * pl.nfy;
   const int m = b % pl.M;
@@ -68,9 +65,9 @@ __device__ void finish_weight(const BlockWgradPlan &pl, const float *__restrict_
   const int cb = b % pl.c_blocks, fx = b / pl.c_blocks;
   const int ct = tile / pl.nfy, fy = tile - ct * pl.nfy, c = (cb * pl.ctb + ct) * 32 + cl;
   const int mb = m / m_t, ml = m - mb * m_t;
-  const int slices = pl.row[fx].slices, blocks = pl.m_blocks * pl.c_blocks;
+  const int slices = pl.slices[fx], blocks = pl.m_blocks * pl.c_blocks;
   const i64 stride = (i64)blocks * m_t * cols;
-  const float *p = ws + ((i64)pl.row[fx].slice0 * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols + tile * 32 + cl;
+  const float *p = ws + ((i64)pl.slice0[fx] * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols + tile * 32 + cl;
   const int lo = slices * grp / 8, hi = slices * (grp + 1) / 8;
   red[grp][cl] = add_chain(p + lo * stride, stride, hi - lo, 0.f);
   __syncthreads();
@@ -85,15 +82,17 @@ __device__ void finish_weight(const BlockWgradPlan &pl, const float *__restrict_
 // The same for weights that are many and have few slices (less than 16 on average: a block per 32 weights would mostly wait, and write 4 bytes of
 // every line): a block owns an output channel and 32 input channels with all their taps, which it writes side by side.
 template <typename T>
-__device__ void finish_weight_taps(const BlockWgradPlan &pl, const float *__restrict__ ws, T *__restrict__ gw, int b, float (*sum)[33]) {
-  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.wm * pl.mt * 32, c_tiles = (pl.C + 31) / 32, taps = pl.nfx * pl.nfy;
+__device__ void finish_weight_taps(const WeightSums &pl, int b, float (*sum)[33]) {
+  const float *__restrict__ ws = pl.partial;
+  T *__restrict__ gw = (T *)pl.grad;
+  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.m_t, c_tiles = (pl.C + 31) / 32, taps = pl.nfx * pl.nfy;
   const int m = b / c_tiles, ct_all = b - m * c_tiles, cl = threadIdx.x & 31;
   const int mb = m / m_t, ml = m - mb * m_t, cb = ct_all / pl.ctb, ct = ct_all - cb * pl.ctb;
   const int blocks = pl.m_blocks * pl.c_blocks;
   const i64 stride = (i64)blocks * m_t * cols;
   for (int tap = threadIdx.x >> 5; tap < taps; tap += kFinishThreads / 32) {
-    const int fx = tap / pl.nfy, fy = tap - fx * pl.nfy, slices = pl.row[fx].slices;
-    const float *p = ws + ((i64)pl.row[fx].slice0 * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols +
+    const int fx = tap / pl.nfy, fy = tap - fx * pl.nfy, slices = pl.slices[fx];
+    const float *p = ws + ((i64)pl.slice0[fx] * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols +
                      (ct * pl.nfy + fy) * 32 + cl;
     sum[tap][cl] = add_chain(p, stride, slices, 0.f);
   }
@@ -200,31 +199,37 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
   __shared__ float red[8][32], taps[kFinishTaps][33];
   const int tid = threadIdx.x;
   unsigned b = blockIdx.x;
-  if (b < a.w_blocks) {
-    if (a.w_taps) finish_weight_taps<TG>(a.w, a.w_partial, (TG *)a.gw, (int)b, taps);
-    else finish_weight<TG>(a.w, a.w_partial, (TG *)a.gw, (int)b, red);
-    return;
+  for (int i = 0; i < a.n_weights; ++i) {
+    const WeightSums &w = a.w[i];
+    if (b < w.blocks) {
+      if (w.taps) finish_weight_taps<TG>(w, (int)b, taps);
+      else finish_weight<TG>(w, (int)b, red);
+      return;
+    }
+    b -= w.blocks;
+    if (b < w.zero_blocks) {                           // filter columns that have no tap at all: zeros
+      const i64 at = (i64)b * kFinishThreads + tid;
+      const int fy = (int)(at % w.f_pitch);
+      if (at < (i64)w.M * w.C * w.nfx * w.f_pitch && (fy < w.f_off || fy >= w.f_off + w.nfy)) ((TG *)w.grad)[at] = (TG)0;
+      return;
+    }
+    b -= w.zero_blocks;
   }
-  b -= a.w_blocks;
-  if (b < a.w_zero_blocks) {                           // filter columns that have no tap at all: zeros
-    const i64 i = (i64)b * kFinishThreads + tid;
-    const int fy = (int)(i % a.w.f_pitch);
-    if (i < (i64)a.w.M * a.w.C * a.w.nfx * a.w.f_pitch && (fy < a.w.f_off || fy >= a.w.f_off + a.w.nfy)) ((TG *)a.gw)[i] = (TG)0;
-    return;
-  }
-  b -= a.w_zero_blocks;
-  if (b < a.b_blocks) {
-    // one channel: thread sums, a shuffle tree per wavefront, the wavefronts in order
-    const float *p = a.b_partial + (i64)b * a.b_count;
-    float s = tid < a.b_count ? add_chain(p + tid, kFinishThreads, (int)((a.b_count - tid + kFinishThreads - 1) / kFinishThreads), 0.f) : 0.f;
+  for (int i = 0; i < a.n_biases; ++i) {
+    const BiasSums &c = a.b[i];
+    if (b < c.channels) {
+      // one channel: thread sums, a shuffle tree per wavefront, the wavefronts in order
+      const float *p = c.partial + (i64)b * c.count;
+      float s = tid < c.count ? add_chain(p + tid, kFinishThreads, (int)((c.count - tid + kFinishThreads - 1) / kFinishThreads), 0.f) : 0.f;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o);
-    if ((tid & 63) == 0) red[0][tid >> 6] = s;
-    __syncthreads();
-    if (tid == 0) ((TG *)a.gb)[b] = (TG)(red[0][0] + red[0][1] + red[0][2] + red[0][3]);
-    return;
+      for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o);
+      if ((tid & 63) == 0) red[0][tid >> 6] = s;
+      __syncthreads();
+      if (tid == 0) ((TG *)c.grad)[b] = (TG)(red[0][0] + red[0][1] + red[0][2] + red[0][3]);
+      return;
+    }
+    b -= c.channels;
   }
-  b -= a.b_blocks;
   if (a.sa.blocked || a.sa.grad) {
     finish_units<T>(a, (int)b, red);
     return;
@@ -258,23 +263,31 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
 
 }  // namespace
 
+void BlockFinish::add_weight(const BlockWgradPlan &pl, const void *partial, void *grad) {
+  WeightSums &w = weight[n_weights++];
+  w = WeightSums{(const float *)partial, grad, pl.M, pl.C, pl.nfx, pl.nfy, pl.f_pitch, pl.f_off, pl.ctb, pl.wm * pl.mt * 32, pl.m_blocks,
+                 pl.c_blocks, 0, 0, 0, {}, {}};
+  for (int f = 0; f < pl.nfx; ++f) {
+    w.slice0[f] = (unsigned short)pl.row[f].slice0;
+    w.slices[f] = (unsigned short)pl.row[f].slices;
+  }
+  w.taps = pl.slices < 16 * pl.nfx && pl.nfx * pl.nfy <= kFinishTaps && (i64)pl.M * pl.C >= 1 << 14;
+  w.blocks = w.taps ? (unsigned)(pl.M * ((pl.C + 31) / 32)) : (unsigned)(pl.nfx * pl.c_blocks * pl.ctb * pl.nfy * pl.M);
+  if (pl.nfy != pl.f_pitch) w.zero_blocks = (unsigned)(((i64)pl.M * pl.C * pl.nfx * pl.f_pitch + kFinishThreads - 1) / kFinishThreads);
+}
+
 hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipStream_t stream) {
   FinishArgs a = {};
-  if (job.weight) {
-    a.w = *job.weight;
-    a.w_partial = job.weight_partial;
-    a.gw = job.grad_weight;
-    a.w_taps = a.w.slices < 16 * a.w.nfx && a.w.nfx * a.w.nfy <= kFinishTaps && (i64)a.w.M * a.w.C >= 1 << 14;
-    a.w_blocks = a.w_taps ? (unsigned)(a.w.M * ((a.w.C + 31) / 32))
-                          : (unsigned)(a.w.nfx * a.w.c_blocks * a.w.ctb * a.w.nfy * a.w.M);
-    if (a.w.nfy != a.w.f_pitch)
-      a.w_zero_blocks = (unsigned)(((i64)a.w.M * a.w.C * a.w.nfx * a.w.f_pitch + kFinishThreads - 1) / kFinishThreads);
+  i64 blocks = 0;
+  a.n_weights = job.n_weights;
+  a.n_biases = job.n_biases;
+  for (int i = 0; i < job.n_weights; ++i) {
+    a.w[i] = job.weight[i];
+    blocks += (i64)a.w[i].blocks + a.w[i].zero_blocks;
   }
-  if (job.grad_bias) {
-    a.b_partial = job.bias_partial;
-    a.gb = job.grad_bias;
-    a.b_count = job.bias_count;
-    a.b_blocks = (unsigned)job.channels;
+  for (int i = 0; i < job.n_biases; ++i) {
+    a.b[i] = job.bias[i];
+    blocks += a.b[i].channels;
   }
   i64 s_blocks = 0;
   if (job.slices && job.slices->rest > 0) {
@@ -285,7 +298,7 @@ hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipS
     const i64 each = a.sa.blocked || a.sa.grad ? kFinishThreads * 8 : kSliceValues;
     s_blocks = (i64)a.s.rest * a.s.m_tiles * ((values + each - 1) / each);
   }
-  const i64 blocks = (i64)a.w_blocks + a.w_zero_blocks + a.b_blocks + s_blocks;
+  blocks += s_blocks;
   if (blocks == 0) return hipSuccess;
   const dim3 grid((unsigned)blocks), threads(kFinishThreads);
   if (f16 && wide) hipLaunchKernelGGL((block_finish_kernel<_Float16, float>), grid, threads, 0, stream, a);

@@ -118,7 +118,7 @@ size_t pack_partial_count(i64 batch, i64 channels, i64 plane);
 // A filter to pack for `pl`, and on Mellin axes the output rows in the order of their classes: f (fp32 or half; wide: fp32
 // where the tensors are half) of `channels` contracted channels -> filter_bytes at `frag`.  `copy`: the filter's
 // `copy_count` floats, rounded to half.
-struct PackFilter {
+struct PackFilterHead {
   const void *f;
   char *frag;
   void *copy;
@@ -128,11 +128,11 @@ struct PackFilter {
   int kind_x, nox, ngx, sx, dx, px, ux;
   unsigned mg_p1;
   int n_classes, cls_stride;
-  BlockClass cls[kBlockClasses];
 };
+struct PackFilter : PackFilterHead { BlockClass cls[kBlockClasses]; };
 PackFilter pack_filter(const BlockPlan &pl, int channels, const void *f, void *frag, void *copy, i64 copy_count);
-// Everything a pass reads, in one launch (one for every kPackFilters filters): up to two tensors (null: not there) and filters.
-constexpr int kPackFilters = 6;
+// Everything a pass reads, in one launch (more of them for more filters or classes than a launch's arguments hold): up to two
+// tensors (null: not there) and filters.
 hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b, const PackFilter *filters, int n_filters,
                              hipStream_t stream);
 
@@ -145,16 +145,32 @@ hipError_t launch_block_pool_grad(bool f16, const void *grad_y, const void *y, c
                                   i64 cols, void *grad_x, float *partial, hipStream_t stream);
 size_t pool_partial_count(i64 batch, i64 channels, i64 rows, i64 cols);
 
-// The sums that end a pass, in one launch; null pointers for those there are not.
+// The sums that end passes, in one launch.
+constexpr int kFinishJobs = 16;
+struct WeightSums {                // a weight gradient from its partial blocks
+  const float *partial;
+  void *grad;
+  int M, C, nfx, nfy, f_pitch, f_off, ctb, m_t, m_blocks, c_blocks;    // (m_t: output channels of a block)
+  int taps;                        // a block of threads takes all taps of its weights
+  unsigned blocks, zero_blocks;    // blocks of threads; of those for columns without a tap
+  unsigned short slice0[kBlockFilterRows], slices[kBlockFilterRows];
+};
+struct BiasSums {                  // a bias gradient: `count` partial sums of each of `channels`
+  const float *partial;
+  void *grad;
+  i64 count;
+  unsigned channels;
+};
 struct BlockFinish {
-  const BlockWgradPlan *weight;    // weight gradient from its partial blocks
-  const float *weight_partial;
-  void *grad_weight;
-  const float *bias_partial;       // bias gradient: `bias_count` partial sums of each of `channels`
-  void *grad_bias;
-  i64 bias_count, channels;
-  const BlockPlan *slices;         // what a block_gemm called with `args` made of tiles in slices
+  int n_weights, n_biases;
+  WeightSums weight[kFinishJobs];
+  BiasSums bias[kFinishJobs];
+  const BlockPlan *slices;         // what a block_gemm called with `args` made of tiles in slices (null: none)
   BlockGemmArgs args;
+  void add_weight(const BlockWgradPlan &pl, const void *partial, void *grad);
+  void add_bias(const void *partial, i64 count, i64 channels, void *grad) {
+    bias[n_biases++] = BiasSums{(const float *)partial, grad, count, (unsigned)channels};
+  }
 };
 // (wide: the gradients are float where the tensors are half)
 hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipStream_t stream);

@@ -104,7 +104,7 @@ __device__ __forceinline__ void pack_signal(const PackPart &pt, unsigned block, 
 //   frag[((mt * (CG * nfx * nfy + 1) + (cg * nfx + fx) * nfy + fy) * parts + p) * 32 + r]   (16-byte words)
 // and a unit of zeros behind each tile of 32 channels.
 template <bool F16, typename From>
-__device__ __forceinline__ void pack_fragments(const PackFilter &pl, i64 idx) {
+__device__ __forceinline__ void pack_fragments(const PackFilterHead &pl, i64 idx) {
   typedef typename std::conditional<F16, _Float16, float>::type T;
   const int taps = pl.nfx * pl.nfy, per_tile = pl.CG * taps + 1;
   const i64 total = (i64)pl.tiles * per_tile * 32;
@@ -136,32 +136,39 @@ __device__ __forceinline__ void pack_fragments(const PackFilter &pl, i64 idx) {
 }
 
 // Output row `row` of a Mellin axis in the order of its classes, with the filter rows that have a tap for it.
-__device__ __forceinline__ int2 class_row(const PackFilter &pl, int row) {
+__device__ __forceinline__ int2 class_row(const PackFilterHead &pl, const BlockClass *cls, int row) {
   int ox = row;
   for (int k = 0; k < pl.n_classes; ++k)
-    if (row >= pl.cls[k].start) ox = pl.cls[k].first + (row - pl.cls[k].start) * pl.cls_stride;
+    if (row >= cls[k].start) ox = cls[k].first + (row - cls[k].start) * pl.cls_stride;
   int mask = 0;
   for (int f = 0; f < pl.nfx; ++f)
     if (mellin_tap32(pl.kind_x, ox, f, pl.ngx, pl.sx, pl.dx, pl.px + 1, pl.ux, pl.mg_p1) >= 0) mask |= 1 << f;
   return make_int2(ox, mask);
 }
 
+// The filters of a stack of 16 layers and their classes go with one launch: with the classes of each at their most, six did,
+// and ten layers took two (one utterance through ten Mellin layers 226.6 -> 223.4 us).
+constexpr int kPackFilters = 16, kPackClasses = 96;
+
 struct PackArgs {
   PackPart a, b;
-  PackFilter filter[kPackFilters];
+  PackFilterHead filter[kPackFilters];
   unsigned rows[kPackFilters], fragments[kPackFilters], copies[kPackFilters];      // blocks
+  short cls_at[kPackFilters];
   int n_filters;
+  BlockClass cls[kPackClasses];
 };
+static_assert(kPackClasses >= kBlockClasses && sizeof(PackArgs) <= 4096, "kernel arguments are limited to 4 KB");
 
 template <bool F16>
 __global__ __launch_bounds__(kPackThreads) void block_pack_kernel(PackArgs args) {
   __shared__ float red[kPackThreads / 64][8];
   unsigned b = blockIdx.x;
   for (int i = 0; i < args.n_filters; ++i) {
-    const PackFilter &fl = args.filter[i];
+    const PackFilterHead &fl = args.filter[i];
     if (b < args.rows[i]) {
       const int row = (int)(b * kPackThreads + threadIdx.x);
-      if (row < fl.nox) ((int2 *)(fl.frag + fl.rows_off))[row] = class_row(fl, row);
+      if (row < fl.nox) ((int2 *)(fl.frag + fl.rows_off))[row] = class_row(fl, args.cls + args.cls_at[i], row);
       return;
     }
     b -= args.rows[i];
@@ -211,9 +218,9 @@ size_t pack_partial_count(i64 batch, i64 channels, i64 plane) {
 }
 
 PackFilter pack_filter(const BlockPlan &pl, int channels, const void *f, void *frag, void *copy, i64 copy_count) {
-  PackFilter pf = {f, (char *)frag, copy, copy_count, pl.f_m, pl.f_c, pl.rows_off, channels, pl.wide, pl.M, pl.CG, pl.nfx, pl.nfy,
+  PackFilter pf = {{f, (char *)frag, copy, copy_count, pl.f_m, pl.f_c, pl.rows_off, channels, pl.wide, pl.M, pl.CG, pl.nfx, pl.nfy,
                    pl.f_pitch, pl.f_off, pl.m_tiles * pl.wm * pl.mt, pl.kind_x, pl.nox, pl.ngx, pl.sx, pl.dx, pl.px, pl.ux, pl.mg_p1,
-                   pl.n_classes, pl.cls_stride, {}};
+                    pl.n_classes, pl.cls_stride}, {}};
   std::copy(pl.cls, pl.cls + kBlockClasses, pf.cls);
   return pf;
 }
@@ -223,16 +230,21 @@ hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b,
   PackArgs args = {};
   if (!pack_part(a, args.a) || !pack_part(b, args.b)) return hipErrorInvalidValue;
   do {
-    args.n_filters = std::min(n_filters, kPackFilters);
     unsigned blocks = args.a.blocks + args.b.blocks;
-    for (int i = 0; i < args.n_filters; ++i) {
-      const PackFilter &fl = args.filter[i] = filters[i];
+    int i = 0, classes = 0;
+    for (; i < std::min(n_filters, kPackFilters) && classes + filters[i].n_classes <= kPackClasses; ++i) {
+      const PackFilter &fl = filters[i];
+      args.filter[i] = fl;
+      args.cls_at[i] = (short)classes;
+      std::copy(fl.cls, fl.cls + fl.n_classes, args.cls + classes);
+      classes += fl.n_classes;
       const i64 units = (i64)fl.tiles * ((i64)fl.CG * fl.nfx * fl.nfy + 1) * 32;
       args.fragments[i] = (unsigned)((units + kPackThreads - 1) / kPackThreads);
       args.rows[i] = fl.kind_x == AX_MCORR || fl.kind_x == AX_MCONV ? (unsigned)((fl.nox + kPackThreads - 1) / kPackThreads) : 0;
       args.copies[i] = fl.copy ? (unsigned)((fl.copy_count + 4 * kPackThreads - 1) / (4 * kPackThreads)) : 0;
       blocks += args.rows[i] + args.fragments[i] + args.copies[i];
     }
+    args.n_filters = i;
     if (blocks) {
       if (f16) hipLaunchKernelGGL(block_pack_kernel<true>, dim3(blocks), dim3(kPackThreads), 0, stream, args);
       else hipLaunchKernelGGL(block_pack_kernel<false>, dim3(blocks), dim3(kPackThreads), 0, stream, args);

@@ -210,6 +210,10 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   // adds up.  Measured on this chip, and rounded:
   //   a step's matrix instructions at 55-80 % of their rate (larger tiles: the higher; 128 channels x 128 positions of two by
   //   two wavefronts measure that of 64 x 512), shared by a CU's workgroups;
+  //   -- all but wavefronts that share a tile, two workgroups of which in a single turn take 1.5 of one's time: one's
+  //   fragments come too late for its next step (256 -> 256 channels, 4 x 4 taps, one utterance of 337 x 5, in two slices: 35
+  //   -> 24 us and 5 for the sums; taken everywhere 46 drawn passes change, and take 1.04 of their time, 0.80 to 1.45; 1.2 for
+  //   1.5: seven, 1.01);
   //   a stage at least 4000 (the latency of its loads);
   //   per tile 5000 for its tables (9000 where wavefronts share it in fp32: nothing runs under them) and its output at 9
   //   bytes a cycle; 9000 for a launch's start, as much for the kernel that adds the slices, and 2400 bytes a cycle for
@@ -231,7 +235,7 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
     const double tile = pl.wk > 1 && !f16 ? 9000 : 5000;
     auto turns_cost = [&](i64 items, double stages) {
       const i64 full = items / per_m, left = items - full * per_m;
-      auto turn = [&](i64 n) { return stages * std::max(4000.0, steps * (n * pl.m_tiles > slots / 2 ? 2 : 1)) + tile + output; };
+      auto turn = [&](i64 n) { return stages * std::max(4000.0, steps * (n * pl.m_tiles > slots / 2 ? pl.wk > 1 && full == 0 ? 1.5 : 2 : 1)) + tile + output; };
       return full * turn(per_m) + (left ? turn(left) : 0);
     };
     double best = 9000 + turns_cost(total, c_stages * subsets);

@@ -201,14 +201,26 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   const int wk = WK > 1 ? wave : 0, wm = WM > 1 ? wave & (WM - 1) : 0, wn = WK > 1 ? 0 : wave / WM;
   const bool mellin_x = JOINT || pl.kind_x == AX_MCORR || pl.kind_x == AX_MCONV;
   const int taps = pl.nfx * pl.nfy;
-  const int m_tile = blockIdx.y;
+  const int items = pl.whole + pl.rest * pl.slices;
+  // Wavefronts that share a tile, 2, 4 or 8 tiles of channels: XCD k (workgroups k, k + 8, ...) takes one of those, and its
+  // share of the filter is all that the XCD's L2 sees: one utterance of a Mellin stack, layers of 128 to 256 channels on 337 x
+  // 10 and 337 x 5, 16.9, 17.9, 26.2 and 36.2 us -> 15.9, 16.8, 24.5 and 35.3.  (Filters below 1 MB: nothing gained; 48
+  // channels on one axis 84.2 -> 86.0 us a step.)  The position tiles are dealt to a tile of channels' XCDs in turn: those of a
+  // class with many filter rows follow each other, and an eighth of all tiles without a gap left XCDs waiting (113 us).
+  int m_tile = blockIdx.y, item = blockIdx.x;
+  if constexpr (WK > 1)
+    if (gridDim.y != (unsigned)pl.m_tiles) {
+      const int xcd = item & 7, each = 8 / pl.m_tiles;
+      m_tile = xcd / each;
+      item = (item >> 3) * each + xcd - m_tile * each;
+      if (item >= items) return;
+    }
   const unsigned zero_frag = (unsigned)(pl.CG * taps * PARTS * 512);       // the tile's fragment of zeros, behind the others
   const unsigned af_tile = zero_frag + PARTS * 512;                        // bytes of 32 channels' fragments
   const char *AFm = AF + (i64)(m_tile * WM + wm) * MT * af_tile, *AFm1 = AFm + af_tile;
   const i64 plane_bytes = (i64)(pl.plane + 1) * UB;
   const unsigned lds0 = lds_address((const float *)blk_lds);
-  const int items = pl.whole + pl.rest * pl.slices;
-  const int my_tiles = (items - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int my_tiles = WK > 1 ? 1 : (items - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
 
   if (tid < M_T) {
     const int m = m_tile * M_T + tid;
@@ -348,7 +360,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       for (int pt = 0; pt < PARTS; ++pt) o.a[k][pt] = *(const uintx4 *)((k ? AFm1 : AFm) + off + pt * 512);
   };
 
-  BlockTile tg = block_tile<P, JOINT>(pl, rows, (int)blockIdx.x, mellin_x), next_tg = tg;
+  BlockTile tg = block_tile<P, JOINT>(pl, rows, item, mellin_x), next_tg = tg;
   if (my_tiles <= 0) return;
   int n_ents = build_tile(tg, 0, nullptr), next_ents = n_ents;
   __syncthreads();
@@ -534,7 +546,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       const bool as_half = F16 && !BLOCKED && whole;
       const int ES = as_half ? 2 : 4, h_m = (whole ? (int)pl.h_m : P) * ES;
       char *base = whole ? (char *)Hv + ((i64)tg.n * pl.h_n + (i64)m0 * (int)pl.h_m) * ES
-                         : (char *)(sums + (((i64)tg.slot * gridDim.y + m_tile) * M_T + wm * MT * 32) * P);
+                         : (char *)(sums + (((i64)tg.slot * pl.m_tiles + m_tile) * M_T + wm * MT * 32) * P);
       const __amdgpu_buffer_rsrc_t rsrc =
           BLOCKED && whole ? __builtin_amdgcn_make_buffer_rsrc((char *)Hv + tg.n * image_bytes, 0, all_images, 0x00020000)
                            : __builtin_amdgcn_make_buffer_rsrc(base, 0, max(0, min(MT * 32, pl.M - m0)) * h_m + (whole && JOINT ? (pl.batch - 1) * (int)pl.h_n * ES : 0), 0x00020000);
@@ -734,7 +746,10 @@ hipError_t launch_joint(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t
   static std::atomic<int> lds_allowed{0};
   hipError_t e = allow_large_lds((const void *)kern, pl.lds_bytes, lds_allowed);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)pl.grid_x, (unsigned)pl.m_tiles), dim3(kThreads), pl.lds_bytes, stream, pl,
+  dim3 grid((unsigned)pl.grid_x, (unsigned)pl.m_tiles);
+  if (WK > 1 && (pl.m_tiles == 2 || pl.m_tiles == 4 || pl.m_tiles == 8) && pl.filter_bytes >= (size_t)1 << 20)   // by XCD: see the kernel
+    grid = dim3((unsigned)((pl.grid_x + 8 / pl.m_tiles - 1) / (8 / pl.m_tiles) * 8));
+  hipLaunchKernelGGL(kern, grid, dim3(kThreads), pl.lds_bytes, stream, pl,
                      (const char *)a.signal, (const char *)a.frag, a.bias, a.out, a.sums, (const char *)a.mask, a.chan_sums);
   return hipGetLastError();
 }

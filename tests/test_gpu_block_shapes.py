@@ -60,3 +60,23 @@ def test_tile_shapes_match_checker(case, half):
             assert np.all(err <= 2.0 ** -10 * np.abs(ref) + 2e-5 * fan ** 0.5), what
         else:
             assert_close(got, ref, fan, what)
+
+
+@pytest.mark.parametrize("case", [
+    # several tiles of channels dealt to the XCDs: two, four and eight of them, position tiles that do not divide evenly; two
+    # workgroups a CU by slices
+    ("mcorr", 1, 256, 128, (4, 4), (61, 5), (1, 1), (1, 1), (1, 1), (31, 2)),
+    ("mcorr", 1, 256, 256, (4, 4), (337, 5), (1, 1), (1, 1), (1, 1), (169, 2)),
+    ("lcorr", 1, 128, 512, (3, 3), (30, 9), (1, 1), (1, 1), (1, 1), (1, 1)),
+    ("lcorr", 1, 128, 450, (3, 3), (7, 5), (1, 1), (1, 1), (1, 1), (1, 1)),
+], ids=str)
+def test_channel_tiles_by_xcd_match_checker(case):
+    op, n, c_in, c_out, nf, ng, s, d, p, r = case
+    rng = np.random.default_rng(7400 + c_out)
+    x = rng.standard_normal((n, c_in) + ng).astype(np.float32)
+    w = (rng.standard_normal((c_out, c_in) + nf) * (c_in * nf[0] * nf[1]) ** -0.5).astype(np.float32)
+    fwd = oracle.mcorrlcorr if op == "mcorr" else oracle.lcorrlcorr
+    exp = fwd(x.astype(np.float64), w.astype(np.float64), None, s, d, p, (1, 1), r)
+    out = (mconv._ext_mcorrlcorr if op == "mcorr" else mconv._ext_lcorrlcorr)(to_gpu(x), to_gpu(w), None, s, d, p, (1, 1), r)
+    assert hip.last_variant() == "mfma-blocks"
+    assert_close(out, exp, c_in * nf[0] * nf[1], "out")

@@ -16,15 +16,19 @@ constexpr int kFinishThreads = 256;
 constexpr int kFinishTaps = 64;
 constexpr int kSliceValues = kFinishThreads * 4;       // values of a tile that a block adds up
 
-struct FinishArgs {
-  int n_weights, n_biases;
-  WeightSums w[kFinishJobs];
-  BiasSums b[kFinishJobs];
+// (JOBS: 1 or kFinishJobs: a layer's launch does not carry a stack's arguments; measured at kPackFilters)
+struct SliceSums {
   BlockPlan s;
   BlockGemmArgs sa;
   const int2 *s_rows;
 };
-static_assert(sizeof(FinishArgs) <= 4096, "kernel arguments are limited to 4 KB");
+template <int JOBS>
+struct FinishArgs : SliceSums {
+  int n_weights, n_biases;
+  WeightSums w[JOBS];
+  BiasSums b[JOBS];
+};
+static_assert(sizeof(FinishArgs<kFinishJobs>) <= 4096, "kernel arguments are limited to 4 KB");
 
 // p[0] + p[step] + .. + p[(count - 1) step], added to `s` in that order.  Eight loads are on their way at a time: a sum is a
 // chain of trips to memory, and with one or four the sums of a few channels over an image's many tiles took 20-27 us a
@@ -108,7 +112,7 @@ __device__ void finish_weight_taps(const WeightSums &pl, int b, float (*sum)[33]
 // Tiles in slices whose output is blocked or passes a ReLU: a thread makes a unit (eight channels of a position); a block
 // has 256 of a tile's, the positions side by side.
 template <typename T>
-__device__ void finish_units(const FinishArgs &a, int b, float (*red)[32]) {
+__device__ void finish_units(const SliceSums &a, int b, float (*red)[32]) {
   constexpr bool F16 = sizeof(T) == 2;
   constexpr int UB = F16 ? 16 : 48;
   const BlockPlan &pl = a.s;
@@ -194,8 +198,8 @@ __device__ void finish_units(const FinishArgs &a, int b, float (*red)[32]) {
   }
 }
 
-template <typename T, typename TG>                     // tensors, gradients of the parameters
-__global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs a) {
+template <typename T, typename TG, int JOBS>           // tensors, gradients of the parameters
+__global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs<JOBS> a) {
   __shared__ float red[8][32], taps[kFinishTaps][33];
   const int tid = threadIdx.x;
   unsigned b = blockIdx.x;
@@ -276,8 +280,9 @@ void BlockFinish::add_weight(const BlockWgradPlan &pl, const void *partial, void
   if (pl.nfy != pl.f_pitch) w.zero_blocks = (unsigned)(((i64)pl.M * pl.C * pl.nfx * pl.f_pitch + kFinishThreads - 1) / kFinishThreads);
 }
 
-hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipStream_t stream) {
-  FinishArgs a = {};
+template <int JOBS>
+static hipError_t launch_finish(bool f16, bool wide, const BlockFinish &job, hipStream_t stream) {
+  FinishArgs<JOBS> a = {};
   i64 blocks = 0;
   a.n_weights = job.n_weights;
   a.n_biases = job.n_biases;
@@ -301,10 +306,14 @@ hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipS
   blocks += s_blocks;
   if (blocks == 0) return hipSuccess;
   const dim3 grid((unsigned)blocks), threads(kFinishThreads);
-  if (f16 && wide) hipLaunchKernelGGL((block_finish_kernel<_Float16, float>), grid, threads, 0, stream, a);
-  else if (f16) hipLaunchKernelGGL((block_finish_kernel<_Float16, _Float16>), grid, threads, 0, stream, a);
-  else hipLaunchKernelGGL((block_finish_kernel<float, float>), grid, threads, 0, stream, a);
+  if (f16 && wide) hipLaunchKernelGGL((block_finish_kernel<_Float16, float, JOBS>), grid, threads, 0, stream, a);
+  else if (f16) hipLaunchKernelGGL((block_finish_kernel<_Float16, _Float16, JOBS>), grid, threads, 0, stream, a);
+  else hipLaunchKernelGGL((block_finish_kernel<float, float, JOBS>), grid, threads, 0, stream, a);
   return hipGetLastError();
+}
+
+hipError_t launch_block_finish(bool f16, bool wide, const BlockFinish &job, hipStream_t stream) {
+  return job.n_weights <= 1 && job.n_biases <= 1 ? launch_finish<1>(f16, wide, job, stream) : launch_finish<kFinishJobs>(f16, wide, job, stream);
 }
 
 }  // namespace mellin

@@ -204,8 +204,8 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   const int items = pl.whole + pl.rest * pl.slices;
   // Wavefronts that share a tile, 2, 4 or 8 tiles of channels: XCD k (workgroups k, k + 8, ...) takes one of those, and its
   // share of the filter is all that the XCD's L2 sees: one utterance of a Mellin stack, layers of 128 to 256 channels on 337 x
-  // 10 and 337 x 5, 16.9, 17.9, 26.2 and 36.2 us -> 15.9, 16.8, 24.5 and 35.3.  (Filters below 1 MB: nothing gained; 48
-  // channels on one axis 84.2 -> 86.0 us a step.)  The position tiles are dealt to a tile of channels' XCDs in turn: those of a
+  // 10 and 337 x 5, 16.9, 17.9, 26.2 and 36.2 us -> 15.9, 16.8, 24.5 and 35.3.  (Filters below 1 MB: nothing gained;
+  // 41 -> 128 channels on one axis 84.2 -> 86.0 us a step.)  The position tiles are dealt to a tile of channels' XCDs in turn: those of a
   // class with many filter rows follow each other, and an eighth of all tiles without a gap left XCDs waiting (113 us).
   int m_tile = blockIdx.y, item = blockIdx.x;
   if constexpr (WK > 1)

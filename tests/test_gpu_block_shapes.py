@@ -69,8 +69,12 @@ def test_tile_shapes_match_checker(case, half):
     ("mcorr", 1, 256, 256, (4, 4), (337, 5), (1, 1), (1, 1), (1, 1), (169, 2)),
     ("lcorr", 1, 128, 512, (3, 3), (30, 9), (1, 1), (1, 1), (1, 1), (1, 1)),
     ("lcorr", 1, 128, 450, (3, 3), (7, 5), (1, 1), (1, 1), (1, 1), (1, 1)),
+    # tiles of 32 channels for an odd number of them
+    ("lcorr", 2, 64, 67, (4, 4), (60, 40), (1, 1), (1, 1), (1, 1), (1, 1)),
+    ("mcorr", 1, 96, 160, (3, 3), (50, 20), (1, 1), (1, 1), (1, 1), (25, 1)),
+    ("lcorr", 24, 48, 90, (3, 3), (60, 40), (1, 1), (1, 1), (1, 1), (1, 1)),
 ], ids=str)
-def test_channel_tiles_by_xcd_match_checker(case):
+def test_channel_tiles_match_checker(case):
     op, n, c_in, c_out, nf, ng, s, d, p, r = case
     rng = np.random.default_rng(7400 + c_out)
     x = rng.standard_normal((n, c_in) + ng).astype(np.float32)

@@ -278,17 +278,17 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   const bool can_join = mellin && masks && pl.batch > 1 && Q * pl.batch < lim && (i64)pl.batch * pl.CG * (plane + 1) * unit_bytes < most &&
                         (i64)pl.batch * pl.out_groups * (Q + 1) * unit_bytes < most && (i64)pl.batch * pl.M * Q * 4 < most &&
                         pl.h_n == (i64)pl.M * Q;
-  // Tiles of 32 channels are tried as well where those of 64 leave half of the last one empty (65 to 96 channels, 129 to
-  // 160, ..): 28 passes of 400 drawn layers take them, in 0.92 of the time in the geometric mean (0.82 to 0.99).  Everywhere 178
-  // passes did, in 0.96 (0.70 to 1.20).
+  // Tiles of 32 channels are tried as well: where those of 64 leave half of the last one empty (65 to 96 channels, 129 to 160,
+  // ..) they are taken like any other (28 passes of 400 drawn layers, 0.92 of the time in the geometric mean, 0.82 to 0.99),
+  // elsewhere if the model gains a seventh (8 passes on few workgroups, 0.95, 0.91 to 1.00; with any gain 150, 0.97, 0.70 to 1.20).
   const int mt = pl.mt;
-  const bool odd = mt == 2 && (pr.c_out + 31) / 32 % 2 == 1;
+  const double narrow = (pr.c_out + 31) / 32 % 2 == 1 ? 1 : 0.85;
   BlockPlan best_plan;
   double best_cost = 0;
   for (int joint = 0; joint <= (can_join ? 1 : 0); ++joint) {
     double limit = joint && best_cost > 0 ? 0.9 * best_cost : 0;
     set_joint(joint);
-    for (pl.mt = mt; pl.mt >= (odd ? 1 : mt); --pl.mt)
+    for (pl.mt = mt; pl.mt >= 1; --pl.mt)
       for (const auto &sh : shapes) {
         if (pl.mt < mt && sh[1] == 2) continue;
         if (f16 ? sh[0] == 2 && sh[1] == 2 : sh[0] == 4 || (sh[0] == 2 && sh[2] == 4)) continue;
@@ -296,7 +296,7 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
         if (!shape(sh[0], sh[1], sh[2])) continue;
         const double c = cost();
         if (!f16 && sh[1] == 2 && ((i64)pl.whole + (i64)pl.rest * pl.slices) * pl.m_tiles <= slots / 2) continue;
-        if (limit == 0 || c < limit) { limit = best_cost = c; best_plan = pl; }
+        if (limit == 0 || c < (pl.mt < mt ? narrow : 1) * limit) { limit = best_cost = c; best_plan = pl; }
       }
   }
   if (best_cost == 0) return false;

@@ -71,6 +71,8 @@ for _t in ("f32", "f16"):
     SYMBOLS["mellin_pool_pairs_backward_" + _t] = (_int, [_ptr, _ptr, _i64, _i64, _ptr, _ptr])
 SYMBOLS["mellin_log_lift_forward_logs_f32"] = (_int, [_ptr, _ptr, _ptr, _int, _i64, _i64, _i64, _ptr, _ptr])
 SYMBOLS["mellin_log_lift_backward_logs_f32"] = (_int, [_ptr] * 4 + [_int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _size_t, _ptr])
+SYMBOLS["mellin_log_lift_forward_keep_f32"] = (_int, [_ptr, _ptr, _ptr, _int, _i64, _i64, _i64, _ptr, _ptr, _ptr])
+SYMBOLS["mellin_log_lift_backward_kept_f32"] = (_int, [_ptr] * 3 + [_int, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _size_t, _ptr])
 SYMBOLS["mellin_pack_windows_f32"] = (_int, [_ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr])
 SYMBOLS["mellin_static_scratch_bytes"] = (_size_t, [])
 SYMBOLS["mellin_static_scratch_prepare"] = (_int, [])

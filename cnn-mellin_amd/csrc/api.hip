@@ -936,33 +936,44 @@ int check_log_lift(const char *fn, double eps, int flags, i64 outer, i64 t, i64 
 
 template <typename T>
 int log_lift_forward(const char *fn, const T *x, double eps, double tau, int flags, i64 outer, i64 t, i64 inner,
-                     T *y, void *stream, const T *eps_at = nullptr, const T *tau_at = nullptr, bool logs = false) {
+                     T *y, void *stream, const T *eps_at = nullptr, const T *tau_at = nullptr, bool logs = false,
+                     T *kept = nullptr) {
   int rc;
   if ((rc = check_log_lift(fn, eps, flags, outer, t, inner))) return rc;
   if (outer * t * inner == 0) return MELLIN_OK;
   if (!x || !y) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", fn);
   hipError_t e = launch_log_lift_forward<T>(x, (T)eps, (T)tau, flags & MELLIN_PW_LOG, flags & MELLIN_PW_LIFT,
-                                            outer, t, inner, y, (hipStream_t)stream, eps_at, tau_at, logs);
+                                            outer, t, inner, y, (hipStream_t)stream, eps_at, tau_at, logs, kept);
   if (e != hipSuccess) return fail(MELLIN_ERR_RUNTIME, "%s: %s", fn, hipGetErrorString(e));
   return MELLIN_OK;
 }
 
 template <typename T>
-int log_lift_backward(const char *fn, const T *x, const T *gy, double eps, double tau, int flags, i64 outer,
-                      i64 t, i64 inner, T *gx, T *grad_params, void *workspace, size_t workspace_bytes,
-                      void *stream, const T *eps_at = nullptr, const T *tau_at = nullptr, bool logs = false) {
+int log_lift_gradients(const char *fn, const T *x, const T *gy, double eps, double tau, int flags, i64 outer,
+                      i64 t, i64 inner, T *gx, T *grad_eps, T *grad_tau, void *workspace, size_t workspace_bytes,
+                      void *stream, const T *eps_at = nullptr, const T *tau_at = nullptr, bool logs = false, bool of_logs = false) {
   int rc;
   if ((rc = check_log_lift(fn, eps, flags, outer, t, inner))) return rc;
-  if (!grad_params) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", fn);
   const size_t need = log_lift_workspace_bytes(outer, t, inner, sizeof(T));
-  if (need && (!x || !gy || (!gx && !logs))) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", fn);
+  if (need && (!x || !gy || (!gx && !of_logs))) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", fn);
   if (need && (!workspace || workspace_bytes < need))
     return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", fn, need, workspace_bytes);
   hipError_t e = launch_log_lift_backward<T>(x, gy, (T)eps, (T)tau, flags & MELLIN_PW_LOG, flags & MELLIN_PW_LIFT,
-                                             outer, t, inner, gx, grad_params, (T *)workspace,
-                                             (hipStream_t)stream, eps_at, tau_at, logs);
+                                             outer, t, inner, gx, grad_eps, grad_tau, (T *)workspace,
+                                             (hipStream_t)stream, eps_at, tau_at, logs, of_logs);
   if (e != hipSuccess) return fail(MELLIN_ERR_RUNTIME, "%s: %s", fn, hipGetErrorString(e));
   return MELLIN_OK;
+}
+// (the parameters' gradients side by side)
+template <typename T>
+int log_lift_backward(const char *fn, const T *x, const T *gy, double eps, double tau, int flags, i64 outer,
+                      i64 t, i64 inner, T *gx, T *grad_params, void *workspace, size_t workspace_bytes,
+                      void *stream, const T *eps_at = nullptr, const T *tau_at = nullptr, bool logs = false) {
+  const int rc = check_log_lift(fn, eps, flags, outer, t, inner);
+  if (rc) return rc;
+  if (!grad_params) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", fn);
+  return log_lift_gradients<T>(fn, x, gy, eps, tau, flags, outer, t, inner, gx, grad_params, grad_params + 1, workspace,
+                               workspace_bytes, stream, eps_at, tau_at, logs, logs);
 }
 
 #define CORR2D_ARGS                                                            \
@@ -1347,6 +1358,20 @@ int mellin_log_lift_backward_logs_f32(const float *x, const float *grad_y, const
   if (((flags & MELLIN_PW_LOG) && !log_eps) || ((flags & MELLIN_PW_LIFT) && !log_tau)) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
   return log_lift_backward<float>(__func__, x, grad_y, 1.0, 0.0, flags, outer, t, inner, grad_x, grad_params, workspace,
                                   workspace_bytes, stream, log_eps, log_tau, true);
+}
+// the same in two calls between which the parameters may change
+int mellin_log_lift_forward_keep_f32(const float *x, const float *log_eps, const float *log_tau, int flags, int64_t outer, int64_t t,
+                                     int64_t inner, float *y, float *params, void *stream) {
+  if (!params || ((flags & MELLIN_PW_LOG) && !log_eps) || ((flags & MELLIN_PW_LIFT) && !log_tau))
+    return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  return log_lift_forward<float>(__func__, x, 1.0, 0.0, flags, outer, t, inner, y, stream, log_eps, log_tau, true, params);
+}
+int mellin_log_lift_backward_kept_f32(const float *x, const float *grad_y, const float *params, int flags, int64_t outer, int64_t t,
+                                      int64_t inner, float *grad_x, float *grad_log_eps, float *grad_log_tau, void *workspace,
+                                      size_t workspace_bytes, void *stream) {
+  if (!params) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
+  return log_lift_gradients<float>(__func__, x, grad_y, 1.0, 0.0, flags, outer, t, inner, grad_x, grad_log_eps, grad_log_tau,
+                                   workspace, workspace_bytes, stream, params, params + 1, false, true);
 }
 int mellin_pack_windows_f32(const float *x, const int64_t *at, int64_t windows, int64_t frames, int64_t row, float *out, void *stream) {
   if (windows < 0 || frames < 0 || row < 0 || windows >= (int64_t)1 << 31 || (frames > 0 && row >= ((int64_t)1 << 31) / frames))

@@ -160,16 +160,17 @@ hipError_t launch_fold_xy(const Axis &x, const Axis &y, i64 batch_cin, int nf_pa
                           float *grad_input, hipStream_t stream);
 
 // pointwise.hip: log compression and dilation lift over x viewed as (outer, t, inner).
-// eps_at, tau_at (device memory, or null): read by the kernels instead of the arguments; logs: their logarithms, and the
-// gradients are those of the logarithms.  gx may be null.
+// eps_at, tau_at (device memory, or null): read by the kernels instead of the arguments; logs: their logarithms; kept (or
+// null): the forward pass leaves {eps, tau} there; of_logs: the gradients are those of the logarithms.  gx, and either of the
+// parameters' gradients, may be null.
 size_t log_lift_workspace_bytes(i64 outer, i64 t, i64 inner, size_t elem);
 template <typename T>
 hipError_t launch_log_lift_forward(const T *x, T eps, T tau, bool with_log, bool with_lift, i64 outer, i64 t,
-                                   i64 inner, T *y, hipStream_t stream, const T *eps_at, const T *tau_at, bool logs);
+                                   i64 inner, T *y, hipStream_t stream, const T *eps_at, const T *tau_at, bool logs, T *kept);
 template <typename T>
 hipError_t launch_log_lift_backward(const T *x, const T *gy, T eps, T tau, bool with_log, bool with_lift,
-                                    i64 outer, i64 t, i64 inner, T *gx, T *grad_params, T *workspace,
-                                    hipStream_t stream, const T *eps_at, const T *tau_at, bool logs);
+                                    i64 outer, i64 t, i64 inner, T *gx, T *grad_eps, T *grad_tau, T *workspace,
+                                    hipStream_t stream, const T *eps_at, const T *tau_at, bool logs, bool of_logs);
 // windows[k] (run 4-byte values, rows of `row`): the at[k] >> 32 rows of x from row (unsigned)at[k] on, then zeros
 hipError_t launch_pack_windows(const void *x, const i64 *at, i64 windows, int run, int row, void *out, hipStream_t stream);
 

@@ -28,10 +28,12 @@ constexpr int kPwThreads = 256;
 template <typename T> __device__ __forceinline__ T sign_of(T v) { return v > T(0) ? T(1) : (v < T(0) ? T(-1) : T(0)); }
 
 // eps and tau where they live on the device (null: the kernel's arguments); logs: their logarithms, as the modules' parameters
-// are (two launches of exp, and as many in the backward pass, on one value each)
+// are (two launches of exp, and as many in the backward pass, on one value each); of_logs: a backward pass's gradients are those
+// of the logarithms.  kept: where a forward pass leaves {eps, tau}, for a backward pass that parameters may have changed before.
 template <typename T> struct LiftParams {
   const T *eps, *tau;
-  int logs;
+  int logs, of_logs;
+  T *kept;
   __device__ __forceinline__ void read(T &e, T &t) const {
     if (eps) e = logs ? exp(*eps) : *eps;
     if (tau) t = logs ? exp(*tau) : *tau;
@@ -45,6 +47,7 @@ __global__ __launch_bounds__(kPwThreads) void log_lift_forward_kernel(
   const i64 col = (i64)blockIdx.x * kPwThreads + threadIdx.x;      // t * inner + i
   if (col >= plane) return;
   params.read(eps, tau);
+  if (params.kept && col == 0 && blockIdx.y == 0) { params.kept[0] = eps; params.kept[1] = tau; }
   T p = T(1);
   if (LIFT) p = pow((T)(col / inner + 1), tau);
   const i64 n0 = (i64)blockIdx.y * rows_per_block, n1 = min(outer, n0 + rows_per_block);
@@ -105,11 +108,12 @@ __global__ __launch_bounds__(kPwThreads) void log_lift_backward_kernel(
   }
 }
 
-// grad_params[0 .. 1] = sums of the partials, in index order (one wavefront:
+// *grad_eps, *grad_tau (null: not wanted) = sums of the partials, in index order (one wavefront:
 // lane l adds partials l, l + 64, ..., then a fixed shuffle tree)
 template <typename T>
 __global__ __launch_bounds__(64) void log_lift_reduce_kernel(const T *__restrict__ partial, i64 blocks,
-                                                             T *__restrict__ grad_params, LiftParams<T> params) {
+                                                             T *__restrict__ grad_eps, T *__restrict__ grad_tau,
+                                                             LiftParams<T> params) {
   T a = T(0), b = T(0);
   for (i64 i = threadIdx.x; i < blocks; i += 64) { a += partial[2 * i]; b += partial[2 * i + 1]; }
 #pragma unroll
@@ -118,14 +122,14 @@ __global__ __launch_bounds__(64) void log_lift_reduce_kernel(const T *__restrict
     b += __shfl_down(b, o);
   }
   if (threadIdx.x == 0) {
-    if (params.logs) {                                     // d/d log v = v d/d v
+    if (params.of_logs) {                                  // d/d log v = v d/d v
       T eps = T(0), tau = T(0);
       params.read(eps, tau);
       a *= eps;
       b *= tau;
     }
-    grad_params[0] = a;
-    grad_params[1] = b;
+    if (grad_eps) *grad_eps = a;
+    if (grad_tau) *grad_tau = b;
   }
 }
 
@@ -152,12 +156,12 @@ size_t log_lift_workspace_bytes(i64 outer, i64 t, i64 inner, size_t elem) {
 
 template <typename T>
 hipError_t launch_log_lift_forward(const T *x, T eps, T tau, bool with_log, bool with_lift, i64 outer, i64 t,
-                                   i64 inner, T *y, hipStream_t stream, const T *eps_at, const T *tau_at, bool logs) {
+                                   i64 inner, T *y, hipStream_t stream, const T *eps_at, const T *tau_at, bool logs, T *kept) {
   if (outer <= 0 || t <= 0 || inner <= 0) return hipSuccess;
   dim3 grid;
   i64 rpb;
   shape_grid(outer, t * inner, grid, rpb);
-  const LiftParams<T> params = {eps_at, tau_at, logs};
+  const LiftParams<T> params = {eps_at, tau_at, logs, 0, kept};
 #define MELLIN_PW_FWD(L_, F_)                                                                    \
   hipLaunchKernelGGL((log_lift_forward_kernel<T, L_, F_>), grid, dim3(kPwThreads), 0, stream, x, \
                      eps, tau, params, outer, t * inner, inner, rpb, y)
@@ -170,11 +174,11 @@ hipError_t launch_log_lift_forward(const T *x, T eps, T tau, bool with_log, bool
 
 template <typename T>
 hipError_t launch_log_lift_backward(const T *x, const T *gy, T eps, T tau, bool with_log, bool with_lift,
-                                    i64 outer, i64 t, i64 inner, T *gx, T *grad_params, T *workspace,
-                                    hipStream_t stream, const T *eps_at, const T *tau_at, bool logs) {
-  const LiftParams<T> params = {eps_at, tau_at, logs};
+                                    i64 outer, i64 t, i64 inner, T *gx, T *grad_eps, T *grad_tau, T *workspace,
+                                    hipStream_t stream, const T *eps_at, const T *tau_at, bool logs, bool of_logs) {
+  const LiftParams<T> params = {eps_at, tau_at, logs, of_logs, nullptr};
   if (outer <= 0 || t <= 0 || inner <= 0) {
-    hipLaunchKernelGGL((log_lift_reduce_kernel<T>), dim3(1), dim3(64), 0, stream, workspace, (i64)0, grad_params, params);
+    hipLaunchKernelGGL((log_lift_reduce_kernel<T>), dim3(1), dim3(64), 0, stream, workspace, (i64)0, grad_eps, grad_tau, params);
     return hipGetLastError();
   }
   dim3 grid;
@@ -190,7 +194,7 @@ hipError_t launch_log_lift_backward(const T *x, const T *gy, T eps, T tau, bool 
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((log_lift_reduce_kernel<T>), dim3(1), dim3(64), 0, stream, workspace,
-                     (i64)grid.x * grid.y, grad_params, params);
+                     (i64)grid.x * grid.y, grad_eps, grad_tau, params);
   return hipGetLastError();
 }
 
@@ -480,12 +484,13 @@ hipError_t launch_cast_pair(bool to_half, const void *a, void *to_a, i64 na, con
 }
 
 template hipError_t launch_log_lift_forward<float>(const float *, float, float, bool, bool, i64, i64, i64, float *, hipStream_t,
-                                                   const float *, const float *, bool);
+                                                   const float *, const float *, bool, float *);
 template hipError_t launch_log_lift_forward<double>(const double *, double, double, bool, bool, i64, i64, i64, double *, hipStream_t,
-                                                    const double *, const double *, bool);
+                                                    const double *, const double *, bool, double *);
 template hipError_t launch_log_lift_backward<float>(const float *, const float *, float, float, bool, bool, i64, i64, i64, float *,
-                                                    float *, float *, hipStream_t, const float *, const float *, bool);
+                                                    float *, float *, float *, hipStream_t, const float *, const float *, bool, bool);
 template hipError_t launch_log_lift_backward<double>(const double *, const double *, double, double, bool, bool, i64, i64, i64, double *,
-                                                     double *, double *, hipStream_t, const double *, const double *, bool);
+                                                     double *, double *, double *, hipStream_t, const double *, const double *, bool,
+                                                     bool);
 
 }  // namespace mellin

@@ -455,41 +455,42 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
-// The gradients of LogCompressionLift.
+// The gradients of LogCompressionLift, at the eps and tau of the forward call, which it left in `params_`: the parameters
+// themselves may be another step's by now (a second loss whose graph is older than the step).
 struct LogLiftBackward : public torch::autograd::Node {
-  torch::autograd::SavedVariable input_, log_eps_, log_tau_;
+  torch::autograd::SavedVariable input_, params_;
+  at::DimVector eps_sizes, tau_sizes;
   int64_t outer = 0, t = 0, inner = 0;
 
   std::string name() const override { return "LogLiftBackward"; }
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
     input_.reset_data();
-    log_eps_.reset_data();
-    log_tau_.reset_data();
+    params_.reset_data();
   }
 
   torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
     at::AutoGradMode no_grad(false);
-    Tensor input, log_eps, log_tau;
+    Tensor input, params;
     {
       std::lock_guard<std::mutex> lock(mutex_);
       input = input_.unpack();
-      log_eps = log_eps_.unpack();
-      log_tau = log_tau_.unpack();
+      params = params_.unpack();
     }
     if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
     const Tensor grad = grads[0].contiguous();
     const c10::OptionalDeviceGuard guard(input.device());
-    Tensor grad_input, params = at::empty({2}, input.options());
+    Tensor grad_input, grad_params = at::empty({2}, input.options());
     if (task_should_compute_output(0)) grad_input = at::empty_like(input, at::MemoryFormat::Contiguous);
     const size_t need = mellin_log_lift_backward_workspace(4, outer, t, inner);
     Tensor ws = scratch(input, need);
-    check(mellin_log_lift_backward_logs_f32((const float *)pointer(input), (const float *)pointer(grad), (const float *)pointer(log_eps),
-                                            (const float *)pointer(log_tau), MELLIN_PW_LOG | MELLIN_PW_LIFT, outer, t, inner,
-                                            grad_input.defined() ? (float *)grad_input.data_ptr() : nullptr, (float *)params.data_ptr(),
-                                            ws.defined() ? ws.data_ptr() : nullptr, need, launch_stream(input)));
-    return {grad_input, task_should_compute_output(1) ? params.select(0, 0).view(log_eps.sizes()) : Tensor(),
-            task_should_compute_output(2) ? params.select(0, 1).view(log_tau.sizes()) : Tensor()};
+    check(mellin_log_lift_backward_kept_f32((const float *)pointer(input), (const float *)pointer(grad), (const float *)pointer(params),
+                                            MELLIN_PW_LOG | MELLIN_PW_LIFT, outer, t, inner,
+                                            grad_input.defined() ? (float *)grad_input.data_ptr() : nullptr, (float *)grad_params.data_ptr(),
+                                            (float *)grad_params.data_ptr() + 1, ws.defined() ? ws.data_ptr() : nullptr, need,
+                                            launch_stream(input)));
+    return {grad_input, task_should_compute_output(1) ? grad_params.select(0, 0).view(eps_sizes) : Tensor(),
+            task_should_compute_output(2) ? grad_params.select(0, 1).view(tau_sizes) : Tensor()};
   }
 };
 
@@ -511,20 +512,23 @@ PyObject *log_lift(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     int64_t outer = 1, inner = 1;
     for (int64_t i = 0; i < input0.dim(); ++i) (i < dim ? outer : inner) *= i == dim ? 1 : input0.size(i);
     const int64_t t = input0.size(dim);
-    Tensor input;
+    Tensor input, params;
     {
       at::AutoGradMode no_grad(false);
       input = input0.contiguous();
       out = at::empty_like(input, at::MemoryFormat::Contiguous);
-      check(mellin_log_lift_forward_logs_f32((const float *)pointer(input), (const float *)pointer(log_eps), (const float *)pointer(log_tau),
-                                             MELLIN_PW_LOG | MELLIN_PW_LIFT, outer, t, inner, (float *)out.data_ptr(), launch_stream(input)));
+      params = at::empty({2}, input.options());
+      check(mellin_log_lift_forward_keep_f32((const float *)pointer(input), (const float *)pointer(log_eps), (const float *)pointer(log_tau),
+                                             MELLIN_PW_LOG | MELLIN_PW_LIFT, outer, t, inner, (float *)out.data_ptr(),
+                                             (float *)params.data_ptr(), launch_stream(input)));
     }
     if (differentiable) {
       auto node = std::shared_ptr<LogLiftBackward>(new LogLiftBackward(), torch::autograd::deleteNode);
       node->set_next_edges(torch::autograd::collect_next_edges(input0, log_eps, log_tau));
       node->input_ = torch::autograd::SavedVariable(input, false);
-      node->log_eps_ = torch::autograd::SavedVariable(log_eps, false);
-      node->log_tau_ = torch::autograd::SavedVariable(log_tau, false);
+      node->params_ = torch::autograd::SavedVariable(params, false);
+      node->eps_sizes = at::DimVector(log_eps.sizes());
+      node->tau_sizes = at::DimVector(log_tau.sizes());
       node->outer = outer;
       node->t = t;
       node->inner = inner;

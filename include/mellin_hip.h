@@ -375,6 +375,16 @@ int mellin_log_lift_backward_logs_f32(const float *x, const float *grad_y,
                                       float *grad_params, void *workspace,
                                       size_t workspace_bytes, void *stream);
 
+/* The same for two calls between which the parameters may change: forward also leaves params = {eps, tau} in device memory, and
+ * backward takes those.  grad_x and either gradient may be null; the gradients lie wherever the caller wants them. */
+int mellin_log_lift_forward_keep_f32(const float *x, const float *log_eps, const float *log_tau,
+                                     int flags, int64_t outer, int64_t t, int64_t inner,
+                                     float *y, float *params, void *stream);
+int mellin_log_lift_backward_kept_f32(const float *x, const float *grad_y, const float *params,
+                                      int flags, int64_t outer, int64_t t, int64_t inner,
+                                      float *grad_x, float *grad_log_eps, float *grad_log_tau,
+                                      void *workspace, size_t workspace_bytes, void *stream);
+
 /* Windows of a feature batch x, rows of `row` values: out (windows, frames, row), window k being the at[k] >> 32 rows from row
  * (uint32_t)at[k] of x on, and zeros behind those (models.py:395-411: windows that reach past the batch's last frame are
  * padded).  `at`, in device memory, comes from the caller and is not checked. */

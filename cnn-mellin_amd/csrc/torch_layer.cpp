@@ -480,17 +480,20 @@ struct LogLiftBackward : public torch::autograd::Node {
     if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
     const Tensor grad = grads[0].contiguous();
     const c10::OptionalDeviceGuard guard(input.device());
-    Tensor grad_input, grad_params = at::empty({2}, input.options());
+    // (gradients become .grad as they are: each has memory of its own)
+    Tensor grad_input, grad_eps, grad_tau;
+    if (task_should_compute_output(1)) grad_eps = at::empty(eps_sizes, input.options());
+    if (task_should_compute_output(2)) grad_tau = at::empty(tau_sizes, input.options());
     if (task_should_compute_output(0)) grad_input = at::empty_like(input, at::MemoryFormat::Contiguous);
     const size_t need = mellin_log_lift_backward_workspace(4, outer, t, inner);
     Tensor ws = scratch(input, need);
     check(mellin_log_lift_backward_kept_f32((const float *)pointer(input), (const float *)pointer(grad), (const float *)pointer(params),
                                             MELLIN_PW_LOG | MELLIN_PW_LIFT, outer, t, inner,
-                                            grad_input.defined() ? (float *)grad_input.data_ptr() : nullptr, (float *)grad_params.data_ptr(),
-                                            (float *)grad_params.data_ptr() + 1, ws.defined() ? ws.data_ptr() : nullptr, need,
-                                            launch_stream(input)));
-    return {grad_input, task_should_compute_output(1) ? grad_params.select(0, 0).view(eps_sizes) : Tensor(),
-            task_should_compute_output(2) ? grad_params.select(0, 1).view(tau_sizes) : Tensor()};
+                                            grad_input.defined() ? (float *)grad_input.data_ptr() : nullptr,
+                                            grad_eps.defined() ? (float *)grad_eps.data_ptr() : nullptr,
+                                            grad_tau.defined() ? (float *)grad_tau.data_ptr() : nullptr,
+                                            ws.defined() ? ws.data_ptr() : nullptr, need, launch_stream(input)));
+    return {grad_input, grad_eps, grad_tau};
   }
 };
 

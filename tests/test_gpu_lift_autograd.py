@@ -27,3 +27,11 @@ def test_gradients_are_those_of_the_forward_call(through):
     got = torch.autograd.grad(ya, (xa, module.log_eps, module.log_tau), grad)
     want = torch.autograd.grad(yb, (xb, module.log_eps, module.log_tau), grad)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_gradients_have_memory_of_their_own():
+    module, x, grad = _module_and_data()
+    module(x).backward(grad)
+    a, b = module.log_eps.grad, module.log_tau.grad
+    assert a.untyped_storage().data_ptr() != b.untyped_storage().data_ptr()
+    assert a.untyped_storage().nbytes() == b.untyped_storage().nbytes() == 4

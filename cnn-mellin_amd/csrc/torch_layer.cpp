@@ -477,8 +477,7 @@ struct LogLiftBackward : public torch::autograd::Node {
       input = input_.unpack();
       params = params_.unpack();
     }
-    if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
-    const Tensor grad = grads[0].contiguous();
+    const Tensor grad = grads[0].defined() ? grads[0].contiguous() : at::zeros(input.sizes(), input.options());
     const c10::OptionalDeviceGuard guard(input.device());
     // (gradients become .grad as they are: each has memory of its own)
     Tensor grad_input, grad_eps, grad_tau;

@@ -35,3 +35,21 @@ def test_gradients_have_memory_of_their_own():
     a, b = module.log_eps.grad, module.log_tau.grad
     assert a.untyped_storage().data_ptr() != b.untyped_storage().data_ptr()
     assert a.untyped_storage().nbytes() == b.untyped_storage().nbytes() == 4
+
+
+class _NoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, y):
+        return y * 1
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+def test_a_gradient_that_is_not_there_counts_as_zeros():
+    module, x, _ = _module_and_data()
+    xg = x.requires_grad_()
+    _NoGradient.apply(module(xg)).sum().backward()
+    for g in (xg.grad, module.log_eps.grad, module.log_tau.grad):
+        assert g is not None and not g.any()

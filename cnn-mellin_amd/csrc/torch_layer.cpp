@@ -500,7 +500,7 @@ PyObject *log_lift(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
   if (n_args != 4 || followed()) Py_RETURN_NONE;
   for (int i = 0; i < 3; ++i)
-    if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
+    if (!THPVariable_CheckExact(args[i])) Py_RETURN_NONE;
   const Tensor &input0 = THPVariable_Unpack(args[0]), &log_eps = THPVariable_Unpack(args[1]), &log_tau = THPVariable_Unpack(args[2]);
   const int64_t dim = PyLong_AsLongLong(args[3]);
   if (!plain(input0) || input0.scalar_type() != at::kFloat || dim < 0 || dim >= input0.dim() || input0.numel() == 0) Py_RETURN_NONE;
@@ -547,7 +547,7 @@ PyObject *log_lift(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
 // packing by PyTorch took 58 to 92 us of host time and a synchronous copy).
 PyObject *pack_windows(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  if (n_args != 4 || followed() || !THPVariable_Check(args[0]) || !THPVariable_Check(args[1]) || !PyLong_CheckExact(args[2]) ||
+  if (n_args != 4 || followed() || !THPVariable_CheckExact(args[0]) || !THPVariable_CheckExact(args[1]) || !PyLong_CheckExact(args[2]) ||
       !PyLong_CheckExact(args[3]))
     Py_RETURN_NONE;
   const Tensor &x0 = THPVariable_Unpack(args[0]), &lens0 = THPVariable_Unpack(args[1]);

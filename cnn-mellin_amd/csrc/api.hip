@@ -1676,7 +1676,7 @@ static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockP
   if (!lp.known[0]) {
     SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
     pr.out_half = half;
-    lp.known[0] = make_block_plan(pr, half, lp.forward) ? 1 : -1;
+    lp.known[0] = make_block_plan(pr, half, false, lp.forward) ? 1 : -1;
   }
   if (lp.known[0] > 0) bp = lp.forward;
   return lp.known[0] > 0;
@@ -1687,7 +1687,7 @@ static bool plan_block_input(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPla
   if (!lp.known[1]) {
     SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
     pr.out_half = half;
-    lp.known[1] = make_block_plan(pr, half, lp.input) ? 1 : -1;
+    lp.known[1] = make_block_plan(pr, half, true, lp.input) ? 1 : -1;
   }
   if (lp.known[1] > 0) bp = lp.input;
   return lp.known[1] > 0;
@@ -1730,6 +1730,17 @@ static i64 blocked_images(i64 batch, i64 channels, i64 plane, bool half) {
 static bool layer_elements(int elem) { return elem == 2 || elem == 4 || elem == MELLIN_ELEM_HALF_FLOAT; }
 static int bad_elements(const char *who, int elem) {
   return fail(MELLIN_ERR_ARGUMENT, "%s: elements of 2 (half) or 4 (float) bytes, or MELLIN_ELEM_HALF_FLOAT, only (got %d)", who, elem);
+}
+
+// (a layer's plan, for tests and profiling)
+int mellin_layer_plan(int kind_x, int elem_bytes, int gradient, MELLIN_CORR2D_DIMS, int *plan) {
+  if (!plan || !layer_elements(elem_bytes) || check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
+  const bool half = elem_bytes != 4;
+  BlockPlan bp;
+  if (!(gradient ? plan_block_input(kind_x, half, CORR2D_ARGS, bp) : plan_block_forward(kind_x, half, CORR2D_ARGS, bp))) return 0;
+  const int words[MELLIN_LAYER_PLAN_WORDS] = {bp.mt, bp.nt, bp.wm, bp.wk, bp.joint, bp.F, bp.G, bp.whole, bp.rest, bp.slices};
+  std::copy(words, words + MELLIN_LAYER_PLAN_WORDS, plan);
+  return 1;
 }
 
 size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {

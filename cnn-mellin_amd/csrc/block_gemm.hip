@@ -52,7 +52,7 @@ void plan_classes(const Axis &x, BlockPlan &pl) {
 
 }  // namespace
 
-bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
+bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) {
   const Axis &X = pr.x, &Y = pr.y;
   const i64 lim = (i64)1 << 30;
   if (pr.accumulate || pr.batch < 1 || pr.c_out < 1 || pr.c_in < 1 || X.nf < 1 || Y.nf < 1 || X.nf > kBlockFilterRows) return false;
@@ -272,10 +272,15 @@ bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl) {
   // an output row of several images has the filter rows of that row alone, and no image ends inside a tile.  96 passes of
   // windows of 5 to 20 frames and of deep layers take them: 1.36 times as fast in the geometric mean (up to 2.6; 0.92 to 1.05
   // where the model gains less than a tenth, which is why it has to).  Windows of ten frames, 64 channels: input gradients
-  // 319 -> 181 us; the training step 2014 -> 1575.  Channels that end inside a tile are left out (their rows would be the
-  // next image's in the stores), and offsets into all images have 32 bits.
+  // 319 -> 181 us.  Channels that end inside a tile are left out (their rows would be the next image's in the stores), and
+  // offsets into all images have 32 bits.
+  // Input gradients only.  A stage's filter rows decide the order of the sums, and the signs of a forward pass's outputs
+  // decide what their ReLU lets through: a value within its rounding error of zero passes a whole gradient on in one order
+  // and none in another.  On those windows up to five flags of 74 million are not those of 64 bits, and log_eps's gradient,
+  // one sum that nearly cancels, moves by up to 2e-2, where 3e-6 is its error against 64 bits at given flags.  Forward passes
+  // therefore keep the tiles of an image (joint ones: the training step 1364 -> 1205 us).
   const i64 unit_bytes = 16 * parts, most = (i64)1 << 31;
-  const bool can_join = mellin && masks && pl.batch > 1 && Q * pl.batch < lim && (i64)pl.batch * pl.CG * (plane + 1) * unit_bytes < most &&
+  const bool can_join = gradient && mellin && masks && pl.batch > 1 && Q * pl.batch < lim && (i64)pl.batch * pl.CG * (plane + 1) * unit_bytes < most &&
                         (i64)pl.batch * pl.out_groups * (Q + 1) * unit_bytes < most && (i64)pl.batch * pl.M * Q * 4 < most &&
                         pl.h_n == (i64)pl.M * Q;
   // Tiles of 32 channels are tried as well: where those of 64 leave half of the last one empty (65 to 96 channels, 129 to 160,

@@ -61,8 +61,8 @@ struct BlockPlan {
   int joint, tile_batch, tile_q;
 };
 
-// False: the kernel does not apply.
-bool make_block_plan(const SepConv &pr, bool f16, BlockPlan &pl);
+// False: the kernel does not apply.  gradient: of an input (a forward pass has no joint tiles).
+bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl);
 // out = [relu](bias + sum) from a blocked signal and packed filter; bias (fp32 / half, or null), relu as the plan says.
 // With `grad`, the input gradient of a layer behind a ReLU: zero where `mask`, the blocked output of that ReLU, is not
 // positive; its sums over the positions go to chan_sums ([channel][pl.chan_slots]: partial sums for launch_block_finish).

@@ -1,0 +1,45 @@
+"""Which tiles the blocked kernels take for a pass (`mellin_layer_plan`; the plans are made on the host)."""
+import ctypes
+
+import pytest
+
+import _mellin_hip as hip
+import mconv
+from conv_stack import ConvStackParams, layer_plan
+
+WORDS = "mt nt wm wk joint F G whole rest slices".split()
+
+
+def stack_dims(batch, frames, bins, params):
+    """The dimensions of a stack's layers as the library's entry points take them."""
+    x, y = frames, bins
+    for lay in layer_plan(params, frames, bins):
+        (kx, ky), s, d, p, r = lay["kernel"], lay["s"], lay["d"], lay["p"], lay["r"]
+        valid = mconv.mcorr_valid_size if params.mellin else mconv.lcorr_valid_size
+        ox, oy = valid(kx, x, s[0], d[0], p[0]) + r[0], mconv.lcorr_valid_size(ky, y, s[1], d[1], p[1]) + r[1]
+        yield [batch, lay["in_channels"], lay["out_channels"], kx, ky, x, y, ox, oy, *s, *d, *p, 1, 1]
+        x, y = lay["out_size"]
+
+
+def plan(kind, elem_bytes, gradient, dims):
+    words = (ctypes.c_int * len(WORDS))()
+    if not hip.lib.mellin_layer_plan(kind, elem_bytes, gradient, *dims, words):
+        return None
+    return dict(zip(WORDS, words))
+
+
+# (kernel, channels, layers, batch, frames, bins)
+SMALL_IMAGES = [((5, 3), 64, 5, 1177, 10, 41), ((5, 3), 64, 3, 300, 10, 41), ((5, 3), 128, 3, 250, 10, 40), ((4, 3), 128, 4, 200, 7, 23)]
+
+
+@pytest.mark.parametrize("elem_bytes", [4, 2])
+@pytest.mark.parametrize("case", SMALL_IMAGES)
+def test_joint_tiles_are_for_input_gradients(case, elem_bytes):
+    """The order of a forward pass's sums decides which values a ReLU lets through."""
+    kernel, channels, layers, batch, frames, bins = case
+    params = ConvStackParams(layers=layers, kernel_time=kernel[0], kernel_freq=kernel[1], initial_channels=channels, factor_schedule=2,
+                             time_factor=2)
+    dims = list(stack_dims(batch, frames, bins, params))[1:]
+    plans = [[plan(hip.AX_MCORR, elem_bytes, gradient, d) for d in dims] for gradient in (0, 1)]
+    assert not any(p["joint"] for p in plans[0])
+    assert any(p["joint"] for p in plans[1])

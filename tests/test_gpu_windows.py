@@ -3,7 +3,9 @@ parameters -- against the same through PyTorch and through `log_compression_lift
 import pytest
 import torch
 
-from conv_stack import pack_windows
+import _mellin_hip as hip
+from conv_stack import ConvStack, ConvStackParams, pack_windows
+from test_block_plans import plan, stack_dims
 from layers import LogCompressionLift, log_compression_lift
 
 pytestmark = pytest.mark.gpu
@@ -61,3 +63,78 @@ def test_lift_from_its_own_parameters(shape, dim):
     assert all(a.shape == b.shape and torch.equal(a, b) for a, b in zip(got, want))
     only = torch.autograd.grad(module(x), (module.log_tau,), grad)         # (no gradient of the input)
     assert torch.equal(only[0], want[2])
+
+
+def _layer64(x, weight, bias, lay, out_size):
+    """A Mellin x linear layer of `layer_plan` in float64, a matrix product per output row."""
+    (c_out, c_in, kx, ky), n, (ox, oy) = weight.shape, x.shape[0], out_size
+    (sx, sy), (dx, dy), (px, py) = lay["s"], lay["d"], lay["p"]
+    x = torch.nn.functional.pad(x, (py, max(0, sy * (oy - 1) + dy * (ky - 1) + 1 - x.shape[3] - py)))
+    rows = []
+    for h in range(ox):
+        taps = [(f, (h + sx) * (f + dx) // (px + 1) - 1) for f in range(kx) if (h + sx) * (f + dx) % (px + 1) == 0]
+        taps = [(f, g, fy) for f, g in taps if g < x.shape[2] for fy in range(ky)]
+        row = bias.view(-1, 1).expand(c_out, n * oy)
+        if taps:
+            cols = torch.stack([x[:, :, g, fy * dy:fy * dy + sy * (oy - 1) + 1:sy] for _, g, fy in taps])      # (taps, n, c_in, oy)
+            w = torch.stack([weight[:, :, f, fy] for f, _, fy in taps], 1).reshape(c_out, -1)
+            row = row + w @ cols.permute(0, 2, 1, 3).reshape(-1, n * oy)
+        rows.append(row.view(c_out, n, oy))
+    return torch.stack(rows, 2).transpose(0, 1)
+
+
+@pytest.mark.parametrize("lens,bins,window,stride,kernel,channels,layers", [
+    ([190, 151, 77, 33], 41, 10, 1, (5, 3), 64, 4),    # joint tiles in the input gradients
+    ([120, 64], 20, 7, 2, (3, 3), 24, 3),              # channels that end inside a tile
+])
+def test_training_step_against_float64_at_its_own_flags(lens, bins, window, stride, kernel, channels, layers):
+    """A whole step, front end and stack, with the ReLUs' choices of the step itself: what another order of the sums makes of
+    values near zero stays out of the comparison, and what is left is rounding."""
+    torch.manual_seed(21)
+    params = ConvStackParams(layers=layers, kernel_time=kernel[0], kernel_freq=kernel[1], initial_channels=channels, factor_schedule=2,
+                             time_factor=2)
+    stack, lift = ConvStack(window, bins, params).cuda(), LogCompressionLift(dim=2).cuda()
+    with torch.no_grad():
+        for conv in stack.convs:
+            conv.weight.uniform_(-1, 1).mul_((6 / conv.weight[0].numel()) ** 0.5)
+            conv.bias.uniform_(-0.1, 0.1)
+    x = torch.randn(len(lens), max(lens), bins, device="cuda").exp()
+    windows, _ = pack_windows(x, torch.tensor(lens), window, stride)
+    out = stack(lift(windows))
+    grad = torch.randn_like(out)
+    leaves = list(stack.parameters()) + list(lift.parameters())
+    got = [out.detach()] + list(torch.autograd.grad(out, leaves, grad))
+    if channels == 64:
+        dims = list(stack_dims(windows.shape[0], window, bins, params))
+        assert any(plan(hip.AX_MCORR, 4, 1, d)["joint"] for d in dims[1:])
+    # the flags: a layer's output is that of the stack that ends there
+    flags = []
+    with torch.no_grad():
+        for k in range(1, layers + 1):
+            shorter = ConvStackParams(**{**vars(params), "layers": k})
+            part = ConvStack(window, bins, shorter).cuda()
+            for a, b in zip(part.convs, stack.convs):
+                a.load_state_dict(b.state_dict())
+            flags.append(part(lift(windows)) > 0)
+    assert torch.equal(flags[-1], out > 0)
+    leaves64 = [p.detach().double().requires_grad_() for p in leaves]
+    log_eps, log_tau = leaves64[-2:]
+    t = torch.arange(1, window + 1, device="cuda", dtype=torch.float64).view(-1, 1)
+    y = (log_eps.exp() + windows.double().abs()).log() * t ** log_tau.exp()
+    y.retain_grad()
+    first = y
+    for i, (lay, d) in enumerate(zip(stack.plan, stack_dims(windows.shape[0], window, bins, params))):
+        y = _layer64(y, leaves64[2 * i], leaves64[2 * i + 1], lay, d[7:9]) * flags[i]
+    y.backward(grad.double())
+    want = [y.detach()] + [p.grad for p in leaves64]
+    # the lift's gradients are sums that nearly cancel: their scale is the 2-norm of what is added
+    scales = [float(w.norm()) for w in want[:-2]]
+    inner = first.grad * t ** log_tau.detach().exp()
+    a = log_eps.detach().exp() + windows.double().abs()
+    scales += [float((inner * log_eps.detach().exp() / a).norm()),
+               float((inner * a.log() * t.log() * log_tau.detach().exp()).norm())]
+    # fp32 sums of up to 10^3 products a layer, `layers` of them behind each other, forward and backward: 2^-24 each, times
+    # the square root of their number and of the layers, with room of three
+    bound = 3 * 2 ** -24 * (2 * layers) ** 0.5 * 10
+    for name, g, w, scale in zip(["out"] + [n for n, _ in stack.named_parameters()] + ["log_eps", "log_tau"], got, want, scales):
+        assert float((g.double() - w).norm()) <= bound * scale, (name, float((g.double() - w).norm()) / scale)

@@ -1610,8 +1610,9 @@ static bool blocks_allowed(bool half) {
          !g_no_yfold && !g_gather && !g_no_narrow && (half || g_math != MATH_FP32));
 }
 // Plans of the layer entry points, kept per thread: a layer asks for the same ones with every step (its workspace, then
-// the launch), and choosing among tile shapes takes some microseconds.  The sizes decide the plan, so nothing has to be
-// thrown away.
+// the launch), and choosing among tile shapes takes 0.5 to 4 microseconds a pass (ten Mellin layers of a new length: 17 served,
+// 32 to 55 with their gradients, in the caller's thread and again in autograd's).  The sizes decide the plan, so nothing has to
+// be thrown away.
 struct LayerPlans {
   int known[5];                                        // 0 not yet, 1 applies, -1 does not
   size_t bias_bytes;                                   // section 2's weight gradient: for the bias gradient beside it (known[3])

@@ -5,6 +5,7 @@
 #include <cmath>
 
 #include "block_gemm_kernel.hpp"
+#include "tap_runs.hpp"
 
 namespace mellin {
 
@@ -110,38 +111,47 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
   pl.mt = pr.c_out > 32 ? 2 : 1;
   pl.wm = 1;
 
+  // Tile shapes: tiles of 32 positions of a wavefront, wavefronts along the channels, wavefronts that share a tile.
+  constexpr int kShapes = 7;
+  static const int shapes[kShapes][3] = {{4, 2, 1}, {4, 1, 1}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}, {2, 1, 4}, {1, 1, 4}};
   // A tile shape's stage: the channel groups and filter rows that fit twice into the LDS that a
   // workgroup may take, two workgroups to a CU
-  auto shape = [&](int nt, int wm, int wk) {
+  struct Stage { i64 rows; int F, G; };
+  Stage stages[2][kShapes] = {};
+  int groups[8], n_groups = 0;                         // the channel groups of a stage that divide all, most first
+  for (int G = std::min(pl.CG, 8); G >= 1; --G)
+    if (pl.CG % G == 0) groups[n_groups++] = G;
+  auto shape = [&](int at) {
+    const int nt = shapes[at][0], wm = shapes[at][1], wk = shapes[at][2];
     const int P = (kWaves / wk / wm) * nt * 32, M_T = wm * pl.mt * 32;
     const i64 RT = std::min<i64>(pl.joint ? (i64)pl.nox * pl.batch : pl.nox, (P - 1 + pl.noy - 1) / pl.noy + 1);
     const i64 vrows = mellin ? RT : (i64)pl.ax * (RT - 1) + pl.bx_span + 1;
     const i64 tab = ((mellin ? vrows * pl.nfx : vrows) * pl.RS + 64 + 64 + 3) & ~(i64)3;
     const i64 row_src = mellin ? 4 * RT * pl.nfx : 0;
-    auto pad = [&](i64 halves) { return std::max<i64>((halves + 2 * wk - 1) / (2 * wk) * (2 * wk), 4 * wk); };
-    int best_f = 0, best_g = 0;
-    double best = 0;
-    for (int F = mellin ? pl.nfx : 1; F >= 1; --F) {
-      const int rows = mellin ? F : pl.nfx;
-      const i64 units = vrows * (mellin ? F : 1) * pl.RS;
-      const i64 gb = (units * parts + 63) / 64 * 1024;
-      for (int G = std::min(pl.CG, 8); G >= 1; --G) {
-        if (pl.CG % G) continue;
-        const i64 ents = (mellin ? (pl.nfx + F - 1) / F : 1) * pad((i64)rows * pl.nfy * G) + 8 * wk;
-        const i64 bytes = 2 * gb * G + 4 * tab + 16 * ents + row_src + M_T * 4;
-        if (bytes > 79 * 1024) continue;
-        // what a stage's steps fill of their whole pairs, against what a stage costs on top (its barrier and first reads)
-        const i64 halves = (i64)rows * pl.nfy * G;
-        const double rate = (double)halves / (double)(pad(halves) + 2 * wk);
-        if (rate > best) { best = rate; best_f = F; best_g = G; }
+    auto pad = [&](int halves) { return std::max((halves + 2 * wk - 1) & -(2 * wk), 4 * wk); };      // (wk: 1 or 4)
+    Stage &st = stages[pl.mt - 1][at];                 // (joint tiles mostly have as many rows as those of an image)
+    if (st.rows != RT) {
+      st = Stage{RT, 0, 0};
+      int best_halves = 0, best_all = 1;               // the best rate so far, as a fraction
+      for (int F = mellin ? pl.nfx : 1; F >= 1; --F) {
+        const int rows = mellin ? F : pl.nfx, subsets = mellin ? (pl.nfx + F - 1) / F : 1;
+        const i64 gb = (vrows * (mellin ? F : 1) * pl.RS * parts + 63) / 64 * 1024, fixed = 4 * tab + row_src + M_T * 4;
+        if (2 * gb + fixed > 79 * 1024) continue;
+        for (int k = 0; k < n_groups; ++k) {
+          const int G = groups[k], halves = rows * pl.nfy * G, all = pad(halves);
+          if (2 * gb * G + fixed + 16 * (i64)(subsets * all + 8 * wk) > 79 * 1024) continue;
+          // what a stage's steps fill of their whole pairs, against what a stage costs on top (its barrier and first reads)
+          if (halves * best_all > best_halves * (all + 2 * wk)) { best_halves = halves; best_all = all + 2 * wk; st.F = F; st.G = G; }
+        }
       }
     }
+    const int best_f = st.F, best_g = st.G;
     if (!best_f) return false;
     const i64 units = vrows * (mellin ? best_f : 1) * pl.RS;
     pl.F = mellin ? best_f : pl.nfx;
     pl.G = best_g;
     pl.tab_units = (int)tab;
-    pl.ents = (int)((mellin ? (pl.nfx + pl.F - 1) / pl.F : 1) * pad((i64)pl.F * pl.nfy * best_g) + 8 * wk);
+    pl.ents = (mellin ? (pl.nfx + pl.F - 1) / pl.F : 1) * pad(pl.F * pl.nfy * best_g) + 8 * wk;
     pl.group_bytes = (int)((units * parts + 63) / 64 * 1024);
     pl.buf_bytes = pl.group_bytes * best_g;
     pl.nt = nt; pl.wm = wm; pl.wk = wk;
@@ -162,44 +172,40 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
     pl.tile_batch = joint ? 1 : pl.batch;
     pl.tile_q = joint ? pl.nox * pl.batch * pl.noy : pl.Q;
   };
-  // Mellin axes: which filter rows have a tap inside the signal, per output row in the order of the classes (axes of
+  // Mellin axes: which filter rows have a tap inside the signal, for runs of output rows in the order of the classes (axes of
   // more rows, of which a tile's share a class: those of the class)
-  constexpr int kMaskRows = 4096;
-  unsigned row_mask[kMaskRows];
-  const bool masks = mellin && pl.nox <= kMaskRows;
+  static_assert(TapRuns::kFilterRows == kBlockFilterRows, "");
+  TapRuns runs;
+  const bool masks = mellin && pl.nox <= TapRuns::kRows;
   double class_rows = 0;
-  if (mellin)
+  if (mellin) {
+    const TapAxis axis = {X.kind == AX_MCORR, pl.nfx, pl.ngx, pl.sx, pl.dx, pl.px + 1, pl.ux};
     for (int k = 0; k < pl.n_classes; ++k) {
       const int end = k + 1 < pl.n_classes ? pl.cls[k + 1].start : pl.nox;
       class_rows += __builtin_popcount(pl.cls[k].mask) * (double)(end - pl.cls[k].start) / pl.nox;
-      for (int at = pl.cls[k].start; masks && at < end; ++at) {
-        const unsigned h = (unsigned)(pl.cls[k].first + (at - pl.cls[k].start) * pl.cls_stride + pl.sx), p1 = (unsigned)pl.px + 1;
-        unsigned mask = 0;
-        for (int f = 0; f < pl.nfx; ++f) {
-          const unsigned fd = (unsigned)(f + pl.dx), num = X.kind == AX_MCORR ? h * fd : h * p1, den = X.kind == AX_MCORR ? p1 : fd;
-          const unsigned q = num / den;
-          if (q * den == num && q >= (unsigned)pl.ux && q - (unsigned)pl.ux < (unsigned)pl.ngx) mask |= 1u << f;
-        }
-        row_mask[at] = mask;
-      }
+      if (masks) runs.add_class(axis, pl.cls[k].first, pl.cls_stride, end - pl.cls[k].start);
     }
+  }
   // What a tile of P positions stages: filter rows, and stages of them, on average.  (Counted over the tile's rows together:
   // with the average of single rows small images of many classes got tiles that stage nearly every filter row; windows of
   // ten frames 1989 -> 1968 us a step, a ten-layer Mellin stack of 24 to 192 channels on two utterances 1175 -> 1117 us.)
-  auto tile_rows = [&](int P, double &filter_rows, double &subsets) {
+  // Tiles of P positions are counted once for all shapes.
+  struct Tiles { int joint, of[TapRuns::kFilterRows + 1]; } tiles_by_p[5] = {{-1, {}}, {-1, {}}, {-1, {}}, {-1, {}}, {-1, {}}};
+  // (F: filter rows of a stage)
+  auto tile_rows = [&](int P, int F, double &filter_rows, double &subsets) {
     filter_rows = mellin ? std::max(1.0, class_rows) : pl.nfx;
-    subsets = mellin ? std::ceil(filter_rows / pl.F) : 1;
+    subsets = mellin ? std::ceil(filter_rows / F) : 1;
     if (!masks) return;
-    i64 rows = 0, stages = 0, tiles = 0;
-    const i64 per_row = pl.joint ? (i64)pl.batch * pl.noy : pl.noy, all = pl.tile_q;
-    // (rows of many tiles: as if each began one)
-    for (i64 q0 = 0; q0 < all; q0 = per_row >= 8 * P ? q0 + per_row : q0 + P, ++tiles) {
-      const i64 last = per_row >= 8 * P ? q0 / per_row : (std::min<i64>(q0 + P, all) - 1) / per_row;
-      unsigned mask = 0;
-      for (i64 r = q0 / per_row; r <= last; ++r) mask |= row_mask[r];
-      const int n = std::max(1, __builtin_popcount(mask));
-      rows += n;
-      stages += (n + pl.F - 1) / pl.F;
+    Tiles &count = tiles_by_p[__builtin_ctz((unsigned)P) - 5];            // (32 to 512)
+    if (count.joint != pl.joint) {
+      count = Tiles{pl.joint, {}};
+      runs.count_tiles(P, pl.joint ? pl.batch * pl.noy : pl.noy, count.of);
+    }
+    int rows = 0, stages = 0, tiles = 0;
+    for (int n = 1; n <= pl.nfx; ++n) {
+      rows += n * count.of[n];
+      stages += (n + F - 1) / F * count.of[n];
+      tiles += count.of[n];
     }
     filter_rows = (double)rows / tiles;
     subsets = (double)stages / tiles;
@@ -222,40 +228,64 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
   // fragments, which the steps' rate leaves out.  Of 3000 passes of half layers and stacks drawn over 1 to 32 images of 100 to
   // 780 rows, 1183 take other plans with 9000; 276 of those take 0.86 of the time with 5000 in the geometric mean (0.53 to
   // 1.20, twelve of them more than 1.03).  In fp32 it decides 361 of 3000, for either side: 205 of them 0.66 to 1.29.
-  const i64 slots = 512;
-  auto cost = [&]() {
-    const int M_T = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32;
-    const i64 total = (i64)((pl.tile_q + P - 1) / P) * pl.tile_batch, per_m = std::max<i64>(1, slots / pl.m_tiles), c_stages = pl.CG / pl.G;
+  const int slots = 512;
+  struct Launch { int M_T, P, m_tiles, per_m; i64 total; double rate, tile, output; };
+  auto launch_of = [&](int nt, int wm, int wk) {
+    Launch l;
+    l.M_T = wm * pl.mt * 32; l.P = kWaves / wk / wm * nt * 32;
+    l.m_tiles = ((int)pr.c_out + l.M_T - 1) / l.M_T;
+    l.per_m = std::max(1, slots / l.m_tiles);
+    l.total = (i64)((pl.tile_q + l.P - 1) / l.P) * pl.tile_batch;
+    l.rate = pl.mt * nt * wm >= 8 ? 0.8 : pl.mt * nt >= 4 ? 0.65 : 0.55;
+    l.tile = wk > 1 && !f16 ? 9000 : 5000;
+    l.output = (double)l.M_T * l.P * (f16 ? 2 : 4) / 9;
+    return l;
+  };
+  // Whether a shape costs `wanted` and more whatever its stages and slices are: full turns of whole steps without gaps.
+  // (Choosing among the shapes is host time that every new size pays: a ten-layer Mellin stack on 32 x 700 frames took
+  // 1.15 ms to plan where tiles were counted one by one for every shape and none was passed over, and takes 0.035.)
+  auto hopeless = [&](const int *sh, double wanted) {
+    const int nt = sh[0], wk = sh[2];
+    const Launch l = launch_of(nt, sh[1], wk);
     double filter_rows, subsets;
-    tile_rows(P, filter_rows, subsets);
-    const double rows = filter_rows / subsets;
-    const double rate = pl.mt * pl.nt * pl.wm >= 8 ? 0.8 : pl.mt * pl.nt >= 4 ? 0.65 : 0.55;
-    const double steps = std::ceil(rows * pl.nfy * pl.G / (2 * pl.wk)) * pl.mt * pl.nt * (f16 ? 1 : 6) * 32 / rate;
-    const double output = (double)M_T * P * (f16 ? 2 : 4) / 9;
-    const double tile = pl.wk > 1 && !f16 ? 9000 : 5000;
-    auto turns_cost = [&](i64 items, double stages) {
-      const i64 full = items / per_m, left = items - full * per_m;
-      auto turn = [&](i64 n) { return stages * std::max(4000.0, steps * (n * pl.m_tiles > slots / 2 ? pl.wk > 1 && full == 0 ? 1.5 : 2 : 1)) + tile + output; };
+    tile_rows(l.P, pl.nfx, filter_rows, subsets);
+    const double steps = filter_rows * pl.nfy * pl.CG / (2 * wk) * pl.mt * nt * (f16 ? 1 : 6) * 32 / l.rate;
+    const double least = 9000 + (double)l.total / l.per_m * (steps * (wk > 1 ? 1.5 : 2) + l.tile + l.output);
+    return least >= wanted * (1 + 1e-9);
+  };
+  // (wanted, or 0: what costs as much is not taken)
+  auto cost = [&](double wanted) {
+    const Launch l = launch_of(pl.nt, pl.wm, pl.wk);
+    const int M_T = l.M_T, P = l.P, total = (int)l.total, per_m = l.per_m, c_stages = pl.CG / pl.G;      // (shape(): less than 2^26 tiles)
+    double filter_rows, subsets;
+    tile_rows(P, pl.F, filter_rows, subsets);
+    const double rows = filter_rows / subsets, tile = l.tile, output = l.output;
+    const double steps = std::ceil(rows * pl.nfy * pl.G / (2 * pl.wk)) * pl.mt * pl.nt * (f16 ? 1 : 6) * 32 / l.rate;
+    auto turns_cost = [&](int items, double stages) {
+      const int full = items / per_m, left = items - full * per_m;
+      auto turn = [&](int n) { return stages * std::max(4000.0, steps * (n * pl.m_tiles > slots / 2 ? pl.wk > 1 && full == 0 ? 1.5 : 2 : 1)) + tile + output; };
       return full * turn(per_m) + (left ? turn(left) : 0);
     };
     double best = 9000 + turns_cost(total, c_stages * subsets);
     pl.slices = 1;
-    i64 rest = 0;
+    int rest = 0;
     for (int all = 0; all < 2; ++all) {
-      const i64 r = all ? total : total % per_m;
+      const int r = all ? total : total % per_m;
       if (r == 0 || (all && total >= 2 * per_m) || (pl.wk > 1 && !all)) continue;
-      for (i64 s = 2; s <= std::min<i64>(c_stages, 16); ++s) {
+      const double whole = 9000 + turns_cost(total - r, c_stages * subsets);
+      const double least = whole + subsets * std::max(4000.0, steps) + tile + output + 9000;      // (a slice is a stage or more)
+      if (least >= 0.95 * best || (wanted > 0 && best >= wanted && least >= wanted * (1 + 1e-9))) continue;
+      for (int s = 2; s <= std::min(c_stages, 16); ++s) {
         const double bytes = (double)r * s * pl.m_tiles * M_T * P * 8;
-        const double c = 9000 + turns_cost(total - r, c_stages * subsets) + turns_cost(r * s, std::ceil((double)c_stages / s) * subsets) +
-                         9000 + bytes / 2400;
-        if (c < 0.95 * best) { best = c; pl.slices = (int)s; rest = r; }
+        const double c = whole + turns_cost(r * s, (c_stages + s - 1) / s * subsets) + 9000 + bytes / 2400;
+        if (c < 0.95 * best) { best = c; pl.slices = s; rest = r; }
       }
     }
-    pl.rest = (int)rest;
-    pl.whole = (int)(total - rest);
-    pl.chan_slots = (int)total * (pl.wk > 1 ? pl.nt : kWaves / pl.wm);
-    const i64 items = (i64)pl.whole + (i64)pl.rest * pl.slices;
-    pl.grid_x = (int)(pl.wk > 1 ? items : std::min<i64>(per_m, items));      // (wavefronts that share a tile's steps take one tile)
+    pl.rest = rest;
+    pl.whole = total - rest;
+    pl.chan_slots = total * (pl.wk > 1 ? pl.nt : kWaves / pl.wm);
+    const int items = pl.whole + pl.rest * pl.slices;
+    pl.grid_x = pl.wk > 1 ? items : std::min(per_m, items);      // (wavefronts that share a tile's steps take one tile)
     pl.slice_bytes = (size_t)pl.rest * pl.slices * pl.m_tiles * (size_t)(M_T * P) * 4;
     return best;
   };
@@ -267,7 +297,6 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
   // many products, and a stage has twice the steps (128 -> 256 channels, 3 x 3, 32 x 256 x 41: 1075 -> 905 us).  77 passes of
   // stacks and layers drawn over 1 to 32 images take it: with more workgroups than CUs 1.15 times as fast in the geometric mean
   // (0.99 to 1.46), with less, which leave nothing on a CU to run beside a workgroup's waits, 0.95 (0.73 to 1.18): not those.
-  static const int shapes[][3] = {{4, 2, 1}, {4, 1, 1}, {2, 2, 1}, {2, 1, 1}, {1, 1, 1}, {2, 1, 4}, {1, 1, 4}};   // nt, wm, wk
   // Joint tiles (Mellin axes): on small images a tile has rows of every class, and multiplies the filter rows of all of them;
   // an output row of several images has the filter rows of that row alone, and no image ends inside a tile.  96 passes of
   // windows of 5 to 20 frames and of deep layers take them: 1.36 times as fast in the geometric mean (up to 2.6; 0.92 to 1.05
@@ -294,14 +323,18 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
     double limit = joint && best_cost > 0 ? 0.9 * best_cost : 0;
     set_joint(joint);
     for (pl.mt = mt; pl.mt >= 1; --pl.mt)
-      for (const auto &sh : shapes) {
+      for (int k = 0; k < kShapes; ++k) {
+        const int *const sh = shapes[k];
         if (pl.mt < mt && sh[1] == 2) continue;
         if (f16 ? sh[0] == 2 && sh[1] == 2 : sh[0] == 4 || (sh[0] == 2 && sh[2] == 4)) continue;
         if (sh[1] == 2 && pr.c_out <= 96) continue;      // (two wavefronts along the channels: most of 128)
-        if (!shape(sh[0], sh[1], sh[2])) continue;
-        const double c = cost();
+        const double wanted = (pl.mt < mt ? narrow : 1) * limit;
+        // (joint tiles often have no stage that fits, and take longer to count)
+        if (limit > 0 && !joint && hopeless(sh, wanted)) continue;
+        if (!shape(k) || (limit > 0 && joint && hopeless(sh, wanted))) continue;
+        const double c = cost(wanted);
         if (!f16 && sh[1] == 2 && ((i64)pl.whole + (i64)pl.rest * pl.slices) * pl.m_tiles <= slots / 2) continue;
-        if (limit == 0 || c < (pl.mt < mt ? narrow : 1) * limit) { limit = best_cost = c; best_plan = pl; }
+        if (limit == 0 || c < wanted) { limit = best_cost = c; best_plan = pl; }
       }
   }
   if (best_cost == 0) return false;

@@ -391,6 +391,9 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
   // Block shape: wavefronts side by side along the output channels (wm) and along the column tiles, MT x NT tiles each.
   // What counts: the share of the tiles that are of use, and how often a fetched operand is (MT NT / (MT + NT)).
   const int ct_all = (pl.C + 31) / 32, mt_all = (pl.M + 31) / 32;
+  const i64 R = (KS - 1 + pl.noy - 1) / pl.noy + 1;
+  const i64 vu = std::max<i64>(pl.ay * (KS - 1) + span + 1, pl.ay * (KS - R) + R * (span + 1));
+  const i64 vp = ((vu + span + 1 - 4 + 7) / 8) * 8 + 4;
   double best = 0;
   for (int nw = 4; nw <= 8; nw *= 2)
     for (int mt = 1; mt <= 2; ++mt)
@@ -398,9 +401,6 @@ bool make_block_wgrad_plan(const SepConv &fwd, bool f16, BlockWgradPlan &pl) {
         for (int ctb = 1; ctb <= ct_all; ++ctb) {
           const int wn = nw / wm, tiles = ctb * pl.nfy, nt = (tiles + wn - 1) / wn;
           if (nt > (f16 || mt == 1 ? 4 : 3)) break;    // (fp32: registers)
-          const i64 R = (KS - 1 + pl.noy - 1) / pl.noy + 1;
-          const i64 vu = std::max<i64>(pl.ay * (KS - 1) + span + 1, pl.ay * (KS - R) + R * (span + 1));
-          const i64 vp = ((vu + span + 1 - 4 + 7) / 8) * 8 + 4;
           if (KS + vp > nw * 64) break;
           const i64 bytes = 2 * UB * ((i64)wm * mt * 4 * (KS + 4) + (i64)ctb * 4 * vp) + 12 * (2 * KS + vp);
           if (bytes > (nw == 4 ? 79 : 158) * 1024) continue;

@@ -264,7 +264,8 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_gemm_kernel(
 // once more (27 us and 5 to reduce, of a step's 230, for three channels to 64, 32 x 505 x 38 outputs: 198 us without them;
 // on Mellin rows, 32 x 64 x 38, 81.5 -> 74.8).  A lane adds in pairs, then steps of a unit or row, then units; the halves of
 // a wavefront, the wavefronts and (wgrad_reduce_kernel) the workgroups follow, in pairs as well: error against 64 bits over
-// these two layers and twenty drawn ones 1.09e-7 with launches of their own, 1.06e-7 so (added in turn: 1.7e-7).
+// these two layers and twenty drawn ones 1.09e-7 with launches of their own, 1.06e-7 so (added in turn: 1.7e-7).  BIAS: the
+// sums are vector instructions in the matrix loop, and a weight gradient without them is an instance of its own.
 template <int MT>
 __device__ __forceinline__ void bias_to_lds(const float (&bias)[MT], float *dst, int wave, int half, int l32) {
 #pragma unroll
@@ -280,7 +281,7 @@ __device__ __forceinline__ float bias_of_waves(const float *src, int m) {
 }
 
 constexpr int kRowsMemo = 8;                       // 64-word blocks per wave whose staging sources are kept
-template <int MT, int JT>
+template <int MT, int JT, bool BIAS>
 __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
     WgradPlan wp, const float *__restrict__ A, const float *__restrict__ G,
     float *__restrict__ ws, float *__restrict__ bias_ws) {
@@ -417,7 +418,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
       for (int i = 0; i < MT; ++i) row_sum[i] = 0.f;
       int s = 0;
       for (; s + 8 <= pairs; s += 8) {
-        float last[MT], sum[MT];                         // (pairs of steps, then their sums, so that a rounding error meets few others)
+        [[maybe_unused]] float last[MT], sum[MT];        // (pairs of steps, then their sums, so that a rounding error meets few others)
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
           float a[MT], b[JT];
@@ -425,21 +426,23 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
           for (int i = 0; i < MT; ++i) a[i] = As[ao + i * 32 * wp.GSS + 2 * k];
 #pragma unroll
           for (int t = 0; t < JT; ++t) b[t] = Xs[bo[t] + 2 * k];
+          if constexpr (BIAS)
 #pragma unroll
-          for (int i = 0; i < MT; ++i) {
-            if (k & 1) last[i] += a[i];
-            else last[i] = a[i];
-            if (k == 1) sum[i] = last[i];
-            else if (k & 1) sum[i] += last[i];
-          }
+            for (int i = 0; i < MT; ++i) {
+              if (k & 1) last[i] += a[i];
+              else last[i] = a[i];
+              if (k == 1) sum[i] = last[i];
+              else if (k & 1) sum[i] += last[i];
+            }
 #pragma unroll
           for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int t = 0; t < JT; ++t)
               acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[t], acc[i][t], 0, 0, 0);
         }
+        if constexpr (BIAS)
 #pragma unroll
-        for (int i = 0; i < MT; ++i) row_sum[i] += sum[i];
+          for (int i = 0; i < MT; ++i) row_sum[i] += sum[i];
         ao += 16;
 #pragma unroll
         for (int t = 0; t < JT; ++t) bo[t] += 16;
@@ -462,8 +465,9 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
 #pragma unroll
             for (int t = 0; t < JT; ++t) b[t] = half ? 0.f : b[t];
           }
+          if constexpr (BIAS)
 #pragma unroll
-          for (int i = 0; i < MT; ++i) row_sum[i] += a[i];
+            for (int i = 0; i < MT; ++i) row_sum[i] += a[i];
 #pragma unroll
           for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -511,7 +515,8 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
   // has several words in flight per thread.
   __syncthreads();
   float *red = lds;                                   // [2][M_T][J_T], then the bias sums
-  if (bias_ws && jg == 0) bias_to_lds<MT>(bias, red + 2 * M_T * J_T, wave, half, l32);
+  if constexpr (BIAS)
+    if (jg == 0) bias_to_lds<MT>(bias, red + 2 * M_T * J_T, wave, half, l32);
   for (int phase = 0; phase < 2; ++phase) {
     if ((wave & 1) == phase) {
       float *slab = red + (wave >> 1) * (M_T * J_T);
@@ -529,7 +534,8 @@ __global__ __launch_bounds__(kThreads) void wgrad_rows_kernel(
     }
     __syncthreads();
   }
-  if (bias_ws && jg == 0 && tid < M_T) bias_ws[(i64)blockIdx.x * wp.M_pad + m0 + tid] = bias_of_waves<M_T>(red + 2 * M_T * J_T, tid);
+  if constexpr (BIAS)
+    if (jg == 0 && tid < M_T) bias_ws[(i64)blockIdx.x * wp.M_pad + m0 + tid] = bias_of_waves<M_T>(red + 2 * M_T * J_T, tid);
   float *out = ws + (i64)blockIdx.x * wp.M_pad * wp.J_pad + (i64)m0 * wp.J_pad + j0;
   constexpr int kTrip = 4;                             // words a thread has in flight (M_T * J_T is a multiple of 1024)
   for (int e0 = tid; e0 < M_T * J_T; e0 += kTrip * kThreads) {
@@ -915,11 +921,11 @@ hipError_t launch_variant(const WgradPlan &wp, size_t lds_bytes, dim3 grid, cons
   return hipGetLastError();
 }
 
-template <int MT, int JT>
+template <int MT, int JT, bool BIAS>
 hipError_t launch_rows(const WgradPlan &wp, dim3 grid, const float *a, const float *g, float *ws, float *bias_ws,
                        hipStream_t stream) {
-  auto kern = wgrad_rows_kernel<MT, JT>;
-  const size_t lds = bias_ws ? std::max(wp.lds_bytes, 4 * (size_t)(2 * MT * 32 * JT * 32 + kWaves * MT * 32)) : wp.lds_bytes;
+  auto kern = wgrad_rows_kernel<MT, JT, BIAS>;
+  const size_t lds = BIAS ? std::max(wp.lds_bytes, 4 * (size_t)(2 * MT * 32 * JT * 32 + kWaves * MT * 32)) : wp.lds_bytes;
   {
     static std::atomic<int> lds_allowed{0};                // (one per kernel instance)
     hipError_t e = allow_large_lds((const void *)kern, lds, lds_allowed);
@@ -1138,7 +1144,9 @@ hipError_t launch_wgrad(const WgradPlan &wp, const float *grad_out, const float 
 #undef MELLIN_STREAM_CASE
   } else if (wp.rows_mode) {
 #define MELLIN_ROWS_CASE(MT_, JT_)                                                         \
-  if (wp.mt == MT_ && wp.jt == JT_) e = launch_rows<MT_, JT_>(wp, grid, grad_out, input, workspace, bias_ws, stream);
+  if (wp.mt == MT_ && wp.jt == JT_)                                                         \
+    e = bias_ws ? launch_rows<MT_, JT_, true>(wp, grid, grad_out, input, workspace, bias_ws, stream)         \
+                : launch_rows<MT_, JT_, false>(wp, grid, grad_out, input, workspace, nullptr, stream);
     MELLIN_ROWS_CASE(1, 1) MELLIN_ROWS_CASE(1, 2) MELLIN_ROWS_CASE(1, 3)
     MELLIN_ROWS_CASE(2, 1) MELLIN_ROWS_CASE(2, 2) MELLIN_ROWS_CASE(2, 3)
 #undef MELLIN_ROWS_CASE

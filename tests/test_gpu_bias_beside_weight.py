@@ -45,3 +45,17 @@ def test_bias_gradient_beside_the_weight_gradient(case, offset):
     # been added so far, of 300 steps at most
     err = np.abs(bg.grad.double().cpu().numpy() - go64.sum((0, 2, 3)))
     assert np.all(err <= 300 * 2.0 ** -24 * np.abs(go64).sum((0, 2, 3))), err.max()
+
+
+@pytest.mark.parametrize("case", CASES, ids=[str(i) for i in range(len(CASES))])
+def test_weight_gradient_has_the_same_bits_without_a_bias(case):
+    """A weight gradient without a bias is a kernel of its own, without the sums, on the same tiles."""
+    op, n, c_in, c_out, nf, ng, p, r = case
+    torch.manual_seed(4200 + CASES.index(case))
+    x, w = torch.randn(n, c_in, *ng, device="cuda"), torch.randn(c_out, c_in, *nf, device="cuda", requires_grad=True)
+    b = torch.zeros(c_out, device="cuda", requires_grad=True)
+    layer = mconv._ext_mcorrlcorr if op == "mcorr" else mconv._ext_lcorrlcorr
+    outs = [layer(x, w, bias, (1, 1), (1, 1), p, (1, 1), r) for bias in (b, None)]
+    go = torch.randn_like(outs[0])
+    grads = [torch.autograd.grad(out, w, go)[0] for out in outs[1:]] + [torch.autograd.grad(outs[0], (w, b), go)[0]]
+    assert torch.equal(*grads)

@@ -1609,12 +1609,17 @@ static bool blocks_allowed(bool half) {
   return g_settled || (g_forced == 0 && !g_no_blocks && !g_widen && !g_no_classes && !g_all_classes && !g_split_classes && !g_whole_classes &&
          !g_no_yfold && !g_gather && !g_no_narrow && (half || g_math != MATH_FP32));
 }
+// How a stack's first layer runs: a call of its own, the blocked kernels, or the tiled kernel with `tiles`.
+enum FirstLayer { FIRST_OWN, FIRST_BLOCKS, FIRST_TILES };
+struct FirstPlan { FirstLayer route; TilePlan tiles; size_t lds; int mt, nt; };
 // Plans of the layer entry points, kept per thread: a layer asks for the same ones with every step (its workspace, then
 // the launch), and choosing among tile shapes takes 0.5 to 4 microseconds a pass (ten Mellin layers of a new length: 17 served,
 // 32 to 55 with their gradients, in the caller's thread and again in autograd's).  The sizes decide the plan, so nothing has to
 // be thrown away.
 struct LayerPlans {
   int known[5];                                        // 0 not yet, 1 applies, -1 does not
+  int first_known;                                     // 0 not yet, else 1 + the math mode that `first` was made for
+  FirstPlan first;
   size_t bias_bytes;                                   // section 2's weight gradient: for the bias gradient beside it (known[3])
   BlockPlan forward, input;
   BlockWgradPlan weight;
@@ -1989,6 +1994,43 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   (l).dims[0], (l).dims[1], (l).dims[2], (l).dims[3], (l).dims[4], (l).dims[5], (l).dims[6], (l).dims[7], (l).dims[8],  \
       (l).dims[9], (l).dims[10], (l).dims[11], (l).dims[12], (l).dims[13], (l).dims[14], (l).dims[15], (l).dims[16]
 
+// How a stack's first layer runs.  Where its kernel can store blocked tensors its output goes straight into the second
+// layer's input: as a plain tensor it is written, read back and laid out by a pass of its own, three trips to memory more
+// (32 x 780 x 41, 1 -> 32 channels: fp32 141 -> 78 us with the filters' packing, half 70 -> 40), and 131 MB of scratch memory.
+// A backward call, which goes by the forward call's settings whatever has been set since, has no use for it.
+static FirstPlan plan_first_layer(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
+  FirstPlan fp = {};
+  BlockPlan bp;
+  if (plan_block_forward(kind_x, half, CORR2D_ARGS, bp)) {
+    fp.route = blocked_images(batch, c_in, ngx * ngy, half) < batch ? FIRST_OWN : FIRST_BLOCKS;
+    return fp;
+  }
+  if (c_in * nfx * nfy * ngx * ngy == 0) return fp;
+  SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
+  pr.relu = 1;
+  if (half) {
+    HalfNative hn;
+    if (!plan_half_native(pr, hn) || hn.classes || hn.frag_bytes) return fp;
+    fp.tiles = hn.pl; fp.lds = hn.lds; fp.mt = hn.mt; fp.nt = hn.nt;
+  } else {
+    ClassPlans cp;
+    NarrowPlan np;
+    if (plan_mellin_classes(pr, cp) || make_narrow_plan(pr, np, false) || !make_tile_plan(pr, fp.tiles, &fp.lds, &fp.mt, &fp.nt)) return fp;
+  }
+  if (tile_writes_blocked(fp.tiles, fp.mt)) fp.route = FIRST_TILES;
+  return fp;
+}
+static FirstPlan first_layer(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
+  if (g_settled || !blocks_allowed(half)) return FirstPlan{};
+  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
+  const int math = g_math;
+  if (lp.first_known != math + 1) {
+    lp.first = plan_first_layer(kind_x, half, CORR2D_ARGS);
+    lp.first_known = math + 1;
+  }
+  return lp.first;
+}
+
 constexpr int kStackLayers = 64;
 // Partial sums of weight and bias gradients that a stack's backward keeps at a time: those of layers that follow each other
 // are added up by one launch (nine layers, 64 channels and up, 4 x 252 frames, training: 718 -> 673 us with those of nine;
@@ -2008,6 +2050,7 @@ struct StackLayer {
 // needs whichever of the layers above is the lowest that it is asked for.
 struct StackPlan {
   StackLayer l[kStackLayers];
+  FirstPlan first;
   size_t saved, forward, backward;
   size_t f_first, f_own, f_filters, f_unpooled, f_sums, f_turn[2], own_bytes;                          // forward workspace
   size_t b_grad[2], b_unpooled, b_partial, partial_bytes, b_sums, b_first, b_own, b_own_bytes;         // backward workspace
@@ -2081,7 +2124,8 @@ static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const
   auto take = [&](size_t bytes) { const size_t off = at; at += align256(bytes); return off; };
   const StackLayer &l0 = sp.l[0];
   const size_t dense = (size_t)(l0.batch * l0.c_out * l0.q) * (half ? 2 : 4);
-  sp.f_first = take(dense);
+  sp.first = first_layer(kind_x, half, STACK_DIMS(layers[0]));
+  sp.f_first = take(sp.first.route == FIRST_OWN ? dense : 0);
   sp.own_bytes = mellin_layer_forward_workspace(kind_x, elem, STACK_DIMS(layers[0]));
   sp.f_own = take(sp.own_bytes);
   sp.f_filters = take(frags);
@@ -2133,31 +2177,6 @@ static int stack_checks(const char *who, bool planned, const StackPlan &sp, cons
   return MELLIN_OK;
 }
 
-// How a stack's first layer runs.  Where its kernel can store blocked tensors its output goes straight into the second
-// layer's input: as a plain tensor it is written, read back and laid out by a pass of its own, three trips to memory more
-// (32 x 780 x 41, 1 -> 32 channels: fp32 141 -> 78 us with the filters' packing, half 70 -> 40).
-enum FirstLayer { FIRST_OWN, FIRST_BLOCKS, FIRST_TILES };   // a call of its own; the blocked kernels; the tiled kernel
-struct FirstPlan { BlockPlan blocks; TilePlan tiles; size_t lds; int mt, nt; };
-static FirstLayer first_layer(int kind_x, bool half, MELLIN_CORR2D_DIMS, FirstPlan &fp) {
-  if (plan_block_forward(kind_x, half, CORR2D_ARGS, fp.blocks))
-    return blocked_images(batch, c_in, ngx * ngy, half) < batch ? FIRST_OWN : FIRST_BLOCKS;
-  if (c_in * nfx * nfy * ngx * ngy == 0 || g_forced || g_gather > 0) return FIRST_OWN;
-  SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
-  pr.relu = 1;
-  if (half) {
-    HalfNative hn;
-    if (!plan_half_native(pr, hn) || hn.classes || hn.frag_bytes) return FIRST_OWN;
-    fp.tiles = hn.pl; fp.lds = hn.lds; fp.mt = hn.mt; fp.nt = hn.nt;
-  } else {
-    ClassPlans cp;
-    NarrowPlan np;
-    if (plan_mellin_classes(pr, cp) || (g_no_narrow <= 0 && make_narrow_plan(pr, np, g_no_narrow < 0)) ||
-        !make_tile_plan(pr, fp.tiles, &fp.lds, &fp.mt, &fp.nt))
-      return FIRST_OWN;
-  }
-  return tile_writes_blocked(fp.tiles, fp.mt) ? FIRST_TILES : FIRST_OWN;
-}
-
 int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, const mellin_stack_layer *layers, const void *input,
                          void *out, void *saved, size_t saved_bytes, void *workspace, size_t workspace_bytes, void *stream) {
   StackPlan sp;
@@ -2176,8 +2195,8 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
   const mellin_stack_layer &ly0 = layers[0];
   const i64 n_w0 = ly0.dims[1] * ly0.dims[2] * ly0.dims[3] * ly0.dims[4];
   char *own = ws + sp.f_own;
-  FirstPlan fp;
-  const FirstLayer route = first_layer(kind_x, half, STACK_DIMS(ly0), fp);
+  const FirstPlan &fp = sp.first;
+  const FirstLayer route = fp.route;
   hipError_t e = hipSuccess;
   if (route == FIRST_OWN) {
     rc = mellin_layer_forward(kind_x, elem_bytes, MELLIN_ACT_RELU, input, ly0.weight, ly0.bias, STACK_DIMS(ly0), ws + sp.f_first,
@@ -2204,7 +2223,8 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
     e = launch_block_pack(half, &dense, nullptr, filters, n_layers - 1, st);
   } else if (route == FIRST_BLOCKS) {
     const StackLayer &l0 = sp.l[0];
-    BlockPlan &p0 = fp.blocks;
+    BlockPlan p0;
+    plan_block_forward(kind_x, half, STACK_DIMS(ly0), p0);
     p0.relu = 1;
     p0.wide = wide;
     const size_t filter_at = blocked_region(l0.batch, l0.c_in, l0.plane, half), sums_at = filter_at + align256(p0.filter_bytes);

@@ -50,6 +50,32 @@ class _StackLayer(ctypes.Structure):
     _fields_ = [("dims", ctypes.c_int64 * 17), ("pool", ctypes.c_int)] + [(n, ctypes.c_void_p) for n in "weight bias half gw gb".split()]
 
 
+def stack_bytes(batch, frames, bins, params, elem_bytes, train):
+    """What a stack's calls ask for: bytes of what is kept, of the forward and of the backward workspace."""
+    layers, sizes = (_StackLayer * params.layers)(), [ctypes.c_size_t() for _ in range(3)]
+    for layer, dims in zip(layers, stack_dims(batch, frames, bins, params)):
+        layer.dims[:] = dims
+    kind = hip.AX_MCORR if params.mellin else hip.AX_LCORR
+    assert hip.lib.mellin_stack_bytes(kind, elem_bytes, train, params.layers, ctypes.cast(layers, ctypes.c_void_p), *map(ctypes.byref, sizes))
+    return [size.value for size in sizes]
+
+
+@pytest.mark.parametrize("elem_bytes", [4, 2])
+@pytest.mark.parametrize("c_in, kernel, frames, batch, own", [
+    (1, (4, 4), 780, 32, False),                       # the tiled kernel stores the second layer's input
+    (24, (4, 4), 100, 4, False),                       # the blocked kernels do
+    (5, (5, 3), 780, 32, True),                        # float: staged in chunks of channels, and laid out afterwards
+])
+def test_first_layers_output_takes_workspace_where_it_is_a_tensor(c_in, kernel, frames, batch, own, elem_bytes):
+    params = ConvStackParams(layers=2, kernel_time=kernel[0], kernel_freq=kernel[1], initial_channels=32, factor_schedule=2,
+                             time_factor=1, in_channels=c_in)
+    n, _, channels, _, _, ngx, ngy, nhx, nhy = next(iter(stack_dims(batch, frames, 41, params)))[:9]
+    forward = stack_bytes(batch, frames, 41, params, elem_bytes, 1)[1]
+    # (besides: where the blocked kernels take the first layer, its signal in their layout)
+    signal = n * c_in * (ngx * ngy + 1) * (6 if elem_bytes == 4 else 2) if c_in >= 16 else 0
+    assert (forward - signal >= n * channels * nhx * nhy * elem_bytes) == (own and elem_bytes == 4)
+
+
 def test_new_sizes_are_planned_in_little_time():
     """A batch's longest utterance changes from step to step: what the choice of tiles takes comes on top of each.  (A count of all
     tiles of all images for every tile shape took 1150 us, this takes 35.)"""

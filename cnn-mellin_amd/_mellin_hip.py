@@ -88,6 +88,8 @@ SYMBOLS["mellin_layer_forward"] = (_int, [_int, _int, _int, _ptr, _ptr, _ptr] + 
 SYMBOLS["mellin_layer_backward_workspace"] = (_size_t, [_int, _int, _int] + _DIMS)
 SYMBOLS["mellin_layer_backward"] = (_int, [_int, _int, _int] + [_ptr] * 4 + _DIMS + [_ptr] * 4 + [_size_t, _ptr])
 SYMBOLS["mellin_layer_plan"] = (_int, [_int, _int, _int] + _DIMS + [_ptr])
+SYMBOLS["mellin_layer_bias_route"] = (_int, [_int, _int, _int] + _DIMS)
+SYMBOLS["mellin_stack_first_layer"] = (_int, [_int, _int] + _DIMS)
 SYMBOLS["mellin_stack_bytes"] = (_int, [_int, _int, _int, _int] + [_ptr] * 4)
 SYMBOLS["mellin_stack_forward"] = (_int, [_int, _int, _int, _int] + [_ptr] * 4 + [_size_t, _ptr, _size_t, _ptr])
 SYMBOLS["mellin_stack_backward"] = (_int, [_int, _int, _int] + [_ptr] * 5 + [_size_t, _ptr, _ptr, _size_t, _ptr])

@@ -1610,7 +1610,7 @@ static bool blocks_allowed(bool half) {
          !g_no_yfold && !g_gather && !g_no_narrow && (half || g_math != MATH_FP32));
 }
 // How a stack's first layer runs: a call of its own, the blocked kernels, or the tiled kernel with `tiles`.
-enum FirstLayer { FIRST_OWN, FIRST_BLOCKS, FIRST_TILES };
+enum FirstLayer { FIRST_OWN = MELLIN_FIRST_OWN, FIRST_BLOCKS = MELLIN_FIRST_BLOCKS, FIRST_TILES = MELLIN_FIRST_TILES };
 struct FirstPlan { FirstLayer route; TilePlan tiles; size_t lds; int mt, nt; };
 // Plans of the layer entry points, kept per thread: a layer asks for the same ones with every step (its workspace, then
 // the launch), and choosing among tile shapes takes 0.5 to 4 microseconds a pass (ten Mellin layers of a new length: 17 served,
@@ -1989,6 +1989,14 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
 }
 
 
+// (which launches make a layer's bias gradient, for tests)
+int mellin_layer_bias_route(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS) {
+  if (!layer_elements(elem_bytes) || !(want & MELLIN_WANT_BIAS) || check_corr2d(__func__, kind_x, CORR2D_ARGS)) return MELLIN_BIAS_NONE;
+  LayerBackward lb;
+  plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb);
+  return lb.bias_beside ? MELLIN_BIAS_BESIDE_WEIGHT : lb.bias_packed ? MELLIN_BIAS_PACKED : MELLIN_BIAS_OWN;
+}
+
 // ---- stacks --------------------------------------------------------------------------------
 #define STACK_DIMS(l)                                                                                                   \
   (l).dims[0], (l).dims[1], (l).dims[2], (l).dims[3], (l).dims[4], (l).dims[5], (l).dims[6], (l).dims[7], (l).dims[8],  \
@@ -2029,6 +2037,12 @@ static FirstPlan first_layer(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
     lp.first_known = math + 1;
   }
   return lp.first;
+}
+
+// (for tests)
+int mellin_stack_first_layer(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
+  if (!layer_elements(elem_bytes) || check_corr2d(__func__, kind_x, CORR2D_ARGS)) return MELLIN_FIRST_OWN;
+  return first_layer(kind_x, elem_bytes != 4, CORR2D_ARGS).route;
 }
 
 constexpr int kStackLayers = 64;

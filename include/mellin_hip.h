@@ -498,6 +498,20 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
 #define MELLIN_LAYER_PLAN_WORDS 10
 int mellin_layer_plan(int kind_x, int elem_bytes, int gradient, MELLIN_CORR2D_DIMS, int *plan);
 
+/* Where a layer's backward call makes the bias gradient for `want` (for tests): nowhere (not wanted), in launches of its own,
+ * beside the weight gradient, in the pass that lays grad_out out for the blocked kernels. */
+#define MELLIN_BIAS_NONE 0
+#define MELLIN_BIAS_OWN 1
+#define MELLIN_BIAS_BESIDE_WEIGHT 2
+#define MELLIN_BIAS_PACKED 3
+int mellin_layer_bias_route(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS);
+/* How such a layer runs as the first of a stack (for tests): as a layer's forward call, whose output is laid out afterwards, or
+ * by the blocked or the tiled kernel, which store the second layer's input themselves. */
+#define MELLIN_FIRST_OWN 0
+#define MELLIN_FIRST_BLOCKS 1
+#define MELLIN_FIRST_TILES 2
+int mellin_stack_first_layer(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS);
+
 /* Name of the kernel variant the most recent operator-level call of the
  * process (on any thread: PyTorch runs backward passes on a thread of its own)
  * dispatched to (for tests and profiling): "generic", "mfma" (tiled

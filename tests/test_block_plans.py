@@ -29,6 +29,21 @@ def plan(kind, elem_bytes, gradient, dims):
     return dict(zip(WORDS, words))
 
 
+WANT_INPUT, WANT_WEIGHT, WANT_BIAS, WANT_RELU = 1, 2, 4, 8
+BIAS_OWN, BIAS_BESIDE_WEIGHT, BIAS_PACKED = 1, 2, 3
+FIRST_OWN, FIRST_BLOCKS, FIRST_TILES = 0, 1, 2
+
+
+def bias_route(kind, elem_bytes, want, dims):
+    """Where a layer's bias gradient is made: BIAS_*."""
+    return hip.lib.mellin_layer_bias_route(kind, elem_bytes, want, *dims)
+
+
+def first_layer(kind, elem_bytes, dims):
+    """How a layer runs as the first of a stack: FIRST_*."""
+    return hip.lib.mellin_stack_first_layer(kind, elem_bytes, *dims)
+
+
 # (kernel, channels, layers, batch, frames, bins)
 SMALL_IMAGES = [((5, 3), 64, 5, 1177, 10, 41), ((5, 3), 64, 3, 300, 10, 41), ((5, 3), 128, 3, 250, 10, 40), ((4, 3), 128, 4, 200, 7, 23)]
 

@@ -5,9 +5,11 @@ import numpy as np
 import pytest
 import torch
 
+import _mellin_hip as hip
 import mconv
 from _gpu import assert_close, to_gpu
 from oracle import oracle
+from test_block_plans import BIAS_BESIDE_WEIGHT, BIAS_OWN, WANT_BIAS, WANT_WEIGHT, bias_route
 
 pytestmark = pytest.mark.gpu
 
@@ -21,8 +23,11 @@ CASES = [
     ("mcorr", 9, 3, 64, (8, 4), (301, 41), (0, 0), (0, 0)),
     ("mcorr", 5, 7, 50, (6, 2), (400, 20), (1, 0), (0, 0)),          # odd rows of 19
     ("mcorr", 6, 2, 129, (3, 3), (200, 41), (0, 1), (0, 1)),
-    ("mcorr", 4, 3, 64, (4, 4), (200, 41), (1, 1), (100, 1)),        # rows past the support: a launch of its own
+    ("mcorr", 4, 3, 64, (4, 4), (200, 41), (1, 1), (100, 1)),        # more rows than whole filters reach
+    ("mcorr", 4, 3, 64, (4, 4), (200, 41), (1, 1), (350, 1)),        # rows past the support: a launch of its own
 ]
+#: where a bias gradient wanted with the weight gradient is made
+ROUTES = 9 * [BIAS_BESIDE_WEIGHT] + [BIAS_OWN]
 
 
 @pytest.mark.parametrize("offset", [0.0, 3.0], ids=["centred", "offset"])
@@ -34,6 +39,8 @@ def test_bias_gradient_beside_the_weight_gradient(case, offset):
     w = rng.standard_normal((c_out, c_in) + nf).astype(np.float32)
     xg, wg, bg = to_gpu(x), to_gpu(w).requires_grad_(), torch.zeros(c_out, device="cuda", requires_grad=True)
     out = (mconv._ext_mcorrlcorr if op == "mcorr" else mconv._ext_lcorrlcorr)(xg, wg, bg, (1, 1), (1, 1), p, (1, 1), r)
+    assert bias_route(hip.AX_MCORR if op == "mcorr" else hip.AX_LCORR, 4, WANT_WEIGHT | WANT_BIAS,
+                      [n, c_in, c_out, *nf, *ng, *out.shape[2:], 1, 1, 1, 1, *p, 1, 1]) == ROUTES[CASES.index(case)]
     go = (rng.standard_normal(tuple(out.shape)) + offset).astype(np.float32)
     out.backward(to_gpu(go))
     go64 = go.astype(np.float64)
@@ -57,5 +64,4 @@ def test_weight_gradient_has_the_same_bits_without_a_bias(case):
     layer = mconv._ext_mcorrlcorr if op == "mcorr" else mconv._ext_lcorrlcorr
     outs = [layer(x, w, bias, (1, 1), (1, 1), p, (1, 1), r) for bias in (b, None)]
     go = torch.randn_like(outs[0])
-    grads = [torch.autograd.grad(out, w, go)[0] for out in outs[1:]] + [torch.autograd.grad(outs[0], (w, b), go)[0]]
-    assert torch.equal(*grads)
+    assert torch.equal(torch.autograd.grad(outs[0], (w, b), go)[0], torch.autograd.grad(outs[1], w, go)[0])

@@ -4,8 +4,10 @@ import numpy as np
 import pytest
 import torch
 
+import _mellin_hip as hip
 import mconv
 from _gpu import assert_close, to_gpu
+from test_block_plans import BIAS_PACKED, WANT_BIAS, WANT_INPUT, WANT_RELU, WANT_WEIGHT, bias_route
 
 pytestmark = pytest.mark.gpu
 
@@ -23,6 +25,8 @@ def test_bias_gradient_beside_blocked_input_gradient(shape, relu, kind):
     xg, wg, bg = (to_gpu(a).requires_grad_() for a in (x, w, b))
     with torch.autocast("cuda", torch.float16, enabled=kind == "amp"):
         out = mconv._ext_mcorr1d(xg, wg, bg, 1, 2, 1, 1, 0, "relu" if relu else None)
+    assert bias_route(hip.AX_MCORR, 4 if kind == "f32" else 2, WANT_INPUT | WANT_WEIGHT | WANT_BIAS | (WANT_RELU if relu else 0),
+                      [n, c_in, c_out, 8, 1, t, 1, out.shape[2], 1, 1, 1, 2, 1, 1, 0, 1, 1]) == BIAS_PACKED
     go = to_gpu(rng.standard_normal(tuple(out.shape)).astype(np.float16 if out.dtype == torch.float16 else np.float32))
     out.backward(go)
     g = go.double().cpu().numpy() * ((out.detach() > 0).cpu().numpy() if relu else 1)

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+import _mellin_hip as hip
 import mconv
 from _gpu import assert_close, to_gpu
 from oracle import oracle
@@ -42,6 +43,7 @@ def test_weight_gradient_matches_checker(case, half):
     bwd = oracle.mcorrlcorr_backward if op == "mcorr" else oracle.lcorrlcorr_backward
     ref = bwd(x.astype(np.float64), w.astype(np.float64), go.astype(np.float64), s, d, p, u)[1]
     out.backward(to_gpu(go))
+    assert hip.last_variant() == ("mfma-f16-blocks" if half else "mfma-blocks")
     positions = n * out.shape[2] * out.shape[3]
     if half:                                           # one rounding of a result whose sum has an error of its own
         err = np.abs(wg.grad.double().cpu().numpy() - ref)

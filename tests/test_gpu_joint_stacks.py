@@ -1,6 +1,7 @@
 """Input gradients inside a stack whose tiles run over the images of an output row, in every form their ending takes there --
-masked, blocked, with the channels' sums; whole tiles, tiles in slices of the contracted channels, both; wavefronts that share a
-tile, wavefronts along the channels -- against the same layers called one by one, whose gradients are plain tensors."""
+masked, blocked, with the channels' sums, or blocked alone above a pooling; whole tiles, tiles in slices of the contracted
+channels, both; wavefronts that share a tile, wavefronts along the channels -- against the same layers called one by one, whose
+gradients are plain tensors."""
 import pytest
 import torch
 
@@ -13,29 +14,40 @@ pytestmark = pytest.mark.gpu
 WHOLE, SLICES = (True, False), (False, True)
 CASES = [
     # (element bytes, (wavefronts along the channels, that share a tile), (whole tiles, in slices), the layer (its input gradient),
-    #  layers, kernel, channels, schedule, channel_factor, time_factor, batch, frames, bins)
-    (4, (1, 1), WHOLE, 2, 4, (5, 3), 32, 3, 1, 1, 60, 60, 5),
-    (4, (1, 1), SLICES, 2, 4, (5, 3), 96, 4, 1, 1, 2, 5, 5),
-    (4, (1, 1), (True, True), 2, 4, (3, 4), 96, 2, 2, 1, 60, 10, 20),
-    (4, (1, 4), WHOLE, 2, 4, (4, 4), 64, 3, 1, 2, 2, 10, 5),
-    (4, (1, 4), SLICES, 2, 4, (3, 4), 64, 3, 2, 2, 4, 5, 3),
-    (4, (2, 1), WHOLE, 3, 4, (3, 3), 128, 3, 2, 1, 60, 120, 3),
-    (4, (2, 1), SLICES, 2, 3, (5, 2), 128, 2, 2, 1, 300, 5, 3),
-    (4, (2, 1), (True, True), 3, 4, (4, 1), 64, 2, 2, 1, 300, 60, 5),
-    (2, (1, 1), WHOLE, 3, 4, (4, 3), 32, 4, 1, 2, 60, 120, 5),
-    (2, (1, 1), SLICES, 3, 4, (5, 3), 128, 2, 2, 1, 150, 5, 10),
-    (2, (1, 1), (True, True), 3, 4, (5, 4), 96, 2, 2, 1, 150, 60, 5),
-    (2, (1, 4), WHOLE, 2, 3, (5, 4), 64, 3, 2, 1, 4, 5, 10),
-    (2, (1, 4), SLICES, 3, 4, (5, 3), 128, 2, 2, 1, 9, 5, 10),
-    (2, (2, 1), WHOLE, 2, 4, (4, 1), 64, 2, 2, 1, 300, 60, 5),
+    #  layers, kernel, channels, schedule, channel_factor, time_factor, batch, frames, bins, pooled behind the layer)
+    (4, (1, 1), WHOLE, 2, 4, (5, 3), 32, 3, 1, 1, 60, 60, 5, None),
+    (4, (1, 1), SLICES, 2, 4, (5, 3), 96, 4, 1, 1, 2, 5, 5, None),
+    (4, (1, 1), (True, True), 2, 4, (3, 4), 96, 2, 2, 1, 60, 10, 20, None),
+    (4, (1, 4), WHOLE, 2, 4, (4, 4), 64, 3, 1, 2, 2, 10, 5, None),
+    (4, (1, 4), SLICES, 2, 4, (3, 4), 64, 3, 2, 2, 4, 5, 3, None),
+    (4, (2, 1), WHOLE, 3, 4, (3, 3), 128, 3, 2, 1, 60, 120, 3, None),
+    (4, (2, 1), SLICES, 2, 3, (5, 2), 128, 2, 2, 1, 300, 5, 3, None),
+    (4, (2, 1), (True, True), 3, 4, (4, 1), 64, 2, 2, 1, 300, 60, 5, None),
+    (2, (1, 1), WHOLE, 3, 4, (4, 3), 32, 4, 1, 2, 60, 120, 5, None),
+    (2, (1, 1), SLICES, 3, 4, (5, 3), 128, 2, 2, 1, 150, 5, 10, None),
+    (2, (1, 1), (True, True), 3, 4, (5, 4), 96, 2, 2, 1, 150, 60, 5, None),
+    (2, (1, 4), WHOLE, 2, 3, (5, 4), 64, 3, 2, 1, 4, 5, 10, None),
+    (2, (1, 4), SLICES, 3, 4, (5, 3), 128, 2, 2, 1, 9, 5, 10, None),
+    (2, (2, 1), WHOLE, 2, 4, (4, 1), 64, 2, 2, 1, 300, 60, 5, None),
+    (4, (1, 1), WHOLE, 2, 4, (5, 3), 32, 3, 1, 2, 60, 60, 10, 2),
+    (4, (1, 1), SLICES, 2, 3, (5, 3), 96, 4, 2, 1, 2, 5, 10, 2),
+    (4, (1, 1), (True, True), 2, 3, (4, 4), 96, 3, 1, 2, 9, 252, 20, 2),
+    (4, (1, 4), WHOLE, 2, 4, (5, 4), 32, 4, 1, 2, 4, 5, 10, 2),
+    (4, (1, 4), SLICES, 2, 4, (4, 3), 128, 3, 2, 1, 2, 5, 5, 2),
+    (4, (2, 1), WHOLE, 2, 3, (5, 1), 128, 2, 2, 1, 300, 20, 7, 2),
+    (4, (2, 1), SLICES, 2, 4, (5, 2), 128, 2, 2, 1, 60, 5, 41, 2),
+    (2, (1, 1), WHOLE, 2, 3, (4, 3), 32, 3, 2, 2, 60, 120, 10, 2),
+    (2, (1, 4), WHOLE, 2, 3, (5, 4), 32, 3, 2, 2, 4, 10, 7, 2),
+    (2, (1, 4), SLICES, 2, 4, (5, 4), 128, 3, 2, 2, 9, 10, 7, 2),
 ]
 
 
 @pytest.mark.parametrize("case", CASES, ids=[str(i) for i in range(len(CASES))])
-def test_masked_blocked_endings_of_joint_tiles(case):
-    elem_bytes, wavefronts, tiles, layer, layers, kernel, channels, schedule, cf, tf, batch, frames, bins = case
+def test_blocked_endings_of_joint_tiles(case):
+    elem_bytes, wavefronts, tiles, layer, layers, kernel, channels, schedule, cf, tf, batch, frames, bins, pooled = case
     params = ConvStackParams(layers=layers, kernel_time=kernel[0], kernel_freq=kernel[1], initial_channels=channels,
-                             factor_schedule=schedule, channel_factor=cf, time_factor=tf, in_channels=1)
+                             factor_schedule=schedule, channel_factor=cf, time_factor=tf, in_channels=1,
+                             freq_pool_after=(pooled,) if pooled else ())
     p = plan(hip.AX_MCORR, elem_bytes, 1, list(stack_dims(batch, frames, bins, params))[layer])
     assert p["joint"] and (p["wm"], p["wk"]) == wavefronts and (p["whole"] > 0, p["rest"] > 0) == tiles, p
     torch.manual_seed(9700 + CASES.index(case))

@@ -25,8 +25,8 @@
 // of a tile have taps for the same filter rows and only those are staged and multiplied; filter
 // rows none of whose taps lies inside the signal for the tile's rows are left out as well.
 //
-// Small images on Mellin axes (JOINT): a tile's positions run over the images of an output row, whose rows have taps for the
-// same filter rows; its virtual rows are those of (output row, image) pairs.
+// Input gradients of small images on Mellin axes (JOINT): a tile's positions run over the images of an output row, whose rows
+// have taps for the same filter rows; its virtual rows are those of (output row, image) pairs.
 //
 // Few tiles (one utterance, deep layers): WK = 4 wavefronts share the positions of a tile and
 // take every fourth step of a stage; their sums are added in wavefront order through LDS.
@@ -205,7 +205,9 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   // Wavefronts that share a tile, 2, 4 or 8 tiles of channels: XCD k (workgroups k, k + 8, ...) takes one of those, and its
   // share of the filter is all that the XCD's L2 sees: one utterance of a Mellin stack, layers of 128 to 256 channels on 337 x
   // 10 and 337 x 5, 16.9, 17.9, 26.2 and 36.2 us -> 15.9, 16.8, 24.5 and 35.3.  (Filters below 1 MB: nothing gained;
-  // 41 -> 128 channels on one axis 84.2 -> 86.0 us a step.)  The position tiles are dealt to a tile of channels' XCDs in turn: those of a
+  // 41 -> 128 channels on one axis 84.2 -> 86.0 us a step.  Other numbers of tiles do not divide the XCDs evenly: of three
+  // the slowest would have two XCDs for a third of the work, 1.3 times an even share, of five, six and seven one for a fifth,
+  // a sixth and a seventh, 1.6, 1.3 and 1.1 times.)  The position tiles are dealt to a tile of channels' XCDs in turn: those of a
   // class with many filter rows follow each other, and an eighth of all tiles without a gap left XCDs waiting (113 us).
   int m_tile = blockIdx.y, item = blockIdx.x;
   if constexpr (WK > 1)

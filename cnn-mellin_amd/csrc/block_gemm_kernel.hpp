@@ -115,34 +115,6 @@ __device__ __forceinline__ BlockTile block_tile(ConstBlockPlan &pl, const int2 *
 
 typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
 
-// Value `I` of the four lanes that this lane belongs to; the lanes' values exchanged in pairs.
-template <int I>
-__device__ __forceinline__ int quad_lane(int v) { return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xf, 0xf, true); }
-__device__ __forceinline__ unsigned swap1(unsigned v) { return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true); }
-__device__ __forceinline__ unsigned swap2(unsigned v) { return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true); }
-
-// 4 x 4 transpose over four neighbouring lanes: lane j gets the four lanes' values v[j].
-__device__ __forceinline__ uintx4 transpose_words(const float4 &v, int lane) {
-  const unsigned a = __float_as_uint(v.x), b = __float_as_uint(v.y), c = __float_as_uint(v.z), d = __float_as_uint(v.w);
-  const bool odd = lane & 1, upper = lane & 2;
-  const unsigned a1 = swap1(a), b1 = swap1(b), c1 = swap1(c), d1 = swap1(d);     // (by every lane, so not in the selections)
-  const unsigned n0 = odd ? b1 : a, n1 = odd ? b : a1, n2 = odd ? d1 : c, n3 = odd ? d : c1;
-  const unsigned m0 = swap2(n0), m1 = swap2(n1), m2 = swap2(n2), m3 = swap2(n3);
-  return uintx4{upper ? m2 : n0, upper ? m3 : n1, upper ? n2 : m0, upper ? n3 : m1};
-}
-// the same of values rounded to half
-__device__ __forceinline__ uintx2 transpose_half(const float4 &v, int lane) {
-  auto pair = [](float lo, float hi) {
-    return (unsigned)__builtin_bit_cast(unsigned short, (_Float16)lo) | ((unsigned)__builtin_bit_cast(unsigned short, (_Float16)hi) << 16);
-  };
-  const unsigned ab = pair(v.x, v.y), cd = pair(v.z, v.w);
-  const bool odd = lane & 1, upper = lane & 2;
-  const unsigned ab2 = swap2(ab), cd2 = swap2(cd);
-  const unsigned n0 = upper ? cd2 : ab, n1 = upper ? cd : ab2;                   // two channels at positions 0/1 and 2/3
-  const unsigned sel = odd ? 0x03020706u : 0x05040100u;                          // high halves (other, own) or low halves (own, other)
-  return uintx2{__builtin_amdgcn_perm(swap1(n0), n0, sel), __builtin_amdgcn_perm(swap1(n1), n1, sel)};
-}
-
 // Sums of sixteen values over the 32 lanes of each half of a wavefront: lane 16 a + 8 b + 4 c + 2 d + e of a half gets the
 // sum of value 8 a + 4 b + 2 c + d (halves of the values exchanged at each step: 38 additions instead of 80).
 __device__ __forceinline__ float lane_sums(const float (&v)[16], int lane) {
@@ -175,6 +147,19 @@ __device__ __forceinline__ float lane_sums(const float (&v)[16], int lane) {
   const float keep = up ? c[1] : c[0], send = up ? c[0] : c[1];
   const float d = keep + other(send, 2);
   return d + other(d, 1);
+}
+
+// A value, and a buffer descriptor of `bytes` at `base`, that are the same in every lane.  Said here: the compiler takes what
+// comes from a tile's fields for values of a lane, and then repeats every store for each descriptor that it finds among the
+// lanes (a dozen more instructions a store; 33 -> 67 channels, 5 x 3 taps, 7 x 333 x 37 half values: 39.7 us with that and
+// stores of four transposed positions, 23.9 without).
+__device__ __forceinline__ int wave_value(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ char *wave_value(const void *p) {
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)(size_t)p), hi = __builtin_amdgcn_readfirstlane((unsigned)((size_t)p >> 32));
+  return (char *)((unsigned long long)hi << 32 | lo);
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t wave_buffer(const void *base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(wave_value(base), 0, wave_value(bytes), 0x00020000);
 }
 
 template <int MT, int NT, int WM, int WK, bool F16, int OUT, bool JOINT>
@@ -523,7 +508,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       const int all_images = (int)image_bytes * (JOINT ? pl.batch : 1);
       __amdgpu_buffer_rsrc_t mask_rsrc;
       if constexpr (GRAD)
-        mask_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(mask) + tg.n * image_bytes, 0, all_images, 0x00020000);
+        mask_rsrc = wave_buffer(mask + tg.n * image_bytes, all_images);
       int unit_at[NT];                                 // the lane's quarter unit in its group (none: past any end)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
@@ -546,12 +531,11 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       // lanes without a position (an offset past any end) are dropped by its range check.  A slice's sums are fp32, in
       // the order of the tile.
       const bool as_half = F16 && !BLOCKED && whole;
-      const int ES = as_half ? 2 : 4, h_m = (whole ? (int)pl.h_m : P) * ES;
-      char *base = whole ? (char *)Hv + ((i64)tg.n * pl.h_n + (i64)m0 * (int)pl.h_m) * ES
-                         : (char *)(sums + (((i64)tg.slot * pl.m_tiles + m_tile) * M_T + wm * MT * 32) * P);
-      const __amdgpu_buffer_rsrc_t rsrc =
-          BLOCKED && whole ? __builtin_amdgcn_make_buffer_rsrc((char *)Hv + tg.n * image_bytes, 0, all_images, 0x00020000)
-                           : __builtin_amdgcn_make_buffer_rsrc(base, 0, max(0, min(MT * 32, pl.M - m0)) * h_m + (whole && JOINT ? (pl.batch - 1) * (int)pl.h_n * ES : 0), 0x00020000);
+      const int ES = as_half ? 2 : 4, h_m = wave_value((whole ? (int)pl.h_m : P) * ES);
+      char *const base = wave_value(whole ? (char *)Hv + ((i64)tg.n * pl.h_n + (i64)m0 * (int)pl.h_m) * ES
+                                          : (char *)(sums + (((i64)tg.slot * pl.m_tiles + m_tile) * M_T + wm * MT * 32) * P));
+      const int base_bytes = wave_value(max(0, min(MT * 32, pl.M - m0)) * h_m + (whole && JOINT ? (pl.batch - 1) * (int)pl.h_n * ES : 0));
+      const __amdgpu_buffer_rsrc_t rsrc = BLOCKED && whole ? wave_buffer((char *)Hv + tg.n * image_bytes, all_images) : wave_buffer(base, base_bytes);
       int at[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
@@ -563,7 +547,6 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
         else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rsrc, to, 0, 0);
       };
       auto relu4 = [&](float4 v) { return !GRAD && relu ? make_float4(fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f)) : v; };
-      auto last4 = [&](float4 v) { return BLOCKED ? v : relu4(v); };       // (blocked: of slices only)
       auto store_four = [&](float4 v, int to) {        // four channels of the lane's position
         store_one(v.x, to);
         store_one(v.y, to + h_m);
@@ -644,6 +627,29 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
             }
           }
         }
+        if constexpr (!GRAD)
+          if (relu)
+#pragma unroll
+            for (int k = 0; k < MT; ++k)
+#pragma unroll
+              for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[k][t][r] = fmaxf(acc[k][t][r], 0.f);
+        // Tensors as they lie, and slices: a value at a time, 32 positions of a channel side by side.  (Four positions a lane,
+        // by transposes over four lanes, are a quarter of the stores but no fewer bytes or lines: stores alone, 64 channels x
+        // 256 positions a workgroup, fp32 18.7 us in singles and 20.7 in fours, half 13.0 and 26.8 where channels have an odd
+        // number of positions.)
+        auto store_all = [&](auto store) {
+#pragma unroll
+          for (int k = 0; k < MT; ++k)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              const int row = k * 32 + (r >> 2) * 8 + (r & 3);                   // (and four further on in the upper half)
+              const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(base + row * h_m, 0, max(0, base_bytes - row * h_m), 0x00020000);
+#pragma unroll
+              for (int t = 0; t < NT; ++t) store(acc[k][t][r], to, at[t] + row0);
+            }
+        };
         if (BLOCKED && whole) {
           // the halves of a wavefront exchange quarters, so that a lane stores whole units: the lower one groups 0 and 2
           // of a tile's four, the upper one groups 1 and 3
@@ -657,8 +663,8 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
 #pragma unroll
               for (int t = 0; t < NT; ++t) {
                 unsigned lo[PARTS][2], hi[PARTS][2];
-                cut_four<F16>(relu4(make_float4(acc[k][t][4 * p2], acc[k][t][4 * p2 + 1], acc[k][t][4 * p2 + 2], acc[k][t][4 * p2 + 3])), lo);
-                cut_four<F16>(relu4(make_float4(acc[k][t][4 * p2 + 4], acc[k][t][4 * p2 + 5], acc[k][t][4 * p2 + 6], acc[k][t][4 * p2 + 7])), hi);
+                cut_four<F16>(make_float4(acc[k][t][4 * p2], acc[k][t][4 * p2 + 1], acc[k][t][4 * p2 + 2], acc[k][t][4 * p2 + 3]), lo);
+                cut_four<F16>(make_float4(acc[k][t][4 * p2 + 4], acc[k][t][4 * p2 + 5], acc[k][t][4 * p2 + 6], acc[k][t][4 * p2 + 7]), hi);
 #pragma unroll
                 for (int pt = 0; pt < PARTS; ++pt) {
                   const auto s0 = __builtin_amdgcn_permlane32_swap(lo[pt][0], hi[pt][0], false, false);
@@ -669,45 +675,12 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
                 __builtin_amdgcn_sched_barrier(0);     // (one block's registers at a time)
               }
             }
+        } else if (as_half) {
+          store_all([](float v, const __amdgpu_buffer_rsrc_t &to, int at) {
+            __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(short, (_Float16)v), to, at, 0, 0);
+          });
         } else {
-        // A 4 x 4 transpose over four lanes makes four channels of a position four positions of a channel, side by side
-        // in memory: a quarter of the stores (128 x 256 half values: 22000 -> 12000 cycles).  Not for the rows of a class
-        // (n_classes > 1), which do not follow each other; the last positions of an image, less than four, go one by one.
-        bool single = true;
-        if (BLOCKED || (pl.n_classes == 1 && !JOINT) || !whole) {
-          int to[NT];
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            const int first = quad_lane<0>(at[t]), last = quad_lane<3>(at[t]);
-            to[t] = last >= 0 ? row0 + (lane & 3) * h_m + first : (int)0x80000000u;
-            if (last >= 0) at[t] = (int)0x80000000u;
-          }
-#pragma unroll
-          for (int k = 0; k < MT; ++k)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4)
-#pragma unroll
-              for (int t = 0; t < NT; ++t) {
-                const float4 v = last4(make_float4(acc[k][t][4 * g4], acc[k][t][4 * g4 + 1], acc[k][t][4 * g4 + 2], acc[k][t][4 * g4 + 3]));
-                if (as_half) __builtin_amdgcn_raw_buffer_store_b64(transpose_half(v, lane), rsrc, to[t], 0, 0);
-                else __builtin_amdgcn_raw_buffer_store_b128(transpose_words(v, lane), rsrc, to[t], 0, 0);
-                to[t] += 8 * h_m;
-              }
-          single = tg.count & 3;
-        }
-        if (single) {
-#pragma unroll
-          for (int t = 0; t < NT; ++t) at[t] += row0;
-#pragma unroll
-          for (int k = 0; k < MT; ++k)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4)
-#pragma unroll
-              for (int t = 0; t < NT; ++t) {
-                store_four(last4(make_float4(acc[k][t][4 * g4], acc[k][t][4 * g4 + 1], acc[k][t][4 * g4 + 2], acc[k][t][4 * g4 + 3])), at[t]);
-                at[t] += 8 * h_m;
-              }
-        }
+          store_all([](float v, const __amdgpu_buffer_rsrc_t &to, int at) { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), to, at, 0, 0); });
         }
       }
       if constexpr (BLOCKED)

@@ -1624,9 +1624,10 @@ struct LayerPlans {
   BlockPlan forward, input;
   BlockWgradPlan weight;
 };
-static LayerPlans &layer_plans(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
+// (pool: a pass beside frequency pooling: the kind of BlockPool, and 4 for an odd number of columns in front of it)
+static LayerPlans &layer_plans(int kind_x, bool half, MELLIN_CORR2D_DIMS, int pool = 0) {
   static thread_local PlanTable<LayerPlans, 64, 18> table;
-  return table.at({kind_x * 2 + half + 1, CORR2D_ARGS});
+  return table.at({pool * 16 + kind_x * 2 + half + 1, CORR2D_ARGS});
 }
 // Layers with few channels leave most of a channel block empty, and have kernels of their own in section 2.  Measured over
 // 80 layers with 1 to 15 input channels: for the gradients of short layers, bound by launches (up to these
@@ -1676,24 +1677,32 @@ static bool blocks_apply(int pass, int kind_x, bool half, MELLIN_CORR2D_DIMS) {
   if (pass != PASS_INPUT) return false;
   return (half && kind_x == AX_LCORR && c_in >= 8 && nfx * nfy <= 16) || few_channels_input(kind_x, half, CORR2D_ARGS);
 }
-static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp) {
+// (pooled: pairs of the output's columns are pooled behind the layer, by the kernel if the plan's `pool` says so)
+static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp, bool pooled = false) {
   if (!blocks_apply(PASS_FORWARD, kind_x, half, CORR2D_ARGS)) return false;
-  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
+  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS, pooled);
   if (!lp.known[0]) {
     SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
     pr.out_half = half;
-    lp.known[0] = make_block_plan(pr, half, false, lp.forward) ? 1 : -1;
+    bool applies = make_block_plan(pr, half, false, BlockPool{}, nullptr, bp);
+    lp.forward = bp;
+    if (applies && pooled) {
+      pr.y.nh -= pr.y.nh & 1;
+      if (!make_block_plan(pr, half, false, BlockPool{1, (int)nhy}, &bp, lp.forward)) lp.forward = bp;
+    }
+    lp.known[0] = applies ? 1 : -1;
   }
   if (lp.known[0] > 0) bp = lp.forward;
   return lp.known[0] > 0;
 }
-static bool plan_block_input(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp) {
+// (pooled_cols: the columns that were pooled into the layer's input, or 0)
+static bool plan_block_input(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp, i64 pooled_cols = 0) {
   if (!blocks_apply(PASS_INPUT, kind_x, half, CORR2D_ARGS)) return false;
-  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
+  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS, pooled_cols ? 2 + 4 * (pooled_cols & 1) : 0);
   if (!lp.known[1]) {
     SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
     pr.out_half = half;
-    lp.known[1] = make_block_plan(pr, half, true, lp.input) ? 1 : -1;
+    lp.known[1] = make_block_plan(pr, half, true, BlockPool{pooled_cols ? 2 : 0, (int)pooled_cols}, nullptr, lp.input) ? 1 : -1;
   }
   if (lp.known[1] > 0) bp = lp.input;
   return lp.known[1] > 0;
@@ -1743,10 +1752,10 @@ int mellin_layer_plan(int kind_x, int elem_bytes, int gradient, MELLIN_CORR2D_DI
   if (!plan || !layer_elements(elem_bytes) || check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
   const bool half = elem_bytes != 4;
   BlockPlan bp;
-  if (!(gradient ? plan_block_input(kind_x, half, CORR2D_ARGS, bp) : plan_block_forward(kind_x, half, CORR2D_ARGS, bp))) return 0;
+  if (!(gradient == 1 ? plan_block_input(kind_x, half, CORR2D_ARGS, bp) : plan_block_forward(kind_x, half, CORR2D_ARGS, bp, gradient == 2))) return 0;
   const int words[MELLIN_LAYER_PLAN_WORDS] = {bp.mt, bp.nt, bp.wm, bp.wk, bp.joint, bp.F, bp.G, bp.whole, bp.rest, bp.slices};
   std::copy(words, words + MELLIN_LAYER_PLAN_WORDS, plan);
-  return 1;
+  return bp.pool ? 2 : 1;
 }
 
 size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
@@ -2067,13 +2076,13 @@ struct StackPlan {
   FirstPlan first;
   size_t saved, forward, backward;
   size_t f_first, f_own, f_filters, f_unpooled, f_sums, f_turn[2], own_bytes;                          // forward workspace
-  size_t b_grad[2], b_unpooled, b_partial, partial_bytes, b_sums, b_first, b_own, b_own_bytes;         // backward workspace
+  size_t b_grad[2], b_partial, partial_bytes, b_sums, b_first, b_own, b_own_bytes;         // backward workspace
 };
 static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const mellin_stack_layer *layers, StackPlan &sp) {
   const bool half = elem != 4;
   if (n < 2 || n > kStackLayers || first < 0 || first >= n) return false;
   size_t saved = 0, in_turn[2] = {0, 0}, frags = 0, unpooled = 0, sums = 0, x_bytes[kStackLayers], which_bytes[kStackLayers];
-  size_t grad[2] = {0, 0}, b_unpooled = 0, b_frags = 0, b_sums = 0, partials = 0, most_partials = 0;
+  size_t grad[2] = {0, 0}, b_frags = 0, b_sums = 0, partials = 0, most_partials = 0;
   auto region = [&](i64 channels, i64 plane, i64 batch) { return align256(blocked_bytes(batch, channels, plane, half)); };
   for (int i = 0; i < n; ++i) {
     const mellin_stack_layer &ly = layers[i];
@@ -2087,26 +2096,21 @@ static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const
     const mellin_stack_layer &before = layers[i - 1];
     if (l.c_in != before.dims[2] || ly.dims[5] != before.dims[7] || ly.dims[6] != (before.pool ? before.dims[8] / 2 : before.dims[8])) return false;
     BlockPlan bp;
-    if (!plan_block_forward(kind_x, half, STACK_DIMS(ly), bp)) return false;
+    if (!plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool)) return false;
     x_bytes[i] = region(l.c_in, l.plane, l.batch);
     which_bytes[i] = before.pool ? align256((size_t)(l.batch * ((l.c_in + 7) / 8) * l.plane) * 8) : 0;
     l.frag_off = frags;                                // (forward; the backward call lays out its own)
     frags += align256(bp.filter_bytes);
     sums = std::max(sums, bp.slice_bytes);
-    if (ly.pool) unpooled = std::max(unpooled, region(l.c_out, l.q, l.batch));
+    if (ly.pool && !bp.pool) unpooled = std::max(unpooled, region(l.c_out, l.q, l.batch));
     if (!train) continue;
     BlockPlan ip;
     BlockWgradPlan wp;
-    if (!plan_block_input(kind_x, half, STACK_DIMS(ly), ip) || !plan_block_weight(kind_x, half, STACK_DIMS(ly), wp)) return false;
+    if (!plan_block_input(kind_x, half, STACK_DIMS(ly), ip, before.pool ? before.dims[8] : 0) || !plan_block_weight(kind_x, half, STACK_DIMS(ly), wp)) return false;
     b_frags += align256(ip.filter_bytes);
     b_sums = std::max(b_sums, ip.slice_bytes);
     grad[i & 1] = std::max(grad[i & 1], region(l.c_out, l.q, l.batch));
-    if (before.pool) {
-      b_unpooled = std::max(b_unpooled, region(l.c_in, l.plane, l.batch));
-      sp.l[i - 1].bias_bytes = align256(pool_partial_count(l.batch, l.c_in, before.dims[7], before.dims[8]) * 4);
-    } else {
-      sp.l[i - 1].bias_bytes = align256((size_t)l.c_in * ip.chan_slots * 4);
-    }
+    sp.l[i - 1].bias_bytes = align256((size_t)l.c_in * ip.chan_slots * 4);
     const size_t both = align256(wp.ws_bytes) + sp.l[i - 1].bias_bytes;
     partials += both;
     most_partials = std::max(most_partials, both);
@@ -2152,7 +2156,6 @@ static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const
   if (!train) return true;
   sp.b_grad[0] = take(grad[0]);
   sp.b_grad[1] = take(grad[1]);
-  sp.b_unpooled = take(b_unpooled);
   sp.partial_bytes = std::min(partials, std::max(kStackPartialBytes, most_partials));
   sp.b_partial = take(sp.partial_bytes);
   sp.b_sums = take(b_sums);
@@ -2162,7 +2165,7 @@ static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const
   sp.backward = at + b_frags;
   for (int i = 1; i < n; ++i) {
     BlockPlan ip;
-    plan_block_input(kind_x, half, STACK_DIMS(layers[i]), ip);
+    plan_block_input(kind_x, half, STACK_DIMS(layers[i]), ip, layers[i - 1].pool ? layers[i - 1].dims[8] : 0);
     sp.l[i].frag_off = at;                             // (with train: the backward's; mellin_stack_forward counts its own)
     at += align256(ip.filter_bytes);
   }
@@ -2223,7 +2226,7 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
   BlockPlan bp;
   for (int i = 1; i < n_layers; ++i) {
     const mellin_stack_layer &ly = layers[i];
-    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp);
+    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool);
     bp.wide = wide;
     filters[i - 1] = pack_filter(bp, (int)ly.dims[1], ly.weight, ws + at, wide ? ly.weight_half : nullptr,
                                  ly.dims[1] * ly.dims[2] * ly.dims[3] * ly.dims[4]);
@@ -2270,20 +2273,21 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
     const mellin_stack_layer &ly = layers[i];
     const StackLayer &l = sp.l[i];
     const bool last = i == n_layers - 1;
-    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp);
+    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool);
     bp.relu = 1;
     bp.wide = wide;
-    char *to = last ? (char *)out : ly.pool ? ws + sp.f_unpooled : input_of(i + 1);
-    const BlockGemmArgs args = {input_of(i), ws + frag_off[i], ly.bias, to, (float *)(ws + sp.f_sums), !last, false, nullptr, nullptr};
+    char *const which = ly.pool && train && i + 1 > first ? keep + sp.l[i + 1].which_off : nullptr;
+    const bool pool_after = ly.pool && !bp.pool;
+    char *to = last ? (char *)out : pool_after ? ws + sp.f_unpooled : input_of(i + 1);
+    const BlockGemmArgs args = {input_of(i), ws + frag_off[i], ly.bias, to, (float *)(ws + sp.f_sums), !last, false, nullptr, nullptr, which};
     e = launch_block_gemm(bp, args, st);
     if (e == hipSuccess && bp.rest > 0) {
       BlockFinish fin = {};
       fin.slices = &bp; fin.args = args;
       e = launch_block_finish(half, wide, fin, st);
     }
-    if (e == hipSuccess && ly.pool)
-      e = launch_block_pool(half, to, l.batch, l.c_out, l.rows, l.cols, input_of(i + 1),
-                            train && i + 1 > first ? keep + sp.l[i + 1].which_off : nullptr, st);
+    if (e == hipSuccess && pool_after)
+      e = launch_block_pool(half, to, l.batch, l.c_out, l.rows, l.cols, input_of(i + 1), which, st);
   }
   g_variant = half ? "mfma-f16-blocks" : "mfma-blocks";
   g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
@@ -2316,7 +2320,7 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
     const mellin_stack_layer &ly = layers[i];
     const void *w = wide ? ly.weight_half : ly.weight;
     if (!w) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
-    plan_block_input(kind_x, half, STACK_DIMS(ly), ip);
+    plan_block_input(kind_x, half, STACK_DIMS(ly), ip, layers[i - 1].pool ? layers[i - 1].dims[8] : 0);
     filters[n_filters++] = pack_filter(ip, (int)ly.dims[2], w, ws + sp.l[i].frag_off, nullptr, 0);
   }
   const int top = n_layers - 1;
@@ -2354,11 +2358,11 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
     float *const bias_below = go_on ? (float *)take(bias_bytes) : nullptr;
     i64 bias_count = 0;
     if (go_on) {
-      plan_block_input(kind_x, half, STACK_DIMS(ly), ip);
+      plan_block_input(kind_x, half, STACK_DIMS(ly), ip, pooled ? layers[i - 1].dims[8] : 0);
       ip.relu = 0;
-      char *to = first_dense ? ws + sp.b_first : pooled ? ws + sp.b_unpooled : ws + sp.b_grad[below];
-      const BlockGemmArgs args = {ws + sp.b_grad[here], ws + l.frag_off, nullptr, to, (float *)(ws + sp.b_sums), !first_dense, !pooled,
-                                  keep + l.x_off, bias_below};
+      const BlockGemmArgs args = {ws + sp.b_grad[here], ws + l.frag_off, nullptr, first_dense ? ws + sp.b_first : ws + sp.b_grad[below],
+                                  (float *)(ws + sp.b_sums), !first_dense, true, keep + l.x_off, bias_below,
+                                  pooled ? (char *)keep + l.which_off : nullptr};
       bias_count = ip.chan_slots;
       e = launch_block_gemm(ip, args, st);
       if (e == hipSuccess && ip.rest > 0) {            // (what goes on from here needs the whole tiles: the sums go along)
@@ -2366,12 +2370,6 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
         fin.args = args;
         e = finish();
       }
-    }
-    if (go_on && pooled && e == hipSuccess) {
-      const mellin_stack_layer &before = layers[i - 1];
-      e = launch_block_pool_grad(half, ws + sp.b_unpooled, keep + l.x_off, keep + l.which_off, l.batch, l.c_in, before.dims[7],
-                                 before.dims[8], ws + sp.b_grad[below], bias_below, st);
-      bias_count = (i64)pool_partial_count(l.batch, 1, before.dims[7], before.dims[8]);
     }
     if (go_on && layers[i - 1].grad_bias) fin.add_bias(bias_below, bias_count, l.c_in, layers[i - 1].grad_bias);
   }

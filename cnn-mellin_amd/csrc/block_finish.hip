@@ -109,67 +109,104 @@ __device__ void finish_weight_taps(const WeightSums &pl, int b, float (*sum)[33]
   }
 }
 
-// Tiles in slices whose output is blocked or passes a ReLU: a thread makes a unit (eight channels of a position); a block
-// has 256 of a tile's, the positions side by side.
+// Eight values as a unit of a blocked tensor.
+template <typename T>
+__device__ __forceinline__ void make_unit(const float (&v)[8], uintx4 (&u)[sizeof(T) == 2 ? 1 : 3]) {
+  if constexpr (sizeof(T) == 2) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      u[0][j] = (unsigned)__builtin_bit_cast(unsigned short, (_Float16)v[2 * j]) | ((unsigned)__builtin_bit_cast(unsigned short, (_Float16)v[2 * j + 1]) << 16);
+  } else {
+    split8(v, u[0], u[1], u[2]);
+  }
+}
+
+// Tiles in slices whose output is blocked or passes a ReLU: a thread makes a unit (eight channels of a position) -- of pooled
+// ones the maxima of two positions, or both positions that a maximum was taken from; a block has 256 of a tile's, the positions
+// side by side.
 template <typename T>
 __device__ void finish_units(const SliceSums &a, int b, float (*red)[32]) {
   constexpr bool F16 = sizeof(T) == 2;
-  constexpr int UB = F16 ? 16 : 48;
+  constexpr int PARTS = F16 ? 1 : 3, UB = 16 * PARTS;
   const BlockPlan &pl = a.s;
-  const int m_t = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32, units = m_t / 8 * P;
+  const bool pool = pl.pool == 1, unpool = pl.pool == 2;
+  const int m_t = pl.wm * pl.mt * 32, P = kWaves / pl.wk / pl.wm * pl.nt * 32, each_p = pool ? 2 : 1, PU = P / each_p, units = m_t / 8 * PU;
   const int chunks = (units + kFinishThreads - 1) / kFinishThreads;
   const int tm = b / chunks, at = (b - tm * chunks) * kFinishThreads + (int)threadIdx.x;      // (tile, tile of channels), unit in it
-  const int r = tm / pl.m_tiles, g_t = at / P, p = at - g_t * P, group = (tm - r * pl.m_tiles) * (m_t / 8) + g_t;
+  const int r = tm / pl.m_tiles, g_t = at / PU, p = (at - g_t * PU) * each_p, group = (tm - r * pl.m_tiles) * (m_t / 8) + g_t;
   const int id = pl.whole + r, qt = id / pl.tile_batch, q0 = qt * P, count = min(P, pl.tile_q - q0);
   int n = id - qt * pl.tile_batch;
   const bool live = at < units && group < pl.out_groups && p < count;
   float v[8];
 #pragma unroll
   for (int c = 0; c < 8; ++c) v[c] = 0.f;
-  int q = 0;
   if (live) {
     const i64 slice = (i64)pl.rest * pl.m_tiles * m_t * P;
     const float *from = a.sa.sums + (i64)tm * m_t * P + (i64)g_t * 8 * P + p;
-    for (int k = 0; k < pl.slices; ++k)
+    auto add_slices = [&](const float *from, float (&v)[8]) {
+      for (int k = 0; k < pl.slices; ++k)
 #pragma unroll
-      for (int c = 0; c < 8; ++c) v[c] += from[k * slice + c * P];
-    // (channels past the last have no sums: the matrix kernel's stores end with the last channel, and what the workspace
-    // held there must not become a blocked tensor's padding)
+        for (int c = 0; c < 8; ++c) v[c] += from[k * slice + c * P];
+      // (channels past the last have no sums: the matrix kernel's stores end with the last channel, and what the workspace
+      // held there must not become a blocked tensor's padding)
 #pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] = group * 8 + c < pl.M ? v[c] : 0.f;
+      for (int c = 0; c < 8; ++c) v[c] = group * 8 + c < pl.M ? v[c] : 0.f;
+      if (!a.sa.grad && pl.relu)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) v[c] = fmaxf(v[c], 0.f);
+    };
+    add_slices(from, v);
     int row = (q0 + p) / pl.noy;
     const int oy = q0 + p - row * pl.noy;
     if (pl.joint) { n = row % pl.batch; row /= pl.batch; }
-    q = (a.s_rows ? a.s_rows[row].x : row) * pl.noy + oy;
-    const i64 unit = ((i64)n * pl.out_groups + group) * (pl.Q + 1) + q;
+    if (a.s_rows) row = a.s_rows[row].x;
+    const int q = row * pl.noy + oy;
+    const i64 of_group = (i64)n * pl.out_groups + group;
+    const i64 unit = of_group * (pl.out_q + 1) + (pool ? q / 2 : unpool ? row * pl.out_cols + 2 * oy : q);
+    unsigned long long which = 0;
     if (a.sa.grad) {
-      const uintx4 x = *(const uintx4 *)((const char *)a.sa.mask + unit * UB);
+      const uintx4 x = *(const uintx4 *)((const char *)a.sa.mask + (of_group * (pl.Q + 1) + q) * UB);
 #pragma unroll
       for (int c = 0; c < 8; ++c)
         if (!((short)(x[c >> 1] >> (16 * (c & 1))) > 0)) v[c] = 0.f;
-    } else if (pl.relu) {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) v[c] = fmaxf(v[c], 0.f);
+      if (unpool) which = ((const unsigned long long *)a.sa.which)[of_group * pl.Q + q];
     }
+    if (pool) {
+      float w[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) w[c] = 0.f;
+      add_slices(from + 1, w);
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        if ((T)w[c] > (T)v[c]) {                       // (of the values as they would be stored)
+          which |= 1ull << (8 * c);
+          v[c] = w[c];
+        }
+      if (a.sa.which) ((unsigned long long *)a.sa.which)[of_group * pl.out_q + q / 2] = which;
+    }
+    const uintx4 zero = {0, 0, 0, 0};
     if (a.sa.blocked) {
-      uintx4 *o = (uintx4 *)((char *)a.sa.out + unit * UB);
-      if constexpr (F16) {
+      uintx4 *o = (uintx4 *)((char *)a.sa.out + unit * UB), u[PARTS];
+      make_unit<T>(v, u);
+      if (unpool) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          o[0][j] = (unsigned)__builtin_bit_cast(unsigned short, (_Float16)v[2 * j]) |
-                    ((unsigned)__builtin_bit_cast(unsigned short, (_Float16)v[2 * j + 1]) << 16);
+        for (int i = 0; i < PARTS; ++i) {
+          uintx4 m;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) m[j] = ((which >> (16 * j)) & 1 ? 0xFFFFu : 0u) | ((which >> (16 * j + 8)) & 1 ? 0xFFFF0000u : 0u);
+          o[i] = u[i] & ~m;
+          o[PARTS + i] = u[i] & m;
+          if (oy == pl.noy - 1 && (pl.out_cols & 1)) o[2 * PARTS + i] = zero;
+        }
       } else {
-        uintx4 hi, mid, lo;
-        split8(v, hi, mid, lo);
-        o[0] = hi;
-        o[1] = mid;
-        o[2] = lo;
-      }
-      if (pl.joint ? q == pl.Q - 1 : q0 + p == pl.Q - 1) {     // the unit of zeros behind the image
-        uintx4 *z = (uintx4 *)((char *)a.sa.out + (((i64)n * pl.out_groups + group) * (pl.Q + 1) + pl.Q) * UB);
-        const uintx4 zero = {0, 0, 0, 0};
 #pragma unroll
-        for (int j = 0; j < UB / 16; ++j) z[j] = zero;
+        for (int i = 0; i < PARTS; ++i) o[i] = u[i];
+      }
+      // the unit of zeros behind the image
+      if (pl.joint ? q == pl.Q - 1 : q0 + p + each_p == pl.Q) {
+        uintx4 *z = (uintx4 *)((char *)a.sa.out + (of_group * (pl.out_q + 1) + pl.out_q) * UB);
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i) z[i] = zero;
       }
     } else {
       T *o = (T *)a.sa.out + n * pl.h_n + (i64)group * 8 * pl.h_m + q;

@@ -53,20 +53,22 @@ void plan_classes(const Axis &x, BlockPlan &pl) {
 
 }  // namespace
 
-bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) {
+bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool &pool, const BlockPlan *like, BlockPlan &pl) {
   const Axis &X = pr.x, &Y = pr.y;
   const i64 lim = (i64)1 << 30;
   if (pr.accumulate || pr.batch < 1 || pr.c_out < 1 || pr.c_in < 1 || X.nf < 1 || Y.nf < 1 || X.nf > kBlockFilterRows) return false;
   if (Y.kind != AX_LCORR && Y.kind != AX_LCONV) return false;
-  const i64 plane = X.ng * Y.ng, Q = X.nh * Y.nh;
+  const i64 plane = X.ng * Y.ng, Q = X.nh * Y.nh, out_q = pool.kind == 1 ? Q / 2 : pool.kind == 2 ? X.nh * pool.cols : Q;
+  if (pool.kind == 1 && Y.nh % 2) return false;        // (and a gradient's `cols` are 2 nh or 2 nh + 1)
   if (plane < 1 || Q < 1 || plane >= (i64)1 << 22 || Q >= (i64)1 << 22) return false;
   if (pr.batch > 65535 || pr.c_in > 8 * 65535 || pr.c_out * Q >= lim / 2 || Q >= (i64)1 << 20 ||
-      (pr.c_out + 7) / 8 * (Q + 1) * 48 >= (i64)1 << 31)
+      (pr.c_out + 7) / 8 * (std::max(Q, out_q) + 1) * 48 >= (i64)1 << 31)
     return false;                                      // (32-bit byte offsets)
   if (X.s > 4096 || X.d > 4096 || X.u > 4096 || X.p > 4096 || X.p < -lim || Y.s > 64 || Y.d > 4096 || Y.u > 64 || Y.p > lim || Y.p < -lim)
     return false;
   pl.f16 = f16;
   pl.wide = 0;
+  pl.pool = pool.kind; pl.out_q = (int)out_q; pl.out_cols = pool.cols;
   pl.out_groups = (int)((pr.c_out + 7) / 8);
   pl.batch = (int)pr.batch; pl.M = (int)pr.c_out; pl.CG = (int)((pr.c_in + 7) / 8);
   pl.nox = (int)X.nh; pl.noy = (int)Y.nh; pl.Q = (int)Q;
@@ -84,6 +86,15 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
   pl.nfx = (int)X.nf; pl.nfy = (int)(fy_hi - fy_lo + 1);
   pl.f_pitch = (int)Y.nf; pl.f_off = (int)fy_lo;
   if (pl.nfy > 64) return false;
+  // A pooled output's sums keep the order of the unpooled one's, which decides what its ReLU lets through (see can_join), and
+  // are those of the layer called by itself bit for bit: the same channel groups and filter columns to a stage, the same
+  // slices.  Tiles hold other positions than without the pooling (an odd last column is in none), so the order must not depend on
+  // what a tile holds: not on its being one of those in slices, nor, on Mellin axes, on the filter rows of its other output
+  // rows -- they shift the pairs that share a step where a row's taps and groups are odd in number, and the steps that
+  // wavefronts share.
+  if (like && (like->nfy != pl.nfy || like->f_off != pl.f_off || (like->whole && like->rest) ||
+               ((X.kind == AX_MCORR || X.kind == AX_MCONV) && (like->wk > 1 || like->nfy * like->G % 2))))
+    return false;
   const i64 py = Y.p - Y.d * fy_lo;
   pl.ay = (int)Y.s; pl.by = Y.kind == AX_LCORR ? (int)Y.d : -(int)Y.d; pl.cy = Y.kind == AX_LCORR ? -(int)py : (int)py;
   pl.uy = (int)Y.u;
@@ -120,7 +131,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
   Stage stages[2][kShapes] = {};
   int groups[8], n_groups = 0;                         // the channel groups of a stage that divide all, most first
   for (int G = std::min(pl.CG, 8); G >= 1; --G)
-    if (pl.CG % G == 0) groups[n_groups++] = G;
+    if (pl.CG % G == 0 && (!like || G == like->G)) groups[n_groups++] = G;
   auto shape = [&](int at) {
     const int nt = shapes[at][0], wm = shapes[at][1], wk = shapes[at][2];
     const int P = (kWaves / wk / wm) * nt * 32, M_T = wm * pl.mt * 32;
@@ -267,9 +278,9 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
       return full * turn(per_m) + (left ? turn(left) : 0);
     };
     double best = 9000 + turns_cost(total, c_stages * subsets);
-    pl.slices = 1;
-    int rest = 0;
-    for (int all = 0; all < 2; ++all) {
+    pl.slices = like ? like->slices : 1;
+    int rest = like && like->rest ? total : 0;
+    for (int all = 0; all < (like ? 0 : 2); ++all) {
       const int r = all ? total : total % per_m;
       if (r == 0 || (all && total >= 2 * per_m) || (pl.wk > 1 && !all)) continue;
       const double whole = 9000 + turns_cost(total - r, c_stages * subsets);
@@ -310,7 +321,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
   // therefore keep the tiles of an image (joint ones: the training step 1364 -> 1205 us).
   const i64 unit_bytes = 16 * parts, most = (i64)1 << 31;
   const bool can_join = gradient && mellin && masks && pl.batch > 1 && Q * pl.batch < lim && (i64)pl.batch * pl.CG * (plane + 1) * unit_bytes < most &&
-                        (i64)pl.batch * pl.out_groups * (Q + 1) * unit_bytes < most && (i64)pl.batch * pl.M * Q * 4 < most &&
+                        (i64)pl.batch * pl.out_groups * (std::max(Q, out_q) + 1) * unit_bytes < most && (i64)pl.batch * pl.M * Q * 4 < most &&
                         pl.h_n == (i64)pl.M * Q;
   // Tiles of 32 channels are tried as well: where those of 64 leave half of the last one empty (65 to 96 channels, 129 to 160,
   // ..) they are taken like any other (28 passes of 400 drawn layers, 0.92 of the time in the geometric mean, 0.82 to 0.99),
@@ -326,6 +337,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
       for (int k = 0; k < kShapes; ++k) {
         const int *const sh = shapes[k];
         if (pl.mt < mt && sh[1] == 2) continue;
+        if (like && (sh[0] != like->nt || sh[1] != like->wm || sh[2] != like->wk)) continue;
         if (f16 ? sh[0] == 2 && sh[1] == 2 : sh[0] == 4 || (sh[0] == 2 && sh[2] == 4)) continue;
         if (sh[1] == 2 && pr.c_out <= 96) continue;      // (two wavefronts along the channels: most of 128)
         const double wanted = (pl.mt < mt ? narrow : 1) * limit;
@@ -349,6 +361,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl) 
 }
 
 hipError_t launch_block_gemm(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream) {
+  if (pl.pool) return a.grad ? launch_grad_pooled(pl, a, stream) : launch_out_pooled(pl, a, stream);
   if (a.grad) return a.blocked ? launch_grad_blocked(pl, a, stream) : launch_grad_plain(pl, a, stream);
   return a.blocked ? launch_out_blocked(pl, a, stream) : launch_shape<OUT_PLAIN>(pl, a, stream);
 }

@@ -42,6 +42,7 @@ struct BlockPlan {
   // leave workgroups without one, are dealt out in `slices` of the contracted channels, whose sums go to the workspace
   int whole, rest, slices;
   int out_groups, chan_slots;      // groups of eight output channels; partial sums of a channel over the positions
+  int pool, out_q, out_cols;       // pairs of columns: 1 stored as their maxima, 2 a gradient of such; positions and columns of what is stored
   unsigned mg_batch, mg_noy, mg_per_row, mg_full, mg_G;      // floor(2^32 / d) (see udiv)
   i64 h_n, h_m;
   int relu, half_out;
@@ -61,8 +62,14 @@ struct BlockPlan {
   int joint, tile_batch, tile_q;
 };
 
-// False: the kernel does not apply.  gradient: of an input (a forward pass has no joint tiles).
-bool make_block_plan(const SepConv &pr, bool f16, bool gradient, BlockPlan &pl);
+// Frequency pooling behind the layer: a forward pass of an even number of columns (`pr` leaves an odd last one out) stores the
+// maxima of pairs of them; an input gradient of `pr`, whose output is that of the maxima, is stored as that of the `cols`
+// columns they were taken from (an odd last one of them: zeros).
+struct BlockPool { int kind, cols; };  // kind: 0 no pooling, 1 forward, 2 input gradient
+
+// False: the kernel does not apply.  gradient: of an input (a forward pass has no joint tiles).  `like`: the plan of the same
+// layer without the pooling, whose order of sums is kept (false as well where that cannot be).
+bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool &pool, const BlockPlan *like, BlockPlan &pl);
 // out = [relu](bias + sum) from a blocked signal and packed filter; bias (fp32 / half, or null), relu as the plan says.
 // With `grad`, the input gradient of a layer behind a ReLU: zero where `mask`, the blocked output of that ReLU, is not
 // positive; its sums over the positions go to chan_sums ([channel][pl.chan_slots]: partial sums for launch_block_finish).
@@ -74,11 +81,14 @@ struct BlockGemmArgs {
   bool blocked, grad;              // out: blocked
   const void *mask;
   float *chan_sums;
+  void *which;                     // of pooled pairs, eight bytes a unit: 1 where the second is the larger (forward: null where nobody asks)
 };
 hipError_t launch_block_gemm(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
 hipError_t launch_out_blocked(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
 hipError_t launch_grad_plain(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
 hipError_t launch_grad_blocked(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
+hipError_t launch_out_pooled(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
+hipError_t launch_grad_pooled(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream);
 
 // The rows of one filter row in the weight gradient: output rows ox0 + i step and input rows gx0 + i gstep for
 // i < count; its share of the launch: `slices` workgroups from slice0 on.
@@ -139,11 +149,6 @@ hipError_t launch_block_pack(bool f16, const PackSignal *a, const PackSignal *b,
 // Maximum over pairs of neighbouring columns of a blocked tensor (batch, channels, rows, cols), as pool_pairs: y is blocked
 // with cols / 2 columns; `which` (eight bytes a unit of y): 1 where the second was taken.
 hipError_t launch_block_pool(bool f16, const void *x, i64 batch, i64 channels, i64 rows, i64 cols, void *y, void *which, hipStream_t stream);
-// Its backward pass behind a ReLU: grad_x from grad_y (blocked), zero where y is not positive; the sums of a channel's
-// gradients go to `partial` (pool_partial_count(): floats, for launch_block_finish).
-hipError_t launch_block_pool_grad(bool f16, const void *grad_y, const void *y, const void *which, i64 batch, i64 channels, i64 rows,
-                                  i64 cols, void *grad_x, float *partial, hipStream_t stream);
-size_t pool_partial_count(i64 batch, i64 channels, i64 rows, i64 cols);
 
 // The sums that end passes, in one launch.
 constexpr int kFinishJobs = 16;

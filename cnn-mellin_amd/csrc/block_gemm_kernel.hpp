@@ -50,7 +50,11 @@ namespace {
 // What a launch makes of its sums: the tensor as it lies, or blocked (block_gemm.hpp) for the kernels that read it
 // next; an output [relu](bias + sum), or a gradient, which passes the ReLU in front of the layer (where its blocked
 // output `mask` is positive) and whose sums over the positions, the bias gradient of the layer before, go to `chan_sums`.
-enum { OUT_PLAIN, OUT_BLOCKED, GRAD_PLAIN, GRAD_BLOCKED };
+// Where pairs of neighbouring columns are pooled behind the layer, an output is stored as their maxima (OUT_POOLED; `which`:
+// one byte a value, 1 where the second was the larger), and the gradient of such maxima as that of the values they were taken
+// from (GRAD_POOLED): the unpooled output is never written, nor the gradient of the maxima.  (Passes of their own, 64
+// channels, 32 x 780 x 41, moved 0.6 and 0.7 GB in fp32: 125 and 190 us; half 32 and 51 us.)
+enum { OUT_PLAIN, OUT_BLOCKED, GRAD_PLAIN, GRAD_BLOCKED, OUT_POOLED, GRAD_POOLED };
 
 // The plan stays in the kernel arguments and is read by scalar loads where it is used: held in
 // registers for a whole stage its fields would not fit the scalar register file.
@@ -166,11 +170,13 @@ template <int MT, int NT, int WM, int WK, bool F16, int OUT, bool JOINT>
 __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_arg, const char *__restrict__ X,
                                                                  const char *__restrict__ AF, const void *__restrict__ bias,
                                                                  void *__restrict__ Hv, float *__restrict__ sums,
-                                                                 const char *__restrict__ mask, float *__restrict__ chan_sums) {
+                                                                 const char *__restrict__ mask, float *__restrict__ chan_sums,
+                                                                 unsigned char *__restrict__ which) {
   constexpr int PARTS = F16 ? 1 : 3, UB = 16 * PARTS;
   constexpr int WN = kWaves / WK / WM, P = WN * NT * 32, M_T = WM * MT * 32;
   constexpr int kALoads = 2 * MT * PARTS;              // fragment loads of two steps
-  constexpr bool BLOCKED = OUT == OUT_BLOCKED || OUT == GRAD_BLOCKED, GRAD = OUT == GRAD_PLAIN || OUT == GRAD_BLOCKED;
+  constexpr bool POOLED = OUT == OUT_POOLED, UNPOOLED = OUT == GRAD_POOLED;
+  constexpr bool BLOCKED = OUT == OUT_BLOCKED || OUT == GRAD_BLOCKED || POOLED || UNPOOLED, GRAD = OUT == GRAD_PLAIN || OUT == GRAD_BLOCKED || UNPOOLED;
   extern __shared__ __align__(16) char blk_lds[];
   ConstBlockPlan *plp = (ConstBlockPlan *)__builtin_amdgcn_kernarg_segment_ptr();
 #define pl (*plp)
@@ -493,8 +499,9 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       const bool whole = tg.slot < 0, relu = pl.relu && whole;
       const int m0 = m_tile * M_T + wm * MT * 32;
       // A gradient's mask, and the sums of its channels over the tile's positions
-      const unsigned unit_row = (unsigned)(pl.Q + 1) * UB;                  // bytes of a channel group of a blocked output
-      const i64 image_bytes = (i64)pl.out_groups * unit_row;
+      const unsigned unit_row = (unsigned)(pl.out_q + 1) * UB;              // bytes of a channel group of a blocked output
+      const unsigned mask_row = UNPOOLED ? (unsigned)(pl.Q + 1) * UB : unit_row;
+      const i64 image_bytes = (i64)pl.out_groups * unit_row, mask_bytes = (i64)pl.out_groups * mask_row;
       // joint: the images of the lane's positions
       int lane_n[NT];
 #pragma unroll
@@ -505,16 +512,53 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
           lane_n[t] = pair - udiv(pair, pl.batch, pl.mg_batch) * pl.batch;
         }
       }
-      const int all_images = (int)image_bytes * (JOINT ? pl.batch : 1);
-      __amdgpu_buffer_rsrc_t mask_rsrc;
-      if constexpr (GRAD)
-        mask_rsrc = wave_buffer(mask + tg.n * image_bytes, all_images);
-      int unit_at[NT];                                 // the lane's quarter unit in its group (none: past any end)
+      const int images = JOINT ? pl.batch : 1, all_images = (int)image_bytes * images;
+      __amdgpu_buffer_rsrc_t mask_rsrc, which_rsrc;
+      if constexpr (GRAD) mask_rsrc = wave_buffer(mask + tg.n * mask_bytes, (int)mask_bytes * images);
+      const int which_row = 8 * (POOLED ? pl.out_q : pl.Q), which_bytes = pl.out_groups * which_row;
+      if constexpr (POOLED || UNPOOLED) which_rsrc = wave_buffer(which + (i64)tg.n * which_bytes, which ? which_bytes * images : 0);
+      // the lane's quarter unit in its group, in the output and in the mask (none: past any end)
+      int unit_at[NT], mask_at[NT];
+      const bool odd_cols = UNPOOLED && (pl.out_cols & 1);
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-        unit_at[t] = (wn * NT + t) * 32 + l32 < tg.count ? lane_n[t] * (int)image_bytes + lane_q[t] * UB + half * 8 : (int)0x80000000u;
+      for (int t = 0; t < NT; ++t) {
+        const bool there = (wn * NT + t) * 32 + l32 < tg.count;
+        int unit = lane_q[t];
+        if constexpr (POOLED) unit >>= 1;              // (an even number of columns)
+        if constexpr (UNPOOLED) unit = 2 * unit + (odd_cols ? udiv(unit, pl.noy, pl.mg_noy) : 0);
+        unit_at[t] = there ? lane_n[t] * (int)image_bytes + unit * UB + half * 8 : (int)0x80000000u;
+        mask_at[t] = !UNPOOLED ? unit_at[t] : there ? lane_n[t] * (int)mask_bytes + lane_q[t] * UB + half * 8 : (int)0x80000000u;
+      }
       auto load_mask = [&](int group, int at) -> uintx2 {
-        return __builtin_amdgcn_raw_buffer_load_b64(mask_rsrc, at < 0 ? at : at + (int)(group * unit_row), 0, 0);   // (none: zeros)
+        return __builtin_amdgcn_raw_buffer_load_b64(mask_rsrc, at < 0 ? at : at + (int)(group * mask_row), 0, 0);   // (none: zeros)
+      };
+      // GRAD_POOLED: the four bytes of a lane's quarter unit as masks over its values, for the pair's second value
+      auto load_which = [&](int group, int t) -> unsigned {
+        const int at = lane_n[t] * which_bytes + lane_q[t] * 8 + half * 4 + group * which_row;
+        return __builtin_amdgcn_raw_buffer_load_b32(which_rsrc, mask_at[t] < 0 ? mask_at[t] : at, 0, 0);
+      };
+      auto second_mask = [](unsigned w) {
+        const unsigned bytes = (w << 8) - w;           // 0 or 255 each
+        return uintx2{__builtin_amdgcn_perm(0, bytes, 0x01010000), __builtin_amdgcn_perm(0, bytes, 0x03030202)};
+      };
+      // the unit behind a row's last pair where there is an odd column, which took no part: zeros
+      auto odd_at = [&](int t, int to) { return to >= 0 && lane_q[t] - udiv(lane_q[t], pl.noy, pl.mg_noy) * pl.noy == pl.noy - 1 ? to + 2 * UB : (int)0x80000000u; };
+      // OUT_POOLED: of two values a lane, the pair's that the lane keeps -- with its neighbour, an even lane that of the first,
+      // an odd lane that of the second -- and whether its second value is the larger
+      auto pool = [&](float a, float b, bool &second) {
+        if constexpr (F16) { a = (float)(_Float16)a; b = (float)(_Float16)b; }         // (the stored values are compared)
+        const bool odd = lane & 1;
+        const float keep = odd ? b : a, send = odd ? a : b;
+        const float got = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), 0xb1, 0xf, 0xf, true));
+        const float one = odd ? got : keep, two = odd ? keep : got;
+        second = two > one;                            // (behind a ReLU: no NaN)
+        return second ? two : one;
+      };
+      auto pool4 = [&](const float4 &a, const float4 &b, unsigned &seconds) {
+        bool s0, s1, s2, s3;
+        const float4 v = make_float4(pool(a.x, b.x, s0), pool(a.y, b.y, s1), pool(a.z, b.z, s2), pool(a.w, b.w, s3));
+        seconds = (s0 ? 1u : 0u) | (s1 ? 0x100u : 0u) | (s2 ? 0x10000u : 0u) | (s3 ? 0x1000000u : 0u);
+        return v;
       };
       auto masked = [&](float4 v, uintx2 x) {
         auto keep = [](float f, unsigned sixteen) { return (short)sixteen > 0 ? f : 0.f; };
@@ -559,7 +603,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
         const float *red = (const float *)bufs;
         for (int kt = wk; kt < MT * NT; kt += WK) {
           const int k = kt / NT, t = kt - k * NT;
-          const int unit = NT > 1 && t ? unit_at[NT - 1] : unit_at[0];
+          const int unit = NT > 1 && t ? unit_at[NT - 1] : unit_at[0], m_at = NT > 1 && t ? mask_at[NT - 1] : mask_at[0];
           int to = (NT > 1 && t ? at[NT - 1] : at[0]) + row0 + k * 32 * h_m;
           float s[16];
 #pragma unroll
@@ -574,16 +618,29 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
             const int group = m0 / 8 + k * 4 + r4;
             if constexpr (GRAD) {
               if (whole) {
-                v = masked(v, load_mask(group, unit));
+                v = masked(v, load_mask(group, m_at));
                 s[4 * r4] = v.x; s[4 * r4 + 1] = v.y; s[4 * r4 + 2] = v.z; s[4 * r4 + 3] = v.w;
               }
             }
             if (BLOCKED && whole) {
-              unsigned w[PARTS][2];
+              unsigned w[PARTS][2], seconds = 0;
+              if constexpr (POOLED) v = pool4(v, v, seconds);
               cut_four<F16>(v, w);
+              const int o = unit < 0 || (POOLED && (lane & 1)) ? (int)0x80000000u : unit + (int)(group * unit_row);
+              if constexpr (POOLED) __builtin_amdgcn_raw_buffer_store_b32(seconds, which_rsrc, o < 0 ? o : group * which_row + (unit - half * 8) / (2 * PARTS) + half * 4, 0, 0);
+              uintx2 m2 = {0, 0};
+              if constexpr (UNPOOLED) m2 = second_mask(load_which(group, NT > 1 && t ? NT - 1 : 0));
 #pragma unroll
-              for (int pt = 0; pt < PARTS; ++pt)
-                __builtin_amdgcn_raw_buffer_store_b64(uintx2{w[pt][0], w[pt][1]}, rsrc, unit < 0 ? unit : unit + (int)(group * unit_row) + pt * 16, 0, 0);
+              for (int pt = 0; pt < PARTS; ++pt) {
+                const uintx2 x = {w[pt][0], w[pt][1]};
+                __builtin_amdgcn_raw_buffer_store_b64(x & ~m2, rsrc, o < 0 ? o : o + pt * 16, 0, 0);
+                if constexpr (UNPOOLED) __builtin_amdgcn_raw_buffer_store_b64(x & m2, rsrc, o < 0 ? o : o + UB + pt * 16, 0, 0);
+              }
+              if (odd_cols) {
+                const int z = odd_at(NT > 1 && t ? NT - 1 : 0, o);
+#pragma unroll
+                for (int pt = 0; pt < PARTS; ++pt) __builtin_amdgcn_raw_buffer_store_b64(uintx2{0, 0}, rsrc, z < 0 ? z : z + pt * 16, 0, 0);
+              }
             } else {
               store_four(v, to);
             }
@@ -602,7 +659,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
             uintx2 mask_of[kAhead][NT];
             auto request = [&](int i) {
 #pragma unroll
-              for (int t = 0; t < NT; ++t) mask_of[i % kAhead][t] = load_mask(m0 / 8 + i, unit_at[t]);
+              for (int t = 0; t < NT; ++t) mask_of[i % kAhead][t] = load_mask(m0 / 8 + i, mask_at[t]);
             };
 #pragma unroll
             for (int i = 0; i < kAhead; ++i) request(i);
@@ -653,28 +710,66 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
         if (BLOCKED && whole) {
           // the halves of a wavefront exchange quarters, so that a lane stores whole units: the lower one groups 0 and 2
           // of a tile's four, the upper one groups 1 and 3
-          int to[NT];
+          // (pooled: of two blocks of 32 positions the even lanes store the maxima of one, the odd lanes those of the other)
+          constexpr int NS = POOLED ? (NT + 1) / 2 : NT;
+          int to[NS], which_at[NS];
 #pragma unroll
-          for (int t = 0; t < NT; ++t) to[t] = unit_at[t] < 0 ? unit_at[t] : unit_at[t] - half * 8 + (int)((m0 / 8 + half) * unit_row);
+          for (int t = 0; t < NS; ++t) {
+            const bool odd = lane & 1;
+            int u = POOLED ? (odd ? (2 * t + 1 < NT ? unit_at[POOLED && 2 * t + 1 < NT ? 2 * t + 1 : 0] : (int)0x80000000u) : unit_at[POOLED ? 2 * t : 0]) : unit_at[t];
+            to[t] = u < 0 ? u : u - half * 8 + (int)((m0 / 8 + half) * unit_row);
+            which_at[t] = u < 0 ? u : (u - half * 8) / (2 * PARTS) + (m0 / 8 + half) * which_row;
+          }
 #pragma unroll
-          for (int k = 0; k < MT; ++k)
+          for (int k = 0; k < MT; ++k) {
+            unsigned seconds_of[UNPOOLED ? 4 : 1][UNPOOLED ? NT : 1];
+            if constexpr (UNPOOLED) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) seconds_of[i][t] = load_which(m0 / 8 + k * 4 + i, t);
+              __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int p2 = 0; p2 < 4; p2 += 2) {
 #pragma unroll
-              for (int t = 0; t < NT; ++t) {
-                unsigned lo[PARTS][2], hi[PARTS][2];
-                cut_four<F16>(make_float4(acc[k][t][4 * p2], acc[k][t][4 * p2 + 1], acc[k][t][4 * p2 + 2], acc[k][t][4 * p2 + 3]), lo);
-                cut_four<F16>(make_float4(acc[k][t][4 * p2 + 4], acc[k][t][4 * p2 + 5], acc[k][t][4 * p2 + 6], acc[k][t][4 * p2 + 7]), hi);
+              for (int t = 0; t < NS; ++t) {
+                unsigned lo[PARTS][2], hi[PARTS][2], lo2 = 0, hi2 = 0;
+                auto four = [&](int tile, int r) { return make_float4(acc[k][tile][r], acc[k][tile][r + 1], acc[k][tile][r + 2], acc[k][tile][r + 3]); };
+                if constexpr (POOLED) {
+                  const int other = 2 * t + 1 < NT ? 2 * t + 1 : 2 * t;
+                  cut_four<F16>(pool4(four(2 * t, 4 * p2), four(other, 4 * p2), lo2), lo);
+                  cut_four<F16>(pool4(four(2 * t, 4 * p2 + 4), four(other, 4 * p2 + 4), hi2), hi);
+                  const auto s2 = __builtin_amdgcn_permlane32_swap(lo2, hi2, false, false);
+                  __builtin_amdgcn_raw_buffer_store_b64(uintx2{s2[0], s2[1]}, which_rsrc, which_at[t], 0, 0);
+                  if (which_at[t] >= 0) which_at[t] += 2 * which_row;
+                } else {
+                  cut_four<F16>(four(t, 4 * p2), lo);
+                  cut_four<F16>(four(t, 4 * p2 + 4), hi);
+                }
+                uintx2 lo_m = {0, 0}, hi_m = {0, 0};
+                if constexpr (UNPOOLED) { lo_m = second_mask(seconds_of[p2][t]); hi_m = second_mask(seconds_of[p2 + 1][t]); }
+                auto put = [&](int pt, uintx2 a, uintx2 b, int o) {
+                  const auto s0 = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+                  const auto s1 = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+                  __builtin_amdgcn_raw_buffer_store_b128(uintx4{s0[0], s1[0], s0[1], s1[1]}, rsrc, o < 0 ? o : o + pt * 16, 0, 0);
+                };
 #pragma unroll
                 for (int pt = 0; pt < PARTS; ++pt) {
-                  const auto s0 = __builtin_amdgcn_permlane32_swap(lo[pt][0], hi[pt][0], false, false);
-                  const auto s1 = __builtin_amdgcn_permlane32_swap(lo[pt][1], hi[pt][1], false, false);
-                  __builtin_amdgcn_raw_buffer_store_b128(uintx4{s0[0], s1[0], s0[1], s1[1]}, rsrc, to[t] < 0 ? to[t] : to[t] + pt * 16, 0, 0);
+                  const uintx2 a = {lo[pt][0], lo[pt][1]}, b = {hi[pt][0], hi[pt][1]};
+                  put(pt, a & ~lo_m, b & ~hi_m, to[t]);
+                  if constexpr (UNPOOLED) put(pt, a & lo_m, b & hi_m, to[t] < 0 ? to[t] : to[t] + UB);
+                }
+                if (odd_cols) {
+                  const int z = odd_at(t, to[t]);
+#pragma unroll
+                  for (int pt = 0; pt < PARTS; ++pt) __builtin_amdgcn_raw_buffer_store_b128(uintx4{0, 0, 0, 0}, rsrc, z < 0 ? z : z + pt * 16, 0, 0);
                 }
                 if (to[t] >= 0) to[t] += (int)(2 * unit_row);
                 __builtin_amdgcn_sched_barrier(0);     // (one block's registers at a time)
               }
             }
+          }
         } else if (as_half) {
           store_all([](float v, const __amdgpu_buffer_rsrc_t &to, int at) {
             __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(short, (_Float16)v), to, at, 0, 0);
@@ -689,14 +784,14 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
           const int tiles = max(pl.whole, 1), lo = (int)((i64)tg.id * pl.batch / tiles), hi = whole ? (int)((i64)(tg.id + 1) * pl.batch / tiles) : lo;
           for (int i = tid; i < (hi - lo) * (M_T / 8); i += kThreads) {
             const int n = lo + i / (M_T / 8), group = m_tile * (M_T / 8) + i % (M_T / 8);
-            uintx4 *z = (uintx4 *)((char *)Hv + n * image_bytes + (i64)group * unit_row + (i64)pl.Q * UB);
+            uintx4 *z = (uintx4 *)((char *)Hv + n * image_bytes + (i64)group * unit_row + (i64)pl.out_q * UB);
             const uintx4 zero = {0, 0, 0, 0};
 #pragma unroll
             for (int pt = 0; pt < PARTS; ++pt) z[pt] = zero;
           }
         } else if (whole && tg.q0 + tg.count == pl.Q && tid < M_T / 8 && m_tile * (M_T / 8) + tid < pl.out_groups) {
           // the units of zeros behind an image's last positions
-          uintx4 *z = (uintx4 *)((char *)Hv + tg.n * image_bytes + (i64)(m_tile * (M_T / 8) + tid) * unit_row + (i64)pl.Q * UB);
+          uintx4 *z = (uintx4 *)((char *)Hv + tg.n * image_bytes + (i64)(m_tile * (M_T / 8) + tid) * unit_row + (i64)pl.out_q * UB);
           const uintx4 zero = {0, 0, 0, 0};
 #pragma unroll
           for (int pt = 0; pt < PARTS; ++pt) z[pt] = zero;
@@ -725,13 +820,15 @@ hipError_t launch_joint(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t
   if (WK > 1 && (pl.m_tiles == 2 || pl.m_tiles == 4 || pl.m_tiles == 8) && pl.filter_bytes >= (size_t)1 << 20)   // by XCD: see the kernel
     grid = dim3((unsigned)((pl.grid_x + 8 / pl.m_tiles - 1) / (8 / pl.m_tiles) * 8));
   hipLaunchKernelGGL(kern, grid, dim3(kThreads), pl.lds_bytes, stream, pl,
-                     (const char *)a.signal, (const char *)a.frag, a.bias, a.out, a.sums, (const char *)a.mask, a.chan_sums);
+                     (const char *)a.signal, (const char *)a.frag, a.bias, a.out, a.sums, (const char *)a.mask, a.chan_sums, (unsigned char *)a.which);
   return hipGetLastError();
 }
 
 template <int MT, int NT, int WM, int WK, bool F16, int OUT>
 hipError_t launch_instance(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t stream) {
-  return pl.joint ? launch_joint<MT, NT, WM, WK, F16, OUT, true>(pl, a, stream) : launch_joint<MT, NT, WM, WK, F16, OUT, false>(pl, a, stream);
+  if constexpr (OUT != OUT_POOLED)                     // (no joint tiles of those: make_block_plan)
+    if (pl.joint) return launch_joint<MT, NT, WM, WK, F16, OUT, true>(pl, a, stream);
+  return launch_joint<MT, NT, WM, WK, F16, OUT, false>(pl, a, stream);
 }
 
 template <int OUT>

@@ -491,8 +491,9 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
                           const void *out, const void *grad_out, const void *saved, size_t saved_bytes, void *grad_input,
                           void *workspace, size_t workspace_bytes, void *stream);
 
-/* How the blocked kernels run a layer's forward pass, or with `gradient` its input gradient (for tests and profiling): 0 if they
- * do not take it, else 1 and plan = {tiles of 32 channels and of 32 positions of a wavefront, wavefronts along the channels,
+/* How the blocked kernels run a layer's forward pass, or with `gradient` 1 its input gradient, 2 its forward pass in a stack that
+ * pools behind it (for tests and profiling): 0 if they do not take it, else 1 (2 where they store the pooled output
+ * themselves) and plan = {tiles of 32 channels and of 32 positions of a wavefront, wavefronts along the channels,
  * wavefronts that share a tile, 1 where a tile's positions run over the images of an output row, filter rows and channel groups
  * of a stage, tiles that a workgroup makes whole, tiles whose channels are dealt to several, to how many}. */
 #define MELLIN_LAYER_PLAN_WORDS 10

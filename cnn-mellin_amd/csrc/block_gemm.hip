@@ -352,7 +352,21 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
   if (best_cost == 0) return false;
   pl = best_plan;
   const i64 per_row = (i64)pl.nfy * pl.G, pairs = 2 * pl.wk;
-  pl.mg_per_row = magic(per_row); pl.mg_G = magic(pl.G);
+  // Whole tiles with fewer filter rows than a stage holds have stages of more channel groups, as many as its LDS has room for: a
+  // stage of one row of three, two groups and three columns is three steps, shorter than the trip of the next one's loads (128 <-
+  // 256 channels, 3 x 3 taps, p = 2, 32 x 256 x 41, half: 182 -> 165 us; fp32, whose steps are six times as long: 96 channels, 6 x 3 taps, p = 2, 640 -> 629
+  // us a step).  Input gradients only: in a forward pass the order of a value's sums would depend on the tile that it lies
+  // in, and that order decides what the ReLUs let through (see can_join, `like`); in half it gained a twentieth there.
+  const i64 tile_rows_most = std::min<i64>(pl.joint ? (i64)pl.nox * pl.batch : pl.nox, (kWaves / pl.wk / pl.wm * pl.nt * 32 + pl.noy - 2) / pl.noy + 1);
+  for (int n = 1; n <= pl.F; ++n) {
+    int G = pl.G;
+    if (mellin && gradient)
+      for (int k = n_groups - 1; k >= 0; --k)              // (fewest first)
+        if (groups[k] > G && n * groups[k] <= pl.F * pl.G &&
+            groups[k] * ((n * tile_rows_most * pl.RS * parts + 63) / 64 * 1024) <= pl.buf_bytes)
+          G = groups[k];
+    pl.stage[n - 1] = BlockStage{G, magic(G), magic((i64)pl.nfy * G)};
+  }
   pl.mg_full = magic(std::max<i64>((pl.F * per_row + pairs - 1) / pairs * pairs, 2 * pairs));
   pl.rows_off = (size_t)pl.m_tiles * pl.wm * pl.mt * ((size_t)pl.CG * pl.nfx * pl.nfy + 1) * parts * 512;
   if (pl.rows_off >= (size_t)lim) return false;

@@ -22,6 +22,9 @@ inline size_t blocked_bytes(i64 batch, i64 channels, i64 plane, bool f16) {
 // A class of output rows: every `stride`-th row from `first` on, with the filter rows of `mask`.
 struct BlockClass { int first, start; unsigned mask; };     // start: the class's first row in the order of the classes
 
+// Channel groups to a stage (see BlockPlan::stage), and what divides by them and by a filter row's halves of steps (udiv).
+struct BlockStage { int G; unsigned mg_G, mg_per_row; };
+
 struct BlockPlan {
   int f16;
   int wide;                        // f16: filter and bias are float (rounded to half where they are read)
@@ -35,6 +38,7 @@ struct BlockPlan {
   int ay, by, cy, uy, by_min;      // y axis: (ay oy + by fy + cy) / uy
   int RS;                          // units per virtual row
   int F, G;                        // filter rows and channel groups of a stage
+  BlockStage stage[kBlockFilterRows];                        // of a whole tile with one, two, .. F (and more) filter rows
   int tab_units;                   // positions of a tile's source table
   int ents;                        // operand offsets of a tile's steps
   int group_bytes, buf_bytes;      // LDS of one group of a stage, of a stage
@@ -43,7 +47,7 @@ struct BlockPlan {
   int whole, rest, slices;
   int out_groups, chan_slots;      // groups of eight output channels; partial sums of a channel over the positions
   int pool, out_q, out_cols;       // pairs of columns: 1 stored as their maxima, 2 a gradient of such; positions and columns of what is stored
-  unsigned mg_batch, mg_noy, mg_per_row, mg_full, mg_G;      // floor(2^32 / d) (see udiv)
+  unsigned mg_batch, mg_noy, mg_full;      // floor(2^32 / d) (see udiv)
   i64 h_n, h_m;
   int relu, half_out;
   int n_classes, cls_stride;

@@ -67,6 +67,7 @@ struct BlockTile {
   int vx_min, vrows, units;        // linear axes: first coordinate; virtual rows and positions of the whole tile
   unsigned long long filter_rows;  // Mellin axes: the filter rows with a tap for some row of the tile, four bits each
   int nv;                          // how many
+  int G, at_stage, group_bytes;    // channel groups of its stages, their place in the plan's table, LDS bytes of one
 };
 
 __device__ __forceinline__ int filter_row(const BlockTile &g, int j) { return (int)(g.filter_rows >> (4 * j)) & 15; }
@@ -74,7 +75,7 @@ __device__ __forceinline__ int filter_row(const BlockTile &g, int j) { return (i
 // Item `id` of the launch: the images of a position tile lie side by side, so that the position tiles
 // with the most filter rows come first for all images and every workgroup gets its share of them.
 // `rows`: the output rows in the order of their classes, with their filter rows (Mellin axes).
-template <int P, bool JOINT>
+template <int P, int PARTS, bool JOINT>
 __device__ __forceinline__ BlockTile block_tile(ConstBlockPlan &pl, const int2 *__restrict__ rows, int id, bool mellin_x) {
   BlockTile g;
   g.c_first = 0;
@@ -114,6 +115,9 @@ __device__ __forceinline__ BlockTile block_tile(ConstBlockPlan &pl, const int2 *
     g.vrows = pl.ax * (g.rows - 1) + pl.bx_span + 1;
   }
   g.units = g.vrows * pl.RS;
+  g.at_stage = (g.slot < 0 ? min(g.nv, pl.F) : pl.F) - 1;
+  g.G = pl.stage[g.at_stage].G;
+  g.group_bytes = mellin_x ? (min(g.nv, pl.F) * g.rows * pl.RS * PARTS + 63) >> 6 << 10 : pl.group_bytes;
   return g;
 }
 
@@ -228,11 +232,11 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   auto build_tile = [&](const BlockTile &g, int parity, int2 *before) {
     // (fields of the plan, read together: one wait for the scalar loads instead of one each)
     int RS = pl.RS, cy = pl.cy + pl.by_min, uy = pl.uy, ux = pl.ux, ngx = pl.ngx, ngy = pl.ngy, tab_units = pl.tab_units, F = pl.F,
-        G = pl.G, nfx = pl.nfx, nfy = pl.nfy, none = pl.plane, group_bytes = pl.group_bytes, n_before = pl.ents;
+        G = g.G, nfx = pl.nfx, nfy = pl.nfy, none = pl.plane, group_bytes = g.group_bytes, n_before = pl.ents;
     asm volatile("" : "+s"(RS), "+s"(cy), "+s"(uy), "+s"(ux), "+s"(ngx), "+s"(ngy), "+s"(tab_units), "+s"(F), "+s"(G), "+s"(nfx),
                  "+s"(nfy), "+s"(none), "+s"(group_bytes), "+s"(n_before));
     int kx = pl.kind_x, sx = pl.sx, dx = pl.dx, px = pl.px, bx = pl.bx, bx_min = pl.bx_min, by = pl.by, by_min = pl.by_min;
-    unsigned mg_p1 = pl.mg_p1, mg_full = pl.mg_full, mg_per_row = pl.mg_per_row, mg_G = pl.mg_G;
+    unsigned mg_p1 = pl.mg_p1, mg_full = pl.mg_full, mg_per_row = pl.stage[g.at_stage].mg_per_row, mg_G = pl.stage[g.at_stage].mg_G;
     asm volatile("" : "+s"(kx), "+s"(sx), "+s"(dx), "+s"(px), "+s"(bx), "+s"(bx_min), "+s"(by), "+s"(by_min), "+s"(mg_p1),
                  "+s"(mg_full), "+s"(mg_per_row), "+s"(mg_G));
     if (mellin_x) {
@@ -309,7 +313,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
     const int *from = tab + (mellin_x ? j0 * g.rows * pl.RS : 0);
     const char *src0 = X + ((i64)g.n * pl.CG + c0) * plane_bytes;
     const unsigned dst0 = lds0 + (unsigned)(buf * pl.buf_bytes);
-    int groups = pl.G, group_bytes = pl.group_bytes;
+    int groups = g.G, group_bytes = g.group_bytes;
     asm volatile("" : "+s"(groups), "+s"(group_bytes));      // (kept in registers: a scalar load in the loop would wait for LDS as well)
     for (int b = wave; b < blocks; b += 4 * kWaves) {
       unsigned at[4];
@@ -353,7 +357,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       for (int pt = 0; pt < PARTS; ++pt) o.a[k][pt] = *(const uintx4 *)((k ? AFm1 : AFm) + off + pt * 512);
   };
 
-  BlockTile tg = block_tile<P, JOINT>(pl, rows, item, mellin_x), next_tg = tg;
+  BlockTile tg = block_tile<P, PARTS, JOINT>(pl, rows, item, mellin_x), next_tg = tg;
   if (my_tiles <= 0) return;
   int n_ents = build_tile(tg, 0, nullptr), next_ents = n_ents;
   __syncthreads();
@@ -412,10 +416,10 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
     };
     fetch_b(e0, B0);
     // ---- the stage after this one: its loads are issued under this stage's steps, its first fragments in the last two
-    const int halves = stage_halves((mellin_x ? min(pl.F, tg.nv - j0) : tg.nv) * pl.nfy * pl.G);
+    const int halves = stage_halves((mellin_x ? min(pl.F, tg.nv - j0) : tg.nv) * pl.nfy * tg.G);
     const int steps = halves / (2 * WK);
     int nj0 = mellin_x ? j0 + pl.F : tg.nv, nc0 = c0, n_se = se + halves;
-    if (nj0 >= tg.nv) { nj0 = 0; nc0 = c0 + pl.G; n_se = 0; }
+    if (nj0 >= tg.nv) { nj0 = 0; nc0 = c0 + tg.G; n_se = 0; }
     const bool last = nc0 >= tg.c_end;
     const bool more = !last || ti + 1 < my_tiles;
     const int2 *ep = my_ents + (ti & 1) * pl.ents + se;
@@ -424,7 +428,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
       nj0 = 0;
       if (more) {
         // another tile: its tables (every load of this tile has been issued, every wavefront is past the barrier)
-        next_tg = block_tile<P, JOINT>(pl, rows, (int)blockIdx.x + (ti + 1) * (int)gridDim.x, mellin_x);
+        next_tg = block_tile<P, PARTS, JOINT>(pl, rows, (int)blockIdx.x + (ti + 1) * (int)gridDim.x, mellin_x);
         next_ents = build_tile(next_tg, (ti + 1) & 1, ents + (ti & 1) * pl.ents + n_ents);
         lds_barrier();
         nc0 = next_tg.c_first;

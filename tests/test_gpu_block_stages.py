@@ -1,0 +1,54 @@
+"""Stages of the channel-blocked matrix kernel: how many channel groups and steps one has, from tile to tile of a launch; output
+and gradients against the float64 checker."""
+import numpy as np
+import pytest
+
+import _mellin_hip as hip
+import mconv
+from _gpu import assert_close, to_gpu
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # (op, n, c_in, c_out, nf, ng, s, d, p, r)
+    # input gradients on Mellin axes whose rows have one, two or all filter rows: stages of the plan's groups, of two, three and
+    # four times as many, of a number that the groups leave no room for (5 and 7 groups have no divisor), tiles of several
+    # classes, tiles over the images of a row, tiles in slices of the contracted channels
+    ("mcorr", 6, 64, 128, (3, 3), (64, 41), (1, 1), (2, 1), (2, 1), (2, 1)),
+    ("mcorr", 4, 48, 96, (6, 3), (100, 40), (1, 1), (1, 1), (2, 1), (2, 1)),
+    ("mcorr", 3, 32, 40, (4, 2), (70, 21), (1, 1), (1, 1), (3, 0), (5, 0)),
+    ("mcorr", 3, 32, 56, (5, 1), (130, 7), (1, 1), (1, 1), (1, 0), (40, 0)),
+    ("mcorr", 90, 32, 64, (4, 3), (9, 20), (1, 1), (1, 1), (1, 1), (3, 1)),
+    ("mcorr", 1, 32, 128, (7, 1), (300, 1), (1, 1), (1, 1), (2, 0), (0, 0)),
+    ("mcorr", 1, 64, 256, (4, 4), (60, 5), (1, 1), (1, 1), (1, 1), (30, 2)),
+]
+
+
+@pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("case", CASES, ids=[str(i) for i in range(len(CASES))])
+def test_stages_match_checker(case, half):
+    op, n, c_in, c_out, nf, ng, s, d, p, r = case
+    rng = np.random.default_rng(7700 + CASES.index(case))
+    kind = np.float16 if half else np.float32
+    x = rng.standard_normal((n, c_in) + ng).astype(kind)
+    w = (rng.standard_normal((c_out, c_in) + nf) * (c_in * nf[0] * nf[1]) ** -0.5).astype(kind)
+    b = rng.standard_normal(c_out).astype(kind)
+    fwd = oracle.mcorrlcorr if op == "mcorr" else oracle.lcorrlcorr
+    bwd = oracle.mcorrlcorr_backward if op == "mcorr" else oracle.lcorrlcorr_backward
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    exp = fwd(x64, w64, b.astype(np.float64), s, d, p, (1, 1), r)
+    go = rng.standard_normal(exp.shape).astype(kind)
+    egi, egw, _ = bwd(x64, w64, go.astype(np.float64), s, d, p, (1, 1))
+    xg, wg, bg = (to_gpu(a).requires_grad_() for a in (x, w, b))
+    out = (mconv._ext_mcorrlcorr if op == "mcorr" else mconv._ext_lcorrlcorr)(xg, wg, bg, s, d, p, (1, 1), r)
+    assert hip.last_variant() == ("mfma-f16-blocks" if half else "mfma-blocks")
+    out.backward(to_gpu(go))
+    taps, positions = nf[0] * nf[1], n * exp.shape[2] * exp.shape[3]
+    for got, ref, fan, what in ((out, exp, c_in * taps, "out"), (xg.grad, egi, c_out * taps, "grad_input"),
+                                (wg.grad, egw, positions, "grad_weight")):
+        if half:                                       # one rounding of a result whose sum has an error of its own
+            err = np.abs(got.detach().double().cpu().numpy() - ref)
+            assert np.all(err <= 2.0 ** -10 * np.abs(ref) + 2e-5 * fan ** 0.5), what
+        else:
+            assert_close(got, ref, fan, what)

@@ -139,7 +139,8 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
     const i64 vrows = mellin ? RT : (i64)pl.ax * (RT - 1) + pl.bx_span + 1;
     const i64 tab = ((mellin ? vrows * pl.nfx : vrows) * pl.RS + 64 + 64 + 3) & ~(i64)3;
     const i64 row_src = mellin ? 4 * RT * pl.nfx : 0;
-    auto pad = [&](int halves) { return std::max((halves + 2 * wk - 1) & -(2 * wk), 4 * wk); };      // (wk: 1 or 4)
+    const bool deep = deep_fragments(f16, wk);
+    auto pad = [&](int halves) { return std::max((halves + 2 * wk - 1) & -(2 * wk), (deep ? 8 : 4) * wk); };      // (wk: 1 or 4)
     Stage &st = stages[pl.mt - 1][at];                 // (joint tiles mostly have as many rows as those of an image)
     if (st.rows != RT) {
       st = Stage{RT, 0, 0};
@@ -150,7 +151,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
         if (2 * gb + fixed > 79 * 1024) continue;
         for (int k = 0; k < n_groups; ++k) {
           const int G = groups[k], halves = rows * pl.nfy * G, all = pad(halves);
-          if (2 * gb * G + fixed + 16 * (i64)(subsets * all + 8 * wk) > 79 * 1024) continue;
+          if (2 * gb * G + fixed + 16 * (i64)(subsets * all + (deep ? 12 : 8) * wk) > 79 * 1024) continue;
           // what a stage's steps fill of their whole pairs, against what a stage costs on top (its barrier and first reads)
           if (halves * best_all > best_halves * (all + 2 * wk)) { best_halves = halves; best_all = all + 2 * wk; st.F = F; st.G = G; }
         }
@@ -162,7 +163,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
     pl.F = mellin ? best_f : pl.nfx;
     pl.G = best_g;
     pl.tab_units = (int)tab;
-    pl.ents = (mellin ? (pl.nfx + pl.F - 1) / pl.F : 1) * pad(pl.F * pl.nfy * best_g) + 8 * wk;
+    pl.ents = (mellin ? (pl.nfx + pl.F - 1) / pl.F : 1) * pad(pl.F * pl.nfy * best_g) + (deep ? 12 : 8) * wk;
     pl.group_bytes = (int)((units * parts + 63) / 64 * 1024);
     pl.buf_bytes = pl.group_bytes * best_g;
     pl.nt = nt; pl.wm = wm; pl.wk = wk;
@@ -367,7 +368,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
           G = groups[k];
     pl.stage[n - 1] = BlockStage{G, magic(G), magic((i64)pl.nfy * G)};
   }
-  pl.mg_full = magic(std::max<i64>((pl.F * per_row + pairs - 1) / pairs * pairs, 2 * pairs));
+  pl.mg_full = magic(std::max<i64>((pl.F * per_row + pairs - 1) / pairs * pairs, (deep_fragments(f16, pl.wk) ? 4 : 2) * pairs));
   pl.rows_off = (size_t)pl.m_tiles * pl.wm * pl.mt * ((size_t)pl.CG * pl.nfx * pl.nfy + 1) * parts * 512;
   if (pl.rows_off >= (size_t)lim) return false;
   pl.filter_bytes = pl.rows_off + (mellin ? 8 * (size_t)pl.nox : 0);

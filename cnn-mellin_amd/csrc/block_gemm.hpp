@@ -66,6 +66,9 @@ struct BlockPlan {
   int joint, tile_batch, tile_q;
 };
 
+// Whether the kernel requests filter fragments four steps ahead and not two (see there); a stage then has four steps or more.
+constexpr bool deep_fragments(bool f16, int wk) { return f16 && wk == 1; }
+
 // Frequency pooling behind the layer: a forward pass of an even number of columns (`pr` leaves an odd last one out) stores the
 // maxima of pairs of them; an input gradient of `pr`, whose output is that of the maxima, is stored as that of the `cols`
 // columns they were taken from (an odd last one of them: zeros).

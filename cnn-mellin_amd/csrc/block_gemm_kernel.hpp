@@ -19,7 +19,7 @@
 // a buffer needs no memory of what it held.  The sources of a tile's virtual positions are worked
 // out once per tile into an LDS table.  While a stage multiplies, the next one's loads are issued
 // a few at a time between the steps.  Filter fragments come from L1 / L2 straight to registers,
-// two steps ahead: the WN wavefronts of a workgroup use the same ones at the same time.
+// two or four steps ahead: the WN wavefronts of a workgroup use the same ones at the same time.
 //
 // Mellin axes: output rows are taken in the order of the residue classes of the axis, so the rows
 // of a tile have taps for the same filter rows and only those are staged and multiplied; filter
@@ -178,7 +178,12 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
                                                                  unsigned char *__restrict__ which) {
   constexpr int PARTS = F16 ? 1 : 3, UB = 16 * PARTS;
   constexpr int WN = kWaves / WK / WM, P = WN * NT * 32, M_T = WM * MT * 32;
-  constexpr int kALoads = 2 * MT * PARTS;              // fragment loads of two steps
+  // Steps that a filter fragment is requested ahead of its own: two, whose products in fp32 take longer than the trip to L2.  In
+  // half they are a sixth, and a wavefront waited for its fragments in every step: four, where wavefronts do not share a tile.
+  // 128 -> 128 channels, 4 x 4 taps, 32 x 774 x 7: 85.7 -> 78.3 us (67 where every step takes the same fragment, which then
+  // comes out of L1); input gradient of 256 <- 128 on 771 x 5: 154 -> 131; ten linear layers' step 2903 -> 2682.
+  constexpr int AD = deep_fragments(F16, WK) ? 4 : 2;
+  constexpr int kALoads = AD * MT * PARTS;             // fragment loads of that many steps
   constexpr bool POOLED = OUT == OUT_POOLED, UNPOOLED = OUT == GRAD_POOLED;
   constexpr bool BLOCKED = OUT == OUT_BLOCKED || OUT == GRAD_BLOCKED || POOLED || UNPOOLED, GRAD = OUT == GRAD_PLAIN || OUT == GRAD_BLOCKED || UNPOOLED;
   extern __shared__ __align__(16) char blk_lds[];
@@ -227,8 +232,8 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   }
 
   // the sources of a tile's virtual positions, and the operand offsets of its steps
-  constexpr int kWrap = 4 * WK;                        // halves of two steps of every wavefront that shares a tile's steps
-  auto stage_halves = [](int n) { return max((n + 2 * WK - 1) / (2 * WK) * (2 * WK), kWrap); };
+  constexpr int kWrap = (AD == 4 ? 10 : 4) * WK;       // halves of the steps that a stage reads on, of every wavefront that shares a tile's
+  auto stage_halves = [](int n) { return max((n + 2 * WK - 1) / (2 * WK) * (2 * WK), 2 * AD * WK); };
   auto build_tile = [&](const BlockTile &g, int parity, int2 *before) {
     // (fields of the plan, read together: one wait for the scalar loads instead of one each)
     int RS = pl.RS, cy = pl.cy + pl.by_min, uy = pl.uy, ux = pl.ux, ngx = pl.ngx, ngy = pl.ngy, tab_units = pl.tab_units, F = pl.F,
@@ -285,13 +290,14 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
     }
     if (tid < 64 && g.units + tid < tab_units) tab[g.units + tid] = none * UB;
     // Entries of the tile's stages one behind the other (a last odd half is paired with the fragment of zeros), then
-    // the first two steps again: a stage reads on into the one that follows it.  `before`: the first two steps of
+    // the first steps again: a stage reads on into the one that follows it.  `before`: the first steps of
     // this tile also go behind the entries of the tile before it, whose last stage is running.
     int2 *out = ents + parity * n_before;
     const int per_row = nfy * G, full = stage_halves(F * per_row), subsets = (g.nv + F - 1) / F;
     const int tail = stage_halves((g.nv - (subsets - 1) * F) * per_row), n_ents = (subsets - 1) * full + tail;
     for (int e = tid; e < n_ents + kWrap; e += kThreads) {
-      const int at0 = e < n_ents ? e : e - n_ents;                       // (n_ents >= kWrap)
+      int at0 = e < n_ents ? e : e - n_ents;
+      if (AD == 4 && at0 >= n_ents) at0 -= n_ents;                       // (a stage has AD steps or more)
       const int sub = min(udiv(at0, full, mg_full), subsets - 1), at = at0 - sub * full;
       const int n_e = min(F, g.nv - sub * F) * per_row, k = min(at, n_e - 1);
       const int jj = udiv(k, per_row, mg_per_row), rest = k - jj * per_row, fy = udiv(rest, G, mg_G), gi = rest - fy * G;
@@ -345,7 +351,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   int lane_vpos[NT], lane_q[NT];
   struct Operands { uintx4 a[MT][PARTS]; };
   struct SignalOps { uintx4 b[NT][PARTS]; };
-  Operands A0, A1;
+  Operands A0, A1, A2, A3;                             // (AD == 2: A0, A1)
   SignalOps B0, B1;
 
   const unsigned lane_frag = (unsigned)(l32 * 16), zero_at = zero_frag + lane_frag;
@@ -369,6 +375,10 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
   int2 e0 = my_ents[0], e1 = my_ents[2 * WK];
   fetch_a(e0, af_c, A0);
   fetch_a(e1, af_c, A1);
+  if constexpr (AD == 4) {
+    fetch_a(my_ents[4], af_c, A2);
+    fetch_a(my_ents[6], af_c, A3);
+  }
   wait_and_barrier<0>();
 
   for (bool first = true;;) {
@@ -439,41 +449,79 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
     }
     const unsigned n_af = (unsigned)(nc0 * taps * PARTS * 512);
     // A step: the next step's signal operands are requested before its multiplies and the fragments of the step
-    // after next behind them (pinned: the scheduler moves reads next to their use).  Nothing here depends on which
+    // AD further on behind them (pinned: the scheduler moves reads next to their use).  Nothing here depends on which
     // step it is, so that every wait counts exactly what is younger: the last pair's last signal reads are of no use,
     // and its fragment fetches are the next stage's.
     auto multiply = [&](const Operands &a, const SignalOps &b) {
       if constexpr (LOW) block_multiply_low<MT, NT>(acc, low, a.a, b.b);
       else block_multiply<MT, NT, PARTS>(acc, a.a, b.b);
     };
-    int2 e2 = ep[4 * WK];
-    for (int i = 0; i + 1 < steps; i += 2) {
-      fetch_b(e1, B1);
-      const int2 e3 = ep[6 * WK];
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(A0, B0);
-      __builtin_amdgcn_sched_barrier(0);
-      fetch_a(e2, i + 2 < steps ? af_c : n_af, A0);
-      fetch_b(e2, B0);
-      const int2 e4 = ep[8 * WK];
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(A1, B1);
-      __builtin_amdgcn_sched_barrier(0);
-      fetch_a(e3, i + 3 < steps ? af_c : n_af, A1);
-      e0 = e2;
-      e1 = e3;
-      e2 = e4;
-      ep += 4 * WK;
+    if constexpr (AD == 4) {
+      // (entries: e1 of the step after this one, ahead the offset of the fragments that are requested next)
+      unsigned ahead = (unsigned)ep[8].y;
+      e1 = ep[2];
+      int at = 0;
+      auto step = [&](Operands &a, const SignalOps &b, SignalOps &next) {
+        fetch_b(e1, next);
+        e0 = e1;
+        e1.x = ep[4].x;
+        const unsigned further = (unsigned)ep[10].y;
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(a, b);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_a(make_int2(0, (int)ahead), at + 4 < steps ? af_c : n_af, a);
+        ahead = further;
+        ep += 2;
+        ++at;
+      };
+      while (at + 3 < steps) {
+        step(A0, B0, B1);
+        step(A1, B1, B0);
+        step(A2, B0, B1);
+        step(A3, B1, B0);
+      }
+      // (the fragments of the next stage's first steps move to their places)
+      if (steps & 2) {
+        step(A0, B0, B1);
+        step(A1, B1, B0);
+        const Operands a0 = A0, a1 = A1;
+        A0 = A2; A1 = A3; A2 = a0; A3 = a1;
+      }
+      if (steps & 1) {
+        step(A0, B0, B1);
+        const Operands a0 = A0;
+        A0 = A1; A1 = A2; A2 = A3; A3 = a0;
+      }
+    } else {
+      int2 e2 = ep[4 * WK];
+      for (int i = 0; i + 1 < steps; i += 2) {
+        fetch_b(e1, B1);
+        const int2 e3 = ep[6 * WK];
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(A0, B0);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_a(e2, i + 2 < steps ? af_c : n_af, A0);
+        fetch_b(e2, B0);
+        const int2 e4 = ep[8 * WK];
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(A1, B1);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_a(e3, i + 3 < steps ? af_c : n_af, A1);
+        e0 = e2;
+        e1 = e3;
+        e2 = e4;
+        ep += 4 * WK;
+      }
+      if (steps & 1) {
+        // one step left, whose operands are in A0 and B0; A1 holds the next stage's first fragments where its second's belong
+        multiply(A0, B0);
+        e0 = e1;
+        e1 = e2;
+        fetch_a(e0, n_af, A0);
+        fetch_a(e1, n_af, A1);
+      }
     }
-    if (steps & 1) {
-      // one step left, whose operands are in A0 and B0; A1 holds the next stage's first fragments where its second's belong
-      multiply(A0, B0);
-      e0 = e1;
-      e1 = e2;
-      fetch_a(e0, n_af, A0);
-      fetch_a(e1, n_af, A1);
-    }
-    // every wavefront's loads for the next stage have landed (the newest in flight are the two fragment fetches),
+    // every wavefront's loads for the next stage have landed (the newest in flight are the fragments of AD steps),
     // and every wavefront is done with this stage's buffer
     wait_and_barrier<kALoads>();
     first = last;
@@ -659,7 +707,7 @@ __global__ __launch_bounds__(kThreads, 2) void block_gemm_kernel(BlockPlan plan_
             // The masks of kAhead groups of channels are requested before the first is used, in registers that are free
             // here (fp32: of `low`; half: of the signal's operands); read where they were used, each of the tile's 16 or
             // 32 waits took a trip to memory: 28000 of 90000 cycles of a tile of 64 x 512 half values.
-            constexpr int kGroups = MT * 4, kAhead = F16 ? (16 / NT < kGroups ? 16 / NT : kGroups) : kGroups;
+            constexpr int kGroups = MT * 4, kAhead = F16 ? (8 / NT < kGroups ? 8 / NT : kGroups) : kGroups;
             uintx2 mask_of[kAhead][NT];
             auto request = [&](int i) {
 #pragma unroll

@@ -22,6 +22,16 @@ CASES = [
     ("mcorr", 90, 32, 64, (4, 3), (9, 20), (1, 1), (1, 1), (1, 1), (3, 1)),
     ("mcorr", 1, 32, 128, (7, 1), (300, 1), (1, 1), (1, 1), (2, 0), (0, 0)),
     ("mcorr", 1, 64, 256, (4, 4), (60, 5), (1, 1), (1, 1), (1, 1), (30, 2)),
+    # stages of one, two, three, four, five, six and seven steps: half tiles request fragments four steps ahead, and one stage
+    # (one tile, or several, or many of a workgroup) reads into the next
+    ("lcorr", 20, 16, 64, (2, 1), (200, 20), (1, 1), (1, 1), (0, 0), (0, 0)),
+    ("lcorr", 20, 16, 64, (2, 2), (200, 20), (1, 1), (1, 1), (0, 0), (0, 0)),
+    ("lcorr", 20, 16, 64, (3, 1), (200, 20), (1, 1), (1, 1), (1, 0), (1, 0)),
+    ("lcorr", 20, 24, 64, (3, 1), (200, 20), (1, 1), (1, 1), (1, 0), (1, 0)),
+    ("lcorr", 20, 40, 40, (2, 1), (200, 20), (1, 1), (1, 1), (0, 0), (0, 0)),
+    ("lcorr", 70, 16, 128, (3, 2), (90, 20), (1, 1), (1, 1), (1, 0), (1, 0)),
+    ("lcorr", 20, 56, 104, (2, 1), (200, 20), (1, 1), (1, 1), (0, 0), (0, 0)),
+    ("mcorr", 30, 24, 72, (3, 1), (150, 20), (1, 1), (1, 1), (2, 0), (60, 0)),
 ]
 
 

@@ -338,7 +338,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
       for (int k = 0; k < kShapes; ++k) {
         const int *const sh = shapes[k];
         if (pl.mt < mt && sh[1] == 2) continue;
-        if (like && (sh[0] != like->nt || sh[1] != like->wm || sh[2] != like->wk)) continue;
+        if (like && (like->mt * like->nt * like->wm != pl.mt * sh[0] * sh[1] || kWaves / like->wm * like->nt != kWaves / sh[1] * sh[0] || sh[2] != like->wk)) continue;
         if (f16 ? sh[0] == 2 && sh[1] == 2 : sh[0] == 4 || (sh[0] == 2 && sh[2] == 4)) continue;
         if (sh[1] == 2 && pr.c_out <= 96) continue;      // (two wavefronts along the channels: most of 128)
         const double wanted = (pl.mt < mt ? narrow : 1) * limit;
@@ -352,6 +352,14 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
   }
   if (best_cost == 0) return false;
   pl = best_plan;
+  if (!f16 && pl.mt == 2 && pl.nt == 1 && pl.wk == 1) {
+    // fp32, 64 channels x 128 positions: two by two wavefronts of 32 channels x 64 positions.  Four side by side take each
+    // filter fragment from L1 four times, 64 bytes a cycle and CU, which is all that it gives; two by two take half of that and
+    // twice the signal's operands out of LDS, also 64 of its 128 (64 -> 64 channels, 5 x 3 taps on 1177 x 10 x 41: 195 -> 178
+    // us; on 5 x 41: 180 -> 167).  Tile, stage and order of sums are the same.
+    pl.mt = 1; pl.nt = 2; pl.wm = 2;
+    pl.chan_slots = (pl.whole + pl.rest) * (kWaves / pl.wm);
+  }
   const i64 per_row = (i64)pl.nfy * pl.G, pairs = 2 * pl.wk;
   // Whole tiles with fewer filter rows than a stage holds have stages of more channel groups, as many as its LDS has room for: a
   // stage of one row of three, two groups and three columns is three steps, shorter than the trip of the next one's loads (128 <-

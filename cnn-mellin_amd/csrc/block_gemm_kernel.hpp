@@ -897,9 +897,10 @@ hipError_t launch_shape(const BlockPlan &pl, const BlockGemmArgs &a, hipStream_t
   }
   if (pl.f16 && pl.nt == 2 && pl.wk == 4)
     return pl.mt == 2 ? launch_instance<2, 2, 1, 4, true, OUT>(pl, a, stream) : launch_instance<1, 2, 1, 4, true, OUT>(pl, a, stream);
-  if (!pl.f16 && pl.wm == 2) return launch_instance<2, 2, 2, 1, false, OUT>(pl, a, stream);
+  if (!pl.f16 && pl.wm == 2)
+    return pl.mt == 2 ? launch_instance<2, 2, 2, 1, false, OUT>(pl, a, stream) : launch_instance<1, 2, 2, 1, false, OUT>(pl, a, stream);
+  if (pl.f16 && pl.mt == 2 && pl.nt == 1 && pl.wk == 1) return launch_instance<2, 1, 1, 1, true, OUT>(pl, a, stream);
   MELLIN_BLOCK_CASE(2, 2, 1, 1)
-  MELLIN_BLOCK_CASE(2, 1, 1, 1)
   MELLIN_BLOCK_CASE(1, 2, 1, 1)
   MELLIN_BLOCK_CASE(1, 1, 1, 1)
   MELLIN_BLOCK_CASE(2, 1, 1, 4)

@@ -88,12 +88,15 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
   if (pl.nfy > 64) return false;
   // A pooled output's sums keep the order of the unpooled one's, which decides what its ReLU lets through (see can_join), and
   // are those of the layer called by itself bit for bit: the same channel groups and filter columns to a stage, the same
-  // slices.  Tiles hold other positions than without the pooling (an odd last column is in none), so the order must not depend on
-  // what a tile holds: not on its being one of those in slices, nor, on Mellin axes, on the filter rows of its other output
-  // rows -- they shift the pairs that share a step where a row's taps and groups are odd in number, and the steps that
-  // wavefronts share.
-  if (like && (like->nfy != pl.nfy || like->f_off != pl.f_off || (like->whole && like->rest) ||
-               ((X.kind == AX_MCORR || X.kind == AX_MCONV) && (like->wk > 1 || like->nfy * like->G % 2))))
+  // slices.  An even number of columns makes the same tiles of them (one utterance of a ten-layer Mellin stack, whose wavefronts
+  // share tiles: 212 -> 207 us with two of its three poolings inside the products).  An odd last column is in no tile, so these hold other
+  // positions than without the pooling, and the order must not depend on what a tile holds: not on its being one of those in
+  // slices, nor, on Mellin axes, on the filter rows of its other output rows -- they shift the pairs that share a step where a
+  // row's taps and groups are odd in number, and the steps that wavefronts share.
+  const bool same_tiles = like && like->noy == pl.noy;
+  if (like && (like->nfy != pl.nfy || like->f_off != pl.f_off)) return false;
+  if (like && !same_tiles && ((like->whole && like->rest) ||
+                              ((X.kind == AX_MCORR || X.kind == AX_MCONV) && (like->wk > 1 || like->nfy * like->G % 2))))
     return false;
   const i64 py = Y.p - Y.d * fy_lo;
   pl.ay = (int)Y.s; pl.by = Y.kind == AX_LCORR ? (int)Y.d : -(int)Y.d; pl.cy = Y.kind == AX_LCORR ? -(int)py : (int)py;
@@ -280,7 +283,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
     };
     double best = 9000 + turns_cost(total, c_stages * subsets);
     pl.slices = like ? like->slices : 1;
-    int rest = like && like->rest ? total : 0;
+    int rest = !like || !like->rest ? 0 : same_tiles ? like->rest : total;
     for (int all = 0; all < (like ? 0 : 2); ++all) {
       const int r = all ? total : total % per_m;
       if (r == 0 || (all && total >= 2 * per_m) || (pl.wk > 1 && !all)) continue;
@@ -338,7 +341,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
       for (int k = 0; k < kShapes; ++k) {
         const int *const sh = shapes[k];
         if (pl.mt < mt && sh[1] == 2) continue;
-        if (like && (like->mt * like->nt * like->wm != pl.mt * sh[0] * sh[1] || kWaves / like->wm * like->nt != kWaves / sh[1] * sh[0] || sh[2] != like->wk)) continue;
+        if (like && (like->mt * like->wm != pl.mt * sh[1] || kWaves / like->wm * like->nt != kWaves / sh[1] * sh[0] || sh[2] != like->wk)) continue;
         if (f16 ? sh[0] == 2 && sh[1] == 2 : sh[0] == 4 || (sh[0] == 2 && sh[2] == 4)) continue;
         if (sh[1] == 2 && pr.c_out <= 96) continue;      // (two wavefronts along the channels: most of 128)
         const double wanted = (pl.mt < mt ? narrow : 1) * limit;

@@ -33,9 +33,15 @@ CASES = [
     ((4, True, 3, (4, 4), 70, 2, 1, 2, 1, 10, 10), 2, dict(mt=1, nt=1, whole=0)),
     ((4, True, 4, (4, 2), 20, 2, 2, 1, 60, 200, 7), 2, dict(mt=2, nt=2)),
     ((4, True, 4, (2, 1), 64, 2, 2, 1, 20, 100, 20), 2, dict(mt=2, nt=2, wm=2)),
-    # the order of the sums would depend on what a tile holds: a pass of its own
-    ((4, True, 3, (5, 3), 32, 3, 1, 2, 60, 60, 10), 1, dict(wk=1)),
-    ((4, True, 4, (5, 1), 20, 3, 1, 2, 2, 5, 6), 1, dict(wk=4)),
+    # an even number of columns: the same tiles, whatever the order of their sums depends on
+    ((4, True, 3, (5, 3), 32, 3, 1, 2, 60, 60, 10), 2, dict(wk=1)),
+    ((4, True, 4, (5, 1), 20, 3, 1, 2, 2, 5, 6), 2, dict(wk=4)),
+    ((2, True, 3, (4, 4), 40, 3, 1, 1, 1, 70, 20), 2, dict(wk=4)),
+    ((4, True, 3, (4, 4), 128, 3, 1, 1, 1, 337, 10), 2, dict(wk=4, whole=0)),
+    ((4, True, 4, (5, 3), 64, 3, 1, 2, 300, 10, 20), 2, dict(mt=1, nt=2, wm=2)),
+    # an odd one, and an order of the sums that would depend on what a tile holds: a pass of its own
+    ((4, True, 3, (5, 3), 32, 3, 1, 2, 60, 60, 11), 1, dict(wk=1)),
+    ((4, True, 4, (5, 1), 20, 3, 1, 2, 2, 5, 7), 1, dict(wk=4)),
     ((4, False, 4, (3, 4), 70, 2, 1, 1, 60, 100, 5), 1, dict(whole=170, rest=10)),
 ]
 

@@ -87,6 +87,11 @@ SYMBOLS["mellin_layer_forward_workspace"] = (_size_t, [_int, _int] + _DIMS)
 SYMBOLS["mellin_layer_forward"] = (_int, [_int, _int, _int, _ptr, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _ptr, _size_t, _ptr])
 SYMBOLS["mellin_layer_backward_workspace"] = (_size_t, [_int, _int, _int] + _DIMS)
 SYMBOLS["mellin_layer_backward"] = (_int, [_int, _int, _int] + [_ptr] * 4 + _DIMS + [_ptr] * 4 + [_size_t, _ptr])
+SYMBOLS["mellin_layer_kept_bytes"] = (_size_t, [_int, _int] + _DIMS)
+SYMBOLS["mellin_layer_forward_kept_workspace"] = (_size_t, [_int, _int] + _DIMS)
+SYMBOLS["mellin_layer_forward_kept"] = (_int, [_int, _int, _int, _ptr, _ptr, _ptr] + _DIMS + [_ptr, _ptr, _ptr, _ptr, _size_t, _ptr])
+SYMBOLS["mellin_layer_backward_kept_workspace"] = (_size_t, [_int, _int, _int] + _DIMS)
+SYMBOLS["mellin_layer_backward_kept"] = (_int, [_int, _int, _int] + [_ptr] * 4 + _DIMS + [_ptr] * 5 + [_size_t, _ptr])
 SYMBOLS["mellin_layer_plan"] = (_int, [_int, _int, _int] + _DIMS + [_ptr])
 SYMBOLS["mellin_layer_bias_route"] = (_int, [_int, _int, _int] + _DIMS)
 SYMBOLS["mellin_stack_first_layer"] = (_int, [_int, _int] + _DIMS)

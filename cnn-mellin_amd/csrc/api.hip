@@ -1758,6 +1758,23 @@ int mellin_layer_plan(int kind_x, int elem_bytes, int gradient, MELLIN_CORR2D_DI
   return bp.pool ? 2 : 1;
 }
 
+// A training step's weight gradient reads the blocked input that the forward pass has made, and makes it again if nobody
+// kept it: a pass that reads the tensor and writes it once or, in fp32, one and a half times.  128 -> 256 channels, 3 x 3 taps,
+// 32 x 256 x 41, us a step: half on Mellin rows 567 -> 498, fp32 linear 3139 -> 3045.  Up to 256 MiB, which the graph then holds
+// beside the input between the two calls (the backward call had as much as scratch memory).  From 4 MiB: smaller ones are
+// blocked beside grad_out, in a launch that is made anyway, within its 7 us, and their steps wait for the host (41 -> 128
+// channels, 8 taps, 32 x 780: fp32, 7 MB, 83.7 -> 82.9; half, 2 MB, no difference).
+constexpr size_t kLeastKeptBytes = (size_t)4 << 20, kMostKeptBytes = (size_t)256 << 20;
+size_t mellin_layer_kept_bytes(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
+  const bool half = elem_bytes != 4;
+  if (batch < 1 || c_in < 1 || ngx < 1 || ngy < 1 || batch > 65535 || c_in > 1 << 24 || ngx > 1 << 22 || ngy > 1 << 22) return 0;
+  if ((double)batch * ngx * ngy * c_in > 1e12) return 0;
+  const size_t bytes = blocked_region(batch, c_in, ngx * ngy, half);
+  if (bytes < kLeastKeptBytes || bytes > kMostKeptBytes || !layer_elements(elem_bytes) || check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
+  BlockPlan bp;
+  BlockWgradPlan wp;
+  return plan_block_forward(kind_x, half, CORR2D_ARGS, bp) && plan_block_weight(kind_x, half, CORR2D_ARGS, wp) ? bytes : 0;
+}
 size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
   if (!layer_elements(elem_bytes)) return 0;
   if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
@@ -1773,18 +1790,29 @@ size_t mellin_layer_forward_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_
   const size_t own = mellin_corr2d_forward_f16_workspace(kind_x, CORR2D_ARGS);
   return elem_bytes == 2 ? own : align256(own) + align256(c_out * c_in * nfx * nfy * 2) + c_out * 2;
 }
+size_t mellin_layer_forward_kept_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
+  return mellin_layer_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS) - mellin_layer_kept_bytes(kind_x, elem_bytes, CORR2D_ARGS);
+}
 int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void *input, const void *weight,
                          const void *bias, MELLIN_CORR2D_DIMS, void *out, void *weight_half, void *workspace,
                          size_t workspace_bytes, void *stream) {
+  return mellin_layer_forward_kept(kind_x, elem_bytes, activation, input, weight, bias, CORR2D_ARGS, out, weight_half, nullptr, workspace,
+                                   workspace_bytes, stream);
+}
+int mellin_layer_forward_kept(int kind_x, int elem_bytes, int activation, const void *input, const void *weight,
+                              const void *bias, MELLIN_CORR2D_DIMS, void *out, void *weight_half, void *kept, void *workspace,
+                              size_t workspace_bytes, void *stream) {
   int rc;
   if (!layer_elements(elem_bytes)) return bad_elements(__func__, elem_bytes);
   if ((rc = check_corr2d(__func__, kind_x, CORR2D_ARGS))) return rc;
+  if (kept && !mellin_layer_kept_bytes(kind_x, elem_bytes, CORR2D_ARGS))
+    return fail(MELLIN_ERR_ARGUMENT, "%s: this layer keeps nothing (mellin_layer_kept_bytes)", __func__);
   const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT;
   const i64 n_w = c_out * c_in * nfx * nfy;
   hipStream_t st = (hipStream_t)stream;
   BlockPlan bp;
   if (plan_block_forward(kind_x, half, CORR2D_ARGS, bp)) {
-    const size_t signal = blocked_region(batch, c_in, ngx * ngy, half), filter = align256(bp.filter_bytes);
+    const size_t signal = kept ? 0 : blocked_region(batch, c_in, ngx * ngy, half), filter = align256(bp.filter_bytes);
     const i64 per = blocked_images(batch, c_in, ngx * ngy, half);
     const size_t need = per < batch ? mellin_layer_forward_workspace(kind_x, elem_bytes, CORR2D_ARGS) : signal + filter + bp.slice_bytes;
     if (!workspace || workspace_bytes < need)
@@ -1805,12 +1833,12 @@ int mellin_layer_forward(int kind_x, int elem_bytes, int activation, const void 
     bp.wide = wide;
     g_variant = half ? "mfma-f16-blocks" : "mfma-blocks";
     g_last_math = half ? (int)MELLIN_MATH_F16 : (int)MATH_BF16X3;
-    char *ws = (char *)workspace;
+    char *ws = (char *)workspace, *blocked = kept ? (char *)kept : ws;
     float *sums = (float *)(ws + signal + filter);
-    const PackSignal x = {input, nullptr, ws, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
+    const PackSignal x = {input, nullptr, blocked, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
     const PackFilter f = pack_filter(bp, (int)c_in, weight, ws + signal, wide ? weight_half : nullptr, n_w);
     hipError_t e = launch_block_pack(half, &x, nullptr, &f, 1, st);
-    const BlockGemmArgs args = {ws, ws + signal, bias, out, sums, false, false, nullptr, nullptr};
+    const BlockGemmArgs args = {blocked, ws + signal, bias, out, sums, false, false, nullptr, nullptr};
     if (e == hipSuccess) e = launch_block_gemm(bp, args, st);
     if (e == hipSuccess && bp.rest > 0) {
       BlockFinish fin = {};
@@ -1848,7 +1876,8 @@ struct LayerBackward {
   BlockPlan bp;
   BlockWgradPlan wp;
 };
-static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS, LayerBackward &lb) {
+// (kept: the forward pass's blocked input is there)
+static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS, LayerBackward &lb, bool kept = false) {
   const bool half = elem_bytes != 4, wide = elem_bytes == MELLIN_ELEM_HALF_FLOAT;
   const int elem = half ? 2 : 4;
   const bool wi = want & MELLIN_WANT_INPUT, ww = want & MELLIN_WANT_WEIGHT;
@@ -1866,7 +1895,7 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
   auto take = [&](size_t bytes) { const size_t off = at; at += align256(bytes); return off; };
   lb.masked_off = take(lb.plain && (want & MELLIN_WANT_RELU) ? (size_t)(batch * c_out * nhx * nhy) * elem : 0);
   lb.go_off = take(any ? blocked_bytes(batch, c_out, nhx * nhy, half) : 0);
-  lb.x_off = take(lb.weight_blocked ? blocked_bytes(batch, c_in, ngx * ngy, half) : 0);
+  lb.x_off = take(lb.weight_blocked && !kept ? blocked_bytes(batch, c_in, ngx * ngy, half) : 0);
   lb.frag_off = take(lb.input_blocked ? lb.bp.filter_bytes : 0);
   lb.slice_off = take(lb.input_blocked ? lb.bp.slice_bytes : 0);
   lb.bias_off = take(lb.bias_packed ? pack_partial_count(batch, c_out, nhx * nhy) * 4 : 0);
@@ -1895,20 +1924,32 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
 static i64 backward_images(const LayerBackward &lb, bool half, MELLIN_CORR2D_DIMS) {
   return lb.input_blocked ? blocked_images(batch, c_out, nhx * nhy, half) : batch;
 }
-size_t mellin_layer_backward_workspace(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS) {
+static size_t layer_backward_workspace(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS, bool kept) {
   if (!layer_elements(elem_bytes)) return 0;
-  if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
+  if (check_corr2d("mellin_layer_backward_workspace", kind_x, CORR2D_ARGS)) return 0;
   LayerBackward lb;
-  plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb);
+  plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb, kept);
   const i64 per = backward_images(lb, elem_bytes != 4, CORR2D_ARGS);
   if (per == batch) return lb.total;
-  auto part = [&](int want, i64 batch) { return mellin_layer_backward_workspace(kind_x, elem_bytes, want, CORR2D_ARGS); };
+  auto part = [&](int want, i64 batch) { return layer_backward_workspace(kind_x, elem_bytes, want, CORR2D_ARGS, kept); };
   const size_t need = std::max(part(INPUT_ONLY(want), per), part(INPUT_ONLY(want), (batch - 1) % per + 1));
   return want & (MELLIN_WANT_WEIGHT | MELLIN_WANT_BIAS) ? std::max(need, part(want & ~MELLIN_WANT_INPUT, batch)) : need;
+}
+size_t mellin_layer_backward_workspace(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS) {
+  return layer_backward_workspace(kind_x, elem_bytes, want, CORR2D_ARGS, false);
+}
+size_t mellin_layer_backward_kept_workspace(int kind_x, int elem_bytes, int want, MELLIN_CORR2D_DIMS) {
+  return layer_backward_workspace(kind_x, elem_bytes, want, CORR2D_ARGS, true);
 }
 int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *input, const void *weight,
                           const void *grad_out, const void *out, MELLIN_CORR2D_DIMS, void *grad_input,
                           void *grad_weight, void *grad_bias, void *workspace, size_t workspace_bytes, void *stream) {
+  return mellin_layer_backward_kept(kind_x, elem_bytes, want, input, weight, grad_out, out, CORR2D_ARGS, grad_input, grad_weight, grad_bias,
+                                    nullptr, workspace, workspace_bytes, stream);
+}
+int mellin_layer_backward_kept(int kind_x, int elem_bytes, int want, const void *input, const void *weight,
+                               const void *grad_out, const void *out, MELLIN_CORR2D_DIMS, void *grad_input, void *grad_weight,
+                               void *grad_bias, const void *kept, void *workspace, size_t workspace_bytes, void *stream) {
   int rc;
   if (!layer_elements(elem_bytes)) return bad_elements(__func__, elem_bytes);
   if ((rc = check_corr2d(__func__, kind_x, CORR2D_ARGS))) return rc;
@@ -1916,16 +1957,16 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
       ((want & MELLIN_WANT_WEIGHT) && !grad_weight) || ((want & MELLIN_WANT_BIAS) && !grad_bias))
     return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
   LayerBackward lb;
-  plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb);
+  plan_layer_backward(kind_x, elem_bytes, want, CORR2D_ARGS, lb, kept != nullptr);
   const i64 per = backward_images(lb, elem_bytes != 4, CORR2D_ARGS);
-  const size_t need = per < batch ? mellin_layer_backward_workspace(kind_x, elem_bytes, want, CORR2D_ARGS) : lb.total;
+  const size_t need = per < batch ? layer_backward_workspace(kind_x, elem_bytes, want, CORR2D_ARGS, kept != nullptr) : lb.total;
   if (need && (!workspace || workspace_bytes < need))
     return fail(MELLIN_ERR_WORKSPACE, "%s: needs %zu bytes of workspace, got %zu", __func__, need, workspace_bytes);
   if (per < batch) {
     if (!grad_out || !weight) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
     if (want & (MELLIN_WANT_WEIGHT | MELLIN_WANT_BIAS))
-      rc = mellin_layer_backward(kind_x, elem_bytes, want & ~MELLIN_WANT_INPUT, input, weight, grad_out, out, CORR2D_ARGS, nullptr,
-                                 grad_weight, grad_bias, workspace, workspace_bytes, stream);
+      rc = mellin_layer_backward_kept(kind_x, elem_bytes, want & ~MELLIN_WANT_INPUT, input, weight, grad_out, out, CORR2D_ARGS, nullptr,
+                                      grad_weight, grad_bias, kept, workspace, workspace_bytes, stream);
     const i64 size = elem_bytes == 4 ? 4 : 2, x_image = c_in * ngx * ngy * size, h_image = c_out * nhx * nhy * size;
     auto part = [&](i64 first, i64 batch) {
       return mellin_layer_backward(kind_x, elem_bytes, INPUT_ONLY(want), nullptr, weight, (const char *)grad_out + first * h_image,
@@ -1980,7 +2021,7 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
                          (int)batch, (int)c_out, (int)(nhx * nhy)};
   const PackSignal x = {input, nullptr, ws + lb.x_off, nullptr, (int)batch, (int)c_in, (int)(ngx * ngy)};
   const PackFilter f = lb.input_blocked ? pack_filter(lb.bp, (int)c_out, weight, ws + lb.frag_off, nullptr, 0) : PackFilter{};
-  e = launch_block_pack(half, &go, lb.weight_blocked ? &x : nullptr, &f, lb.input_blocked, st);
+  e = launch_block_pack(half, &go, lb.weight_blocked && !kept ? &x : nullptr, &f, lb.input_blocked, st);
   BlockFinish fin = {};
   if (lb.input_blocked) {
     lb.bp.relu = 0;
@@ -1990,7 +2031,7 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
   }
   if (lb.weight_blocked) {
     fin.add_weight(lb.wp, ws + lb.wgrad_off, grad_weight);
-    if (e == hipSuccess) e = launch_block_wgrad(lb.wp, ws + lb.go_off, ws + lb.x_off, (float *)(ws + lb.wgrad_off), st);
+    if (e == hipSuccess) e = launch_block_wgrad(lb.wp, ws + lb.go_off, kept ? kept : ws + lb.x_off, (float *)(ws + lb.wgrad_off), st);
   }
   if (sums) fin.add_bias(ws + lb.bias_off, (i64)pack_partial_count(batch, 1, nhx * nhy), c_out, grad_bias);
   if (e == hipSuccess) e = launch_block_finish(half, wide, fin, st);

@@ -63,12 +63,14 @@ struct Corr2dBackward : public torch::autograd::Node {
   int elem = 4;                          // as the library's entry points take it
   at::ScalarType param_kind = at::kFloat;
   torch::autograd::SavedVariable input_, weight_, out_;
+  Tensor kept_;                          // the forward call's copy of the input in the kernels' layout, if it left one
   std::vector<int64_t> out_sizes;
   at::TensorOptions options;
 
   std::string name() const override { return "Corr2dBackward"; }
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
+    kept_.reset();
     input_.reset_data();
     weight_.reset_data();
     out_.reset_data();
@@ -76,9 +78,10 @@ struct Corr2dBackward : public torch::autograd::Node {
 
   torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
     at::AutoGradMode no_grad(false);
-    Tensor input, weight, out;
+    Tensor input, weight, out, kept;
     {
       std::lock_guard<std::mutex> lock(mutex_);
+      kept = kept_;
       input = input_.unpack();
       weight = weight_.unpack();
       if (relu) out = out_.unpack(shared_from_this());
@@ -93,13 +96,13 @@ struct Corr2dBackward : public torch::autograd::Node {
     if (task_should_compute_output(1)) { want |= MELLIN_WANT_WEIGHT; grad_weight = at::empty(weight.sizes(), weight.options().dtype(param_kind)); }
     if (has_bias && task_should_compute_output(2)) { want |= MELLIN_WANT_BIAS; grad_bias = at::empty({g.c_out}, weight.options().dtype(param_kind)); }
     if (want & ~MELLIN_WANT_RELU) {
-      const size_t need = mellin_layer_backward_workspace(g.kind, elem, want, GEOMETRY_ARGS(g));
+      const size_t need = (kept.defined() ? mellin_layer_backward_kept_workspace : mellin_layer_backward_workspace)(g.kind, elem, want, GEOMETRY_ARGS(g));
       Tensor ws = scratch(input, need);
-      check(mellin_layer_backward(g.kind, elem, want, pointer(input), pointer(weight), pointer(grad_out), pointer(out),
-                                  GEOMETRY_ARGS(g), grad_input.defined() ? grad_input.data_ptr() : nullptr,
-                                  grad_weight.defined() ? grad_weight.data_ptr() : nullptr,
-                                  grad_bias.defined() ? grad_bias.data_ptr() : nullptr,
-                                  ws.defined() ? ws.data_ptr() : nullptr, need, launch_stream(input)));
+      check(mellin_layer_backward_kept(g.kind, elem, want, pointer(input), pointer(weight), pointer(grad_out), pointer(out),
+                                       GEOMETRY_ARGS(g), grad_input.defined() ? grad_input.data_ptr() : nullptr,
+                                       grad_weight.defined() ? grad_weight.data_ptr() : nullptr,
+                                       grad_bias.defined() ? grad_bias.data_ptr() : nullptr, pointer(kept),
+                                       ws.defined() ? ws.data_ptr() : nullptr, need, launch_stream(input)));
     }
     return {grad_input, grad_weight, grad_bias};
   }
@@ -212,7 +215,7 @@ PyObject *corr(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     // half tensors of a layer with float parameters: the library rounds them, and keeps the rounded weight for the backward
     const bool wide = kind_of == at::kHalf && weight0.scalar_type() == at::kFloat && (!bias0.defined() || bias0.scalar_type() == at::kFloat);
     const int elem = wide ? MELLIN_ELEM_HALF_FLOAT : kind_of == at::kHalf ? 2 : 4;
-    Tensor input, weight, bias, weight_half;
+    Tensor input, weight, bias, weight_half, kept;
     {
       at::AutoGradMode no_grad(false);
       input = input0.scalar_type() == kind_of ? input0.contiguous() : input0.to(kind_of).contiguous();
@@ -226,11 +229,15 @@ PyObject *corr(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
       }
       out = dims == 2 ? at::empty({g.batch, g.c_out, g.nh[0], g.nh[1]}, input.options())
                       : at::empty({g.batch, g.c_out, g.nh[0]}, input.options());
-      const size_t need = mellin_layer_forward_workspace(g.kind, elem, GEOMETRY_ARGS(g));
+      // (hooks on saved tensors decide where those live, and what the backward call reads)
+      if (differentiable && weight0.requires_grad() && !at::SavedTensorDefaultHooks::get_hooks())
+        kept = scratch(input, mellin_layer_kept_bytes(g.kind, elem, GEOMETRY_ARGS(g)));
+      const size_t need = (kept.defined() ? mellin_layer_forward_kept_workspace : mellin_layer_forward_workspace)(g.kind, elem, GEOMETRY_ARGS(g));
       Tensor ws = scratch(input, need);
-      check(mellin_layer_forward(g.kind, elem, relu ? MELLIN_ACT_RELU : MELLIN_ACT_NONE, pointer(input), pointer(weight),
-                                 pointer(bias), GEOMETRY_ARGS(g), out.data_ptr(),
-                                 weight_half.defined() ? weight_half.data_ptr() : nullptr, ws.defined() ? ws.data_ptr() : nullptr, need, launch_stream(input)));
+      check(mellin_layer_forward_kept(g.kind, elem, relu ? MELLIN_ACT_RELU : MELLIN_ACT_NONE, pointer(input), pointer(weight),
+                                      pointer(bias), GEOMETRY_ARGS(g), out.data_ptr(),
+                                      weight_half.defined() ? weight_half.data_ptr() : nullptr, kept.defined() ? kept.data_ptr() : nullptr,
+                                      ws.defined() ? ws.data_ptr() : nullptr, need, launch_stream(input)));
     }
     if (differentiable) {
       auto node = std::shared_ptr<Corr2dBackward>(new Corr2dBackward(), torch::autograd::deleteNode);
@@ -238,6 +245,7 @@ PyObject *corr(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
       node->g = g;
       node->relu = relu;
       node->has_bias = bias0.defined();
+      node->kept_ = kept;
       node->input_ = torch::autograd::SavedVariable(input, false);
       node->weight_ = torch::autograd::SavedVariable(wide ? weight_half : weight, false);
       node->elem = elem;

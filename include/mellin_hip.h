@@ -441,6 +441,11 @@ int mellin_pool_pairs_backward_f16(const void *grad_y, const unsigned char *whic
  * of the *_workspace call under the same settings, 256-byte aligned; copies of tensors in the
  * kernels' own layout (6 bytes a float, 2 a half) take at most 4 GiB of it each: larger layers
  * go through it in parts.
+ * A training step's forward call can leave its copy of the input in the kernels' layout for the
+ * weight gradient: mellin_layer_kept_bytes says how many bytes that takes (0: this layer keeps
+ * nothing).  The *_kept calls take a buffer of that size, 256-byte aligned, and scratch as their
+ * own *_workspace calls say.  The backward call still takes `input`, for settings that have
+ * changed in between.
  * ------------------------------------------------------------------------ */
 #define MELLIN_WANT_INPUT 1
 #define MELLIN_WANT_WEIGHT 2
@@ -459,6 +464,19 @@ int mellin_layer_backward(int kind_x, int elem_bytes, int want, const void *inpu
                           MELLIN_CORR2D_DIMS, void *grad_input, void *grad_weight,
                           void *grad_bias, void *workspace, size_t workspace_bytes,
                           void *stream);
+size_t mellin_layer_kept_bytes(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS);
+size_t mellin_layer_forward_kept_workspace(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS);
+int mellin_layer_forward_kept(int kind_x, int elem_bytes, int activation, const void *input,
+                              const void *weight, const void *bias, MELLIN_CORR2D_DIMS,
+                              void *out, void *weight_half, void *kept, void *workspace,
+                              size_t workspace_bytes, void *stream);
+size_t mellin_layer_backward_kept_workspace(int kind_x, int elem_bytes, int want,
+                                            MELLIN_CORR2D_DIMS);
+int mellin_layer_backward_kept(int kind_x, int elem_bytes, int want, const void *input,
+                               const void *weight, const void *grad_out, const void *out,
+                               MELLIN_CORR2D_DIMS, void *grad_input, void *grad_weight,
+                               void *grad_bias, const void *kept, void *workspace,
+                               size_t workspace_bytes, void *stream);
 
 /* A stack of layers, each followed by a ReLU, in one call per direction.  Between layers the tensors stay in the layout of
  * the matrix kernels (channel-blocked), so nothing is laid out anew, and the backward of the ReLUs, the bias gradients and

@@ -13,7 +13,6 @@ namespace mellin {
 namespace {
 
 constexpr int kFinishThreads = 256;
-constexpr int kFinishTaps = 64;
 constexpr int kSliceValues = kFinishThreads * 4;       // values of a tile that a block adds up
 
 // (JOBS: 1 or kFinishJobs: a layer's launch does not carry a stack's arguments; measured at kPackFilters)
@@ -52,60 +51,59 @@ __device__ __forceinline__ float add_chain(const float *__restrict__ p, i64 step
   return s;
 }
 
-// gw[m, c, fx, fy] = the sum of its partial sums in slice order.  A block owns 32 weights that lie side by side in
-// the partial blocks; its eight groups of 32 threads add an eighth of the slices each, and those sums are added in order.
-template <typename T>
-__device__ void finish_weight(const WeightSums &pl, int b, float (*red)[32]) {
-  const float *__restrict__ ws = pl.partial;
-  T *__restrict__ gw = (T *)pl.grad;
-  const int cl = threadIdx.x & 31, grp = threadIdx.x >> 5;
-  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.m_t;
-  // block -> (filter row, column tile, channel)
-  const int tiles = pl.ctb * pl.nfy;
-  const int m = b % pl.M;
-  b /= pl.M;
-  const int tile = b % tiles;
-  b /= tiles;
-  const int cb = b % pl.c_blocks, fx = b / pl.c_blocks;
-  const int ct = tile / pl.nfy, fy = tile - ct * pl.nfy, c = (cb * pl.ctb + ct) * 32 + cl;
-  const int mb = m / m_t, ml = m - mb * m_t;
-  const int slices = pl.slices[fx], blocks = pl.m_blocks * pl.c_blocks;
-  const i64 stride = (i64)blocks * m_t * cols;
-  const float *p = ws + ((i64)pl.slice0[fx] * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols + tile * 32 + cl;
-  const int lo = slices * grp / 8, hi = slices * (grp + 1) / 8;
-  red[grp][cl] = add_chain(p + lo * stride, stride, hi - lo, 0.f);
-  __syncthreads();
-  if (grp == 0 && c < pl.C) {
-    float a = red[0][cl];
+// The same of four values side by side, eight of them added pairwise at a time (which rounds less than one after the other).
+__device__ __forceinline__ float4 add_chain4(const float *__restrict__ p, i64 step, int count) {
+  constexpr int kAtOnce = 8;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int k = 0; k < count; k += kAtOnce, p += kAtOnce * step) {
+    float4 v[kAtOnce];
 #pragma unroll
-    for (int i = 1; i < 8; ++i) a += red[i][cl];
-    gw[(((i64)m * pl.C + c) * pl.nfx + fx) * pl.f_pitch + pl.f_off + fy] = (T)a;
+    for (int i = 0; i < kAtOnce; ++i) v[i] = k + i < count ? *(const float4 *)(p + i * step) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int n = kAtOnce / 2; n > 0; n /= 2)
+#pragma unroll
+      for (int i = 0; i < n; ++i) {
+        v[i].x += v[i + n].x; v[i].y += v[i + n].y; v[i].z += v[i + n].z; v[i].w += v[i + n].w;
+      }
+    s.x += v[0].x; s.y += v[0].y; s.z += v[0].z; s.w += v[0].w;
   }
+  return s;
 }
 
-// The same for weights that are many and have few slices (less than 16 on average: a block per 32 weights would mostly wait, and write 4 bytes of
-// every line): a block owns an output channel and 32 input channels with all their taps, which it writes side by side.
+// gw[m, c, fx, fy] = the sum of its partial sums.  A block owns an output channel and 32 input channels with `tap_chunk` of their
+// taps, which it writes side by side; eight threads add the partial sums of a tap over one of `parts` of the slices, 16 bytes a
+// thread, and the parts are added in order.  What bounds it is reading the partial sums, 64 KB of each of the weight
+// gradient's workgroups.  A block of 32 weights of one tap, or all slices a thread, four bytes at a time, took up to twice the
+// time, and wrote four bytes of every line: half, 128 -> 128 channels, 4 x 4 taps 20.6 -> 14.2 us, 256 -> 256 25 -> 14.3 and 128 ->
+// 256, 3 x 3 taps, fp32 28 -> 22.
 template <typename T>
-__device__ void finish_weight_taps(const WeightSums &pl, int b, float (*sum)[33]) {
-  const float *__restrict__ ws = pl.partial;
-  T *__restrict__ gw = (T *)pl.grad;
-  const int cols = pl.ctb * pl.nfy * 32, m_t = pl.m_t, c_tiles = (pl.C + 31) / 32, taps = pl.nfx * pl.nfy;
-  const int m = b / c_tiles, ct_all = b - m * c_tiles, cl = threadIdx.x & 31;
-  const int mb = m / m_t, ml = m - mb * m_t, cb = ct_all / pl.ctb, ct = ct_all - cb * pl.ctb;
-  const int blocks = pl.m_blocks * pl.c_blocks;
-  const i64 stride = (i64)blocks * m_t * cols;
-  for (int tap = threadIdx.x >> 5; tap < taps; tap += kFinishThreads / 32) {
-    const int fx = tap / pl.nfy, fy = tap - fx * pl.nfy, slices = pl.slices[fx];
-    const float *p = ws + ((i64)pl.slice0[fx] * blocks + mb * pl.c_blocks + cb) * (i64)m_t * cols + (i64)ml * cols +
-                     (ct * pl.nfy + fy) * 32 + cl;
-    sum[tap][cl] = add_chain(p, stride, slices, 0.f);
+__device__ void finish_weight(const WeightSums &pl, int b, float *__restrict__ red) {
+  constexpr int kRow = 33;
+  const int all_taps = pl.nfx * pl.nfy, c_tiles = (pl.C + 31) / 32;
+  const int m = b % pl.M;
+  b /= pl.M;
+  const int chunk = b / c_tiles, c_tile = b - chunk * c_tiles, tap0 = chunk * pl.tap_chunk, taps = min(pl.tap_chunk, all_taps - tap0);
+  const int parts = pl.parts, t = threadIdx.x, c4 = (t & 7) * 4, part = (t >> 3) / taps, tap = (t >> 3) - part * taps;
+  if (part < parts) {
+    const int fx = (tap0 + tap) / pl.nfy, fy = tap0 + tap - fx * pl.nfy, slices = pl.slices[fx];
+    const int lo = slices * part / parts, hi = slices * (part + 1) / parts;
+    const int mb = m / pl.m_t, ml = m - mb * pl.m_t, cb = c_tile / pl.ctb, ct = c_tile - cb * pl.ctb;
+    const int cols = pl.ctb * pl.nfy * 32, blocks = pl.m_blocks * pl.c_blocks;
+    const i64 stride = (i64)blocks * pl.m_t * cols;
+    const float4 s = add_chain4(pl.partial + ((i64)pl.slice0[fx] * blocks + mb * pl.c_blocks + cb) * (i64)pl.m_t * cols + (i64)ml * cols +
+                                    (ct * pl.nfy + fy) * 32 + c4 + lo * stride,
+                                stride, hi - lo);
+    float *to = red + (part * taps + tap) * kRow + c4;
+    to[0] = s.x; to[1] = s.y; to[2] = s.z; to[3] = s.w;
   }
   __syncthreads();
-  const int live = min(32, pl.C - ct_all * 32);
-  T *out = gw + ((i64)m * pl.C + ct_all * 32) * pl.nfx * pl.f_pitch + pl.f_off;
-  for (int i = threadIdx.x; i < live * taps; i += kFinishThreads) {
-    const int c = i / taps, tap = i - c * taps, fx = tap / pl.nfy, fy = tap - fx * pl.nfy;
-    out[(c * pl.nfx + fx) * pl.f_pitch + fy] = (T)sum[tap][c];
+  const int live = min(32, pl.C - c_tile * 32) * taps;
+  T *out = (T *)pl.grad + ((i64)m * pl.C + c_tile * 32) * pl.nfx * pl.f_pitch + pl.f_off;
+  for (int i = t; i < live; i += kFinishThreads) {
+    const int c = i / taps, tp = i - c * taps, fx = (tap0 + tp) / pl.nfy, fy = tap0 + tp - fx * pl.nfy;
+    float a = red[tp * kRow + c];
+    for (int k = 1; k < parts; ++k) a += red[(k * taps + tp) * kRow + c];
+    out[(c * pl.nfx + fx) * pl.f_pitch + fy] = (T)a;
   }
 }
 
@@ -237,14 +235,13 @@ __device__ void finish_units(const SliceSums &a, int b, float (*red)[32]) {
 
 template <typename T, typename TG, int JOBS>           // tensors, gradients of the parameters
 __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs<JOBS> a) {
-  __shared__ float red[8][32], taps[kFinishTaps][33];
+  __shared__ float red[8][32], weight_sums[kFinishThreads / 8 * 33];
   const int tid = threadIdx.x;
   unsigned b = blockIdx.x;
   for (int i = 0; i < a.n_weights; ++i) {
     const WeightSums &w = a.w[i];
     if (b < w.blocks) {
-      if (w.taps) finish_weight_taps<TG>(w, (int)b, taps);
-      else finish_weight<TG>(w, (int)b, red);
+      finish_weight<TG>(w, (int)b, weight_sums);
       return;
     }
     b -= w.blocks;
@@ -307,13 +304,24 @@ __global__ __launch_bounds__(kFinishThreads) void block_finish_kernel(FinishArgs
 void BlockFinish::add_weight(const BlockWgradPlan &pl, const void *partial, void *grad) {
   WeightSums &w = weight[n_weights++];
   w = WeightSums{(const float *)partial, grad, pl.M, pl.C, pl.nfx, pl.nfy, pl.f_pitch, pl.f_off, pl.ctb, pl.wm * pl.mt * 32, pl.m_blocks,
-                 pl.c_blocks, 0, 0, 0, {}, {}};
+                 pl.c_blocks, 0, 0, 0, 0, {}, {}};
   for (int f = 0; f < pl.nfx; ++f) {
     w.slice0[f] = (unsigned short)pl.row[f].slice0;
     w.slices[f] = (unsigned short)pl.row[f].slices;
   }
-  w.taps = pl.slices < 16 * pl.nfx && pl.nfx * pl.nfy <= kFinishTaps && (i64)pl.M * pl.C >= 1 << 14;
-  w.blocks = w.taps ? (unsigned)(pl.M * ((pl.C + 31) / 32)) : (unsigned)(pl.nfx * pl.c_blocks * pl.ctb * pl.nfy * pl.M);
+  // as many taps to a block as its threads hold -- longer runs of weights -- and leave two blocks a CU, or four where a thread's
+  // share of the slices would be more than the eight loads that are on their way at a time (64 -> 64 channels, 5 x 3 taps, 100
+  // slices a filter row: 10.0 -> 9.2 us with four; 41 -> 128 channels, 8 taps, 8 slices: 4.6 -> 5.5)
+  const int taps = pl.nfx * pl.nfy;
+  const i64 tiles = (i64)pl.M * ((pl.C + 31) / 32);
+  w.tap_chunk = std::min(taps, kFinishThreads / 8);
+  auto few = [&](int chunk) {
+    const i64 blocks = tiles * ((taps + chunk - 1) / chunk);
+    return blocks < 512 || (blocks < 1024 && pl.slices > pl.nfx * 8 * (kFinishThreads / 8 / chunk));
+  };
+  while (w.tap_chunk > 1 && few(w.tap_chunk)) w.tap_chunk = (w.tap_chunk + 1) / 2;
+  w.parts = kFinishThreads / 8 / w.tap_chunk;
+  w.blocks = (unsigned)(tiles * ((taps + w.tap_chunk - 1) / w.tap_chunk));
   if (pl.nfy != pl.f_pitch) w.zero_blocks = (unsigned)(((i64)pl.M * pl.C * pl.nfx * pl.f_pitch + kFinishThreads - 1) / kFinishThreads);
 }
 

@@ -163,7 +163,7 @@ struct WeightSums {                // a weight gradient from its partial blocks
   const float *partial;
   void *grad;
   int M, C, nfx, nfy, f_pitch, f_off, ctb, m_t, m_blocks, c_blocks;    // (m_t: output channels of a block)
-  int taps;                        // a block of threads takes all taps of its weights
+  int tap_chunk, parts;            // taps of a block of threads; parts that the slices are added in
   unsigned blocks, zero_blocks;    // blocks of threads; of those for columns without a tap
   unsigned short slice0[kBlockFilterRows], slices[kBlockFilterRows];
 };

@@ -698,7 +698,7 @@ int corr2d_backward_input(const char *fn, int kind_x, const T *weight,
                           i64 nfx, i64 nfy, i64 ngx, i64 ngy, i64 nhx, i64 nhy,
                           i64 sx, i64 sy, i64 dx, i64 dy, i64 px, i64 py, i64 ux,
                           i64 uy, T *grad_input, void *workspace, size_t workspace_bytes,
-                          void *stream, void *half_out = nullptr, bool *wrote_half = nullptr) {
+                          void *stream, void *half_out = nullptr, bool *wrote_half = nullptr, WgradReduce *beside = nullptr) {
   if (wrote_half) *wrote_half = false;
   int rc = check_corr2d(fn, kind_x, batch, c_in, c_out, nfx, nfy, ngx, ngy, nhx,
                         nhy, sx, sy, dx, dy, px, py, ux, uy);
@@ -719,7 +719,7 @@ int corr2d_backward_input(const char *fn, int kind_x, const T *weight,
       g_variant = "mfma-fused";
       g_last_math = ips.fused.stream ? MATH_BF16X3 : MATH_FP32;
       return check_hip(launch_igrad(ips.fused, (const float *)weight, (const float *)grad_out,
-                                    (float *)grad_input, (float *)workspace, (hipStream_t)stream), fn);
+                                    (float *)grad_input, (float *)workspace, (hipStream_t)stream, beside), fn);
     }
     if (which == IN_TAPS) {
       // tap products through the workspace, then a gather (any x axis kind)
@@ -731,10 +731,10 @@ int corr2d_backward_input(const char *fn, int kind_x, const T *weight,
         const Axis fx = make_axis(conv_x, nfx, nhx, ngx, ux, dx, px, sx);
         const Axis fy = make_axis(AX_LCONV, nfy, nhy, ngy, uy, dy, py, sy);
         if (ips.taps.yfold)                                  // (the kernel has summed the filter columns)
-          e = launch_fold_x(fx, batch * c_in, ngx, ngy, (const float *)workspace, grad_input, (hipStream_t)stream);
+          e = launch_fold_x(fx, batch * c_in, ngx, ngy, (const float *)workspace, grad_input, (hipStream_t)stream, false, beside);
         else
           e = launch_fold_xy(fx, fy, batch * c_in, ips.taps.nf_pad, (const float *)workspace,
-                             (float *)grad_input, (hipStream_t)stream);
+                             (float *)grad_input, (hipStream_t)stream, beside);
       }
       return check_hip(e, fn);
     }
@@ -745,7 +745,7 @@ int corr2d_backward_input(const char *fn, int kind_x, const T *weight,
       hipError_t e = launch_first_pass(tp, weight, grad_out, workspace, 4, (hipStream_t)stream);
       if (e == hipSuccess)
         e = launch_fold_x(tp.fold, batch * c_in, ngx, ngy, (const float *)workspace,
-                          (float *)grad_input, (hipStream_t)stream);
+                          (float *)grad_input, (hipStream_t)stream, false, beside);
       return check_hip(e, fn);
     }
   }
@@ -786,7 +786,8 @@ int corr2d_backward_weight(const char *fn, int kind_x, const T *input,
                            i64 nfx, i64 nfy, i64 ngx, i64 ngy, i64 nhx, i64 nhy,
                            i64 sx, i64 sy, i64 dx, i64 dy, i64 px, i64 py, i64 ux,
                            i64 uy, T *grad_weight, void *workspace,
-                           size_t workspace_bytes, void *stream, float *bias_ws = nullptr, float *grad_bias = nullptr) {
+                           size_t workspace_bytes, void *stream, float *bias_ws = nullptr, float *grad_bias = nullptr,
+                           WgradReduce *later = nullptr) {
   int rc = check_corr2d(fn, kind_x, batch, c_in, c_out, nfx, nfy, ngx, ngy, nhx,
                         nhy, sx, sy, dx, dy, px, py, ux, uy);
   if (rc) return rc;
@@ -817,7 +818,7 @@ int corr2d_backward_weight(const char *fn, int kind_x, const T *input,
       g_last_math = wp.rows_mode == 2 ? MATH_BF16X3 : MATH_FP32;
       return check_hip(launch_wgrad(wp, (const float *)grad_out, (const float *)input,
                                     (float *)grad_weight, (float *)workspace,
-                                    (hipStream_t)stream, bias_ws, grad_bias), fn);
+                                    (hipStream_t)stream, bias_ws, grad_bias, later), fn);
     }
   }
   SepReduce pr;
@@ -1872,7 +1873,7 @@ struct LayerBackward {
   bool input_blocked, weight_blocked, plain;           // plain: some gradient takes the section-2 kernels
   bool bias_beside;                                    // section 2's weight gradient makes the bias gradient as well
   bool bias_packed;                                    // the pass that blocks grad_out adds it up
-  size_t masked_off, go_off, x_off, frag_off, slice_off, bias_off, wgrad_off, gw_off, gb_off, beside_off, pass_off, pass_bytes, total;
+  size_t masked_off, go_off, x_off, frag_off, slice_off, bias_off, wgrad_off, gw_off, gb_off, beside_off, pass_off, pass_bytes, weight_off, weight_bytes, total;
   BlockPlan bp;
   BlockWgradPlan wp;
 };
@@ -1911,11 +1912,14 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
   if (wi && !lb.input_blocked)
     pass = std::max(pass, half ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS)
                                : mellin_corr2d_backward_input_workspace(kind_x, elem, CORR2D_ARGS));
-  if (ww && !lb.weight_blocked)
-    pass = std::max(pass, half ? mellin_corr2d_backward_weight_f16_workspace(kind_x, CORR2D_ARGS)
-                               : mellin_corr2d_backward_weight_workspace(kind_x, elem, CORR2D_ARGS));
+  // (float: beside the input gradient's, whose last launch also ends the weight gradient)
+  lb.weight_bytes = !ww || lb.weight_blocked ? 0 : half ? mellin_corr2d_backward_weight_f16_workspace(kind_x, CORR2D_ARGS)
+                                                        : mellin_corr2d_backward_weight_workspace(kind_x, elem, CORR2D_ARGS);
+  const bool together = !half && wi && !lb.input_blocked && lb.weight_bytes > 0;
+  if (!together) pass = std::max(pass, lb.weight_bytes);
   lb.pass_bytes = pass;
   lb.pass_off = take(pass);
+  lb.weight_off = together ? take(lb.weight_bytes) : lb.pass_off;
   lb.total = at;
 }
 // The images that the input gradient takes at a time; less than `batch`: in calls of their own (INPUT_ONLY), beside one for
@@ -1991,20 +1995,32 @@ int mellin_layer_backward_kept(int kind_x, int elem_bytes, int want, const void 
     if (rc) return rc;
     if (masked) grad_out = masked;
   }
-  if ((want & MELLIN_WANT_INPUT) && !lb.input_blocked) {
-    rc = half ? mellin_corr2d_backward_input_f16(kind_x, weight, grad_out, CORR2D_ARGS, grad_input, pass, lb.pass_bytes, stream)
-              : mellin_corr2d_backward_input_f32(kind_x, (const float *)weight, (const float *)grad_out, CORR2D_ARGS,
-                                                 (float *)grad_input, pass, lb.pass_bytes, stream);
-    if (rc) return rc;
-  }
+  // The weight gradient first: the sums that end it are left to the input gradient's last launch, whose blocks wait for memory
+  // as they do (8 x 4 taps, 3 -> 64 channels, 32 x 512 x 41, us a step: Mellin rows 74.1 -> 69.8, linear ones within the noise).
+  WgradReduce sums_later = {};
   if ((want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked) {
-    rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, wide ? ws + lb.gw_off : grad_weight, pass,
-                                                  lb.pass_bytes, stream)
+    const bool leave = lb.weight_off != lb.pass_off;
+    rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, wide ? ws + lb.gw_off : grad_weight,
+                                                  ws + lb.weight_off, lb.weight_bytes, stream)
               : corr2d_backward_weight<float>(__func__, kind_x, (const float *)input, (const float *)grad_out, CORR2D_ARGS,
-                                              (float *)grad_weight, pass, lb.pass_bytes, stream,
-                                              lb.bias_beside ? (float *)(ws + lb.beside_off) : nullptr, (float *)grad_bias);
+                                              (float *)grad_weight, ws + lb.weight_off, lb.weight_bytes, stream,
+                                              lb.bias_beside ? (float *)(ws + lb.beside_off) : nullptr, (float *)grad_bias,
+                                              leave ? &sums_later : nullptr);
     if (rc) return rc;
   }
+  if ((want & MELLIN_WANT_INPUT) && !lb.input_blocked) {
+    const char *const variant = g_variant;             // (the weight gradient's is the one that a step reports)
+    const int math = g_last_math;
+    rc = half ? mellin_corr2d_backward_input_f16(kind_x, weight, grad_out, CORR2D_ARGS, grad_input, pass, lb.pass_bytes, stream)
+              : corr2d_backward_input<float>(__func__, kind_x, (const float *)weight, (const float *)grad_out, CORR2D_ARGS,
+                                             (float *)grad_input, pass, lb.pass_bytes, stream, nullptr, nullptr, &sums_later);
+    if (rc) return rc;
+    if ((want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked) {
+      g_variant = variant;
+      g_last_math = math;
+    }
+  }
+  if (sums_later.blocks > 0 && (e = launch_wgrad_reduce(sums_later, st)) != hipSuccess) return check_hip(e, __func__);
   if (wide) {
     const bool gw = (want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked, gb = bias_here;
     e = launch_cast_pair(false, gw ? ws + lb.gw_off : nullptr, grad_weight, c_out * c_in * nfx * nfy, gb ? ws + lb.gb_off : nullptr,

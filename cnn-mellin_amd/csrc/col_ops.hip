@@ -19,6 +19,7 @@
 #include <algorithm>
 
 #include "mellin_common.hpp"
+#include "wgrad_reduce.hpp"
 
 namespace mellin {
 
@@ -122,16 +123,22 @@ template <typename T, typename O = T>
 __global__ __launch_bounds__(256) void col2spec_plane_kernel(const T *__restrict__ gg, O *__restrict__ g,
                                                              Axis x, Axis y, int c_in, int batch,
                                                              int transposed_g, int transposed_gg,
-                                                             i64 per_pair) {   // words from one pair's columns to the next
+                                                             i64 per_pair,     // words from one pair's columns to the next
+                                                             unsigned blocks_x, unsigned blocks_z, WgradReduce beside) {
+  // the sums that end the weight gradient beside this one, if any, come first: their chains of loads are the longer ones
+  if (blockIdx.x < (unsigned)beside.blocks) {
+    wgrad_reduce_block(beside, blockIdx.x);
+    return;
+  }
   constexpr int NB = 8, FY = 4;
   const int plane = (int)(x.nh * y.nh), nfx = (int)x.nf, nfy = (int)y.nf;
   // Workgroups are dealt to the eight dies in turn, each with an L2 of its own: renumber them so
   // that a die takes one contiguous run of (pair group, 256-position block), whose neighbouring
   // rows of gg share cache lines.
-  const unsigned total = gridDim.x * gridDim.z, lin = blockIdx.x + gridDim.x * blockIdx.z;
+  const unsigned total = blocks_x * blocks_z, lin = blockIdx.x - beside.blocks;
   const unsigned die = lin & 7u, slot = lin >> 3;
   const unsigned mine = die * (total >> 3) + min(die, total & 7u) + slot;
-  const unsigned block_z = mine / gridDim.x, block_x = mine - block_z * gridDim.x;
+  const unsigned block_z = mine / blocks_x, block_x = mine - block_z * blocks_x;
   const int q = (int)block_x * 256 + threadIdx.x;
   if (q >= plane) return;
   int gx = (int)((float)q * (1.0f / (float)y.nh));
@@ -145,7 +152,7 @@ __global__ __launch_bounds__(256) void col2spec_plane_kernel(const T *__restrict
   int oy_first[FY];
   y_taps(0, oy_first);
   const int pairs = batch * c_in;
-  for (int nc0 = (int)block_z * NB; nc0 < pairs; nc0 += gridDim.z * NB) {   // nc: pairs in g's own order
+  for (int nc0 = (int)block_z * NB; nc0 < pairs; nc0 += blocks_z * NB) {   // nc: pairs in g's own order
     const T *src[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -219,6 +226,16 @@ bool fits_plane_kernels(const Axis &x, const Axis &y, i64 c_in, i64 batch, i64 p
          batch * c_in < ((i64)1 << 30) && x.nf * y.nf <= 65535 && x.ng * y.ng < ((i64)1 << 31);
 }
 
+// what a launch makes beside its own work
+WgradReduce take_beside(WgradReduce *beside) {
+  WgradReduce r = {};
+  if (beside) {
+    r = *beside;
+    beside->blocks = 0;
+  }
+  return r;
+}
+
 unsigned blocks_for(i64 total) {
   i64 b = (total + 255) / 256;
   if (b > (1 << 20)) b = 1 << 20;
@@ -248,15 +265,16 @@ hipError_t launch_spec2col(const Axis &x, const Axis &y, i64 c_in, i64 batch, in
 
 template <typename T, typename O>
 hipError_t launch_col2spec(const Axis &x, const Axis &y, i64 c_in, i64 batch, int transposed_g,
-                           int transposed_gg, const T *gg, O *g, hipStream_t stream) {
+                           int transposed_gg, const T *gg, O *g, hipStream_t stream, WgradReduce *beside) {
   const i64 total = batch * c_in * x.nh * y.nh;
   if (total == 0) return hipSuccess;
   const i64 plane = x.nh * y.nh;
   if (fits_plane_kernels(x, y, c_in, batch, plane, x.nf * y.nf * x.ng * y.ng)) {
     const i64 gx = (plane + 255) / 256, groups = (batch * c_in + 7) / 8;
     const i64 gz = std::max<i64>(1, std::min<i64>(groups, std::min<i64>(65535, (8192 + gx - 1) / gx)));
-    hipLaunchKernelGGL((col2spec_plane_kernel<T, O>), dim3((unsigned)gx, 1, (unsigned)gz), dim3(256), 0, stream, gg,
-                       g, x, y, (int)c_in, (int)batch, transposed_g, transposed_gg, x.nf * y.nf * x.ng * y.ng);
+    const WgradReduce first = take_beside(beside);
+    hipLaunchKernelGGL((col2spec_plane_kernel<T, O>), dim3((unsigned)(gx * gz + first.blocks)), dim3(256), 0, stream, gg,
+                       g, x, y, (int)c_in, (int)batch, transposed_g, transposed_gg, x.nf * y.nf * x.ng * y.ng, (unsigned)gx, (unsigned)gz, first);
     return hipGetLastError();
   }
   hipLaunchKernelGGL((col2spec_kernel<T, O>), dim3(blocks_for(total)), dim3(256), 0, stream, gg, g, x, y, c_in,
@@ -267,13 +285,14 @@ hipError_t launch_col2spec(const Axis &x, const Axis &y, i64 c_in, i64 batch, in
 // The same adjoint over columns whose tap planes are padded to `taps_padded` per pair
 // (the tap products of the input gradient); false if the plane kernel's range is exceeded.
 bool launch_col2spec_padded(const Axis &x, const Axis &y, i64 pairs, i64 taps_padded, const float *gg,
-                            float *g, hipStream_t stream, hipError_t *err) {
+                            float *g, hipStream_t stream, hipError_t *err, WgradReduce *beside) {
   const i64 plane = x.nh * y.nh, per_pair = taps_padded * x.ng * y.ng;
   if (!fits_plane_kernels(x, y, pairs, 1, plane, per_pair)) return false;
   const i64 gx = (plane + 255) / 256, groups = (pairs + 7) / 8;
   const i64 gz = std::max<i64>(1, std::min<i64>(groups, std::min<i64>(65535, (8192 + gx - 1) / gx)));
-  hipLaunchKernelGGL(col2spec_plane_kernel<float>, dim3((unsigned)gx, 1, (unsigned)gz), dim3(256), 0, stream, gg,
-                     g, x, y, (int)pairs, 1, 0, 0, per_pair);
+  const WgradReduce first = take_beside(beside);
+  hipLaunchKernelGGL(col2spec_plane_kernel<float>, dim3((unsigned)(gx * gz + first.blocks)), dim3(256), 0, stream, gg,
+                     g, x, y, (int)pairs, 1, 0, 0, per_pair, (unsigned)gx, (unsigned)gz, first);
   *err = hipGetLastError();
   return true;
 }
@@ -283,10 +302,10 @@ template hipError_t launch_spec2col<float>(const Axis &, const Axis &, i64, i64,
 template hipError_t launch_spec2col<double>(const Axis &, const Axis &, i64, i64, int, int, const double *,
                                             double *, hipStream_t);
 template hipError_t launch_col2spec<float, float>(const Axis &, const Axis &, i64, i64, int, int, const float *,
-                                                  float *, hipStream_t);
+                                                  float *, hipStream_t, WgradReduce *);
 template hipError_t launch_col2spec<float, _Float16>(const Axis &, const Axis &, i64, i64, int, int, const float *,
-                                                     _Float16 *, hipStream_t);
+                                                     _Float16 *, hipStream_t, WgradReduce *);
 template hipError_t launch_col2spec<double, double>(const Axis &, const Axis &, i64, i64, int, int, const double *,
-                                                    double *, hipStream_t);
+                                                    double *, hipStream_t, WgradReduce *);
 
 }  // namespace mellin

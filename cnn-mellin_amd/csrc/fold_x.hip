@@ -92,14 +92,14 @@ __global__ __launch_bounds__(256) void fold_xy_kernel(Axis x, Axis y, i64 batch_
 }  // namespace
 
 hipError_t launch_fold_xy(const Axis &x, const Axis &y, i64 batch_cin, int nf_pad, const float *Z,
-                          float *grad_input, hipStream_t stream) {
+                          float *grad_input, hipStream_t stream, WgradReduce *beside) {
   const i64 total = batch_cin * x.nh * y.nh;
   if (total == 0) return hipSuccess;
   {
     // the column-to-signal adjoint over padded tap planes: a thread works out a
     // position's taps once for eight (image, channel) pairs
     hipError_t e = hipSuccess;
-    if (launch_col2spec_padded(x, y, batch_cin, nf_pad, Z, grad_input, stream, &e)) return e;
+    if (launch_col2spec_padded(x, y, batch_cin, nf_pad, Z, grad_input, stream, &e, beside)) return e;
   }
   i64 blocks = (total + 255) / 256;
   if (blocks > (1 << 20)) blocks = 1 << 20;
@@ -115,13 +115,13 @@ hipError_t launch_fold_xy(const Axis &x, const Axis &y, i64 batch_cin, int nf_pa
 }
 
 hipError_t launch_fold_x(const Axis &x, i64 batch_cin, i64 ngx, i64 ngy, const float *Y,
-                         void *grad_input, hipStream_t stream, bool half_out) {
+                         void *grad_input, hipStream_t stream, bool half_out, WgradReduce *beside) {
   // x: convolution-kind axis with nf = nfx, ng = nhx (rows of Y), nh = ngx (rows of grad_input);
   // Y is (batch_cin, nfx, 1, nhx, ngy): columns with an identity y axis
   (void)ngx;
   const Axis y = make_axis(AX_LCONV, 1, ngy, ngy, 1, 1, 0, 1);
   if (half_out) return launch_col2spec<float, _Float16>(x, y, batch_cin, 1, 0, 0, Y, (_Float16 *)grad_input, stream);
-  return launch_col2spec<float, float>(x, y, batch_cin, 1, 0, 0, Y, (float *)grad_input, stream);
+  return launch_col2spec<float, float>(x, y, batch_cin, 1, 0, 0, Y, (float *)grad_input, stream, beside);
 }
 
 }  // namespace mellin

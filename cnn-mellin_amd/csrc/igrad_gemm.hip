@@ -37,6 +37,7 @@
 
 #include "igrad_gemm.hpp"
 #include "tile_stage.hpp"
+#include "wgrad_reduce.hpp"
 
 namespace mellin {
 
@@ -406,9 +407,15 @@ __global__ __launch_bounds__((KSTEPS * NT <= 128 ? 768 : 512)) void igrad_kernel
 template <typename O>                                  // O: float, or _Float16 (the sum rounded once)
 __global__ __launch_bounds__(256) void igrad_combine_kernel(const IgradPlan pl,
                                                             const float *__restrict__ WS,
-                                                            O *__restrict__ GI) {
-  const int b = blockIdx.x + 1;                        // boundary between strips b - 1 and b
-  const i64 nc = blockIdx.y;
+                                                            O *__restrict__ GI, WgradReduce beside) {
+  // (the sums that end the weight gradient beside this one, if any, come first)
+  if (blockIdx.x < (unsigned)beside.blocks) {
+    wgrad_reduce_block(beside, blockIdx.x);
+    return;
+  }
+  const unsigned lin = blockIdx.y * gridDim.x + blockIdx.x - beside.blocks;
+  const i64 nc = lin / (unsigned)(pl.strips - 1);
+  const int b = (int)(lin - (unsigned)nc * (pl.strips - 1)) + 1;      // boundary between strips b - 1 and b
   const int g_b = pl.sx * b * pl.Th - pl.px;           // first row the boundary can share
   const float *src = WS + ((nc * (pl.strips - 1) + (b - 1)) * pl.nshared * 2) * pl.ngy;
   O *out = GI + nc * pl.ngx * pl.ngy;
@@ -427,9 +434,23 @@ __global__ __launch_bounds__(256) void igrad_combine_kernel(const IgradPlan pl,
   }
 }
 
+template <typename O>
+hipError_t launch_combine(const IgradPlan &pl, const float *ws, O *gi, hipStream_t stream, WgradReduce *beside) {
+  WgradReduce first = {};
+  dim3 grid((unsigned)(pl.strips - 1), (unsigned)(pl.batch * pl.c_in));
+  const i64 blocks = (i64)grid.x * grid.y + (beside ? beside->blocks : 0);
+  if (beside && blocks < (i64)1 << 23) {               // (a grid has less than 2^32 threads along x)
+    first = *beside;
+    beside->blocks = 0;
+    grid = dim3((unsigned)blocks);
+  }
+  hipLaunchKernelGGL(igrad_combine_kernel<O>, grid, dim3(256), 0, stream, pl, ws, gi, first);
+  return hipGetLastError();
+}
+
 template <int KSTEPS, int NT, bool PIPE>
 hipError_t launch_instance(const IgradPlan &pl, const float *w, const float *go, float *gi,
-                           float *ws, hipStream_t stream) {
+                           float *ws, hipStream_t stream, WgradReduce *beside) {
   auto kern = igrad_kernel<KSTEPS, NT, PIPE>;
   {
     static std::atomic<int> lds_allowed{0};                // (one per kernel instance)
@@ -441,10 +462,7 @@ hipError_t launch_instance(const IgradPlan &pl, const float *w, const float *go,
                      pl.lds_bytes, stream, pl, w, go, gi, ws);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || pl.ws_bytes == 0) return e;
-  hipLaunchKernelGGL(igrad_combine_kernel<float>,
-                     dim3((unsigned)(pl.strips - 1), (unsigned)(pl.batch * pl.c_in)), dim3(256), 0,
-                     stream, pl, ws, gi);
-  return hipGetLastError();
+  return launch_combine(pl, ws, gi, stream, beside);
 }
 
 // The same input gradient on the bf16 matrix cores (tile_stage.hpp: every fp32 operand as
@@ -848,7 +866,7 @@ __global__ __launch_bounds__(256, 2) void igrad_stream_kernel(const IgradPlan pl
 
 template <int MTT, int NT, bool F16 = false>
 hipError_t launch_stream_instance(const IgradPlan &pl, const void *w, const void *go, void *gi,
-                                  float *ws, hipStream_t stream) {
+                                  float *ws, hipStream_t stream, WgradReduce *beside = nullptr) {
   auto kern = igrad_stream_kernel<MTT, NT, F16>;
   {
     static std::atomic<int> lds_allowed{0};                // (one per kernel instance)
@@ -859,13 +877,8 @@ hipError_t launch_stream_instance(const IgradPlan &pl, const void *w, const void
                      ws);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || pl.ws_bytes == 0) return e;
-  const dim3 cgrid((unsigned)(pl.strips - 1), (unsigned)(pl.batch * pl.c_in));
-  if (F16)
-    hipLaunchKernelGGL(igrad_combine_kernel<_Float16>, cgrid, dim3(256), 0, stream, pl, (const float *)ws,
-                       (_Float16 *)gi);
-  else
-    hipLaunchKernelGGL(igrad_combine_kernel<float>, cgrid, dim3(256), 0, stream, pl, (const float *)ws, (float *)gi);
-  return hipGetLastError();
+  if (F16) return launch_combine(pl, ws, (_Float16 *)gi, stream, beside);
+  return launch_combine(pl, ws, (float *)gi, stream, beside);
 }
 
 // Tap products for the gather-fold input gradient (any x axis kind):
@@ -1246,18 +1259,18 @@ hipError_t launch_igrad_half(const IgradPlan &pl, const void *weight, const void
 }
 
 hipError_t launch_igrad(const IgradPlan &pl, const float *weight, const float *grad_out,
-                        float *grad_input, float *workspace, hipStream_t stream) {
+                        float *grad_input, float *workspace, hipStream_t stream, WgradReduce *beside) {
   if (pl.stream) {
-    if (pl.c_in == 1) return launch_stream_instance<1, 2>(pl, weight, grad_out, grad_input, workspace, stream);
-    if (pl.c_in == 2) return launch_stream_instance<2, 1>(pl, weight, grad_out, grad_input, workspace, stream);
-    return launch_stream_instance<3, 1>(pl, weight, grad_out, grad_input, workspace, stream);
+    if (pl.c_in == 1) return launch_stream_instance<1, 2>(pl, weight, grad_out, grad_input, workspace, stream, beside);
+    if (pl.c_in == 2) return launch_stream_instance<2, 1>(pl, weight, grad_out, grad_input, workspace, stream, beside);
+    return launch_stream_instance<3, 1>(pl, weight, grad_out, grad_input, workspace, stream, beside);
   }
   // the pipelined fold needs batches that cannot collide and no padded matrix rows
   const bool pipe = pl.pipe && pl.nt == 2;
 #define MELLIN_IGRAD_CASE(KS, NT_)                                                       \
   if (pl.ksteps == KS && pl.nt == NT_)                                                   \
-    return pipe ? launch_instance<KS, NT_, (NT_ == 2)>(pl, weight, grad_out, grad_input, workspace, stream) \
-                : launch_instance<KS, NT_, false>(pl, weight, grad_out, grad_input, workspace, stream);
+    return pipe ? launch_instance<KS, NT_, (NT_ == 2)>(pl, weight, grad_out, grad_input, workspace, stream, beside) \
+                : launch_instance<KS, NT_, false>(pl, weight, grad_out, grad_input, workspace, stream, beside);
   MELLIN_IGRAD_CASE(16, 2) MELLIN_IGRAD_CASE(16, 4)
   MELLIN_IGRAD_CASE(32, 2) MELLIN_IGRAD_CASE(32, 4)
   MELLIN_IGRAD_CASE(64, 2) MELLIN_IGRAD_CASE(64, 4)

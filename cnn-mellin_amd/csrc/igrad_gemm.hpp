@@ -41,7 +41,7 @@ bool make_igrad_plan(int kind_x, i64 batch, i64 c_in, i64 c_out, i64 nfx, i64 nf
                      int math = MATH_FP32);
 
 hipError_t launch_igrad(const IgradPlan &pl, const float *weight, const float *grad_out,
-                        float *grad_input, float *workspace, hipStream_t stream);
+                        float *grad_input, float *workspace, hipStream_t stream, WgradReduce *beside = nullptr);
 
 // The `stream` form of a plan on half-precision tensors (f16 matrix cores; the workspace
 // keeps fp32 partial rows): weight, grad_out and grad_input are half-precision storage.

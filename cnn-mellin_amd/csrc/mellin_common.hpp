@@ -141,9 +141,20 @@ template <typename T>
 hipError_t launch_sepreduce_generic(const SepReduce &pr, const T *a, const T *g,
                                     T *w, hipStream_t stream);
 
+// The sums that end a weight gradient (wgrad_reduce.hpp), for a launch that can make them beside its own work.  Its taker sets
+// `blocks`, of 256 threads, to zero.
+struct WgradReduce {
+  const float *ws;
+  float *W;
+  int S, M, J, M_pad, J_pad;
+  const float *bias_ws;
+  float *gb;
+  int blocks;
+};
+
 // (half_out: grad_input is half-precision storage, each fp32 sum rounded once)
 hipError_t launch_fold_x(const Axis &x, i64 batch_cin, i64 ngx, i64 ngy, const float *Y,
-                         void *grad_input, hipStream_t stream, bool half_out = false);
+                         void *grad_input, hipStream_t stream, bool half_out = false, WgradReduce *beside = nullptr);
 
 template <typename T>
 hipError_t launch_spec2col(const Axis &x, const Axis &y, i64 c_in, i64 batch, int transposed_g,
@@ -151,13 +162,13 @@ hipError_t launch_spec2col(const Axis &x, const Axis &y, i64 c_in, i64 batch, in
 // (O: the type g is stored in; sums are formed in T)
 template <typename T, typename O = T>
 hipError_t launch_col2spec(const Axis &x, const Axis &y, i64 c_in, i64 batch, int transposed_g,
-                           int transposed_gg, const T *gg, O *g, hipStream_t stream);
+                           int transposed_gg, const T *gg, O *g, hipStream_t stream, WgradReduce *beside = nullptr);
 
 bool launch_col2spec_padded(const Axis &x, const Axis &y, i64 pairs, i64 taps_padded, const float *gg,
-                            float *g, hipStream_t stream, hipError_t *err);
+                            float *g, hipStream_t stream, hipError_t *err, WgradReduce *beside = nullptr);
 
 hipError_t launch_fold_xy(const Axis &x, const Axis &y, i64 batch_cin, int nf_pad, const float *Z,
-                          float *grad_input, hipStream_t stream);
+                          float *grad_input, hipStream_t stream, WgradReduce *beside = nullptr);
 
 // pointwise.hip: log compression and dilation lift over x viewed as (outer, t, inner).
 // eps_at, tau_at (device memory, or null): read by the kernels instead of the arguments; logs: their logarithms; kept (or

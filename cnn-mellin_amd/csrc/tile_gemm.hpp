@@ -122,9 +122,11 @@ bool make_wgrad_plan(const SepConv &fwd, WgradPlan &wp, bool allow_rows = true, 
                      int rows_nbuf = 0, int rows_rpw = 0);
 
 // With bias_ws (wgrad_bias_bytes(): its size, 0 where the kernel does not do it) the sums of grad_out go to grad_bias.
+// With `later` the sums that end it are left to the caller.
 size_t wgrad_bias_bytes(const WgradPlan &wp);
 hipError_t launch_wgrad(const WgradPlan &wp, const float *grad_out, const float *input, float *grad_weight, float *workspace,
-                        hipStream_t stream, float *bias_ws = nullptr, float *grad_bias = nullptr);
+                        hipStream_t stream, float *bias_ws = nullptr, float *grad_bias = nullptr, WgradReduce *later = nullptr);
+hipError_t launch_wgrad_reduce(const WgradReduce &r, hipStream_t stream);
 
 // wgrad_gemm.hip: W[m, j] = the sum of `partials` blocks of (M_pad x J_pad) floats, in index order;
 // W is float storage, or half-precision storage (rounded once) when half_out

@@ -25,6 +25,7 @@
 #include "mellin_common.hpp"
 #include "tile_gemm.hpp"
 #include "tile_stage.hpp"
+#include "wgrad_reduce.hpp"
 
 namespace mellin {
 
@@ -867,45 +868,12 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 3 : 2)) void wgrad_stream_kern
   }
 }
 
-// W[m, j] = sum over the S partial blocks, in a fixed order.  A block of 256
-// threads handles 16 outputs: 16 threads per output add every 16th partial,
-// then thread 0 of each output adds the 16 sums in pairs.  Behind the M J weights
-// come, with bias_ws, the M sums of grad_out: gb[m] of the partial sums bias_ws[s, m].
 template <typename O>                                  // O: float, or _Float16 (rounded once)
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restrict__ ws,
                                                            O *__restrict__ W, int S, int M,
                                                            int J, int M_pad, int J_pad, const float *__restrict__ bias_ws,
                                                            O *__restrict__ gb) {
-  __shared__ float part[16][17];
-  const int el = threadIdx.x & 15, ph = threadIdx.x >> 4;
-  const int e = blockIdx.x * 16 + el, outputs = M * J + (bias_ws ? M : 0);
-  float sum = 0.f;
-  if (e < outputs) {
-    const int m = e / J, j = e - m * J;
-    const bool weight = e < M * J;
-    const float *src = weight ? ws + (i64)m * J_pad + j : bias_ws + (e - M * J);
-    const i64 stride = weight ? (i64)M_pad * J_pad : M_pad;
-    int s = ph;
-    for (; s + 48 < S; s += 64) {
-      const float v0 = src[(i64)s * stride], v1 = src[(i64)(s + 16) * stride];
-      const float v2 = src[(i64)(s + 32) * stride], v3 = src[(i64)(s + 48) * stride];
-      sum += (v0 + v1) + (v2 + v3);
-    }
-    for (; s < S; s += 16) sum += src[(i64)s * stride];
-  }
-  part[ph][el] = sum;
-  __syncthreads();
-  if (ph == 0 && e < outputs) {
-    float v[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) v[k] = part[k][el];
-#pragma unroll
-    for (int n = 8; n > 0; n >>= 1)
-#pragma unroll
-      for (int k = 0; k < n; ++k) v[k] += v[k + n];
-    const float tot = v[0];
-    (e < M * J ? W[e] : gb[e - M * J]) = (O)tot;
-  }
+  wgrad_reduce_block<O>(ws, W, S, M, J, M_pad, J_pad, bias_ws, gb, blockIdx.x);
 }
 
 template <int MT, int JT, int NT>
@@ -1131,7 +1099,7 @@ size_t wgrad_bias_bytes(const WgradPlan &wp) {
 }
 
 hipError_t launch_wgrad(const WgradPlan &wp, const float *grad_out, const float *input,
-                        float *grad_weight, float *workspace, hipStream_t stream, float *bias_ws, float *grad_bias) {
+                        float *grad_weight, float *workspace, hipStream_t stream, float *bias_ws, float *grad_bias, WgradReduce *later) {
   dim3 grid((unsigned)wp.S, (unsigned)(wp.m_groups * wp.j_groups));
   hipError_t e = hipErrorInvalidValue;
   if (wp.rows_mode == 2) {
@@ -1161,8 +1129,17 @@ hipError_t launch_wgrad(const WgradPlan &wp, const float *grad_out, const float 
   }
   if (e != hipSuccess) return e;
   const int outputs = wp.t.M * wp.J + (bias_ws ? wp.t.M : 0);
-  hipLaunchKernelGGL(wgrad_reduce_kernel<float>, dim3((unsigned)((outputs + 15) / 16)), dim3(256), 0, stream,
-                     (const float *)workspace, grad_weight, wp.S, wp.t.M, wp.J, wp.M_pad, wp.J_pad, (const float *)bias_ws, grad_bias);
+  const WgradReduce r = {workspace, grad_weight, wp.S, wp.t.M, wp.J, wp.M_pad, wp.J_pad, bias_ws, grad_bias, (outputs + 15) / 16};
+  if (later) {
+    *later = r;
+    return hipSuccess;
+  }
+  return launch_wgrad_reduce(r, stream);
+}
+
+hipError_t launch_wgrad_reduce(const WgradReduce &r, hipStream_t stream) {
+  hipLaunchKernelGGL(wgrad_reduce_kernel<float>, dim3((unsigned)r.blocks), dim3(256), 0, stream, r.ws, r.W, r.S, r.M, r.J, r.M_pad, r.J_pad,
+                     r.bias_ws, r.gb);
   return hipGetLastError();
 }
 

@@ -692,13 +692,33 @@ int choose_input_plan(int kind_x, i64 batch, i64 c_in, i64 c_out, i64 nfx, i64 n
   return IN_GATHER;
 }
 
+// The launch that ends a float input gradient of several: the rows that strips share, or the fold of tap products.
+struct InputEnd {
+  int which;                                           // IN_FUSED, IN_TAPS, IN_TWO_PASS; IN_GATHER: none
+  bool over_x;                                         // the fold has no columns
+  IgradPlan fused;
+  Axis fx, fy;
+  i64 planes, ngx, ngy;
+  int nf_pad;
+  const float *workspace;
+  float *grad_input;
+};
+hipError_t launch_input_end(const InputEnd &end, hipStream_t stream, WgradReduce *beside) {
+  if (end.which == IN_GATHER) return hipSuccess;
+  if (end.which == IN_FUSED) return launch_igrad_end(end.fused, end.workspace, end.grad_input, stream, beside);
+  if (end.over_x) return launch_fold_x(end.fx, end.planes, end.ngx, end.ngy, end.workspace, end.grad_input, stream, false, beside);
+  return launch_fold_xy(end.fx, end.fy, end.planes, end.nf_pad, end.workspace, end.grad_input, stream, beside);
+}
+
+// (later: the launch that ends it is left to the caller)
 template <typename T>
 int corr2d_backward_input(const char *fn, int kind_x, const T *weight,
                           const T *grad_out, i64 batch, i64 c_in, i64 c_out,
                           i64 nfx, i64 nfy, i64 ngx, i64 ngy, i64 nhx, i64 nhy,
                           i64 sx, i64 sy, i64 dx, i64 dy, i64 px, i64 py, i64 ux,
                           i64 uy, T *grad_input, void *workspace, size_t workspace_bytes,
-                          void *stream, void *half_out = nullptr, bool *wrote_half = nullptr, WgradReduce *beside = nullptr) {
+                          void *stream, void *half_out = nullptr, bool *wrote_half = nullptr, InputEnd *later = nullptr) {
+  if (later) later->which = IN_GATHER;
   if (wrote_half) *wrote_half = false;
   int rc = check_corr2d(fn, kind_x, batch, c_in, c_out, nfx, nfy, ngx, ngy, nhx,
                         nhy, sx, sy, dx, dy, px, py, ux, uy);
@@ -715,37 +735,37 @@ int corr2d_backward_input(const char *fn, int kind_x, const T *weight,
     if (which != IN_GATHER && ips.ws_bytes && (!workspace || workspace_bytes < ips.ws_bytes))
       return fail(MELLIN_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", fn, ips.ws_bytes,
                   workspace_bytes);
+    InputEnd end = {};
+    end.which = which;
+    end.planes = batch * c_in; end.ngx = ngx; end.ngy = ngy;
+    end.workspace = (const float *)workspace;
+    end.grad_input = (float *)grad_input;
+    hipError_t e = hipSuccess;
     if (which == IN_FUSED) {
       g_variant = "mfma-fused";
       g_last_math = ips.fused.stream ? MATH_BF16X3 : MATH_FP32;
-      return check_hip(launch_igrad(ips.fused, (const float *)weight, (const float *)grad_out,
-                                    (float *)grad_input, (float *)workspace, (hipStream_t)stream, beside), fn);
-    }
-    if (which == IN_TAPS) {
+      end.fused = ips.fused;
+      e = launch_igrad(ips.fused, (const float *)weight, (const float *)grad_out, (float *)grad_input, (float *)workspace, (hipStream_t)stream);
+    } else if (which == IN_TAPS) {
       // tap products through the workspace, then a gather (any x axis kind)
       g_variant = "mfma-taps+fold";
       g_last_math = MATH_FP32;
-      hipError_t e = launch_tap_product(ips.taps, (const float *)weight, (const float *)grad_out,
-                                        (float *)workspace, (hipStream_t)stream);
-      if (e == hipSuccess) {
-        const Axis fx = make_axis(conv_x, nfx, nhx, ngx, ux, dx, px, sx);
-        const Axis fy = make_axis(AX_LCONV, nfy, nhy, ngy, uy, dy, py, sy);
-        if (ips.taps.yfold)                                  // (the kernel has summed the filter columns)
-          e = launch_fold_x(fx, batch * c_in, ngx, ngy, (const float *)workspace, grad_input, (hipStream_t)stream, false, beside);
-        else
-          e = launch_fold_xy(fx, fy, batch * c_in, ips.taps.nf_pad, (const float *)workspace,
-                             (float *)grad_input, (hipStream_t)stream, beside);
-      }
-      return check_hip(e, fn);
-    }
-    if (which == IN_TWO_PASS) {
+      end.fx = make_axis(conv_x, nfx, nhx, ngx, ux, dx, px, sx);
+      end.fy = make_axis(AX_LCONV, nfy, nhy, ngy, uy, dy, py, sy);
+      end.over_x = ips.taps.yfold;                           // (the kernel has summed the filter columns)
+      end.nf_pad = ips.taps.nf_pad;
+      e = launch_tap_product(ips.taps, (const float *)weight, (const float *)grad_out, (float *)workspace, (hipStream_t)stream);
+    } else if (which == IN_TWO_PASS) {
       const TwoPassInput &tp = ips.two;
       g_variant = tp.rows ? "mfma-filter-rows+fold" : "mfma+fold";
       g_last_math = tp.rows || tp.plan.split ? MATH_BF16X3 : MATH_FP32;
-      hipError_t e = launch_first_pass(tp, weight, grad_out, workspace, 4, (hipStream_t)stream);
-      if (e == hipSuccess)
-        e = launch_fold_x(tp.fold, batch * c_in, ngx, ngy, (const float *)workspace,
-                          (float *)grad_input, (hipStream_t)stream, false, beside);
+      end.fx = tp.fold;
+      end.over_x = true;
+      e = launch_first_pass(tp, weight, grad_out, workspace, 4, (hipStream_t)stream);
+    }
+    if (which != IN_GATHER) {
+      if (later) *later = end;
+      else if (e == hipSuccess) e = launch_input_end(end, (hipStream_t)stream, nullptr);
       return check_hip(e, fn);
     }
   }
@@ -1529,14 +1549,19 @@ int mellin_corr2d_forward_ws_f32(int kind_x, int activation, const float *input,
   return corr2d_forward<float>(__func__, kind_x, input, weight, bias, CORR2D_ARGS, out, stream, activation, nullptr,
                                nullptr, workspace, workspace_bytes);
 }
-size_t mellin_corr2d_backward_input_workspace(int kind_x, int elem_bytes,
-                                              MELLIN_CORR2D_DIMS) {
-  if (elem_bytes != 4 || g_forced == 1) return 0;
-  if (check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
+// (which: the InputForm of a float layer)
+static size_t input_workspace(int kind_x, MELLIN_CORR2D_DIMS, int *which) {
+  *which = IN_GATHER;
+  if (g_forced == 1 || check_corr2d("mellin_corr2d_backward_input_workspace", kind_x, CORR2D_ARGS)) return 0;
   if (!batch || !c_in || !c_out || !nfx || !nfy || !ngx || !ngy || !nhx || !nhy) return 0;
   InputPlans ips;
-  choose_input_plan(kind_x, CORR2D_ARGS, ips);
+  *which = choose_input_plan(kind_x, CORR2D_ARGS, ips);
   return ips.ws_bytes;
+}
+size_t mellin_corr2d_backward_input_workspace(int kind_x, int elem_bytes,
+                                              MELLIN_CORR2D_DIMS) {
+  int which;
+  return elem_bytes == 4 ? input_workspace(kind_x, CORR2D_ARGS, &which) : 0;
 }
 int mellin_corr2d_backward_input_f32(int kind_x, const float *weight,
                                      const float *grad_out, MELLIN_CORR2D_DIMS,
@@ -1874,6 +1899,7 @@ struct LayerBackward {
   bool bias_beside;                                    // section 2's weight gradient makes the bias gradient as well
   bool bias_packed;                                    // the pass that blocks grad_out adds it up
   size_t masked_off, go_off, x_off, frag_off, slice_off, bias_off, wgrad_off, gw_off, gb_off, beside_off, pass_off, pass_bytes, weight_off, weight_bytes, total;
+  bool weight_first;                                   // of two gradients by section 2's kernels
   BlockPlan bp;
   BlockWgradPlan wp;
 };
@@ -1909,9 +1935,10 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
   const int want_pass = want & (MELLIN_WANT_RELU | (lb.bias_beside || lb.bias_packed ? 0 : MELLIN_WANT_BIAS));
   if (lb.plain && want_pass)                           // (a ReLU's backward writes the bias gradient, asked for or not)
     pass = align256(mellin_bias_grad_workspace(batch, c_out, nhx * nhy)) + align256((size_t)c_out * elem);
+  int which = IN_GATHER;
   if (wi && !lb.input_blocked)
-    pass = std::max(pass, half ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS)
-                               : mellin_corr2d_backward_input_workspace(kind_x, elem, CORR2D_ARGS));
+    pass = std::max(pass, half ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS) : input_workspace(kind_x, CORR2D_ARGS, &which));
+  lb.weight_first = which == IN_TAPS || which == IN_TWO_PASS;
   // (float: beside the input gradient's, whose last launch also ends the weight gradient)
   lb.weight_bytes = !ww || lb.weight_blocked ? 0 : half ? mellin_corr2d_backward_weight_f16_workspace(kind_x, CORR2D_ARGS)
                                                         : mellin_corr2d_backward_weight_workspace(kind_x, elem, CORR2D_ARGS);
@@ -1995,32 +2022,44 @@ int mellin_layer_backward_kept(int kind_x, int elem_bytes, int want, const void 
     if (rc) return rc;
     if (masked) grad_out = masked;
   }
-  // The weight gradient first: the sums that end it are left to the input gradient's last launch, whose blocks wait for memory
-  // as they do (8 x 4 taps, 3 -> 64 channels, 32 x 512 x 41, us a step: Mellin rows 74.1 -> 69.8, linear ones within the noise).
+  // The launches that end a float layer's two gradients wait for memory and little else: they are one (8 x 4 taps, 3 -> 64
+  // channels, 32 x 512 x 41, us a step: Mellin rows 74.1 -> 69.8, linear ones 200.0 -> 197.0).  Tap products, which the last
+  // launch folds, are made behind the weight gradient, while caches still hold them; strips in front of it: grad_out is
+  // read from memory by whichever goes first, which costs the strips less (weight gradient 70 us behind them and 76 before).
+  const bool together = lb.weight_off != lb.pass_off;
+  InputEnd input_end = {};
+  input_end.which = IN_GATHER;
   WgradReduce sums_later = {};
-  if ((want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked) {
-    const bool leave = lb.weight_off != lb.pass_off;
-    rc = half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, wide ? ws + lb.gw_off : grad_weight,
-                                                  ws + lb.weight_off, lb.weight_bytes, stream)
-              : corr2d_backward_weight<float>(__func__, kind_x, (const float *)input, (const float *)grad_out, CORR2D_ARGS,
-                                              (float *)grad_weight, ws + lb.weight_off, lb.weight_bytes, stream,
-                                              lb.bias_beside ? (float *)(ws + lb.beside_off) : nullptr, (float *)grad_bias,
-                                              leave ? &sums_later : nullptr);
-    if (rc) return rc;
+  auto plain_input = [&]() -> int {
+    if (!(want & MELLIN_WANT_INPUT) || lb.input_blocked) return MELLIN_OK;
+    return half ? mellin_corr2d_backward_input_f16(kind_x, weight, grad_out, CORR2D_ARGS, grad_input, pass, lb.pass_bytes, stream)
+                : corr2d_backward_input<float>("mellin_layer_backward", kind_x, (const float *)weight, (const float *)grad_out, CORR2D_ARGS,
+                                               (float *)grad_input, pass, lb.pass_bytes, stream, nullptr, nullptr,
+                                               together ? &input_end : nullptr);
+  };
+  auto plain_weight = [&]() -> int {
+    if (!(want & MELLIN_WANT_WEIGHT) || lb.weight_blocked) return MELLIN_OK;
+    return half ? mellin_corr2d_backward_weight_f16(kind_x, input, grad_out, CORR2D_ARGS, wide ? ws + lb.gw_off : grad_weight,
+                                                    ws + lb.weight_off, lb.weight_bytes, stream)
+                : corr2d_backward_weight<float>("mellin_layer_backward", kind_x, (const float *)input, (const float *)grad_out, CORR2D_ARGS,
+                                                (float *)grad_weight, ws + lb.weight_off, lb.weight_bytes, stream,
+                                                lb.bias_beside ? (float *)(ws + lb.beside_off) : nullptr, (float *)grad_bias,
+                                                together ? &sums_later : nullptr);
+  };
+  const bool weight_first = together && lb.weight_first;
+  if ((rc = weight_first ? plain_weight() : plain_input())) return rc;
+  const char *const variant = g_variant;               // (a step reports the weight gradient's)
+  const int math = g_last_math;
+  if ((rc = weight_first ? plain_input() : plain_weight())) return rc;
+  if (weight_first) {
+    g_variant = variant;
+    g_last_math = math;
   }
-  if ((want & MELLIN_WANT_INPUT) && !lb.input_blocked) {
-    const char *const variant = g_variant;             // (the weight gradient's is the one that a step reports)
-    const int math = g_last_math;
-    rc = half ? mellin_corr2d_backward_input_f16(kind_x, weight, grad_out, CORR2D_ARGS, grad_input, pass, lb.pass_bytes, stream)
-              : corr2d_backward_input<float>(__func__, kind_x, (const float *)weight, (const float *)grad_out, CORR2D_ARGS,
-                                             (float *)grad_input, pass, lb.pass_bytes, stream, nullptr, nullptr, &sums_later);
-    if (rc) return rc;
-    if ((want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked) {
-      g_variant = variant;
-      g_last_math = math;
-    }
+  if (together) {
+    e = launch_input_end(input_end, st, &sums_later);
+    if (e == hipSuccess && sums_later.blocks > 0) e = launch_wgrad_reduce(sums_later, st);
+    if (e != hipSuccess) return check_hip(e, __func__);
   }
-  if (sums_later.blocks > 0 && (e = launch_wgrad_reduce(sums_later, st)) != hipSuccess) return check_hip(e, __func__);
   if (wide) {
     const bool gw = (want & MELLIN_WANT_WEIGHT) && !lb.weight_blocked, gb = bias_here;
     e = launch_cast_pair(false, gw ? ws + lb.gw_off : nullptr, grad_weight, c_out * c_in * nfx * nfy, gb ? ws + lb.gb_off : nullptr,

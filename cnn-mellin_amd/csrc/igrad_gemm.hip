@@ -436,6 +436,7 @@ __global__ __launch_bounds__(256) void igrad_combine_kernel(const IgradPlan pl,
 
 template <typename O>
 hipError_t launch_combine(const IgradPlan &pl, const float *ws, O *gi, hipStream_t stream, WgradReduce *beside) {
+  if (pl.ws_bytes == 0) return hipSuccess;
   WgradReduce first = {};
   dim3 grid((unsigned)(pl.strips - 1), (unsigned)(pl.batch * pl.c_in));
   const i64 blocks = (i64)grid.x * grid.y + (beside ? beside->blocks : 0);
@@ -450,7 +451,7 @@ hipError_t launch_combine(const IgradPlan &pl, const float *ws, O *gi, hipStream
 
 template <int KSTEPS, int NT, bool PIPE>
 hipError_t launch_instance(const IgradPlan &pl, const float *w, const float *go, float *gi,
-                           float *ws, hipStream_t stream, WgradReduce *beside) {
+                           float *ws, hipStream_t stream) {
   auto kern = igrad_kernel<KSTEPS, NT, PIPE>;
   {
     static std::atomic<int> lds_allowed{0};                // (one per kernel instance)
@@ -460,9 +461,7 @@ hipError_t launch_instance(const IgradPlan &pl, const float *w, const float *go,
   const int groups = (pl.batch + pl.jobs - 1) / pl.jobs;
   hipLaunchKernelGGL(kern, dim3((unsigned)(groups * pl.strips)), dim3(64 * pl.units * pl.jobs),
                      pl.lds_bytes, stream, pl, w, go, gi, ws);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || pl.ws_bytes == 0) return e;
-  return launch_combine(pl, ws, gi, stream, beside);
+  return hipGetLastError();
 }
 
 // The same input gradient on the bf16 matrix cores (tile_stage.hpp: every fp32 operand as
@@ -866,7 +865,7 @@ __global__ __launch_bounds__(256, 2) void igrad_stream_kernel(const IgradPlan pl
 
 template <int MTT, int NT, bool F16 = false>
 hipError_t launch_stream_instance(const IgradPlan &pl, const void *w, const void *go, void *gi,
-                                  float *ws, hipStream_t stream, WgradReduce *beside = nullptr) {
+                                  float *ws, hipStream_t stream) {
   auto kern = igrad_stream_kernel<MTT, NT, F16>;
   {
     static std::atomic<int> lds_allowed{0};                // (one per kernel instance)
@@ -875,10 +874,7 @@ hipError_t launch_stream_instance(const IgradPlan &pl, const void *w, const void
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)(pl.batch * pl.strips)), dim3(256), pl.lds_bytes, stream, pl, w, go, gi,
                      ws);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || pl.ws_bytes == 0) return e;
-  if (F16) return launch_combine(pl, ws, (_Float16 *)gi, stream, beside);
-  return launch_combine(pl, ws, (float *)gi, stream, beside);
+  return hipGetLastError();
 }
 
 // Tap products for the gather-fold input gradient (any x axis kind):
@@ -1253,24 +1249,29 @@ bool make_igrad_plan(int kind_x, i64 batch, i64 c_in, i64 c_out, i64 nfx, i64 nf
 hipError_t launch_igrad_half(const IgradPlan &pl, const void *weight, const void *grad_out,
                              void *grad_input, float *workspace, hipStream_t stream) {
   if (!pl.stream) return hipErrorInvalidValue;
-  if (pl.c_in == 1) return launch_stream_instance<1, 2, true>(pl, weight, grad_out, grad_input, workspace, stream);
-  if (pl.c_in == 2) return launch_stream_instance<2, 1, true>(pl, weight, grad_out, grad_input, workspace, stream);
-  return launch_stream_instance<3, 1, true>(pl, weight, grad_out, grad_input, workspace, stream);
+  const hipError_t e = pl.c_in == 1 ? launch_stream_instance<1, 2, true>(pl, weight, grad_out, grad_input, workspace, stream)
+                       : pl.c_in == 2 ? launch_stream_instance<2, 1, true>(pl, weight, grad_out, grad_input, workspace, stream)
+                                      : launch_stream_instance<3, 1, true>(pl, weight, grad_out, grad_input, workspace, stream);
+  return e == hipSuccess ? launch_combine(pl, workspace, (_Float16 *)grad_input, stream, nullptr) : e;
+}
+
+hipError_t launch_igrad_end(const IgradPlan &pl, const float *workspace, float *grad_input, hipStream_t stream, WgradReduce *beside) {
+  return launch_combine(pl, workspace, grad_input, stream, beside);
 }
 
 hipError_t launch_igrad(const IgradPlan &pl, const float *weight, const float *grad_out,
-                        float *grad_input, float *workspace, hipStream_t stream, WgradReduce *beside) {
+                        float *grad_input, float *workspace, hipStream_t stream) {
   if (pl.stream) {
-    if (pl.c_in == 1) return launch_stream_instance<1, 2>(pl, weight, grad_out, grad_input, workspace, stream, beside);
-    if (pl.c_in == 2) return launch_stream_instance<2, 1>(pl, weight, grad_out, grad_input, workspace, stream, beside);
-    return launch_stream_instance<3, 1>(pl, weight, grad_out, grad_input, workspace, stream, beside);
+    if (pl.c_in == 1) return launch_stream_instance<1, 2>(pl, weight, grad_out, grad_input, workspace, stream);
+    if (pl.c_in == 2) return launch_stream_instance<2, 1>(pl, weight, grad_out, grad_input, workspace, stream);
+    return launch_stream_instance<3, 1>(pl, weight, grad_out, grad_input, workspace, stream);
   }
   // the pipelined fold needs batches that cannot collide and no padded matrix rows
   const bool pipe = pl.pipe && pl.nt == 2;
 #define MELLIN_IGRAD_CASE(KS, NT_)                                                       \
   if (pl.ksteps == KS && pl.nt == NT_)                                                   \
-    return pipe ? launch_instance<KS, NT_, (NT_ == 2)>(pl, weight, grad_out, grad_input, workspace, stream, beside) \
-                : launch_instance<KS, NT_, false>(pl, weight, grad_out, grad_input, workspace, stream, beside);
+    return pipe ? launch_instance<KS, NT_, (NT_ == 2)>(pl, weight, grad_out, grad_input, workspace, stream) \
+                : launch_instance<KS, NT_, false>(pl, weight, grad_out, grad_input, workspace, stream);
   MELLIN_IGRAD_CASE(16, 2) MELLIN_IGRAD_CASE(16, 4)
   MELLIN_IGRAD_CASE(32, 2) MELLIN_IGRAD_CASE(32, 4)
   MELLIN_IGRAD_CASE(64, 2) MELLIN_IGRAD_CASE(64, 4)

@@ -40,8 +40,10 @@ bool make_igrad_plan(int kind_x, i64 batch, i64 c_in, i64 c_out, i64 nfx, i64 nf
                      i64 ux, i64 uy, IgradPlan &pl, int force_nt = 0, int force_Th = 0, int force_pipe = -1,
                      int math = MATH_FP32);
 
+// All but the rows that strips share; launch_igrad_end sums those (and may do nothing).
 hipError_t launch_igrad(const IgradPlan &pl, const float *weight, const float *grad_out,
-                        float *grad_input, float *workspace, hipStream_t stream, WgradReduce *beside = nullptr);
+                        float *grad_input, float *workspace, hipStream_t stream);
+hipError_t launch_igrad_end(const IgradPlan &pl, const float *workspace, float *grad_input, hipStream_t stream, WgradReduce *beside = nullptr);
 
 // The `stream` form of a plan on half-precision tensors (f16 matrix cores; the workspace
 // keeps fp32 partial rows): weight, grad_out and grad_input are half-precision storage.

@@ -135,6 +135,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
   int groups[8], n_groups = 0;                         // the channel groups of a stage that divide all, most first
   for (int G = std::min(pl.CG, 8); G >= 1; --G)
     if (pl.CG % G == 0 && (!like || G == like->G)) groups[n_groups++] = G;
+  i64 room = 79 * 1024;                                // LDS of a workgroup
   auto shape = [&](int at) {
     const int nt = shapes[at][0], wm = shapes[at][1], wk = shapes[at][2];
     const int P = (kWaves / wk / wm) * nt * 32, M_T = wm * pl.mt * 32;
@@ -151,10 +152,10 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
       for (int F = mellin ? pl.nfx : 1; F >= 1; --F) {
         const int rows = mellin ? F : pl.nfx, subsets = mellin ? (pl.nfx + F - 1) / F : 1;
         const i64 gb = (vrows * (mellin ? F : 1) * pl.RS * parts + 63) / 64 * 1024, fixed = 4 * tab + row_src + M_T * 4;
-        if (2 * gb + fixed > 79 * 1024) continue;
+        if (2 * gb + fixed > room) continue;
         for (int k = 0; k < n_groups; ++k) {
           const int G = groups[k], halves = rows * pl.nfy * G, all = pad(halves);
-          if (2 * gb * G + fixed + 16 * (i64)(subsets * all + (deep ? 12 : 8) * wk) > 79 * 1024) continue;
+          if (2 * gb * G + fixed + 16 * (i64)(subsets * all + (deep ? 12 : 8) * wk) > room) continue;
           // what a stage's steps fill of their whole pairs, against what a stage costs on top (its barrier and first reads)
           if (halves * best_all > best_halves * (all + 2 * wk)) { best_halves = halves; best_all = all + 2 * wk; st.F = F; st.G = G; }
         }
@@ -178,7 +179,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
     bytes += 4 * (size_t)tab + 16 * (size_t)pl.ents + row_src + M_T * 4;
     pl.lds_bytes = bytes;
     pl.m_tiles = (int)((pr.c_out + M_T - 1) / M_T);
-    return bytes <= 79 * 1024;
+    return bytes <= room;
   };
   auto magic = [](i64 d) { return d <= 1 ? 0xFFFFFFFFu : (unsigned)(0x100000000ull / (unsigned)d); };
   pl.mg_batch = magic(pl.batch); pl.mg_noy = magic(pl.noy);
@@ -355,6 +356,18 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
   }
   if (best_cost == 0) return false;
   pl = best_plan;
+  // Wavefronts that share a tile, more workgroups than two a CU: stages that leave room for a third, where it has registers,
+  // if they are not much smaller for it (or half on linear axes, whose steps are short).  Input gradient of 41 -> 128
+  // channels, 8 taps, 32 x 780, p = 3, 800 workgroups: 29.5 -> 24.6 us.  Of 40 drawn passes of more than 512 workgroups 13 take
+  // it, 0.80 to 0.98 of their time; those with smaller stages 0.97 to 1.26.  Input gradients only: a stage decides which
+  // wavefront adds what (see can_join).
+  if (gradient && pl.wk > 1 && ((i64)pl.whole + (i64)pl.rest * pl.slices) * pl.m_tiles > slots) {
+    const int at = pl.nt == 2 ? 5 : 6, fg = pl.F * pl.G, g = pl.G;
+    room = 53 * 1024;
+    stages[pl.mt - 1][at].rows = -1;
+    const bool fits = shape(at), large = (pl.G == g && 2 * pl.F * pl.G >= fg) || (2 * pl.G >= g && 5 * pl.F * pl.G >= 3 * fg);
+    if (!fits || !(large || (f16 && !mellin))) pl = best_plan;
+  }
   if (!f16 && pl.mt == 2 && pl.nt == 1 && pl.wk == 1) {
     // fp32, 64 channels x 128 positions: two by two wavefronts of 32 channels x 64 positions.  Four side by side take each
     // filter fragment from L1 four times, 64 bytes a cycle and CU, which is all that it gives; two by two take half of that and

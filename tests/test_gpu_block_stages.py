@@ -32,6 +32,9 @@ CASES = [
     ("lcorr", 70, 16, 128, (3, 2), (90, 20), (1, 1), (1, 1), (1, 0), (1, 0)),
     ("lcorr", 20, 56, 104, (2, 1), (200, 20), (1, 1), (1, 1), (0, 0), (0, 0)),
     ("mcorr", 30, 24, 72, (3, 1), (150, 20), (1, 1), (1, 1), (2, 0), (60, 0)),
+    # input gradients by wavefronts that share a tile, stages that leave room for a third workgroup on a CU (float; half)
+    ("mcorr", 16, 41, 128, (6, 1), (1201, 1), (1, 1), (1, 1), (2, 0), (0, 0)),
+    ("lcorr", 7, 24, 110, (4, 4), (130, 41), (1, 1), (1, 1), (1, 1), (1, 1)),
 ]
 
 

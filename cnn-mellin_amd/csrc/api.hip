@@ -2187,18 +2187,18 @@ static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const
     l.batch = ly.dims[0]; l.c_in = ly.dims[1]; l.c_out = ly.dims[2];
     l.plane = ly.dims[5] * ly.dims[6]; l.rows = ly.dims[7]; l.cols = ly.dims[8]; l.q = l.rows * l.cols;
     if (l.batch < 1 || l.batch > 65535 || l.c_out < 1 || l.c_out > 65535 || l.plane < 1 || l.q < 1 || l.batch != layers[0].dims[0]) return false;
-    if (ly.pool && (i == 0 || i == n - 1)) return false;
+    if (ly.pool && (i == 0 || (i == n - 1) != (ly.pool == MELLIN_STACK_NO_RELU))) return false;
     if (i == 0) continue;
     const mellin_stack_layer &before = layers[i - 1];
     if (l.c_in != before.dims[2] || ly.dims[5] != before.dims[7] || ly.dims[6] != (before.pool ? before.dims[8] / 2 : before.dims[8])) return false;
     BlockPlan bp;
-    if (!plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool)) return false;
+    if (!plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool == 1)) return false;
     x_bytes[i] = region(l.c_in, l.plane, l.batch);
     which_bytes[i] = before.pool ? align256((size_t)(l.batch * ((l.c_in + 7) / 8) * l.plane) * 8) : 0;
     l.frag_off = frags;                                // (forward; the backward call lays out its own)
     frags += align256(bp.filter_bytes);
     sums = std::max(sums, bp.slice_bytes);
-    if (ly.pool && !bp.pool) unpooled = std::max(unpooled, region(l.c_out, l.q, l.batch));
+    if (ly.pool == 1 && !bp.pool) unpooled = std::max(unpooled, region(l.c_out, l.q, l.batch));
     if (!train) continue;
     BlockPlan ip;
     BlockWgradPlan wp;
@@ -2322,7 +2322,7 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
   BlockPlan bp;
   for (int i = 1; i < n_layers; ++i) {
     const mellin_stack_layer &ly = layers[i];
-    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool);
+    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool == 1);
     bp.wide = wide;
     filters[i - 1] = pack_filter(bp, (int)ly.dims[1], ly.weight, ws + at, wide ? ly.weight_half : nullptr,
                                  ly.dims[1] * ly.dims[2] * ly.dims[3] * ly.dims[4]);
@@ -2369,11 +2369,11 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
     const mellin_stack_layer &ly = layers[i];
     const StackLayer &l = sp.l[i];
     const bool last = i == n_layers - 1;
-    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool);
-    bp.relu = 1;
+    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool == 1);
+    bp.relu = ly.pool != MELLIN_STACK_NO_RELU;
     bp.wide = wide;
-    char *const which = ly.pool && train && i + 1 > first ? keep + sp.l[i + 1].which_off : nullptr;
-    const bool pool_after = ly.pool && !bp.pool;
+    char *const which = ly.pool == 1 && train && i + 1 > first ? keep + sp.l[i + 1].which_off : nullptr;
+    const bool pool_after = ly.pool == 1 && !bp.pool;
     char *to = last ? (char *)out : pool_after ? ws + sp.f_unpooled : input_of(i + 1);
     const BlockGemmArgs args = {input_of(i), ws + frag_off[i], ly.bias, to, (float *)(ws + sp.f_sums), !last, false, nullptr, nullptr, which};
     e = launch_block_gemm(bp, args, st);
@@ -2430,7 +2430,7 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
     return r;
   };
   const StackLayer &lt = sp.l[top];
-  const PackSignal go = {grad_out, out, ws + sp.b_grad[top & 1], (float *)take(lt.bias_bytes), (int)lt.batch, (int)lt.c_out, (int)lt.q};
+  const PackSignal go = {grad_out, layers[top].pool == MELLIN_STACK_NO_RELU ? nullptr : out, ws + sp.b_grad[top & 1], (float *)take(lt.bias_bytes), (int)lt.batch, (int)lt.c_out, (int)lt.q};
   hipError_t e = launch_block_pack(half, &go, nullptr, filters, n_filters, st);
   if (layers[top].grad_bias) fin.add_bias(go.partial, (i64)pack_partial_count(lt.batch, 1, lt.q), lt.c_out, layers[top].grad_bias);
   for (int i = top; i >= std::max(lowest, 1) && e == hipSuccess; --i) {

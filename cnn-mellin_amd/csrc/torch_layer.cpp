@@ -386,11 +386,11 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     const int64_t dims[17] = {GEOMETRY_ARGS(g)};
     layers[i] = mellin_stack_layer{};
     std::copy(dims, dims + 17, layers[i].dims);
-    layers[i].pool = PyTuple_GET_ITEM(t, 6) == Py_True;
+    layers[i].pool = PyTuple_GET_ITEM(t, 6) == Py_True ? 1 : PyTuple_GET_ITEM(t, 6) == Py_None ? MELLIN_STACK_NO_RELU : 0;
     if (wt.requires_grad() || (bt.defined() && bt.requires_grad())) first = std::min(first, (int)i);
     c = g.c_out;
     x = g.nh[0];
-    y = layers[i].pool ? g.nh[1] / 2 : g.nh[1];
+    y = layers[i].pool == 1 ? g.nh[1] / 2 : g.nh[1];
   }
   // float parameters of half tensors (autocast) are rounded by the library; any other mixture is not for this path
   const bool wide = kind_of == at::kHalf && param_kind == at::kFloat;
@@ -621,7 +621,8 @@ PyMethodDef methods[] = {
     {"pack_windows", (PyCFunction)(void *)pack_windows, METH_FASTCALL,
      "pack_windows(x, lens, size, stride): (data, batch_sizes, sorted_indices, unsorted_indices), or None if not handled"},
     {"stack", (PyCFunction)(void *)stack, METH_FASTCALL,
-     "stack(kind, input, [(weight, bias, s, d, p, r, pool), ...]): the last layer's output behind its ReLU, or None if not handled"},
+     "stack(kind, input, [(weight, bias, s, d, p, r, pool), ...]): the last layer's output behind its ReLU (without one if its "
+     "pool is None), or None if not handled"},
     {"corr", (PyCFunction)(void *)corr, METH_FASTCALL,
      "corr(kind, dims, input, weight, bias, s, d, p, u, r, activation): the layer's output, or None if not handled"},
     {nullptr, nullptr, 0, nullptr}};

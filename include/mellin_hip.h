@@ -482,7 +482,8 @@ int mellin_layer_backward_kept(int kind_x, int elem_bytes, int want, const void 
  * the matrix kernels (channel-blocked), so nothing is laid out anew, and the backward of the ReLUs, the bias gradients and
  * the pooling ride along with the kernels.  Layer i reads what layer i - 1 leaves: dims are those of MELLIN_CORR2D_DIMS, in
  * order; with `pool` its output is first reduced to the maxima of pairs of neighbouring columns (y axis, an odd last one is
- * dropped; not after the first layer or the last).  elem_bytes as for a layer; weight_half: where the forward call leaves a
+ * dropped; not after the first layer or the last).  pool = MELLIN_STACK_NO_RELU: the last layer, an output layer, has no ReLU
+ * behind it.  elem_bytes as for a layer; weight_half: where the forward call leaves a
  * float weight rounded to half, which the backward call takes (MELLIN_ELEM_HALF_FLOAT in training; null otherwise);
  * grad_weight, grad_bias: null for gradients that are not wanted.
  * mellin_stack_bytes: 1 if the stack can be run so under the settings in force, 0 if not (layers with too few channels for
@@ -493,6 +494,7 @@ int mellin_layer_backward_kept(int kind_x, int elem_bytes, int want, const void 
  * train = 2: for the backward call of a forward call already made, which goes on whatever has been set since (the first
  * layer's kernels follow the settings, so its workspace may have another size).
  * out: the last layer's output, as it lies. */
+#define MELLIN_STACK_NO_RELU 2
 typedef struct {
   int64_t dims[17];
   int pool;

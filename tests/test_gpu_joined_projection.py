@@ -16,6 +16,11 @@ CASES = [
 ]
 
 
+class Through(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
 @pytest.mark.parametrize("how", ["autocast", "half", "no bias", "frozen"])
 @pytest.mark.parametrize("case", CASES, ids=range(len(CASES)))
 def test_joined_and_apart(case, how):
@@ -86,5 +91,41 @@ def test_sizes_and_types_that_stay_apart():
                 model(torch.randn(2, 3, 40, bins, device="cuda"))
         with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
             assert model._scores(x) is None
+        with Through():
+            assert model._scores(x) is None
         many = FrameClassifier(ConvStack(40, 7, params), 9).cuda()
         assert many._scores(torch.randn(2, 3, 40, 7, device="cuda")) is None                     # more than 6 bins
+
+
+@pytest.mark.parametrize("how", ["autocast", "half", "no bias", "frozen"])
+def test_second_derivatives_of_the_projection(how):
+    params = ConvStackParams(layers=2, kernel_time=3, kernel_freq=3, initial_channels=32, factor_schedule=2, time_factor=1,
+                             in_channels=3)
+    torch.manual_seed(9700)
+    model = FrameClassifier(ConvStack(40, 5, params), 9).cuda()
+    if how == "no bias":
+        model.out.bias = None
+    if how == "frozen":
+        model.stack.requires_grad_(False)
+    x = torch.randn(2, 3, 40, 5, device="cuda")
+    if how == "half":
+        model, x = model.half(), x.half()
+    labels = torch.randint(9, (80,), device="cuda")
+    leaves = [p for p in model.parameters() if p.requires_grad]
+
+    def penalty():
+        with torch.autocast("cuda", torch.float16, enabled=how != "half"):
+            out = model(x)
+        loss = torch.nn.functional.nll_loss(out.flatten(0, 1).float(), labels)
+        first = torch.autograd.grad(loss, list(model.out.parameters()), create_graph=True)
+        return [v.detach() for v in first] + list(torch.autograd.grad(sum(v.float().square().sum() for v in first) * 64, leaves))
+
+    joined = penalty()
+    hook = model.out.register_forward_hook(lambda *a: None)
+    apart = penalty()
+    hook.remove()
+    # half features, gradients and their gradients: a few roundings of 2^-11 each, in sums whose terms partly cancel
+    for got, want in zip(joined, apart):
+        assert got.dtype == want.dtype and got.shape == want.shape
+        rel = float((got.double() - want.double()).norm() / want.double().norm())
+        assert rel < 2e-2, rel

@@ -21,11 +21,16 @@ namespace mellin {
 namespace {
 
 constexpr int kPackThreads = 256;
-constexpr int kPackPositions = 4;                  // per thread
+constexpr int kPackPositions = 4;                  // per thread at most
+// Positions that a thread takes one after the other: one where four would leave fewer than this many blocks, each of which waits
+// for memory as often as it has positions; with more blocks than fill the chip, half blocks of one position lose (us: 33 half channels of 7 x 333 x 37, 455 blocks of four,
+// 11.6 -> 9.5; a 1-D half layer's two launches, 32 x 780 with 41 and 128 channels, 192 and 704 blocks, 8.3 -> 6.8 each, fp32 8.9 -> 8.4;
+// 128 half channels of 32 x 256 x 41 and 256 of 32 x 194 x 41, 5600 and 8200 blocks of four, 49.2 -> 71.4 on average, so they keep four).
+constexpr i64 kPackBlocks = 1024;
 
 struct PackPart {                                  // a signal, dealt to blocks as (image, group, chunk of its plane)
   PackSignal s;
-  int groups, chunks;
+  int groups, positions, chunks;
   unsigned blocks;
 };
 
@@ -43,9 +48,10 @@ __device__ __forceinline__ void pack_signal(const PackPart &pt, unsigned block, 
   float sum[8];
 #pragma unroll
   for (int c = 0; c < 8; ++c) sum[c] = 0.f;
-  const int q0 = chunk * (kPackThreads * kPackPositions) + threadIdx.x;
+  const int q0 = chunk * (kPackThreads * pt.positions) + threadIdx.x;
 #pragma unroll
   for (int i = 0; i < kPackPositions; ++i) {
+    if (i >= pt.positions) break;
     const int q = q0 + i * kPackThreads;
     if (q < plane) {
       T v[8];
@@ -203,14 +209,18 @@ __global__ __launch_bounds__(kPackThreads) void block_pack_kernel(PackArgs<FILTE
   }
 }
 
-i64 pack_chunks(i64 plane) { return plane / (kPackThreads * kPackPositions) + 1; }     // (plane + 1 units)
+i64 pack_chunks(i64 plane, int positions) { return plane / (kPackThreads * positions) + 1; }     // (plane + 1 units)
+int pack_positions(i64 batch, i64 channels, i64 plane) {
+  return batch * ((channels + 7) / 8) * pack_chunks(plane, kPackPositions) < kPackBlocks ? 1 : kPackPositions;
+}
 
 bool pack_part(const PackSignal *s, PackPart &pt) {
   pt = PackPart{};
   if (!s) return true;
   pt.s = *s;
   pt.groups = (s->channels + 7) / 8;
-  pt.chunks = (int)pack_chunks(s->plane);
+  pt.positions = pack_positions(s->batch, s->channels, s->plane);
+  pt.chunks = (int)pack_chunks(s->plane, pt.positions);
   const i64 blocks = (i64)s->batch * pt.groups * pt.chunks;
   pt.blocks = (unsigned)blocks;
   return blocks < (i64)1 << 30;
@@ -219,7 +229,7 @@ bool pack_part(const PackSignal *s, PackPart &pt) {
 }  // namespace
 
 size_t pack_partial_count(i64 batch, i64 channels, i64 plane) {
-  return (size_t)(batch * channels * pack_chunks(plane));
+  return (size_t)(batch * channels * pack_chunks(plane, pack_positions(batch, channels, plane)));
 }
 
 PackFilter pack_filter(const BlockPlan &pl, int channels, const void *f, void *frag, void *copy, i64 copy_count) {

@@ -2088,7 +2088,7 @@ int mellin_layer_backward_kept(int kind_x, int elem_bytes, int want, const void 
     fin.add_weight(lb.wp, ws + lb.wgrad_off, grad_weight);
     if (e == hipSuccess) e = launch_block_wgrad(lb.wp, ws + lb.go_off, kept ? kept : ws + lb.x_off, (float *)(ws + lb.wgrad_off), st);
   }
-  if (sums) fin.add_bias(ws + lb.bias_off, (i64)pack_partial_count(batch, c_out, nhx * nhy) / c_out, c_out, grad_bias);
+  if (sums) fin.add_bias(ws + lb.bias_off, (i64)pack_partial_count(batch, 1, nhx * nhy), c_out, grad_bias);
   if (e == hipSuccess) e = launch_block_finish(half, wide, fin, st);
   return check_hip(e, __func__);
 }
@@ -2432,7 +2432,7 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
   const StackLayer &lt = sp.l[top];
   const PackSignal go = {grad_out, layers[top].pool == MELLIN_STACK_NO_RELU ? nullptr : out, ws + sp.b_grad[top & 1], (float *)take(lt.bias_bytes), (int)lt.batch, (int)lt.c_out, (int)lt.q};
   hipError_t e = launch_block_pack(half, &go, nullptr, filters, n_filters, st);
-  if (layers[top].grad_bias) fin.add_bias(go.partial, (i64)pack_partial_count(lt.batch, lt.c_out, lt.q) / lt.c_out, lt.c_out, layers[top].grad_bias);
+  if (layers[top].grad_bias) fin.add_bias(go.partial, (i64)pack_partial_count(lt.batch, 1, lt.q), lt.c_out, layers[top].grad_bias);
   for (int i = top; i >= std::max(lowest, 1) && e == hipSuccess; --i) {
     const mellin_stack_layer &ly = layers[i];
     const StackLayer &l = sp.l[i];

@@ -22,10 +22,12 @@ namespace {
 
 constexpr int kPackThreads = 256;
 constexpr int kPackPositions = 4;                  // per thread at most
-// Positions that a thread takes one after the other: one where four would leave fewer than this many blocks, each of which waits
-// for memory as often as it has positions; with more blocks than fill the chip, half blocks of one position lose (us: 33 half channels of 7 x 333 x 37, 455 blocks of four,
-// 11.6 -> 9.5; a 1-D half layer's two launches, 32 x 780 with 41 and 128 channels, 192 and 704 blocks, 8.3 -> 6.8 each, fp32 8.9 -> 8.4;
-// 128 half channels of 32 x 256 x 41 and 256 of 32 x 194 x 41, 5600 and 8200 blocks of four, 49.2 -> 71.4 on average, so they keep four).
+// Positions that a thread takes one after the other.  Without sums: one in fp32 (us: 128 channels of 32 x 256 x 41,
+// averaged with 256 that have sums, 154.9 -> 143), and in half one where four would
+// leave fewer than kPackBlocks blocks, each of which waits for memory as often as it has positions (33 half channels of
+// 7 x 333 x 37, 455 blocks of four, 11.6 -> 9.5); with more blocks than fill the chip, half blocks of one position lose (128
+// channels of 32 x 256 x 41 and 256 of 32 x 194 x 41, 5600 and 8200 blocks, 49.2 -> 71.4 on average).  With sums: four, the
+// order of sums that gives a bias gradient the same bits whether the input gradient is asked for beside it or not.
 constexpr i64 kPackBlocks = 1024;
 
 struct PackPart {                                  // a signal, dealt to blocks as (image, group, chunk of its plane)
@@ -210,16 +212,17 @@ __global__ __launch_bounds__(kPackThreads) void block_pack_kernel(PackArgs<FILTE
 }
 
 i64 pack_chunks(i64 plane, int positions) { return plane / (kPackThreads * positions) + 1; }     // (plane + 1 units)
-int pack_positions(i64 batch, i64 channels, i64 plane) {
-  return batch * ((channels + 7) / 8) * pack_chunks(plane, kPackPositions) < kPackBlocks ? 1 : kPackPositions;
+int pack_positions(bool half, const PackSignal &s, int groups) {
+  if (s.partial) return kPackPositions;
+  return !half || (i64)s.batch * groups * pack_chunks(s.plane, kPackPositions) < kPackBlocks ? 1 : kPackPositions;
 }
 
-bool pack_part(const PackSignal *s, PackPart &pt) {
+bool pack_part(bool half, const PackSignal *s, PackPart &pt) {
   pt = PackPart{};
   if (!s) return true;
   pt.s = *s;
   pt.groups = (s->channels + 7) / 8;
-  pt.positions = pack_positions(s->batch, s->channels, s->plane);
+  pt.positions = pack_positions(half, *s, pt.groups);
   pt.chunks = (int)pack_chunks(s->plane, pt.positions);
   const i64 blocks = (i64)s->batch * pt.groups * pt.chunks;
   pt.blocks = (unsigned)blocks;
@@ -229,7 +232,7 @@ bool pack_part(const PackSignal *s, PackPart &pt) {
 }  // namespace
 
 size_t pack_partial_count(i64 batch, i64 channels, i64 plane) {
-  return (size_t)(batch * channels * pack_chunks(plane, pack_positions(batch, channels, plane)));
+  return (size_t)(batch * channels * pack_chunks(plane, kPackPositions));
 }
 
 PackFilter pack_filter(const BlockPlan &pl, int channels, const void *f, void *frag, void *copy, i64 copy_count) {
@@ -244,7 +247,7 @@ template <int FILTERS>
 static hipError_t launch_pack(bool f16, const PackSignal *a, const PackSignal *b, const PackFilter *filters, int n_filters,
                               hipStream_t stream) {
   PackArgs<FILTERS> args = {};
-  if (!pack_part(a, args.a) || !pack_part(b, args.b)) return hipErrorInvalidValue;
+  if (!pack_part(f16, a, args.a) || !pack_part(f16, b, args.b)) return hipErrorInvalidValue;
   do {
     unsigned blocks = args.a.blocks + args.b.blocks;
     int i = 0, classes = 0;

@@ -13,7 +13,6 @@ layers.  Layers are this package's `MCorrLCorr` (Mellin x linear) or
 `LCorrLCorr` (linear x linear, in place of the reference's
 ``torch.nn.Conv2d``, models.py:329-338, with the same padding rule).
 """
-import functools
 from typing import Callable, List, Optional, Sequence, Tuple
 
 import torch
@@ -259,28 +258,9 @@ class FrameClassifier(torch.nn.Module):
         y = _native_stack(kind, x, [(conv.weight, conv.bias, conv.s, conv.d, conv.p, conv.r, bool(lay["pool"]))
                                     for conv, lay in zip(stack.convs, stack.plan)] +
                           [(weight.view(-1, channels, 1, bins), out.bias, (1, 1), (1, 1), (0, 0), (0, 0), None)])
-        if y is None or y.shape[3] != 1:
+        if y is None:
             return None
-        if y.grad_fn is not None:
-            y.grad_fn.register_hook(functools.partial(self._projection_grads, x, torch.is_autocast_enabled("cuda")))
         return y.squeeze(3).transpose(1, 2).contiguous()
-
-    def _projection_grads(self, x, cast, grads, grad_y):
-        """With ``create_graph``: the projection's gradients as operations, since the stack's call has no second derivative."""
-        if not torch.is_grad_enabled() or grad_y[0] is None or (grads[-2] is None and grads[-1] is None):
-            return None
-        g = grad_y[0]                                       # (N, n_out, T', 1)
-        last = list(grads[-2:])
-        if last[0] is not None:
-            with torch.autocast("cuda", torch.float16, enabled=cast):
-                h = self.stack(x).to(g.dtype)               # (N, C, T', F')
-            h = h.permute(0, 2, 1, 3).flatten(2).flatten(0, 1)
-            by_class = g.squeeze(3).transpose(0, 1).flatten(1)
-            with torch.autocast("cuda", enabled=False):
-                last[0] = (by_class @ h).to(grads[-2].dtype).view(grads[-2].shape)
-        if last[1] is not None:
-            last[1] = g.sum((0, 2, 3)).to(grads[-1].dtype)
-        return tuple(grads[:-2]) + tuple(last)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         scores = self._scores(x)

@@ -260,7 +260,15 @@ PyObject *corr(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
-// The gradients of a stack of layers with ReLUs.  Edges: the input, then weight and bias of every layer.
+// A tensor in the kernels' layout, [image][group of eight channels][plane + behind][8 channels], from byte `at` on, as it lies.
+Tensor unblocked(const Tensor &bytes, int64_t at, at::ScalarType kind, int64_t n, int64_t c, int64_t rows, int64_t cols, int64_t behind) {
+  const int64_t groups = (c + 7) / 8, plane = rows * cols, count = n * groups * (plane + behind) * 8;
+  return bytes.narrow(0, at, count * (int64_t)c10::elementSize(kind)).view(kind).view({n, groups, plane + behind, 8})
+      .narrow(2, 0, plane).permute({0, 1, 3, 2}).reshape({n, groups * 8, rows, cols}).narrow(1, 0, c);
+}
+
+// The gradients of a stack of layers with ReLUs.  Edges: the input, then weight and bias of every layer.  The last layer may be
+// a projection of a row's columns (MELLIN_STACK_NO_RELU; half tensors): only what it is made of can be differentiated twice.
 struct StackBackward : public torch::autograd::Node {
   int kind = 0, elem = 4;
   std::vector<mellin_stack_layer> layers;              // geometry; the pointers are filled in for each call
@@ -272,6 +280,10 @@ struct StackBackward : public torch::autograd::Node {
   size_t workspace = 0;
   at::ScalarType param_kind = at::kFloat;
 
+  bool projects() const { return layers.back().pool == MELLIN_STACK_NO_RELU; }
+  // A projection alone learns.
+  bool frozen() const { return projects() && first == (int)layers.size() - 1; }
+
   std::string name() const override { return "StackBackward"; }
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -282,6 +294,7 @@ struct StackBackward : public torch::autograd::Node {
   }
 
   torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+    const bool create_graph = at::GradMode::is_enabled();
     at::AutoGradMode no_grad(false);
     const size_t n = layers.size();
     Tensor input, out, saved;
@@ -325,7 +338,68 @@ struct StackBackward : public torch::autograd::Node {
       if (mellin_stack_bytes(kind, elem, 2, (int)n, call.data(), &ignored[0], &ignored[1], &bytes)) rc = launch(bytes);
     }
     check(rc);
+    if (create_graph && projects() && grads[0].defined() && (result[2 * n - 1].defined() || result[2 * n].defined()))
+      differentiable_projection(grads[0], input, weights, saved, result[2 * n - 1], result[2 * n]);
     return result;
+  }
+
+  // With create_graph: the projection's gradients as operations on the features that the forward call saved.
+  void differentiable_projection(const Tensor &grad, const Tensor &input, const std::vector<Tensor> &weights, const Tensor &saved,
+                                 Tensor &grad_weight, Tensor &grad_bias) {
+    const c10::impl::ExcludeDispatchKeyGuard no_cast(c10::autocast_dispatch_keyset);
+    at::AutoGradMode with_grad(true);
+    const Tensor g = grad.to(at::kHalf);               // (N, classes, T', 1)
+    if (grad_bias.defined()) grad_bias = g.sum(at::IntArrayRef({0, 2, 3})).to(param_kind);
+    if (!grad_weight.defined()) return;
+    const Tensor h = features(input, weights, saved);  // (N, C, T', F')
+    grad_weight = g.squeeze(3).transpose(0, 1).flatten(1).mm(h.permute({0, 2, 1, 3}).flatten(2).flatten(0, 1)).to(param_kind)
+                      .view(grad_weight.sizes());
+  }
+
+  // The projection's input as the forward call saved it, with the layers below as its graph: the same node over them alone,
+  // whose part of `saved` comes last.
+  Tensor features(const Tensor &input, const std::vector<Tensor> &weights, const Tensor &saved) {
+    const size_t below = layers.size() - 1;
+    const int64_t *d = layers[below].dims, n = d[0], c = d[1], rows = d[5], cols = d[6];
+    Tensor h, second, out;
+    std::shared_ptr<StackBackward> node;
+    {
+      at::AutoGradMode no_grad(false);
+      h = unblocked(saved, 0, at::kHalf, n, c, rows, cols, 1).contiguous();
+      if (frozen()) return h;
+      node = std::shared_ptr<StackBackward>(new StackBackward(), torch::autograd::deleteNode);
+      node->layers.assign(layers.begin(), layers.end() - 1);
+      mellin_stack_layer &top = node->layers.back();
+      const bool pooled = top.pool;
+      top.pool = 0;                                    // (its output below is that in front of the pooling)
+      size_t saved_bytes = 0, forward_bytes = 0;
+      TORCH_CHECK(mellin_stack_bytes(kind, elem, first << 8 | 2, (int)below, node->layers.data(), &saved_bytes, &forward_bytes, &node->workspace),
+                  "libmellin_hip: no backward call for the layers below a projection");
+      const int64_t rest = saved.numel() - (int64_t)saved_bytes;
+      node->saved_ = saved.narrow(0, rest, (int64_t)saved_bytes);
+      out = h;
+      if (pooled) {                                    // the larger of a pair where it was, zeros elsewhere
+        const int64_t which_bytes = n * ((c + 7) / 8) * rows * cols * 8;
+        second = unblocked(saved, rest - (which_bytes + 255) / 256 * 256, at::kByte, n, c, rows, cols, 0).to(at::kBool);
+        out = at::zeros({n, c, rows, top.dims[8]}, h.options());
+        out.slice(3, 0, 2 * cols, 2).copy_(h.masked_fill(second, 0));
+        out.slice(3, 1, 2 * cols, 2).copy_(h.masked_fill(second.logical_not(), 0));
+      }
+    }
+    torch::autograd::edge_list edges(next_edges().begin(), next_edges().begin() + 1 + 2 * below);
+    node->set_next_edges(std::move(edges));
+    node->kind = kind;
+    node->elem = elem;
+    node->first = first;
+    node->param_kind = param_kind;
+    node->input_ = torch::autograd::SavedVariable(input, false);
+    for (size_t i = 0; i < below; ++i) {
+      node->weights_.emplace_back(weights[i], false);
+      node->has_bias.push_back(has_bias[i]);
+    }
+    torch::autograd::set_history(out, node);
+    node->out_ = torch::autograd::SavedVariable(out, true);
+    return second.defined() ? at::where(second, out.slice(3, 1, 2 * cols, 2), out.slice(3, 0, 2 * cols, 2)) : out;
   }
 };
 
@@ -386,7 +460,13 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     const int64_t dims[17] = {GEOMETRY_ARGS(g)};
     layers[i] = mellin_stack_layer{};
     std::copy(dims, dims + 17, layers[i].dims);
-    layers[i].pool = PyTuple_GET_ITEM(t, 6) == Py_True ? 1 : PyTuple_GET_ITEM(t, 6) == Py_None ? MELLIN_STACK_NO_RELU : 0;
+    layers[i].pool = PyTuple_GET_ITEM(t, 6) == Py_True ? 1 : 0;
+    if (PyTuple_GET_ITEM(t, 6) == Py_None) {           // a projection of a row's columns
+      if (i != n - 1 || n < 3 || kind_of != at::kHalf || g.nf[0] != 1 || g.nf[1] != y || g.nh[0] != x || g.nh[1] != 1 || g.s[0] != 1 || g.d[0] != 1 ||
+          g.p[0] != 0 || g.d[1] != 1 || g.p[1] != 0)
+        Py_RETURN_NONE;
+      layers[i].pool = MELLIN_STACK_NO_RELU;
+    }
     if (wt.requires_grad() || (bt.defined() && bt.requires_grad())) first = std::min(first, (int)i);
     c = g.c_out;
     x = g.nh[0];
@@ -622,7 +702,7 @@ PyMethodDef methods[] = {
      "pack_windows(x, lens, size, stride): (data, batch_sizes, sorted_indices, unsorted_indices), or None if not handled"},
     {"stack", (PyCFunction)(void *)stack, METH_FASTCALL,
      "stack(kind, input, [(weight, bias, s, d, p, r, pool), ...]): the last layer's output behind its ReLU (without one if its "
-     "pool is None), or None if not handled"},
+     "pool is None: a projection of each row's columns, in half), or None if not handled"},
     {"corr", (PyCFunction)(void *)corr, METH_FASTCALL,
      "corr(kind, dims, input, weight, bias, s, d, p, u, r, activation): the layer's output, or None if not handled"},
     {nullptr, nullptr, 0, nullptr}};

@@ -281,7 +281,7 @@ struct StackBackward : public torch::autograd::Node {
   at::ScalarType param_kind = at::kFloat;
 
   bool projects() const { return layers.back().pool == MELLIN_STACK_NO_RELU; }
-  // A projection alone learns.
+  // A projection alone learns: its weight, the input and the layers below are not read again, and may change.
   bool frozen() const { return projects() && first == (int)layers.size() - 1; }
 
   std::string name() const override { return "StackBackward"; }
@@ -301,10 +301,10 @@ struct StackBackward : public torch::autograd::Node {
     std::vector<Tensor> weights(n);
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      input = input_.unpack();                         // (raises if the variables have been released)
-      out = out_.unpack(shared_from_this());
-      for (size_t i = 0; i < n; ++i) weights[i] = weights_[i].unpack();
+      out = out_.unpack(shared_from_this());           // (raises if the variables have been released)
       saved = saved_;
+      input = frozen() ? saved : input_.unpack();      // (frozen: some memory)
+      for (size_t i = 0; i < n; ++i) weights[i] = weights_[i].unpack();
     }
     torch::autograd::variable_list result(1 + 2 * n);
     Tensor grad_out = grads[0].defined() ? grads[0] : at::zeros_like(out);
@@ -315,14 +315,15 @@ struct StackBackward : public torch::autograd::Node {
     if (task_should_compute_output(0)) result[0] = at::empty_like(input, at::MemoryFormat::Contiguous);
     for (size_t i = 0; i < n; ++i) {
       const Tensor &w = weights[i];
-      if (elem != MELLIN_ELEM_HALF_FLOAT) call[i].weight = w.const_data_ptr();
-      else if ((int)i >= first) call[i].weight_half = w.data_ptr();
+      const int64_t *d = layers[i].dims;
+      if (elem != MELLIN_ELEM_HALF_FLOAT) call[i].weight = pointer(w);
+      else if ((int)i >= first) call[i].weight_half = const_cast<void *>(pointer(w));
       if (task_should_compute_output(1 + 2 * i)) {
-        result[1 + 2 * i] = at::empty(w.sizes(), w.options().dtype(param_kind));
+        result[1 + 2 * i] = at::empty({d[2], d[1], d[3], d[4]}, out.options().dtype(param_kind));
         call[i].grad_weight = result[1 + 2 * i].data_ptr();
       }
       if (has_bias[i] && task_should_compute_output(2 + 2 * i)) {
-        result[2 + 2 * i] = at::empty({w.size(0)}, w.options().dtype(param_kind));
+        result[2 + 2 * i] = at::empty({d[2]}, out.options().dtype(param_kind));
         call[i].grad_bias = result[2 + 2 * i].data_ptr();
       }
     }
@@ -523,7 +524,6 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
       for (Py_ssize_t i = 0; i < n; ++i) {
         edge(weights[i]);
         edge(biases[i]);
-        node->weights_.emplace_back(kept[i], false);
         node->has_bias.push_back(biases[i].defined());
       }
       node->set_next_edges(std::move(edges));
@@ -531,7 +531,9 @@ PyObject *stack(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
       node->elem = elem;
       node->first = first;
       node->layers = std::move(layers);
-      node->input_ = torch::autograd::SavedVariable(input, false);
+      const bool frozen = node->frozen();
+      for (Py_ssize_t i = 0; i < n; ++i) node->weights_.emplace_back(frozen ? Tensor() : kept[i], false);
+      if (!frozen) node->input_ = torch::autograd::SavedVariable(input, false);
       node->saved_ = std::move(saved);
       node->workspace = backward_bytes;
       node->param_kind = wide ? at::kFloat : kind_of;

@@ -56,7 +56,7 @@ def change(model, x):
 
 
 @pytest.mark.parametrize("changed", [False, True])
-@pytest.mark.parametrize("how", ["autocast", "no bias", "input"])
+@pytest.mark.parametrize("how", ["autocast", "no bias", "frozen", "frozen half", "input"])
 @pytest.mark.parametrize("case", CASES, ids=range(len(CASES)))
 def test_gradients_are_those_of_the_forward_call(case, how, changed, monkeypatch):
     calls, counts, native = [], [], conv_stack._native_stack

@@ -2174,6 +2174,11 @@ struct StackPlan {
   size_t f_first, f_own, f_filters, f_unpooled, f_sums, f_turn[2], own_bytes;                          // forward workspace
   size_t b_grad[2], b_partial, partial_bytes, b_sums, b_first, b_own, b_own_bytes;         // backward workspace
 };
+// What `pool` says of layer i: whatever is not zero pools behind an inner one; of the last, see mellin_hip.h.
+static bool pools(const mellin_stack_layer *layers, int n, int i) { return layers[i].pool != 0 && i < n - 1; }
+static bool has_relu(const mellin_stack_layer *layers, int n, int i) { return i < n - 1 || layers[i].pool != MELLIN_STACK_NO_RELU; }
+// The columns that were pooled into layer i's input, or 0.
+static i64 pooled_cols(const mellin_stack_layer *layers, int n, int i) { return pools(layers, n, i - 1) ? layers[i - 1].dims[8] : 0; }
 static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const mellin_stack_layer *layers, StackPlan &sp) {
   const bool half = elem != 4;
   if (n < 2 || n > kStackLayers || first < 0 || first >= n) return false;
@@ -2187,22 +2192,23 @@ static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const
     l.batch = ly.dims[0]; l.c_in = ly.dims[1]; l.c_out = ly.dims[2];
     l.plane = ly.dims[5] * ly.dims[6]; l.rows = ly.dims[7]; l.cols = ly.dims[8]; l.q = l.rows * l.cols;
     if (l.batch < 1 || l.batch > 65535 || l.c_out < 1 || l.c_out > 65535 || l.plane < 1 || l.q < 1 || l.batch != layers[0].dims[0]) return false;
-    if (ly.pool && (i == 0 || (i == n - 1) != (ly.pool == MELLIN_STACK_NO_RELU))) return false;
+    if (ly.pool && (i == 0 || (i == n - 1 && has_relu(layers, n, i)))) return false;
     if (i == 0) continue;
     const mellin_stack_layer &before = layers[i - 1];
-    if (l.c_in != before.dims[2] || ly.dims[5] != before.dims[7] || ly.dims[6] != (before.pool ? before.dims[8] / 2 : before.dims[8])) return false;
+    const i64 from_cols = pooled_cols(layers, n, i);
+    if (l.c_in != before.dims[2] || ly.dims[5] != before.dims[7] || ly.dims[6] != (from_cols ? from_cols / 2 : before.dims[8])) return false;
     BlockPlan bp;
-    if (!plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool == 1)) return false;
+    if (!plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, pools(layers, n, i))) return false;
     x_bytes[i] = region(l.c_in, l.plane, l.batch);
-    which_bytes[i] = before.pool ? align256((size_t)(l.batch * ((l.c_in + 7) / 8) * l.plane) * 8) : 0;
+    which_bytes[i] = from_cols ? align256((size_t)(l.batch * ((l.c_in + 7) / 8) * l.plane) * 8) : 0;
     l.frag_off = frags;                                // (forward; the backward call lays out its own)
     frags += align256(bp.filter_bytes);
     sums = std::max(sums, bp.slice_bytes);
-    if (ly.pool == 1 && !bp.pool) unpooled = std::max(unpooled, region(l.c_out, l.q, l.batch));
+    if (pools(layers, n, i) && !bp.pool) unpooled = std::max(unpooled, region(l.c_out, l.q, l.batch));
     if (!train) continue;
     BlockPlan ip;
     BlockWgradPlan wp;
-    if (!plan_block_input(kind_x, half, STACK_DIMS(ly), ip, before.pool ? before.dims[8] : 0) || !plan_block_weight(kind_x, half, STACK_DIMS(ly), wp)) return false;
+    if (!plan_block_input(kind_x, half, STACK_DIMS(ly), ip, from_cols) || !plan_block_weight(kind_x, half, STACK_DIMS(ly), wp)) return false;
     b_frags += align256(ip.filter_bytes);
     b_sums = std::max(b_sums, ip.slice_bytes);
     grad[i & 1] = std::max(grad[i & 1], region(l.c_out, l.q, l.batch));
@@ -2261,7 +2267,7 @@ static bool plan_stack(int kind_x, int elem, bool train, int first, int n, const
   sp.backward = at + b_frags;
   for (int i = 1; i < n; ++i) {
     BlockPlan ip;
-    plan_block_input(kind_x, half, STACK_DIMS(layers[i]), ip, layers[i - 1].pool ? layers[i - 1].dims[8] : 0);
+    plan_block_input(kind_x, half, STACK_DIMS(layers[i]), ip, pooled_cols(layers, n, i));
     sp.l[i].frag_off = at;                             // (with train: the backward's; mellin_stack_forward counts its own)
     at += align256(ip.filter_bytes);
   }
@@ -2322,7 +2328,7 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
   BlockPlan bp;
   for (int i = 1; i < n_layers; ++i) {
     const mellin_stack_layer &ly = layers[i];
-    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool == 1);
+    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, pools(layers, n_layers, i));
     bp.wide = wide;
     filters[i - 1] = pack_filter(bp, (int)ly.dims[1], ly.weight, ws + at, wide ? ly.weight_half : nullptr,
                                  ly.dims[1] * ly.dims[2] * ly.dims[3] * ly.dims[4]);
@@ -2369,11 +2375,12 @@ int mellin_stack_forward(int kind_x, int elem_bytes, int train, int n_layers, co
     const mellin_stack_layer &ly = layers[i];
     const StackLayer &l = sp.l[i];
     const bool last = i == n_layers - 1;
-    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, ly.pool == 1);
-    bp.relu = ly.pool != MELLIN_STACK_NO_RELU;
+    const bool pooled = pools(layers, n_layers, i);
+    plan_block_forward(kind_x, half, STACK_DIMS(ly), bp, pooled);
+    bp.relu = has_relu(layers, n_layers, i);
     bp.wide = wide;
-    char *const which = ly.pool == 1 && train && i + 1 > first ? keep + sp.l[i + 1].which_off : nullptr;
-    const bool pool_after = ly.pool == 1 && !bp.pool;
+    char *const which = pooled && train && i + 1 > first ? keep + sp.l[i + 1].which_off : nullptr;
+    const bool pool_after = pooled && !bp.pool;
     char *to = last ? (char *)out : pool_after ? ws + sp.f_unpooled : input_of(i + 1);
     const BlockGemmArgs args = {input_of(i), ws + frag_off[i], ly.bias, to, (float *)(ws + sp.f_sums), !last, false, nullptr, nullptr, which};
     e = launch_block_gemm(bp, args, st);
@@ -2416,7 +2423,7 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
     const mellin_stack_layer &ly = layers[i];
     const void *w = wide ? ly.weight_half : ly.weight;
     if (!w) return fail(MELLIN_ERR_ARGUMENT, "%s: null pointer", __func__);
-    plan_block_input(kind_x, half, STACK_DIMS(ly), ip, layers[i - 1].pool ? layers[i - 1].dims[8] : 0);
+    plan_block_input(kind_x, half, STACK_DIMS(ly), ip, pooled_cols(layers, n_layers, i));
     filters[n_filters++] = pack_filter(ip, (int)ly.dims[2], w, ws + sp.l[i].frag_off, nullptr, 0);
   }
   const int top = n_layers - 1;
@@ -2430,14 +2437,14 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
     return r;
   };
   const StackLayer &lt = sp.l[top];
-  const PackSignal go = {grad_out, layers[top].pool == MELLIN_STACK_NO_RELU ? nullptr : out, ws + sp.b_grad[top & 1], (float *)take(lt.bias_bytes), (int)lt.batch, (int)lt.c_out, (int)lt.q};
+  const PackSignal go = {grad_out, has_relu(layers, n_layers, top) ? out : nullptr, ws + sp.b_grad[top & 1], (float *)take(lt.bias_bytes), (int)lt.batch, (int)lt.c_out, (int)lt.q};
   hipError_t e = launch_block_pack(half, &go, nullptr, filters, n_filters, st);
   if (layers[top].grad_bias) fin.add_bias(go.partial, (i64)pack_partial_count(lt.batch, 1, lt.q), lt.c_out, layers[top].grad_bias);
   for (int i = top; i >= std::max(lowest, 1) && e == hipSuccess; --i) {
     const mellin_stack_layer &ly = layers[i];
     const StackLayer &l = sp.l[i];
     const int here = i & 1, below = here ^ 1;
-    const bool first_dense = i == 1, pooled = layers[i - 1].pool;
+    const bool first_dense = i == 1, pooled = pools(layers, n_layers, i - 1);
     const bool go_on = i > lowest;
     BlockWgradPlan wp;
     if (ly.grad_weight) plan_block_weight(kind_x, half, STACK_DIMS(ly), wp);
@@ -2454,7 +2461,7 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
     float *const bias_below = go_on ? (float *)take(bias_bytes) : nullptr;
     i64 bias_count = 0;
     if (go_on) {
-      plan_block_input(kind_x, half, STACK_DIMS(ly), ip, pooled ? layers[i - 1].dims[8] : 0);
+      plan_block_input(kind_x, half, STACK_DIMS(ly), ip, pooled_cols(layers, n_layers, i));
       ip.relu = 0;
       const BlockGemmArgs args = {ws + sp.b_grad[here], ws + l.frag_off, nullptr, first_dense ? ws + sp.b_first : ws + sp.b_grad[below],
                                   (float *)(ws + sp.b_sums), !first_dense, true, keep + l.x_off, bias_below,

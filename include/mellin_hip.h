@@ -481,11 +481,11 @@ int mellin_layer_backward_kept(int kind_x, int elem_bytes, int want, const void 
 /* A stack of layers, each followed by a ReLU, in one call per direction.  Between layers the tensors stay in the layout of
  * the matrix kernels (channel-blocked), so nothing is laid out anew, and the backward of the ReLUs, the bias gradients and
  * the pooling ride along with the kernels.  Layer i reads what layer i - 1 leaves: dims are those of MELLIN_CORR2D_DIMS, in
- * order; with `pool` its output is first reduced to the maxima of pairs of neighbouring columns (y axis, an odd last one is
- * dropped; not after the first layer or the last).  pool = MELLIN_STACK_NO_RELU: the last layer, an output layer, has no ReLU
- * behind it.  elem_bytes as for a layer; weight_half: where the forward call leaves a
- * float weight rounded to half, which the backward call takes (MELLIN_ELEM_HALF_FLOAT in training; null otherwise);
- * grad_weight, grad_bias: null for gradients that are not wanted.
+ * order; where `pool` is not 0 its output is first reduced to the maxima of pairs of neighbouring columns (y axis, an odd last
+ * one is dropped; not after the first layer or the last).  The last layer's pool = MELLIN_STACK_NO_RELU: it is an output layer,
+ * with no ReLU behind it; 0 otherwise.  elem_bytes as for a layer; weight_half: where the forward call leaves a float weight
+ * rounded to half, which the backward call takes (MELLIN_ELEM_HALF_FLOAT in training; null otherwise); grad_weight, grad_bias:
+ * null for gradients that are not wanted.
  * mellin_stack_bytes: 1 if the stack can be run so under the settings in force, 0 if not (layers with too few channels for
  * the blocked kernels behind the first: call them one by one), and the bytes of `saved` (what the forward call keeps: for
  * the backward call, with train), of the forward call's workspace and of the backward call's; all 256-byte aligned.

@@ -366,7 +366,8 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
     room = 53 * 1024;
     stages[pl.mt - 1][at].rows = -1;
     const bool fits = shape(at), large = (pl.G == g && 2 * pl.F * pl.G >= fg) || (2 * pl.G >= g && 5 * pl.F * pl.G >= 3 * fg);
-    if (!fits || !(large || (f16 && !mellin))) pl = best_plan;
+    const bool dealt = pl.rest == 0 || pl.slices <= pl.CG / pl.G;        // (a slice is a stage or more)
+    if (!fits || !dealt || !(large || (f16 && !mellin))) pl = best_plan;
   }
   if (!f16 && pl.mt == 2 && pl.nt == 1 && pl.wk == 1) {
     // fp32, 64 channels x 128 positions: two by two wavefronts of 32 channels x 64 positions.  Four side by side take each

@@ -1,5 +1,6 @@
 """Which tiles the blocked kernels take for a pass (`mellin_layer_plan`; the plans are made on the host)."""
 import ctypes
+import random
 import time
 
 import pytest
@@ -105,3 +106,28 @@ def test_new_sizes_are_planned_in_little_time():
         assert hip.lib.mellin_stack_bytes(hip.AX_MCORR, 4, 1, params.layers, ctypes.cast(layers, ctypes.c_void_p), *map(ctypes.byref, sizes))
         times.append(time.perf_counter() - begin)
     assert sorted(times)[len(times) // 4] < 3e-4, sorted(times)
+
+
+def test_every_slice_has_a_stage():
+    """A slice without channels would still run a stage, on channels that are another's."""
+    rng = random.Random(9970)
+    size = lambda low, high: int(round(low * (high / low) ** rng.random()))      # noqa: E731
+    seen = {"slices": 0, "gradients by shared tiles": 0}
+    for _ in range(4000):
+        kind, c_in, c_out, batch = rng.choice((hip.AX_MCORR, hip.AX_LCORR)), size(8, 700), size(8, 700), size(1, 32)
+        kx, ky, x, y = rng.randint(1, 8), rng.randint(1, 4), size(5, 800), rng.choice((1, 2, 5, 10, 41))
+        d, p = rng.choice((1, 1, 2)), rng.randint(0, 3)
+        valid = mconv.mcorr_valid_size if kind == hip.AX_MCORR else mconv.lcorr_valid_size
+        ox, oy = valid(kx, x, 1, d, p) + (0 if kind == hip.AX_MCORR else p), mconv.lcorr_valid_size(ky, y, 1, 1, ky // 2) + ky // 2
+        if ox < 1 or oy < 1:
+            continue
+        dims = [batch, c_in, c_out, kx, ky, x, y, ox, oy, 1, 1, d, 1, p, ky // 2, 1, 1]
+        for elem_bytes in (4, 2):
+            for gradient in (0, 1, 2):
+                got = plan(kind, elem_bytes, gradient, dims)
+                if got and got["rest"]:
+                    groups = (c_out if gradient == 1 else c_in) + 7 >> 3
+                    assert groups % got["G"] == 0 and 1 <= got["slices"] <= groups // got["G"], (dims, elem_bytes, gradient, got)
+                    seen["slices"] += 1
+                    seen["gradients by shared tiles"] += gradient == 1 and got["wk"] > 1
+    assert all(n > 200 for n in seen.values()), seen

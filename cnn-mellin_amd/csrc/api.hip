@@ -1787,7 +1787,8 @@ int mellin_layer_plan(int kind_x, int elem_bytes, int gradient, MELLIN_CORR2D_DI
 // A training step's weight gradient reads the blocked input that the forward pass has made, and makes it again if nobody
 // kept it: a pass that reads the tensor and writes it once or, in fp32, one and a half times.  128 -> 256 channels, 3 x 3 taps,
 // 32 x 256 x 41, us a step: half on Mellin rows 567 -> 498, fp32 linear 3139 -> 3045.  Up to 256 MiB, which the graph then holds
-// beside the input between the two calls (the backward call had as much as scratch memory).  From 4 MiB: smaller ones are
+// beside the input between the two calls (the backward call had as much as scratch memory, one layer at a time: a caller of
+// many layers bounds what they keep in sum).  From 4 MiB: smaller ones are
 // blocked beside grad_out, in a launch that is made anyway, within its 7 us, and their steps wait for the host (41 -> 128
 // channels, 8 taps, 32 x 780: fp32, 7 MB, 83.7 -> 82.9; half, 2 MB, no difference).
 constexpr size_t kLeastKeptBytes = (size_t)4 << 20, kMostKeptBytes = (size_t)256 << 20;
@@ -1939,7 +1940,7 @@ static void plan_layer_backward(int kind_x, int elem_bytes, int want, MELLIN_COR
   if (wi && !lb.input_blocked)
     pass = std::max(pass, half ? mellin_corr2d_backward_input_f16_workspace(kind_x, CORR2D_ARGS) : input_workspace(kind_x, CORR2D_ARGS, &which));
   lb.weight_first = which == IN_TAPS || which == IN_TWO_PASS;
-  // (float: beside the input gradient's, whose last launch also ends the weight gradient)
+  // (float: beside the input gradient's, whose last launch also ends the weight gradient: 13 MB more at most, of 300 drawn layers)
   lb.weight_bytes = !ww || lb.weight_blocked ? 0 : half ? mellin_corr2d_backward_weight_f16_workspace(kind_x, CORR2D_ARGS)
                                                         : mellin_corr2d_backward_weight_workspace(kind_x, elem, CORR2D_ARGS);
   const bool together = !half && wi && !lb.input_blocked && lb.weight_bytes > 0;

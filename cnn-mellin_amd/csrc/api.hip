@@ -1706,32 +1706,48 @@ static bool blocks_apply(int pass, int kind_x, bool half, MELLIN_CORR2D_DIMS) {
 // (pooled: pairs of the output's columns are pooled behind the layer, by the kernel if the plan's `pool` says so)
 static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp, bool pooled = false) {
   if (!blocks_apply(PASS_FORWARD, kind_x, half, CORR2D_ARGS)) return false;
-  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS, pooled);
-  if (!lp.known[0]) {
+  LayerPlans *lp = &layer_plans(kind_x, half, CORR2D_ARGS, pooled);
+  if (!lp->known[0]) {
     SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
     pr.out_half = half;
-    bool applies = make_block_plan(pr, half, false, BlockPool{}, nullptr, bp);
-    lp.forward = bp;
-    if (applies && pooled) {
-      pr.y.nh -= pr.y.nh & 1;
-      if (!make_block_plan(pr, half, false, BlockPool{1, (int)nhy}, &bp, lp.forward)) lp.forward = bp;
+    bool applies;
+    if (pooled) {                                      // from the plan without pooling, which an equal layer may have
+      applies = plan_block_forward(kind_x, half, CORR2D_ARGS, bp);
+      lp = &layer_plans(kind_x, half, CORR2D_ARGS, pooled);      // (which may have taken the place)
+      lp->forward = bp;
+      const BlockPool pool = {1, (int)nhy};
+      if (applies && !(nhy % 2 == 0 && pool_block_plan(pool, lp->forward))) {
+        pr.y.nh -= nhy % 2;
+        if (!make_block_plan(pr, half, false, pool, &bp, lp->forward)) lp->forward = bp;
+      }
+    } else {
+      applies = make_block_plan(pr, half, false, BlockPool{}, nullptr, lp->forward);
     }
-    lp.known[0] = applies ? 1 : -1;
+    lp->known[0] = applies ? 1 : -1;
   }
-  if (lp.known[0] > 0) bp = lp.forward;
-  return lp.known[0] > 0;
+  if (lp->known[0] > 0) bp = lp->forward;
+  return lp->known[0] > 0;
 }
 // (pooled_cols: the columns that were pooled into the layer's input, or 0)
 static bool plan_block_input(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp, i64 pooled_cols = 0) {
   if (!blocks_apply(PASS_INPUT, kind_x, half, CORR2D_ARGS)) return false;
-  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS, pooled_cols ? 2 + 4 * (pooled_cols & 1) : 0);
-  if (!lp.known[1]) {
-    SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
-    pr.out_half = half;
-    lp.known[1] = make_block_plan(pr, half, true, BlockPool{pooled_cols ? 2 : 0, (int)pooled_cols}, nullptr, lp.input) ? 1 : -1;
+  const int key = pooled_cols ? 2 + 4 * (pooled_cols & 1) : 0;
+  LayerPlans *lp = &layer_plans(kind_x, half, CORR2D_ARGS, key);
+  if (!lp->known[1]) {
+    const BlockPool pool = {pooled_cols ? 2 : 0, (int)pooled_cols};
+    bool applies = pooled_cols && plan_block_input(kind_x, half, CORR2D_ARGS, bp);
+    lp = &layer_plans(kind_x, half, CORR2D_ARGS, key);            // (which may have taken the place)
+    if (applies) lp->input = bp;
+    if (!applies || !pool_block_plan(pool, lp->input)) {
+      SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
+      pr.out_half = half;
+      lp->input = BlockPlan{};
+      applies = make_block_plan(pr, half, true, pool, nullptr, lp->input);
+    }
+    lp->known[1] = applies ? 1 : -1;
   }
-  if (lp.known[1] > 0) bp = lp.input;
-  return lp.known[1] > 0;
+  if (lp->known[1] > 0) bp = lp->input;
+  return lp->known[1] > 0;
 }
 static bool plan_block_weight(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockWgradPlan &wp) {
   if (!blocks_apply(PASS_WEIGHT, kind_x, half, CORR2D_ARGS)) return false;

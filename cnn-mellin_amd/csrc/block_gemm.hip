@@ -88,15 +88,14 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
   if (pl.nfy > 64) return false;
   // A pooled output's sums keep the order of the unpooled one's, which decides what its ReLU lets through (see can_join), and
   // are those of the layer called by itself bit for bit: the same channel groups and filter columns to a stage, the same
-  // slices.  An even number of columns makes the same tiles of them (one utterance of a ten-layer Mellin stack, whose wavefronts
-  // share tiles: 212 -> 207 us with two of its three poolings inside the products).  An odd last column is in no tile, so these hold other
+  // slices.  An even number of columns makes the same tiles of them (pool_block_plan; one utterance of a ten-layer Mellin stack,
+  // whose wavefronts share tiles: 212 -> 207 us with two of its three poolings inside the products).  An odd last column, as
+  // here, is in no tile, so these hold other
   // positions than without the pooling, and the order must not depend on what a tile holds: not on its being one of those in
   // slices, nor, on Mellin axes, on the filter rows of its other output rows -- they shift the pairs that share a step where a
   // row's taps and groups are odd in number, and the steps that wavefronts share.
-  const bool same_tiles = like && like->noy == pl.noy;
-  if (like && (like->nfy != pl.nfy || like->f_off != pl.f_off)) return false;
-  if (like && !same_tiles && ((like->whole && like->rest) ||
-                              ((X.kind == AX_MCORR || X.kind == AX_MCONV) && (like->wk > 1 || like->nfy * like->G % 2))))
+  if (like && (like->nfy != pl.nfy || like->f_off != pl.f_off || (like->whole && like->rest) ||
+               ((X.kind == AX_MCORR || X.kind == AX_MCONV) && (like->wk > 1 || like->nfy * like->G % 2))))
     return false;
   const i64 py = Y.p - Y.d * fy_lo;
   pl.ay = (int)Y.s; pl.by = Y.kind == AX_LCORR ? (int)Y.d : -(int)Y.d; pl.cy = Y.kind == AX_LCORR ? -(int)py : (int)py;
@@ -284,7 +283,7 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
     };
     double best = 9000 + turns_cost(total, c_stages * subsets);
     pl.slices = like ? like->slices : 1;
-    int rest = !like || !like->rest ? 0 : same_tiles ? like->rest : total;
+    int rest = !like || !like->rest ? 0 : total;
     for (int all = 0; all < (like ? 0 : 2); ++all) {
       const int r = all ? total : total % per_m;
       if (r == 0 || (all && total >= 2 * per_m) || (pl.wk > 1 && !all)) continue;
@@ -397,6 +396,16 @@ bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool
   pl.rows_off = (size_t)pl.m_tiles * pl.wm * pl.mt * ((size_t)pl.CG * pl.nfx * pl.nfy + 1) * parts * 512;
   if (pl.rows_off >= (size_t)lim) return false;
   pl.filter_bytes = pl.rows_off + (mellin ? 8 * (size_t)pl.nox : 0);
+  return true;
+}
+
+bool pool_block_plan(const BlockPool &pool, BlockPlan &pl) {
+  const i64 out_q = pool.kind == 1 ? pl.Q / 2 : (i64)pl.nox * pool.cols, most = (i64)1 << 31;
+  if (pl.out_groups * (out_q + 1) * 48 >= most) return false;    // (32-bit byte offsets, as make_block_plan)
+  if (pl.joint && pl.batch * pl.out_groups * (out_q + 1) * (pl.f16 ? 16 : 48) >= most) return false;
+  pl.pool = pool.kind;
+  pl.out_q = (int)out_q;
+  pl.out_cols = pool.cols;
   return true;
 }
 

@@ -77,6 +77,9 @@ struct BlockPool { int kind, cols; };  // kind: 0 no pooling, 1 forward, 2 input
 // False: the kernel does not apply.  gradient: of an input (a forward pass has no joint tiles).  `like`: the plan of the same
 // layer without the pooling, whose order of sums is kept (false as well where that cannot be).
 bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool &pool, const BlockPlan *like, BlockPlan &pl);
+// A plan without pooling as that of the same pass beside it (a forward pass: of an even number of columns): tiles and sums are
+// the same.  False: the tensor in front of the pooling is too large for it.
+bool pool_block_plan(const BlockPool &pool, BlockPlan &pl);
 // out = [relu](bias + sum) from a blocked signal and packed filter; bias (fp32 / half, or null), relu as the plan says.
 // With `grad`, the input gradient of a layer behind a ReLU: zero where `mask`, the blocked output of that ReLU, is not
 // positive; its sums over the positions go to chan_sums ([channel][pl.chan_slots]: partial sums for launch_block_finish).

@@ -131,3 +131,22 @@ def test_every_slice_has_a_stage():
                     seen["slices"] += 1
                     seen["gradients by shared tiles"] += gradient == 1 and got["wk"] > 1
     assert all(n > 200 for n in seen.values()), seen
+
+
+@pytest.mark.parametrize("elem_bytes", [4, 2])
+def test_pooled_passes_of_even_columns_have_the_layers_own_plan(elem_bytes):
+    """Such a plan is taken from the one without pooling, not made again."""
+    params = ConvStackParams(layers=10, kernel_time=4, kernel_freq=4, initial_channels=32, factor_schedule=3, channel_factor=2,
+                             time_factor=1, in_channels=3)
+    for mellin in (True, False):
+        params.mellin = mellin
+        kind, pooled = hip.AX_MCORR if mellin else hip.AX_LCORR, 0
+        for batch, frames, bins in ((1, 337, 40), (32, 780, 20), (3, 100, 10), (7, 61, 2)):
+            for dims in list(stack_dims(batch, frames, bins, params))[1:]:
+                if dims[8] % 2:
+                    continue
+                words = [(ctypes.c_int * len(WORDS))() for _ in range(2)]
+                took = [hip.lib.mellin_layer_plan(kind, elem_bytes, gradient, *dims, w) for gradient, w in zip((0, 2), words)]
+                assert took[0] == (took[1] > 0) and list(words[0]) == list(words[1])
+                pooled += took[1] == 2
+        assert pooled

@@ -93,6 +93,8 @@ SYMBOLS["mellin_layer_forward_kept"] = (_int, [_int, _int, _int, _ptr, _ptr, _pt
 SYMBOLS["mellin_layer_backward_kept_workspace"] = (_size_t, [_int, _int, _int] + _DIMS)
 SYMBOLS["mellin_layer_backward_kept"] = (_int, [_int, _int, _int] + [_ptr] * 4 + _DIMS + [_ptr] * 5 + [_size_t, _ptr])
 SYMBOLS["mellin_layer_plan"] = (_int, [_int, _int, _int] + _DIMS + [_ptr])
+SYMBOLS["mellin_layer_stages"] = (_int, [_int, _int, _int] + _DIMS + [_ptr])
+SYMBOLS["mellin_layer_weight_sums"] = (_int, [_int, _int] + _DIMS + [_ptr])
 SYMBOLS["mellin_layer_bias_route"] = (_int, [_int, _int, _int] + _DIMS)
 SYMBOLS["mellin_stack_first_layer"] = (_int, [_int, _int] + _DIMS)
 SYMBOLS["mellin_stack_bytes"] = (_int, [_int, _int, _int, _int] + [_ptr] * 4)

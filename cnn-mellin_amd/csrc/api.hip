@@ -1800,6 +1800,28 @@ int mellin_layer_plan(int kind_x, int elem_bytes, int gradient, MELLIN_CORR2D_DI
   return bp.pool ? 2 : 1;
 }
 
+int mellin_layer_stages(int kind_x, int elem_bytes, int gradient, MELLIN_CORR2D_DIMS, int *words) {
+  if (!words || !layer_elements(elem_bytes) || check_corr2d(__func__, kind_x, CORR2D_ARGS)) return 0;
+  BlockPlan bp;
+  if (!(gradient ? plan_block_input(kind_x, elem_bytes != 4, CORR2D_ARGS, bp) : plan_block_forward(kind_x, elem_bytes != 4, CORR2D_ARGS, bp))) return 0;
+  for (int n = 0; n < MELLIN_LAYER_STAGE_WORDS - 1; ++n) words[n] = bp.stage[std::min(n, bp.F - 1)].G;
+  words[MELLIN_LAYER_STAGE_WORDS - 1] = (int)bp.lds_bytes;
+  return 1;
+}
+int mellin_layer_weight_sums(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS, int *words) {
+  BlockWgradPlan wp;
+  if (!words || !layer_elements(elem_bytes) || check_corr2d(__func__, kind_x, CORR2D_ARGS) ||
+      !plan_block_weight(kind_x, elem_bytes != 4, CORR2D_ARGS, wp))
+    return 0;
+  BlockFinish fin = {};
+  fin.add_weight(wp, nullptr, nullptr);
+  words[0] = fin.weight[0].tap_chunk;
+  words[1] = fin.weight[0].parts;
+  words[2] = (int)fin.weight[0].blocks;
+  words[3] = (int)fin.weight[0].zero_blocks;
+  return 1;
+}
+
 // A training step's weight gradient reads the blocked input that the forward pass has made, and makes it again if nobody
 // kept it: a pass that reads the tensor and writes it once or, in fp32, one and a half times.  128 -> 256 channels, 3 x 3 taps,
 // 32 x 256 x 41, us a step: half on Mellin rows 567 -> 498, fp32 linear 3139 -> 3045.  Up to 256 MiB, which the graph then holds

@@ -518,6 +518,14 @@ int mellin_stack_backward(int kind_x, int elem_bytes, int n_layers, const mellin
  * of a stage, tiles that a workgroup makes whole, tiles whose channels are dealt to several, to how many}. */
 #define MELLIN_LAYER_PLAN_WORDS 10
 int mellin_layer_plan(int kind_x, int elem_bytes, int gradient, MELLIN_CORR2D_DIMS, int *plan);
+/* More of such a plan: channel groups of a stage of a tile with one, two, .. sixteen filter rows (Mellin axes; tiles that a
+ * workgroup makes whole), and the LDS bytes of a workgroup. */
+#define MELLIN_LAYER_STAGE_WORDS 17
+int mellin_layer_stages(int kind_x, int elem_bytes, int gradient, MELLIN_CORR2D_DIMS, int *words);
+/* How the partial sums of a layer's weight gradient are added up: 0 if the blocked kernels do not make it, else 1 and words =
+ * {taps of a block of threads, parts that a tap's slices are added in, blocks, blocks for filter columns without a tap}. */
+#define MELLIN_LAYER_WEIGHT_SUMS_WORDS 4
+int mellin_layer_weight_sums(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS, int *words);
 
 /* Where a layer's backward call makes the bias gradient for `want` (for tests): nowhere (not wanted), in launches of its own,
  * beside the weight gradient, in the pass that lays grad_out out for the blocked kernels. */

@@ -1,12 +1,14 @@
 """The sums that make a weight gradient of its workgroups' partial ones (`block_finish.hip`), where a block of threads takes all
 taps of its channels, some of them, or one; where the taps or the input channels do not fill the last block; where filter columns
 without a tap are left to zeros: against float64."""
+import ctypes
+
 import pytest
 import torch
 
+import _mellin_hip as hip
 import mconv
-
-pytestmark = pytest.mark.gpu
+from test_gpu_kept_inputs import dims_of
 
 CASES = [
     # channels in and out, kernel, input size, s, d, p, r, batch
@@ -18,11 +20,36 @@ CASES = [
     (256, 128, (3, 3), (20, 20), (1, 1), (2, 1), (2, 1), (2, 1), 2),   # all nine taps a block
     (512, 40, (8, 4), (20, 10), (1, 1), (1, 1), (3, 1), (3, 1), 2),    # 32 taps: a part
     (513, 33, (9, 4), (20, 10), (1, 1), (1, 1), (3, 1), (3, 1), 2),    # more taps than a block has threads for
-    (40, 48, (3, 5), (30, 2), (1, 1), (1, 1), (1, 2), (1, 2), 3),      # columns 0 and 4 of five meet padding only in part
+    (40, 48, (3, 5), (30, 2), (1, 1), (1, 1), (1, 2), (1, 2), 3),      # columns 0 and 4 of five meet padding only
     (24, 40, (3, 4), (30, 1), (1, 1), (1, 1), (1, 1), (1, 1), 3),      # filter columns without a tap
 ]
 
+# taps of a block of threads; whether there are filter columns without a tap
+ROUTES = [({1}, False), ({4}, False), ({1}, False), ({2}, False), ({5, 9}, False), ({9}, False), ({32}, False), ({32}, False),
+          ({1}, True), ({1}, True)]
 
+
+def test_cases_have_the_blocks_that_they_are_there_for():
+    for (ci, co, kernel, size, s, d, p, r, batch), (chunks, columns) in zip(CASES, ROUTES):
+        seen = set()
+        for cls in (mconv.MCorrLCorr, mconv.LCorrLCorr):
+            kind, dims = dims_of((cls, ci, co, kernel, size, s, d, p, r, batch))
+            for elem_bytes in (4, 2):
+                words = (ctypes.c_int * 4)()
+                assert hip.lib.mellin_layer_weight_sums(kind, elem_bytes, *dims, words)
+                chunk, parts, blocks, zeros = words
+                seen.add(chunk)
+                assert parts == 32 // chunk and blocks == co * -(-ci // 32) * -(-kernel[0] * live(kernel, size, s, d, p, dims) // chunk)
+                assert (zeros > 0) == columns
+        assert seen == chunks
+
+
+def live(kernel, size, s, d, p, dims):
+    """Filter columns with a tap."""
+    return sum(any(0 <= s[1] * oy + d[1] * fy - p[1] < size[1] for oy in range(dims[8])) for fy in range(kernel[1]))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("mellin", [False, True])
 @pytest.mark.parametrize("case", CASES, ids=range(len(CASES)))

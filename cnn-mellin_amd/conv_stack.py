@@ -242,13 +242,13 @@ class FrameClassifier(torch.nn.Module):
         Mellin layers (5 bins behind the last) 3690 -> 3435, linear ones (1 bin) 2854 -> 2700; eight other half stacks 0.90 to
         1.00 up to 6 bins.  Its input gradient multiplies all bins' taps, of which one meets a frame: at 10 bins 1.00 to 1.02, and
         in float32, where a product costs six times as much, nothing is left at 5 either."""
+        # (what no call of this module can change comes first, and in front of the walk over the layers, which the stack makes
+        # again: 5 us of the 105 that a call with 41 bins and seven layers takes the host)
+        stack = self._modules["stack"]
+        if type(stack) is not ConvStack or stack.plan[-1]["out_size"][1] > _JOIN_BINS or len(stack.plan) < 2:
+            return None
         half = torch.get_autocast_dtype("cuda") == torch.float16 if torch.is_autocast_enabled("cuda") else x.dtype == torch.float16
         if not (half and x.is_cuda and x.dim() == 4):
-            return None
-        # (what no call of this module can change comes in front of the walk over the layers, which the stack makes again:
-        # 5 us of the 105 that a call with 41 bins and seven layers takes the host)
-        stack = self.stack
-        if type(stack) is not ConvStack or stack.out_size[1] > _JOIN_BINS or len(stack.convs) < 2:
             return None
         out = self.out
         if not (_unhooked(stack, ConvStack) and _unhooked(out, torch.nn.Linear) and

@@ -1826,10 +1826,11 @@ int mellin_layer_weight_sums(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS, int
 // kept it: a pass that reads the tensor and writes it once or, in fp32, one and a half times.  128 -> 256 channels, 3 x 3 taps,
 // 32 x 256 x 41, us a step: half on Mellin rows 567 -> 498, fp32 linear 3139 -> 3045.  Up to 256 MiB, which the graph then holds
 // beside the input between the two calls (the backward call had as much as scratch memory, one layer at a time: a caller of
-// many layers bounds what they keep in sum).  From 4 MiB: smaller ones are
-// blocked beside grad_out, in a launch that is made anyway, within its 7 us, and their steps wait for the host (41 -> 128
-// channels, 8 taps, 32 x 780: fp32, 7 MB, 83.7 -> 82.9; half, 2 MB, no difference).
-constexpr size_t kLeastKeptBytes = (size_t)4 << 20, kMostKeptBytes = (size_t)256 << 20;
+// many layers bounds what they keep in sum).  From 10 MiB: smaller ones are
+// blocked beside grad_out, in a launch that is made anyway, and their steps wait for the host, which what is kept takes another
+// allocation and a few look-ups (seventeen layers, a step without over one with: 0.94 to 0.99 from 4 to 10 MB, 1.01 at 11, 1.02 to
+// 1.07 from 12 MB on).
+constexpr size_t kLeastKeptBytes = (size_t)10 << 20, kMostKeptBytes = (size_t)256 << 20;
 size_t mellin_layer_kept_bytes(int kind_x, int elem_bytes, MELLIN_CORR2D_DIMS) {
   const bool half = elem_bytes != 4;
   if (batch < 1 || c_in < 1 || ngx < 1 || ngy < 1 || batch > 65535 || c_in > 1 << 24 || ngx > 1 << 22 || ngy > 1 << 22) return 0;

@@ -8,10 +8,10 @@ import mconv
 
 CASES = [
     # (module, channels in and out, kernel, input size, s, d, p, r, batch)
-    (mconv.MCorr1d, 41, 128, 8, (391,), 1, 1, 3, 0, 128),
-    (mconv.LCorr1d, 17, 33, 3, (1001,), 2, 2, 1, 1, 96),
-    (mconv.MCorrLCorr, 64, 40, (3, 3), (31, 11), (1, 1), (2, 1), (2, 1), (2, 1), 101),
-    (mconv.LCorrLCorr, 16, 96, (5, 3), (33, 37), (1, 1), (1, 1), (2, 1), (2, 1), 111),
+    (mconv.MCorr1d, 41, 128, 8, (391,), 1, 1, 3, 0, 300),
+    (mconv.LCorr1d, 17, 33, 3, (1001,), 2, 2, 1, 1, 300),
+    (mconv.MCorrLCorr, 64, 40, (3, 3), (31, 11), (1, 1), (2, 1), (2, 1), (2, 1), 300),
+    (mconv.LCorrLCorr, 16, 96, (5, 3), (33, 37), (1, 1), (1, 1), (2, 1), (2, 1), 300),
 ]
 
 
@@ -39,7 +39,7 @@ def test_what_is_kept_leaves_the_scratch_memory(case, elem_bytes):
     few = list(dims)
     few[1] = 3                                         # section 2's forward pass
     assert hip.lib.mellin_layer_kept_bytes(kind, elem_bytes, *few) == 0
-    for batch in (-(-(n << 28) // kept) + 1, (n << 22) // kept - 1):           # more than 256 MiB, less than 4
+    for batch in (-(-(n << 28) // kept) + 1, n * (10 << 20) // kept - 1):           # more than 256 MiB, less than 10
         assert hip.lib.mellin_layer_kept_bytes(kind, elem_bytes, batch, *dims[1:]) == 0
 
 

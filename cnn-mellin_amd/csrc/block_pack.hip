@@ -22,13 +22,14 @@ namespace {
 
 constexpr int kPackThreads = 256;
 constexpr int kPackPositions = 4;                  // per thread at most
-// Positions that a thread takes one after the other.  Without sums: one in fp32 (us: 128 channels of 32 x 256 x 41,
-// averaged with 256 that have sums, 154.9 -> 143), and in half one where four would
-// leave fewer than kPackBlocks blocks, each of which waits for memory as often as it has positions (33 half channels of
-// 7 x 333 x 37, 455 blocks of four, 11.6 -> 9.5); with more blocks than fill the chip, half blocks of one position lose (128
-// channels of 32 x 256 x 41 and 256 of 32 x 194 x 41, 5600 and 8200 blocks, 49.2 -> 71.4 on average).  With sums: four, the
-// order of sums that gives a bias gradient the same bits whether the input gradient is asked for beside it or not.
-constexpr i64 kPackBlocks = 1024;
+// Positions that a thread takes one after the other, by the blocks that four would leave (30 signals each, 33 to 128 channels, us
+// with four over us with one).  Few blocks wait for memory as often as they have positions: one in half below 1024 blocks
+// (1.02 to 1.38 up to 780 of them; 0.97 to 1.04 from 1040 to 1280, 0.74 to 1.02 from 1560 to 19200: 128 channels of 32 x 256 x
+// 41, 44.2 and 45.8) and in fp32 below 512 (0.98 to 1.12).  From there to the 2048 blocks that the chip holds at a time, four in
+// fp32 (0.77 to 1.05); beyond, one, whose last round leaves less of the chip empty (1.05 to 1.46: 128 channels of 32 x 256 x 41,
+// 104 and 81).  With sums: four, the order of sums that gives a bias gradient the same bits whether the input gradient is asked
+// for beside it or not.
+constexpr i64 kHalfBlocks = 1024, kFloatBlocks = 512, kResidentBlocks = 2048;
 
 struct PackPart {                                  // a signal, dealt to blocks as (image, group, chunk of its plane)
   PackSignal s;
@@ -214,7 +215,8 @@ __global__ __launch_bounds__(kPackThreads) void block_pack_kernel(PackArgs<FILTE
 i64 pack_chunks(i64 plane, int positions) { return plane / (kPackThreads * positions) + 1; }     // (plane + 1 units)
 int pack_positions(bool half, const PackSignal &s, int groups) {
   if (s.partial) return kPackPositions;
-  return !half || (i64)s.batch * groups * pack_chunks(s.plane, kPackPositions) < kPackBlocks ? 1 : kPackPositions;
+  const i64 blocks = (i64)s.batch * groups * pack_chunks(s.plane, kPackPositions);
+  return blocks < (half ? kHalfBlocks : kFloatBlocks) || (!half && blocks >= kResidentBlocks) ? 1 : kPackPositions;
 }
 
 bool pack_part(bool half, const PackSignal *s, PackPart &pt) {

@@ -244,7 +244,7 @@ class FrameClassifier(torch.nn.Module):
         in float32, where a product costs six times as much, nothing is left at 5 either."""
         # (what no call of this module can change comes first, and in front of the walk over the layers, which the stack makes
         # again: 5 us of the 105 that a call with 41 bins and seven layers takes the host)
-        stack = self._modules["stack"]
+        stack = self._modules.get("stack")
         if type(stack) is not ConvStack or stack.plan[-1]["out_size"][1] > _JOIN_BINS or len(stack.plan) < 2:
             return None
         half = torch.get_autocast_dtype("cuda") == torch.float16 if torch.is_autocast_enabled("cuda") else x.dtype == torch.float16

@@ -1640,20 +1640,19 @@ enum FirstLayer { FIRST_OWN = MELLIN_FIRST_OWN, FIRST_BLOCKS = MELLIN_FIRST_BLOC
 struct FirstPlan { FirstLayer route; TilePlan tiles; size_t lds; int mt, nt; };
 // Plans of the layer entry points, kept per thread: a layer asks for the same ones with every step (its workspace, then
 // the launch), and choosing among tile shapes takes 0.5 to 4 microseconds a pass (ten Mellin layers of a new length: 17 served,
-// 32 to 55 with their gradients, in the caller's thread and again in autograd's).  The sizes decide the plan, so nothing has to
-// be thrown away.
+// 36 in fp32 and 51 in half with their gradients, in the caller's thread and again in autograd's).  The sizes decide the plan, so
+// nothing has to be thrown away.
 struct LayerPlans {
-  int known[5];                                        // 0 not yet, 1 applies, -1 does not
+  int known[6];                                        // 0 not yet, 1 applies, -1 does not
   int first_known;                                     // 0 not yet, else 1 + the math mode that `first` was made for
   FirstPlan first;
   size_t bias_bytes;                                   // section 2's weight gradient: for the bias gradient beside it (known[3])
-  BlockPlan forward, input;
+  BlockPlan forward, input, forward_pooled;            // (pooled: of an odd number of columns, known[5])
   BlockWgradPlan weight;
 };
-// (pool: a pass beside frequency pooling: the kind of BlockPool, and 4 for an odd number of columns in front of it)
-static LayerPlans &layer_plans(int kind_x, bool half, MELLIN_CORR2D_DIMS, int pool = 0) {
+static LayerPlans &layer_plans(int kind_x, bool half, MELLIN_CORR2D_DIMS) {
   static thread_local PlanTable<LayerPlans, 64, 18> table;
-  return table.at({pool * 16 + kind_x * 2 + half + 1, CORR2D_ARGS});
+  return table.at({kind_x * 2 + half + 1, CORR2D_ARGS});
 }
 // Layers with few channels leave most of a channel block empty, and have kernels of their own in section 2.  Measured over
 // 80 layers with 1 to 15 input channels: for the gradients of short layers, bound by launches (up to these
@@ -1706,48 +1705,37 @@ static bool blocks_apply(int pass, int kind_x, bool half, MELLIN_CORR2D_DIMS) {
 // (pooled: pairs of the output's columns are pooled behind the layer, by the kernel if the plan's `pool` says so)
 static bool plan_block_forward(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp, bool pooled = false) {
   if (!blocks_apply(PASS_FORWARD, kind_x, half, CORR2D_ARGS)) return false;
-  LayerPlans *lp = &layer_plans(kind_x, half, CORR2D_ARGS, pooled);
-  if (!lp->known[0]) {
+  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
+  auto make = [&](const BlockPool &pool, const BlockPlan *like, BlockPlan &plan) {
     SepConv pr = forward_problem(kind_x, CORR2D_ARGS);
     pr.out_half = half;
-    bool applies;
-    if (pooled) {                                      // from the plan without pooling, which an equal layer may have
-      applies = plan_block_forward(kind_x, half, CORR2D_ARGS, bp);
-      lp = &layer_plans(kind_x, half, CORR2D_ARGS, pooled);      // (which may have taken the place)
-      lp->forward = bp;
-      const BlockPool pool = {1, (int)nhy};
-      if (applies && !(nhy % 2 == 0 && pool_block_plan(pool, lp->forward))) {
-        pr.y.nh -= nhy % 2;
-        if (!make_block_plan(pr, half, false, pool, &bp, lp->forward)) lp->forward = bp;
-      }
-    } else {
-      applies = make_block_plan(pr, half, false, BlockPool{}, nullptr, lp->forward);
-    }
-    lp->known[0] = applies ? 1 : -1;
-  }
-  if (lp->known[0] > 0) bp = lp->forward;
-  return lp->known[0] > 0;
+    if (like) pr.y.nh -= 1;
+    return make_block_plan(pr, half, false, pool, like, plan) ? 1 : -1;
+  };
+  if (!lp.known[0]) lp.known[0] = make(BlockPool{}, nullptr, lp.forward);
+  if (lp.known[0] < 0) return false;
+  bp = lp.forward;
+  if (!pooled) return true;
+  const BlockPool pool = {1, (int)nhy};
+  if (nhy % 2 == 0) return pool_block_plan(pool, bp);
+  if (!lp.known[5]) lp.known[5] = make(pool, &lp.forward, lp.forward_pooled);
+  if (lp.known[5] > 0) bp = lp.forward_pooled;
+  return true;
 }
 // (pooled_cols: the columns that were pooled into the layer's input, or 0)
 static bool plan_block_input(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockPlan &bp, i64 pooled_cols = 0) {
   if (!blocks_apply(PASS_INPUT, kind_x, half, CORR2D_ARGS)) return false;
-  const int key = pooled_cols ? 2 + 4 * (pooled_cols & 1) : 0;
-  LayerPlans *lp = &layer_plans(kind_x, half, CORR2D_ARGS, key);
-  if (!lp->known[1]) {
-    const BlockPool pool = {pooled_cols ? 2 : 0, (int)pooled_cols};
-    bool applies = pooled_cols && plan_block_input(kind_x, half, CORR2D_ARGS, bp);
-    lp = &layer_plans(kind_x, half, CORR2D_ARGS, key);            // (which may have taken the place)
-    if (applies) lp->input = bp;
-    if (!applies || !pool_block_plan(pool, lp->input)) {
-      SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
-      pr.out_half = half;
-      lp->input = BlockPlan{};
-      applies = make_block_plan(pr, half, true, pool, nullptr, lp->input);
-    }
-    lp->known[1] = applies ? 1 : -1;
-  }
-  if (lp->known[1] > 0) bp = lp->input;
-  return lp->known[1] > 0;
+  LayerPlans &lp = layer_plans(kind_x, half, CORR2D_ARGS);
+  auto make = [&](const BlockPool &pool, BlockPlan &plan) {
+    SepConv pr = input_gather_problem(kind_x, CORR2D_ARGS);
+    pr.out_half = half;
+    return make_block_plan(pr, half, true, pool, nullptr, plan);
+  };
+  if (!lp.known[1]) lp.known[1] = make(BlockPool{}, lp.input) ? 1 : -1;
+  if (lp.known[1] < 0) return false;
+  bp = lp.input;
+  const BlockPool pool = {2, (int)pooled_cols};
+  return !pooled_cols || pool_block_plan(pool, bp) || (bp = BlockPlan{}, make(pool, bp));
 }
 static bool plan_block_weight(int kind_x, bool half, MELLIN_CORR2D_DIMS, BlockWgradPlan &wp) {
   if (!blocks_apply(PASS_WEIGHT, kind_x, half, CORR2D_ARGS)) return false;

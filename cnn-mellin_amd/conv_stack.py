@@ -16,6 +16,7 @@ layers.  Layers are this package's `MCorrLCorr` (Mellin x linear) or
 from typing import Callable, List, Optional, Sequence, Tuple
 
 import torch
+from torch.utils._device import DeviceContext
 
 import mconv
 import _mellin_hip as _hip
@@ -215,6 +216,12 @@ def _unhooked(module: torch.nn.Module, cls: type) -> bool:
                                         d["_backward_hooks"] or d["_backward_pre_hooks"])
 
 
+def _shown_to_modes() -> bool:
+    """Whether a function mode sees the calls one by one.  That of ``torch.device`` and ``torch.set_default_device`` is shown
+    nothing that it would change."""
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+
+
 #: A projection joins the stack's call up to this many bins (`FrameClassifier._scores`)
 _JOIN_BINS = 6
 
@@ -251,8 +258,7 @@ class FrameClassifier(torch.nn.Module):
         if not (half and x.is_cuda and x.dim() == 4):
             return None
         out = self.out
-        if not (_unhooked(stack, ConvStack) and _unhooked(out, torch.nn.Linear) and
-                stack._fused() and stack._plain()) or torch._C._len_torch_function_stack():  # (such modes see the projection)
+        if not (_unhooked(stack, ConvStack) and _unhooked(out, torch.nn.Linear) and stack._fused() and stack._plain()) or _shown_to_modes():
             return None
         bins, channels = stack.out_size[1], stack.out_channels
         weight = out.weight

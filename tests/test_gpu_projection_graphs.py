@@ -131,3 +131,14 @@ def test_stacks_that_are_not_joined_are_not_looked_through_twice(monkeypatch):
         with torch.no_grad(), torch.autocast("cuda", torch.float16):
             model(x)
         assert len(looked) == 1
+
+
+def test_default_devices_change_nothing():
+    model, x, labels, leaves = classifier(CASES[0], "autocast")
+    for context in (torch.device("cuda"), torch.device("cpu")):
+        with context, torch.autocast("cuda", torch.float16):
+            assert model._scores(x) is not None
+    with torch.autocast("cuda", torch.float16):
+        joined = model(x)
+        with torch.device("cpu"):
+            assert torch.equal(model(x), joined)

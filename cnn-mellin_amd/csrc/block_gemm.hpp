@@ -74,8 +74,9 @@ constexpr bool deep_fragments(bool f16, int wk) { return f16 && wk == 1; }
 // columns they were taken from (an odd last one of them: zeros).
 struct BlockPool { int kind, cols; };  // kind: 0 no pooling, 1 forward, 2 input gradient
 
-// False: the kernel does not apply.  gradient: of an input (a forward pass has no joint tiles).  `like`: the plan of the same
-// layer without the pooling, whose order of sums is kept (false as well where that cannot be).
+// False: the kernel does not apply.  gradient: of an input (a forward pass has no joint tiles).  `like`, for a pooled forward pass
+// without an odd last column: the plan of the same layer without the pooling, whose order of sums is kept (false as well where
+// that cannot be).
 bool make_block_plan(const SepConv &pr, bool f16, bool gradient, const BlockPool &pool, const BlockPlan *like, BlockPlan &pl);
 // A plan without pooling as that of the same pass beside it (a forward pass: of an even number of columns): tiles and sums are
 // the same.  False: the tensor in front of the pooling is too large for it.

@@ -222,8 +222,8 @@ def _shown_to_modes() -> bool:
     return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
 
 
-#: A projection joins the stack's call up to this many bins (`FrameClassifier._scores`)
-_JOIN_BINS = 6
+#: A projection joins the stack's call up to this many bins and classes (`FrameClassifier._scores`)
+_JOIN_BINS, _JOIN_CLASSES = 6, 256
 
 
 class FrameClassifier(torch.nn.Module):
@@ -248,16 +248,20 @@ class FrameClassifier(torch.nn.Module):
         back around PyTorch's products.  In half precision, us a step of ten layers, 3 -> 256 channels on 32 x 780 x 41:
         Mellin layers (5 bins behind the last) 3690 -> 3435, linear ones (1 bin) 2854 -> 2700; eight other half stacks 0.90 to
         1.00 up to 6 bins.  Its input gradient multiplies all bins' taps, of which one meets a frame: at 10 bins 1.00 to 1.02, and
-        in float32, where a product costs six times as much, nothing is left at 5 either."""
+        in float32, where a product costs six times as much, nothing is left at 5 either.  The layouts that it spares do not grow
+        with the classes, and PyTorch's product is the faster of the two: four stacks of two to four layers, 128 and 256 channels,
+        3 to 6 bins, 1 to 64 utterances of 780 frames, training and not: joined over apart 0.52 to 1.01 with 256 classes, 0.51 to
+        1.10 with 448, 0.55 to 1.32 with 1000, 0.68 to 2.06 with 4000."""
         # (what no call of this module can change comes first, and in front of the walk over the layers, which the stack makes
         # again: 5 us of the 105 that a call with 41 bins and seven layers takes the host)
-        stack = self._modules.get("stack")
+        stack, out = self._modules.get("stack"), self._modules.get("out")
         if type(stack) is not ConvStack or stack.plan[-1]["out_size"][1] > _JOIN_BINS or len(stack.plan) < 2:
+            return None
+        if type(out) is not torch.nn.Linear or out.out_features > _JOIN_CLASSES:
             return None
         half = torch.get_autocast_dtype("cuda") == torch.float16 if torch.is_autocast_enabled("cuda") else x.dtype == torch.float16
         if not (half and x.is_cuda and x.dim() == 4):
             return None
-        out = self.out
         if not (_unhooked(stack, ConvStack) and _unhooked(out, torch.nn.Linear) and stack._fused() and stack._plain()) or _shown_to_modes():
             return None
         bins, channels = stack.out_size[1], stack.out_channels

@@ -123,13 +123,14 @@ def test_stacks_that_are_not_joined_are_not_looked_through_twice(monkeypatch):
     looked = []
     plain = ConvStack._plain
     monkeypatch.setattr(ConvStack, "_plain", lambda self: looked.append(1) or plain(self))
-    for layers, bins in ((2, 7), (1, 5)):              # more than six bins; one layer
+    for layers, bins, classes in ((2, 7, 9), (1, 5, 9), (2, 5, 257)):              # more than six bins; one layer; many classes
         params = ConvStackParams(layers=layers, kernel_time=3, kernel_freq=3, initial_channels=32, factor_schedule=2, time_factor=1,
                                  in_channels=3)
-        model, x = FrameClassifier(ConvStack(40, bins, params), 9).cuda(), torch.randn(2, 3, 40, bins, device="cuda")
+        model, x = FrameClassifier(ConvStack(40, bins, params), classes).cuda(), torch.randn(2, 3, 40, bins, device="cuda")
         del looked[:]
         with torch.no_grad(), torch.autocast("cuda", torch.float16):
             model(x)
+            assert model._scores(x) is None
         assert len(looked) == 1
 
 
